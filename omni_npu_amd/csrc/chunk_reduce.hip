@@ -6,34 +6,11 @@
 
 namespace mlahip {
 
-constexpr int kBlk = kPlanBlk;                             // tokens per block of the chunk plan
-constexpr int kSegCost = kPlanSegCost;                     // start-up cost of a segment, in blocks
-
-__device__ __forceinline__ int plan_num_blocks(int len) { return len > 0 ? (len + kBlk - 1) / kBlk : 0; }
-__device__ __forceinline__ int plan_units(int len) { return len > 0 ? (len + kBlk - 1) / kBlk + kSegCost : 0; }
-static_assert(kBlk == kPlanBlk && kSegCost == kPlanSegCost, "the merge kernels recompute the chunk plan with these constants");
-__device__ __forceinline__ int wave_sum_i32(int v) {
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
-  return v;
-}
-__device__ __forceinline__ int wave_max_i32(int v) {
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) v = max(v, __shfl_xor(v, d, 64));
-  return v;
-}
-__device__ __forceinline__ int wave_incl_scan_i32(int v, int lane) {
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) { const int t = __shfl_up(v, d, 64); v += lane >= d ? t : 0; }
-  return v;
-}
-
-typedef __attribute__((address_space(4))) const int32_t* ConstI32Ptr;   // scalar (constant-cache) loads
-
 // N-way merge of the partials of the query rows (src/omni_npu/attention/ops.py:109-141), for the chunk layout written
 // by the split kernels (decode_v3.hip, decode_v3_fp8.hip).  The partials of sequence b are those of the chunks that hold blocks of it, numbered
-// chunk + b.  A wavefront merges kRedRows consecutive rows of one sequence (lane l owns columns 8l..8l+7): it derives
-// the chunk list once, fetches the per-row records of up to kRedParts partials with scalar loads, then asks for the
+// chunk + b: the consecutive numbers between the two that the split kernel left in seg_ids (every chunk of the plan holds
+// at least one unit of work, so none in between is empty).  A wavefront merges kRedRows consecutive rows of one sequence
+// (lane l owns columns 8l..8l+7): it fetches the per-row records of up to kRedParts partials with scalar loads, then asks for the
 // partials and the latent vectors of the flagged dominant keys together before it uses any of them - the kernel is a
 // chain of dependent memory round trips, and this keeps the vector part of the chain at one.  (One row per wave keeps it
 // at four waves per SIMD; the gathers of the dominant keys' vectors are a third of its time.)
@@ -77,27 +54,8 @@ __global__ __launch_bounds__(kWide ? 64 * kWideWaves : 256) void mla_chunk_reduc
   const int rows = qlen * p.num_heads;
   if (row0 >= rows) continue;
 
-  // (everything that depends on b only is requested together: one memory round trip, not three)
   const int id_first = p.seg_ids[2 * b], id_last = p.seg_ids[2 * b + 1];
-  const int mine = plan_units(p.seq_lens[b]);
-  int tot_units = 0, before = 0;
-  for (int i = lane; i < p.batch; i += 64) {
-    const int c = plan_units(p.seq_lens[i]);
-    tot_units += c;
-    before += i < b ? c : 0;
-  }
-  tot_units = __builtin_amdgcn_readfirstlane(wave_sum_i32(tot_units));
-  before = __builtin_amdgcn_readfirstlane(wave_sum_i32(before));
-  const int64_t G = p.num_chunks, T = tot_units;
-  // does chunk c hold blocks of this sequence (units [before, before + mine), the first kSegCost of them start-up)?
-  auto holds_blocks = [&](int64_t c) -> bool {
-    const int64_t cb = c * T / G, ce = (c + 1) * T / G;
-    const int64_t lo = cb > before ? cb : before, hi = ce < before + mine ? ce : before + mine;
-    int64_t rlo = lo - before - kSegCost, rhi = hi - before - kSegCost;
-    rlo = rlo < 0 ? 0 : rlo;
-    rhi = rhi < 0 ? 0 : rhi;
-    return rhi > rlo;
-  };
+  const bool any = p.seq_lens[b] > 0;                        // (an empty sequence has no partial and no numbers either)
 
   typedef _Float16 h8 __attribute__((ext_vector_type(8)));
   float m[kRedRows], tot[kRedRows], a[kRedRows][8];
@@ -108,35 +66,17 @@ __global__ __launch_bounds__(kWide ? 64 * kWideWaves : 256) void mla_chunk_reduc
 #pragma unroll
     for (int e = 0; e < 8; e++) a[j][e] = 0.f;
   }
-  if (mine > 0) {
-    // With at least one unit per chunk every chunk between the sequence's first and last segment holds blocks of it, and
-    // the split kernel left those two partial numbers behind.  Otherwise (tiny workloads) some chunks are empty and the
-    // chunk boundaries are worked out here: chunk c starts at unit floor(c*T/G), the chunk holding unit x is the
-    // largest c with c*T < (x+1)*G.
-    const bool dense_chunks = T >= G;
-    int c, c_last;
-    if (dense_chunks) {
-      c = id_first - b;
-      c_last = id_last - b;
-    } else {
-      c = (int)((((int64_t)before + 1) * G - 1) / T);
-      c_last = (int)((((int64_t)before + mine) * G - 1) / T);
-    }
-    // wide: wavefront w takes the chunks c + w, c + w + 8, ...; where chunks have to be tested one by one (tiny
-    // workloads, a handful of partials) wavefront 0 takes them all
-    int c_step = 1;
-    if constexpr (kWide) {
-      if (dense_chunks) { c += wave; c_step = kWideWaves; }
-      else if (wave != 0) c = c_last + 1;
-    }
-    while (c <= c_last) {
-      int64_t part[kRedParts];                               // partial numbers of this pass (uniform), -1 = none
+  if (any) {
+    // wide: wavefront w takes the partials first + w, first + w + kWideWaves, ...
+    int c = id_first + (kWide ? wave : 0);
+    constexpr int c_step = kWide ? kWideWaves : 1;
+    while (c <= id_last) {
+      int64_t part[kRedParts];                               // rows of this pass's partials (uniform)
       int np = 0;
 #pragma unroll
       for (int q = 0; q < kRedParts; q++) {
-        while (c <= c_last && !dense_chunks && !holds_blocks(c)) c++;     // wrote nothing for this sequence
-        part[q] = c <= c_last ? (int64_t)(c + b) * r_max + row0 : -1;
-        if (c <= c_last) { np++; c += c_step; }
+        part[q] = c <= id_last ? (int64_t)c * r_max + row0 : -1;
+        if (c <= id_last) { np++; c += c_step; }
       }
       // The per-row records (log-sum-exp, correction factor, address of the dominant key's latent vector) are uniform:
       // scalar loads.  One-wavefront form: once they are here the partials AND the latent vectors of the flagged segments

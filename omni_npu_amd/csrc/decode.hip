@@ -86,8 +86,9 @@ static int decode_split_impl(const void* q_nope, int64_t qn_stride_t, int64_t qn
   v.win_skip = win_skip; v.win_sink = win_sink; v.win_size = win_size;
   v.new_c = (const __bf16*)new_c; v.new_c_st = new_c_stride; v.new_r = (const __bf16*)new_r; v.new_r_st = new_r_stride;
   v.new_slots = new_slots;
-  // one workgroup per (balanced chunk, group of 128 query rows)
-  const dim3 grid((unsigned)(batch * num_splits), 1, (unsigned)((r_max + kRowsPerWg - 1) / kRowsPerWg));
+  // one workgroup per (balanced chunk, group of 128 query rows); the chunk axis in whole eighths, one per XCD
+  v.num_chunks = plan_num_chunks(batch, num_splits, r_max);
+  const dim3 grid((unsigned)((v.num_chunks + 7) / 8 * 8), 1, (unsigned)((r_max + kRowsPerWg - 1) / kRowsPerWg));
   if (fp8) return launch_decode_v3_fp8(v, grid, stream);
   return launch_decode_v3(v, sparse_rows != nullptr, grid, stream);
 }
@@ -202,7 +203,7 @@ extern "C" int mla_splitkv_reduce(const void* workspace, size_t workspace_bytes,
   cp.corr_scale = cp.lse_part + rows; cp.corr_row = (const __bf16* const*)(cp.lse_part + 2 * rows);
   cp.seg_ids = (const int32_t*)(cp.lse_part + 4 * rows);
   cp.seq_lens = seq_lens; cp.qsl = query_start_loc;
-  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = batch * num_splits;
+  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = plan_num_chunks(batch, num_splits, r_max);
   cp.out = (__bf16*)out; cp.out_st = out_stride_t; cp.out_sh = out_stride_h;
   cp.lse_out = lse_out; cp.lse_st = num_heads;
   return launch_chunk_reduce(cp, stream);

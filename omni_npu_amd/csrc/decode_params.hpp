@@ -13,7 +13,7 @@ struct DecodeParams {
   const int32_t* block_table; int64_t bt_stride; int32_t max_blocks;
   const int32_t* seq_lens;
   const int32_t* qsl;
-  int32_t batch, max_q_len, num_heads;
+  int32_t batch, max_q_len, num_heads, num_chunks;   // num_chunks: the most chunks the plan may cut (plan_num_chunks)
   int64_t num_pages;
   float scale_log2;
   _Float16* o_part;              // [chunks + B, R_max, 512] fp16, normalised
@@ -48,6 +48,26 @@ int launch_chunk_reduce(const ChunkReduceParams& p, hipStream_t stream);
 constexpr int kPlanBlk = 32;
 constexpr int kPlanSegCost = 8;
 __device__ __forceinline__ int plan_work_units(int len) { return len > 0 ? (len + kPlanBlk - 1) / kPlanBlk + kPlanSegCost : 0; }
+
+// How many chunks the work is cut into.  The host names the most a launch can use: a workgroup has a CU to itself (its LDS
+// fills one), so batch * num_splits chunks are cut down to a whole number of rounds over the CUs - 288 workgroups on 256
+// CUs take as long as 512 would (48 requests x 6 splits, 32 rows: 105 us against 74 with 256 chunks).  The device, which
+// knows the lengths, cuts no finer than kPlanMinUnits units: block tables as wide as the longest context a server accepts
+// ask for hundreds of chunks where the requests at hand hold a few dozen blocks, and each chunk is one more partial to merge.
+constexpr int kPlanMinUnits = 4;
+constexpr int kPlanCUs = 256;                              // MI355X
+inline int plan_num_chunks(int64_t batch, int64_t num_splits, int64_t query_rows) {
+  const int64_t total = batch * num_splits, groups = (query_rows + 127) / 128;
+  const int64_t rounds = total * groups / kPlanCUs;
+  if (rounds < 1) return (int)total;
+  int64_t g = rounds * kPlanCUs / groups;
+  if (g >= 64) g &= ~int64_t(7);                           // (whole eighths, one per XCD)
+  return (int)(g < 1 ? 1 : (g < total ? g : total));
+}
+__device__ __forceinline__ int plan_chunk_count(int total_units, int num_chunks) {
+  const int g = total_units / kPlanMinUnits;
+  return g < 1 ? 1 : (g < num_chunks ? g : num_chunks);
+}
 
 // Merge of the partials fused with the value up-projection (reduce_vup.hip): out[t, n*128 + v] = merged o[t,n,:] . W_UV[n,:,v]
 int launch_reduce_vup(const ChunkReduceParams& r, const void* w_uv, int64_t w_stride_n, int64_t w_stride_k,

@@ -118,13 +118,10 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
   // read the same bytes and are renumbered to sit on one XCD: the row groups of one chunk (more than 128 query rows)
   // stream the same cache rows; consecutive chunks belong to the same sequence and load the same queries, so every XCD
   // takes a contiguous eighth of the chunks.
-  int chunk = blockIdx.x, grp = blockIdx.z;
-  if ((gridDim.x & 7) == 0) {
-    const int lin = blockIdx.x + gridDim.x * blockIdx.z;    // launch order
-    const int j = lin >> 3;                                  // j-th workgroup of XCD lin & 7
-    grp = j % gridDim.z;
-    chunk = (lin & 7) * (gridDim.x >> 3) + j / gridDim.z;
-  }
+  // (the launch pads the chunk axis to whole eighths: j counts the workgroups of XCD lin & 7)
+  const int lin = blockIdx.x + gridDim.x * blockIdx.z;      // launch order
+  const int xcd = lin & 7, xcd_j = (lin >> 3) / gridDim.z;
+  const int grp = (lin >> 3) % gridDim.z;
   const int r_max = p.max_q_len * p.num_heads;
   if (grp * kGrpRows >= r_max) return;
   const uint32_t lds0 = lds_addr_of(lds);
@@ -140,12 +137,12 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
 
   // ---- which blocks are mine: the balanced chunk plan (see mla_chunk_reduce_kernel, which recomputes it) ----
   // Every non-empty sequence is kSegCost units of start-up followed by its 32-key blocks, the sequences end to end, and
-  // that line is cut into gridDim.x chunks of equal length; a chunk that crosses a sequence boundary runs several
+  // that line is cut into plan_chunk_count() chunks of equal length; a chunk that crosses a sequence boundary runs several
   // segments; the segment of sequence b in chunk c writes partial number c + b.
   // With up to 64 sequences a lane holds one sequence's length and query range: everything the plan and the first
   // segment need comes from one round of loads issued together at the start of the kernel (each dependent round trip
   // to memory costs more than a microsecond there, with cold caches).
-  int seg_b;
+  int chunk, seg_b;
   int64_t v_cur, v_end, v_seq;
   int first_L = -1, first_q0 = 0, first_q1 = 0;               // the first segment's sequence, if known from the plan's loads
   {
@@ -166,16 +163,18 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
     else tot = __builtin_amdgcn_readfirstlane(wave_sum_i32(tot));
     // chunk c covers units [floor(c * tot / G), floor((c + 1) * tot / G)); with G <= 65536 that is 32-bit arithmetic:
     // c * tot / G = c * (tot / G) + c * (tot % G) / G exactly (a 64-bit division is a long software routine)
+    const int chunks = plan_chunk_count(tot, p.num_chunks), per_xcd = (chunks + 7) >> 3;
+    chunk = xcd * per_xcd + xcd_j;
+    if (xcd_j >= per_xcd || chunk >= chunks || tot == 0) return;
     int64_t cb, ce;
-    if (gridDim.x <= 65536u) {
-      const uint32_t G = gridDim.x, q = (uint32_t)tot / G, r = (uint32_t)tot - q * G;
+    if (chunks <= 65536) {
+      const uint32_t G = (uint32_t)chunks, q = (uint32_t)tot / G, r = (uint32_t)tot - q * G;
       cb = (int64_t)chunk * q + (uint32_t)chunk * r / G;
       ce = (int64_t)(chunk + 1) * q + ((uint32_t)chunk + 1u) * r / G;
     } else {
-      cb = (int64_t)chunk * tot / gridDim.x;
-      ce = (int64_t)(chunk + 1) * tot / gridDim.x;
+      cb = (int64_t)chunk * tot / chunks;
+      ce = (int64_t)(chunk + 1) * tot / chunks;
     }
-    if (cb == ce) return;
     int carry = 0, b0 = 0, pb0 = 0;
     if (one_pass) {
       // the running totals do not decrease from lane to lane: the sequences that end at or before the chunk's first unit
@@ -1073,7 +1072,7 @@ static int launch_rows(const DecodeParams& p, dim3 grid, hipStream_t stream) {
   // chunk sit next to each other on one XCD and share the cache rows in its L2).  Measured on row lists of 2048 keys,
   // 128 heads, eight chunks per token: 4 tokens 36.1 -> 26.9 us, 8 tokens 37.7 -> 28.8, 16 tokens 40.4 -> 33.3.
   {
-    const int64_t wgs = (int64_t)grid.x * grid.z;
+    const int64_t wgs = (int64_t)p.num_chunks * grid.z;
     if (wgs * 4 <= kNumCUs) { grid.z = (unsigned)((r_max + 31) / 32); return launch_form<kSparse, kWindow, 1, kWrite>(p, grid, stream); }
     if (wgs * 2 <= kNumCUs) { grid.z = (unsigned)((r_max + 63) / 64); return launch_form<kSparse, kWindow, 2, kWrite>(p, grid, stream); }
   }

@@ -8,8 +8,13 @@
 // into the caller's output: four launches and three round trips through memory for 2 MB of result.
 //
 // One workgroup = one head and a run of tokens.  Its 16 wavefronts first ask for the head's W_UV (512 x 128 bf16 =
-// 128 KiB) as global -> LDS copies, then each merges the partials of ONE token's row (the copies land underneath),
-// writes the bf16 row into a 16-row LDS tile, and four wavefronts multiply the tile with W_UV out of LDS: W^T is the
+// 128 KiB) as global -> LDS copies, then merge the partials of the tokens' rows (the copies land underneath).  With many
+// tokens a wavefront merges ONE row; with few, 2 to 16 wavefronts share a row's partials (each takes every 2nd to 16th)
+// and add their states up through LDS, pairs of wavefronts at a time, in an order that depends on the shape only: the
+// kernel is a chain of round trips, and sharing keeps it as long for 64 partials of a row as for four (one request of 1k
+// keys under a plan for 64 chunks: 27 us of separate merge + 10 of GEMM + a copy -> 9 us; 128k keys in 256 partials: 18 + 10
+// + 4 -> 15 us).  The
+// bf16 rows go into a 16-row LDS tile, and four wavefronts multiply the tile with W_UV out of LDS: W^T is the
 // first MFMA operand (32 output columns per wavefront), read with transposed LDS reads exactly like V^T in the decode
 // kernel, the merged rows are the second operand, so a lane ends up with four consecutive output columns of one token.
 #include "mla_common.hpp"
@@ -23,7 +28,8 @@ constexpr int kVupV = 128;                      // v_head_dim
 constexpr int kVupWB = kDNope * kVupV * 2;      // 131072: W_UV of one head, row c at c * 256
 constexpr int kVupOB = kVupTok * kDNope * 2;    // 16384: merged rows of one pass, 1 KiB each
 constexpr int kVupFlagOff = kVupWB + kVupOB;    // one int per token of the pass: its row is valid
-constexpr int kVupLdsB = kVupFlagOff + 64;
+constexpr int kVupStateOff = kVupFlagOff + 64;  // eight (maximum, sum) pairs of an exchange between wavefronts
+constexpr int kVupLdsB = kVupStateOff + 64;
 constexpr int kVupParts = 6;                    // partials of a row asked for together
 constexpr int kVupAhead = 4;                    // GEMM steps whose operands are requested ahead (at most 4: the wait ladder)
 
@@ -33,51 +39,23 @@ __device__ __forceinline__ int vup_wave_sum(int v) {
   return v;
 }
 
-// Merge of the partials of row `row` of sequence b (all arguments wave-uniform), lane l owning columns 8l .. 8l+7.
-// Same bookkeeping as mla_chunk_reduce_kernel: the partials of a sequence are those of the chunks that hold blocks of
-// it, numbered chunk + b; with at least one work unit per chunk they are the consecutive numbers between the two the
-// split kernel left in seg_ids, otherwise the chunk boundaries are worked out from the sequence lengths.
-__device__ __forceinline__ void vup_merge_row(const ChunkReduceParams& p, int b, int row, int lane, float& m, float& tot,
-                                              float (&a)[8]) {
+// Merge of every `step`-th partial, from the `first`-th on, of row `row` of sequence b (all arguments wave-uniform), lane l
+// owning columns 8l .. 8l+7.  Same bookkeeping as mla_chunk_reduce_kernel: the partials of a sequence are the consecutive
+// numbers between the two the split kernel left in seg_ids.
+__device__ __forceinline__ void vup_merge_row(const ChunkReduceParams& p, int b, int row, int lane, int first, int step,
+                                              float& m, float& tot, float (&a)[8]) {
   typedef _Float16 h8 __attribute__((ext_vector_type(8)));
   const int r_max = p.max_q_len * p.num_heads;
   const int id_first = p.seg_ids[2 * b], id_last = p.seg_ids[2 * b + 1];
-  const int mine = plan_work_units(p.seq_lens[b]);
-  int tot_units = 0, before = 0;
-  for (int i = lane; i < p.batch; i += 64) {
-    const int c = plan_work_units(p.seq_lens[i]);
-    tot_units += c;
-    before += i < b ? c : 0;
-  }
-  tot_units = __builtin_amdgcn_readfirstlane(vup_wave_sum(tot_units));
-  before = __builtin_amdgcn_readfirstlane(vup_wave_sum(before));
-  if (mine <= 0) return;
-  const int64_t G = p.num_chunks, T = tot_units;
-  auto holds_blocks = [&](int64_t c) -> bool {
-    const int64_t cb = c * T / G, ce = (c + 1) * T / G;
-    const int64_t lo = cb > before ? cb : before, hi = ce < before + mine ? ce : before + mine;
-    int64_t rlo = lo - before - kPlanSegCost, rhi = hi - before - kPlanSegCost;
-    rlo = rlo < 0 ? 0 : rlo;
-    rhi = rhi < 0 ? 0 : rhi;
-    return rhi > rlo;
-  };
-  const bool dense_chunks = T >= G;
-  int c, c_last;
-  if (dense_chunks) {
-    c = id_first - b;
-    c_last = id_last - b;
-  } else {
-    c = (int)((((int64_t)before + 1) * G - 1) / T);
-    c_last = (int)((((int64_t)before + mine) * G - 1) / T);
-  }
-  while (c <= c_last) {
+  if (p.seq_lens[b] <= 0) return;
+  int c = id_first + first;
+  while (c <= id_last) {
     int64_t part[kVupParts];
     int np = 0;
 #pragma unroll
     for (int q = 0; q < kVupParts; q++) {
-      while (c <= c_last && !dense_chunks && !holds_blocks(c)) c++;
-      part[q] = c <= c_last ? (int64_t)(c + b) * r_max + row : 0;
-      if (c <= c_last) { np++; c++; }
+      part[q] = c <= id_last ? (int64_t)c * r_max + row : 0;
+      if (c <= id_last) { np++; c += step; }
     }
     // records by scalar loads (uniform addresses), then the partials and the latent vectors of the flagged dominant
     // keys in one vector round trip
@@ -121,7 +99,8 @@ __device__ __forceinline__ void vup_merge_row(const ChunkReduceParams& p, int b,
 struct ReduceVupParams {
   ChunkReduceParams r;                 // r.out: [T, N * 128] through (out_st, out_sh)
   const __bf16* w_uv; int64_t w_sn, w_sk;   // W_UV [N, 512, 128]: head stride, row stride (elements)
-  int32_t num_tokens, passes;          // a workgroup handles passes * 16 consecutive tokens
+  int32_t num_tokens, passes;          // a workgroup handles passes * (16 / share) consecutive tokens
+  int32_t share_log2;                  // log2 of the wavefronts that share a row
 };
 
 __global__ __launch_bounds__(1024) void mla_reduce_vup_kernel(const ReduceVupParams pp) {
@@ -155,9 +134,11 @@ __global__ __launch_bounds__(1024) void mla_reduce_vup_kernel(const ReduceVupPar
   }
 
   const int h32 = lane & 31, half = lane >> 5;
+  const int share = 1 << pp.share_log2, toks = kVupTok >> pp.share_log2;      // wavefronts per row, tokens per pass
+  const int sub = wave & (share - 1), slot = wave >> pp.share_log2;           // this wavefront's part and row of the pass
   for (int pass = 0; pass < pp.passes; pass++) {
-    // ---- one row per wavefront: token t, this head ----
-    const int t = (tb * pp.passes + pass) * kVupTok + wave;
+    // ---- token t, this head ----
+    const int t = (tb * pp.passes + pass) * toks + slot;
     bool valid = t < pp.num_tokens;
     int b = 0, t_local = 0;
     if (valid) {
@@ -180,20 +161,44 @@ __global__ __launch_bounds__(1024) void mla_reduce_vup_kernel(const ReduceVupPar
       valid = valid && t_local >= 0 && t_local < qlen;
     }
     float m = -INFINITY, tot = 0.f, a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (valid) vup_merge_row(p, b, t_local * p.num_heads + head, lane, m, tot, a);
+    if (valid) vup_merge_row(p, b, t_local * p.num_heads + head, lane, sub, share, m, tot, a);
+    // the states of the wavefronts that share a row, halves added up until one is left (the exchange uses the row tile,
+    // which is written after it: 8 states of 2 KiB, and the flags' place behind it for their maxima and sums)
+    for (int s = share >> 1; s >= 1; s >>= 1) {
+      const int at = slot * s + (sub - s);
+      if (sub >= s && sub < 2 * s) {
+        *(f32x4*)(lds + kVupWB + at * 2048 + lane * 16) = f32x4{a[0], a[1], a[2], a[3]};
+        *(f32x4*)(lds + kVupWB + at * 2048 + 1024 + lane * 16) = f32x4{a[4], a[5], a[6], a[7]};
+        if (lane == 0) *(f32x2*)(lds + kVupStateOff + at * 8) = f32x2{m, tot};
+      }
+      lds_barrier();
+      if (sub < s) {
+        const int from = slot * s + sub;
+        const f32x2 mt = *(const f32x2*)(lds + kVupStateOff + from * 8);
+        const f32x4 a0 = *(const f32x4*)(lds + kVupWB + from * 2048 + lane * 16);
+        const f32x4 a1 = *(const f32x4*)(lds + kVupWB + from * 2048 + 1024 + lane * 16);
+        const float mn = fmaxf(m, mt[0]);
+        const float f0 = m == -INFINITY ? 0.f : __expf(m - mn), f1 = mt[0] == -INFINITY ? 0.f : __expf(mt[0] - mn);
+        m = mn;
+        tot = tot * f0 + mt[1] * f1;
+#pragma unroll
+        for (int e = 0; e < 4; e++) { a[e] = a[e] * f0 + a0[e] * f1; a[4 + e] = a[4 + e] * f0 + a1[e] * f1; }
+      }
+      lds_barrier();
+    }
     // The bf16 row goes to LDS in the order the MFMA wants its contraction index: within every 16 columns the first
     // granule holds columns {0..3, 8..11}, the second {4..7, 12..15} (the transposed reads of W deliver them in that
     // order), and granule g of row r sits at position g ^ r so that 16 rows read at the same g hit different banks.
-    {
+    if (sub == 0) {
       const float inv = tot > 0.f ? 1.f / tot : 0.f;
       bf16x4 lo, hi;
 #pragma unroll
       for (int e = 0; e < 4; e++) { lo[e] = (__bf16)(a[e] * inv); hi[e] = (__bf16)(a[4 + e] * inv); }
-      char* rowp = lds + kVupWB + wave * 1024 + (lane & 1) * 8;
+      char* rowp = lds + kVupWB + slot * 1024 + (lane & 1) * 8;
       const int g0 = (lane >> 1) * 2;
-      *(bf16x4*)(rowp + (((g0) ^ wave) << 4)) = lo;
-      *(bf16x4*)(rowp + (((g0 + 1) ^ wave) << 4)) = hi;
-      if (lane == 0) *(int*)(lds + kVupFlagOff + wave * 4) = valid ? 1 : 0;
+      *(bf16x4*)(rowp + (((g0) ^ slot) << 4)) = lo;
+      *(bf16x4*)(rowp + (((g0 + 1) ^ slot) << 4)) = hi;
+      if (lane == 0) *(int*)(lds + kVupFlagOff + slot * 4) = valid ? 1 : 0;
     }
     MLA_WAIT_VMCNT(0);                                        // this wavefront's share of W_UV has landed
     lds_barrier();
@@ -239,8 +244,8 @@ __global__ __launch_bounds__(1024) void mla_reduce_vup_kernel(const ReduceVupPar
         }
 #undef VUP_READ
       }
-      const int tt = (tb * pp.passes + pass) * kVupTok + tr;
-      const bool ok = h32 < kVupTok && *(const int*)(lds + kVupFlagOff + tr * 4) != 0;
+      const int tt = (tb * pp.passes + pass) * toks + tr;
+      const bool ok = h32 < toks && *(const int*)(lds + kVupFlagOff + tr * 4) != 0;
       if (ok) {
         __bf16* o = p.out + (int64_t)tt * p.out_st + (int64_t)head * p.out_sh + wave * 32 + 4 * half;
 #pragma unroll
@@ -264,12 +269,18 @@ int launch_reduce_vup(const ChunkReduceParams& r, const void* w_uv, int64_t w_st
   pp.r = r;
   pp.w_uv = (const __bf16*)w_uv; pp.w_sn = w_stride_n; pp.w_sk = w_stride_k;
   pp.num_tokens = num_tokens;
-  // about one workgroup per compute unit: 16 tokens per pass, as many passes as that takes
-  const int64_t blocks16 = ((int64_t)num_tokens + kVupTok - 1) / kVupTok;
-  int64_t passes = (blocks16 * r.num_heads + 255) / 256;
+  // About one workgroup per compute unit.  As many wavefronts share a row as leave no more workgroups than compute units
+  // (16 tokens per pass and workgroup where a row has a wavefront to itself), but not more than the row has partials.
+  const int64_t parts = r.batch > 0 ? (r.num_chunks + r.batch - 1) / r.batch + 1 : 1;
+  int lg = 0;
+  while (lg < 4 && (2 << lg) <= parts && (((int64_t)num_tokens + (kVupTok >> (lg + 1)) - 1) / (kVupTok >> (lg + 1))) * r.num_heads <= 256) lg++;
+  const int toks = kVupTok >> lg;
+  const int64_t blocks = ((int64_t)num_tokens + toks - 1) / toks;
+  int64_t passes = (blocks * r.num_heads + 255) / 256;
   passes = passes < 1 ? 1 : (passes > 64 ? 64 : passes);
   pp.passes = (int32_t)passes;
-  const int64_t tbs = (blocks16 + passes - 1) / passes;
+  pp.share_log2 = lg;
+  const int64_t tbs = (blocks + passes - 1) / passes;
   hipLaunchKernelGGL(mla_reduce_vup_kernel, dim3((unsigned)tbs, (unsigned)r.num_heads), dim3(1024), kVupLdsB, stream, pp);
   return check_launch("mla_reduce_vup_kernel");
 }
@@ -306,7 +317,7 @@ extern "C" int mla_splitkv_reduce_vup(const void* workspace, size_t workspace_by
   cp.corr_scale = cp.lse_part + rows; cp.corr_row = (const __bf16* const*)(cp.lse_part + 2 * rows);
   cp.seg_ids = (const int32_t*)(cp.lse_part + 4 * rows);
   cp.seq_lens = seq_lens; cp.qsl = query_start_loc;
-  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = batch * num_splits;
+  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = plan_num_chunks(batch, num_splits, r_max);
   cp.out = (__bf16*)out; cp.out_st = out_stride_t; cp.out_sh = out_stride_h;
   cp.lse_out = nullptr; cp.lse_st = 0;
   return launch_reduce_vup(cp, w_uv, w_stride_n, w_stride_k, num_tokens, stream);

@@ -133,3 +133,15 @@ def test_fused_up_projection_after_fp8_and_sparse_decode(dev):
     unfused_s = torch.bmm(o_s.transpose(0, 1).float(), w.float()).transpose(0, 1).reshape(4, heads * 128)
     torch.cuda.synchronize()
     assert (out_s.float() - unfused_s).abs().max().item() <= unfused_s.abs().max().item() * 2 ** -7
+
+
+@pytest.mark.parametrize("batch,heads,q_len,lo,hi,splits", [
+    (1, 16, 1, 1, 1, 64), (1, 16, 1, 33, 33, 64),             # one block, two blocks under a plan for 64 chunks
+    (1, 16, 1, 1000, 1000, 64), (2, 16, 1, 900, 2000, 99),    # 16 wavefronts share a row
+    (2, 128, 1, 900, 2000, 99), (7, 128, 1, 1, 900, 37),      # 8, then 4
+    (9, 32, 1, 100, 900, 20), (17, 16, 2, 60, 600, 9),        # 2; and a last pass that is not full
+    (48, 16, 2, 40, 700, 6), (65, 128, 1, 30, 200, 4),        # batch x splits above the CUs: 288 -> 256, 260 -> 256 chunks
+    (90, 40, 3, 1, 120, 3), (70, 16, 1, 1, 40, 4),            # two row groups: 128 chunks each; fewer units than chunks
+])
+def test_chunk_plan_and_shared_rows_at_their_edges(dev, batch, heads, q_len, lo, hi, splits):
+    test_fused_merge_and_up_projection(dev, batch, heads, q_len, lo, hi, splits)
