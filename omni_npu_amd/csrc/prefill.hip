@@ -9,8 +9,21 @@
 //
 // One workgroup = 4 wavefronts = (128 query rows, one head, one sequence); each wavefront owns 32 rows with its
 // 192-wide query in registers (B operand of S^T = K Q^T) and a 128 x 32 fp32 accumulator O^T.  Key tiles of 64 keys
-// (nope 64 x 256 B, rope 64 x 128 B, V 64 x 256 B) are copied global -> LDS without touching registers, double
-// buffered; V^T operands come from transposed LDS reads, so P^T stays in registers exactly as in the decode kernel.
+// (five sub-tiles of 64 x 128 B) are copied global -> LDS without touching registers, double buffered; V^T operands come
+// from transposed LDS reads, so P^T stays in registers exactly as in the decode kernel.
+//
+// What bounds it: the socket's power cap.  On the 4 x 2048 over 16k, 128-head context launch the matrix pipe is busy 61 %
+// of the cycles and the clock settles at 1.67 GHz at 1350 W, so what pays is fewer instructions per score and what lets
+// the clock settle lower:
+//  * a tile costs one fused multiply-add, one exponential, half a conversion and half a v_dot2 (the sum) per score.  A
+//    row's reference is its first tile's maximum and is raised only where a probability outgrows it by 2^13: no maximum
+//    and no rescaling in the steady state (136 -> 76 instructions per wavefront and 32 keys, 11 970 -> 11 110 us);
+//  * both 32-key blocks of a tile are scored before the first exponential, at a raised wave priority (s_setprio), so the
+//    two wavefronts of a SIMD fall out of step and one's vector work runs beside the other's MFMAs (11 110 -> 10 350 us =
+//    1.06 PFLOP/s; causal 4 x 2048 994 -> 860 us).
+// Tried beside it: tiles without a mask in a code path of their own, with and without a prescribed interleaving of the second
+// block's MFMAs and the first block's exponentials (10 860-10 940 us); eight wavefronts of 32 rows, half the tile copies
+// (10 130 us, but causal launches 860 -> 917 and ragged prompts 321 -> 355); heavy query blocks first (no change).
 //
 // P.V runs on fp16: the V part of a landed tile is converted from bf16 to fp16 where it lies (same size, same swizzle:
 // element by element), once for the four wavefronts, and the probabilities are rounded to fp16, so they keep 11
@@ -23,21 +36,20 @@
 namespace mlahip {
 
 constexpr int kPfTile = 64;
-constexpr int kPfKnB = kPfTile * 256;            // 16384  k_nope tile
-constexpr int kPfKrB = kPfTile * 128;            // 8192   k_pe tile
-constexpr int kPfVB = kPfTile * 256;             // 16384  v tile
-constexpr int kPfBufB = kPfKnB + kPfKrB + kPfVB; // 40960
-constexpr int kPfLdsB = 2 * kPfBufB;             // 81920
+constexpr int kPfSubB = kPfTile * 128;           // 8192   64 columns (128 bytes) of the 64 keys of a tile
+constexpr int kPfVOff = 3 * kPfSubB;             // 24576  sub-tiles 0, 1: k_nope, 2: k_pe, 3, 4: v
+constexpr int kPfBufB = 5 * kPfSubB;             // 40960
+constexpr int kPfLdsB = 2 * kPfBufB;             // 81920: two workgroups per CU
 constexpr int kPfRows = 128;
+// A probability may reach 2^13 of its row's reference before the reference is raised (fp16 holds 65504)
+constexpr float kPfRaise = 8192.f;
+constexpr float kPfNoRef = -1e30f;               // reference of a row that has seen no key
 
-__device__ __forceinline__ int pf_swz16(int r) {  // bijection of r % 16, also spreads 4 consecutive rows x 64 B
-  int r0 = r & 1, r1 = (r >> 1) & 1, r2 = (r >> 2) & 1, r3 = (r >> 3) & 1;
-  return ((r1 ^ r3) << 3) | (r0 << 2) | (r1 << 1) | r2;
-}
-__device__ __forceinline__ int pf_swz8(int r) {
-  int r0 = r & 1, r1 = (r >> 1) & 1, r2 = (r >> 2) & 1, r3 = (r >> 3) & 1;
-  return ((r0 ^ r3) << 2) | (r1 << 1) | r2;
-}
+// Row r of a sub-tile keeps its 16-byte granule g at position g ^ pf_swz(r).  The sixteen rows of a phase of a 16-byte read
+// then hit sixteen different bank groups, and so do the four rows of a transposed read (whose two 32-byte halves lie in
+// granules that differ in bit 0 and 1).  Rows are 128 bytes and not the 256 of a key's 128 columns, so that the column
+// step of the operand reads is an XOR of two address bits (four base registers) and an immediate offset.
+__device__ __forceinline__ int pf_swz(int r) { return ((r >> 1) & 1) << 2 | ((r >> 2) & 1) << 1 | ((r >> 3) & 1); }
 
 struct PrefillParams {
   const __bf16* q_nope; int64_t qn_st, qn_sh;
@@ -57,47 +69,19 @@ struct PrefillParams {
   const float* prev_lse;  // [T, N]
 };
 
-// copy one 64-key tile (keys k0 .. k0+63 of the flat key axis, clamped to klast) of head `head`
-__device__ __forceinline__ void pf_issue_tile(const PrefillParams& p, int64_t k0, int64_t klast, int head, uint32_t buf,
-                                              int wave, int lane) {
-  // k_nope and v: 16 granules per row, one wave instruction covers 4 rows; 16 instructions per tensor, 4 per wave
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int r = (wave * 4 + i) * 4 + (lane >> 4);
-    int64_t key = k0 + r;
-    key = key < klast ? key : klast;
-    const int c = (lane & 15) ^ pf_swz16(r & 15);
-    dma16_v(p.k_nope + key * p.kn_st + (int64_t)head * p.kn_sh + c * 8, buf + (wave * 4 + i) * 1024);
-    dma16_v(p.v + key * p.v_st + (int64_t)head * p.v_sh + c * 8, buf + kPfKnB + kPfKrB + (wave * 4 + i) * 1024);
-  }
-  // k_pe: 8 granules per row, one wave instruction covers 8 rows; 8 instructions, 2 per wave
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int r = (wave * 2 + i) * 8 + (lane >> 3);
-    int64_t key = k0 + r;
-    key = key < klast ? key : klast;
-    const int c = (lane & 7) ^ pf_swz8(r & 15);
-    dma16_v(p.k_pe + key * p.kp_st + c * 8, buf + kPfKnB + (wave * 2 + i) * 1024);
-  }
-}
-
-// Per-lane source offsets of a FULL tile (all 64 keys exist), relative to the tile's first key: the copies then need one
-// uniform base per tensor and no per-lane address arithmetic.
-struct PfLaneOffsets { uint32_t kn[4], v[4], kp[2]; };
+// One 64-key tile of head `head`, keys k0 .. k0 + 63 of the flat key axis (clamped to klast): 40 copy instructions of eight
+// 128-byte rows, ten per wavefront (rows 16w .. 16w + 15 of the five sub-tiles).  off: per-lane source offsets of the
+// wavefront's two row groups relative to the tile's first key, when all 64 keys exist.
+struct PfLaneOffsets { uint32_t kn[2], v[2], kp[2]; };
 __device__ __forceinline__ PfLaneOffsets pf_lane_offsets(const PrefillParams& p, int wave, int lane) {
   PfLaneOffsets o;
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int r = (wave * 4 + i) * 4 + (lane >> 4);
-    const int c = (lane & 15) ^ pf_swz16(r & 15);
-    o.kn[i] = (uint32_t)(r * p.kn_st * 2 + c * 16);
-    o.v[i] = (uint32_t)(r * p.v_st * 2 + c * 16);
-  }
-#pragma unroll
   for (int i = 0; i < 2; i++) {
-    const int r = (wave * 2 + i) * 8 + (lane >> 3);
-    const int c = (lane & 7) ^ pf_swz8(r & 15);
-    o.kp[i] = (uint32_t)(r * p.kp_st * 2 + c * 16);
+    const int r = wave * 16 + i * 8 + (lane >> 3);
+    const int c = ((lane & 7) ^ pf_swz(r & 15)) * 16;
+    o.kn[i] = (uint32_t)(r * p.kn_st * 2 + c);
+    o.v[i] = (uint32_t)(r * p.v_st * 2 + c);
+    o.kp[i] = (uint32_t)(r * p.kp_st * 2 + c);
   }
   return o;
 }
@@ -107,12 +91,32 @@ __device__ __forceinline__ void pf_issue_full_tile(const PrefillParams& p, const
   const char* vv = (const char*)(p.v + k0 * p.v_st + (int64_t)head * p.v_sh);
   const char* kp = (const char*)(p.k_pe + k0 * p.kp_st);
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    dma16_sv(kn, o.kn[i], buf + (wave * 4 + i) * 1024);
-    dma16_sv(vv, o.v[i], buf + kPfKnB + kPfKrB + (wave * 4 + i) * 1024);
+  for (int i = 0; i < 2; i++) {
+    const uint32_t dst = buf + (wave * 2 + i) * 1024;
+    dma16_sv(kn, o.kn[i], dst);
+    dma16_sv(kn + 128, o.kn[i], dst + kPfSubB);
+    dma16_sv(kp, o.kp[i], dst + 2 * kPfSubB);
+    dma16_sv(vv, o.v[i], dst + 3 * kPfSubB);
+    dma16_sv(vv + 128, o.v[i], dst + 4 * kPfSubB);
   }
+}
+__device__ __forceinline__ void pf_issue_tile(const PrefillParams& p, int64_t k0, int64_t klast, int head, uint32_t buf,
+                                              int wave, int lane) {
 #pragma unroll
-  for (int i = 0; i < 2; i++) dma16_sv(kp, o.kp[i], buf + kPfKnB + (wave * 2 + i) * 1024);
+  for (int i = 0; i < 2; i++) {
+    const int r = wave * 16 + i * 8 + (lane >> 3);
+    int64_t key = k0 + r;
+    key = key < klast ? key : klast;
+    const int c = ((lane & 7) ^ pf_swz(r & 15)) * 8;
+    const __bf16* kn = p.k_nope + key * p.kn_st + (int64_t)head * p.kn_sh + c;
+    const __bf16* vv = p.v + key * p.v_st + (int64_t)head * p.v_sh + c;
+    const uint32_t dst = buf + (wave * 2 + i) * 1024;
+    dma16_v(kn, dst);
+    dma16_v(kn + 64, dst + kPfSubB);
+    dma16_v(p.k_pe + key * p.kp_st + c, dst + 2 * kPfSubB);
+    dma16_v(vv, dst + 3 * kPfSubB);
+    dma16_v(vv + 64, dst + 4 * kPfSubB);
+  }
 }
 
 // kHalf: k_nope, k_pe and v hold fp16 instead of bf16 (a caller that makes them with an fp16 GEMM): both products run on
@@ -185,7 +189,7 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
   for (int i = 0; i < 4; i++)
 #pragma unroll
     for (int r = 0; r < 16; r++) acc[i][r] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
+  float m_run = kPfNoRef, l_run = 0.f;
   if (p.prev_out != nullptr && row_ok) {
     // Continue from (out, lse) over other keys: running maximum = lse (as a base-2 exponent), running sum = 1, accumulator
     // = out.  A row without earlier keys comes with lse = -inf (+inf is read the same way, as the two-way merge does) and
@@ -237,25 +241,19 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
         }
       }
     }
-    // per-lane LDS offsets
-    const int fk = pf_swz16(h32 & 15), fr = pf_swz8(h32 & 15);
-    int koff[8], roff[4];
+    // per-lane LDS offsets: K granule 2 j + half of a row (j = 0..3 inside a sub-tile), V rows v_row and v_row + 8 with the
+    // 32-column halves of a sub-tile
+    int koff[4], voff[2][2];
 #pragma unroll
-    for (int j = 0; j < 8; j++) koff[j] = h32 * 256 + (((j * 2 + half) ^ fk) << 4);
-#pragma unroll
-    for (int j = 0; j < 4; j++) roff[j] = kPfKnB + h32 * 128 + (((j * 2 + half) ^ fr) << 4);
+    for (int j = 0; j < 4; j++) koff[j] = h32 * 128 + (((j * 2 + half) ^ pf_swz(h32 & 15)) << 4);
     const int g16 = lane >> 4, j16 = lane & 15;
     const int v_row = 4 * (g16 >> 1) + (j16 >> 2);
     const int v_cl = 2 * (g16 & 1) + ((j16 & 3) >> 1);
-    const int v_in = (j16 & 1) * 8;
-    int voff[2][4];                                           // [rd][db]
 #pragma unroll
-    for (int rd = 0; rd < 2; rd++) {
-      const int rr = v_row + 8 * rd;
-      const int f = pf_swz16(rr & 15);
+    for (int rd = 0; rd < 2; rd++)
 #pragma unroll
-      for (int db = 0; db < 4; db++) voff[rd][db] = kPfKnB + kPfKrB + rr * 256 + v_in + (((db * 4 + v_cl) ^ f) << 4);
-    }
+      for (int e = 0; e < 2; e++)
+        voff[rd][e] = kPfVOff + (v_row + 8 * rd) * 128 + (j16 & 1) * 8 + (((e * 4 + v_cl) ^ pf_swz(v_row + 8 * rd)) << 4);
 
     for (int tile = first_tile; tile < tiles; tile++) {
       char* buf = lds + (tile & 1) * kPfBufB;
@@ -267,7 +265,7 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
       // V of this tile goes from bf16 to fp16 where it lies (thread t takes the 16-byte pieces t, t + 256, ...), then a
       // barrier: the four wavefronts read each other's pieces.  (Tried: the conversion's arithmetic and writes behind the
       // first block's score MFMAs, and the next tile converted between the two blocks of this one - both slower.)
-      char* vt = buf + kPfKnB + kPfKrB + (int)threadIdx.x * 16;
+      char* vt = buf + kPfVOff + (int)threadIdx.x * 16;
       if constexpr (!kHalf) {
         u32x4 w[4];
 #pragma unroll
@@ -284,74 +282,82 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
         for (int i = 0; i < 4; i++) *(u32x4*)(vt + i * 4096) = w[i];
         lds_barrier();
       }
-#pragma unroll 1
-      for (int tb = 0; tb < 2; tb++) {
-        const bool active = key_base + tb * 32 < wave_max_limit && key_base + tb * 32 + 32 > wg_lo;
-        if (!active) continue;
-        f32x16 s;
+      if (key_base >= wave_max_limit || key_base + kPfTile <= wg_lo) continue;   // no row of this wavefront sees the tile
+
+      f32x16 s[2];
+      f16x2 pb[2][8];
+      auto scores = [&](int tb) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) s[r] = 0.f;
+        for (int r = 0; r < 16; r++) s[tb][r] = 0.f;
 #pragma unroll
-        for (int kk = 0; kk < 8; kk++) {
-          bf16x8 a = *(const bf16x8*)(buf + tb * 32 * 256 + koff[kk]);
-          if constexpr (kHalf) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, qf[kk]), s, 0, 0, 0);
-          else s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[kk], s, 0, 0, 0);
+        for (int kk = 0; kk < 12; kk++) {
+          const bf16x8 a = *(const bf16x8*)(buf + koff[kk & 3] + (kk >> 2) * kPfSubB + tb * 4096);
+          if constexpr (kHalf) s[tb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, qf[kk]), s[tb], 0, 0, 0);
+          else s[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[kk], s[tb], 0, 0, 0);
         }
+      };
+      // probabilities against the row's reference as fp16 pairs, and the sum of what was rounded (v_dot2 adds a pair)
+      auto probs = [&](int tb, float sum) -> float {
+        const float neg = -m_run;
 #pragma unroll
-        for (int kk = 0; kk < 4; kk++) {
-          bf16x8 a = *(const bf16x8*)(buf + tb * 32 * 128 + roff[kk]);
-          if constexpr (kHalf) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, qf[8 + kk]), s, 0, 0, 0);
-          else s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[8 + kk], s, 0, 0, 0);
+        for (int r = 0; r < 8; r++) {
+          pb[tb][r] = __builtin_convertvector((f32x2{fast_exp2(__builtin_fmaf(s[tb][2 * r], p.scale_log2, neg)),
+                                                     fast_exp2(__builtin_fmaf(s[tb][2 * r + 1], p.scale_log2, neg))}), f16x2);
+          sum = __builtin_amdgcn_fdot2(pb[tb][r], f16x2{(_Float16)1.f, (_Float16)1.f}, sum, false);
         }
-        // Only blocks that some row of this wave cannot see in full pay for the mask (causal diagonal, end of the keys,
-        // rows past the end of the sequence); everywhere else the scores go straight to the maximum.  The scale is
-        // folded into the exponent's multiply-add (scale > 0, so the maximum of the raw scores is the raw maximum).
-        if (key_base + tb * 32 + 32 > wave_min_limit || key_base + tb * 32 < wave_max_lo) {
-          const int key_lane0 = key_base + tb * 32 + 4 * half;
+        return sum;
+      };
+      __builtin_amdgcn_s_setprio(1);
+      scores(0);
+      scores(1);
+      __builtin_amdgcn_s_setprio(0);
+      // Only tiles that some row of this wave cannot see in full pay for the mask (causal diagonal, end of the keys,
+      // rows past the end of the sequence).
+      if (key_base + kPfTile > wave_min_limit || key_base < wave_max_lo) {
+#pragma unroll
+        for (int tb = 0; tb < 2; tb++)
 #pragma unroll
           for (int r = 0; r < 16; r++) {
-            const int key = key_lane0 + 8 * (r >> 2) + (r & 3);
-            s[r] = (key < limit && key >= lo) ? s[r] : -INFINITY;
-          }
-        }
-        float mx = fmaxf(fmaxf(s[0], s[1]), s[2]);
-#pragma unroll
-        for (int r = 3; r < 15; r += 2) mx = fmaxf(fmaxf(mx, s[r]), s[r + 1]);
-        mx = fmaxf(mx, s[15]);
-        mx = fmaxf(mx, xor32(mx)) * p.scale_log2;
-        const float m_new = fmaxf(m_run, mx);
-        const float m_safe = m_new == -INFINITY ? 0.f : m_new;
-        const float alpha = fast_exp2(m_run - m_safe);
-        const float neg = -m_safe;
-        float psum = 0.f;
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-          s[r] = fast_exp2(__builtin_fmaf(s[r], p.scale_log2, neg));
-          psum += s[r];
-        }
-        l_run = l_run * alpha + psum;
-        m_run = m_new;
-        if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
-#pragma unroll
-          for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][r] *= alpha;
-        }
-        f16x8 pb[2];
-#pragma unroll
-        for (int kb = 0; kb < 2; kb++)
-#pragma unroll
-          for (int e = 0; e < 8; e++) pb[kb][e] = (_Float16)s[kb * 8 + e];
-#pragma unroll
-        for (int db = 0; db < 4; db++)
-#pragma unroll
-          for (int kb = 0; kb < 2; kb++) {
-            bf16x4 lo = lds_read_tr16(buf + (tb * 32 + kb * 16) * 256 + voff[0][db]);
-            bf16x4 hi = lds_read_tr16(buf + (tb * 32 + kb * 16) * 256 + voff[1][db]);
-            bf16x8 a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-            acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), pb[kb], acc[db], 0, 0, 0);
+            const int key = key_base + tb * 32 + 4 * half + 8 * (r >> 2) + (r & 3);
+            s[tb][r] = (key < limit && key >= lo) ? s[tb][r] : -INFINITY;
           }
       }
+      float psum = probs(1, probs(0, 0.f));
+      // A row's reference is raised only when its probabilities outgrow it by 2^13, so the maximum of a tile, the rescaling
+      // of the accumulator and the dependent exponential are paid in the first tile of a row and hardly ever after it.
+      if (__builtin_amdgcn_ballot_w64(psum > kPfRaise) != 0) {
+        float mx = fmaxf(s[0][0], s[1][0]);
+#pragma unroll
+        for (int r = 1; r < 16; r++) mx = fmaxf(fmaxf(mx, s[0][r]), s[1][r]);
+        const float m_new = fmaxf(m_run, fmaxf(mx, xor32(mx)) * p.scale_log2);
+        const float alpha = fast_exp2(m_run - m_new);
+        m_run = m_new;
+        l_run *= alpha;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) acc[i][r] *= alpha;
+        psum = probs(1, probs(0, 0.f));
+      }
+      l_run += psum;
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int tb = 0; tb < 2; tb++)
+#pragma unroll
+        for (int kb = 0; kb < 2; kb++) {
+          f16x8 pv;
+#pragma unroll
+          for (int e = 0; e < 8; e++) pv[e] = pb[tb][kb * 4 + (e >> 1)][e & 1];
+#pragma unroll
+          for (int db = 0; db < 4; db++) {
+            const char* vb = buf + (db >> 1) * kPfSubB + tb * 4096 + kb * 2048;
+            const bf16x4 v_lo = lds_read_tr16(vb + voff[0][db & 1]);
+            const bf16x4 v_hi = lds_read_tr16(vb + voff[1][db & 1]);
+            const bf16x8 a = __builtin_shufflevector(v_lo, v_hi, 0, 1, 2, 3, 4, 5, 6, 7);
+            acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), pv, acc[db], 0, 0, 0);
+          }
+        }
+      __builtin_amdgcn_s_setprio(0);
     }
   }
 

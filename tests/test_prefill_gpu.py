@@ -305,3 +305,32 @@ def test_values_outside_the_fp16_range_saturate_and_stay_finite(dev):
     attn_close(got[mask].view(1, -1), ref[mask].view(1, -1), 2e-2, 4e-4)
     sat = got[40:, 0, 3]
     assert (sat > 0).all() and (sat <= 65504.0 * 1.001).all()
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("sq,sk,causal,window", [(1, 1, True, None), (31, 33, False, None), (64, 64, True, None), (65, 129, True, None),
+                                                 (129, 191, True, 70), (200, 500, False, None)])
+def test_scores_that_climb_tile_by_tile_raise_the_reference(dev, half, sq, sk, causal, window):
+    """Keys ordered by score, so that every tile of 64 outgrows the row's reference (by far more than the 2^13 a
+    probability may reach before the reference is raised, up to the fp16 range and beyond it), and the same keys in
+    falling order, where it never moves; sizes around the edges of a tile and of a row block.  Bar of the bf16 output."""
+    from omni_npu_amd import kernels as K
+    g = torch.Generator().manual_seed(sq * 1000 + sk)
+    n, scale = 3, 192 ** -0.5
+    ramp = torch.linspace(-40, 40, sk).view(sk, 1, 1)          # in units of the score
+    qn, qp = torch.randn(sq, n, 128, generator=g), torch.randn(sq, n, 64, generator=g)
+    qn[..., 0] = 1 / scale / 4
+    kn, kp, v = torch.randn(sk, n, 128, generator=g) * 0.3, torch.randn(sk, 64, generator=g) * 0.3, torch.randn(sk, n, 128, generator=g)
+    for sign in (1, -1):
+        k = kn.clone()
+        k[..., 0:1] = ramp * sign * 4
+        a = [x.bfloat16() for x in (qn, qp, k, kp, v)]
+        kvt = (lambda x: x.to(torch.float16)) if half else (lambda x: x)
+        out = torch.empty(sq, n, 128, dtype=torch.bfloat16, device=dev)
+        lse = torch.empty(sq, n, device=dev)
+        cu = lambda m: torch.tensor([0, m], dtype=torch.int32, device=dev)
+        K.prefill_varlen(a[0].to(dev), a[1].to(dev), *(kvt(x).to(dev) for x in a[2:]), cu(sq), cu(sk), sq, scale, causal, out, lse,
+                         window=window)
+        ref, ref_lse = O.attention_varlen(*a, [0, sq], [0, sk], scale, causal, window=window)
+        attn_close(out, ref, 2e-2, 2e-3)
+        assert torch.allclose(lse.cpu(), ref_lse, atol=2e-2, rtol=1e-3)
