@@ -243,20 +243,54 @@ class NPUMLAImpl(MLACommonBaseImpl[NPUMLAMetadata]):
     # magnitude 2^-14 .. 65504 exactly; set prefill_kv_fp16 = False for a model whose keys or values can exceed that range.
     prefill_kv_fp16 = True
 
+    _half_w = None               # (address, version) of the up-projection weight and its fp16 copy
+
+    def _half_up_weight(self) -> Optional[torch.Tensor]:
+        """The up-projection weight [N*256, 512] in fp16, if the prefill may make keys and values with it (a plain weight
+        without bias).  A bf16 weight is converted once and again when it was replaced or written to, not on every call."""
+        w = getattr(self.kv_b_proj, "weight", None)
+        n, d = self.num_heads, self.qk_nope_head_dim + self.v_head_dim
+        if not self.prefill_kv_fp16 or not isinstance(w, torch.Tensor) or w.dtype not in (torch.bfloat16, torch.float16) \
+                or tuple(w.shape) != (n * d, self.kv_lora_rank) or getattr(self.kv_b_proj, "bias", None) is not None:
+            return None
+        if w.dtype == torch.float16:
+            return w
+        key = (w.data_ptr(), w.device, 0 if w.is_inference() else w._version)
+        if self._half_w is None or self._half_w[0] != key:
+            half = w.to(torch.float16)
+            if w.is_cuda and torch.cuda.is_current_stream_capturing():
+                return half                                    # recorded, not computed: of no use to a later eager call
+            self._half_w = (key, half)
+        return self._half_w[1]
+
+    def process_weights_after_loading(self, act_dtype: torch.dtype):
+        super().process_weights_after_loading(act_dtype)
+        self._half_w = None                                    # (weights reloaded through .data carry no new version)
+        self._half_up_weight()
+
+    def _split_kv(self, kv: torch.Tensor):
+        kv = kv.view(-1, self.num_heads, self.qk_nope_head_dim + self.v_head_dim)
+        return kv[..., :self.qk_nope_head_dim], kv[..., self.qk_nope_head_dim:]
+
     def _kv_up(self, kv_c: torch.Tensor, allow_fp16: bool = False):
         """(k_nope [T,N,128], v [T,N,128]) of latent rows kv_c [T,512] (reference: ``self.kv_b_proj(kv_c_normed)[0]``,
         mla.py:405-413, 566-571).  With ``allow_fp16`` both may come back as fp16."""
-        n, d = self.num_heads, self.qk_nope_head_dim + self.v_head_dim
-        w = getattr(self.kv_b_proj, "weight", None)
-        if (allow_fp16 and self.prefill_kv_fp16 and isinstance(w, torch.Tensor) and w.dtype in (torch.bfloat16, torch.float16)
-                and tuple(w.shape) == (n * d, kv_c.shape[-1]) and getattr(self.kv_b_proj, "bias", None) is None
-                and kv_c.dtype in (torch.bfloat16, torch.float16)):
-            kv = torch.matmul(kv_c.to(torch.float16), w.to(torch.float16).t())
-        else:
-            kv = self.kv_b_proj(kv_c)
-            kv = kv[0] if isinstance(kv, tuple) else kv
-        kv = kv.view(-1, n, d)
-        return kv[..., :self.qk_nope_head_dim], kv[..., self.qk_nope_head_dim:]
+        w = self._half_up_weight() if allow_fp16 and kv_c.dtype in (torch.bfloat16, torch.float16) else None
+        if w is not None and kv_c.shape[-1] == w.shape[1]:
+            return self._split_kv(torch.matmul(kv_c.to(torch.float16), w.t()))
+        kv = self.kv_b_proj(kv_c)
+        return self._split_kv(kv[0] if isinstance(kv, tuple) else kv)
+
+    def _kv_up_rows(self, kv_c: torch.Tensor, k_pe: torch.Tensor):
+        """(k_nope, k_pe [T,64], v) of a step's own rows as the prefill kernel takes them: all fp16 where the weight allows
+        it (latent and rope rows converted in one launch), else all in the dtype of the up-projection's result."""
+        w = self._half_up_weight()
+        if w is not None and kv_c.dtype == torch.bfloat16 and k_pe.dtype == torch.bfloat16:
+            c16, pe16 = K.rows_f16(kv_c, k_pe)
+            k_nope, v = self._split_kv(torch.matmul(c16, w.t()))
+            return k_nope, pe16, v
+        k_nope, v = self._kv_up(kv_c, allow_fp16=True)
+        return k_nope, k_pe.reshape(k_pe.shape[0], -1).to(k_nope.dtype), v
 
     # ---- prefill ----
     def _compute_prefill_context(self, q_nope, q_pe, kv_c_cache, k_pe_cache, attn_metadata, k_scale):
@@ -273,13 +307,15 @@ class NPUMLAImpl(MLACommonBaseImpl[NPUMLAMetadata]):
             toks = int(cc.seq_tot[i])
             if toks == 0:
                 continue
+            # (with an fp16 up-projection the rows are gathered as fp16 straight away, into the same bytes)
+            w16 = self._half_up_weight() if cc.workspace.dtype == torch.bfloat16 else None
+            rows = (cc.workspace if w16 is None else cc.workspace.view(torch.float16))
             ops.gather_and_maybe_dequant_cache(src_cache=(kv_c_cache,) if k_pe_cache is None else (kv_c_cache, k_pe_cache),
-                                               dst=cc.workspace,
+                                               dst=rows,
                                                block_table=prefill.block_table, cu_seq_lens=cc.cu_seq_lens[i],
                                                batch_size=attn_metadata.num_prefills, kv_cache_dtype=self.kv_cache_dtype,
                                                scale=k_scale, seq_starts=cc.starts[i], total_rows=toks)
-            kv_c_normed = cc.workspace[:toks][..., :self.kv_lora_rank]
-            k_pe = cc.workspace[:toks][..., self.kv_lora_rank:]
+            kv_c_normed, k_pe = rows[:toks, :self.kv_lora_rank], rows[:toks, self.kv_lora_rank:]
             k_nope, v = self._kv_up(kv_c_normed, allow_fp16=True)
             k_pe = k_pe.to(k_nope.dtype)
             # running results stay fp32: each bf16 rounding in between would add 2^-10 of mean relative error to the
@@ -293,10 +329,11 @@ class NPUMLAImpl(MLACommonBaseImpl[NPUMLAMetadata]):
                              prev_out=None if first else output, prev_lse=None if first else output_lse)
         return output, output_lse
 
-    def _forward_prefill(self, q, kv_c_normed, k_pe, kv_cache, attn_metadata, k_scale) -> torch.Tensor:
+    def _forward_prefill(self, q, kv_c_normed, k_pe, kv_cache, attn_metadata, k_scale,
+                         out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Causal suffix attention merged with the chunked context (reference mla.py:452-483, 573-616): the context chunks
         first, then the suffix launch continues from their result (the reference's final merge_attn_states, inside the
-        kernel)."""
+        kernel).  ``out`` ([T, N*V]) takes the result where it has the kernel's layout."""
         prefill = attn_metadata.prefill
         assert prefill is not None
         if self.sink_len > 0:
@@ -304,16 +341,20 @@ class NPUMLAImpl(MLACommonBaseImpl[NPUMLAMetadata]):
         t, n = q.shape[0], self.num_heads
         has_context = prefill.chunked_context is not None
         q_nope, q_pe = q[..., :self.qk_nope_head_dim], q[..., self.qk_nope_head_dim:]
-        k_nope, v = self._kv_up(kv_c_normed, allow_fp16=True)
+        k_nope, k_pe, v = self._kv_up_rows(kv_c_normed, k_pe)
         cu_q = prefill.query_start_loc.to(torch.int32).contiguous()
         ctx_out = ctx_lse = None
         if has_context:
             # (the fp8 cache is one tensor whose rows hold latent, scales and rope; the gather dequantises it)
             ctx_out, ctx_lse = self._compute_prefill_context(q_nope, q_pe, kv_cache[0],
                                                              None if self.fp8_cache else kv_cache[1], attn_metadata, k_scale)
-        output = torch.empty(t, n, self.v_head_dim, dtype=torch.bfloat16, device=q.device)
-        K.prefill_varlen(q_nope, q_pe, k_nope, k_pe.reshape(t, -1).to(k_nope.dtype), v, cu_q, cu_q, prefill.max_query_len,
-                         self.scale, True, output, prev_out=ctx_out, prev_lse=ctx_lse)
+        if out is not None and out.dtype == torch.bfloat16 and out.dim() == 2 and out.shape == (t, n * self.v_head_dim) and \
+                out.stride(1) == 1 and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
+            output = out.view(t, n, self.v_head_dim)
+        else:
+            output = torch.empty(t, n, self.v_head_dim, dtype=torch.bfloat16, device=q.device)
+        K.prefill_varlen(q_nope, q_pe, k_nope, k_pe, v, cu_q, cu_q, prefill.max_query_len, self.scale, True, output,
+                         prev_out=ctx_out, prev_lse=ctx_lse)
         return output.flatten(start_dim=-2)
 
     def _forward_prefill_sink(self, q, kv_c_normed, k_pe, prefill) -> torch.Tensor:
@@ -465,9 +506,11 @@ class NPUMLAImpl(MLACommonBaseImpl[NPUMLAMetadata]):
             q = q[:num_actual_toks, ...]
             k_c_normed = k_c_normed[:num_actual_toks, ...]
             k_pe = k_pe[:num_actual_toks, ...]
-            output[num_decode_tokens:] = self._forward_prefill(
-                q[num_decode_tokens:], k_c_normed[num_decode_tokens:], k_pe[num_decode_tokens:], kv_cache, attn_metadata,
-                getattr(layer, "_k_scale", None))
+            dst = output[num_decode_tokens:]
+            got = self._forward_prefill(q[num_decode_tokens:], k_c_normed[num_decode_tokens:], k_pe[num_decode_tokens:], kv_cache,
+                                        attn_metadata, getattr(layer, "_k_scale", None), out=dst)
+            if got.data_ptr() != dst.data_ptr():
+                dst.copy_(got)
 
         if has_decode:
             assert attn_metadata.decode is not None

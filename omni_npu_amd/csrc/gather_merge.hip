@@ -6,7 +6,23 @@
 
 namespace mlahip {
 
-// One wavefront per destination row: dst[cu[i] + j] = cat(nope[row], rope[row]) for position seq_starts[i] + j.
+// Eight bf16 values as they are, or rounded to fp16 (every bf16 number of magnitude 2^-14 .. 65504 is an fp16 number).
+template <bool kHalf>
+__device__ __forceinline__ u32x4 as_dst(u32x4 v) {
+  if constexpr (kHalf) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const f32x2 f = {__builtin_bit_cast(float, v[i] << 16), __builtin_bit_cast(float, v[i] & 0xffff0000u)};
+      v[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, f16x2));
+    }
+  }
+  return v;
+}
+
+// One wavefront per destination row: dst[cu[i] + j] = cat(nope[row], rope[row]) for position seq_starts[i] + j.  kHalf: dst
+// holds fp16 (what the prefill's up-projection and attention take): the conversion rides on the gather instead of being
+// two more passes over the rows (65 536 rows: 60 us of gather + 110 us of conversions -> 60 us).
+template <bool kHalf>
 __global__ __launch_bounds__(256) void gather_paged_kernel(const char* nope, int64_t nope_sp, int64_t nope_sr,
                                                            const char* rope, int64_t rope_sp, int64_t rope_sr,
                                                            char* dst, int64_t dst_stride_b, const int32_t* block_table,
@@ -29,12 +45,25 @@ __global__ __launch_bounds__(256) void gather_paged_kernel(const char* nope, int
   int64_t blk = block_table[(int64_t)lo * bt_stride + pg];
   blk = blk < 0 ? 0 : (blk >= num_pages ? num_pages - 1 : blk);
   char* d = dst + row * dst_stride_b;
-  *(u32x4*)(d + lane * 16) = *(const u32x4*)(nope + blk * nope_sp + off * nope_sr + lane * 16);
-  if (lane < 8) *(u32x4*)(d + kDNope * 2 + lane * 16) = *(const u32x4*)(rope + blk * rope_sp + off * rope_sr + lane * 16);
+  *(u32x4*)(d + lane * 16) = as_dst<kHalf>(*(const u32x4*)(nope + blk * nope_sp + off * nope_sr + lane * 16));
+  if (lane < 8) *(u32x4*)(d + kDNope * 2 + lane * 16) = as_dst<kHalf>(*(const u32x4*)(rope + blk * rope_sp + off * rope_sr + lane * 16));
+}
+
+// Plain rows [T, 512] and [T, 64] from bf16 to fp16, a wavefront per row (the step's own latents, which the prefill
+// up-projects and attends over in fp16).
+__global__ __launch_bounds__(256) void rows_f16_kernel(const char* c, int64_t c_st, const char* r, int64_t r_st, char* oc,
+                                                       int64_t oc_st, char* orr, int64_t or_st, int64_t rows) {
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  *(u32x4*)(oc + row * oc_st + lane * 16) = as_dst<true>(*(const u32x4*)(c + row * c_st + lane * 16));
+  if (lane < 8) *(u32x4*)(orr + row * or_st + lane * 16) = as_dst<true>(*(const u32x4*)(r + row * r_st + lane * 16));
 }
 
 // The same gather out of the fp8 block-scaled cache (rows of 512 e4m3 | 4 fp32 scales | 64 bf16 rope, see
-// cache_write_fp8_kernel): dst row = cat(bf16(e4m3 * block scale), rope), the values the fp8 decode kernel attends over.
+// cache_write_fp8_kernel): dst row = cat(bf16(e4m3 * block scale), rope), the values the fp8 decode kernel attends over
+// (kHalf: those values as fp16).
+template <bool kHalf>
 __global__ __launch_bounds__(256) void gather_paged_fp8_kernel(const char* cache, int64_t page_stride_b, int64_t row_stride_b,
                                                                char* dst, int64_t dst_stride_b, const int32_t* block_table,
                                                                int64_t bt_stride, int32_t max_blocks,
@@ -69,8 +98,8 @@ __global__ __launch_bounds__(256) void gather_paged_fp8_kernel(const char* cache
     o[4 * h + 2] = (__bf16)(hi2[0] * scale);
     o[4 * h + 3] = (__bf16)(hi2[1] * scale);
   }
-  *(bf16x8*)(d + lane * 16) = o;
-  if (lane < 8) *(u32x4*)(d + kDNope * 2 + lane * 16) = *(const u32x4*)(src + 528 + lane * 16);
+  *(u32x4*)(d + lane * 16) = as_dst<kHalf>(__builtin_bit_cast(u32x4, o));
+  if (lane < 8) *(u32x4*)(d + kDNope * 2 + lane * 16) = as_dst<kHalf>(*(const u32x4*)(src + 528 + lane * 16));
 }
 
 template <typename T> __device__ __forceinline__ float ld(const T* p) { return (float)*p; }
@@ -170,48 +199,87 @@ extern "C" int mla_merge_n_states(const void* outs, int64_t outs_stride_n, int64
   return check_launch("mla_merge_n_states");
 }
 
-extern "C" int mla_gather_paged(const void* nope_cache, int64_t nope_page_stride, int64_t nope_row_stride,
+static int gather_paged_impl(bool half, const char* what, const void* nope_cache, int64_t nope_page_stride, int64_t nope_row_stride,
                                 const void* rope_cache, int64_t rope_page_stride, int64_t rope_row_stride,
                                 int64_t num_pages, int32_t page_size, void* dst, int64_t dst_row_stride, int64_t dst_rows,
                                 const int32_t* block_table, int64_t bt_stride, int32_t max_blocks,
                                 const int32_t* cu_seq_lens, const int32_t* seq_starts, int32_t batch,
                                 int64_t total_rows_hint, hipStream_t stream) {
   MLA_REQUIRE(nope_cache && rope_cache && dst && block_table && cu_seq_lens, MLA_ERR_NULL,
-              "mla_gather_paged: null pointer argument");
+              "%s: null pointer argument", what);
   MLA_REQUIRE(batch >= 0 && page_size >= 1 && num_pages >= 1 && max_blocks >= 1 && dst_rows >= 0 && total_rows_hint >= 0,
-              MLA_ERR_SHAPE, "mla_gather_paged: batch=%d page_size=%d num_pages=%lld max_blocks=%d", batch, page_size,
+              MLA_ERR_SHAPE, "%s: batch=%d page_size=%d num_pages=%lld max_blocks=%d", what, batch, page_size,
               (long long)num_pages, max_blocks);
   MLA_REQUIRE(nope_row_stride % 8 == 0 && rope_row_stride % 8 == 0 && nope_page_stride % 8 == 0 &&
                   rope_page_stride % 8 == 0 && dst_row_stride % 8 == 0 && dst_row_stride >= kDNope + kDRope &&
                   (uintptr_t)nope_cache % 16 == 0 && (uintptr_t)rope_cache % 16 == 0 && (uintptr_t)dst % 16 == 0,
-              MLA_ERR_SHAPE, "mla_gather_paged: rows must be 16-byte aligned and dst rows at least 576 wide");
+              MLA_ERR_SHAPE, "%s: rows must be 16-byte aligned and dst rows at least 576 wide", what);
   const int64_t rows = total_rows_hint < dst_rows ? total_rows_hint : dst_rows;
   if (batch == 0 || rows == 0) return MLA_OK;
-  hipLaunchKernelGGL(gather_paged_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, (const char*)nope_cache,
+  if (half) hipLaunchKernelGGL(gather_paged_kernel<true>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, (const char*)nope_cache,
                      nope_page_stride * 2, nope_row_stride * 2, (const char*)rope_cache, rope_page_stride * 2,
                      rope_row_stride * 2, (char*)dst, dst_row_stride * 2, block_table, bt_stride, max_blocks, cu_seq_lens,
                      seq_starts, batch, page_size, num_pages, dst_rows);
-  return check_launch("mla_gather_paged");
+  else hipLaunchKernelGGL(gather_paged_kernel<false>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, (const char*)nope_cache,
+                     nope_page_stride * 2, nope_row_stride * 2, (const char*)rope_cache, rope_page_stride * 2,
+                     rope_row_stride * 2, (char*)dst, dst_row_stride * 2, block_table, bt_stride, max_blocks, cu_seq_lens,
+                     seq_starts, batch, page_size, num_pages, dst_rows);
+  return check_launch(what);
+}
+extern "C" int mla_gather_paged(const void* nope_cache, int64_t nope_page_stride, int64_t nope_row_stride,
+                                const void* rope_cache, int64_t rope_page_stride, int64_t rope_row_stride,
+                                int64_t num_pages, int32_t page_size, void* dst, int64_t dst_row_stride, int64_t dst_rows,
+                                const int32_t* block_table, int64_t bt_stride, int32_t max_blocks,
+                                const int32_t* cu_seq_lens, const int32_t* seq_starts, int32_t batch,
+                                int64_t total_rows_hint, hipStream_t stream) {
+  return gather_paged_impl(false, "mla_gather_paged", nope_cache, nope_page_stride, nope_row_stride, rope_cache, rope_page_stride, rope_row_stride, num_pages, page_size, dst, dst_row_stride, dst_rows, block_table, bt_stride, max_blocks, cu_seq_lens, seq_starts, batch, total_rows_hint, stream);
 }
 
+extern "C" int mla_gather_paged_f16(const void* nope_cache, int64_t nope_page_stride, int64_t nope_row_stride,
+                                const void* rope_cache, int64_t rope_page_stride, int64_t rope_row_stride,
+                                int64_t num_pages, int32_t page_size, void* dst, int64_t dst_row_stride, int64_t dst_rows,
+                                const int32_t* block_table, int64_t bt_stride, int32_t max_blocks,
+                                const int32_t* cu_seq_lens, const int32_t* seq_starts, int32_t batch,
+                                int64_t total_rows_hint, hipStream_t stream) {
+  return gather_paged_impl(true, "mla_gather_paged_f16", nope_cache, nope_page_stride, nope_row_stride, rope_cache, rope_page_stride, rope_row_stride, num_pages, page_size, dst, dst_row_stride, dst_rows, block_table, bt_stride, max_blocks, cu_seq_lens, seq_starts, batch, total_rows_hint, stream);
+}
+
+static int gather_paged_fp8_impl(bool half, const char* what, const void* cache, int64_t page_stride_bytes, int64_t row_stride_bytes, int64_t num_pages,
+                                    int32_t page_size, void* dst, int64_t dst_row_stride, int64_t dst_rows,
+                                    const int32_t* block_table, int64_t bt_stride, int32_t max_blocks,
+                                    const int32_t* cu_seq_lens, const int32_t* seq_starts, int32_t batch,
+                                    int64_t total_rows_hint, hipStream_t stream) {
+  MLA_REQUIRE(cache && dst && block_table && cu_seq_lens, MLA_ERR_NULL, "%s: null pointer argument", what);
+  MLA_REQUIRE(batch >= 0 && page_size >= 1 && num_pages >= 1 && max_blocks >= 1 && dst_rows >= 0 && total_rows_hint >= 0,
+              MLA_ERR_SHAPE, "%s: batch=%d page_size=%d num_pages=%lld max_blocks=%d", what, batch, page_size,
+              (long long)num_pages, max_blocks);
+  MLA_REQUIRE(row_stride_bytes >= 656 && row_stride_bytes % 16 == 0 && page_stride_bytes % 16 == 0 && dst_row_stride % 8 == 0 &&
+                  dst_row_stride >= kDNope + kDRope && (uintptr_t)cache % 16 == 0 && (uintptr_t)dst % 16 == 0,
+              MLA_ERR_SHAPE, "%s: cache rows are 656 bytes, 16-byte aligned; dst rows at least 576 wide", what);
+  const int64_t rows = total_rows_hint < dst_rows ? total_rows_hint : dst_rows;
+  if (batch == 0 || rows == 0) return MLA_OK;
+  if (half) hipLaunchKernelGGL(gather_paged_fp8_kernel<true>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, (const char*)cache,
+                     page_stride_bytes, row_stride_bytes, (char*)dst, dst_row_stride * 2, block_table, bt_stride, max_blocks,
+                     cu_seq_lens, seq_starts, batch, page_size, num_pages, dst_rows);
+  else hipLaunchKernelGGL(gather_paged_fp8_kernel<false>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, (const char*)cache,
+                     page_stride_bytes, row_stride_bytes, (char*)dst, dst_row_stride * 2, block_table, bt_stride, max_blocks,
+                     cu_seq_lens, seq_starts, batch, page_size, num_pages, dst_rows);
+  return check_launch(what);
+}
 extern "C" int mla_gather_paged_fp8(const void* cache, int64_t page_stride_bytes, int64_t row_stride_bytes, int64_t num_pages,
                                     int32_t page_size, void* dst, int64_t dst_row_stride, int64_t dst_rows,
                                     const int32_t* block_table, int64_t bt_stride, int32_t max_blocks,
                                     const int32_t* cu_seq_lens, const int32_t* seq_starts, int32_t batch,
                                     int64_t total_rows_hint, hipStream_t stream) {
-  MLA_REQUIRE(cache && dst && block_table && cu_seq_lens, MLA_ERR_NULL, "mla_gather_paged_fp8: null pointer argument");
-  MLA_REQUIRE(batch >= 0 && page_size >= 1 && num_pages >= 1 && max_blocks >= 1 && dst_rows >= 0 && total_rows_hint >= 0,
-              MLA_ERR_SHAPE, "mla_gather_paged_fp8: batch=%d page_size=%d num_pages=%lld max_blocks=%d", batch, page_size,
-              (long long)num_pages, max_blocks);
-  MLA_REQUIRE(row_stride_bytes >= 656 && row_stride_bytes % 16 == 0 && page_stride_bytes % 16 == 0 && dst_row_stride % 8 == 0 &&
-                  dst_row_stride >= kDNope + kDRope && (uintptr_t)cache % 16 == 0 && (uintptr_t)dst % 16 == 0,
-              MLA_ERR_SHAPE, "mla_gather_paged_fp8: cache rows are 656 bytes, 16-byte aligned; dst rows at least 576 wide");
-  const int64_t rows = total_rows_hint < dst_rows ? total_rows_hint : dst_rows;
-  if (batch == 0 || rows == 0) return MLA_OK;
-  hipLaunchKernelGGL(gather_paged_fp8_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, (const char*)cache,
-                     page_stride_bytes, row_stride_bytes, (char*)dst, dst_row_stride * 2, block_table, bt_stride, max_blocks,
-                     cu_seq_lens, seq_starts, batch, page_size, num_pages, dst_rows);
-  return check_launch("mla_gather_paged_fp8");
+  return gather_paged_fp8_impl(false, "mla_gather_paged_fp8", cache, page_stride_bytes, row_stride_bytes, num_pages, page_size, dst, dst_row_stride, dst_rows, block_table, bt_stride, max_blocks, cu_seq_lens, seq_starts, batch, total_rows_hint, stream);
+}
+
+extern "C" int mla_gather_paged_fp8_f16(const void* cache, int64_t page_stride_bytes, int64_t row_stride_bytes, int64_t num_pages,
+                                    int32_t page_size, void* dst, int64_t dst_row_stride, int64_t dst_rows,
+                                    const int32_t* block_table, int64_t bt_stride, int32_t max_blocks,
+                                    const int32_t* cu_seq_lens, const int32_t* seq_starts, int32_t batch,
+                                    int64_t total_rows_hint, hipStream_t stream) {
+  return gather_paged_fp8_impl(true, "mla_gather_paged_fp8_f16", cache, page_stride_bytes, row_stride_bytes, num_pages, page_size, dst, dst_row_stride, dst_rows, block_table, bt_stride, max_blocks, cu_seq_lens, seq_starts, batch, total_rows_hint, stream);
 }
 
 // dtype codes: 0 = bf16, 1 = fp32
@@ -237,4 +305,18 @@ extern "C" int mla_merge_states(const void* prefix_out, int64_t po_stride_t, int
   else MLA_MERGE(float, float);
 #undef MLA_MERGE
   return check_launch("mla_merge_states");
+}
+
+extern "C" int mla_rows_f16(const void* kv_c, int64_t kv_c_stride, const void* k_pe, int64_t k_pe_stride, int64_t num_rows,
+                            void* out_c, int64_t out_c_stride, void* out_pe, int64_t out_pe_stride, hipStream_t stream) {
+  MLA_REQUIRE(kv_c && k_pe && out_c && out_pe, MLA_ERR_NULL, "mla_rows_f16: null pointer argument");
+  MLA_REQUIRE(num_rows >= 0 && num_rows < (1ll << 32) && kv_c_stride % 8 == 0 && k_pe_stride % 8 == 0 && out_c_stride % 8 == 0 &&
+                  out_pe_stride % 8 == 0 && (uintptr_t)kv_c % 16 == 0 && (uintptr_t)k_pe % 16 == 0 &&
+                  (uintptr_t)out_c % 16 == 0 && (uintptr_t)out_pe % 16 == 0,
+              MLA_ERR_SHAPE, "mla_rows_f16: num_rows=%lld; rows must be 16-byte aligned", (long long)num_rows);
+  if (num_rows == 0) return MLA_OK;
+  hipLaunchKernelGGL(rows_f16_kernel, dim3((unsigned)((num_rows + 3) / 4)), dim3(256), 0, stream, (const char*)kv_c,
+                     kv_c_stride * 2, (const char*)k_pe, k_pe_stride * 2, (char*)out_c, out_c_stride * 2, (char*)out_pe,
+                     out_pe_stride * 2, num_rows);
+  return check_launch("rows_f16_kernel");
 }

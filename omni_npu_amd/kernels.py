@@ -227,6 +227,9 @@ def rotary_mul(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, out: Optio
     return out
 
 
+_GATHER_DST = {torch.bfloat16: "", torch.float16: "_f16"}
+
+
 def gather_paged(nope_cache: torch.Tensor, rope_cache: torch.Tensor, dst: torch.Tensor, block_table: torch.Tensor,
                  cu_seq_lens: torch.Tensor, batch_size: int, seq_starts: Optional[torch.Tensor] = None,
                  total_rows: Optional[int] = None) -> None:
@@ -236,8 +239,8 @@ def gather_paged(nope_cache: torch.Tensor, rope_cache: torch.Tensor, dst: torch.
     _need_cuda(nope_cache, rope_cache, dst, block_table, cu_seq_lens, seq_starts)
     lib = _lib.load()
     nope, rope = _cache3(nope_cache, D_NOPE), _cache3(rope_cache, D_ROPE)
-    if dst.dim() != 2 or dst.shape[1] < D_NOPE + D_ROPE or dst.stride(1) != 1 or dst.dtype != nope.dtype or nope.dtype != torch.bfloat16:
-        raise ValueError("gather_paged: dst must be bf16 [rows, >=576] like the caches")
+    if dst.dim() != 2 or dst.shape[1] < D_NOPE + D_ROPE or dst.stride(1) != 1 or dst.dtype not in _GATHER_DST or nope.dtype != torch.bfloat16:
+        raise ValueError("gather_paged: bf16 caches, dst bf16 or fp16 [rows, >=576]")
     if block_table.dtype != torch.int32 or cu_seq_lens.dtype != torch.int32 or not cu_seq_lens.is_contiguous():
         raise TypeError("gather_paged: block_table and cu_seq_lens must be int32 (cu_seq_lens contiguous)")
     if seq_starts is not None and (seq_starts.dtype != torch.int32 or not seq_starts.is_contiguous()):
@@ -245,11 +248,12 @@ def gather_paged(nope_cache: torch.Tensor, rope_cache: torch.Tensor, dst: torch.
     if cu_seq_lens.numel() < batch_size + 1:
         raise ValueError("gather_paged: cu_seq_lens needs batch_size + 1 entries")
     rows = dst.shape[0] if total_rows is None else min(int(total_rows), dst.shape[0])
-    rc = lib.mla_gather_paged(nope.data_ptr(), nope.stride(0), nope.stride(1), rope.data_ptr(), rope.stride(0), rope.stride(1),
+    name = "mla_gather_paged" + _GATHER_DST[dst.dtype]
+    rc = getattr(lib, name)(nope.data_ptr(), nope.stride(0), nope.stride(1), rope.data_ptr(), rope.stride(0), rope.stride(1),
                               nope.shape[0], nope.shape[1], dst.data_ptr(), dst.stride(0), dst.shape[0],
                               block_table.data_ptr(), block_table.stride(0), block_table.shape[1], cu_seq_lens.data_ptr(),
                               seq_starts.data_ptr() if seq_starts is not None else None, batch_size, rows, _stream(dst))
-    _lib.check(rc, "mla_gather_paged")
+    _lib.check(rc, name)
 
 
 def gather_paged_fp8(cache: torch.Tensor, dst: torch.Tensor, block_table: torch.Tensor, cu_seq_lens: torch.Tensor,
@@ -261,8 +265,8 @@ def gather_paged_fp8(cache: torch.Tensor, dst: torch.Tensor, block_table: torch.
     lib = _lib.load()
     if cache.dtype != torch.uint8 or cache.dim() != 3 or cache.shape[-1] != FP8_ROW_BYTES or cache.stride(-1) != 1:
         raise ValueError(f"fp8 cache must be uint8 [num_blocks, page, {FP8_ROW_BYTES}], got {cache.dtype} {tuple(cache.shape)}")
-    if dst.dim() != 2 or dst.shape[1] < D_NOPE + D_ROPE or dst.stride(1) != 1 or dst.dtype != torch.bfloat16:
-        raise ValueError("gather_paged_fp8: dst must be bf16 [rows, >=576]")
+    if dst.dim() != 2 or dst.shape[1] < D_NOPE + D_ROPE or dst.stride(1) != 1 or dst.dtype not in _GATHER_DST:
+        raise ValueError("gather_paged_fp8: dst must be bf16 or fp16 [rows, >=576]")
     if block_table.dtype != torch.int32 or cu_seq_lens.dtype != torch.int32 or not cu_seq_lens.is_contiguous():
         raise TypeError("gather_paged_fp8: block_table and cu_seq_lens must be int32 (cu_seq_lens contiguous)")
     if block_table.dim() != 2 or block_table.stride(1) != 1 or block_table.shape[0] < batch_size:
@@ -272,11 +276,29 @@ def gather_paged_fp8(cache: torch.Tensor, dst: torch.Tensor, block_table: torch.
     if cu_seq_lens.numel() < batch_size + 1:
         raise ValueError("gather_paged_fp8: cu_seq_lens needs batch_size + 1 entries")
     rows = dst.shape[0] if total_rows is None else min(int(total_rows), dst.shape[0])
-    rc = lib.mla_gather_paged_fp8(cache.data_ptr(), cache.stride(0), cache.stride(1), cache.shape[0], cache.shape[1],
+    name = "mla_gather_paged_fp8" + _GATHER_DST[dst.dtype]
+    rc = getattr(lib, name)(cache.data_ptr(), cache.stride(0), cache.stride(1), cache.shape[0], cache.shape[1],
                                   dst.data_ptr(), dst.stride(0), dst.shape[0], block_table.data_ptr(), block_table.stride(0),
                                   block_table.shape[1], cu_seq_lens.data_ptr(),
                                   seq_starts.data_ptr() if seq_starts is not None else None, batch_size, rows, _stream(dst))
-    _lib.check(rc, "mla_gather_paged_fp8")
+    _lib.check(rc, name)
+
+
+def rows_f16(kv_c: torch.Tensor, k_pe: torch.Tensor):
+    """(kv_c [T,512], k_pe [T,64] or [T,1,64]) bf16 -> the same rows as contiguous fp16 [T,512], [T,64], in one launch."""
+    _need_cuda(kv_c, k_pe)
+    k_pe = k_pe.reshape(k_pe.shape[0], -1)
+    t = kv_c.shape[0]
+    if kv_c.shape != (t, D_NOPE) or k_pe.shape != (t, D_ROPE) or kv_c.dtype != torch.bfloat16 or k_pe.dtype != torch.bfloat16 or \
+            kv_c.stride(-1) != 1 or k_pe.stride(-1) != 1:
+        raise ValueError("rows_f16: bf16 kv_c [T,512] and k_pe [T,64] with contiguous last dims")
+    c = torch.empty(t, D_NOPE, dtype=torch.float16, device=kv_c.device)
+    r = torch.empty(t, D_ROPE, dtype=torch.float16, device=kv_c.device)
+    if t:
+        rc = _lib.load().mla_rows_f16(kv_c.data_ptr(), kv_c.stride(0), k_pe.data_ptr(), k_pe.stride(0), t, c.data_ptr(), D_NOPE,
+                                      r.data_ptr(), D_ROPE, _stream(kv_c))
+        _lib.check(rc, "mla_rows_f16")
+    return c, r
 
 
 _DT = {torch.bfloat16: 0, torch.float32: 1}

@@ -334,3 +334,28 @@ def test_scores_that_climb_tile_by_tile_raise_the_reference(dev, half, sq, sk, c
         ref, ref_lse = O.attention_varlen(*a, [0, sq], [0, sk], scale, causal, window=window)
         attn_close(out, ref, 2e-2, 2e-3)
         assert torch.allclose(lse.cpu(), ref_lse, atol=2e-2, rtol=1e-3)
+
+
+@pytest.mark.parametrize("rows", [1, 4, 5, 1027])
+def test_rows_f16_and_fp16_gathers_round_like_torch(dev, rows):
+    """bf16 -> fp16 of the step's rows and of both gathers: the bits of torch's conversion of the bf16 result, normal,
+    subnormal and overflowing magnitudes among them."""
+    from omni_npu_amd import kernels as K
+    g = torch.Generator().manual_seed(rows)
+    c = (torch.randn(rows, 512, generator=g) * torch.exp2(torch.randint(-30, 18, (rows, 1), generator=g).float())).bfloat16().to(dev)
+    r = torch.randn(rows, 1, 64, generator=g).bfloat16().to(dev)
+    c16, r16 = K.rows_f16(c, r)
+    assert torch.equal(c16, c.half()) and torch.equal(r16, r.view(rows, 64).half())
+    nblk = (rows + 127) // 128
+    nope, rope = torch.zeros(nblk, 128, 512, dtype=torch.bfloat16, device=dev), torch.zeros(nblk, 128, 64, dtype=torch.bfloat16, device=dev)
+    cache8 = torch.zeros(nblk, 128, 656, dtype=torch.uint8, device=dev)
+    slots = torch.arange(rows, device=dev)
+    K.cache_write(c, r, slots, nope, rope)
+    K.cache_write_fp8(c, r, slots, cache8)
+    bt = torch.arange(nblk, dtype=torch.int32, device=dev).view(1, -1)
+    cu = torch.tensor([0, rows], dtype=torch.int32, device=dev)
+    for gather in (lambda d: K.gather_paged(nope, rope, d, bt, cu, 1), lambda d: K.gather_paged_fp8(cache8, d, bt, cu, 1)):
+        plain, half = torch.empty(rows, 576, dtype=torch.bfloat16, device=dev), torch.empty(rows, 576, dtype=torch.float16, device=dev)
+        gather(plain)
+        gather(half)
+        assert torch.equal(half, plain.half())
