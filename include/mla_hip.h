@@ -309,6 +309,18 @@ int mla_prefill_varlen_continue(const void* q_nope, int64_t qn_stride_t, int64_t
                                 float* lse_out, const float* prev_out, int64_t prev_stride_t, int64_t prev_stride_h,
                                 const float* prev_lse, mlahip_stream_t stream);
 
+/* mla_prefill_varlen over a selection of keys: bit j of pick[t] (32-bit words, rows pick_stride words apart, pick_words of
+ * them valid, whole 64-key tiles) says whether query token t attends over key j of its sequence, within what causal
+ * allows.  out_dtype must carry MLA_PREFILL_KV_F16.  The sparse attention of attention/backends/dsa.py:259-291 over the
+ * up-projected keys and values of a prompt. */
+int mla_prefill_varlen_pick(const void* q_nope, int64_t qn_stride_t, int64_t qn_stride_h, const void* q_pe, int64_t qp_stride_t,
+                            int64_t qp_stride_h, const void* k_nope, int64_t kn_stride_t, int64_t kn_stride_h, const void* k_pe,
+                            int64_t kp_stride_t, const void* v, int64_t v_stride_t, int64_t v_stride_h, const int32_t* cu_q,
+                            const int32_t* cu_k, int32_t batch, int32_t num_heads, int32_t max_q_len, int32_t causal,
+                            float scale, const uint32_t* pick, int64_t pick_stride, int32_t pick_words, void* out,
+                            int64_t out_stride_t, int64_t out_stride_h, int32_t out_dtype, float* lse_out,
+                            mlahip_stream_t stream);
+
 /* ---- DSA lightning indexer --------------------------------------------------------------------
  * Replaces torch.ops.custom.npu_lightning_indexer, v1/layers/attention/npu_dsa.py:92-103 and
  * vllm_patches/patches/models/deepseek/patch_dsv32_indexer.py:133-146, in two steps:
@@ -324,6 +336,17 @@ int dsa_indexer_scores_fp8(const void* q8, int64_t q_stride_t, int64_t q_stride_
                            int64_t bt_stride, int32_t max_blocks, const int32_t* seq_lens,
                            const int32_t* query_start_loc, int32_t batch, int32_t max_q_len, int32_t num_heads,
                            int32_t max_seq_len, float* logits, int64_t logits_stride, mlahip_stream_t stream);
+
+/* dsa_indexer_scores_fp8 without the logits of query tokens that see at most skip_up_to keys: a top-k of that many takes all
+ * of their keys whatever they score.  Those rows of logits may hold anything afterwards. */
+int dsa_indexer_scores_fp8_above(const void* q8, int64_t q_stride_t, int64_t q_stride_h, const float* weights,
+                           int64_t w_stride_t, const float* q_scale /* may be NULL */, int64_t qs_stride_t,
+                           const void* k8_cache, int64_t k_page_stride, int64_t k_row_stride, const float* k_scale_cache,
+                           int64_t ks_page_stride, int64_t num_pages, int32_t page_size, const int32_t* block_table,
+                           int64_t bt_stride, int32_t max_blocks, const int32_t* seq_lens,
+                           const int32_t* query_start_loc, int32_t batch, int32_t max_q_len, int32_t num_heads,
+                           int32_t max_seq_len, float* logits, int64_t logits_stride, int32_t skip_up_to,
+                                 mlahip_stream_t stream);
 
 /* Per-row e4m3 quantisation of 128-wide bf16 rows (scale = amax/448 per row), optionally scattered through a slot
  * mapping into the paged fp8 indexer-K cache and its scale cache: the indexer-K scatter of patch_dsv32_indexer.py:116-121
@@ -357,6 +380,12 @@ int dsa_topk_rows(const float* logits, int64_t logits_stride, const int32_t* seq
                   const int32_t* block_table, int64_t bt_stride, int32_t max_blocks, int32_t page_size, int64_t num_pages,
                   int32_t* rows, int64_t rows_stride, int32_t* counts, void* workspace /* may be NULL */,
                   size_t workspace_bytes, mlahip_stream_t stream);
+
+/* dsa_topk with the picks also as bits: bit (i & 7) of byte i >> 3 of mask[t] (rows mask_stride bytes apart) says whether
+ * position i is picked, for the positions token t sees; bits behind them are undefined.  16-byte aligned logits rows. */
+int dsa_topk_mask(const float* logits, int64_t logits_stride, const int32_t* seq_lens, const int32_t* query_start_loc,
+                  int32_t batch, int32_t max_q_len, int32_t k, int32_t* out_indices, int64_t out_stride, void* mask,
+                  int64_t mask_stride, void* workspace, size_t workspace_bytes, mlahip_stream_t stream);
 
 /* ---- sparse MLA over the selected keys ----------------------------------------------------------
  * Replaces torch.ops.custom.npu_sparse_flash_attention, attention/backends/dsa.py:259-291 (sparse_block_size 1,

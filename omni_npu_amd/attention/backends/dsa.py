@@ -17,12 +17,19 @@ from typing import ClassVar, Optional, Tuple
 import torch
 
 from ... import kernels as K
-from .mla import _caller_wrote_cache, _persistent_int32
+from .mla import HalfUpProjection, _caller_wrote_cache, _persistent_int32
 from ..._vllm_compat import (PAD_SLOT_ID, AttentionCGSupport, AttentionType, MLACommonBackend, MLACommonBaseImpl,
                              MLACommonDecodeMetadata, MLACommonMetadata, MLACommonMetadataBuilder,
                              MLACommonPrefillMetadata, QueryLenSupport, get_current_vllm_config)
 
 INDEX_HEAD_DIM = 128
+# Scores and values of a (token, key) pair and head cost 640 flops on up-projected keys and 2176 on latents (the up-projection
+# costs what absorbing the queries and up-projecting the outputs does), and the latents have to be gathered per token: leaving
+# out most of the pairs that were scored still pays up to this many visible pairs per picked one.  Measured with 128 heads
+# and k = 2048, us for one prompt, masked / gathered: 2k tokens 397 / 1109, 8k (2.2 pairs per pick) 4432 / 6595, 12k (3.2)
+# 9274 / 10 555, 16k (4.2) 15 407 / 14 897.  With fewer heads the scores get cheaper and the gather does not (16 heads, 16k
+# tokens: 4689 / 14 254), so the limit grows as the heads shrink.
+MASKED_PAIRS_PER_PICK = 3.5
 
 
 def indexer_cache_views(index_cache: torch.Tensor):
@@ -70,6 +77,17 @@ class NPUDSABackend(MLACommonBackend):
 class NPUDSAPrefillMetadata(MLACommonPrefillMetadata):
     query_cumlens: torch.Tensor = None
     seq_lens: torch.Tensor = None
+    # prompt lengths on the host, where every prefill request starts at its first token (else None)
+    prompt_lens: list = None
+
+    def over_up_projected(self, k: int, pairs_per_pick: float) -> bool:
+        """Whether the prefill attends over up-projected keys and values with a mask of the k picks instead of gathering
+        the picked latents: while there are at most ``pairs_per_pick`` visible (token, key) pairs per picked one."""
+        if self.prompt_lens is None or not pairs_per_pick:
+            return False
+        seen = sum(n * (n + 1) // 2 for n in self.prompt_lens)
+        picked = sum(n * (n + 1) // 2 if n <= k else k * (k + 1) // 2 + (n - k) * k for n in self.prompt_lens)
+        return seen <= pairs_per_pick * picked
 
 
 @dataclass
@@ -128,6 +146,10 @@ class NPUDSAMetadataBuilder(MLACommonMetadataBuilder[NPUDSAMetadata]):
             # sparse attention over the cache needs each prefill request's total cached length
             nd = metadata.num_decodes
             metadata.prefill.kv_lens = common_attn_metadata.seq_lens[nd:].to(torch.int32)
+            done = getattr(common_attn_metadata, "num_computed_tokens_cpu", None)
+            if done is not None and not bool((done[nd:nd + metadata.num_prefills] > 0).any()):
+                starts = common_attn_metadata.query_start_loc_cpu[nd:nd + metadata.num_prefills + 1]
+                metadata.prefill.prompt_lens = (starts[1:] - starts[:-1]).tolist()
         if metadata.prefill is not None and metadata.prefill.chunked_context is not None:
             raise RuntimeError("Chunked prefill is not enabled yet.")
         return metadata
@@ -154,6 +176,11 @@ class LightningIndexer:
         self.rows_buffer = torch.zeros((max_tokens, topk_tokens), dtype=torch.int32, device=device)
         self.counts_buffer = torch.zeros((max_tokens,), dtype=torch.int32, device=device)
         self._rows_meta = None       # the metadata object the row buffers were filled for
+        # Up to how many visible pairs per pick the attention behind this selection wants a step's prompts as bits over their
+        # own keys instead of cache rows (NPUDSAImpl says so once its weights are loaded); the bits, and the metadata object
+        # they were made for
+        self.masked_pairs_per_pick = 0.0
+        self._mask, self._mask_meta = None, None
         self._logits = None
         self._logits_kept = []       # outgrown score buffers: a captured graph may still hold their address, never freed
 
@@ -171,6 +198,7 @@ class LightningIndexer:
         w = weights.float().contiguous()
         out = self.topk_indices_buffer[:t]
         off = 0
+        self._rows_meta = self._mask_meta = self._mask = None
         for meta, nreq in ((attn_metadata.decode, attn_metadata.num_decodes), (attn_metadata.prefill, attn_metadata.num_prefills)):
             if meta is None or nreq == 0:
                 continue
@@ -180,7 +208,11 @@ class LightningIndexer:
                 ntok = t - off
                 lens, q_len = meta.kv_lens, meta.max_query_len
                 qsl = meta.query_start_loc.to(torch.int32).contiguous()
+            masked = (self.masked_pairs_per_pick > 0 and meta is attn_metadata.prefill
+                      and meta.over_up_projected(self.topk_tokens, self.masked_pairs_per_pick))
             max_len = meta.block_table.shape[1] * k8.shape[1]
+            if masked:                                              # (the longest prompt, not the longest the server takes)
+                max_len = min(max_len, (q_len + 63) // 64 * 64)
             stride = K.indexer_logits_stride(max_len)
             if self._logits is None or self._logits.shape[0] < ntok or self._logits.shape[1] < stride:
                 if self._logits is not None:
@@ -191,13 +223,25 @@ class LightningIndexer:
                 self._logits = torch.empty(ntok_a, stride_a, dtype=torch.float32, device=q.device)
             lg = self._logits[:ntok, :stride]
             sl = slice(off, off + ntok)
-            K.indexer_scores(q8[sl], w[sl], k8, ks, meta.block_table, lens, lg, q_len=q_len, q_scale=qs[sl],
-                             query_start_loc=qsl, max_seq_len=max_len)
-            K.topk(lg, lens, self.topk_tokens, out[sl], q_len=q_len, query_start_loc=qsl, block_table=meta.block_table,
-                   page_size=k8.shape[1], num_pages=k8.shape[0], rows=self.rows_buffer[sl], counts=self.counts_buffer[sl])
+            if not masked or q_len > self.topk_tokens:              # (else every token takes all the keys it sees)
+                K.indexer_scores(q8[sl], w[sl], k8, ks, meta.block_table, lens, lg, q_len=q_len, q_scale=qs[sl],
+                                 query_start_loc=qsl, max_seq_len=max_len, skip_up_to=self.topk_tokens)
+            if masked:
+                self._mask = torch.empty(ntok, stride // 64 * 2 + 2, dtype=torch.int32, device=q.device)
+                self._mask_meta = attn_metadata
+                K.topk(lg, lens, self.topk_tokens, out[sl], q_len=q_len, query_start_loc=qsl, mask=self._mask)
+            else:
+                K.topk(lg, lens, self.topk_tokens, out[sl], q_len=q_len, query_start_loc=qsl, block_table=meta.block_table,
+                       page_size=k8.shape[1], num_pages=k8.shape[0], rows=self.rows_buffer[sl],
+                       counts=self.counts_buffer[sl])
+                self._rows_meta = attn_metadata
             off += ntok
-        self._rows_meta = attn_metadata
         return out.view(t, 1, self.topk_tokens)
+
+    def mask_for(self, attn_metadata):
+        """The picks of the step's prompt tokens as bits [T, W] (kernels.topk's mask) if the last selection made them for this
+        very metadata object, else None.  The row buffers hold the step's decode tokens only then."""
+        return self._mask if attn_metadata is not None and self._mask_meta is attn_metadata else None
 
     def rows_for(self, attn_metadata):
         """(cache rows [max_tokens, k], counts [max_tokens]) of the picks if the last selection ran for this very metadata
@@ -207,7 +251,7 @@ class LightningIndexer:
         return None
 
 
-class NPUDSAImpl(MLACommonBaseImpl[NPUDSAMetadata]):
+class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
     can_return_lse_for_decode: bool = False
     cache_written_for = None     # see NPUMLAImpl.cache_written_for
 
@@ -233,6 +277,16 @@ class NPUDSAImpl(MLACommonBaseImpl[NPUDSAMetadata]):
         if kv_cache_dtype in ("fp8", "fp8_e4m3"):
             raise NotImplementedError("NPUDSAImpl writes the bf16 cache layout (latent, rope, indexer keys) only: "
                                       "an fp8 KV cache is not supported for DSA models")
+
+    def process_weights_after_loading(self, act_dtype: torch.dtype):
+        super().process_weights_after_loading(act_dtype)
+        self.offer_masked_prompts(getattr(self.indexer, "select", self.indexer))
+
+    def offer_masked_prompts(self, select) -> None:
+        """Tells the selection whether, and for how many pairs per pick, this layer attends over masked prompts."""
+        if hasattr(select, "masked_pairs_per_pick"):
+            select.masked_pairs_per_pick = (MASKED_PAIRS_PER_PICK * max(1.0, 128 / self.num_heads)
+                                            if self._plain_up_weight() is not None else 0.0)
 
     def _v_up_proj(self, x: torch.Tensor, out: torch.Tensor):
         """[T,N,512] token-major -> out [T, N*V]  (reference dsa.py:233-240)."""
@@ -274,6 +328,21 @@ class NPUDSAImpl(MLACommonBaseImpl[NPUDSAMetadata]):
         out = torch.empty(bs, self.num_heads, self.kv_lora_rank, dtype=q_nope.dtype, device=q_nope.device)
         K.sparse_decode(q_nope, q_pe, nope, rope, rows, counts, self.scale, out, counts_bounded=True)
         return out
+
+    def _forward_prompts(self, q, kv_c_normed, k_pe, prefill, pick, out: torch.Tensor) -> bool:
+        """Sparse attention of whole prompts over their own up-projected keys and values, with the picks as a mask
+        (NPUDSAPrefillMetadata.over_up_projected); False, and nothing done, where the shapes do not allow it."""
+        t, n = q.shape[0], self.num_heads
+        if pick is None or self._half_up_weight() is None or self.qk_nope_head_dim != 128 or self.v_head_dim != 128 or \
+                q.dtype != torch.bfloat16 or q.stride(-1) != 1 or kv_c_normed.dtype != torch.bfloat16 or \
+                k_pe.dtype != torch.bfloat16 or kv_c_normed.stride(-1) != 1 or out.dtype != torch.bfloat16 or \
+                tuple(out.shape) != (t, n * 128) or out.stride(1) != 1 or out.stride(0) % 8 or out.data_ptr() % 16:
+            return False
+        k_nope, pe, v = self._kv_up_rows(kv_c_normed, k_pe)
+        cu = prefill.query_start_loc.to(torch.int32).contiguous()
+        K.prefill_varlen(q[..., :128], q[..., 128:], k_nope, pe, v, cu, cu, prefill.max_query_len, self.scale, True,
+                         out.view(t, n, 128), pick=pick)
+        return True
 
     def forward(self, layer, q: torch.Tensor, k_c_normed: torch.Tensor, k_pe: torch.Tensor,
                 kv_cache: Tuple[torch.Tensor, torch.Tensor, torch.Tensor], attn_metadata: NPUDSAMetadata,
@@ -323,14 +392,18 @@ class NPUDSAImpl(MLACommonBaseImpl[NPUDSAMetadata]):
         if has_prefill:
             p = attn_metadata.prefill
             assert p is not None
-            q_nope, q_pe = self._absorb_prolog(q[ndt:])
-            fused = output[ndt:] if self._fusable_w_uv(output[ndt:]) else None
-            attn_out = self._apply_sparse_attention(q_nope, q_pe, kv_cache, p, p.kv_lens, p.max_query_len,
-                                                    p.query_start_loc.to(torch.int32).contiguous(),
-                                                    topk[ndt:num_actual_toks], proj_out=fused,
-                                                    rows_counts=part(ndt, num_actual_toks))
-            if fused is None:
-                self._v_up_proj(attn_out, out=output[ndt:])
+            mask_for = getattr(self.indexer, "mask_for", None)
+            pick = mask_for(attn_metadata) if mask_for is not None else None
+            if not self._forward_prompts(q[ndt:], k_c_normed[ndt:num_actual_toks], k_pe[ndt:num_actual_toks], p, pick,
+                                         output[ndt:]):
+                q_nope, q_pe = self._absorb_prolog(q[ndt:])
+                fused = output[ndt:] if self._fusable_w_uv(output[ndt:]) else None
+                attn_out = self._apply_sparse_attention(q_nope, q_pe, kv_cache, p, p.kv_lens, p.max_query_len,
+                                                        p.query_start_loc.to(torch.int32).contiguous(),
+                                                        topk[ndt:num_actual_toks], proj_out=fused,
+                                                        rows_counts=None if pick is not None else part(ndt, num_actual_toks))
+                if fused is None:
+                    self._v_up_proj(attn_out, out=output[ndt:])
         if has_decode:
             d = attn_metadata.decode
             assert d is not None

@@ -188,7 +188,73 @@ def _caller_wrote_cache(impl, attn_metadata, num_tokens: int) -> bool:
     return meta is attn_metadata and rows >= num_tokens
 
 
-class NPUMLAImpl(MLACommonBaseImpl[NPUMLAMetadata]):
+class HalfUpProjection:
+    """Keys and values of prefill tokens, made in fp16 where the model's up-projection is a plain weight."""
+
+    # The prefill kernel multiplies the probabilities with fp16 values (the bf16 bar of the output leaves no room for bf16
+    # probabilities), so it converts every value tile it is given in bf16.  Where the up-projection is a plain weight the
+    # keys and values are made in fp16 in the first place - the same GEMM on fp16 copies of its operands, no extra pass -
+    # and the kernel converts nothing (configs of 4 x 2048 over 16k: 13.2 -> 12.2 ms).  fp16 holds every bf16 number of
+    # magnitude 2^-14 .. 65504 exactly; set prefill_kv_fp16 = False for a model whose keys or values can exceed that range.
+    prefill_kv_fp16 = True
+
+    _half_w = None               # (address, version) of the up-projection weight and its fp16 copy
+
+    def _plain_up_weight(self) -> Optional[torch.Tensor]:
+        """The up-projection weight [N*256, 512] if the prefill may make fp16 keys and values with it: plain, without bias."""
+        w = getattr(self.kv_b_proj, "weight", None)
+        n, d = self.num_heads, self.qk_nope_head_dim + self.v_head_dim
+        if not self.prefill_kv_fp16 or not isinstance(w, torch.Tensor) or w.dtype not in (torch.bfloat16, torch.float16) \
+                or tuple(w.shape) != (n * d, self.kv_lora_rank) or getattr(self.kv_b_proj, "bias", None) is not None:
+            return None
+        return w
+
+    def _half_up_weight(self) -> Optional[torch.Tensor]:
+        """That weight in fp16, or None.  A bf16 weight is converted by the first prefill and again when it was replaced or
+        written to, not on every call."""
+        w = self._plain_up_weight()
+        if w is None:
+            return None
+        if w.dtype == torch.float16:
+            return w
+        key = (w.data_ptr(), w.device, 0 if w.is_inference() else w._version)
+        if self._half_w is None or self._half_w[0] != key:
+            half = w.to(torch.float16)
+            if w.is_cuda and torch.cuda.is_current_stream_capturing():
+                return half                                    # recorded, not computed: of no use to a later eager call
+            self._half_w = (key, half)
+        return self._half_w[1]
+
+    def process_weights_after_loading(self, act_dtype: torch.dtype):
+        super().process_weights_after_loading(act_dtype)
+        self._half_w = None                                    # (weights reloaded through .data carry no new version)
+
+    def _split_kv(self, kv: torch.Tensor):
+        kv = kv.view(-1, self.num_heads, self.qk_nope_head_dim + self.v_head_dim)
+        return kv[..., :self.qk_nope_head_dim], kv[..., self.qk_nope_head_dim:]
+
+    def _kv_up(self, kv_c: torch.Tensor, allow_fp16: bool = False):
+        """(k_nope [T,N,128], v [T,N,128]) of latent rows kv_c [T,512] (reference: ``self.kv_b_proj(kv_c_normed)[0]``,
+        mla.py:405-413, 566-571).  With ``allow_fp16`` both may come back as fp16."""
+        w = self._half_up_weight() if allow_fp16 and kv_c.dtype in (torch.bfloat16, torch.float16) else None
+        if w is not None and kv_c.shape[-1] == w.shape[1]:
+            return self._split_kv(torch.matmul(kv_c.to(torch.float16), w.t()))
+        kv = self.kv_b_proj(kv_c)
+        return self._split_kv(kv[0] if isinstance(kv, tuple) else kv)
+
+    def _kv_up_rows(self, kv_c: torch.Tensor, k_pe: torch.Tensor):
+        """(k_nope, k_pe [T,64], v) of a step's own rows as the prefill kernel takes them: all fp16 where the weight allows
+        it (latent and rope rows converted in one launch), else all in the dtype of the up-projection's result."""
+        w = self._half_up_weight()
+        if w is not None and kv_c.dtype == torch.bfloat16 and k_pe.dtype == torch.bfloat16:
+            c16, pe16 = K.rows_f16(kv_c, k_pe)
+            k_nope, v = self._split_kv(torch.matmul(c16, w.t()))
+            return k_nope, pe16, v
+        k_nope, v = self._kv_up(kv_c, allow_fp16=True)
+        return k_nope, k_pe.reshape(k_pe.shape[0], -1).to(k_nope.dtype), v
+
+
+class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
     can_return_lse_for_decode: bool = True
     # Set by a caller whose fused norm + rope launch has already written the step's rows into the cache: the metadata
     # object of that step.  forward() then skips its own write once and clears the mark.
@@ -235,62 +301,6 @@ class NPUMLAImpl(MLACommonBaseImpl[NPUMLAMetadata]):
         x = x.view(self.num_heads, -1, self.kv_lora_rank)
         out2 = torch.bmm(x, self.W_UV)
         return out2.transpose(0, 1).contiguous().view(-1, self.num_heads * self.v_head_dim)
-
-    # The prefill kernel multiplies the probabilities with fp16 values (the bf16 bar of the output leaves no room for bf16
-    # probabilities), so it converts every value tile it is given in bf16.  Where the up-projection is a plain weight the
-    # keys and values are made in fp16 in the first place - the same GEMM on fp16 copies of its operands, no extra pass -
-    # and the kernel converts nothing (configs of 4 x 2048 over 16k: 13.2 -> 12.2 ms).  fp16 holds every bf16 number of
-    # magnitude 2^-14 .. 65504 exactly; set prefill_kv_fp16 = False for a model whose keys or values can exceed that range.
-    prefill_kv_fp16 = True
-
-    _half_w = None               # (address, version) of the up-projection weight and its fp16 copy
-
-    def _half_up_weight(self) -> Optional[torch.Tensor]:
-        """The up-projection weight [N*256, 512] in fp16, if the prefill may make keys and values with it (a plain weight
-        without bias).  A bf16 weight is converted once and again when it was replaced or written to, not on every call."""
-        w = getattr(self.kv_b_proj, "weight", None)
-        n, d = self.num_heads, self.qk_nope_head_dim + self.v_head_dim
-        if not self.prefill_kv_fp16 or not isinstance(w, torch.Tensor) or w.dtype not in (torch.bfloat16, torch.float16) \
-                or tuple(w.shape) != (n * d, self.kv_lora_rank) or getattr(self.kv_b_proj, "bias", None) is not None:
-            return None
-        if w.dtype == torch.float16:
-            return w
-        key = (w.data_ptr(), w.device, 0 if w.is_inference() else w._version)
-        if self._half_w is None or self._half_w[0] != key:
-            half = w.to(torch.float16)
-            if w.is_cuda and torch.cuda.is_current_stream_capturing():
-                return half                                    # recorded, not computed: of no use to a later eager call
-            self._half_w = (key, half)
-        return self._half_w[1]
-
-    def process_weights_after_loading(self, act_dtype: torch.dtype):
-        super().process_weights_after_loading(act_dtype)
-        self._half_w = None                                    # (weights reloaded through .data carry no new version)
-        self._half_up_weight()
-
-    def _split_kv(self, kv: torch.Tensor):
-        kv = kv.view(-1, self.num_heads, self.qk_nope_head_dim + self.v_head_dim)
-        return kv[..., :self.qk_nope_head_dim], kv[..., self.qk_nope_head_dim:]
-
-    def _kv_up(self, kv_c: torch.Tensor, allow_fp16: bool = False):
-        """(k_nope [T,N,128], v [T,N,128]) of latent rows kv_c [T,512] (reference: ``self.kv_b_proj(kv_c_normed)[0]``,
-        mla.py:405-413, 566-571).  With ``allow_fp16`` both may come back as fp16."""
-        w = self._half_up_weight() if allow_fp16 and kv_c.dtype in (torch.bfloat16, torch.float16) else None
-        if w is not None and kv_c.shape[-1] == w.shape[1]:
-            return self._split_kv(torch.matmul(kv_c.to(torch.float16), w.t()))
-        kv = self.kv_b_proj(kv_c)
-        return self._split_kv(kv[0] if isinstance(kv, tuple) else kv)
-
-    def _kv_up_rows(self, kv_c: torch.Tensor, k_pe: torch.Tensor):
-        """(k_nope, k_pe [T,64], v) of a step's own rows as the prefill kernel takes them: all fp16 where the weight allows
-        it (latent and rope rows converted in one launch), else all in the dtype of the up-projection's result."""
-        w = self._half_up_weight()
-        if w is not None and kv_c.dtype == torch.bfloat16 and k_pe.dtype == torch.bfloat16:
-            c16, pe16 = K.rows_f16(kv_c, k_pe)
-            k_nope, v = self._split_kv(torch.matmul(c16, w.t()))
-            return k_nope, pe16, v
-        k_nope, v = self._kv_up(kv_c, allow_fp16=True)
-        return k_nope, k_pe.reshape(k_pe.shape[0], -1).to(k_nope.dtype), v
 
     # ---- prefill ----
     def _compute_prefill_context(self, q_nope, q_pe, kv_c_cache, k_pe_cache, attn_metadata, k_scale):

@@ -37,6 +37,7 @@ struct IndexerParams {
   int32_t batch, max_q_len, num_heads, page_size;
   int64_t num_pages;
   float* logits; int64_t l_st;                        // [T, l_st]
+  int32_t skip_up_to;                                 // tokens that see no more keys than this get no logits (tile kernel)
 };
 
 __device__ __forceinline__ int idx_wave_sum(int v) {
@@ -211,10 +212,116 @@ __global__ __launch_bounds__(256, 2) void dsa_indexer_fp8_kernel(const IndexerPa
   }  // segments
 }
 
+// The same scores for prompts, where neighbouring query tokens see the same keys: the kernel above reads every token's keys
+// for itself (10 168 prompt tokens, 20 M (token, key) pairs: 2.7 GB through the L2s, 980 us).  Here a workgroup keeps the
+// queries of kTileTok tokens of one request in LDS (64 KiB, two workgroups per CU) and each of its wavefronts walks every
+// 4 gridDim.x-th block of 32 keys, held in registers (the next block on its way meanwhile), against all of the tokens: a
+// key is read once per kTileTok tokens, a query operand from LDS at a quarter of its rate, and what is left is the 16 MFMAs
+// and 64 relu-FMAs per token and block.  Same operations in the same order as above: the same bits.
+constexpr int kTileTok = 8;
+constexpr int kTileMinQ = 16;                         // shorter requests (decode, MTP) take the streaming kernel
+constexpr int kTileWOff = kTileTok * 64 * kIdxDim;    // 65536: weights [token][head] behind the query rows
+constexpr int kTileLdsB = kTileWOff + kTileTok * 64 * 4;
+
+__global__ __launch_bounds__(256, 2) void dsa_indexer_tile_kernel(const IndexerParams p) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int key_l = lane & 31, half = lane >> 5;
+  const int b = blockIdx.z, tok0 = blockIdx.y * kTileTok;
+  int q0 = b * p.max_q_len, qlen = p.max_q_len;
+  if (p.qsl) { q0 = p.qsl[b]; qlen = p.qsl[b + 1] - q0; qlen = qlen < p.max_q_len ? qlen : p.max_q_len; }
+  if (tok0 >= qlen) return;
+  const int nt = qlen - tok0 < kTileTok ? qlen - tok0 : kTileTok;
+  const int lim0 = p.seq_lens[b] - qlen + tok0 + 1;          // visible keys of the first token; one more for each later one
+  const int lim_max = lim0 + nt - 1;
+  const int blocks = lim_max > p.skip_up_to ? (lim_max + 31) >> 5 : 0;
+  if ((int)blockIdx.x * 4 >= blocks) return;
+
+  // queries: row (token, head) of 128 bytes, 16-byte granule g at position g ^ ((head >> 1) & 7)
+  const uint32_t lds0 = lds_addr_of(lds);
+#pragma unroll
+  for (int i = 0; i < kTileTok * 2; i++) {
+    const int g = wave * (kTileTok * 2) + i;                 // group of eight rows
+    const int tk = g >> 3 < nt ? g >> 3 : nt - 1, head = (g & 7) * 8 + (lane >> 3);
+    dma16_v(p.q8 + (int64_t)(q0 + tok0 + tk) * p.q_st + (int64_t)head * p.q_sh + (((lane & 7) ^ ((head >> 1) & 7)) << 4),
+            lds0 + g * 1024);
+  }
+#pragma unroll
+  for (int i = 0; i < kTileTok * 64 / 256; i++) {
+    const int e = threadIdx.x + i * 256, head = e & 63, tk = e >> 6 < nt ? e >> 6 : nt - 1;
+    float w = p.weights[(int64_t)(q0 + tok0 + tk) * p.w_st + head];
+    if (p.q_scale) w *= p.q_scale[(int64_t)(q0 + tok0 + tk) * p.qs_st + head];
+    *(float*)(lds + kTileWOff + e * 4) = w;
+  }
+
+  const int stride = (int)gridDim.x * 4;
+  auto load_block = [&](int blk, u32x4 (&kb)[4], float& ks) {
+    const int key0 = blk * 32, pg = key0 / p.page_size;
+    const int pgc = pg < p.max_blocks ? pg : p.max_blocks - 1;
+    int64_t id = ((const __attribute__((address_space(4))) int32_t*)p.block_table)[(int64_t)b * p.bt_stride + pgc];
+    id = id < 0 ? 0 : (id >= p.num_pages ? p.num_pages - 1 : id);
+    const int off = key0 - pg * p.page_size + key_l;
+    const uint8_t* row = p.k8 + id * p.k_sp + (int64_t)off * p.k_sr + half * 64;
+#pragma unroll
+    for (int j = 0; j < 4; j++) kb[j] = *(const u32x4*)(row + j * 16);
+    ks = p.k_scale[id * p.ks_sp + off];
+  };
+  u32x4 kb[4], kn[4];
+  float ks = 0.f, ks_n = 0.f;
+  int blk = (int)blockIdx.x * 4 + wave;
+  if (blk < blocks) load_block(blk, kn, ks_n);
+  MLA_WAIT_VMCNT(0);
+  lds_barrier();
+
+  const int row_off = key_l * kIdxDim, swz = (key_l >> 1) & 7;   // (rows 32 apart share the swizzle)
+  for (; blk < blocks; blk += stride) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) kb[j] = kn[j];
+    ks = ks_n;
+    if (blk + stride < blocks) load_block(blk + stride, kn, ks_n);
+    const int key0 = blk * 32;
+#pragma unroll 1
+    for (int i = 0; i < nt; i++) {
+      const int limit = lim0 + i;
+      if (key0 >= limit || limit <= p.skip_up_to) continue;
+      const char* qp = lds + i * 64 * kIdxDim + row_off;
+      f32x16 c0, c1;
+#pragma unroll
+      for (int r = 0; r < 16; r++) { c0[r] = 0.f; c1[r] = 0.f; }
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int gr = ((4 * half + j) ^ swz) << 4;
+        const u32x4 a0 = *(const u32x4*)(qp + gr), a1 = *(const u32x4*)(qp + 32 * kIdxDim + gr), v = kb[j];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          const long bop = (long)(((uint64_t)v[2 * h + 1] << 32) | v[2 * h]);
+          c0 = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8((long)(((uint64_t)a0[2 * h + 1] << 32) | a0[2 * h]), bop, c0, 0, 0, 0);
+          c1 = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8((long)(((uint64_t)a1[2 * h + 1] << 32) | a1[2 * h]), bop, c1, 0, 0, 0);
+        }
+      }
+      const char* wp = lds + kTileWOff + i * 256 + half * 16;
+      float acc = 0.f;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const f32x4 w0 = *(const f32x4*)(wp + q * 32), w1 = *(const f32x4*)(wp + 128 + q * 32);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          acc = fmaf(w0[e], fmaxf(c0[q * 4 + e], 0.f), acc);
+          acc = fmaf(w1[e], fmaxf(c1[q * 4 + e], 0.f), acc);
+        }
+      }
+      acc += xor32(acc);
+      if (half == 0) p.logits[(int64_t)(q0 + tok0 + i) * p.l_st + key0 + key_l] = key0 + key_l < limit ? acc * ks : -INFINITY;
+    }
+  }
+}
+
 // Per-row e4m3 quantisation of 128-wide bf16 rows (one fp32 scale = amax/448 per row, 1.0 for an all-zero row),
 // optionally scattered through a slot mapping into a paged fp8 cache + scale cache: the indexer-K write of
 // src/omni_npu/vllm_patches/patches/models/deepseek/patch_dsv32_indexer.py:116-121 with quantisation fused in, and
-// the query quantisation (no slot mapping).  One wavefront per row, lane l owns elements 2l, 2l+1.
+// the query quantisation (no slot mapping).  Sixteen lanes per row, lane l owns elements 8l .. 8l + 7: a wavefront's load
+// and store cover four rows, 1 KiB and 512 bytes (a wavefront per row, four bytes a lane: 650 752 query rows 150 us).
 struct QuantRows {
   const __bf16* src; int64_t src_stride, rows;
   const int64_t* slots;
@@ -226,21 +333,46 @@ struct QuantRows {
 __device__ __forceinline__ void quant_row(const __bf16* src, int64_t src_stride, int64_t rows, const int64_t* slots,
                                           uint8_t* dst8, int64_t d_sp, int64_t d_sr, float* dscale, int64_t s_sp,
                                           int32_t page_size, int64_t num_pages, int64_t r) {
-  const int lane = threadIdx.x & 63;
+  const int l16 = threadIdx.x & 15;
   if (r >= rows) return;
-  int64_t slot = slots ? slots[r] : r;
+  const int64_t slot = slots ? slots[r] : r;
   if (slot < 0 || slot >= num_pages * page_size) return;
-  const int64_t pg = slot / page_size, off = slot - pg * page_size;
-  const bf16x2 v = *(const bf16x2*)(src + r * src_stride + lane * 2);
-  const float x0 = (float)v[0], x1 = (float)v[1];
-  float amax = fmaxf(fabsf(x0), fabsf(x1));
+  int64_t pg = 0, off = slot;
+  if (slots) { pg = slot / page_size; off = slot - pg * page_size; }
+  float x[8], amax = 0.f;
+  if ((((uintptr_t)src | (uintptr_t)(src_stride * 2)) & 15) == 0) {
+    const bf16x8 v = *(const bf16x8*)(src + r * src_stride + l16 * 8);
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+    for (int e = 0; e < 8; e++) x[e] = (float)v[e];
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      const bf16x2 v = *(const bf16x2*)(src + r * src_stride + l16 * 8 + e);
+      x[e] = (float)v[0];
+      x[e + 1] = (float)v[1];
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(x[e]));
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
   const float scale = amax > 0.f ? amax / 448.f : 1.f;
-  const float y0 = fminf(fmaxf(x0 / scale, -448.f), 448.f), y1 = fminf(fmaxf(x1 / scale, -448.f), 448.f);
-  const int w = __builtin_amdgcn_cvt_pk_fp8_f32(y0, y1, 0, false);
-  *(uint16_t*)(dst8 + pg * d_sp + off * d_sr + lane * 2) = (uint16_t)(w & 0xFFFF);
-  if (lane == 0) dscale[pg * s_sp + off] = scale;
+  uint32_t w[2];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    float y[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) y[e] = fminf(fmaxf(x[4 * h + e] / scale, -448.f), 448.f);
+    w[h] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(y[2], y[3], __builtin_amdgcn_cvt_pk_fp8_f32(y[0], y[1], 0, false), true);
+  }
+  uint8_t* d = dst8 + pg * d_sp + off * d_sr + l16 * 8;
+  if ((((uintptr_t)dst8 | (uintptr_t)d_sp | (uintptr_t)d_sr) & 7) == 0) {
+    *(u32x2*)d = u32x2{w[0], w[1]};
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; e++) *(uint16_t*)(d + 2 * e) = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+  }
+  if (l16 == 0) dscale[pg * s_sp + off] = scale;
 }
 
 __global__ __launch_bounds__(256) void dsa_quant_rows_kernel(const __bf16* src, int64_t src_stride, int64_t rows,
@@ -248,7 +380,7 @@ __global__ __launch_bounds__(256) void dsa_quant_rows_kernel(const __bf16* src, 
                                                              float* dscale, int64_t s_sp, int32_t page_size,
                                                              int64_t num_pages) {
   quant_row(src, src_stride, rows, slots, dst8, d_sp, d_sr, dscale, s_sp, page_size, num_pages,
-            (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6));
+            (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4));
 }
 
 // Two row sets in one launch (the indexer's step: the query rows into plain buffers, the new key rows into the cache):
@@ -257,7 +389,7 @@ __global__ __launch_bounds__(256) void dsa_quant_rows2_kernel(const QuantRows a,
   const bool first = (int)blockIdx.x < a_blocks;
   const QuantRows& q = first ? a : b;
   quant_row(q.src, q.src_stride, q.rows, q.slots, q.dst8, q.d_sp, q.d_sr, q.dscale, q.s_sp, q.page_size, q.num_pages,
-            (int64_t)(first ? blockIdx.x : blockIdx.x - a_blocks) * 4 + (threadIdx.x >> 6));
+            (int64_t)(first ? blockIdx.x : blockIdx.x - a_blocks) * 16 + (threadIdx.x >> 4));
 }
 
 }  // namespace mlahip
@@ -282,7 +414,7 @@ extern "C" int dsa_quant_qk_fp8(const void* q, int64_t q_stride, int64_t q_rows,
                     (int32_t)(q_rows > 0 ? q_rows : 1), 1};
   const QuantRows b{(const __bf16*)k, k_stride, k_rows, slot_mapping, (uint8_t*)k8_cache, cache_page_stride_bytes,
                     cache_row_stride_bytes, scale_cache, scale_page_stride, page_size, num_pages};
-  const int64_t a_blocks = (q_rows + 3) / 4, b_blocks = (k_rows + 3) / 4;
+  const int64_t a_blocks = (q_rows + 15) / 16, b_blocks = (k_rows + 15) / 16;
   hipLaunchKernelGGL(dsa_quant_rows2_kernel, dim3((unsigned)(a_blocks + b_blocks)), dim3(256), 0, stream, a, b,
                      (int32_t)a_blocks);
   return check_launch("dsa_quant_rows2_kernel");
@@ -298,20 +430,20 @@ extern "C" int dsa_quant_rows_fp8(const void* src, int64_t src_stride, int64_t r
                   dst_page_stride_bytes % 2 == 0,
               MLA_ERR_SHAPE, "dsa_quant_rows_fp8: rows=%lld page_size=%d", (long long)rows, page_size);
   if (rows == 0) return MLA_OK;
-  hipLaunchKernelGGL(dsa_quant_rows_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, (const __bf16*)src,
+  hipLaunchKernelGGL(dsa_quant_rows_kernel, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, (const __bf16*)src,
                      src_stride, rows, slot_mapping, (uint8_t*)dst8, dst_page_stride_bytes, dst_row_stride_bytes, dst_scale,
                      scale_page_stride, page_size, num_pages);
   return check_launch("dsa_quant_rows_kernel");
 }
 
-extern "C" int dsa_indexer_scores_fp8(const void* q8, int64_t q_stride_t, int64_t q_stride_h, const float* weights,
+static int indexer_scores_impl(const void* q8, int64_t q_stride_t, int64_t q_stride_h, const float* weights,
                                       int64_t w_stride_t, const float* q_scale, int64_t qs_stride_t, const void* k8_cache,
                                       int64_t k_page_stride, int64_t k_row_stride, const float* k_scale_cache,
                                       int64_t ks_page_stride, int64_t num_pages, int32_t page_size,
                                       const int32_t* block_table, int64_t bt_stride, int32_t max_blocks,
                                       const int32_t* seq_lens, const int32_t* query_start_loc, int32_t batch,
                                       int32_t max_q_len, int32_t num_heads, int32_t max_seq_len, float* logits,
-                                      int64_t logits_stride, hipStream_t stream) {
+                                      int64_t logits_stride, int32_t skip_up_to, hipStream_t stream) {
   MLA_REQUIRE(q8 && weights && k8_cache && k_scale_cache && block_table && seq_lens && logits, MLA_ERR_NULL,
               "dsa_indexer_scores_fp8: null pointer argument");
   MLA_REQUIRE(num_heads == 64, MLA_ERR_UNSUPPORTED, "dsa_indexer_scores_fp8: 64 index heads only (got %d)", num_heads);
@@ -337,7 +469,21 @@ extern "C" int dsa_indexer_scores_fp8(const void* q8, int64_t q_stride_t, int64_
   p.block_table = block_table; p.bt_stride = bt_stride; p.max_blocks = max_blocks;
   p.seq_lens = seq_lens; p.qsl = query_start_loc;
   p.batch = batch; p.max_q_len = max_q_len; p.num_heads = num_heads; p.page_size = page_size; p.num_pages = num_pages;
-  p.logits = logits; p.l_st = logits_stride;
+  p.logits = logits; p.l_st = logits_stride; p.skip_up_to = skip_up_to;
+  if (max_q_len >= kTileMinQ) {
+    // about 2048 workgroups (four rounds of two per CU), so that the short ones at the start of a prompt even out
+    const int64_t groups = (int64_t)batch * ((max_q_len + kTileTok - 1) / kTileTok);
+    int64_t split = (2048 + groups - 1) / groups;
+    const int64_t most = (max_seq_len + 127) / 128;           // a block per wavefront
+    split = split > 16 ? 16 : split;
+    split = split > most ? most : split;
+    MLA_REQUIRE(batch <= 65535, MLA_ERR_SHAPE, "dsa_indexer_scores_fp8: too many requests");
+    const int rc = ensure_dynamic_lds((const void*)dsa_indexer_tile_kernel, kTileLdsB, "dsa_indexer_scores_fp8");
+    if (rc != MLA_OK) return rc;
+    hipLaunchKernelGGL(dsa_indexer_tile_kernel, dim3((unsigned)split, (unsigned)((max_q_len + kTileTok - 1) / kTileTok), (unsigned)batch),
+                       dim3(256), kTileLdsB, stream, p);
+    return check_launch("dsa_indexer_tile_kernel");
+  }
   // two workgroups per compute unit (what their LDS rings allow), never more wavefronts than 32-key blocks
   static int num_cus = 0;
   if (num_cus == 0) {
@@ -354,4 +500,29 @@ extern "C" int dsa_indexer_scores_fp8(const void* q8, int64_t q_stride_t, int64_
   if (rc != MLA_OK) return rc;
   hipLaunchKernelGGL(dsa_indexer_fp8_kernel, dim3((unsigned)wgs), dim3(256), kIdxLdsB, stream, p);
   return check_launch("dsa_indexer_fp8_kernel");
+}
+
+extern "C" int dsa_indexer_scores_fp8(const void* q8, int64_t q_stride_t, int64_t q_stride_h, const float* weights,
+                                      int64_t w_stride_t, const float* q_scale, int64_t qs_stride_t, const void* k8_cache,
+                                      int64_t k_page_stride, int64_t k_row_stride, const float* k_scale_cache,
+                                      int64_t ks_page_stride, int64_t num_pages, int32_t page_size,
+                                      const int32_t* block_table, int64_t bt_stride, int32_t max_blocks,
+                                      const int32_t* seq_lens, const int32_t* query_start_loc, int32_t batch,
+                                      int32_t max_q_len, int32_t num_heads, int32_t max_seq_len, float* logits,
+                                      int64_t logits_stride, hipStream_t stream) {
+  return indexer_scores_impl(q8, q_stride_t, q_stride_h, weights, w_stride_t, q_scale, qs_stride_t, k8_cache, k_page_stride, k_row_stride, k_scale_cache, ks_page_stride, num_pages, page_size, block_table, bt_stride, max_blocks, seq_lens, query_start_loc, batch, max_q_len, num_heads, max_seq_len, logits, logits_stride, 0, stream);
+}
+
+// The same without the logits of tokens that see at most skip_up_to keys (a selection of that many takes them all, whatever
+// they score): those rows are left as they are or filled, as it suits the launch.
+extern "C" int dsa_indexer_scores_fp8_above(const void* q8, int64_t q_stride_t, int64_t q_stride_h, const float* weights,
+                                      int64_t w_stride_t, const float* q_scale, int64_t qs_stride_t, const void* k8_cache,
+                                      int64_t k_page_stride, int64_t k_row_stride, const float* k_scale_cache,
+                                      int64_t ks_page_stride, int64_t num_pages, int32_t page_size,
+                                      const int32_t* block_table, int64_t bt_stride, int32_t max_blocks,
+                                      const int32_t* seq_lens, const int32_t* query_start_loc, int32_t batch,
+                                      int32_t max_q_len, int32_t num_heads, int32_t max_seq_len, float* logits,
+                                      int64_t logits_stride, int32_t skip_up_to, hipStream_t stream) {
+  MLA_REQUIRE(skip_up_to >= 0, MLA_ERR_SHAPE, "dsa_indexer_scores_fp8_above: skip_up_to=%d", skip_up_to);
+  return indexer_scores_impl(q8, q_stride_t, q_stride_h, weights, w_stride_t, q_scale, qs_stride_t, k8_cache, k_page_stride, k_row_stride, k_scale_cache, ks_page_stride, num_pages, page_size, block_table, bt_stride, max_blocks, seq_lens, query_start_loc, batch, max_q_len, num_heads, max_seq_len, logits, logits_stride, skip_up_to, stream);
 }

@@ -67,6 +67,8 @@ struct PrefillParams {
   // (an earlier context chunk); the launch then returns the attention over the union, as a merge of the two would
   const float* prev_out; int64_t po_st, po_sh;
   const float* prev_lse;  // [T, N]
+  // optional picks (kPick): bit j of a token's row says whether key j of its sequence is one of the keys it attends over
+  const uint32_t* pick; int64_t pick_st; int32_t pick_tiles;   // row stride in words; whole tiles (two words) a row holds
 };
 
 // One 64-key tile of head `head`, keys k0 .. k0 + 63 of the flat key axis (clamped to klast): 40 copy instructions of eight
@@ -121,7 +123,9 @@ __device__ __forceinline__ void pf_issue_tile(const PrefillParams& p, int64_t k0
 
 // kHalf: k_nope, k_pe and v hold fp16 instead of bf16 (a caller that makes them with an fp16 GEMM): both products run on
 // fp16 (the query is converted once, in registers) and no tile is converted.
-template <bool kHalf>
+// kPick: a row attends over the keys its bits name (sparse attention over a selection, for sequences short enough that
+// leaving out scores here costs less than gathering the selected latents; see NPUDSAImpl).
+template <bool kHalf, bool kPick>
 __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const PrefillParams p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63;
@@ -255,11 +259,22 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
       for (int e = 0; e < 2; e++)
         voff[rd][e] = kPfVOff + (v_row + 8 * rd) * 128 + (j16 & 1) * 8 + (((e * 4 + v_cl) ^ pf_swz(v_row + 8 * rd)) << 4);
 
+    // (the bits of a tile are asked for one tile ahead, in front of its copies: the wait that lets those land covers them)
+    const u32x2* pick = nullptr;
+    u32x2 bits_next = {0u, 0u};
+    auto pick_tile = [&](int tile) { return pick[tile < p.pick_tiles ? tile : p.pick_tiles - 1]; };
+    if constexpr (kPick) {
+      pick = (const u32x2*)(p.pick + tq * p.pick_st);
+      bits_next = pick_tile(first_tile);
+    }
+
     for (int tile = first_tile; tile < tiles; tile++) {
       char* buf = lds + (tile & 1) * kPfBufB;
       // this tile has landed (only its copies are in flight here) and everyone is done with the other buffer
       MLA_WAIT_VMCNT(0);
       lds_barrier();
+      const u32x2 bits = bits_next;
+      if constexpr (kPick) bits_next = pick_tile(tile + 1 < tiles ? tile + 1 : tile);
       if (tile + 1 < tiles) issue(tile + 1, lds0 + ((tile + 1) & 1) * kPfBufB);
       const int key_base = tile * kPfTile;
       // V of this tile goes from bf16 to fp16 where it lies (thread t takes the 16-byte pieces t, t + 256, ...), then a
@@ -283,6 +298,19 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
         lds_barrier();
       }
       if (key_base >= wave_max_limit || key_base + kPfTile <= wg_lo) continue;   // no row of this wavefront sees the tile
+
+      uint32_t seen[2] = {0u, 0u};                             // kPick: the row's keys in the tile's two blocks
+      bool mask_tile = key_base + kPfTile > wave_min_limit || key_base < wave_max_lo;
+      if constexpr (kPick) {
+        const int rel = limit - key_base;                     // (keys behind the causal limit have no bits worth reading)
+#pragma unroll
+        for (int tb = 0; tb < 2; tb++) {
+          const int in_blk = rel - tb * 32;
+          seen[tb] = in_blk >= 32 ? bits[tb] : (in_blk <= 0 ? 0u : bits[tb] & ((1u << in_blk) - 1u));
+        }
+        if (__builtin_amdgcn_ballot_w64((seen[0] | seen[1]) != 0u) == 0) continue;
+        mask_tile = __builtin_amdgcn_ballot_w64((seen[0] & seen[1]) != ~0u) != 0;
+      }
 
       f32x16 s[2];
       f16x2 pb[2][8];
@@ -313,13 +341,19 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
       __builtin_amdgcn_s_setprio(0);
       // Only tiles that some row of this wave cannot see in full pay for the mask (causal diagonal, end of the keys,
       // rows past the end of the sequence).
-      if (key_base + kPfTile > wave_min_limit || key_base < wave_max_lo) {
+      if (mask_tile) {
 #pragma unroll
         for (int tb = 0; tb < 2; tb++)
 #pragma unroll
           for (int r = 0; r < 16; r++) {
-            const int key = key_base + tb * 32 + 4 * half + 8 * (r >> 2) + (r & 3);
-            s[tb][r] = (key < limit && key >= lo) ? s[tb][r] : -INFINITY;
+            if constexpr (kPick) {
+              const uint32_t on = (uint32_t)((int32_t)(seen[tb] >> (4 * half) << (31 - (8 * (r >> 2) + (r & 3)))) >> 31);
+              const float v = s[tb][r];                      // (a bit_cast of the element itself reads element 0)
+              s[tb][r] = __uint_as_float((on & __float_as_uint(v)) | (~on & 0xff800000u));
+            } else {
+              const int key = key_base + tb * 32 + 4 * half + 8 * (r >> 2) + (r & 3);
+              s[tb][r] = (key < limit && key >= lo) ? s[tb][r] : -INFINITY;
+            }
           }
       }
       float psum = probs(1, probs(0, 0.f));
@@ -395,7 +429,8 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
                                int32_t batch, int32_t num_heads, int32_t max_q_len, int32_t causal, int32_t window,
                                float scale, void* out, int64_t out_stride_t, int64_t out_stride_h, int32_t out_dtype,
                                float* lse_out, const float* prev_out, int64_t prev_stride_t, int64_t prev_stride_h,
-                               const float* prev_lse, hipStream_t stream) {
+                               const float* prev_lse, const uint32_t* pick, int64_t pick_stride, int32_t pick_words,
+                               hipStream_t stream) {
   MLA_REQUIRE(q_nope && q_pe && k_nope && k_pe && v && cu_q && cu_k && out, MLA_ERR_NULL, "%s: null pointer argument", what);
   MLA_REQUIRE(batch >= 0 && num_heads >= 1 && max_q_len >= 0 && batch <= 65535 && num_heads <= 65535 && window >= 0,
               MLA_ERR_SHAPE, "%s: batch=%d num_heads=%d max_q_len=%d window=%d", what, batch, num_heads, max_q_len, window);
@@ -412,6 +447,9 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
   MLA_REQUIRE((prev_out == nullptr) == (prev_lse == nullptr), MLA_ERR_NULL, "%s: the earlier result and its log-sum-exp go together", what);
   MLA_REQUIRE(prev_out == nullptr || (prev_stride_t % 4 == 0 && prev_stride_h % 4 == 0 && (uintptr_t)prev_out % 16 == 0),
               MLA_ERR_SHAPE, "%s: rows of the earlier result must be 16-byte aligned", what);
+  MLA_REQUIRE(pick == nullptr || (kv_half && window == 0 && pick_words >= 2 && pick_words % 2 == 0 && pick_stride >= pick_words &&
+                                  pick_stride % 2 == 0 && (uintptr_t)pick % 8 == 0),
+              MLA_ERR_SHAPE, "%s: picks go with fp16 keys and values, without a window, in 8-byte aligned rows of whole 64-key tiles", what);
   if (batch == 0 || max_q_len == 0) return MLA_OK;
   PrefillParams p;
   p.q_nope = (const __bf16*)q_nope; p.qn_st = qn_stride_t; p.qn_sh = qn_stride_h;
@@ -424,12 +462,14 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
   p.out = out; p.o_st = out_stride_t; p.o_sh = out_stride_h; p.out_fp32 = out_dtype;
   p.lse = lse_out;
   p.prev_out = prev_out; p.po_st = prev_stride_t; p.po_sh = prev_stride_h; p.prev_lse = prev_lse;
-  int rc = ensure_dynamic_lds((const void*)mla_prefill_varlen_kernel<false>, kPfLdsB, what);
-  if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)mla_prefill_varlen_kernel<true>, kPfLdsB, what);
+  p.pick = pick; p.pick_st = pick_stride; p.pick_tiles = pick_words / 2;
+  auto* kern = pick ? mla_prefill_varlen_kernel<true, true> : kv_half ? mla_prefill_varlen_kernel<true, false> : mla_prefill_varlen_kernel<false, false>;
+  int rc = ensure_dynamic_lds((const void*)mla_prefill_varlen_kernel<false, false>, kPfLdsB, what);
+  if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)mla_prefill_varlen_kernel<true, false>, kPfLdsB, what);
+  if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)mla_prefill_varlen_kernel<true, true>, kPfLdsB, what);
   if (rc != MLA_OK) return rc;
   dim3 grid((max_q_len + kPfRows - 1) / kPfRows, num_heads, batch);
-  if (kv_half) hipLaunchKernelGGL(mla_prefill_varlen_kernel<true>, grid, dim3(256), kPfLdsB, stream, p);
-  else hipLaunchKernelGGL(mla_prefill_varlen_kernel<false>, grid, dim3(256), kPfLdsB, stream, p);
+  hipLaunchKernelGGL(kern, grid, dim3(256), kPfLdsB, stream, p);
   return check_launch("mla_prefill_varlen_kernel");
 }
 
@@ -443,7 +483,7 @@ extern "C" int mla_prefill_varlen(const void* q_nope, int64_t qn_stride_t, int64
   return prefill_varlen_impl("mla_prefill_varlen", q_nope, qn_stride_t, qn_stride_h, q_pe, qp_stride_t, qp_stride_h, k_nope,
                              kn_stride_t, kn_stride_h, k_pe, kp_stride_t, v, v_stride_t, v_stride_h, cu_q, cu_k, batch,
                              num_heads, max_q_len, causal, window, scale, out, out_stride_t, out_stride_h, out_dtype, lse_out,
-                             nullptr, 0, 0, nullptr, stream);
+                             nullptr, 0, 0, nullptr, nullptr, 0, 0, stream);
 }
 
 // The same attention continued from an earlier result over other keys of the same rows (prev_out fp32 [T,N,128] with its
@@ -461,5 +501,23 @@ extern "C" int mla_prefill_varlen_continue(const void* q_nope, int64_t qn_stride
   return prefill_varlen_impl("mla_prefill_varlen_continue", q_nope, qn_stride_t, qn_stride_h, q_pe, qp_stride_t, qp_stride_h,
                              k_nope, kn_stride_t, kn_stride_h, k_pe, kp_stride_t, v, v_stride_t, v_stride_h, cu_q, cu_k, batch,
                              num_heads, max_q_len, causal, window, scale, out, out_stride_t, out_stride_h, out_dtype, lse_out,
-                             prev_out, prev_stride_t, prev_stride_h, prev_lse, stream);
+                             prev_out, prev_stride_t, prev_stride_h, prev_lse, nullptr, 0, 0, stream);
+}
+
+// mla_prefill_varlen over a selection: bit j of pick[t] (32-bit words, rows pick_stride words apart, pick_words of them
+// valid) says whether query token t attends over key j of its sequence, within what causal already allows.  fp16 keys and
+// values, no window.
+extern "C" int mla_prefill_varlen_pick(const void* q_nope, int64_t qn_stride_t, int64_t qn_stride_h, const void* q_pe,
+                                       int64_t qp_stride_t, int64_t qp_stride_h, const void* k_nope, int64_t kn_stride_t,
+                                       int64_t kn_stride_h, const void* k_pe, int64_t kp_stride_t, const void* v,
+                                       int64_t v_stride_t, int64_t v_stride_h, const int32_t* cu_q, const int32_t* cu_k,
+                                       int32_t batch, int32_t num_heads, int32_t max_q_len, int32_t causal, float scale,
+                                       const uint32_t* pick, int64_t pick_stride, int32_t pick_words, void* out,
+                                       int64_t out_stride_t, int64_t out_stride_h, int32_t out_dtype, float* lse_out,
+                                       hipStream_t stream) {
+  MLA_REQUIRE(pick, MLA_ERR_NULL, "mla_prefill_varlen_pick: null pointer argument");
+  return prefill_varlen_impl("mla_prefill_varlen_pick", q_nope, qn_stride_t, qn_stride_h, q_pe, qp_stride_t, qp_stride_h, k_nope,
+                             kn_stride_t, kn_stride_h, k_pe, kp_stride_t, v, v_stride_t, v_stride_h, cu_q, cu_k, batch,
+                             num_heads, max_q_len, causal, 0, scale, out, out_stride_t, out_stride_h, out_dtype, lse_out,
+                             nullptr, 0, 0, nullptr, pick, pick_stride, pick_words, stream);
 }

@@ -68,12 +68,20 @@ struct TopkParams {
   // optional (rows != NULL): also translate every pick into its flat cache row, and count the picks per token
   const int32_t* block_table; int64_t bt_stride; int32_t max_blocks, page_size; int64_t num_pages;
   int32_t* rows; int64_t r_st; int32_t* counts;
+  // optional: the picks again as a bit per position (byte i holds positions 8i .. 8i + 7), rows of m_st bytes
+  uint8_t* mask; int64_t m_st;
 };
 
 // Where pick number `at` of token t (request b) goes: its position into the index buffer and, if asked for, its flat
 // cache row (page * page_size + offset) into the row list that the sparse attention reads.
 struct TopkSink {
   int32_t* out; int32_t* rows; const int32_t* bt; int32_t max_blocks, page_size; int64_t num_pages;
+  uint8_t* mask;
+  // four consecutive positions i .. i + 3 (i a multiple of 4, the lanes of a wavefront side by side): even lanes store a byte
+  __device__ __forceinline__ void put_bits(int i, int n, uint32_t nib) const {
+    const uint32_t up = (uint32_t)__shfl_xor((int)nib, 1, 64);
+    if ((i & 4) == 0 && i < n) mask[i >> 3] = (uint8_t)(nib | (up << 4));
+  }
   __device__ __forceinline__ void put(int at, int pos) const {
     out[at] = pos;
     if (rows) {
@@ -92,6 +100,7 @@ __device__ __forceinline__ TopkSink topk_sink(const TopkParams& p, int b, int t)
   s.rows = p.rows ? p.rows + (int64_t)t * p.r_st : nullptr;
   s.bt = p.rows ? p.block_table + (int64_t)b * p.bt_stride : nullptr;
   s.max_blocks = p.max_blocks; s.page_size = p.page_size; s.num_pages = p.num_pages;
+  s.mask = p.mask ? p.mask + (int64_t)t * p.m_st : nullptr;
   return s;
 }
 
@@ -258,6 +267,7 @@ __device__ __forceinline__ void ordered_write(const float* x, const TopkSink& ou
       for (int e = 0; e < kVec; e++)
         if (tk[e]) { if (at < k) out.put(at, i + e); at++; }
       o += total;
+      if constexpr (kVec == 4) { if (out.mask) out.put_bits(i, r_hi, tk[0] | tk[1] << 1 | tk[2] << 2 | tk[3] << 3); }
     }
   }
 }
@@ -288,6 +298,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_kernel(const TopkParams
     for (int i = tid; i < k; i += kTopkThreads) {
       if (i < n) out.put(i, i); else out.out[i] = -1;
     }
+    if (out.mask) for (int i = tid; i * 8 < n; i += kTopkThreads) out.mask[i] = 0xff;     // (bits at and behind n mean nothing)
     return;
   }
 
@@ -572,6 +583,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_write_kernel(const Topk
       for (int i = tid; i < k; i += kTopkThreads) {
         if (i < n) out.put(i, i); else out.out[i] = -1;
       }
+    if (out.mask && s == 0) for (int i = tid; i * 8 < n; i += kTopkThreads) out.mask[i] = 0xff;
     return;
   }
   if (s * kSliceKeys >= n) return;
@@ -641,6 +653,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_write_kernel(const Topk
     for (int e = 0; e < 4; e++)
       if (tk[e]) { if (at < k) out.put(at, i + e); at++; }
     o += total;
+    if (out.mask) out.put_bits(i, n, tk[0] | tk[1] << 1 | tk[2] << 2 | tk[3] << 3);
   }
 }
 
@@ -714,23 +727,25 @@ static int topk_slices(int64_t tokens, int64_t logits_stride) {
 extern "C" size_t dsa_topk_workspace_bytes(int32_t batch, int32_t max_q_len, int64_t logits_stride) {
   if (batch <= 0 || max_q_len <= 0 || logits_stride <= 0) return 0;
   const size_t tokens = (size_t)batch * max_q_len;
+  if (topk_slices((int64_t)tokens, logits_stride) == 0) return 0;      // (one workgroup per token works without scratch)
   return tokens * ((size_t)kMaxSlices * kBins * 4 + 8 + 16 + (size_t)kMaxSlices * kMwWaves * 4 + (size_t)logits_stride * 8);
 }
 
 static int topk_impl(const float* logits, int64_t logits_stride, const int32_t* seq_lens, const int32_t* query_start_loc,
                      int32_t batch, int32_t max_q_len, int32_t k, int32_t* out_indices, int64_t out_stride,
                      const int32_t* block_table, int64_t bt_stride, int32_t max_blocks, int32_t page_size, int64_t num_pages,
-                     int32_t* rows, int64_t rows_stride, int32_t* counts, void* workspace, size_t workspace_bytes,
-                     hipStream_t stream) {
+                     int32_t* rows, int64_t rows_stride, int32_t* counts, uint8_t* mask, int64_t mask_stride, void* workspace,
+                     size_t workspace_bytes, hipStream_t stream) {
   MLA_REQUIRE(logits && seq_lens && out_indices, MLA_ERR_NULL, "dsa_topk: null pointer argument");
   MLA_REQUIRE(batch >= 0 && max_q_len >= 1 && k >= 1 && out_stride >= k, MLA_ERR_SHAPE,
               "dsa_topk: batch=%d max_q_len=%d k=%d out_stride=%lld", batch, max_q_len, k, (long long)out_stride);
   MLA_REQUIRE(logits_stride < (1ll << 22), MLA_ERR_SHAPE, "dsa_topk: at most 2^22 keys per row");
   if (batch == 0) return MLA_OK;
   TopkParams p{logits, logits_stride, seq_lens, query_start_loc, batch, max_q_len, k, out_indices, out_stride,
-               block_table, bt_stride, max_blocks, page_size, num_pages, rows, rows_stride, counts};
+               block_table, bt_stride, max_blocks, page_size, num_pages, rows, rows_stride, counts, mask, mask_stride};
   // rows that start on 16-byte boundaries are read four keys per load
   const bool vec = ((uintptr_t)logits % 16 == 0) && (logits_stride % 4 == 0);
+  MLA_REQUIRE(!mask || vec, MLA_ERR_SHAPE, "dsa_topk: a pick mask wants 16-byte aligned logits rows");
   const int64_t tokens = (int64_t)batch * max_q_len;
   const int slices = topk_slices(tokens, logits_stride);
   if (!workspace || slices == 0) {
@@ -769,7 +784,7 @@ extern "C" int dsa_topk(const float* logits, int64_t logits_stride, const int32_
                         int32_t batch, int32_t max_q_len, int32_t k, int32_t* out_indices, int64_t out_stride,
                         void* workspace, size_t workspace_bytes, hipStream_t stream) {
   return topk_impl(logits, logits_stride, seq_lens, query_start_loc, batch, max_q_len, k, out_indices, out_stride, nullptr, 0,
-                   1, 1, 1, nullptr, 0, nullptr, workspace, workspace_bytes, stream);
+                   1, 1, 1, nullptr, 0, nullptr, nullptr, 0, workspace, workspace_bytes, stream);
 }
 
 // dsa_topk and dsa_build_rows in one: besides the positions (the reference's index buffer) every pick is translated
@@ -784,7 +799,18 @@ extern "C" int dsa_topk_rows(const float* logits, int64_t logits_stride, const i
               MLA_ERR_SHAPE, "dsa_topk_rows: page_size=%d max_blocks=%d rows_stride=%lld", page_size, max_blocks,
               (long long)rows_stride);
   return topk_impl(logits, logits_stride, seq_lens, query_start_loc, batch, max_q_len, k, out_indices, out_stride, block_table,
-                   bt_stride, max_blocks, page_size, num_pages, rows, rows_stride, counts, workspace, workspace_bytes, stream);
+                   bt_stride, max_blocks, page_size, num_pages, rows, rows_stride, counts, nullptr, 0, workspace, workspace_bytes, stream);
+}
+
+// dsa_topk with the picks also as bits: bit (i & 7) of byte i >> 3 of mask[t] says whether position i is picked, for the
+// positions token t sees (bits behind them are undefined).
+extern "C" int dsa_topk_mask(const float* logits, int64_t logits_stride, const int32_t* seq_lens,
+                             const int32_t* query_start_loc, int32_t batch, int32_t max_q_len, int32_t k,
+                             int32_t* out_indices, int64_t out_stride, void* mask, int64_t mask_stride, void* workspace,
+                             size_t workspace_bytes, hipStream_t stream) {
+  MLA_REQUIRE(mask, MLA_ERR_NULL, "dsa_topk_mask: null pointer argument");
+  return topk_impl(logits, logits_stride, seq_lens, query_start_loc, batch, max_q_len, k, out_indices, out_stride, nullptr, 0,
+                   1, 1, 1, nullptr, 0, nullptr, (uint8_t*)mask, mask_stride, workspace, workspace_bytes, stream);
 }
 
 extern "C" int dsa_build_rows(const int32_t* indices, int64_t indices_stride, const int32_t* block_table, int64_t bt_stride,

@@ -606,12 +606,13 @@ def indexer_logits_stride(max_seq_len: int) -> int:
 def indexer_scores(q8: torch.Tensor, weights: torch.Tensor, k8_cache: torch.Tensor, k_scale_cache: torch.Tensor,
                    block_table: torch.Tensor, seq_lens: torch.Tensor, logits: torch.Tensor, q_len: int = 1,
                    q_scale: Optional[torch.Tensor] = None, query_start_loc: Optional[torch.Tensor] = None,
-                   max_seq_len: Optional[int] = None) -> torch.Tensor:
+                   max_seq_len: Optional[int] = None, skip_up_to: int = 0) -> torch.Tensor:
     """logits[t, s] = k_scale[s] * sum_h w[t,h] (* q_scale[t,h]) * relu(q8[t,h] . k8[s]) for the visible keys s of token t.
 
     q8 [T,64,128] float8_e4m3fn (or uint8 bits), weights fp32 [T,64], k8_cache [nblk,page,128] fp8, k_scale_cache fp32
     [nblk,page], logits fp32 [T, >= round_up(max_seq_len, 32)] (reference call site:
-    src/omni_npu/v1/layers/attention/npu_dsa.py:92-103)."""
+    src/omni_npu/v1/layers/attention/npu_dsa.py:92-103).  Tokens that see at most ``skip_up_to`` keys may be left without
+    logits (a top-k of that many takes all of their keys)."""
     _need_cuda(q8, weights, k8_cache, k_scale_cache, block_table, seq_lens, logits, q_scale)
     lib = _lib.load()
     if k8_cache.dim() == 4 and k8_cache.shape[2] == 1:
@@ -638,13 +639,13 @@ def indexer_scores(q8: torch.Tensor, weights: torch.Tensor, k8_cache: torch.Tens
         raise ValueError("indexer_scores: logits must be [T, >= round_up(max_seq_len, 32)]")
     if query_start_loc is None and t != b * q_len:
         raise ValueError(f"indexer_scores: {t} query tokens != batch {b} x q_len {q_len}")
-    rc = lib.dsa_indexer_scores_fp8(
+    rc = lib.dsa_indexer_scores_fp8_above(
         q8.data_ptr(), q8.stride(0), q8.stride(1), weights.data_ptr(), weights.stride(0),
         q_scale.data_ptr() if q_scale is not None else None, q_scale.stride(0) if q_scale is not None else 0,
         k8_cache.data_ptr(), k8_cache.stride(0), k8_cache.stride(1), k_scale_cache.data_ptr(), k_scale_cache.stride(0),
         k8_cache.shape[0], k8_cache.shape[1], block_table.data_ptr(), block_table.stride(0), block_table.shape[1],
         seq_lens.data_ptr(), query_start_loc.data_ptr() if query_start_loc is not None else None, b, q_len, h,
-        int(max_seq_len), logits.data_ptr(), logits.stride(0), _stream(q8))
+        int(max_seq_len), logits.data_ptr(), logits.stride(0), int(skip_up_to), _stream(q8))
     _lib.check(rc, "dsa_indexer_scores_fp8")
     return logits
 
@@ -652,13 +653,15 @@ def indexer_scores(q8: torch.Tensor, weights: torch.Tensor, k8_cache: torch.Tens
 def topk(logits: torch.Tensor, seq_lens: torch.Tensor, k: int, out: torch.Tensor, q_len: int = 1,
          query_start_loc: Optional[torch.Tensor] = None, workspace: Optional[torch.Tensor] = None,
          single_workgroup: bool = False, block_table: Optional[torch.Tensor] = None, page_size: int = PAGE,
-         num_pages: int = 0, rows: Optional[torch.Tensor] = None, counts: Optional[torch.Tensor] = None) -> torch.Tensor:
+         num_pages: int = 0, rows: Optional[torch.Tensor] = None, counts: Optional[torch.Tensor] = None,
+         mask: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Positions of the k largest logits among each token's visible keys, ties to the lower position, ascending
     position order, -1 padding; out int32 [T,k] or [T,1,k] (patch_dsv32_indexer.py:133-146).
     single_workgroup=True runs the variant that needs no scratch memory (one workgroup per token).
     With block_table / num_pages / rows [T,k] / counts [T] the same launch also fills the flat cache rows and the pick
-    counts that build_sparse_rows would produce from `out`."""
-    _need_cuda(logits, seq_lens, out)
+    counts that build_sparse_rows would produce from `out`.  With mask (int32 [T, W], without rows) it also fills the picks as
+    bits: bit j % 32 of mask[t, j // 32] for every key j that token t sees (bits behind those mean nothing)."""
+    _need_cuda(logits, seq_lens, out, mask)
     lib = _lib.load()
     o2 = out.reshape(out.shape[0], -1) if out.dim() == 3 else out
     if o2.data_ptr() != out.data_ptr():
@@ -683,6 +686,14 @@ def topk(logits: torch.Tensor, seq_lens: torch.Tensor, k: int, out: torch.Tensor
                                num_pages, rows.data_ptr(), rows.stride(0), counts.data_ptr(), ws_ptr, ws_bytes,
                                _stream(logits))
         _lib.check(rc, "dsa_topk_rows")
+        return out
+    if mask is not None:
+        if mask.dtype != torch.int32 or mask.dim() != 2 or mask.shape[0] < o2.shape[0] or mask.stride(1) != 1 or \
+                mask.shape[1] * 32 < logits.shape[1]:
+            raise TypeError("topk: mask must be int32 [T, W] with contiguous rows of a bit per logit")
+        rc = lib.dsa_topk_mask(logits.data_ptr(), logits.stride(0), seq_lens.data_ptr(), qsl, b, q_len, k, o2.data_ptr(),
+                               o2.stride(0), mask.data_ptr(), mask.stride(0) * 4, ws_ptr, ws_bytes, _stream(logits))
+        _lib.check(rc, "dsa_topk_mask")
         return out
     rc = lib.dsa_topk(logits.data_ptr(), logits.stride(0), seq_lens.data_ptr(), qsl, b, q_len, k, o2.data_ptr(),
                       o2.stride(0), ws_ptr, ws_bytes, _stream(logits))
@@ -798,7 +809,8 @@ _PREFILL_KV_F16 = 16                                       # added to the output
 def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tensor, k_pe: torch.Tensor, v: torch.Tensor,
                    cu_q: torch.Tensor, cu_k: torch.Tensor, max_q_len: int, scale: float, causal: bool,
                    out: torch.Tensor, lse_out: Optional[torch.Tensor] = None, window: Optional[int] = None,
-                   prev_out: Optional[torch.Tensor] = None, prev_lse: Optional[torch.Tensor] = None) -> torch.Tensor:
+                   prev_out: Optional[torch.Tensor] = None, prev_lse: Optional[torch.Tensor] = None,
+                   pick: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Varlen non-absorbed MLA attention (reference: the prefill FIA calls, src/omni_npu/attention/backends/mla.py:574-590
     and :415-431).  q_nope [T,N,128], q_pe [T,N,64], k_nope [Tk,N,128], k_pe [Tk,64] (shared by the heads), v [Tk,N,128],
     cu_q / cu_k int32 [B+1] device tensors, out [T,N,128] bf16 or fp32, lse_out fp32 [T,N].  ``window`` keeps only the
@@ -807,7 +819,9 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
     rows; the call then returns the attention over the union, i.e. what this attention followed by merge_attn_states
     (src/omni_npu/attention/ops.py:5-42) gives, in one launch.  ``out`` may be ``prev_out``.
     k_nope, k_pe and v may all three be fp16 (a caller that makes them with an fp16 GEMM): both products then run on fp16
-    and the kernel skips the conversion of the value tiles it otherwise does (the queries stay bf16)."""
+    and the kernel skips the conversion of the value tiles it otherwise does (the queries stay bf16).
+    ``pick`` (int32 [T, W] bits, see topk's mask; W even and wide enough for the longest sequence; fp16 keys and values, no
+    window, no earlier result): a token attends over the keys its bits name."""
     if window is not None and window < 1:
         raise ValueError(f"prefill_varlen: window must be positive (got {window})")
     _need_cuda(q_nope, q_pe, k_nope, k_pe, v, cu_q, cu_k, out, lse_out)
@@ -836,6 +850,12 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
         if prev_out.dtype != torch.float32 or prev_out.shape != (t, n, 128) or prev_out.stride(-1) != 1 or \
                 prev_lse.dtype != torch.float32 or prev_lse.numel() != t * n or not prev_lse.is_contiguous():
             raise TypeError("prefill_varlen: prev_out must be fp32 [T,N,128], prev_lse contiguous fp32 [T,N]")
+    if pick is not None:
+        _need_cuda(pick)
+        if pick.dtype != torch.int32 or pick.dim() != 2 or pick.shape[0] < t or pick.shape[1] % 2 or pick.stride(1) != 1 or \
+                window is not None or prev_out is not None or not kv_half:
+            raise TypeError("prefill_varlen: pick must be int32 [T, W] (W even, rows contiguous), with fp16 keys and values, "
+                            "without a window or an earlier result")
     if k_nope.shape[0] == 0 or t == 0:
         # no keys at all (a context chunk in which every sequence is empty): zeros and lse = -inf, as the kernel gives for
         # an empty key range (the earlier result itself when there is one); empty tensors have no address to hand over
@@ -858,6 +878,15 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
             lse_out.data_ptr() if lse_out is not None else None, prev_out.data_ptr(), prev_out.stride(0), prev_out.stride(1),
             prev_lse.data_ptr(), _stream(q_nope))
         _lib.check(rc, "mla_prefill_varlen_continue")
+        return out
+    if pick is not None:
+        rc = lib.mla_prefill_varlen_pick(
+            q_nope.data_ptr(), q_nope.stride(0), q_nope.stride(1), q_pe.data_ptr(), q_pe.stride(0), q_pe.stride(1),
+            k_nope.data_ptr(), k_nope.stride(0), k_nope.stride(1), k_pe.data_ptr(), k_pe.stride(0), v.data_ptr(), v.stride(0),
+            v.stride(1), cu_q.data_ptr(), cu_k.data_ptr(), cu_q.numel() - 1, n, int(max_q_len), 1 if causal else 0, float(scale),
+            pick.data_ptr(), pick.stride(0), pick.shape[1], out.data_ptr(), out.stride(0), out.stride(1),
+            _DT[out.dtype] | kv_code, lse_out.data_ptr() if lse_out is not None else None, _stream(q_nope))
+        _lib.check(rc, "mla_prefill_varlen_pick")
         return out
     rc = lib.mla_prefill_varlen(q_nope.data_ptr(), q_nope.stride(0), q_nope.stride(1), q_pe.data_ptr(), q_pe.stride(0),
                                 q_pe.stride(1), k_nope.data_ptr(), k_nope.stride(0), k_nope.stride(1), k_pe.data_ptr(),

@@ -51,7 +51,6 @@ class NPUDeepseekSparseAttention(torch.nn.Module):
         latent = self.kv_a_proj_with_mqa(hidden_states)[0]
         q = self.q_b_proj(q_lora)[0].view(-1, self.num_local_heads, self.qk_head_dim)
         t, dev = q.shape[0], q.device
-        ql_nope = torch.bmm(q[..., :self.qk_nope_head_dim].transpose(0, 1), impl.W_UK_T).transpose(0, 1)
         q_pe = q[..., self.qk_nope_head_dim:]                   # rotated in place by the fused launches below
         out = torch.empty(t, self.num_local_heads * self.v_head_dim, dtype=q.dtype, device=dev)
         if meta is None:
@@ -63,18 +62,27 @@ class NPUDeepseekSparseAttention(torch.nn.Module):
             return self.o_proj(out.fill_(0))[0]
         kv_cache = self.attn.kv_cache[ctx.virtual_engine]
         assert len(kv_cache) == 3, f"{len(kv_cache)=}."
+        select = getattr(self.indexer, "select", self.indexer)
+        kv_a = k_pe = None
+        if meta.prefill is not None:                            # prompts may attend over their own rows (_forward_prompts)
+            impl.offer_masked_prompts(select)
+            kv_a = torch.empty(t, self.kv_lora_rank, dtype=q.dtype, device=dev)
+            k_pe = torch.empty(t, self.qk_rope_head_dim, dtype=q.dtype, device=dev)
         K.kv_rmsnorm_rope_cache(latent, self.kv_a_layernorm.weight, cos, sin, meta.slot_mapping, kv_cache[0], kv_cache[1],
-                                eps=self._eps(), q_rope=q_pe)
+                                eps=self._eps(), kv_a_out=kv_a, k_pe_out=k_pe, q_rope=q_pe)
         topk_indices = self.indexer.forward_tables(hidden_states, q_lora, cos, sin, meta, kv_cache)[0]
+        pick = select.mask_for(meta) if hasattr(select, "mask_for") else None
         if meta.prefill is not None:
             p = meta.prefill
+            if impl._forward_prompts(q, kv_a, k_pe, p, pick, out):
+                return self.o_proj(out)[0]
             part, lens, q_len, qsl = p, p.kv_lens, p.max_query_len, p.query_start_loc.to(torch.int32).contiguous()
         else:
             d = meta.decode
             part, lens, q_len, qsl = d, d.seq_lens, d.q_len, d.query_start_loc
+        ql_nope = torch.bmm(q[..., :self.qk_nope_head_dim].transpose(0, 1), impl.W_UK_T).transpose(0, 1)
         fused = out if impl._fusable_w_uv(out) else None
-        select = getattr(self.indexer, "select", self.indexer)
-        rc = select.rows_for(meta) if hasattr(select, "rows_for") else None
+        rc = select.rows_for(meta) if pick is None and hasattr(select, "rows_for") else None
         attn_out = impl._apply_sparse_attention(ql_nope, q_pe, kv_cache, part, lens, q_len, qsl, topk_indices[:t],
                                                 proj_out=fused, rows_counts=None if rc is None else (rc[0][:t], rc[1][:t]))
         if fused is None:

@@ -322,3 +322,43 @@ def test_graph_wrapper_options_act_on_the_capture(dev):
                 y, ssum = w(x)
                 torch.cuda.synchronize()
                 assert torch.equal(y, x * 2 + 1) and torch.equal(ssum, x.float().sum(dim=-1))
+
+
+@pytest.mark.parametrize("q_lens", [[300], [1, 1, 129, 70, 300]])
+def test_dsa_prompts_attend_over_their_own_keys_with_the_picks_as_a_mask(dev, q_lens):
+    """With a plain up-projection weight, prompts without cached tokens go through the prefill kernel with the picks as
+    bits; the same step over gathered latents (no pair count allowed): same picks, same attention within the bar of two
+    bf16 results (each within 2e-3 of the exact one)."""
+    g = torch.Generator().manual_seed(sum(q_lens))
+    n, topk = 16, 64
+    seq_lens = [q if q > 1 else 400 for q in q_lens]
+    common = _common(q_lens, seq_lens)
+    t = common.num_actual_tokens
+    nblk = int(common.block_table_tensor.max()) + 1
+    common.slot_mapping = torch.cat([O.slots_for(common.block_table_tensor, b, s - ql, s)
+                                     for b, (ql, s) in enumerate(zip(q_lens, seq_lens))])
+    raw = torch.randn(nblk * 128 * 704, generator=g).bfloat16().to(dev).view(torch.uint8)
+    kv_cache = dsa.NPUDSABackend.reshape_kv_cache(raw, nblk, 128, 1, 704, dtype=torch.bfloat16)
+    k8v, ksv = dsa.indexer_cache_views(kv_cache[2])
+    k8_ref, ks_ref = O.fp8_quant_token(torch.randn(nblk, 128, 128, generator=g))
+    k8v.copy_(k8_ref.view(torch.uint8)); ksv.copy_(ks_ref)
+    indexer = dsa.LightningIndexer(topk, max_tokens=t, device=dev)
+    impl, w = _mk_impl(dsa.NPUDSAImpl, n, dev, indexer=indexer)
+    impl.kv_b_proj = _PlainLinear(w, dev)
+    impl.process_weights_after_loading(torch.bfloat16)
+    assert indexer.masked_pairs_per_pick > 0
+    meta = dsa.NPUDSAMetadataBuilder(V.AttentionSpec(128, 1, 704, torch.bfloat16), ["l"], _cfg(cap=1), dev).build(0, _to(common, dev))
+    a = [x.to(dev) for x in (torch.randn(t, n, 192, generator=g).bfloat16(), torch.randn(t, 512, generator=g).bfloat16(),
+                             torch.randn(t, 1, 64, generator=g).bfloat16())]
+    i = [x.to(dev) for x in (torch.randn(t, 64, 128, generator=g).bfloat16(), torch.randn(t, 128, generator=g).bfloat16(),
+                             torch.randn(t, 64, generator=g).bfloat16())]
+    got = []
+    for pairs in (1000.0, 0.0):
+        indexer.masked_pairs_per_pick = pairs
+        indexer(*i, kv_cache, meta)
+        assert (indexer.mask_for(meta) is not None) == (pairs > 0)
+        out = torch.zeros(t, n * 128, dtype=torch.bfloat16, device=dev)
+        impl.forward(None, *a, kv_cache, meta, output=out)
+        got.append((indexer.topk_indices_buffer[:t].clone(), out))
+    assert torch.equal(got[0][0], got[1][0])
+    attn_close(got[0][1], got[1][1], 3e-2, 4e-3 + 4e-3)        # (the latent form also rounds absorbed queries and outputs to bf16)

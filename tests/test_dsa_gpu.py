@@ -386,3 +386,77 @@ def test_sparse_decode_method_choice_and_refusals(dev):
     K.sparse_decode(*args, rows.to(dev), cnt.to(dev), c["scale"], out)          # auto -> the split form
     ref = O.sparse_decode(c["q_nope"], c["q_rope"], c["nope"], c["rope"], c["block_table"], c["seq_lens"], idx, c["scale"])
     attn_close(out, ref, 2e-2, 2e-3)
+
+
+@pytest.mark.parametrize("q_lens,extra", [([16], 0), ([17, 40], 0), ([33, 1, 130], 200), ([300], 1000)])
+def test_prompt_scores_are_the_streaming_kernels_bits(dev, q_lens, extra):
+    """Requests of 16 tokens and more take the kernel that keeps eight tokens' queries in LDS.  Every token once more as a
+    request of its own (the streaming kernel): the same logits bit for bit, ragged lengths and last groups included."""
+    from omni_npu_amd import kernels as K
+    g = torch.Generator().manual_seed(sum(q_lens))
+    lens = [q + extra for q in q_lens]
+    nblk = [(n + 127) // 128 for n in lens]
+    bt = torch.zeros(len(lens), max(nblk), dtype=torch.int32)
+    perm, o = torch.randperm(sum(nblk), generator=g).int(), 0
+    for b, n in enumerate(nblk):
+        bt[b, :n] = perm[o:o + n]
+        o += n
+    k8, ks = O.fp8_quant_token(torch.randn(sum(nblk), 128, 128, generator=g))
+    t = sum(q_lens)
+    q8, qs = O.fp8_quant_token(torch.randn(t, 64, 128, generator=g))
+    w = torch.randn(t, 64, generator=g)
+    d = lambda x: x.to(dev)
+    stride = K.indexer_logits_stride(max(lens))
+    lg, ref = torch.full((t, stride), 7.0, device=dev), torch.full((t, stride), 7.0, device=dev)
+    qsl = torch.tensor([0] + q_lens).cumsum(0).int()
+    K.indexer_scores(d(q8), d(w), d(k8), d(ks), d(bt), d(torch.tensor(lens).int()), lg, q_len=max(q_lens), q_scale=d(qs),
+                     query_start_loc=d(qsl), max_seq_len=max(lens))
+    seen = torch.cat([torch.arange(n - q + 1, n + 1) for q, n in zip(q_lens, lens)]).int()
+    req = torch.repeat_interleave(torch.arange(len(lens)), torch.tensor(q_lens))
+    K.indexer_scores(d(q8), d(w), d(k8), d(ks), d(bt[req].contiguous()), d(seen), ref, q_scale=d(qs), max_seq_len=max(lens))
+    assert torch.equal(lg, ref)
+    # without the tokens that see at most `skip` keys: the others' rows are the same
+    skip = max(lens) - 10
+    lg2 = torch.full((t, stride), 7.0, device=dev)
+    K.indexer_scores(d(q8), d(w), d(k8), d(ks), d(bt), d(torch.tensor(lens).int()), lg2, q_len=max(q_lens), q_scale=d(qs),
+                     query_start_loc=d(qsl), max_seq_len=max(lens), skip_up_to=skip)
+    far = d(seen > skip)
+    assert torch.equal(lg2[far], ref[far])
+
+
+@pytest.mark.parametrize("t,n,k", [(1, 40, 64), (3, 65, 64), (300, 700, 64), (5, 9000, 2048), (257, 9001, 2048)])
+def test_topk_mask_names_the_picks(dev, t, n, k):
+    """dsa_topk_mask: the bits of the visible positions are the index list, in the one-workgroup and the sliced variant."""
+    from omni_npu_amd import kernels as K
+    g = torch.Generator().manual_seed(t + n)
+    stride = (n + 63) // 64 * 64
+    lg = torch.randn(t, stride, generator=g).to(dev)
+    lens = torch.tensor([n], dtype=torch.int32, device=dev)
+    out, plain = torch.empty(t, k, dtype=torch.int32, device=dev), torch.empty(t, k, dtype=torch.int32, device=dev)
+    mask = torch.randint(-2 ** 31, 2 ** 31 - 1, (t, stride // 32), generator=g).int().to(dev)
+    K.topk(lg, lens, k, out, q_len=t, mask=mask)
+    K.topk(lg, lens, k, plain, q_len=t)
+    assert torch.equal(out, plain)
+    bits = (mask.cpu().view(t, -1, 1) >> torch.arange(32).view(1, 1, -1) & 1).view(t, -1)
+    for i in range(t):
+        vis = n - t + i + 1
+        want = torch.zeros(vis, dtype=torch.int32)
+        p = plain[i].cpu()
+        want[p[p >= 0].long()] = 1
+        assert torch.equal(bits[i, :vis].int(), want)
+
+
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 70])
+def test_quant_rows_of_unaligned_sources(dev, rows):
+    """Rows that start on 4-byte boundaries only, and targets on 2-byte ones, against aligned ones: the same bytes."""
+    from omni_npu_amd import kernels as K
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, 130, generator=g).bfloat16().to(dev)
+    a8, s_a = torch.zeros(rows, 128, dtype=torch.uint8, device=dev), torch.zeros(rows, device=dev)
+    b8, s_b = torch.zeros(rows, 130, dtype=torch.uint8, device=dev), torch.zeros(rows, device=dev)
+    K.quant_rows_fp8(x[:, 2:], a8, s_a)
+    slots = torch.arange(rows, device=dev)
+    K.quant_rows_fp8(x[:, 2:].contiguous(), b8.view(1, rows, 130)[..., 2:], s_b.view(1, rows), slot_mapping=slots)
+    ref8, ref_s = O.fp8_quant_token(x[:, 2:].float().cpu())
+    assert torch.equal(a8.cpu(), ref8.view(torch.uint8)) and torch.equal(s_a.cpu(), ref_s.view(-1))
+    assert torch.equal(b8[:, 2:].cpu(), ref8.view(torch.uint8)) and torch.equal(s_b.cpu(), ref_s.view(-1))

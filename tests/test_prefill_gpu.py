@@ -359,3 +359,33 @@ def test_rows_f16_and_fp16_gathers_round_like_torch(dev, rows):
         gather(plain)
         gather(half)
         assert torch.equal(half, plain.half())
+
+
+@pytest.mark.parametrize("q_lens,density", [([1], 1.0), ([63, 64, 65], 0.5), ([200, 129], 0.1), ([400], 0.02)])
+def test_prefill_over_picked_keys(dev, q_lens, density):
+    """Causal attention over the keys that a token's bits name (the first visible key always among them), bits behind the
+    causal limit set at random: against fp32 attention with the same mask."""
+    from omni_npu_amd import kernels as K
+    g = torch.Generator().manual_seed(sum(q_lens))
+    n, t, scale = 3, sum(q_lens), 192 ** -0.5
+    q = torch.randn(t, n, 192, generator=g).bfloat16()
+    kv, pe = torch.randn(t, n, 256, generator=g).half(), torch.randn(t, 64, generator=g).half()
+    width = (max(q_lens) + 63) // 64 * 64
+    on = torch.rand(t, width, generator=g) < density
+    on[:, 0] = True
+    words = (on.view(t, -1, 32).long() << torch.arange(32)).sum(-1)
+    pick = torch.where(words >= 2 ** 31, words - 2 ** 32, words).int()
+    cu = torch.tensor([0] + q_lens).cumsum(0).int()
+    out, lse = torch.empty(t, n, 128, dtype=torch.bfloat16, device=dev), torch.empty(t, n, device=dev)
+    d = lambda x: x.to(dev)
+    K.prefill_varlen(d(q)[..., :128], d(q)[..., 128:], d(kv)[..., :128], d(pe), d(kv)[..., 128:], d(cu), d(cu), max(q_lens), scale,
+                     True, out, lse, pick=d(pick))
+    ref, ref_lse = torch.empty(t, n, 128), torch.empty(t, n)
+    for a, e in zip(cu[:-1].tolist(), cu[1:].tolist()):
+        s = (torch.einsum("inp,jnp->nij", q[a:e, :, :128].float(), kv[a:e, :, :128].float())
+             + torch.einsum("inp,jp->nij", q[a:e, :, 128:].float(), pe[a:e].float())) * scale
+        s = s.masked_fill(~(on[a:e, :e - a] & torch.ones(e - a, e - a).tril().bool()), float("-inf"))
+        ref[a:e] = torch.einsum("nij,jnv->inv", s.softmax(-1), kv[a:e, :, 128:].float())
+        ref_lse[a:e] = s.logsumexp(-1).t()
+    attn_close(out, ref, 2e-2, 2e-3)
+    assert torch.allclose(lse.cpu(), ref_lse, atol=2e-2, rtol=1e-3)
