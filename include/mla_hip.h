@@ -363,6 +363,15 @@ int dsa_quant_qk_fp8(const void* q, int64_t q_stride, int64_t q_rows, void* q8, 
                      int64_t cache_page_stride_bytes, int64_t cache_row_stride_bytes, float* scale_cache,
                      int64_t scale_page_stride, int32_t page_size, int64_t num_pages, mlahip_stream_t stream);
 
+/* The same for query rows r = token * heads + head, with the indexer's head weights [tokens, heads] (bf16, or fp32 with w_f32;
+ * w_stride elements from token to token) instead of the plain query scales: w_out[r] = weight * scale of row r, the weights
+ * that dsa_indexer_scores_fp8 takes. */
+int dsa_quant_qkw_fp8(const void* q, int64_t q_stride, int64_t q_rows, void* q8, const void* weights, int32_t w_f32,
+                      int64_t w_stride, int32_t heads, float* w_out, const void* k, int64_t k_stride, int64_t k_rows,
+                      const int64_t* slot_mapping, void* k8_cache, int64_t cache_page_stride_bytes,
+                      int64_t cache_row_stride_bytes, float* scale_cache, int64_t scale_page_stride, int32_t page_size,
+                      int64_t num_pages, mlahip_stream_t stream);
+
 /* With a workspace of dsa_topk_workspace_bytes() the selection of a token is spread over several workgroups (three
  * launches that meet in the workspace: slice histograms, boundary-bin gather, ordered write), which is what a
  * decode step with few tokens and long rows needs; with workspace == NULL one workgroup per token does everything and

@@ -16,6 +16,7 @@ from typing import ClassVar, Optional, Tuple
 
 import torch
 
+from ... import _host
 from ... import kernels as K
 from .mla import HalfUpProjection, _caller_wrote_cache, _persistent_int32
 from ..._vllm_compat import (PAD_SLOT_ID, AttentionCGSupport, AttentionType, MLACommonBackend, MLACommonBaseImpl,
@@ -188,8 +189,11 @@ class LightningIndexer:
         if attn_metadata is None:                                   # profile run (patch_dsv32_indexer.py:104-112)
             return self.topk_indices_buffer
         assert len(kv_cache) >= 3, f"Expected kv_cache to have at least 3 elements, but got {len(kv_cache)}"
-        k8, ks = indexer_cache_views(kv_cache[2])
         t = q.shape[0]
+        if attn_metadata.num_prefills == 0 and attn_metadata.num_decodes > 0 and self._native_select(q, k, weights, kv_cache[2],
+                                                                                                     attn_metadata):
+            return self.topk_indices_buffer[:t].view(t, 1, self.topk_tokens)
+        k8, ks = indexer_cache_views(kv_cache[2])
         q8 = torch.empty(t, self.n_head, self.head_dim, dtype=torch.uint8, device=q.device)
         qs = torch.empty(t, self.n_head, dtype=torch.float32, device=q.device)
         # the new keys into the cache and the queries into plain buffers: one launch
@@ -214,14 +218,7 @@ class LightningIndexer:
             if masked:                                              # (the longest prompt, not the longest the server takes)
                 max_len = min(max_len, (q_len + 63) // 64 * 64)
             stride = K.indexer_logits_stride(max_len)
-            if self._logits is None or self._logits.shape[0] < ntok or self._logits.shape[1] < stride:
-                if self._logits is not None:
-                    self._logits_kept.append(self._logits)
-                    ntok_a, stride_a = max(ntok, self._logits.shape[0]), max(stride, self._logits.shape[1])
-                else:
-                    ntok_a, stride_a = max(ntok, 1), stride
-                self._logits = torch.empty(ntok_a, stride_a, dtype=torch.float32, device=q.device)
-            lg = self._logits[:ntok, :stride]
+            lg = self._scores_buffer(ntok, stride, q.device)
             sl = slice(off, off + ntok)
             if not masked or q_len > self.topk_tokens:              # (else every token takes all the keys it sees)
                 K.indexer_scores(q8[sl], w[sl], k8, ks, meta.block_table, lens, lg, q_len=q_len, q_scale=qs[sl],
@@ -237,6 +234,31 @@ class LightningIndexer:
                 self._rows_meta = attn_metadata
             off += ntok
         return out.view(t, 1, self.topk_tokens)
+
+    def _scores_buffer(self, ntok: int, stride: int, device) -> torch.Tensor:
+        if self._logits is None or self._logits.shape[0] < ntok or self._logits.shape[1] < stride:
+            rows, cols = max(ntok, 1), stride
+            if self._logits is not None:
+                self._logits_kept.append(self._logits)
+                rows, cols = max(rows, self._logits.shape[0]), max(cols, self._logits.shape[1])
+            self._logits = torch.empty(rows, cols, dtype=torch.float32, device=device)
+        return self._logits[:ntok, :stride]
+
+    def _native_select(self, q, k, weights, index_cache, attn_metadata) -> bool:
+        """The selection of a step of decode tokens in one native call; False, with nothing done, where that call does not
+        know the case."""
+        d, ntok = attn_metadata.decode, attn_metadata.num_decode_tokens
+        if not q.is_cuda or self.n_head != 64 or self.head_dim != INDEX_HEAD_DIM or q.dim() != 3:
+            return False
+        max_len = d.block_table.shape[1] * index_cache.shape[1]
+        lg = self._scores_buffer(ntok, K.indexer_logits_stride(max_len), q.device)
+        self._rows_meta = self._mask_meta = self._mask = None
+        if not _host.load().dsa_select(q, k, weights, index_cache, attn_metadata.slot_mapping, d.block_table, d.seq_lens,
+                                       d.query_start_loc, ntok, d.q_len, max_len, self.topk_tokens, lg,
+                                       self.topk_indices_buffer, self.rows_buffer, self.counts_buffer):
+            return False
+        self._rows_meta = attn_metadata
+        return True
 
     def mask_for(self, attn_metadata):
         """The picks of the step's prompt tokens as bits [T, W] (kernels.topk's mask) if the last selection made them for this
@@ -384,9 +406,12 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
         written = _caller_wrote_cache(self, attn_metadata, num_actual_toks)
         if not written:                                            # (else the caller's fused norm + rope launch wrote them)
             K.cache_write(k_c_normed, k_pe, attn_metadata.slot_mapping, k_nope, k_rope)
-        topk = self.indexer.topk_indices_buffer
         rows_for = getattr(self.indexer, "rows_for", None)
         rc = rows_for(attn_metadata) if rows_for is not None else None
+        if has_decode and not has_prefill and rc is not None and _host.load().sparse_decode(
+                q, k_nope, k_rope, rc[0], rc[1], self.W_UK_T, self.W_UV, self.scale, ndt, output):
+            return output_padded
+        topk = self.indexer.topk_indices_buffer
         part = lambda a, b: None if rc is None else (rc[0][a:b], rc[1][a:b])
 
         if has_prefill:

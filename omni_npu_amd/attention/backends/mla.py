@@ -19,6 +19,7 @@ from typing import ClassVar, Optional, Tuple
 
 import torch
 
+from ... import _host
 from ... import kernels as K
 from ..._vllm_compat import (AttentionCGSupport, AttentionType, MLACommonBackend, MLACommonBaseImpl,
                              MLACommonDecodeMetadata, MLACommonMetadata, MLACommonMetadataBuilder,
@@ -472,6 +473,17 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
             K.decode(ql_nope, q_pe, kv_cache[0], kv_cache[1], d.block_table, d.seq_lens, self.scale, out, **kw)
         return o
 
+    def _native_decode(self, q, kv_cache, attn_metadata, output) -> bool:
+        """The decode tokens' absorption, attention and merge + up-projection into ``output`` in one native call.  False, with
+        nothing done, where that call does not know the case."""
+        d = attn_metadata.decode
+        if self.sink_len > 0 and (self.sliding_window is None or self.sink_len % K.PAGE != 0):
+            return False
+        return _host.load().mla_decode(
+            q, kv_cache[0], None if self.fp8_cache else kv_cache[1], d.block_table, d.seq_lens, d.query_start_loc, d.q_len,
+            d.block_table.shape[1] * K.PAGE, self.W_UK_T, self.W_UV, self.scale, attn_metadata.num_decode_tokens, self.sink_len,
+            self.sliding_window if self.sink_len > 0 else 0, output)
+
     def forward(self, layer, q: torch.Tensor, k_c_normed: torch.Tensor, k_pe: torch.Tensor,
                 kv_cache: Tuple[torch.Tensor, ...], attn_metadata: NPUMLAMetadata,
                 output: Optional[torch.Tensor] = None, output_scale: Optional[torch.Tensor] = None,
@@ -499,7 +511,6 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
         has_decode = attn_metadata.num_decodes > 0
         has_prefill = attn_metadata.num_prefills > 0
         num_decode_tokens = attn_metadata.num_decode_tokens
-        decode_q = q[:num_decode_tokens]
 
         # write the latent and rope rows of the new tokens (one launch), unless the caller's fused norm + rope launch has
         # put them there already and said so for this very metadata object
@@ -522,9 +533,9 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
             if got.data_ptr() != dst.data_ptr():
                 dst.copy_(got)
 
-        if has_decode:
+        if has_decode and not self._native_decode(q, kv_cache, attn_metadata, output):
             assert attn_metadata.decode is not None
-            decode_q_nope, decode_q_pe = decode_q.split([self.qk_nope_head_dim, self.qk_rope_head_dim], dim=-1)
+            decode_q_nope, decode_q_pe = q[:num_decode_tokens].split([self.qk_nope_head_dim, self.qk_rope_head_dim], dim=-1)
             # (B, N, P) -> (N, B, P) x (N, P, L) -> (N, B, L) -> (B, N, L) view
             decode_ql_nope = torch.bmm(decode_q_nope.transpose(0, 1), self.W_UK_T).transpose(0, 1)
             ndt = decode_ql_nope.shape[0]

@@ -1,0 +1,334 @@
+// The host side of a decode step in native code: one call from Python per layer and stage.
+//
+// What bounds a small step is not the GPU: through the general Python front end (kernels.py: shape checks, forty pointer and
+// stride look-ups, a ctypes call per launch) one layer of one user took 65 us of host time around 25 us of kernels, and a
+// sparse decode layer 187 us around 142.  The functions here do the checks, the scratch look-up, the library GEMM and the
+// launches of a whole stage.  Each answers false, with nothing launched, when an argument is not what it knows; the caller
+// then takes the general path, which handles the case or says what is wrong with it.  A failing launch raises.
+//
+// Contracts: mla_decode / sparse_decode = NPUMLAImpl.forward / NPUDSAImpl.forward for a step's decode tokens
+// (src/omni_npu/attention/backends/mla.py:868-912, dsa.py:359-389), dsa_select = LightningIndexer for them
+// (src/omni_npu/vllm_patches/patches/models/deepseek/patch_dsv32_indexer.py:104-146), norm_rope_cache =
+// kernels.kv_rmsnorm_rope_cache (src/omni_npu/v1/layers/attention/npu_mla.py:196-210).
+#include <torch/extension.h>
+#include <ATen/core/LegacyTypeDispatch.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+
+#include <map>
+#include <mutex>
+#include <optional>
+#include <utility>
+
+#include "../../../include/mla_hip.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+
+constexpr int64_t kNope = 512, kRope = 64, kPage = 128, kFp8Row = 656, kVDim = 128;
+constexpr int64_t kVupMaxTokens = 256;      // kernels.VUP_MAX_TOKENS: beyond, a separate merge and the library GEMM
+
+void check(int rc, const char* what) {
+  if (rc != 0) throw std::runtime_error(std::string(what) + " failed with code " + std::to_string(rc) + ": " + mlahip_last_error_string());
+}
+
+bool is(const Tensor& t, at::ScalarType dt, int64_t dim, const at::Device& dev) {
+  return t.scalar_type() == dt && t.dim() == dim && t.device() == dev && (t.size(-1) <= 1 || t.stride(-1) == 1);
+}
+bool is_bf16(const Tensor& t, int64_t dim, const at::Device& dev) { return is(t, at::kBFloat16, dim, dev); }
+bool is_i32(const Tensor& t, int64_t dim, const at::Device& dev) { return is(t, at::kInt, dim, dev); }
+
+// The GPU the tensors live on if it is the current one.
+bool current_gpu(const Tensor& t) { return t.is_cuda() && t.get_device() == c10::hip::current_device(); }
+
+using Stream = mlahip_stream_t;
+Stream stream_of(const Tensor& t) { return (Stream)c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+
+// Scratch memory comes from kernels._workspace, which keeps buffers per (device, stream, tag) and never frees one; what it
+// handed out is remembered here and asked for again only when it is too small.
+PyObject* g_workspace = nullptr;
+std::map<std::tuple<int, Stream, int>, Tensor> g_scratch;      // (guarded by the GIL, as the Python side is)
+Tensor& scratch(const Tensor& like, Stream stream, int64_t bytes, int tag) {
+  static const char* const names[] = {"decode", "topk"};
+  Tensor& t = g_scratch[{like.get_device(), stream, tag}];
+  if (!t.defined() || t.numel() < bytes) t = py::cast<Tensor>(py::handle(g_workspace)(like.device(), bytes, names[tag]));
+  return t;
+}
+
+int64_t div_up(int64_t a, int64_t b) { return (a + b - 1) / b; }
+// kernels.default_num_splits
+int default_splits(int64_t batch, int64_t q_len, int64_t heads, int64_t max_seq_len) {
+  const int64_t groups = std::max<int64_t>(batch * div_up(q_len * heads, 128), 1);
+  const int64_t by_length = std::max<int64_t>(1, div_up(max_seq_len, 256));
+  return (int)std::max<int64_t>(1, std::min({std::max<int64_t>(1, div_up(256, groups)), by_length, (int64_t)256}));
+}
+
+struct Cache {
+  const Tensor *nope = nullptr, *rope = nullptr;   // fp8: nope is the 656-byte-row cache and rope is null
+  int64_t n_sp = 0, n_sr = 0, r_sp = 0, r_sr = 0, pages = 0, page = 0;
+};
+// [nblk, page, (1,) width] bf16 pair, or [nblk, 128, 656] uint8
+bool cache_of(const Tensor& nope, const OptTensor& rope, const at::Device& dev, Cache& c) {
+  c.nope = &nope;
+  c.pages = nope.size(0);
+  c.n_sp = nope.stride(0);
+  if (nope.dim() < 3 || nope.device() != dev || c.pages < 1) return false;
+  c.page = nope.size(1);
+  c.n_sr = nope.stride(1);
+  if (!rope) return nope.scalar_type() == at::kByte && nope.dim() == 3 && c.page == kPage && nope.size(2) == kFp8Row && nope.stride(2) == 1;
+  const Tensor& r = *rope;
+  if ((nope.dim() == 4 && nope.size(2) != 1) || nope.dim() > 4 || nope.scalar_type() != at::kBFloat16 || nope.size(-1) != kNope ||
+      nope.stride(-1) != 1 || r.dim() != nope.dim() || (r.dim() == 4 && r.size(2) != 1) || r.scalar_type() != at::kBFloat16 ||
+      r.size(-1) != kRope || r.stride(-1) != 1 || r.device() != dev || r.size(0) != c.pages || r.size(1) != c.page)
+    return false;
+  c.rope = &r;
+  c.r_sp = r.stride(0);
+  c.r_sr = r.stride(1);
+  return true;
+}
+
+// kernels.cache_write / cache_write_fp8: the step's latent and rope rows to their slots.
+bool cache_write(const Tensor& kv_c, const Tensor& k_pe, const Tensor& slots, const Tensor& nope, const OptTensor& rope) {
+  if (!current_gpu(kv_c)) return false;
+  const at::Device dev = kv_c.device();
+  Cache c;
+  if (!is_bf16(kv_c, 2, dev) || kv_c.size(1) != kNope || k_pe.scalar_type() != at::kBFloat16 || k_pe.device() != dev ||
+      k_pe.size(-1) != kRope || k_pe.stride(-1) != 1 || !(k_pe.dim() == 2 || (k_pe.dim() == 3 && k_pe.size(1) == 1)) ||
+      slots.scalar_type() != at::kLong || slots.dim() != 1 || !slots.is_contiguous() || slots.device() != dev ||
+      !cache_of(nope, rope, dev, c))
+    return false;
+  const int64_t t = std::min(slots.numel(), kv_c.size(0));
+  if (t < 1 || k_pe.size(0) < t) return false;
+  Stream st = stream_of(kv_c);
+  if (c.rope)
+    check(mla_cache_write_bf16(kv_c.data_ptr(), kv_c.stride(0), k_pe.data_ptr(), k_pe.stride(0), (const int64_t*)slots.data_ptr(),
+                               (int)t, c.nope->data_ptr(), c.n_sp, c.n_sr, c.rope->data_ptr(), c.r_sp, c.r_sr, (int)c.page,
+                               c.pages, st), "mla_cache_write_bf16");
+  else
+    check(mla_cache_write_fp8(kv_c.data_ptr(), kv_c.stride(0), k_pe.data_ptr(), k_pe.stride(0), (const int64_t*)slots.data_ptr(),
+                              (int)t, c.nope->data_ptr(), c.n_sp, c.n_sr, (int)c.page, c.pages, st), "mla_cache_write_fp8");
+  return true;
+}
+
+// What both decode forms need of the layer: q [T, N, 192], W_UK_T [N, 128, 512], W_UV [N, 512, 128], out [T, N * 128].
+bool layer_ok(const Tensor& q, const Tensor& w_uk, const Tensor& w_uv, const Tensor& out, int64_t t, const at::Device& dev) {
+  if (!is_bf16(q, 3, dev) || t < 1 || q.size(0) < t || q.size(2) != 192 || q.stride(0) % 8 || q.stride(1) % 8) return false;
+  const int64_t n = q.size(1);
+  return is_bf16(w_uk, 3, dev) && w_uk.size(0) == n && w_uk.size(1) == 128 && w_uk.size(2) == kNope && is_bf16(w_uv, 3, dev) &&
+         w_uv.size(0) == n && w_uv.size(1) == kNope && w_uv.size(2) == kVDim && w_uv.stride(0) % 8 == 0 && w_uv.stride(1) % 8 == 0 &&
+         is_bf16(out, 2, dev) && out.size(0) >= t && out.size(1) == n * kVDim && out.stride(0) % 4 == 0;
+}
+// Absorbed queries [N, T, 512] (library GEMM, as in the reference: mla.py:900-905).
+Tensor absorb(const Tensor& q, const Tensor& w_uk, int64_t t) {
+  return at::bmm(q.narrow(0, 0, t).narrow(2, 0, 128).transpose(0, 1), w_uk);
+}
+// Merge of the partials and the value up-projection into out (mla.py:309-315).
+void merge_vup(const Tensor& ws, const Tensor& lens, const OptTensor& qsl, int64_t batch, int64_t q_len, int64_t n, int splits,
+               int64_t t, const Tensor& w_uv, const Tensor& out, Stream st) {
+  const int32_t* qs = qsl ? (const int32_t*)qsl->data_ptr() : nullptr;
+  if (t <= kVupMaxTokens) {
+    check(mla_splitkv_reduce_vup(ws.data_ptr(), ws.numel(), (const int32_t*)lens.data_ptr(), qs, (int)batch, (int)q_len, (int)n,
+                                 splits, (int)t, w_uv.data_ptr(), w_uv.stride(0), w_uv.stride(1), out.data_ptr(), out.stride(0),
+                                 kVDim, st), "mla_splitkv_reduce_vup");
+    return;
+  }
+  Tensor o = at::empty({n, t, kNope}, out.options());
+  check(mla_splitkv_reduce(ws.data_ptr(), ws.numel(), (const int32_t*)lens.data_ptr(), qs, (int)batch, (int)q_len, (int)n, splits,
+                           o.data_ptr(), o.stride(1), o.stride(0), nullptr, st), "mla_splitkv_reduce");
+  Tensor dst = out.narrow(0, 0, t).view({t, n, kVDim}).transpose(0, 1);
+  at::bmm_out(dst, o, w_uv);
+}
+
+// One layer's decode tokens, their rows in the cache already: absorption, split-KV attention, merge + up-projection.  rope =
+// None: the fp8 cache.  window > 0: static sink + sliding window.
+bool mla_decode(const Tensor& q, const Tensor& nope, const OptTensor& rope, const Tensor& block_table, const Tensor& seq_lens, const OptTensor& qsl, int64_t q_len,
+                int64_t max_seq_len, const Tensor& w_uk, const Tensor& w_uv, double scale, int64_t t, int64_t sink, int64_t window,
+                const Tensor& out) {
+  if (!current_gpu(q)) return false;
+  const at::Device dev = q.device();
+  Cache c;
+  if (!layer_ok(q, w_uk, w_uv, out, t, dev) || !cache_of(nope, rope, dev, c) || c.page != kPage || !is_i32(seq_lens, 1, dev) || !seq_lens.is_contiguous() ||
+      !is_i32(block_table, 2, dev) || block_table.size(0) < seq_lens.numel() || block_table.size(1) < 1 || seq_lens.numel() < 1 ||
+      q_len < 1)
+    return false;
+  const int64_t b = seq_lens.numel(), n = q.size(1);
+  if (qsl ? !(is_i32(*qsl, 1, dev) && qsl->is_contiguous() && qsl->numel() == b + 1) : t != b * q_len) return false;
+  at::AutoDispatchBelowAutograd guard;
+  Stream st = stream_of(q);
+  const bool fp8 = !rope;
+  Tensor ql = absorb(q, w_uk, t);
+  if (window > 0) max_seq_len = std::min(max_seq_len, sink + window + 32 + q_len);
+  const int splits = default_splits(b, q_len, n, max_seq_len);
+  const int64_t need = (int64_t)mla_decode_workspace_bytes((int)b, (int)q_len, (int)n, splits);
+  Tensor& ws = scratch(q, st, need, 0);
+  const int32_t* bt = (const int32_t*)block_table.data_ptr();
+  const int64_t bts = block_table.stride(0);
+  const int mb = (int)block_table.size(1);
+  const int32_t* lens = (const int32_t*)seq_lens.data_ptr();
+  const int32_t* qs = qsl ? (const int32_t*)qsl->data_ptr() : nullptr;
+  const char* qr = (const char*)q.data_ptr() + 2 * 128;
+  const int64_t ql_t = ql.stride(1), ql_h = ql.stride(0);
+  Tensor plan;
+  const Tensor* merged_lens = &seq_lens;
+  if (window > 0) {
+    plan = at::empty({2, b}, seq_lens.options());
+    int32_t *short_lens = (int32_t*)plan.data_ptr(), *skip = short_lens + b;
+    check(mla_window_plan(lens, qs, (int)b, (int)q_len, (int)sink, (int)window, short_lens, skip, st), "mla_window_plan");
+    merged_lens = &plan;                                       // (its first row)
+    if (fp8)
+      check(mla_decode_fp8_window_split(ql.data_ptr(), ql_t, ql_h, qr, q.stride(0), q.stride(1), c.nope->data_ptr(), c.n_sp, c.n_sr,
+                                        c.pages, bt, bts, mb, short_lens, skip, qs, (int)b, (int)q_len, (int)n, (int)sink,
+                                        (int)window, (float)scale, ws.data_ptr(), ws.numel(), splits, st), "mla_decode_fp8_window_split");
+    else
+      check(mla_decode_bf16_window_split(ql.data_ptr(), ql_t, ql_h, qr, q.stride(0), q.stride(1), c.nope->data_ptr(), c.n_sp, c.n_sr,
+                                         c.rope->data_ptr(), c.r_sp, c.r_sr, c.pages, bt, bts, mb, short_lens, skip, qs, (int)b,
+                                         (int)q_len, (int)n, (int)sink, (int)window, (float)scale, ws.data_ptr(), ws.numel(),
+                                         splits, st), "mla_decode_bf16_window_split");
+  } else if (fp8) {
+    check(mla_decode_fp8(ql.data_ptr(), ql_t, ql_h, qr, q.stride(0), q.stride(1), c.nope->data_ptr(), c.n_sp, c.n_sr, c.pages, bt,
+                         bts, mb, lens, qs, (int)b, (int)q_len, (int)n, (float)scale, nullptr, 0, 0, nullptr, ws.data_ptr(),
+                         ws.numel(), splits, st), "mla_decode_fp8");
+  } else {
+    check(mla_decode_bf16_split(ql.data_ptr(), ql_t, ql_h, qr, q.stride(0), q.stride(1), c.nope->data_ptr(), c.n_sp, c.n_sr,
+                                c.rope->data_ptr(), c.r_sp, c.r_sr, c.pages, bt, bts, mb, lens, qs, (int)b, (int)q_len, (int)n,
+                                (float)scale, ws.data_ptr(), ws.numel(), splits, st), "mla_decode_bf16_split");
+  }
+  merge_vup(ws, *merged_lens, qsl, b, q_len, n, splits, t, w_uv, out, st);
+  return true;
+}
+
+// One layer's sparse decode tokens over the cache rows of their picks.  (Few enough tokens for one launch; a prefill's
+// thousands take the general path.)
+bool sparse_decode(const Tensor& q, const Tensor& nope, const Tensor& rope, const Tensor& rows, const Tensor& counts, const Tensor& w_uk, const Tensor& w_uv,
+                   double scale, int64_t t, const Tensor& out) {
+  if (!current_gpu(q) || t > kVupMaxTokens) return false;
+  const at::Device dev = q.device();
+  Cache c;
+  const OptTensor r(rope);
+  if (!layer_ok(q, w_uk, w_uv, out, t, dev) || !cache_of(nope, r, dev, c) || !is_i32(rows, 2, dev) || rows.size(0) < t || !is_i32(counts, 1, dev) || !counts.is_contiguous() || counts.numel() < t)
+    return false;
+  const int64_t n = q.size(1);
+  const int splits = default_splits(t, 1, n, rows.size(1));
+  const int64_t need = (int64_t)mla_decode_workspace_bytes((int)t, 1, (int)n, splits);
+  if (need > (256 << 20)) return false;                        // kernels.SPARSE_WORKSPACE_CAP
+  at::AutoDispatchBelowAutograd guard;
+  Stream st = stream_of(q);
+  Tensor ql = absorb(q, w_uk, t);
+  Tensor& ws = scratch(q, st, need, 0);
+  check(dsa_sparse_decode_bf16(ql.data_ptr(), ql.stride(1), ql.stride(0), (const char*)q.data_ptr() + 2 * 128, q.stride(0), q.stride(1),
+                               c.nope->data_ptr(), c.n_sp, c.n_sr, c.rope->data_ptr(), c.r_sp, c.r_sr, c.pages, (int)c.page,
+                               (const int32_t*)rows.data_ptr(), rows.stride(0), (const int32_t*)counts.data_ptr(), (int)t, (int)n,
+                               (float)scale, nullptr, 0, 0, nullptr, ws.data_ptr(), ws.numel(), splits, st),
+        "dsa_sparse_decode_bf16");
+  merge_vup(ws, counts, std::nullopt, t, 1, n, splits, t, w_uv, out, st);
+  return true;
+}
+
+// The selection for a step's decode tokens: queries and new index keys to fp8 (keys into the cache, head weights times query
+// scales), scores, top-k with cache rows.  index_cache: the third DSA cache tensor [nblk, page, 1, 128] of a 2-byte type, whose
+// pages hold page x 128 e4m3 keys, then page fp32 scales.
+bool dsa_select(const Tensor& q, const Tensor& k, const Tensor& weights, const Tensor& index_cache, const Tensor& slots,
+                const Tensor& block_table, const Tensor& seq_lens, const OptTensor& qsl, int64_t t, int64_t q_len, int64_t max_len,
+                int64_t topk, const Tensor& logits, const Tensor& out, const Tensor& rows, const Tensor& counts) {
+  if (!current_gpu(q)) return false;
+  const at::Device dev = q.device();
+  if (!is_bf16(q, 3, dev) || q.size(1) != 64 || q.size(2) != 128 || !q.is_contiguous()) return false;
+  const int64_t b = seq_lens.numel(), page = index_cache.size(1), pages = index_cache.size(0);
+  const at::ScalarType wt = weights.scalar_type();
+  if (t < 1 || q.size(0) < t || !is_bf16(k, 2, dev) || k.size(0) < t || k.size(1) != 128 || (wt != at::kFloat && wt != at::kBFloat16) ||
+      weights.dim() != 2 || weights.size(0) < t || weights.size(1) != 64 || weights.stride(1) != 1 || weights.device() != dev ||
+      !index_cache.is_contiguous() || index_cache.element_size() != 2 || index_cache.device() != dev ||
+      index_cache.numel() != pages * page * 128 || slots.scalar_type() != at::kLong || !slots.is_contiguous() || slots.dim() != 1 ||
+      slots.numel() < t || slots.device() != dev || !is_i32(block_table, 2, dev) || block_table.size(0) < b || b < 1 ||
+      !is_i32(seq_lens, 1, dev) || !seq_lens.is_contiguous() || !is(logits, at::kFloat, 2, dev) || logits.size(0) < t ||
+      logits.size(1) < (max_len + 31) / 32 * 32 || !is_i32(out, 2, dev) || out.size(0) < t || out.size(1) < topk ||
+      !is_i32(rows, 2, dev) || rows.size(0) < t || rows.size(1) < topk || !is_i32(counts, 1, dev) || counts.numel() < t ||
+      !counts.is_contiguous())
+    return false;
+  if (qsl ? !(is_i32(*qsl, 1, dev) && qsl->is_contiguous() && qsl->numel() == b + 1) : t != b * q_len) return false;
+  at::AutoDispatchBelowAutograd guard;
+  Stream st = stream_of(q);
+  // fp8 queries [t, 64, 128], then their head weights times scales [t, 64] fp32
+  Tensor q8 = at::empty({t * 64 * (128 + 4)}, q.options().dtype(at::kByte));
+  float* w = (float*)((char*)q8.data_ptr() + t * 64 * 128);
+  char* k8 = (char*)index_cache.data_ptr();
+  const int32_t* qs = qsl ? (const int32_t*)qsl->data_ptr() : nullptr;
+  const int32_t* lens = (const int32_t*)seq_lens.data_ptr();
+  check(dsa_quant_qkw_fp8(q.data_ptr(), 128, t * 64, q8.data_ptr(), weights.data_ptr(), wt == at::kFloat ? 1 : 0, weights.stride(0),
+                          64, w, k.data_ptr(), k.stride(0), t, (const int64_t*)slots.data_ptr(), k8, page * 256, 128,
+                          (float*)(k8 + page * 128), page * 64, (int)page, pages, st), "dsa_quant_qkw_fp8");
+  check(dsa_indexer_scores_fp8_above(q8.data_ptr(), 64 * 128, 128, w, 64, nullptr, 0, k8, page * 256, 128, (const float*)(k8 + page * 128),
+                                     page * 64, pages, (int)page, (const int32_t*)block_table.data_ptr(), block_table.stride(0),
+                                     (int)block_table.size(1), lens, qs, (int)b, (int)q_len, 64, (int)max_len,
+                                     (float*)logits.data_ptr(), logits.stride(0), (int)topk, st), "dsa_indexer_scores_fp8");
+  const int64_t need = (int64_t)dsa_topk_workspace_bytes((int)b, (int)q_len, logits.stride(0));
+  Tensor& ws = scratch(q, st, need, 1);
+  check(dsa_topk_rows((const float*)logits.data_ptr(), logits.stride(0), lens, qs, (int)b, (int)q_len, (int)topk,
+                      (int32_t*)out.data_ptr(), out.stride(0), (const int32_t*)block_table.data_ptr(), block_table.stride(0),
+                      (int)block_table.size(1), (int)page, pages, (int32_t*)rows.data_ptr(), rows.stride(0),
+                      (int32_t*)counts.data_ptr(), ws.data_ptr(), ws.numel(), st), "dsa_topk_rows");
+  return true;
+}
+
+// kernels.kv_rmsnorm_rope_cache with everything in its usual place: a cache, table "half", contiguous outputs or none.
+bool norm_rope_cache(const Tensor& kv, const Tensor& gamma, const Tensor& cos, const Tensor& sin, const Tensor& slots,
+                     const Tensor& nope, const OptTensor& rope, double eps, const OptTensor& kv_a, const OptTensor& k_pe,
+                     const OptTensor& q_rope, const OptTensor& q_out) {
+  if (!current_gpu(kv)) return false;
+  const at::Device dev = kv.device();
+  Cache c;
+  if (!is_bf16(kv, 2, dev) || kv.size(1) != kNope + kRope || !is_bf16(gamma, 1, dev) || gamma.size(0) != kNope ||
+      !is_bf16(cos, 2, dev) || !is_bf16(sin, 2, dev) || cos.size(1) < 32 || cos.sizes() != sin.sizes() ||
+      cos.stride(0) != sin.stride(0) || slots.scalar_type() != at::kLong || slots.dim() != 1 || !slots.is_contiguous() ||
+      slots.device() != dev || !cache_of(nope, rope, dev, c))
+    return false;
+  const int64_t t = std::min(slots.numel(), kv.size(0));
+  if (t < 1 || cos.size(0) < t) return false;
+  auto row_out = [&](const OptTensor& o, int64_t w) { return !o || (is_bf16(*o, 2, dev) && o->size(0) >= t && o->size(1) == w); };
+  if (!row_out(kv_a, kNope) || !row_out(k_pe, kRope)) return false;
+  const Tensor* qo = q_rope ? (q_out ? &*q_out : &*q_rope) : nullptr;
+  if (q_rope && (!is_bf16(*q_rope, 3, dev) || q_rope->size(0) < t || q_rope->size(2) != kRope || qo->sizes() != q_rope->sizes() ||
+                 !is_bf16(*qo, 3, dev)))
+    return false;
+  Stream st = stream_of(kv);
+  const char* pe_in = (const char*)kv.data_ptr() + 2 * kNope;
+  void* o_c = kv_a ? kv_a->data_ptr() : nullptr;
+  void* o_r = k_pe ? k_pe->data_ptr() : nullptr;
+  const int64_t o_cs = kv_a ? kv_a->stride(0) : 0, o_rs = k_pe ? k_pe->stride(0) : 0, ks = kv.stride(0), cs = cos.stride(0);
+  const int64_t* sl = (const int64_t*)slots.data_ptr();
+  const int pg = (int)c.page;
+  if (c.rope && q_rope)
+    check(mla_kv_rmsnorm_rope_cache_q(kv.data_ptr(), ks, pe_in, ks, gamma.data_ptr(), cos.data_ptr(), sin.data_ptr(), cs, 1, 0, sl,
+                                      (int)t, (float)eps, nope.data_ptr(), c.n_sp, c.n_sr, c.rope->data_ptr(), c.r_sp, c.r_sr, pg,
+                                      c.pages, o_c, o_cs, o_r, o_rs, q_rope->data_ptr(), q_rope->stride(0), q_rope->stride(1),
+                                      (int)q_rope->size(1), qo->data_ptr(), qo->stride(0), qo->stride(1), st),
+          "mla_kv_rmsnorm_rope_cache_q");
+  else if (c.rope)
+    check(mla_kv_rmsnorm_rope_cache(kv.data_ptr(), ks, pe_in, ks, gamma.data_ptr(), cos.data_ptr(), sin.data_ptr(), cs, 1, 0, sl, (int)t,
+                                    (float)eps, nope.data_ptr(), c.n_sp, c.n_sr, c.rope->data_ptr(), c.r_sp, c.r_sr, pg, c.pages,
+                                    o_c, o_cs, o_r, o_rs, st), "mla_kv_rmsnorm_rope_cache");
+  else if (q_rope)
+    check(mla_kv_rmsnorm_rope_cache_q_fp8(kv.data_ptr(), ks, pe_in, ks, gamma.data_ptr(), cos.data_ptr(), sin.data_ptr(), cs, 1, 0, sl,
+                                          (int)t, (float)eps, nope.data_ptr(), c.n_sp, c.n_sr, pg, c.pages, o_c, o_cs, o_r, o_rs,
+                                          q_rope->data_ptr(), q_rope->stride(0), q_rope->stride(1), (int)q_rope->size(1),
+                                          qo->data_ptr(), qo->stride(0), qo->stride(1), st), "mla_kv_rmsnorm_rope_cache_q_fp8");
+  else
+    check(mla_kv_rmsnorm_rope_cache_fp8(kv.data_ptr(), ks, pe_in, ks, gamma.data_ptr(), cos.data_ptr(), sin.data_ptr(), cs, 1, 0, sl,
+                                        (int)t, (float)eps, nope.data_ptr(), c.n_sp, c.n_sr, pg, c.pages, o_c, o_cs, o_r, o_rs, st),
+          "mla_kv_rmsnorm_rope_cache_fp8");
+  return true;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.doc() = "native host side of the MLA / DSA decode steps (see omni_npu_amd/_host.py)";
+  m.def("set_workspace", [](py::object fn) { Py_XDECREF(g_workspace); g_workspace = fn.release().ptr(); });
+  m.def("cache_write", &cache_write);
+  m.def("mla_decode", &mla_decode);
+  m.def("sparse_decode", &sparse_decode);
+  m.def("dsa_select", &dsa_select);
+  m.def("norm_rope_cache", &norm_rope_cache);
+}

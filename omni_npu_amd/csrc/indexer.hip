@@ -326,13 +326,15 @@ struct QuantRows {
   const __bf16* src; int64_t src_stride, rows;
   const int64_t* slots;
   uint8_t* dst8; int64_t d_sp, d_sr;
-  float* dscale; int64_t s_sp;
+  float* dscale; int64_t s_sp;                        // may be null where w_out is given
   int32_t page_size; int64_t num_pages;
+  // optional, rows r = (token, head): w_out[r] = weight[token][head] * the row's scale (the indexer's head weights, bf16 or
+  // fp32, with the query scale folded in)
+  const void* w; int32_t w_f32, heads; int64_t w_st; float* w_out;
 };
 
-__device__ __forceinline__ void quant_row(const __bf16* src, int64_t src_stride, int64_t rows, const int64_t* slots,
-                                          uint8_t* dst8, int64_t d_sp, int64_t d_sr, float* dscale, int64_t s_sp,
-                                          int32_t page_size, int64_t num_pages, int64_t r) {
+__device__ __forceinline__ void quant_row(const QuantRows& q, int64_t r) {
+  const auto [src, src_stride, rows, slots, dst8, d_sp, d_sr, dscale, s_sp, page_size, num_pages, w_in, w_f32, heads, w_st, w_out] = q;
   const int l16 = threadIdx.x & 15;
   if (r >= rows) return;
   const int64_t slot = slots ? slots[r] : r;
@@ -372,52 +374,75 @@ __device__ __forceinline__ void quant_row(const __bf16* src, int64_t src_stride,
 #pragma unroll
     for (int e = 0; e < 4; e++) *(uint16_t*)(d + 2 * e) = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
   }
-  if (l16 == 0) dscale[pg * s_sp + off] = scale;
+  if (l16 == 0) {
+    if (dscale) dscale[pg * s_sp + off] = scale;
+    if (w_out) {
+      const int64_t tk = r / heads, at = tk * w_st + (r - tk * heads);
+      w_out[r] = (w_f32 ? ((const float*)w_in)[at] : (float)((const __bf16*)w_in)[at]) * scale;
+    }
+  }
 }
 
-__global__ __launch_bounds__(256) void dsa_quant_rows_kernel(const __bf16* src, int64_t src_stride, int64_t rows,
-                                                             const int64_t* slots, uint8_t* dst8, int64_t d_sp, int64_t d_sr,
-                                                             float* dscale, int64_t s_sp, int32_t page_size,
-                                                             int64_t num_pages) {
-  quant_row(src, src_stride, rows, slots, dst8, d_sp, d_sr, dscale, s_sp, page_size, num_pages,
-            (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4));
+__global__ __launch_bounds__(256) void dsa_quant_rows_kernel(const QuantRows q) {
+  quant_row(q, (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4));
 }
 
 // Two row sets in one launch (the indexer's step: the query rows into plain buffers, the new key rows into the cache):
 // the first a_blocks workgroups take set a, the others set b.
 __global__ __launch_bounds__(256) void dsa_quant_rows2_kernel(const QuantRows a, const QuantRows b, int32_t a_blocks) {
   const bool first = (int)blockIdx.x < a_blocks;
-  const QuantRows& q = first ? a : b;
-  quant_row(q.src, q.src_stride, q.rows, q.slots, q.dst8, q.d_sp, q.d_sr, q.dscale, q.s_sp, q.page_size, q.num_pages,
-            (int64_t)(first ? blockIdx.x : blockIdx.x - a_blocks) * 16 + (threadIdx.x >> 4));
+  quant_row(first ? a : b, (int64_t)(first ? blockIdx.x : blockIdx.x - a_blocks) * 16 + (threadIdx.x >> 4));
 }
 
 }  // namespace mlahip
 using namespace mlahip;
+
+static int quant_qk_impl(const char* what, const void* q, int64_t q_stride, int64_t q_rows, void* q8, float* q_scale, const void* w,
+                         int32_t w_f32, int64_t w_stride, int32_t heads, float* w_out, const void* k, int64_t k_stride,
+                         int64_t k_rows, const int64_t* slot_mapping, void* k8_cache, int64_t cache_page_stride_bytes,
+                         int64_t cache_row_stride_bytes, float* scale_cache, int64_t scale_page_stride, int32_t page_size,
+                         int64_t num_pages, hipStream_t stream) {
+  MLA_REQUIRE(q && q8 && (q_scale || (w && w_out)) && k && slot_mapping && k8_cache && scale_cache, MLA_ERR_NULL,
+              "%s: null pointer argument", what);
+  MLA_REQUIRE(q_rows >= 0 && k_rows >= 0 && page_size >= 1 && num_pages >= 1 && q_stride % 2 == 0 && k_stride % 2 == 0 &&
+                  cache_row_stride_bytes >= 128 && cache_row_stride_bytes % 2 == 0 && cache_page_stride_bytes % 2 == 0 &&
+                  (uintptr_t)q % 4 == 0 && (uintptr_t)k % 4 == 0 && (uintptr_t)q8 % 2 == 0 && (uintptr_t)k8_cache % 2 == 0 &&
+                  q_rows < (1ll << 31) && k_rows < (1ll << 31) && heads >= 1,
+              MLA_ERR_SHAPE, "%s: q_rows=%lld k_rows=%lld page_size=%d", what, (long long)q_rows, (long long)k_rows, page_size);
+  if (q_rows + k_rows == 0) return MLA_OK;
+  // (set a has no slot mapping: row r is "slot" r of one page that holds them all)
+  const QuantRows a{(const __bf16*)q, q_stride, q_rows, nullptr, (uint8_t*)q8, 0, 128, q_scale, 0,
+                    (int32_t)(q_rows > 0 ? q_rows : 1), 1, w, w_f32, heads, w_stride, w_out};
+  const QuantRows b{(const __bf16*)k, k_stride, k_rows, slot_mapping, (uint8_t*)k8_cache, cache_page_stride_bytes,
+                    cache_row_stride_bytes, scale_cache, scale_page_stride, page_size, num_pages, nullptr, 0, 1, 0, nullptr};
+  const int64_t a_blocks = (q_rows + 15) / 16, b_blocks = (k_rows + 15) / 16;
+  hipLaunchKernelGGL(dsa_quant_rows2_kernel, dim3((unsigned)(a_blocks + b_blocks)), dim3(256), 0, stream, a, b,
+                     (int32_t)a_blocks);
+  return check_launch("dsa_quant_rows2_kernel");
+}
 
 // dsa_quant_rows_fp8 of the query rows (plain outputs) and of the new key rows (into the paged index-key cache) in one launch.
 extern "C" int dsa_quant_qk_fp8(const void* q, int64_t q_stride, int64_t q_rows, void* q8, float* q_scale, const void* k,
                                 int64_t k_stride, int64_t k_rows, const int64_t* slot_mapping, void* k8_cache,
                                 int64_t cache_page_stride_bytes, int64_t cache_row_stride_bytes, float* scale_cache,
                                 int64_t scale_page_stride, int32_t page_size, int64_t num_pages, hipStream_t stream) {
-  MLA_REQUIRE(q && q8 && q_scale && k && slot_mapping && k8_cache && scale_cache, MLA_ERR_NULL,
-              "dsa_quant_qk_fp8: null pointer argument");
-  MLA_REQUIRE(q_rows >= 0 && k_rows >= 0 && page_size >= 1 && num_pages >= 1 && q_stride % 2 == 0 && k_stride % 2 == 0 &&
-                  cache_row_stride_bytes >= 128 && cache_row_stride_bytes % 2 == 0 && cache_page_stride_bytes % 2 == 0 &&
-                  (uintptr_t)q % 4 == 0 && (uintptr_t)k % 4 == 0 && (uintptr_t)q8 % 2 == 0 && (uintptr_t)k8_cache % 2 == 0 &&
-                  q_rows < (1ll << 31) && k_rows < (1ll << 31),
-              MLA_ERR_SHAPE, "dsa_quant_qk_fp8: q_rows=%lld k_rows=%lld page_size=%d", (long long)q_rows, (long long)k_rows,
-              page_size);
-  if (q_rows + k_rows == 0) return MLA_OK;
-  // (set a has no slot mapping: row r is "slot" r of one page that holds them all)
-  const QuantRows a{(const __bf16*)q, q_stride, q_rows, nullptr, (uint8_t*)q8, 0, 128, q_scale, 0,
-                    (int32_t)(q_rows > 0 ? q_rows : 1), 1};
-  const QuantRows b{(const __bf16*)k, k_stride, k_rows, slot_mapping, (uint8_t*)k8_cache, cache_page_stride_bytes,
-                    cache_row_stride_bytes, scale_cache, scale_page_stride, page_size, num_pages};
-  const int64_t a_blocks = (q_rows + 15) / 16, b_blocks = (k_rows + 15) / 16;
-  hipLaunchKernelGGL(dsa_quant_rows2_kernel, dim3((unsigned)(a_blocks + b_blocks)), dim3(256), 0, stream, a, b,
-                     (int32_t)a_blocks);
-  return check_launch("dsa_quant_rows2_kernel");
+  MLA_REQUIRE(q_scale, MLA_ERR_NULL, "dsa_quant_qk_fp8: null pointer argument");
+  return quant_qk_impl("dsa_quant_qk_fp8", q, q_stride, q_rows, q8, q_scale, nullptr, 0, 0, 1, nullptr, k, k_stride, k_rows,
+                       slot_mapping, k8_cache, cache_page_stride_bytes, cache_row_stride_bytes, scale_cache, scale_page_stride,
+                       page_size, num_pages, stream);
+}
+
+// The same for rows r = token * heads + head, with the indexer's head weights (bf16, or fp32 with w_f32) instead of the plain
+// query scales: w_out[r] = weight[token][head] * scale of row r, what dsa_indexer_scores_fp8 takes as weights.
+extern "C" int dsa_quant_qkw_fp8(const void* q, int64_t q_stride, int64_t q_rows, void* q8, const void* weights, int32_t w_f32,
+                                 int64_t w_stride, int32_t heads, float* w_out, const void* k, int64_t k_stride, int64_t k_rows,
+                                 const int64_t* slot_mapping, void* k8_cache, int64_t cache_page_stride_bytes,
+                                 int64_t cache_row_stride_bytes, float* scale_cache, int64_t scale_page_stride,
+                                 int32_t page_size, int64_t num_pages, hipStream_t stream) {
+  MLA_REQUIRE(weights && w_out, MLA_ERR_NULL, "dsa_quant_qkw_fp8: null pointer argument");
+  return quant_qk_impl("dsa_quant_qkw_fp8", q, q_stride, q_rows, q8, nullptr, weights, w_f32, w_stride, heads, w_out, k, k_stride,
+                       k_rows, slot_mapping, k8_cache, cache_page_stride_bytes, cache_row_stride_bytes, scale_cache,
+                       scale_page_stride, page_size, num_pages, stream);
 }
 
 extern "C" int dsa_quant_rows_fp8(const void* src, int64_t src_stride, int64_t rows, const int64_t* slot_mapping,
@@ -430,9 +455,9 @@ extern "C" int dsa_quant_rows_fp8(const void* src, int64_t src_stride, int64_t r
                   dst_page_stride_bytes % 2 == 0,
               MLA_ERR_SHAPE, "dsa_quant_rows_fp8: rows=%lld page_size=%d", (long long)rows, page_size);
   if (rows == 0) return MLA_OK;
-  hipLaunchKernelGGL(dsa_quant_rows_kernel, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, (const __bf16*)src,
-                     src_stride, rows, slot_mapping, (uint8_t*)dst8, dst_page_stride_bytes, dst_row_stride_bytes, dst_scale,
-                     scale_page_stride, page_size, num_pages);
+  const QuantRows q{(const __bf16*)src, src_stride, rows, slot_mapping, (uint8_t*)dst8, dst_page_stride_bytes, dst_row_stride_bytes,
+                    dst_scale, scale_page_stride, page_size, num_pages, nullptr, 0, 1, 0, nullptr};
+  hipLaunchKernelGGL(dsa_quant_rows_kernel, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, q);
   return check_launch("dsa_quant_rows_kernel");
 }
 

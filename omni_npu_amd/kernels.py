@@ -8,7 +8,7 @@ from typing import Optional
 
 import torch
 
-from . import _lib
+from . import _host, _lib
 
 PAGE = 128
 D_NOPE = 512
@@ -39,6 +39,8 @@ def cache_write(kv_c: torch.Tensor, k_pe: torch.Tensor, slot_mapping: torch.Tens
                 nope_cache: torch.Tensor, rope_cache: torch.Tensor) -> None:
     """nope.flatten(0,1)[slot[t]] = kv_c[t]; rope.flatten(0,1)[slot[t]] = k_pe[t]; negative slots skipped
     (reference: store_kv, src/omni_npu/attention/backends/mla.py:868-881)."""
+    if _host.load().cache_write(kv_c, k_pe, slot_mapping, nope_cache, rope_cache):
+        return
     _need_cuda(kv_c, k_pe, slot_mapping, nope_cache, rope_cache)
     lib = _lib.load()
     nope, rope = _cache3(nope_cache, D_NOPE), _cache3(rope_cache, D_ROPE)
@@ -85,6 +87,8 @@ FP8_ROW_BYTES = 656      # 512 e4m3 + 4 fp32 block scales + 64 bf16 rope
 def cache_write_fp8(kv_c: torch.Tensor, k_pe: torch.Tensor, slot_mapping: torch.Tensor, cache: torch.Tensor) -> None:
     """Quantise the new tokens' latent to e4m3 with one fp32 scale per 128 elements and write 656-byte rows
     (512 fp8 | 4 fp32 scales | 64 bf16 rope) into ``cache`` = uint8 [num_blocks, page, 656]."""
+    if _host.load().cache_write(kv_c, k_pe, slot_mapping, cache, None):
+        return
     _need_cuda(kv_c, k_pe, slot_mapping, cache)
     lib = _lib.load()
     k_pe = k_pe.reshape(k_pe.shape[0], -1) if k_pe.dim() == 3 else k_pe
@@ -125,6 +129,10 @@ def kv_rmsnorm_rope_cache(kv: torch.Tensor, gamma: torch.Tensor, cos: torch.Tens
     (``nope_cache`` = uint8 [num_blocks, page, 656]); ``slot_mapping=None`` caches nothing and only fills ``kv_a_out`` / ``k_pe_out``.
     ``q_rope`` (bf16 [T, N, 64], any strides with a contiguous last dim): the rotary embedding of the same tokens' query
     heads (npu_interleave_rope, npu_mla.py:210) runs in the same launch, into ``q_out`` (default: in place)."""
+    if slot_mapping is not None and table == "half" and not interleaved_out and nope_cache is not None and (
+            q_out is None or q_rope is not None) and _host.load().norm_rope_cache(
+            kv, gamma, cos, sin, slot_mapping, nope_cache, rope_cache, eps, kv_a_out, k_pe_out, q_rope, q_out):
+        return
     _need_cuda(kv, gamma, cos, sin, slot_mapping, nope_cache)
     lib = _lib.load()
     kv = kv.reshape(kv.shape[0], -1)

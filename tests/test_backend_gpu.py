@@ -362,3 +362,67 @@ def test_dsa_prompts_attend_over_their_own_keys_with_the_picks_as_a_mask(dev, q_
         got.append((indexer.topk_indices_buffer[:t].clone(), out))
     assert torch.equal(got[0][0], got[1][0])
     attn_close(got[0][1], got[1][1], 3e-2, 4e-3 + 4e-3)        # (the latent form also rounds absorbed queries and outputs to bf16)
+
+
+class _NoNative:
+    """The native host side as it answers for arguments it does not know."""
+    def __getattr__(self, name):
+        return lambda *a: False
+
+
+@pytest.mark.parametrize("kind,q_lens,n", [("bf16", [1], 16), ("bf16", [1, 2, 2], 128), ("fp8", [2] * 3, 40), ("window", [1] * 5, 16),
+                                           ("fp8 window", [1, 2], 16), ("bf16", [1] * 300, 16), ("dsa", [1] * 3, 16), ("dsa", [2, 2], 128),
+                                           ("dsa", [1, 2, 1], 16)])
+def test_native_decode_forward_is_the_general_path(dev, monkeypatch, kind, q_lens, n):
+    """One native call per stage against the general path through kernels.py: the same picks, caches and outputs bit for
+    bit, uniform and ragged queries, more tokens than the fused merge takes, all cache forms."""
+    from omni_npu_amd import _host, kernels as K
+    g = torch.Generator().manual_seed(len(q_lens) + n)
+    sparse, fp8, window = kind == "dsa", "fp8" in kind, "window" in kind
+    seq_lens = [(137 * (i + 2)) % 900 + 40 for i in range(len(q_lens))]
+    common = _common(q_lens, seq_lens)
+    t = common.num_actual_tokens
+    sink = 128 if window else 0
+    if window:                                                 # the sink's page in front of every row
+        common.block_table_tensor = torch.cat([torch.zeros(len(q_lens), 1, dtype=torch.int32), common.block_table_tensor + 1], 1)
+    nblk = int(common.block_table_tensor.max()) + 1
+    common.slot_mapping = torch.cat([O.slots_for(common.block_table_tensor, b, sink + s - ql, sink + s)
+                                     for b, (ql, s) in enumerate(zip(q_lens, seq_lens))])
+    width = 704 if sparse else 576
+    rows = torch.randn(nblk * 128, 576, generator=g).bfloat16().to(dev)
+    if fp8:
+        cache = (torch.zeros(nblk, 128, 656, dtype=torch.uint8, device=dev),)
+        K.cache_write_fp8(rows[:, :512], rows[:, 512:], torch.arange(nblk * 128, device=dev), cache[0])
+    else:
+        raw = torch.zeros(nblk * 128 * width, dtype=torch.bfloat16, device=dev).view(torch.uint8)
+        cls = dsa.NPUDSABackend if sparse else mla.NPUMLABackend
+        cache = cls.reshape_kv_cache(raw, nblk, 128, 1, width, dtype=torch.bfloat16)
+        K.cache_write(rows[:, :512], rows[:, 512:], torch.arange(nblk * 128, device=dev), cache[0], cache[1])
+        if sparse:
+            K.quant_rows_fp8(torch.randn(nblk * 128, 128, generator=g).bfloat16().to(dev), *dsa.indexer_cache_views(cache[2]),
+                             slot_mapping=torch.arange(nblk * 128, device=dev))
+    indexer = dsa.LightningIndexer(64, max_tokens=t, device=dev) if sparse else None
+    impl, _ = _mk_impl(dsa.NPUDSAImpl if sparse else mla.NPUMLAImpl, n, dev, indexer=indexer,
+                       kv_cache_dtype="fp8" if fp8 else "auto", sliding_window=300 if window else None)
+    if window:
+        impl.update_sink_kv(rows[:128, 512:], rows[:128, :512])
+    builder = dsa.NPUDSAMetadataBuilder if sparse else mla.NPUMLAMetadataBuilder
+    meta = builder(V.AttentionSpec(128, 1, width, torch.bfloat16), ["l"], _cfg(cap=2), dev).build(0, _to(common, dev))
+    q, c, pe = (torch.randn(t, *s, generator=g).bfloat16().to(dev) for s in ((n, 192), (512,), (1, 64)))
+    iq, ik, iw = (torch.randn(t, *s, generator=g).bfloat16().to(dev) for s in ((64, 128), (128,), (64,)))
+    got = []
+    calls = []
+    native = _host.load()
+    for load in (lambda: native, lambda: _NoNative()):
+        monkeypatch.setattr(_host, "load", load)
+        mine = tuple(x.clone() for x in cache)
+        out = torch.zeros(t + 1, n * 128, dtype=torch.bfloat16, device=dev)
+        if sparse:
+            indexer(iq, ik, iw, mine, meta)
+        calls.append(impl._native_decode(q, mine, meta, out.clone()) if not sparse else
+                     indexer._native_select(iq, ik, iw, mine[2], meta))
+        impl.forward(None, q, c, pe, mine, meta, output=out)
+        got.append((out, *(x.view(torch.uint8) for x in mine), *((indexer.topk_indices_buffer[:t].clone(),) if sparse else ())))
+    assert calls == [True, False]
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
