@@ -415,7 +415,9 @@ int dsa_build_rows(const int32_t* indices, int64_t indices_stride, const int32_t
  * sees the sink and keys [max(0, L - s + i + 1 - window), L - s + i] behind it.
  * mla_window_plan writes, per sequence, the number of 32-key blocks between the sink and the oldest visible key (skip)
  * and the length of the sequence without them (short_lens); mla_decode_bf16_window_split is mla_decode_bf16_split over
- * those shortened sequences; the merge is mla_splitkv_reduce / mla_splitkv_reduce_vup with seq_lens = short_lens. */
+ * those shortened sequences; the merge is mla_splitkv_reduce / mla_splitkv_reduce_vup with seq_lens = short_lens.  With
+ * skip = NULL the split takes the lengths behind the sink as short_lens and works both out itself (no plan launch); the merge
+ * then takes those lengths as well. */
 int mla_window_plan(const int32_t* seq_lens, const int32_t* query_start_loc, int32_t batch, int32_t max_q_len,
                     int32_t sink_len, int32_t window, int32_t* short_lens, int32_t* skip, mlahip_stream_t stream);
 

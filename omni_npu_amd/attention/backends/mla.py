@@ -481,7 +481,7 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
             return False
         return _host.load().mla_decode(
             q, kv_cache[0], None if self.fp8_cache else kv_cache[1], d.block_table, d.seq_lens, d.query_start_loc, d.q_len,
-            d.block_table.shape[1] * K.PAGE, self.W_UK_T, self.W_UV, self.scale, attn_metadata.num_decode_tokens, self.sink_len,
+            d.max_seq_len, self.W_UK_T, self.W_UV, self.scale, attn_metadata.num_decode_tokens, self.sink_len,
             self.sliding_window if self.sink_len > 0 else 0, output)
 
     def forward(self, layer, q: torch.Tensor, k_c_normed: torch.Tensor, k_pe: torch.Tensor,

@@ -17,7 +17,6 @@
 #include "decode_params.hpp"
 
 namespace mlahip {
-constexpr int kRowsPerWg = 128;
 constexpr int kFp8RowB = 656;
 }  // namespace mlahip
 
@@ -86,11 +85,10 @@ static int decode_split_impl(const void* q_nope, int64_t qn_stride_t, int64_t qn
   v.win_skip = win_skip; v.win_sink = win_sink; v.win_size = win_size;
   v.new_c = (const __bf16*)new_c; v.new_c_st = new_c_stride; v.new_r = (const __bf16*)new_r; v.new_r_st = new_r_stride;
   v.new_slots = new_slots;
-  // one workgroup per (balanced chunk, group of 128 query rows); the chunk axis in whole eighths, one per XCD
-  v.num_chunks = plan_num_chunks(batch, num_splits, r_max);
-  const dim3 grid((unsigned)((v.num_chunks + 7) / 8 * 8), 1, (unsigned)((r_max + kRowsPerWg - 1) / kRowsPerWg));
-  if (fp8) return launch_decode_v3_fp8(v, grid, stream);
-  return launch_decode_v3(v, sparse_rows != nullptr, grid, stream);
+  const PlanForm form = plan_form(batch, num_splits, r_max);
+  v.num_chunks = form.chunks;
+  if (fp8) return launch_decode_v3_fp8(v, form.rg, stream);
+  return launch_decode_v3(v, sparse_rows != nullptr, form.rg, stream);
 }
 
 // Phase 1: one normalised fp16 partial + log-sum-exp per (segment of a chunk, query row) into the workspace.
@@ -112,7 +110,8 @@ extern "C" int mla_decode_bf16_split(const void* q_nope, int64_t qn_stride_t, in
 // Static sink tokens + sliding window on the dense kernel.  mla_window_plan turns the lengths behind the sink into the
 // lengths of the shortened sequences the kernel walks (sink keys + the blocks that hold some token's window) and the
 // number of 32-key blocks left out; mla_decode_bf16_window_split is mla_decode_bf16_split over those, and the merge is
-// the ordinary one with the shortened lengths.
+// the ordinary one with the shortened lengths.  With skip = NULL the kernel takes the lengths behind the sink and works both
+// out for itself (a launch of 5 us less), and the merge takes those lengths too: it only asks which sequences are empty.
 namespace mlahip {
 __global__ void mla_window_plan_kernel(const int32_t* seq_lens, const int32_t* qsl, int32_t batch, int32_t max_q_len,
                                        int32_t sink_len, int32_t window, int32_t* short_lens, int32_t* skip) {
@@ -120,13 +119,9 @@ __global__ void mla_window_plan_kernel(const int32_t* seq_lens, const int32_t* q
   if (b >= batch) return;
   int qlen = qsl ? qsl[b + 1] - qsl[b] : max_q_len;
   qlen = qlen < max_q_len ? qlen : max_q_len;
-  const int len = seq_lens[b];
-  int n0 = len - qlen + 1;                                   // keys the request's first query token sees
-  n0 = n0 < 0 ? 0 : n0;
-  const int lo0 = n0 > window ? n0 - window : 0;             // the oldest key any of its tokens sees
-  const int sk = lo0 / 32;
-  skip[b] = sk;
-  short_lens[b] = len > 0 ? sink_len + len - sk * 32 : 0;
+  const WindowLen w = window_len(seq_lens[b], qlen, sink_len, window);
+  skip[b] = w.skip;
+  short_lens[b] = w.len;
 }
 }  // namespace mlahip
 
@@ -150,7 +145,7 @@ extern "C" int mla_decode_bf16_window_split(const void* q_nope, int64_t qn_strid
                                             int32_t batch, int32_t max_q_len, int32_t num_heads, int32_t sink_len,
                                             int32_t window, float scale, void* workspace, size_t workspace_bytes,
                                             int32_t num_splits, hipStream_t stream) {
-  MLA_REQUIRE(block_table && skip, MLA_ERR_NULL, "mla_decode_bf16_window_split: null block table or skip counts");
+  MLA_REQUIRE(block_table, MLA_ERR_NULL, "mla_decode_bf16_window_split: null block table");
   MLA_REQUIRE(sink_len >= 0 && sink_len % kPage == 0 && window >= 1, MLA_ERR_SHAPE,
               "mla_decode_bf16_window_split: sink_len=%d window=%d", sink_len, window);
   return decode_split_impl(q_nope, qn_stride_t, qn_stride_h, q_rope, qr_stride_t, qr_stride_h, nope_cache,
@@ -168,7 +163,7 @@ extern "C" int mla_decode_fp8_window_split(const void* q_nope, int64_t qn_stride
                                            const int32_t* query_start_loc, int32_t batch, int32_t max_q_len, int32_t num_heads,
                                            int32_t sink_len, int32_t window, float scale, void* workspace,
                                            size_t workspace_bytes, int32_t num_splits, hipStream_t stream) {
-  MLA_REQUIRE(cache && block_table && skip, MLA_ERR_NULL, "mla_decode_fp8_window_split: null pointer argument");
+  MLA_REQUIRE(cache && block_table, MLA_ERR_NULL, "mla_decode_fp8_window_split: null pointer argument");
   MLA_REQUIRE(row_stride_bytes == kFp8RowB && page_stride_bytes >= (int64_t)kPage * kFp8RowB && page_stride_bytes % 16 == 0,
               MLA_ERR_UNSUPPORTED, "mla_decode_fp8_window_split: rows must be exactly 656 bytes apart, pages 128 rows (got %lld / %lld)",
               (long long)row_stride_bytes, (long long)page_stride_bytes);
@@ -203,7 +198,7 @@ extern "C" int mla_splitkv_reduce(const void* workspace, size_t workspace_bytes,
   cp.corr_scale = cp.lse_part + rows; cp.corr_row = (const __bf16* const*)(cp.lse_part + 2 * rows);
   cp.seg_ids = (const int32_t*)(cp.lse_part + 4 * rows);
   cp.seq_lens = seq_lens; cp.qsl = query_start_loc;
-  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = plan_num_chunks(batch, num_splits, r_max);
+  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = plan_form(batch, num_splits, r_max).chunks;
   cp.out = (__bf16*)out; cp.out_st = out_stride_t; cp.out_sh = out_stride_h;
   cp.lse_out = lse_out; cp.lse_st = num_heads;
   return launch_chunk_reduce(cp, stream);

@@ -13,7 +13,7 @@ struct DecodeParams {
   const int32_t* block_table; int64_t bt_stride; int32_t max_blocks;
   const int32_t* seq_lens;
   const int32_t* qsl;
-  int32_t batch, max_q_len, num_heads, num_chunks;   // num_chunks: the most chunks the plan may cut (plan_num_chunks)
+  int32_t batch, max_q_len, num_heads, num_chunks;   // num_chunks: the most chunks the plan may cut (plan_form)
   int64_t num_pages;
   float scale_log2;
   _Float16* o_part;              // [chunks + B, R_max, 512] fp16, normalised
@@ -23,9 +23,10 @@ struct DecodeParams {
   int32_t* seg_ids;              // [B][2]: partial number of the sequence's first / last segment
   const int32_t* sparse_rows; int64_t sparse_stride; int32_t page_size;
   const uint8_t* cache8; int64_t c8_sp;   // fp8 kernel: block-scaled cache, page stride in bytes (rows are 656 bytes apart)
-  // Sink + sliding window (dense bf16 kernel only): seq_lens then holds the length of the sequence with the 32-key
-  // blocks between the sink and the window taken out, win_skip[b] is how many were taken out, and a key behind the
-  // sink is visible to a row only if it is one of the newest win_size keys the row may see.
+  // Sink + sliding window (win_size > 0): seq_lens then holds the length of the sequence with the 32-key blocks between the
+  // sink and the window taken out, and win_skip[b] how many were taken out; without win_skip, seq_lens counts the keys
+  // behind the sink and the kernel works both out (window_len).  A key behind the sink is visible to a row only if it is
+  // one of the newest win_size keys the row may see.
   const int32_t* win_skip; int32_t win_sink, win_size;
   // The step's cache write folded into the dense kernel (null = the cache already holds the new rows): latent row
   // new_c[t] and rope row new_r[t] of query token t go to cache row new_slots[t] (negative = skip), written by the
@@ -56,29 +57,61 @@ __device__ __forceinline__ int plan_work_units(int len) { return len > 0 ? (len 
 // ask for hundreds of chunks where the requests at hand hold a few dozen blocks, and each chunk is one more partial to merge.
 constexpr int kPlanMinUnits = 4;
 constexpr int kPlanCUs = 256;                              // MI355X
-inline int plan_num_chunks(int64_t batch, int64_t num_splits, int64_t query_rows) {
-  const int64_t total = batch * num_splits, groups = (query_rows + 127) / 128;
-  const int64_t rounds = total * groups / kPlanCUs;
-  if (rounds < 1) return (int)total;
+// Query rows per workgroup (32 rg) and most chunks of a launch.  Requests with at most 32 / 64 query rows (tokens x heads)
+// take the forms that leave the missing rows out.  For more rows, batch * num_splits chunks of at least 256 keys each that do
+// not fill the CUs mean that the contexts are short (the caller asks for 256 chunks and more where they are long enough):
+// cutting the keys finer would make every workgroup pay a segment's start and end for a handful of blocks, so the rows are
+// cut instead, into groups of 32 or 64 with a workgroup each over the whole chunk (the groups of a chunk sit next to each other
+// on one XCD and share the cache rows in its L2).  Where the lines lie, 128 heads, us per layer as a graph replay with groups
+// of 32 / 64 / 128 rows: 7 requests of 1k-2k keys 41.6 / 43.4 / 47.5, 16 of 1k-2k 50.4 / 48.2 / 54.5, 7 of 4k-8k 59.5 / 54.9 /
+// 61.0, 16 of 4k-8k 94.7 / 77.5 / 71.8; the fp8 cache, row lists and windows alike.  (Up to three splits a caller may have asked
+// for few chunks itself, whatever the lengths: past half the CUs those keep the 128-row form.)
+struct PlanForm { int rg, chunks; };
+inline PlanForm plan_form(int64_t batch, int64_t num_splits, int64_t query_rows) {
+  const int64_t total = batch * num_splits, groups = (query_rows + 127) / 128, wgs = total * groups;
+  if (query_rows > 64 && wgs * 4 <= kPlanCUs) return {1, (int)total};
+  if (query_rows > 64 && (wgs * 2 <= kPlanCUs || (wgs < kPlanCUs && num_splits > 3))) {
+    const int64_t most = kPlanCUs / ((query_rows + 63) / 64);
+    return {2, (int)(total < most || most < 1 ? total : most)};
+  }
+  const int rg = query_rows <= 32 ? 1 : (query_rows <= 64 ? 2 : 4);
+  const int64_t rounds = wgs / kPlanCUs;
+  if (rounds < 1) return {rg, (int)total};
   int64_t g = rounds * kPlanCUs / groups;
   if (g >= 64) g &= ~int64_t(7);                           // (whole eighths, one per XCD)
-  return (int)(g < 1 ? 1 : (g < total ? g : total));
+  return {rg, (int)(g < 1 ? 1 : (g < total ? g : total))};
 }
 __device__ __forceinline__ int plan_chunk_count(int total_units, int num_chunks) {
   const int g = total_units / kPlanMinUnits;
   return g < 1 ? 1 : (g < num_chunks ? g : num_chunks);
 }
 
+// Sink + window: a sequence of `len` keys behind the sink, of which the request's qlen query tokens see the newest `window` each
+// and the sink, walked without the `skip` 32-key blocks that lie between the sink and the oldest key any of them sees.
+struct WindowLen { int len, skip; };
+__device__ __forceinline__ WindowLen window_len(int len, int qlen, int sink_len, int window) {
+  int n0 = len - qlen + 1;                                   // keys the request's first query token sees
+  n0 = n0 < 0 ? 0 : n0;
+  const int sk = (n0 > window ? n0 - window : 0) / 32;
+  return {len > 0 ? sink_len + len - sk * 32 : 0, sk};
+}
+
 // Merge of the partials fused with the value up-projection (reduce_vup.hip): out[t, n*128 + v] = merged o[t,n,:] . W_UV[n,:,v]
 int launch_reduce_vup(const ChunkReduceParams& r, const void* w_uv, int64_t w_stride_n, int64_t w_stride_k,
                       int32_t num_tokens, hipStream_t stream);
 
-// The eight-wavefront kernel over the bf16 cache (decode_v3.hip): dense, row-list (sparse) and, with p.win_skip set, sink +
+// One workgroup per (balanced chunk, group of 32 rg query rows); the chunk axis in whole eighths, one per XCD.
+inline dim3 plan_grid(const DecodeParams& p, int rg) {
+  const int64_t rows = (int64_t)p.max_q_len * p.num_heads;
+  return dim3((unsigned)((p.num_chunks + 7) / 8 * 8), 1, (unsigned)((rows + 32 * rg - 1) / (32 * rg)));
+}
+// The eight-wavefront kernel over the bf16 cache (decode_v3.hip): dense, row-list (sparse) and, with p.win_size > 0, sink +
 // window.  Returns 0 or a negative error code.
-int launch_decode_v3(const DecodeParams& p, bool sparse, dim3 grid, hipStream_t stream);
+// rg: groups of 32 query rows per workgroup (plan_form).
+int launch_decode_v3(const DecodeParams& p, bool sparse, int rg, hipStream_t stream);
 // The dynamic-LDS limit of all dense bf16 forms raised on the current device, ahead of a launch under stream capture.
 int prepare_decode_v3_dense_forms();
-// The same over the fp8 block-scaled cache p.cache8 (decode_v3_fp8.hip): dense and, with p.win_skip set, sink + window.
-int launch_decode_v3_fp8(const DecodeParams& p, dim3 grid, hipStream_t stream);
+// The same over the fp8 block-scaled cache p.cache8 (decode_v3_fp8.hip): dense and, with p.win_size > 0, sink + window.
+int launch_decode_v3_fp8(const DecodeParams& p, int rg, hipStream_t stream);
 
 }  // namespace mlahip

@@ -135,6 +135,18 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
     return kp;
   };
 
+  // (length of sequence i as the blocks are numbered: of the shortened sequence in the window variant)
+  auto len_of = [&](int i) -> int {
+    const int len = p.seq_lens[i];
+    if constexpr (kWindow) {
+      if (!p.win_skip) {
+        int ql = p.qsl ? p.qsl[i + 1] - p.qsl[i] : p.max_q_len;
+        ql = ql < p.max_q_len ? ql : p.max_q_len;
+        return window_len(len, ql, p.win_sink, p.win_size).len;
+      }
+    }
+    return len;
+  };
   // ---- which blocks are mine: the balanced chunk plan (see mla_chunk_reduce_kernel, which recomputes it) ----
   // Every non-empty sequence is kSegCost units of start-up followed by its 32-key blocks, the sequences end to end, and
   // that line is cut into plan_chunk_count() chunks of equal length; a chunk that crosses a sequence boundary runs several
@@ -151,12 +163,12 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
     int my_len = 0, my_q0 = 0, my_q1 = 0;
     if (one_pass) {
       if (lane < p.batch) {
-        my_len = p.seq_lens[lane];
+        my_len = len_of(lane);
         if (p.qsl) { my_q0 = p.qsl[lane]; my_q1 = p.qsl[lane + 1]; }
       }
       tot = work_units(my_len);
     } else {
-      for (int i = lane; i < p.batch; i += 64) tot += work_units(p.seq_lens[i]);
+      for (int i = lane; i < p.batch; i += 64) tot += work_units(len_of(i));
     }
     int pe1 = 0;
     if (one_pass) { pe1 = wave_incl_scan_dpp(tot); tot = __builtin_amdgcn_readlane(pe1, 63); }
@@ -185,7 +197,7 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
     } else {
       for (int base = 0; base < p.batch; base += 64) {
         const int i = base + lane;
-        const int c = i < p.batch ? work_units(p.seq_lens[i]) : 0;
+        const int c = i < p.batch ? work_units(len_of(i)) : 0;
         const int pe = wave_incl_scan_i32(c, lane) + carry;
         const bool le = i < p.batch && pe <= cb;
         b0 += __builtin_popcountll(__builtin_amdgcn_ballot_w64(le));
@@ -209,7 +221,7 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
   if (seg_b >= p.batch) break;
   const int b = seg_b;
   const bool seg_known = first_L >= 0;                        // (only in the first pass of this loop)
-  const int L = seg_known ? first_L : p.seq_lens[b];
+  const int L = seg_known ? first_L : len_of(b);
   const int known_q0 = first_q0, known_q1 = first_q1;
   first_L = -1;
   const int64_t v_b = v_seq;
@@ -289,7 +301,7 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
       *(u32x2*)(lds + kKTabOff + lane * 8) = kr;
     }
   }
-  const int win_skip = kWindow ? p.win_skip[b] : 0;
+  const int win_skip = !kWindow ? 0 : (p.win_skip ? p.win_skip[b] : window_len(p.seq_lens[b], qlen, p.win_sink, p.win_size).skip);
   const int win_blk0 = kWindow ? p.win_sink / kBlk : 0;
   const int64_t part_base = (int64_t)(chunk + b) * r_max + grp * kGrpRows;   // + row index in the group
 
@@ -1045,17 +1057,14 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
 }  // namespace v3
 
 template <bool kSparse, bool kWindow, int kRG, bool kWrite = false>
-static int launch_form(const DecodeParams& p, dim3 grid, hipStream_t stream) {
+static int launch_form(const DecodeParams& p, hipStream_t stream) {
   const int rc = ensure_dynamic_lds((const void*)v3::mla_decode_v3_kernel<kSparse, kWindow, kRG, kWrite>, v3::kLdsB, "mla_decode_v3_kernel");
   if (rc != MLA_OK) return rc;
-  hipLaunchKernelGGL((v3::mla_decode_v3_kernel<kSparse, kWindow, kRG, kWrite>), grid, dim3(512), v3::kLdsB, stream, p);
+  hipLaunchKernelGGL((v3::mla_decode_v3_kernel<kSparse, kWindow, kRG, kWrite>), plan_grid(p, kRG), dim3(512), v3::kLdsB, stream, p);
   return check_launch("mla_decode_v3_kernel");
 }
-constexpr int kNumCUs = 256;                               // MI355X
 template <bool kSparse, bool kWindow, bool kWrite = false>
-static int launch_rows(const DecodeParams& p, dim3 grid, hipStream_t stream) {
-  // requests with at most 32 / 64 query rows (tokens x heads) take the forms that leave the missing rows out
-  const int64_t r_max = (int64_t)p.max_q_len * p.num_heads;
+static int launch_rows(const DecodeParams& p, int rg, hipStream_t stream) {
   // (the form depends on the shape; all three get their LDS limit with the family's first launch, so that a later launch
   // under stream capture, where the limit cannot be raised, finds every form ready)
   {
@@ -1064,19 +1073,9 @@ static int launch_rows(const DecodeParams& p, dim3 grid, hipStream_t stream) {
     if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)v3::mla_decode_v3_kernel<kSparse, kWindow, 4, kWrite>, v3::kLdsB, "mla_decode_v3_kernel");
     if (rc != MLA_OK) return rc;
   }
-  if (r_max <= 32) return launch_form<kSparse, kWindow, 1, kWrite>(p, grid, stream);
-  if (r_max <= 64) return launch_form<kSparse, kWindow, 2, kWrite>(p, grid, stream);
-  // With few requests and short contexts (and with row lists, which are short by nature) the caller's chunks do not fill
-  // the 256 CUs, and cutting the keys finer makes every workgroup pay a segment's start and end for a handful of blocks.
-  // The rows are cut instead: groups of 64 or 32 rows, each with its own workgroup over the whole chunk (the groups of a
-  // chunk sit next to each other on one XCD and share the cache rows in its L2).  Measured on row lists of 2048 keys,
-  // 128 heads, eight chunks per token: 4 tokens 36.1 -> 26.9 us, 8 tokens 37.7 -> 28.8, 16 tokens 40.4 -> 33.3.
-  {
-    const int64_t wgs = (int64_t)p.num_chunks * grid.z;
-    if (wgs * 4 <= kNumCUs) { grid.z = (unsigned)((r_max + 31) / 32); return launch_form<kSparse, kWindow, 1, kWrite>(p, grid, stream); }
-    if (wgs * 2 <= kNumCUs) { grid.z = (unsigned)((r_max + 63) / 64); return launch_form<kSparse, kWindow, 2, kWrite>(p, grid, stream); }
-  }
-  return launch_form<kSparse, kWindow, 4, kWrite>(p, grid, stream);
+  if (rg == 1) return launch_form<kSparse, kWindow, 1, kWrite>(p, stream);
+  if (rg == 2) return launch_form<kSparse, kWindow, 2, kWrite>(p, stream);
+  return launch_form<kSparse, kWindow, 4, kWrite>(p, stream);
 }
 
 // Raises the dynamic-LDS limit of every dense form on the current device (what a launch does for its own form the first
@@ -1088,11 +1087,11 @@ int prepare_decode_v3_dense_forms() {
   return rc;
 }
 
-int launch_decode_v3(const DecodeParams& p, bool sparse, dim3 grid, hipStream_t stream) {
-  if (sparse) return launch_rows<true, false>(p, grid, stream);
-  if (p.win_skip) return launch_rows<false, true>(p, grid, stream);
-  if (p.new_c) return launch_rows<false, false, true>(p, grid, stream);
-  return launch_rows<false, false>(p, grid, stream);
+int launch_decode_v3(const DecodeParams& p, bool sparse, int rg, hipStream_t stream) {
+  if (sparse) return launch_rows<true, false>(p, rg, stream);
+  if (p.win_size > 0) return launch_rows<false, true>(p, rg, stream);
+  if (p.new_c) return launch_rows<false, false, true>(p, rg, stream);
+  return launch_rows<false, false>(p, rg, stream);
 }
 
 }  // namespace mlahip

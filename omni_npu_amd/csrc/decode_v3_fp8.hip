@@ -119,6 +119,18 @@ __global__ __launch_bounds__(512) void mla_decode_v3_fp8_kernel(const DecodePara
     return kp;
   };
 
+  // (length of sequence i as the blocks are numbered: of the shortened sequence in the window variant)
+  auto len_of = [&](int i) -> int {
+    const int len = p.seq_lens[i];
+    if constexpr (kWindow) {
+      if (!p.win_skip) {
+        int ql = p.qsl ? p.qsl[i + 1] - p.qsl[i] : p.max_q_len;
+        ql = ql < p.max_q_len ? ql : p.max_q_len;
+        return window_len(len, ql, p.win_sink, p.win_size).len;
+      }
+    }
+    return len;
+  };
   // ---- which blocks are mine: the balanced chunk plan (see mla_chunk_reduce_kernel, which recomputes it) ----
   // Every non-empty sequence is kSegCost units of start-up followed by its 32-key blocks, the sequences end to end, and
   // that line is cut into plan_chunk_count() chunks of equal length; a chunk that crosses a sequence boundary runs several
@@ -135,12 +147,12 @@ __global__ __launch_bounds__(512) void mla_decode_v3_fp8_kernel(const DecodePara
     int my_len = 0, my_q0 = 0, my_q1 = 0;
     if (one_pass) {
       if (lane < p.batch) {
-        my_len = p.seq_lens[lane];
+        my_len = len_of(lane);
         if (p.qsl) { my_q0 = p.qsl[lane]; my_q1 = p.qsl[lane + 1]; }
       }
       tot = work_units(my_len);
     } else {
-      for (int i = lane; i < p.batch; i += 64) tot += work_units(p.seq_lens[i]);
+      for (int i = lane; i < p.batch; i += 64) tot += work_units(len_of(i));
     }
     int pe1 = 0;
     if (one_pass) { pe1 = wave_incl_scan_dpp(tot); tot = __builtin_amdgcn_readlane(pe1, 63); }
@@ -169,7 +181,7 @@ __global__ __launch_bounds__(512) void mla_decode_v3_fp8_kernel(const DecodePara
     } else {
       for (int base = 0; base < p.batch; base += 64) {
         const int i = base + lane;
-        const int c = i < p.batch ? work_units(p.seq_lens[i]) : 0;
+        const int c = i < p.batch ? work_units(len_of(i)) : 0;
         const int pe = wave_incl_scan_i32(c, lane) + carry;
         const bool le = i < p.batch && pe <= cb;
         b0 += __builtin_popcountll(__builtin_amdgcn_ballot_w64(le));
@@ -193,7 +205,7 @@ __global__ __launch_bounds__(512) void mla_decode_v3_fp8_kernel(const DecodePara
   if (seg_b >= p.batch) break;
   const int b = seg_b;
   const bool seg_known = first_L >= 0;                        // (only in the first pass of this loop)
-  const int L = seg_known ? first_L : p.seq_lens[b];
+  const int L = seg_known ? first_L : len_of(b);
   const int known_q0 = first_q0, known_q1 = first_q1;
   first_L = -1;
   const int64_t v_b = v_seq;
@@ -248,7 +260,7 @@ __global__ __launch_bounds__(512) void mla_decode_v3_fp8_kernel(const DecodePara
       *(u32x2*)(lds + kKTabOff + lane * 8) = kr;
     }
   }
-  const int win_skip = kWindow ? p.win_skip[b] : 0;
+  const int win_skip = !kWindow ? 0 : (p.win_skip ? p.win_skip[b] : window_len(p.seq_lens[b], qlen, p.win_sink, p.win_size).skip);
   const int win_blk0 = kWindow ? p.win_sink / kBlk : 0;
   const int64_t part_base = (int64_t)(chunk + b) * r_max + grp * kGrpRows;   // + row index in the group
 
@@ -795,16 +807,14 @@ __global__ __launch_bounds__(512) void mla_decode_v3_fp8_kernel(const DecodePara
 }  // namespace f8v3
 
 template <bool kWindow, int kRG>
-static int launch_form_fp8(const DecodeParams& p, dim3 grid, hipStream_t stream) {
+static int launch_form_fp8(const DecodeParams& p, hipStream_t stream) {
   const int rc = ensure_dynamic_lds((const void*)f8v3::mla_decode_v3_fp8_kernel<kWindow, kRG>, f8v3::kLdsB, "mla_decode_v3_fp8_kernel");
   if (rc != MLA_OK) return rc;
-  hipLaunchKernelGGL((f8v3::mla_decode_v3_fp8_kernel<kWindow, kRG>), grid, dim3(512), f8v3::kLdsB, stream, p);
+  hipLaunchKernelGGL((f8v3::mla_decode_v3_fp8_kernel<kWindow, kRG>), plan_grid(p, kRG), dim3(512), f8v3::kLdsB, stream, p);
   return check_launch("mla_decode_v3_fp8_kernel");
 }
 template <bool kWindow>
-static int launch_rows_fp8(const DecodeParams& p, dim3 grid, hipStream_t stream) {
-  // requests with at most 32 / 64 query rows (tokens x heads) take the forms that leave the missing rows out
-  const int64_t r_max = (int64_t)p.max_q_len * p.num_heads;
+static int launch_rows_fp8(const DecodeParams& p, int rg, hipStream_t stream) {
   // (all three forms get their LDS limit with the family's first launch: a later launch under stream capture finds them ready)
   {
     int rc = ensure_dynamic_lds((const void*)f8v3::mla_decode_v3_fp8_kernel<kWindow, 1>, f8v3::kLdsB, "mla_decode_v3_fp8_kernel");
@@ -812,20 +822,14 @@ static int launch_rows_fp8(const DecodeParams& p, dim3 grid, hipStream_t stream)
     if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)f8v3::mla_decode_v3_fp8_kernel<kWindow, 4>, f8v3::kLdsB, "mla_decode_v3_fp8_kernel");
     if (rc != MLA_OK) return rc;
   }
-  if (r_max <= 32) return launch_form_fp8<kWindow, 1>(p, grid, stream);
-  if (r_max <= 64) return launch_form_fp8<kWindow, 2>(p, grid, stream);
-  // (few chunks: the rows are cut into groups of 32 or 64 with a workgroup each, as in the kernel over the bf16 cache)
-  {
-    const int64_t wgs = (int64_t)p.num_chunks * grid.z;
-    if (wgs * 4 <= 256) { grid.z = (unsigned)((r_max + 31) / 32); return launch_form_fp8<kWindow, 1>(p, grid, stream); }
-    if (wgs * 2 <= 256) { grid.z = (unsigned)((r_max + 63) / 64); return launch_form_fp8<kWindow, 2>(p, grid, stream); }
-  }
-  return launch_form_fp8<kWindow, 4>(p, grid, stream);
+  if (rg == 1) return launch_form_fp8<kWindow, 1>(p, stream);
+  if (rg == 2) return launch_form_fp8<kWindow, 2>(p, stream);
+  return launch_form_fp8<kWindow, 4>(p, stream);
 }
 
-int launch_decode_v3_fp8(const DecodeParams& p, dim3 grid, hipStream_t stream) {
-  if (p.win_skip) return launch_rows_fp8<true>(p, grid, stream);
-  return launch_rows_fp8<false>(p, grid, stream);
+int launch_decode_v3_fp8(const DecodeParams& p, int rg, hipStream_t stream) {
+  if (p.win_size > 0) return launch_rows_fp8<true>(p, rg, stream);
+  return launch_rows_fp8<false>(p, rg, stream);
 }
 
 }  // namespace mlahip

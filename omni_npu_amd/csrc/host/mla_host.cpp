@@ -13,6 +13,7 @@
 #include <torch/extension.h>
 #include <ATen/core/LegacyTypeDispatch.h>
 #include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 
 #include <map>
@@ -142,9 +143,11 @@ void merge_vup(const Tensor& ws, const Tensor& lens, const OptTensor& qsl, int64
 }
 
 // One layer's decode tokens, their rows in the cache already: absorption, split-KV attention, merge + up-projection.  rope =
-// None: the fp8 cache.  window > 0: static sink + sliding window.
+// None: the fp8 cache.  window > 0: static sink + sliding window.  The launch is shaped for the step's own longest context
+// (step_max_len, 0 = unknown), and under capture for the longest the block table can hold, as a graph is replayed over others;
+// either way it is right for any length.
 bool mla_decode(const Tensor& q, const Tensor& nope, const OptTensor& rope, const Tensor& block_table, const Tensor& seq_lens, const OptTensor& qsl, int64_t q_len,
-                int64_t max_seq_len, const Tensor& w_uk, const Tensor& w_uv, double scale, int64_t t, int64_t sink, int64_t window,
+                int64_t step_max_len, const Tensor& w_uk, const Tensor& w_uv, double scale, int64_t t, int64_t sink, int64_t window,
                 const Tensor& out) {
   if (!current_gpu(q)) return false;
   const at::Device dev = q.device();
@@ -159,6 +162,9 @@ bool mla_decode(const Tensor& q, const Tensor& nope, const OptTensor& rope, cons
   Stream st = stream_of(q);
   const bool fp8 = !rope;
   Tensor ql = absorb(q, w_uk, t);
+  int64_t max_seq_len = block_table.size(1) * kPage;
+  if (step_max_len > 0 && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None)
+    max_seq_len = std::min(max_seq_len, step_max_len + sink);
   if (window > 0) max_seq_len = std::min(max_seq_len, sink + window + 32 + q_len);
   const int splits = default_splits(b, q_len, n, max_seq_len);
   const int64_t need = (int64_t)mla_decode_workspace_bytes((int)b, (int)q_len, (int)n, splits);
@@ -170,20 +176,14 @@ bool mla_decode(const Tensor& q, const Tensor& nope, const OptTensor& rope, cons
   const int32_t* qs = qsl ? (const int32_t*)qsl->data_ptr() : nullptr;
   const char* qr = (const char*)q.data_ptr() + 2 * 128;
   const int64_t ql_t = ql.stride(1), ql_h = ql.stride(0);
-  Tensor plan;
-  const Tensor* merged_lens = &seq_lens;
   if (window > 0) {
-    plan = at::empty({2, b}, seq_lens.options());
-    int32_t *short_lens = (int32_t*)plan.data_ptr(), *skip = short_lens + b;
-    check(mla_window_plan(lens, qs, (int)b, (int)q_len, (int)sink, (int)window, short_lens, skip, st), "mla_window_plan");
-    merged_lens = &plan;                                       // (its first row)
     if (fp8)
       check(mla_decode_fp8_window_split(ql.data_ptr(), ql_t, ql_h, qr, q.stride(0), q.stride(1), c.nope->data_ptr(), c.n_sp, c.n_sr,
-                                        c.pages, bt, bts, mb, short_lens, skip, qs, (int)b, (int)q_len, (int)n, (int)sink,
+                                        c.pages, bt, bts, mb, lens, nullptr, qs, (int)b, (int)q_len, (int)n, (int)sink,
                                         (int)window, (float)scale, ws.data_ptr(), ws.numel(), splits, st), "mla_decode_fp8_window_split");
     else
       check(mla_decode_bf16_window_split(ql.data_ptr(), ql_t, ql_h, qr, q.stride(0), q.stride(1), c.nope->data_ptr(), c.n_sp, c.n_sr,
-                                         c.rope->data_ptr(), c.r_sp, c.r_sr, c.pages, bt, bts, mb, short_lens, skip, qs, (int)b,
+                                         c.rope->data_ptr(), c.r_sp, c.r_sr, c.pages, bt, bts, mb, lens, nullptr, qs, (int)b,
                                          (int)q_len, (int)n, (int)sink, (int)window, (float)scale, ws.data_ptr(), ws.numel(),
                                          splits, st), "mla_decode_bf16_window_split");
   } else if (fp8) {
@@ -195,7 +195,7 @@ bool mla_decode(const Tensor& q, const Tensor& nope, const OptTensor& rope, cons
                                 c.rope->data_ptr(), c.r_sp, c.r_sr, c.pages, bt, bts, mb, lens, qs, (int)b, (int)q_len, (int)n,
                                 (float)scale, ws.data_ptr(), ws.numel(), splits, st), "mla_decode_bf16_split");
   }
-  merge_vup(ws, *merged_lens, qsl, b, q_len, n, splits, t, w_uv, out, st);
+  merge_vup(ws, seq_lens, qsl, b, q_len, n, splits, t, w_uv, out, st);
   return true;
 }
 

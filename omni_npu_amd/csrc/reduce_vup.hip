@@ -317,7 +317,7 @@ extern "C" int mla_splitkv_reduce_vup(const void* workspace, size_t workspace_by
   cp.corr_scale = cp.lse_part + rows; cp.corr_row = (const __bf16* const*)(cp.lse_part + 2 * rows);
   cp.seg_ids = (const int32_t*)(cp.lse_part + 4 * rows);
   cp.seq_lens = seq_lens; cp.qsl = query_start_loc;
-  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = plan_num_chunks(batch, num_splits, r_max);
+  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = plan_form(batch, num_splits, r_max).chunks;
   cp.out = (__bf16*)out; cp.out_st = out_stride_t; cp.out_sh = out_stride_h;
   cp.lse_out = nullptr; cp.lse_st = 0;
   return launch_reduce_vup(cp, w_uv, w_stride_n, w_stride_k, num_tokens, stream);

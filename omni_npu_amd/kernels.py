@@ -573,9 +573,8 @@ def decode(q_nope: torch.Tensor, q_rope: torch.Tensor, nope_cache: torch.Tensor,
 
 def _decode_window(q_nope, q_rope, nope_cache, rope_cache, block_table, seq_lens, scale, out, q_len, query_start_loc,
                    lse_out, num_splits, max_seq_len, workspace, phase, w_uv, sink_len, window):
-    """decode() with static sink keys and a sliding window: a plan kernel shortens every sequence to sink + window
-    blocks, the dense split kernel walks the shortened sequences, and the ordinary merge (or merge + up-projection)
-    follows with the shortened lengths."""
+    """decode() with static sink keys and a sliding window: the dense split kernel walks every sequence shortened to
+    its sink + window blocks, and the ordinary merge (or merge + up-projection) follows."""
     if phase != "both":
         raise ValueError("decode: the windowed decode runs both phases")
     if window < 1 or sink_len < 0 or sink_len % PAGE != 0:
@@ -589,17 +588,14 @@ def _decode_window(q_nope, q_rope, nope_cache, rope_cache, block_table, seq_lens
     lib, front, ws_args, lse_p, st, qsl, seq_lens, b, n, num_splits = _decode_args(
         q_nope, q_rope, nope_cache, rope_cache, block_table, seq_lens, scale, out if o3 is None else o3,
         D_NOPE if o3 is None else 128, q_len, query_start_loc, lse_out, num_splits, max_seq_len, workspace)
-    plan = torch.empty(2, b, dtype=torch.int32, device=q_nope.device)      # shortened lengths, blocks left out
-    short, skip = plan[0], plan[1]
-    _lib.check(lib.mla_window_plan(seq_lens.data_ptr(), qsl, b, q_len, sink_len, window, short.data_ptr(), skip.data_ptr(), st),
-               "mla_window_plan")
-    rc = lib.mla_decode_bf16_window_split(*front[:16], short.data_ptr(), skip.data_ptr(), qsl, b, q_len, n, sink_len, window,
+    # (lengths behind the sink and no skip counts: the kernels work the shortened lengths out for themselves)
+    rc = lib.mla_decode_bf16_window_split(*front[:16], seq_lens.data_ptr(), None, qsl, b, q_len, n, sink_len, window,
                                           float(scale), *ws_args, num_splits, st)
     _lib.check(rc, "mla_decode_bf16_window_split")
     if o3 is not None:
-        _reduce_vup(lib, ws_args, short, qsl, b, q_len, n, num_splits, t, w_uv, o3, st)
+        _reduce_vup(lib, ws_args, seq_lens, qsl, b, q_len, n, num_splits, t, w_uv, o3, st)
     else:
-        rc = lib.mla_splitkv_reduce(*ws_args, short.data_ptr(), qsl, b, q_len, n, num_splits, out.data_ptr(), out.stride(0),
+        rc = lib.mla_splitkv_reduce(*ws_args, seq_lens.data_ptr(), qsl, b, q_len, n, num_splits, out.data_ptr(), out.stride(0),
                                     out.stride(1), lse_p, st)
         _lib.check(rc, "mla_splitkv_reduce")
     return out
@@ -963,20 +959,16 @@ def decode_fp8(q_nope: torch.Tensor, q_rope: torch.Tensor, cache: torch.Tensor, 
         st = _stream(q_nope)
         qsl = query_start_loc.data_ptr() if query_start_loc is not None else None
         ws_args = (ws.data_ptr(), ws.numel() * ws.element_size())
-        plan = torch.empty(2, b, dtype=torch.int32, device=q_nope.device)  # shortened lengths, blocks left out
-        short, skip = plan[0], plan[1]
-        _lib.check(lib.mla_window_plan(seq_lens.data_ptr(), qsl, b, q_len, sink_len, window, short.data_ptr(),
-                                       skip.data_ptr(), st), "mla_window_plan")
         rc = lib.mla_decode_fp8_window_split(
             q_nope.data_ptr(), q_nope.stride(0), q_nope.stride(1), q_rope.data_ptr(), q_rope.stride(0), q_rope.stride(1),
             cache.data_ptr(), cache.stride(0), cache.stride(1), cache.shape[0], block_table.data_ptr(), block_table.stride(0),
-            block_table.shape[1], short.data_ptr(), skip.data_ptr(), qsl, b, q_len, n, sink_len, window, float(scale),
+            block_table.shape[1], seq_lens.data_ptr(), None, qsl, b, q_len, n, sink_len, window, float(scale),
             *ws_args, num_splits, st)
         _lib.check(rc, "mla_decode_fp8_window_split")
         if o3 is not None:
-            _reduce_vup(lib, ws_args, short, qsl, b, q_len, n, num_splits, t, w_uv, o3, st)
+            _reduce_vup(lib, ws_args, seq_lens, qsl, b, q_len, n, num_splits, t, w_uv, o3, st)
         else:
-            rc = lib.mla_splitkv_reduce(*ws_args, short.data_ptr(), qsl, b, q_len, n, num_splits, out.data_ptr(), out.stride(0),
+            rc = lib.mla_splitkv_reduce(*ws_args, seq_lens.data_ptr(), qsl, b, q_len, n, num_splits, out.data_ptr(), out.stride(0),
                                         out.stride(1), lse_out.data_ptr() if lse_out is not None else None, st)
             _lib.check(rc, "mla_splitkv_reduce")
         return out

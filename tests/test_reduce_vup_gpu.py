@@ -145,3 +145,12 @@ def test_fused_up_projection_after_fp8_and_sparse_decode(dev):
 ])
 def test_chunk_plan_and_shared_rows_at_their_edges(dev, batch, heads, q_len, lo, hi, splits):
     test_fused_merge_and_up_projection(dev, batch, heads, q_len, lo, hi, splits)
+
+
+@pytest.mark.parametrize("batch,heads,q_len,lo,hi,splits", [
+    (2, 128, 1, 40, 300, 32), (3, 128, 2, 40, 300, 16),       # groups of 32 rows: 64 chunks x 4, 48 x 8 (chunks below the CUs)
+    (7, 128, 1, 300, 3000, 32), (24, 128, 1, 100, 700, 8),    # groups of 64: 224 and 192 chunks cut to 128
+    (7, 80, 1, 300, 900, 32), (31, 65, 1, 100, 500, 8),       # a last group of 16 rows, of one
+])
+def test_row_groups_at_their_edges(dev, batch, heads, q_len, lo, hi, splits):
+    test_fused_merge_and_up_projection(dev, batch, heads, q_len, lo, hi, splits)
