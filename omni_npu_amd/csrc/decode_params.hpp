@@ -55,7 +55,12 @@ __device__ __forceinline__ int plan_work_units(int len) { return len > 0 ? (len 
 // CUs take as long as 512 would (48 requests x 6 splits, 32 rows: 105 us against 74 with 256 chunks).  The device, which
 // knows the lengths, cuts no finer than kPlanMinUnits units: block tables as wide as the longest context a server accepts
 // ask for hundreds of chunks where the requests at hand hold a few dozen blocks, and each chunk is one more partial to merge.
+// A block costs a workgroup 1.5 us of dependent steps, so while the partials are few (kPlanFineRows rows of 1 KiB) the cut
+// goes down to kPlanFineUnits: 1021 keys x 16 heads, us of split and merge, 26.0 in chunks of eight blocks, 19.3 of four, 17.6
+// of two; 2 requests of 500-1500 keys x 128 heads 24.9 -> 21.1; 7 of 300-3000 keys, beyond the line, 31.7 -> 33.3.
 constexpr int kPlanMinUnits = 4;
+constexpr int kPlanFineUnits = 2;
+constexpr int kPlanFineRows = 8192;
 constexpr int kPlanCUs = 256;                              // MI355X
 // Query rows per workgroup (32 rg) and most chunks of a launch.  Requests with at most 32 / 64 query rows (tokens x heads)
 // take the forms that leave the missing rows out.  For more rows, batch * num_splits chunks of at least 256 keys each that do
@@ -81,8 +86,10 @@ inline PlanForm plan_form(int64_t batch, int64_t num_splits, int64_t query_rows)
   if (g >= 64) g &= ~int64_t(7);                           // (whole eighths, one per XCD)
   return {rg, (int)(g < 1 ? 1 : (g < total ? g : total))};
 }
-__device__ __forceinline__ int plan_chunk_count(int total_units, int num_chunks) {
-  const int g = total_units / kPlanMinUnits;
+__device__ __forceinline__ int plan_chunk_count(int total_units, int rows_per_seq, int num_chunks) {
+  const int fine = total_units / kPlanFineUnits, few = kPlanFineRows / rows_per_seq;
+  int g = total_units / kPlanMinUnits;
+  g = fine <= few ? fine : (g > few ? g : few);
   return g < 1 ? 1 : (g < num_chunks ? g : num_chunks);
 }
 

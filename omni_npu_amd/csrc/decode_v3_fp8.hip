@@ -159,7 +159,7 @@ __global__ __launch_bounds__(512) void mla_decode_v3_fp8_kernel(const DecodePara
     else tot = __builtin_amdgcn_readfirstlane(wave_sum_i32(tot));
     // chunk c covers units [floor(c * tot / G), floor((c + 1) * tot / G)); with G <= 65536 that is 32-bit arithmetic:
     // c * tot / G = c * (tot / G) + c * (tot % G) / G exactly (a 64-bit division is a long software routine)
-    const int chunks = plan_chunk_count(tot, p.num_chunks), per_xcd = (chunks + 7) >> 3;
+    const int chunks = plan_chunk_count(tot, r_max, p.num_chunks), per_xcd = (chunks + 7) >> 3;
     chunk = xcd * per_xcd + xcd_j;
     if (xcd_j >= per_xcd || chunk >= chunks || tot == 0) return;
     int64_t cb, ce;

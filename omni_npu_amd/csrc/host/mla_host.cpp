@@ -59,11 +59,13 @@ Tensor& scratch(const Tensor& like, Stream stream, int64_t bytes, int tag) {
 }
 
 int64_t div_up(int64_t a, int64_t b) { return (a + b - 1) / b; }
-// kernels.default_num_splits
-int default_splits(int64_t batch, int64_t q_len, int64_t heads, int64_t max_seq_len) {
+// kernels.launch_splits
+int launch_splits(int64_t batch, int64_t q_len, int64_t heads, int64_t max_seq_len) {
   const int64_t groups = std::max<int64_t>(batch * div_up(q_len * heads, 128), 1);
   const int64_t by_length = std::max<int64_t>(1, div_up(max_seq_len, 256));
-  return (int)std::max<int64_t>(1, std::min({std::max<int64_t>(1, div_up(256, groups)), by_length, (int64_t)256}));
+  int64_t splits = std::max<int64_t>(1, std::min({std::max<int64_t>(1, div_up(256, groups)), by_length, (int64_t)256}));
+  if (groups * splits * 4 <= 256) splits = std::max(splits, 256 / (4 * groups));
+  return (int)splits;
 }
 
 struct Cache {
@@ -166,7 +168,7 @@ bool mla_decode(const Tensor& q, const Tensor& nope, const OptTensor& rope, cons
   if (step_max_len > 0 && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None)
     max_seq_len = std::min(max_seq_len, step_max_len + sink);
   if (window > 0) max_seq_len = std::min(max_seq_len, sink + window + 32 + q_len);
-  const int splits = default_splits(b, q_len, n, max_seq_len);
+  const int splits = launch_splits(b, q_len, n, max_seq_len);
   const int64_t need = (int64_t)mla_decode_workspace_bytes((int)b, (int)q_len, (int)n, splits);
   Tensor& ws = scratch(q, st, need, 0);
   const int32_t* bt = (const int32_t*)block_table.data_ptr();
@@ -210,7 +212,7 @@ bool sparse_decode(const Tensor& q, const Tensor& nope, const Tensor& rope, cons
   if (!layer_ok(q, w_uk, w_uv, out, t, dev) || !cache_of(nope, r, dev, c) || !is_i32(rows, 2, dev) || rows.size(0) < t || !is_i32(counts, 1, dev) || !counts.is_contiguous() || counts.numel() < t)
     return false;
   const int64_t n = q.size(1);
-  const int splits = default_splits(t, 1, n, rows.size(1));
+  const int splits = launch_splits(t, 1, n, rows.size(1));
   const int64_t need = (int64_t)mla_decode_workspace_bytes((int)t, 1, (int)n, splits);
   if (need > (256 << 20)) return false;                        // kernels.SPARSE_WORKSPACE_CAP
   at::AutoDispatchBelowAutograd guard;

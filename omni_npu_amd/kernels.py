@@ -418,6 +418,15 @@ def default_num_splits(batch: int, max_q_len: int, num_heads: int, max_seq_len: 
     return int(max(1, min(want, by_length, 256)))
 
 
+def launch_splits(batch: int, max_q_len: int, num_heads: int, max_seq_len: int, num_cus: int = 256) -> int:
+    """The split count the wrappers launch with: default_num_splits, but as many as give every CU a workgroup of 32 query rows
+    where that is more.  (The plan on the device settles the cut: it knows the lengths, and how many partials it takes
+    before finer chunks cost more than they save; workgroups it has no chunk for leave at once.)"""
+    splits = default_num_splits(batch, max_q_len, num_heads, max_seq_len, num_cus)
+    groups = max(1, batch * math.ceil(max_q_len * num_heads / 128))
+    return max(splits, num_cus // (4 * groups)) if groups * splits * 4 <= num_cus else splits
+
+
 def _vup_out(out: torch.Tensor, w_uv: torch.Tensor, t: int, n: int) -> torch.Tensor:
     """The [T,N,128] view of the output of a decode with the value up-projection fused in, after checking w_uv."""
     _need_cuda(w_uv)
@@ -477,7 +486,7 @@ def _decode_args(q_nope, q_rope, nope_cache, rope_cache, block_table, seq_lens, 
     if nope.shape[1] != PAGE:
         raise ValueError("decode: page size must be 128")
     if num_splits is None:
-        num_splits = default_num_splits(b, q_len, n, max_seq_len)
+        num_splits = launch_splits(b, q_len, n, max_seq_len)
     need = lib.mla_decode_workspace_bytes(b, q_len, n, num_splits)
     ws = workspace if workspace is not None else _workspace(q_nope.device, need)
     qsl = query_start_loc.data_ptr() if query_start_loc is not None else None
@@ -780,7 +789,7 @@ def sparse_decode(q_nope: torch.Tensor, q_rope: torch.Tensor, nope_cache: torch.
             _lib.check(rc, "dsa_sparse_decode_heads_bf16")
         return out
     if num_splits is None:
-        num_splits = default_num_splits(t, 1, n, rows.shape[1])
+        num_splits = launch_splits(t, 1, n, rows.shape[1])
     per_token = lib.mla_decode_workspace_bytes(1, 1, n, num_splits)
     cap = workspace.numel() * workspace.element_size() if workspace is not None else SPARSE_WORKSPACE_CAP
     step = max(1, min(t, cap // max(per_token, 1), 32768))
@@ -950,7 +959,7 @@ def decode_fp8(q_nope: torch.Tensor, q_rope: torch.Tensor, cache: torch.Tensor, 
     if window is not None:
         max_seq_len = min(max_seq_len, sink_len + window + 32 + q_len)         # keys of a shortened sequence
     if num_splits is None:
-        num_splits = default_num_splits(b, q_len, n, max_seq_len)
+        num_splits = launch_splits(b, q_len, n, max_seq_len)
     need = lib.mla_decode_workspace_bytes(b, q_len, n, num_splits)
     ws = workspace if workspace is not None else _workspace(q_nope.device, need)
     if window is not None:
