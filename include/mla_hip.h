@@ -262,6 +262,12 @@ int mla_gather_paged_fp8_f16(const void* cache, int64_t page_stride_bytes, int64
 int mla_rows_f16(const void* kv_c, int64_t kv_c_stride, const void* k_pe, int64_t k_pe_stride, int64_t num_rows, void* out_c,
                  int64_t out_c_stride, void* out_pe, int64_t out_pe_stride, mlahip_stream_t stream);
 
+/* Query absorption of a decode step: out[t,n,:] = q_nope[t,n,:] . W_UK[n,:,:]  (q_nope [T,N,128], W_UK [N,128,512], out
+ * [T,N,512], all bf16, strides in elements; attention/backends/mla.py:900-905). */
+int mla_absorb_bf16(const void* q_nope, int64_t q_stride_t, int64_t q_stride_h, const void* w_uk, int64_t w_stride_n,
+                    int64_t w_stride_k, void* out, int64_t out_stride_t, int64_t out_stride_h, int32_t num_tokens,
+                    int32_t num_heads, mlahip_stream_t stream);
+
 int mla_merge_states(const void* prefix_out, int64_t po_stride_t, int64_t po_stride_h, const float* prefix_lse,
                      const void* suffix_out, int64_t so_stride_t, int64_t so_stride_h, const float* suffix_lse,
                      int32_t in_dtype, void* out, int64_t out_stride_t, int64_t out_stride_h, int32_t out_dtype,

@@ -318,7 +318,7 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
 
     def _absorb_prolog(self, q: torch.Tensor):
         q_nope, q_pe = q.split([self.qk_nope_head_dim, self.qk_rope_head_dim], dim=-1)
-        ql_nope = torch.bmm(q_nope.transpose(0, 1), self.W_UK_T).transpose(0, 1)
+        ql_nope = K.absorb(q_nope, self.W_UK_T)
         return ql_nope, q_pe
 
     def _fusable_w_uv(self, out: torch.Tensor) -> bool:

@@ -536,8 +536,7 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
         if has_decode and not self._native_decode(q, kv_cache, attn_metadata, output):
             assert attn_metadata.decode is not None
             decode_q_nope, decode_q_pe = q[:num_decode_tokens].split([self.qk_nope_head_dim, self.qk_rope_head_dim], dim=-1)
-            # (B, N, P) -> (N, B, P) x (N, P, L) -> (N, B, L) -> (B, N, L) view
-            decode_ql_nope = torch.bmm(decode_q_nope.transpose(0, 1), self.W_UK_T).transpose(0, 1)
+            decode_ql_nope = K.absorb(decode_q_nope, self.W_UK_T)
             ndt = decode_ql_nope.shape[0]
             if self._fusable_w_uv(output[:ndt]):
                 self._forward_decode(decode_ql_nope, decode_q_pe, kv_cache, attn_metadata, layer, proj_out=output[:ndt])

@@ -29,6 +29,7 @@ using at::Tensor;
 using OptTensor = std::optional<Tensor>;
 
 constexpr int64_t kNope = 512, kRope = 64, kPage = 128, kFp8Row = 656, kVDim = 128;
+constexpr int64_t kAbsorbMaxTokens = 256;   // kernels.ABSORB_MAX_TOKENS
 constexpr int64_t kVupMaxTokens = 256;      // kernels.VUP_MAX_TOKENS: beyond, a separate merge and the library GEMM
 
 void check(int rc, const char* what) {
@@ -52,7 +53,7 @@ Stream stream_of(const Tensor& t) { return (Stream)c10::hip::getCurrentHIPStream
 PyObject* g_workspace = nullptr;
 std::map<std::tuple<int, Stream, int>, Tensor> g_scratch;      // (guarded by the GIL, as the Python side is)
 Tensor& scratch(const Tensor& like, Stream stream, int64_t bytes, int tag) {
-  static const char* const names[] = {"decode", "topk"};
+  static const char* const names[] = {"decode", "topk", "absorb"};
   Tensor& t = g_scratch[{like.get_device(), stream, tag}];
   if (!t.defined() || t.numel() < bytes) t = py::cast<Tensor>(py::handle(g_workspace)(like.device(), bytes, names[tag]));
   return t;
@@ -123,9 +124,18 @@ bool layer_ok(const Tensor& q, const Tensor& w_uk, const Tensor& w_uv, const Ten
          w_uv.size(0) == n && w_uv.size(1) == kNope && w_uv.size(2) == kVDim && w_uv.stride(0) % 8 == 0 && w_uv.stride(1) % 8 == 0 &&
          is_bf16(out, 2, dev) && out.size(0) >= t && out.size(1) == n * kVDim && out.stride(0) % 4 == 0;
 }
-// Absorbed queries [N, T, 512] (library GEMM, as in the reference: mla.py:900-905).
-Tensor absorb(const Tensor& q, const Tensor& w_uk, int64_t t) {
-  return at::bmm(q.narrow(0, 0, t).narrow(2, 0, 128).transpose(0, 1), w_uk);
+// kernels.absorb: the absorbed queries, in scratch memory or (more tokens, or rows that are not 16-byte aligned) from the library
+struct Absorbed { Tensor keep; const void* ptr; int64_t st, sh; };
+Absorbed absorb(const Tensor& q, const Tensor& w_uk, int64_t t, Stream st) {
+  const int64_t n = q.size(1);
+  if (t <= kAbsorbMaxTokens && !((w_uk.stride(0) | w_uk.stride(1)) & 7) && !(((uintptr_t)q.data_ptr() | (uintptr_t)w_uk.data_ptr()) & 15)) {
+    Tensor& ws = scratch(q, st, t * n * kNope * 2, 2);
+    check(mla_absorb_bf16(q.data_ptr(), q.stride(0), q.stride(1), w_uk.data_ptr(), w_uk.stride(0), w_uk.stride(1), ws.data_ptr(),
+                          n * kNope, kNope, (int)t, (int)n, st), "mla_absorb_bf16");
+    return {Tensor(), ws.data_ptr(), n * kNope, kNope};
+  }
+  Tensor ql = at::bmm(q.narrow(0, 0, t).narrow(2, 0, 128).transpose(0, 1), w_uk);
+  return {ql, ql.data_ptr(), ql.stride(1), ql.stride(0)};
 }
 // Merge of the partials and the value up-projection into out (mla.py:309-315).
 void merge_vup(const Tensor& ws, const Tensor& lens, const OptTensor& qsl, int64_t batch, int64_t q_len, int64_t n, int splits,
@@ -163,7 +173,7 @@ bool mla_decode(const Tensor& q, const Tensor& nope, const OptTensor& rope, cons
   at::AutoDispatchBelowAutograd guard;
   Stream st = stream_of(q);
   const bool fp8 = !rope;
-  Tensor ql = absorb(q, w_uk, t);
+  const Absorbed ql = absorb(q, w_uk, t, st);
   int64_t max_seq_len = block_table.size(1) * kPage;
   if (step_max_len > 0 && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None)
     max_seq_len = std::min(max_seq_len, step_max_len + sink);
@@ -177,23 +187,22 @@ bool mla_decode(const Tensor& q, const Tensor& nope, const OptTensor& rope, cons
   const int32_t* lens = (const int32_t*)seq_lens.data_ptr();
   const int32_t* qs = qsl ? (const int32_t*)qsl->data_ptr() : nullptr;
   const char* qr = (const char*)q.data_ptr() + 2 * 128;
-  const int64_t ql_t = ql.stride(1), ql_h = ql.stride(0);
   if (window > 0) {
     if (fp8)
-      check(mla_decode_fp8_window_split(ql.data_ptr(), ql_t, ql_h, qr, q.stride(0), q.stride(1), c.nope->data_ptr(), c.n_sp, c.n_sr,
+      check(mla_decode_fp8_window_split(ql.ptr, ql.st, ql.sh, qr, q.stride(0), q.stride(1), c.nope->data_ptr(), c.n_sp, c.n_sr,
                                         c.pages, bt, bts, mb, lens, nullptr, qs, (int)b, (int)q_len, (int)n, (int)sink,
                                         (int)window, (float)scale, ws.data_ptr(), ws.numel(), splits, st), "mla_decode_fp8_window_split");
     else
-      check(mla_decode_bf16_window_split(ql.data_ptr(), ql_t, ql_h, qr, q.stride(0), q.stride(1), c.nope->data_ptr(), c.n_sp, c.n_sr,
+      check(mla_decode_bf16_window_split(ql.ptr, ql.st, ql.sh, qr, q.stride(0), q.stride(1), c.nope->data_ptr(), c.n_sp, c.n_sr,
                                          c.rope->data_ptr(), c.r_sp, c.r_sr, c.pages, bt, bts, mb, lens, nullptr, qs, (int)b,
                                          (int)q_len, (int)n, (int)sink, (int)window, (float)scale, ws.data_ptr(), ws.numel(),
                                          splits, st), "mla_decode_bf16_window_split");
   } else if (fp8) {
-    check(mla_decode_fp8(ql.data_ptr(), ql_t, ql_h, qr, q.stride(0), q.stride(1), c.nope->data_ptr(), c.n_sp, c.n_sr, c.pages, bt,
+    check(mla_decode_fp8(ql.ptr, ql.st, ql.sh, qr, q.stride(0), q.stride(1), c.nope->data_ptr(), c.n_sp, c.n_sr, c.pages, bt,
                          bts, mb, lens, qs, (int)b, (int)q_len, (int)n, (float)scale, nullptr, 0, 0, nullptr, ws.data_ptr(),
                          ws.numel(), splits, st), "mla_decode_fp8");
   } else {
-    check(mla_decode_bf16_split(ql.data_ptr(), ql_t, ql_h, qr, q.stride(0), q.stride(1), c.nope->data_ptr(), c.n_sp, c.n_sr,
+    check(mla_decode_bf16_split(ql.ptr, ql.st, ql.sh, qr, q.stride(0), q.stride(1), c.nope->data_ptr(), c.n_sp, c.n_sr,
                                 c.rope->data_ptr(), c.r_sp, c.r_sr, c.pages, bt, bts, mb, lens, qs, (int)b, (int)q_len, (int)n,
                                 (float)scale, ws.data_ptr(), ws.numel(), splits, st), "mla_decode_bf16_split");
   }
@@ -217,9 +226,9 @@ bool sparse_decode(const Tensor& q, const Tensor& nope, const Tensor& rope, cons
   if (need > (256 << 20)) return false;                        // kernels.SPARSE_WORKSPACE_CAP
   at::AutoDispatchBelowAutograd guard;
   Stream st = stream_of(q);
-  Tensor ql = absorb(q, w_uk, t);
+  const Absorbed ql = absorb(q, w_uk, t, st);
   Tensor& ws = scratch(q, st, need, 0);
-  check(dsa_sparse_decode_bf16(ql.data_ptr(), ql.stride(1), ql.stride(0), (const char*)q.data_ptr() + 2 * 128, q.stride(0), q.stride(1),
+  check(dsa_sparse_decode_bf16(ql.ptr, ql.st, ql.sh, (const char*)q.data_ptr() + 2 * 128, q.stride(0), q.stride(1),
                                c.nope->data_ptr(), c.n_sp, c.n_sr, c.rope->data_ptr(), c.r_sp, c.r_sr, c.pages, (int)c.page,
                                (const int32_t*)rows.data_ptr(), rows.stride(0), (const int32_t*)counts.data_ptr(), (int)t, (int)n,
                                (float)scale, nullptr, 0, 0, nullptr, ws.data_ptr(), ws.numel(), splits, st),

@@ -309,6 +309,26 @@ def rows_f16(kv_c: torch.Tensor, k_pe: torch.Tensor):
     return c, r
 
 
+# Tokens up to which the queries of a step are absorbed by this library's kernel; beyond, the work is a plain GEMM
+ABSORB_MAX_TOKENS = 256
+
+
+def absorb(q_nope: torch.Tensor, w_uk: torch.Tensor) -> torch.Tensor:
+    """q_nope [T,N,128] . W_UK_T [N,128,512] -> [T,N,512] (reference: the batched product of mla.py:900-905)."""
+    t, n, k = q_nope.shape
+    if not (q_nope.is_cuda and w_uk.is_cuda and q_nope.dtype == w_uk.dtype == torch.bfloat16 and k == 128 and
+            w_uk.shape == (n, 128, D_NOPE) and 1 <= t <= ABSORB_MAX_TOKENS and q_nope.stride(2) == 1 and w_uk.stride(2) == 1 and
+            not ((q_nope.stride(0) | q_nope.stride(1) | w_uk.stride(0) | w_uk.stride(1)) & 7) and
+            not ((q_nope.data_ptr() | w_uk.data_ptr()) & 15)) or \
+            torch.is_grad_enabled() and (q_nope.requires_grad or w_uk.requires_grad):
+        return torch.bmm(q_nope.transpose(0, 1), w_uk).transpose(0, 1)
+    out = torch.empty(t, n, D_NOPE, dtype=torch.bfloat16, device=q_nope.device)
+    rc = _lib.load().mla_absorb_bf16(q_nope.data_ptr(), q_nope.stride(0), q_nope.stride(1), w_uk.data_ptr(), w_uk.stride(0),
+                                     w_uk.stride(1), out.data_ptr(), out.stride(0), out.stride(1), t, n, _stream(q_nope))
+    _lib.check(rc, "mla_absorb_bf16")
+    return out
+
+
 _DT = {torch.bfloat16: 0, torch.float32: 1}
 
 

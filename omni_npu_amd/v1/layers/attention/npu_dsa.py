@@ -80,7 +80,7 @@ class NPUDeepseekSparseAttention(torch.nn.Module):
         else:
             d = meta.decode
             part, lens, q_len, qsl = d, d.seq_lens, d.q_len, d.query_start_loc
-        ql_nope = torch.bmm(q[..., :self.qk_nope_head_dim].transpose(0, 1), impl.W_UK_T).transpose(0, 1)
+        ql_nope = K.absorb(q[..., :self.qk_nope_head_dim], impl.W_UK_T)
         fused = out if impl._fusable_w_uv(out) else None
         rc = select.rows_for(meta) if pick is None and hasattr(select, "rows_for") else None
         attn_out = impl._apply_sparse_attention(ql_nope, q_pe, kv_cache, part, lens, q_len, qsl, topk_indices[:t],

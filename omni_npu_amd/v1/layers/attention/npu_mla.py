@@ -75,8 +75,7 @@ class NPUDeepseekMLAAttention(torch.nn.Module):
         q = self._q(hidden_states)
         kv = self.kv_a_proj_with_mqa(hidden_states)[0]
         t = q.shape[0]
-        # (N, T, P) @ W_UK_T (N, P, L) -> token-major [T, N, L]
-        ql_nope = torch.bmm(q[..., :self.qk_nope_head_dim].transpose(0, 1), impl.W_UK_T).transpose(0, 1)
+        ql_nope = K.absorb(q[..., :self.qk_nope_head_dim], impl.W_UK_T)
         q_pe = q[..., self.qk_nope_head_dim:]                   # rotated in place by the launch that writes the cache
         K.kv_rmsnorm_rope_cache(kv, self.kv_a_layernorm.weight, cos, sin, meta.slot_mapping, nope_c, rope_c, eps=self._eps(),
                                 q_rope=q_pe)
