@@ -267,6 +267,14 @@ int mla_rows_f16(const void* kv_c, int64_t kv_c_stride, const void* k_pe, int64_
 int mla_absorb_bf16(const void* q_nope, int64_t q_stride_t, int64_t q_stride_h, const void* w_uk, int64_t w_stride_n,
                     int64_t w_stride_k, void* out, int64_t out_stride_t, int64_t out_stride_h, int32_t num_tokens,
                     int32_t num_heads, mlahip_stream_t stream);
+/* mla_absorb_bf16 and mla_cache_write_bf16 (rope_cache = NULL: mla_cache_write_fp8 into nope_cache, whose strides are then in
+ * bytes) of num_new rows in one launch; neither reads what the other writes (attention/backends/mla.py:868-881, 900-905). */
+int mla_absorb_write(const void* q_nope, int64_t q_stride_t, int64_t q_stride_h, const void* w_uk, int64_t w_stride_n,
+                     int64_t w_stride_k, void* out, int64_t out_stride_t, int64_t out_stride_h, int32_t num_tokens,
+                     int32_t num_heads, const void* kv_c, int64_t kv_c_stride, const void* k_pe, int64_t k_pe_stride,
+                     const int64_t* slot_mapping, int32_t num_new, void* nope_cache, int64_t nope_page_stride,
+                     int64_t nope_row_stride, void* rope_cache, int64_t rope_page_stride, int64_t rope_row_stride,
+                     int32_t page_size, int64_t num_pages, mlahip_stream_t stream);
 
 int mla_merge_states(const void* prefix_out, int64_t po_stride_t, int64_t po_stride_h, const float* prefix_lse,
                      const void* suffix_out, int64_t so_stride_t, int64_t so_stride_h, const float* suffix_lse,

@@ -38,6 +38,8 @@ SIGNATURES = {
     "mla_gather_paged_fp8": (c_int32, [P, I64, I64, I64, I32, P, I64, I64, P, I64, I32, P, P, I32, I64, P]),
     "mla_gather_paged_fp8_f16": (c_int32, [P, I64, I64, I64, I32, P, I64, I64, P, I64, I32, P, P, I32, I64, P]),
     "mla_absorb_bf16": (c_int32, [P, I64, I64, P, I64, I64, P, I64, I64, I32, I32, P]),
+    "mla_absorb_write": (c_int32, [P, I64, I64, P, I64, I64, P, I64, I64, I32, I32, P, I64, P, I64, P, I32, P, I64, I64, P, I64,
+                                   I64, I32, I64, P]),
     "mla_rows_f16": (c_int32, [P, I64, P, I64, I64, P, I64, P, I64, P]),
     "mla_merge_states": (c_int32, [P, I64, I64, P, P, I64, I64, P, I32, P, I64, I64, I32, P, I32, I32, I32, P]),
     "mla_merge_n_states": (c_int32, [P, I64, I64, I32, P, I64, P, I64, P, I32, I32, I32, P]),

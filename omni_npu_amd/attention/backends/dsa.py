@@ -404,12 +404,16 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
         has_prefill = attn_metadata.num_prefills > 0
         ndt = attn_metadata.num_decode_tokens
         written = _caller_wrote_cache(self, attn_metadata, num_actual_toks)
-        if not written:                                            # (else the caller's fused norm + rope launch wrote them)
-            K.cache_write(k_c_normed, k_pe, attn_metadata.slot_mapping, k_nope, k_rope)
         rows_for = getattr(self.indexer, "rows_for", None)
         rc = rows_for(attn_metadata) if rows_for is not None else None
-        if has_decode and not has_prefill and rc is not None and _host.load().sparse_decode(
-                q, k_nope, k_rope, rc[0], rc[1], self.W_UK_T, self.W_UV, self.scale, ndt, output):
+        native = None
+        if has_decode and not has_prefill and rc is not None:
+            native = lambda *new: _host.load().sparse_decode(q, k_nope, k_rope, rc[0], rc[1], self.W_UK_T, self.W_UV, self.scale,
+                                                             ndt, output, *new)
+        if written:                                                # (the caller's fused norm + rope launch wrote the rows)
+            if native is not None and native(None, None, None):
+                return output_padded
+        elif K.cache_write(k_c_normed, k_pe, attn_metadata.slot_mapping, k_nope, k_rope, along=native):
             return output_padded
         topk = self.indexer.topk_indices_buffer
         part = lambda a, b: None if rc is None else (rc[0][a:b], rc[1][a:b])

@@ -473,16 +473,17 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
             K.decode(ql_nope, q_pe, kv_cache[0], kv_cache[1], d.block_table, d.seq_lens, self.scale, out, **kw)
         return o
 
-    def _native_decode(self, q, kv_cache, attn_metadata, output) -> bool:
-        """The decode tokens' absorption, attention and merge + up-projection into ``output`` in one native call.  False, with
-        nothing done, where that call does not know the case."""
+    def _native_decode(self, q, kv_cache, attn_metadata, output, new=(None, None, None)) -> bool:
+        """The decode tokens' absorption, attention and merge + up-projection into ``output`` in one native call, the cache
+        write of ``new`` = (latents, rope rows, slots) in front of them where it is still to be done.  False, with nothing
+        done, where that call does not know the case."""
         d = attn_metadata.decode
         if self.sink_len > 0 and (self.sliding_window is None or self.sink_len % K.PAGE != 0):
             return False
         return _host.load().mla_decode(
             q, kv_cache[0], None if self.fp8_cache else kv_cache[1], d.block_table, d.seq_lens, d.query_start_loc, d.q_len,
             d.max_seq_len, self.W_UK_T, self.W_UV, self.scale, attn_metadata.num_decode_tokens, self.sink_len,
-            self.sliding_window if self.sink_len > 0 else 0, output)
+            self.sliding_window if self.sink_len > 0 else 0, output, *new)
 
     def forward(self, layer, q: torch.Tensor, k_c_normed: torch.Tensor, k_pe: torch.Tensor,
                 kv_cache: Tuple[torch.Tensor, ...], attn_metadata: NPUMLAMetadata,
@@ -512,15 +513,19 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
         has_prefill = attn_metadata.num_prefills > 0
         num_decode_tokens = attn_metadata.num_decode_tokens
 
-        # write the latent and rope rows of the new tokens (one launch), unless the caller's fused norm + rope launch has
+        # write the latent and rope rows of the new tokens, unless the caller's fused norm + rope launch has
         # put them there already and said so for this very metadata object
         written = _caller_wrote_cache(self, attn_metadata, num_actual_toks)
-        if written:
-            pass
-        elif self.fp8_cache:
-            K.cache_write_fp8(k_c_normed, k_pe, attn_metadata.slot_mapping, kv_cache[0])
-        else:
-            K.cache_write(k_c_normed, k_pe, attn_metadata.slot_mapping, kv_cache[0], kv_cache[1])
+        if not written:
+            # a pure decode step's rows ride in its first launch
+            along = None if has_prefill or not has_decode else (
+                lambda *new: self._native_decode(q, kv_cache, attn_metadata, output, new))
+            if self.fp8_cache:
+                done = K.cache_write_fp8(k_c_normed, k_pe, attn_metadata.slot_mapping, kv_cache[0], along=along)
+            else:
+                done = K.cache_write(k_c_normed, k_pe, attn_metadata.slot_mapping, kv_cache[0], kv_cache[1], along=along)
+            if done:
+                return output_padded
 
         if has_prefill:
             output = output[:num_actual_toks, ...]

@@ -5,10 +5,16 @@
 // launch and round trips.  One workgroup = one head and 128 of its 512 columns (512 workgroups for 128 heads: two per CU, each
 // with its whole 32 KiB of weights in flight at once); the rows of up to 64 tokens are asked for beside the weights, so the two
 // round trips are one.  us in a queue of launches, library product -> this kernel: 1 token x 16 heads 4.4 -> 3.0, 7 x 128 5.6 ->
-// 3.6, 64 x 128 7.7 -> 5.8 (3.5 TB/s), 128 x 128 10.4 -> 10.0; and 16 -> 4 us of host time per call.  Each of the four wavefronts multiplies its 32 columns: W^T, read with transposed LDS reads, is the first
-// MFMA operand, the rows are the second, and a lane ends up with four consecutive columns of a token at a time; they go through
-// LDS once more, so that a token's 256 bytes leave in one piece.
-#include "mla_common.hpp"
+// 3.6, 64 x 128 7.7 -> 5.8 (3.5 TB/s), 128 x 128 10.4 -> 10.0; and 16 -> 4 us of host time per call.  Each of the four wavefronts multiplies its 32
+// columns: W^T, read with transposed LDS reads, is the first MFMA operand, the rows are the second, and a lane ends up with four
+// consecutive columns of a token at a time; they go through LDS once more, so that a token's 256 bytes leave in one piece.
+//
+// The step's cache rows can ride along (mla_absorb_write): writing them and absorbing the queries touch nothing in common, both
+// stand in front of the attention, and either is mostly launch and round trips, so the workgroups behind the absorbing ones
+// (one more layer of the grid's z) write the rows, a wavefront per token.
+// us per decode layer whose rows were written by a launch of their own before: one user of 1k keys, 16 heads 22.15 -> 20.50;
+// 48 x 2 tokens, 16 heads, replayed 85.7 -> 82.5; one of 128k keys 73.3 -> 72.1; 64 with sink and window 113.3 -> 112.5.
+#include "cache_rows.hpp"
 
 namespace mlahip {
 namespace {
@@ -21,19 +27,40 @@ constexpr int kAbsQB = kAbsTok * kAbsK * 2;     // 16384: query row t at t * 256
 constexpr int kAbsOB = kAbsTok * kAbsCols * 2;  // 16384: result row t at t * 256
 constexpr int kAbsLdsB = kAbsWB + kAbsQB + kAbsOB;
 
+enum class NewRows { kNone, kBf16, kFp8 };
+
 struct AbsorbParams {
   const __bf16* q; int64_t q_st, q_sh;
   const __bf16* w; int64_t w_sn, w_sk;
   __bf16* out; int64_t o_st, o_sh;
   int32_t num_tokens, tokens_wg;       // tokens in all, and of a workgroup (whole passes)
+  // the rows of the step's new tokens: bf16 latent and rope rows, or fp8 rows
+  ScatterSrc lat, pe;
+  Fp8RowSrc f8;
+  const int64_t* slots; int64_t num_pages;
+  int32_t num_new, page_size;
 };
 
 }  // namespace
 
+template <NewRows kNew>
 __global__ __launch_bounds__(256) void mla_absorb_kernel(const AbsorbParams p) {
   __shared__ __attribute__((aligned(1024))) char lds[kAbsLdsB];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if constexpr (kNew != NewRows::kNone) {
+    if (blockIdx.z == gridDim.z - 1) {
+      for (int64_t t = (blockIdx.x + gridDim.x * blockIdx.y) * 4 + wave; t < p.num_new; t += gridDim.x * gridDim.y * 4) {
+        if constexpr (kNew == NewRows::kFp8) {
+          quant_row_fp8(p.f8, p.slots, t, lane, p.page_size, p.num_pages);
+        } else {
+          scatter_row(p.lat, p.slots, t, lane, p.page_size, p.num_pages);
+          scatter_row(p.pe, p.slots, t, lane, p.page_size, p.num_pages);
+        }
+      }
+      return;
+    }
+  }
   const int head = blockIdx.y, c0 = blockIdx.x * kAbsCols;
   const uint32_t lds0 = lds_addr_of(lds);
   const int r4 = lane >> 4, pos = lane & 15;     // a copy instruction brings four rows of 256 bytes
@@ -102,17 +129,16 @@ __global__ __launch_bounds__(256) void mla_absorb_kernel(const AbsorbParams p) {
 }  // namespace mlahip
 using namespace mlahip;
 
-extern "C" int mla_absorb_bf16(const void* q_nope, int64_t q_stride_t, int64_t q_stride_h, const void* w_uk, int64_t w_stride_n,
-                               int64_t w_stride_k, void* out, int64_t out_stride_t, int64_t out_stride_h, int32_t num_tokens,
-                               int32_t num_heads, hipStream_t stream) {
-  MLA_REQUIRE(q_nope && w_uk && out, MLA_ERR_NULL, "mla_absorb_bf16: null pointer argument");
-  MLA_REQUIRE(num_tokens >= 0 && num_heads >= 1 && num_heads <= 65535, MLA_ERR_SHAPE, "mla_absorb_bf16: num_tokens=%d num_heads=%d",
+static int absorb_impl(const char* what, const void* q_nope, int64_t q_stride_t, int64_t q_stride_h, const void* w_uk,
+                       int64_t w_stride_n, int64_t w_stride_k, void* out, int64_t out_stride_t, int64_t out_stride_h,
+                       int32_t num_tokens, int32_t num_heads, NewRows kind, AbsorbParams p, hipStream_t stream) {
+  MLA_REQUIRE(q_nope && w_uk && out, MLA_ERR_NULL, "%s: null pointer argument", what);
+  MLA_REQUIRE(num_tokens >= 0 && num_heads >= 1 && num_heads <= 65535, MLA_ERR_SHAPE, "%s: num_tokens=%d num_heads=%d", what,
               num_tokens, num_heads);
   MLA_REQUIRE(q_stride_t % 8 == 0 && q_stride_h % 8 == 0 && w_stride_n % 8 == 0 && w_stride_k % 8 == 0 && out_stride_t % 8 == 0 &&
                   out_stride_h % 8 == 0 && (uintptr_t)q_nope % 16 == 0 && (uintptr_t)w_uk % 16 == 0 && (uintptr_t)out % 16 == 0,
-              MLA_ERR_SHAPE, "mla_absorb_bf16: rows must be 16-byte aligned");
-  if (num_tokens == 0) return MLA_OK;
-  AbsorbParams p;
+              MLA_ERR_SHAPE, "%s: rows must be 16-byte aligned", what);
+  if (num_tokens == 0 && kind == NewRows::kNone) return MLA_OK;
   p.q = (const __bf16*)q_nope; p.q_st = q_stride_t; p.q_sh = q_stride_h;
   p.w = (const __bf16*)w_uk; p.w_sn = w_stride_n; p.w_sk = w_stride_k;
   p.out = (__bf16*)out; p.o_st = out_stride_t; p.o_sh = out_stride_h;
@@ -122,8 +148,45 @@ extern "C" int mla_absorb_bf16(const void* q_nope, int64_t q_stride_t, int64_t q
   const int passes = (num_tokens + kAbsTok - 1) / kAbsTok, heads_wgs = kDNope / kAbsCols * num_heads;
   int groups = 512 / heads_wgs;
   groups = groups < 1 ? 1 : (groups < passes ? groups : passes);
-  const int passes_wg = (passes + groups - 1) / groups;
+  const int passes_wg = num_tokens ? (passes + groups - 1) / groups : 1;
   p.tokens_wg = passes_wg * kAbsTok;
-  hipLaunchKernelGGL(mla_absorb_kernel, dim3(kDNope / kAbsCols, num_heads, (passes + passes_wg - 1) / passes_wg), dim3(256), 0, stream, p);
+  const int layers = (passes + passes_wg - 1) / passes_wg + (kind == NewRows::kNone ? 0 : 1);
+  auto* kern = kind == NewRows::kNone ? mla_absorb_kernel<NewRows::kNone>
+               : kind == NewRows::kBf16 ? mla_absorb_kernel<NewRows::kBf16> : mla_absorb_kernel<NewRows::kFp8>;
+  hipLaunchKernelGGL(kern, dim3(kDNope / kAbsCols, num_heads, layers), dim3(256), 0, stream, p);
   return check_launch("mla_absorb_kernel");
+}
+
+extern "C" int mla_absorb_bf16(const void* q_nope, int64_t q_stride_t, int64_t q_stride_h, const void* w_uk, int64_t w_stride_n,
+                               int64_t w_stride_k, void* out, int64_t out_stride_t, int64_t out_stride_h, int32_t num_tokens,
+                               int32_t num_heads, hipStream_t stream) {
+  return absorb_impl("mla_absorb_bf16", q_nope, q_stride_t, q_stride_h, w_uk, w_stride_n, w_stride_k, out, out_stride_t,
+                     out_stride_h, num_tokens, num_heads, NewRows::kNone, AbsorbParams{}, stream);
+}
+
+// mla_absorb_bf16 and the cache write of the step's new rows in one launch (rope_cache = NULL: the fp8 cache of 656-byte rows).
+extern "C" int mla_absorb_write(const void* q_nope, int64_t q_stride_t, int64_t q_stride_h, const void* w_uk, int64_t w_stride_n,
+                                int64_t w_stride_k, void* out, int64_t out_stride_t, int64_t out_stride_h, int32_t num_tokens,
+                                int32_t num_heads, const void* kv_c, int64_t kv_c_stride, const void* k_pe, int64_t k_pe_stride,
+                                const int64_t* slot_mapping, int32_t num_new, void* nope_cache, int64_t nope_page_stride,
+                                int64_t nope_row_stride, void* rope_cache, int64_t rope_page_stride, int64_t rope_row_stride,
+                                int32_t page_size, int64_t num_pages, hipStream_t stream) {
+  MLA_REQUIRE(kv_c && k_pe && slot_mapping && nope_cache, MLA_ERR_NULL, "mla_absorb_write: null pointer argument");
+  MLA_REQUIRE(num_new >= 1 && page_size >= 1 && num_pages >= 1, MLA_ERR_SHAPE,
+              "mla_absorb_write: num_new=%d page_size=%d num_pages=%lld", num_new, page_size, (long long)num_pages);
+  const int unit = rope_cache ? 8 : 16;                    // cache strides count bf16 elements, or bytes of the fp8 cache
+  MLA_REQUIRE(kv_c_stride % 8 == 0 && k_pe_stride % 8 == 0 && nope_row_stride % unit == 0 && nope_page_stride % unit == 0 &&
+                  rope_row_stride % 8 == 0 && rope_page_stride % 8 == 0 && (uintptr_t)kv_c % 16 == 0 && (uintptr_t)k_pe % 16 == 0 &&
+                  (uintptr_t)nope_cache % 16 == 0 && (uintptr_t)rope_cache % 16 == 0 && (rope_cache || nope_row_stride >= kFp8RowB),
+              MLA_ERR_SHAPE, "mla_absorb_write: cache rows must be 16-byte aligned");
+  AbsorbParams p{};
+  p.slots = slot_mapping; p.num_new = num_new; p.page_size = page_size; p.num_pages = num_pages;
+  if (rope_cache) {
+    p.lat = ScatterSrc{(const char*)kv_c, kv_c_stride * 2, (char*)nope_cache, nope_page_stride * 2, nope_row_stride * 2, kDNope * 2};
+    p.pe = ScatterSrc{(const char*)k_pe, k_pe_stride * 2, (char*)rope_cache, rope_page_stride * 2, rope_row_stride * 2, kDRope * 2};
+  } else {
+    p.f8 = Fp8RowSrc{(const __bf16*)kv_c, kv_c_stride, (const __bf16*)k_pe, k_pe_stride, (char*)nope_cache, nope_page_stride, nope_row_stride};
+  }
+  return absorb_impl("mla_absorb_write", q_nope, q_stride_t, q_stride_h, w_uk, w_stride_n, w_stride_k, out, out_stride_t,
+                     out_stride_h, num_tokens, num_heads, rope_cache ? NewRows::kBf16 : NewRows::kFp8, p, stream);
 }

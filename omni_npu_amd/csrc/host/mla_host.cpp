@@ -93,26 +93,35 @@ bool cache_of(const Tensor& nope, const OptTensor& rope, const at::Device& dev, 
   return true;
 }
 
-// kernels.cache_write / cache_write_fp8: the step's latent and rope rows to their slots.
+// The latent and rope rows of a step's new tokens and the slots they go to: what kernels.cache_write / cache_write_fp8 take.
+struct NewRows { const Tensor *kv_c, *k_pe, *slots; int64_t t; };
+bool rows_of(const Tensor& kv_c, const Tensor& k_pe, const Tensor& slots, const at::Device& dev, NewRows& r) {
+  if (!is_bf16(kv_c, 2, dev) || kv_c.size(1) != kNope || k_pe.scalar_type() != at::kBFloat16 || k_pe.device() != dev ||
+      k_pe.size(-1) != kRope || k_pe.stride(-1) != 1 || !(k_pe.dim() == 2 || (k_pe.dim() == 3 && k_pe.size(1) == 1)) ||
+      slots.scalar_type() != at::kLong || slots.dim() != 1 || !slots.is_contiguous() || slots.device() != dev)
+    return false;
+  r = {&kv_c, &k_pe, &slots, std::min(slots.numel(), kv_c.size(0))};
+  return r.t >= 1 && k_pe.size(0) >= r.t;
+}
+void write_rows(const NewRows& r, const Cache& c, Stream st) {
+  const Tensor &kv_c = *r.kv_c, &k_pe = *r.k_pe;
+  const int64_t* slots = (const int64_t*)r.slots->data_ptr();
+  if (c.rope)
+    check(mla_cache_write_bf16(kv_c.data_ptr(), kv_c.stride(0), k_pe.data_ptr(), k_pe.stride(0), slots, (int)r.t,
+                               c.nope->data_ptr(), c.n_sp, c.n_sr, c.rope->data_ptr(), c.r_sp, c.r_sr, (int)c.page,
+                               c.pages, st), "mla_cache_write_bf16");
+  else
+    check(mla_cache_write_fp8(kv_c.data_ptr(), kv_c.stride(0), k_pe.data_ptr(), k_pe.stride(0), slots, (int)r.t,
+                              c.nope->data_ptr(), c.n_sp, c.n_sr, (int)c.page, c.pages, st), "mla_cache_write_fp8");
+}
+// kernels.cache_write / cache_write_fp8
 bool cache_write(const Tensor& kv_c, const Tensor& k_pe, const Tensor& slots, const Tensor& nope, const OptTensor& rope) {
   if (!current_gpu(kv_c)) return false;
   const at::Device dev = kv_c.device();
   Cache c;
-  if (!is_bf16(kv_c, 2, dev) || kv_c.size(1) != kNope || k_pe.scalar_type() != at::kBFloat16 || k_pe.device() != dev ||
-      k_pe.size(-1) != kRope || k_pe.stride(-1) != 1 || !(k_pe.dim() == 2 || (k_pe.dim() == 3 && k_pe.size(1) == 1)) ||
-      slots.scalar_type() != at::kLong || slots.dim() != 1 || !slots.is_contiguous() || slots.device() != dev ||
-      !cache_of(nope, rope, dev, c))
-    return false;
-  const int64_t t = std::min(slots.numel(), kv_c.size(0));
-  if (t < 1 || k_pe.size(0) < t) return false;
-  Stream st = stream_of(kv_c);
-  if (c.rope)
-    check(mla_cache_write_bf16(kv_c.data_ptr(), kv_c.stride(0), k_pe.data_ptr(), k_pe.stride(0), (const int64_t*)slots.data_ptr(),
-                               (int)t, c.nope->data_ptr(), c.n_sp, c.n_sr, c.rope->data_ptr(), c.r_sp, c.r_sr, (int)c.page,
-                               c.pages, st), "mla_cache_write_bf16");
-  else
-    check(mla_cache_write_fp8(kv_c.data_ptr(), kv_c.stride(0), k_pe.data_ptr(), k_pe.stride(0), (const int64_t*)slots.data_ptr(),
-                              (int)t, c.nope->data_ptr(), c.n_sp, c.n_sr, (int)c.page, c.pages, st), "mla_cache_write_fp8");
+  NewRows r;
+  if (!rows_of(kv_c, k_pe, slots, dev, r) || !cache_of(nope, rope, dev, c)) return false;
+  write_rows(r, c, stream_of(kv_c));
   return true;
 }
 
@@ -124,11 +133,27 @@ bool layer_ok(const Tensor& q, const Tensor& w_uk, const Tensor& w_uv, const Ten
          w_uv.size(0) == n && w_uv.size(1) == kNope && w_uv.size(2) == kVDim && w_uv.stride(0) % 8 == 0 && w_uv.stride(1) % 8 == 0 &&
          is_bf16(out, 2, dev) && out.size(0) >= t && out.size(1) == n * kVDim && out.stride(0) % 4 == 0;
 }
-// kernels.absorb: the absorbed queries, in scratch memory or (more tokens, or rows that are not 16-byte aligned) from the library
+// kernels.absorb: the absorbed queries, in scratch memory or (more tokens, or rows that are not 16-byte aligned) from the
+// library.  Rows of new tokens (or null) go to the cache in the same launch, or in front of the library's.
 struct Absorbed { Tensor keep; const void* ptr; int64_t st, sh; };
-Absorbed absorb(const Tensor& q, const Tensor& w_uk, int64_t t, Stream st) {
+Absorbed absorb(const Tensor& q, const Tensor& w_uk, int64_t t, const NewRows* rows, const Cache& c, Stream st) {
   const int64_t n = q.size(1);
-  if (t <= kAbsorbMaxTokens && !((w_uk.stride(0) | w_uk.stride(1)) & 7) && !(((uintptr_t)q.data_ptr() | (uintptr_t)w_uk.data_ptr()) & 15)) {
+  const bool own = t <= kAbsorbMaxTokens && !((w_uk.stride(0) | w_uk.stride(1)) & 7) && !(((uintptr_t)q.data_ptr() | (uintptr_t)w_uk.data_ptr()) & 15);
+  if (own && rows) {
+    const Tensor &kv_c = *rows->kv_c, &k_pe = *rows->k_pe;
+    const int64_t unit = c.rope ? 8 : 16, cache_strides = c.n_sp | c.n_sr | (c.rope ? c.r_sp | c.r_sr : 0);
+    const uintptr_t ptrs = (uintptr_t)kv_c.data_ptr() | (uintptr_t)k_pe.data_ptr() | (uintptr_t)c.nope->data_ptr() | (c.rope ? (uintptr_t)c.rope->data_ptr() : 0);
+    if (!((kv_c.stride(0) | k_pe.stride(0)) & 7) && !(cache_strides & (unit - 1)) && !(ptrs & 15) && (c.rope || c.n_sr >= kFp8Row)) {
+      Tensor& ws = scratch(q, st, t * n * kNope * 2, 2);
+      check(mla_absorb_write(q.data_ptr(), q.stride(0), q.stride(1), w_uk.data_ptr(), w_uk.stride(0), w_uk.stride(1), ws.data_ptr(),
+                             n * kNope, kNope, (int)t, (int)n, kv_c.data_ptr(), kv_c.stride(0), k_pe.data_ptr(), k_pe.stride(0),
+                             (const int64_t*)rows->slots->data_ptr(), (int)rows->t, c.nope->data_ptr(), c.n_sp, c.n_sr,
+                             c.rope ? c.rope->data_ptr() : nullptr, c.r_sp, c.r_sr, (int)c.page, c.pages, st), "mla_absorb_write");
+      return {Tensor(), ws.data_ptr(), n * kNope, kNope};
+    }
+  }
+  if (rows) write_rows(*rows, c, st);
+  if (own) {
     Tensor& ws = scratch(q, st, t * n * kNope * 2, 2);
     check(mla_absorb_bf16(q.data_ptr(), q.stride(0), q.stride(1), w_uk.data_ptr(), w_uk.stride(0), w_uk.stride(1), ws.data_ptr(),
                           n * kNope, kNope, (int)t, (int)n, st), "mla_absorb_bf16");
@@ -154,13 +179,13 @@ void merge_vup(const Tensor& ws, const Tensor& lens, const OptTensor& qsl, int64
   at::bmm_out(dst, o, w_uv);
 }
 
-// One layer's decode tokens, their rows in the cache already: absorption, split-KV attention, merge + up-projection.  rope =
-// None: the fp8 cache.  window > 0: static sink + sliding window.  The launch is shaped for the step's own longest context
+// One layer's decode tokens: absorption, split-KV attention, merge + up-projection.  kv_c, k_pe, slots: the step's new rows, which
+// go to the cache first (None: they are there already).  rope = None: the fp8 cache.  window > 0: static sink + sliding window.  The launch is shaped for the step's own longest context
 // (step_max_len, 0 = unknown), and under capture for the longest the block table can hold, as a graph is replayed over others;
 // either way it is right for any length.
 bool mla_decode(const Tensor& q, const Tensor& nope, const OptTensor& rope, const Tensor& block_table, const Tensor& seq_lens, const OptTensor& qsl, int64_t q_len,
                 int64_t step_max_len, const Tensor& w_uk, const Tensor& w_uv, double scale, int64_t t, int64_t sink, int64_t window,
-                const Tensor& out) {
+                const Tensor& out, const OptTensor& kv_c, const OptTensor& k_pe, const OptTensor& slots) {
   if (!current_gpu(q)) return false;
   const at::Device dev = q.device();
   Cache c;
@@ -170,10 +195,13 @@ bool mla_decode(const Tensor& q, const Tensor& nope, const OptTensor& rope, cons
     return false;
   const int64_t b = seq_lens.numel(), n = q.size(1);
   if (qsl ? !(is_i32(*qsl, 1, dev) && qsl->is_contiguous() && qsl->numel() == b + 1) : t != b * q_len) return false;
+  NewRows rows;
+  const bool write = kv_c.has_value();
+  if (write && !(k_pe && slots && rows_of(*kv_c, *k_pe, *slots, dev, rows))) return false;
   at::AutoDispatchBelowAutograd guard;
   Stream st = stream_of(q);
   const bool fp8 = !rope;
-  const Absorbed ql = absorb(q, w_uk, t, st);
+  const Absorbed ql = absorb(q, w_uk, t, write ? &rows : nullptr, c, st);
   int64_t max_seq_len = block_table.size(1) * kPage;
   if (step_max_len > 0 && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None)
     max_seq_len = std::min(max_seq_len, step_max_len + sink);
@@ -210,10 +238,10 @@ bool mla_decode(const Tensor& q, const Tensor& nope, const OptTensor& rope, cons
   return true;
 }
 
-// One layer's sparse decode tokens over the cache rows of their picks.  (Few enough tokens for one launch; a prefill's
+// One layer's sparse decode tokens over the cache rows of their picks, the step's new rows first as in mla_decode.  (Few enough tokens for one launch; a prefill's
 // thousands take the general path.)
 bool sparse_decode(const Tensor& q, const Tensor& nope, const Tensor& rope, const Tensor& rows, const Tensor& counts, const Tensor& w_uk, const Tensor& w_uv,
-                   double scale, int64_t t, const Tensor& out) {
+                   double scale, int64_t t, const Tensor& out, const OptTensor& kv_c, const OptTensor& k_pe, const OptTensor& slots) {
   if (!current_gpu(q) || t > kVupMaxTokens) return false;
   const at::Device dev = q.device();
   Cache c;
@@ -224,9 +252,12 @@ bool sparse_decode(const Tensor& q, const Tensor& nope, const Tensor& rope, cons
   const int splits = launch_splits(t, 1, n, rows.size(1));
   const int64_t need = (int64_t)mla_decode_workspace_bytes((int)t, 1, (int)n, splits);
   if (need > (256 << 20)) return false;                        // kernels.SPARSE_WORKSPACE_CAP
+  NewRows new_rows;
+  const bool write = kv_c.has_value();
+  if (write && !(k_pe && slots && rows_of(*kv_c, *k_pe, *slots, dev, new_rows))) return false;
   at::AutoDispatchBelowAutograd guard;
   Stream st = stream_of(q);
-  const Absorbed ql = absorb(q, w_uk, t, st);
+  const Absorbed ql = absorb(q, w_uk, t, write ? &new_rows : nullptr, c, st);
   Tensor& ws = scratch(q, st, need, 0);
   check(dsa_sparse_decode_bf16(ql.ptr, ql.st, ql.sh, (const char*)q.data_ptr() + 2 * 128, q.stride(0), q.stride(1),
                                c.nope->data_ptr(), c.n_sp, c.n_sr, c.rope->data_ptr(), c.r_sp, c.r_sr, c.pages, (int)c.page,

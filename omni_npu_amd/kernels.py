@@ -36,9 +36,12 @@ def _cache3(c: torch.Tensor, width: int) -> torch.Tensor:
 
 # ------------------------------------------------------------------------------------------------
 def cache_write(kv_c: torch.Tensor, k_pe: torch.Tensor, slot_mapping: torch.Tensor,
-                nope_cache: torch.Tensor, rope_cache: torch.Tensor) -> None:
+                nope_cache: torch.Tensor, rope_cache: torch.Tensor, along=None) -> Optional[bool]:
     """nope.flatten(0,1)[slot[t]] = kv_c[t]; rope.flatten(0,1)[slot[t]] = k_pe[t]; negative slots skipped
-    (reference: store_kv, src/omni_npu/attention/backends/mla.py:868-881)."""
+    (reference: store_kv, src/omni_npu/attention/backends/mla.py:868-881).  ``along(kv_c, k_pe, slot_mapping)`` is asked first
+    whether it takes the rows along in launches of its own; True if it did."""
+    if along is not None and along(kv_c, k_pe, slot_mapping):
+        return True
     if _host.load().cache_write(kv_c, k_pe, slot_mapping, nope_cache, rope_cache):
         return
     _need_cuda(kv_c, k_pe, slot_mapping, nope_cache, rope_cache)
@@ -84,9 +87,12 @@ def scatter_rows(src: torch.Tensor, slot_mapping: torch.Tensor, cache: torch.Ten
 FP8_ROW_BYTES = 656      # 512 e4m3 + 4 fp32 block scales + 64 bf16 rope
 
 
-def cache_write_fp8(kv_c: torch.Tensor, k_pe: torch.Tensor, slot_mapping: torch.Tensor, cache: torch.Tensor) -> None:
+def cache_write_fp8(kv_c: torch.Tensor, k_pe: torch.Tensor, slot_mapping: torch.Tensor, cache: torch.Tensor,
+                    along=None) -> Optional[bool]:
     """Quantise the new tokens' latent to e4m3 with one fp32 scale per 128 elements and write 656-byte rows
-    (512 fp8 | 4 fp32 scales | 64 bf16 rope) into ``cache`` = uint8 [num_blocks, page, 656]."""
+    (512 fp8 | 4 fp32 scales | 64 bf16 rope) into ``cache`` = uint8 [num_blocks, page, 656].  ``along``: see cache_write."""
+    if along is not None and along(kv_c, k_pe, slot_mapping):
+        return True
     if _host.load().cache_write(kv_c, k_pe, slot_mapping, cache, None):
         return
     _need_cuda(kv_c, k_pe, slot_mapping, cache)
