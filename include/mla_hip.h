@@ -405,10 +405,11 @@ int dsa_topk_rows(const float* logits, int64_t logits_stride, const int32_t* seq
                   size_t workspace_bytes, mlahip_stream_t stream);
 
 /* dsa_topk with the picks also as bits: bit (i & 7) of byte i >> 3 of mask[t] (rows mask_stride bytes apart) says whether
- * position i is picked, for the positions token t sees; bits behind them are undefined.  16-byte aligned logits rows. */
+ * position i is picked, for the positions token t sees; bits behind them are undefined.  16-byte aligned logits rows.
+ * max_keys: the most keys any token sees, where that is known to be less than the row stride (0: the stride). */
 int dsa_topk_mask(const float* logits, int64_t logits_stride, const int32_t* seq_lens, const int32_t* query_start_loc,
                   int32_t batch, int32_t max_q_len, int32_t k, int32_t* out_indices, int64_t out_stride, void* mask,
-                  int64_t mask_stride, void* workspace, size_t workspace_bytes, mlahip_stream_t stream);
+                  int64_t mask_stride, int32_t max_keys, void* workspace, size_t workspace_bytes, mlahip_stream_t stream);
 
 /* ---- sparse MLA over the selected keys ----------------------------------------------------------
  * Replaces torch.ops.custom.npu_sparse_flash_attention, attention/backends/dsa.py:259-291 (sparse_block_size 1,

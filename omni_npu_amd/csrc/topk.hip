@@ -29,12 +29,14 @@ __device__ __forceinline__ uint32_t ordered_bits(float x) {
 
 // Workgroup-wide: given hist[kBins] (count per digit, larger digit = larger key) and `need` (>= 1, <= total),
 // find digit d with  count(digit > d) < need <= count(digit >= d).  Returns d, and the count above it via *above.
+template <int kThreads>
 __device__ int select_digit(int* hist, int* scratch, int need, int* above) {
+  constexpr int kOwn = kBins / kThreads;                   // bins of a thread, taken from the top
   const int tid = threadIdx.x;
-  // each thread owns 2 bins taken from the top: bins (kBins-1-2*tid) and (kBins-2-2*tid)
-  const int b0 = kBins - 1 - 2 * tid, b1 = b0 - 1;
-  const int c0 = hist[b0], c1 = hist[b1];
-  int v = c0 + c1;
+  const int b0 = kBins - 1 - kOwn * tid;
+  int c[kOwn], v = 0;
+#pragma unroll
+  for (int i = 0; i < kOwn; i++) { c[i] = hist[b0 - i]; v += c[i]; }
   // inclusive scan over threads (descending bins)
   const int lane = tid & 63, w = tid >> 6;
   int s = v;
@@ -47,11 +49,16 @@ __device__ int select_digit(int* hist, int* scratch, int need, int* above) {
   __syncthreads();
   int base = 0;
   for (int i = 0; i < w; i++) base += scratch[i];
-  const int incl = base + s, excl = incl - v;              // keys in bins above this thread's pair: excl
+  const int incl = base + s, excl = incl - v;              // keys in bins above this thread's: excl
   __syncthreads();
   if (excl < need && need <= incl) {                       // exactly one thread
-    if (need <= excl + c0) { scratch[32] = b0; scratch[33] = excl; }
-    else { scratch[32] = b1; scratch[33] = excl + c0; }
+    int sum = excl;
+    bool found = false;
+#pragma unroll
+    for (int i = 0; i < kOwn; i++) {
+      if (!found && need <= sum + c[i]) { scratch[32] = b0 - i; scratch[33] = sum; found = true; }
+      sum += c[i];
+    }
   }
   __syncthreads();
   const int d = scratch[32];
@@ -173,7 +180,7 @@ __device__ void radix_threshold(Each each, int need, int* hist, int* scratch, ui
     });
     __syncthreads();
     int above;
-    const int d = select_digit(hist, scratch, need, &above);
+    const int d = select_digit<kThreads>(hist, scratch, need, &above);
     need -= above;
     prefix |= (uint32_t)d << sh;
     pmask |= dm << sh;
@@ -192,7 +199,7 @@ __device__ void radix_threshold(Each each, int need, int* hist, int* scratch, ui
     });
     __syncthreads();
     int above;
-    const int d = select_digit(hist, scratch, need, &above);
+    const int d = select_digit<kThreads>(hist, scratch, need, &above);
     need -= above;
     ppre |= (uint32_t)d << psh[pass];
     pm |= 0x7FFu << psh[pass];
@@ -202,14 +209,15 @@ __device__ void radix_threshold(Each each, int need, int* hist, int* scratch, ui
 }
 
 // Threshold among m <= kRankMax candidates in LDS by ranking: the candidate with exactly `need - 1` larger keys.  All
-// 1024 threads take part: thread (c, g) compares candidate c with candidates g, g + G, ... and the partial ranks meet in
+// kThreads (>= kRankMax) threads take part: thread (c, g) compares candidate c with candidates g, g + G, ... and the partial ranks meet in
 // `rank` (LDS, at least kRankMax ints).
+template <int kThreads>
 __device__ __forceinline__ void rank_threshold(const uint32_t* cand_u, const uint32_t* cand_i, int m, int need, int* rank,
                                                int* scratch, uint32_t* prefix_out, uint32_t* pos_out) {
   const int tid = threadIdx.x;
   int mpad = 64;
   while (mpad < m) mpad <<= 1;
-  const int groups = kTopkThreads / mpad;
+  const int groups = kThreads / mpad;
   const int c = tid & (mpad - 1), g = tid / mpad;
   if (tid < kRankMax) rank[tid] = 0;
   __syncthreads();
@@ -329,7 +337,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_kernel(const TopkParams
   sweep<kVec>(x, 0, n, tid, kTopkThreads, [&](float v, int) { atomicAdd(&hist[linear_bin(v, scale, shift)], 1); });
   __syncthreads();
   int above;
-  const int d = select_digit(hist, scratch, k, &above);
+  const int d = select_digit<kTopkThreads>(hist, scratch, k, &above);
   int need = k - above;                                    // wanted among the keys of bin d (>= 1)
   const int in_bin = hist[d];
   __syncthreads();
@@ -355,7 +363,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_kernel(const TopkParams
     });
     __syncthreads();
     if (in_bin <= kRankMax) {
-      rank_threshold(cand_u, cand_i, in_bin, need, hist, scratch, &prefix, &pos_thresh);
+      rank_threshold<kTopkThreads>(cand_u, cand_i, in_bin, need, hist, scratch, &prefix, &pos_thresh);
     } else {
       radix_threshold<kTopkThreads>([&](auto&& f) { for (int j = tid; j < in_bin; j += kTopkThreads) f(cand_u[j], cand_i[j]); }, need, hist,
                       scratch, &prefix, &pos_thresh);
@@ -390,6 +398,171 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_kernel(const TopkParams
   for (int i = 0; i < w; i++) o += scratch[i];
 
   ordered_write<kVec>(x, out, r_lo, r_hi, lane, o, k, prefix, pos_thresh);
+}
+
+// ---- the same selection for many short rows: a prompt's tokens ---------------------------------------------------
+// What bounds the kernel above on such rows is not their bytes but its chain: three reads of the row and a dozen barriers of
+// sixteen wavefronts, two workgroups to a CU.  Here a workgroup is four wavefronts that read the row ONCE into registers
+// (up to kShortKeys keys, wavefront w the contiguous quarter w) and five of them share a CU, so that one's round trips and
+// barriers run beside the others' work; the picks are put together in LDS and leave in whole lines.  us per
+// launch, k = 2048, the kernel above -> this one: 4096 tokens of 2500 / 5000 / 8192 keys 177 / 192 / 208 -> 43 / 55 / 75.
+constexpr int kShortThreads = 256;
+constexpr int kShortGroups = 8;                            // of 256 keys, in the registers of a wavefront
+constexpr int kShortKeys = 4 * kShortGroups * 256;         // 8192
+constexpr int kShortCand = 1024;                           // boundary-bin keys that fit in LDS
+
+__global__ __launch_bounds__(kShortThreads, 4) void dsa_topk_short_kernel(const TopkParams p) {
+  __shared__ __attribute__((aligned(16))) int hist[kBins]; // later: the picks in order
+  __shared__ int scratch[64];
+  __shared__ uint32_t cand_u[kShortCand];
+  __shared__ uint32_t cand_i[kShortCand];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int b = blockIdx.x / p.max_q_len;
+  const int ti = blockIdx.x - b * p.max_q_len;
+  int q0, qlen;
+  if (p.qsl) { q0 = p.qsl[b]; qlen = p.qsl[b + 1] - q0; } else { q0 = b * p.max_q_len; qlen = p.max_q_len; }
+  if (ti >= qlen) return;
+  const int t = q0 + ti;
+  int n = p.seq_lens[b] - qlen + ti + 1;                   // visible keys
+  n = n < 0 ? 0 : (n < kShortKeys ? n : kShortKeys);       // (the rows hold no more)
+  const TopkSink out = topk_sink(p, b, t);
+  const int k = p.k;
+  if (p.counts && tid == 0) p.counts[t] = n < k ? n : k;
+  const bool wide = !out.rows && (k & 3) == 0 && ((uintptr_t)out.out & 15) == 0;
+
+  if (n <= k) {                                            // everything is selected
+    if (wide) {
+      for (int i = tid * 4; i < k; i += kShortThreads * 4)
+        *(i32x4*)(out.out + i) = i32x4{i < n ? i : -1, i + 1 < n ? i + 1 : -1, i + 2 < n ? i + 2 : -1, i + 3 < n ? i + 3 : -1};
+    } else {
+      for (int i = tid; i < k; i += kShortThreads) {
+        if (i < n) out.put(i, i); else out.out[i] = -1;
+      }
+    }
+    if (out.mask) for (int i = tid; i * 8 < n; i += kShortThreads) out.mask[i] = 0xff;    // (bits at and behind n mean nothing)
+    return;
+  }
+
+  // ---- this lane's keys: r_lo + j * 256 + lane * 4 + e, groups behind the wavefront's range left out ----
+  const float* x = p.logits + (int64_t)t * p.l_st;
+  const int per = ((n + 3) / 4 + 255) / 256 * 256;
+  const int r_lo = w * per;
+  const int r_hi = r_lo + per < n ? r_lo + per : n;
+  const int at0 = r_lo + lane * 4;
+  float v[kShortGroups][4];
+#pragma unroll
+  for (int j = 0; j < kShortGroups; j++) {
+    const int i = at0 + j * 256;
+    if (i + 3 < r_hi) {
+      const f32x4 q = *(const f32x4*)(x + i);
+      v[j][0] = q[0]; v[j][1] = q[1]; v[j][2] = q[2]; v[j][3] = q[3];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; e++) v[j][e] = i + e < r_hi ? x[i + e] : 0.f;
+    }
+  }
+  auto each_key = [&](auto&& f) {                          // f(value, position)
+#pragma unroll
+    for (int j = 0; j < kShortGroups; j++)
+      if (r_lo + j * 256 < r_hi) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (at0 + j * 256 + e < r_hi) f(v[j][e], at0 + j * 256 + e);
+      }
+  };
+  for (int i = tid; i < kBins; i += kShortThreads) hist[i] = 0;
+  if (tid == 0) scratch[40] = 0;                           // candidate counter
+
+  // ---- range of the finite logits, histogram over the linear bins, the bin that holds the k-th largest ----
+  float lo = INFINITY, hi = -INFINITY;
+  each_key([&](float f, int) { if (fabsf(f) < INFINITY) { lo = fminf(lo, f); hi = fmaxf(hi, f); } });
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) { lo = fminf(lo, __shfl_xor(lo, o, 64)); hi = fmaxf(hi, __shfl_xor(hi, o, 64)); }
+  if (lane == 0) { scratch[w] = __float_as_int(lo); scratch[8 + w] = __float_as_int(hi); }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; i++) { lo = fminf(lo, __int_as_float(scratch[i])); hi = fmaxf(hi, __int_as_float(scratch[8 + i])); }
+  const float range = hi - lo;
+  const float scale = (range > 0.f && range < INFINITY) ? (float)kBins * 0.99999f / range : 0.f;
+  const float shift = scale != 0.f ? -lo * scale : 0.f;
+  each_key([&](float f, int) { atomicAdd(&hist[linear_bin(f, scale, shift)], 1); });
+  __syncthreads();
+  int above;
+  const int d = select_digit<kShortThreads>(hist, scratch, k, &above);
+  const int need = k - above;                              // wanted among the keys of bin d (>= 1)
+  const int in_bin = hist[d];
+  __syncthreads();
+
+  // ---- exact threshold among the keys of bin d ----
+  uint32_t prefix, pos_thresh;
+  if (in_bin <= kShortCand) {
+    each_key([&](float f, int i) {
+      if (linear_bin(f, scale, shift) == d) {
+        const int slot = atomicAdd(&scratch[40], 1);
+        cand_u[slot] = ordered_bits(f);
+        cand_i[slot] = (uint32_t)i;
+      }
+    });
+    __syncthreads();
+    if (in_bin <= kRankMax)
+      rank_threshold<kShortThreads>(cand_u, cand_i, in_bin, need, hist, scratch, &prefix, &pos_thresh);
+    else
+      radix_threshold<kShortThreads>([&](auto&& f) { for (int j = tid; j < in_bin; j += kShortThreads) f(cand_u[j], cand_i[j]); },
+                                     need, hist, scratch, &prefix, &pos_thresh);
+  } else {
+    // degenerate rows (a large share of equal or nearly equal logits): the radix passes read the row itself
+    radix_threshold<kShortThreads>(
+        [&](auto&& f) {
+#pragma unroll 1
+          for (int i = tid; i < n; i += kShortThreads) {
+            const float g = x[i];
+            if (linear_bin(g, scale, shift) == d) f(ordered_bits(g), (uint32_t)i);
+          }
+        },
+        need, hist, scratch, &prefix, &pos_thresh);
+  }
+
+  // ---- the picks as a bit per key of this lane; where the wavefront's start ----
+  uint32_t picks = 0;
+#pragma unroll
+  for (int j = 0; j < kShortGroups; j++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int i = at0 + j * 256 + e;
+      const uint32_t u = ordered_bits(v[j][e]);
+      picks |= (uint32_t)(i < r_hi && (u > prefix || (u == prefix && (uint32_t)i <= pos_thresh))) << (j * 4 + e);
+    }
+  int cnt = __popc(picks);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
+  __syncthreads();                                         // (the threshold has been read by all, hist is free)
+  if (lane == 0) scratch[w] = cnt;
+  __syncthreads();
+  int o = 0;
+  for (int i = 0; i < w; i++) o += scratch[i];
+  const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+  for (int j = 0; j < kShortGroups; j++) {
+    if (r_lo + j * 256 >= r_hi) break;
+    const uint32_t nib = picks >> (j * 4) & 15;
+    int at = o;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const uint64_t m = __builtin_amdgcn_ballot_w64((nib >> e & 1) != 0);
+      at += __builtin_popcountll(m & below);
+      o += __builtin_popcountll(m);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (nib >> e & 1) hist[at++ & (kBins - 1)] = at0 + j * 256 + e;      // (k picks in all, k <= kBins)
+    if (out.mask) out.put_bits(at0 + j * 256, r_hi, nib);
+  }
+  __syncthreads();
+  if (wide) {
+    for (int i = tid * 4; i < k; i += kShortThreads * 4) *(i32x4*)(out.out + i) = *(const i32x4*)(hist + i);
+  } else {
+    for (int i = tid; i < k; i += kShortThreads) out.put(i, hist[i]);
+  }
 }
 
 // ---- the same selection spread over several workgroups per token ------------------------------------------------
@@ -540,7 +713,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_gather_kernel(const Top
   hist[kTopkThreads + tid] = c1;
   __syncthreads();
   int above;
-  const int d = select_digit(hist, scratch, p.t.k, &above);
+  const int d = select_digit<kTopkThreads>(hist, scratch, p.t.k, &above);
   if (s == 0 && tid == 0) { p.meta[r.slot * 4 + 1] = d; p.meta[r.slot * 4 + 2] = p.t.k - above; }
   uint32_t* cand = p.cand + (int64_t)r.slot * p.cand_cap * 2;
   int cnt = 0;
@@ -614,7 +787,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_write_kernel(const Topk
   uint32_t prefix, pos_thresh;
   const bool in_lds = m <= kMwCandLds;
   if (m <= kRankMax) {
-    rank_threshold(cand_u, cand_i, m, need, hist, scratch, &prefix, &pos_thresh);
+    rank_threshold<kTopkThreads>(cand_u, cand_i, m, need, hist, scratch, &prefix, &pos_thresh);
   } else if (in_lds) {
     radix_threshold<kTopkThreads>([&](auto&& f) { for (int j = tid; j < m; j += kTopkThreads) f(cand_u[j], cand_i[j]); }, need,
                                   hist, scratch, &prefix, &pos_thresh);
@@ -716,6 +889,12 @@ __global__ __launch_bounds__(256) void dsa_build_rows_kernel(const RowsParams p)
 }  // namespace mlahip
 using namespace mlahip;
 
+// Rows of at most kShortKeys keys go to four wavefronts instead of sixteen where that is no slower: any number of rows up to
+// 6144 keys (us for one row of 2500 / 5000 keys: 9.4 against 11.7, 11.2 against 12.2), and more rows than CUs beyond that, as
+// sixteen wavefronts read one long row in less time (8192 keys, 1 / 128 / 256 / 512 rows: 13.9 / 15.1 / 15.5 / 17.2 against
+// 13.1 / 14.6 / 15.1 / 28.0).
+static bool topk_short_rows(int64_t tokens, int64_t max_keys) { return max_keys <= 6144 || (max_keys <= kShortKeys && tokens > 256); }
+
 // slices per token in the multi-workgroup variant, or 0 when the one-workgroup kernel should run: rows too long for
 // kMaxSlices slices, or so many tokens that one workgroup each already fills the chip
 static int topk_slices(int64_t tokens, int64_t logits_stride) {
@@ -734,8 +913,8 @@ extern "C" size_t dsa_topk_workspace_bytes(int32_t batch, int32_t max_q_len, int
 static int topk_impl(const float* logits, int64_t logits_stride, const int32_t* seq_lens, const int32_t* query_start_loc,
                      int32_t batch, int32_t max_q_len, int32_t k, int32_t* out_indices, int64_t out_stride,
                      const int32_t* block_table, int64_t bt_stride, int32_t max_blocks, int32_t page_size, int64_t num_pages,
-                     int32_t* rows, int64_t rows_stride, int32_t* counts, uint8_t* mask, int64_t mask_stride, void* workspace,
-                     size_t workspace_bytes, hipStream_t stream) {
+                     int32_t* rows, int64_t rows_stride, int32_t* counts, uint8_t* mask, int64_t mask_stride, int64_t max_keys,
+                     void* workspace, size_t workspace_bytes, hipStream_t stream) {
   MLA_REQUIRE(logits && seq_lens && out_indices, MLA_ERR_NULL, "dsa_topk: null pointer argument");
   MLA_REQUIRE(batch >= 0 && max_q_len >= 1 && k >= 1 && out_stride >= k, MLA_ERR_SHAPE,
               "dsa_topk: batch=%d max_q_len=%d k=%d out_stride=%lld", batch, max_q_len, k, (long long)out_stride);
@@ -748,6 +927,10 @@ static int topk_impl(const float* logits, int64_t logits_stride, const int32_t* 
   MLA_REQUIRE(!mask || vec, MLA_ERR_SHAPE, "dsa_topk: a pick mask wants 16-byte aligned logits rows");
   const int64_t tokens = (int64_t)batch * max_q_len;
   const int slices = topk_slices(tokens, logits_stride);
+  if (vec && k <= kBins && topk_short_rows(tokens, max_keys ? max_keys : logits_stride)) {
+    hipLaunchKernelGGL(dsa_topk_short_kernel, dim3(batch * max_q_len), dim3(kShortThreads), 0, stream, p);
+    return check_launch("dsa_topk_short_kernel");
+  }
   if (!workspace || slices == 0) {
     if (vec) hipLaunchKernelGGL(dsa_topk_kernel<4>, dim3(batch * max_q_len), dim3(kTopkThreads), 0, stream, p);
     else hipLaunchKernelGGL(dsa_topk_kernel<1>, dim3(batch * max_q_len), dim3(kTopkThreads), 0, stream, p);
@@ -784,7 +967,7 @@ extern "C" int dsa_topk(const float* logits, int64_t logits_stride, const int32_
                         int32_t batch, int32_t max_q_len, int32_t k, int32_t* out_indices, int64_t out_stride,
                         void* workspace, size_t workspace_bytes, hipStream_t stream) {
   return topk_impl(logits, logits_stride, seq_lens, query_start_loc, batch, max_q_len, k, out_indices, out_stride, nullptr, 0,
-                   1, 1, 1, nullptr, 0, nullptr, nullptr, 0, workspace, workspace_bytes, stream);
+                   1, 1, 1, nullptr, 0, nullptr, nullptr, 0, 0, workspace, workspace_bytes, stream);
 }
 
 // dsa_topk and dsa_build_rows in one: besides the positions (the reference's index buffer) every pick is translated
@@ -799,18 +982,19 @@ extern "C" int dsa_topk_rows(const float* logits, int64_t logits_stride, const i
               MLA_ERR_SHAPE, "dsa_topk_rows: page_size=%d max_blocks=%d rows_stride=%lld", page_size, max_blocks,
               (long long)rows_stride);
   return topk_impl(logits, logits_stride, seq_lens, query_start_loc, batch, max_q_len, k, out_indices, out_stride, block_table,
-                   bt_stride, max_blocks, page_size, num_pages, rows, rows_stride, counts, nullptr, 0, workspace, workspace_bytes, stream);
+                   bt_stride, max_blocks, page_size, num_pages, rows, rows_stride, counts, nullptr, 0, 0, workspace, workspace_bytes, stream);
 }
 
 // dsa_topk with the picks also as bits: bit (i & 7) of byte i >> 3 of mask[t] says whether position i is picked, for the
-// positions token t sees (bits behind them are undefined).
+// positions token t sees (bits behind them are undefined).  max_keys: the most keys any token sees, where that is known to be
+// less than the row stride (0: the stride).
 extern "C" int dsa_topk_mask(const float* logits, int64_t logits_stride, const int32_t* seq_lens,
                              const int32_t* query_start_loc, int32_t batch, int32_t max_q_len, int32_t k,
-                             int32_t* out_indices, int64_t out_stride, void* mask, int64_t mask_stride, void* workspace,
-                             size_t workspace_bytes, hipStream_t stream) {
+                             int32_t* out_indices, int64_t out_stride, void* mask, int64_t mask_stride, int32_t max_keys,
+                             void* workspace, size_t workspace_bytes, hipStream_t stream) {
   MLA_REQUIRE(mask, MLA_ERR_NULL, "dsa_topk_mask: null pointer argument");
   return topk_impl(logits, logits_stride, seq_lens, query_start_loc, batch, max_q_len, k, out_indices, out_stride, nullptr, 0,
-                   1, 1, 1, nullptr, 0, nullptr, (uint8_t*)mask, mask_stride, workspace, workspace_bytes, stream);
+                   1, 1, 1, nullptr, 0, nullptr, (uint8_t*)mask, mask_stride, max_keys, workspace, workspace_bytes, stream);
 }
 
 extern "C" int dsa_build_rows(const int32_t* indices, int64_t indices_stride, const int32_t* block_table, int64_t bt_stride,

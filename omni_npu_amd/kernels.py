@@ -731,7 +731,7 @@ def topk(logits: torch.Tensor, seq_lens: torch.Tensor, k: int, out: torch.Tensor
                 mask.shape[1] * 32 < logits.shape[1]:
             raise TypeError("topk: mask must be int32 [T, W] with contiguous rows of a bit per logit")
         rc = lib.dsa_topk_mask(logits.data_ptr(), logits.stride(0), seq_lens.data_ptr(), qsl, b, q_len, k, o2.data_ptr(),
-                               o2.stride(0), mask.data_ptr(), mask.stride(0) * 4, ws_ptr, ws_bytes, _stream(logits))
+                               o2.stride(0), mask.data_ptr(), mask.stride(0) * 4, logits.shape[1], ws_ptr, ws_bytes, _stream(logits))
         _lib.check(rc, "dsa_topk_mask")
         return out
     rc = lib.dsa_topk(logits.data_ptr(), logits.stride(0), seq_lens.data_ptr(), qsl, b, q_len, k, o2.data_ptr(),

@@ -424,6 +424,49 @@ def test_prompt_scores_are_the_streaming_kernels_bits(dev, q_lens, extra):
     assert torch.equal(lg2[far], ref[far])
 
 
+@pytest.mark.parametrize("k", [2048, 2047, 1, 300])
+@pytest.mark.parametrize("n,stride", [(8192, 8192), (8191, 8192), (2300, 2304), (1024, 1024), (257, 8192)])
+def test_topk_of_short_rows_is_the_general_kernel(dev, n, stride, k):
+    """Rows of up to 8192 keys, enough tokens for the four-wavefront kernel, against the same rows one 4-byte column further on
+    (not 16-byte aligned: the general kernel): ragged lengths from nothing to the whole row, ties, equal keys, infinities, NaN;
+    the row lists and the pick bits as well."""
+    from omni_npu_amd import kernels as K
+    t = 300
+    g = torch.Generator().manual_seed(n + k)
+    x = torch.randn(t, n, generator=g)
+    x[0::7] = torch.round(x[0::7] * 4) / 4
+    x[1::7] = 1.0
+    x[2::7, : n // 2] = x[2::7, n - n // 2:]
+    x[3::7, 1::9], x[3::7, 2::11], x[3::7, 3] = float("inf"), float("-inf"), 1e30
+    x[4::7, 5::13] = float("nan")
+    x[5::7, : n // 3] = -0.0
+    lg, odd = torch.zeros(t, stride, device=dev), torch.zeros(t, stride + 5, device=dev)
+    lg[:, :n], odd[:, 1:n + 1] = x.to(dev), x.to(dev)
+    lens = torch.randint(0, n + 1, (t,), generator=g, dtype=torch.int32)
+    lens[:150] = n
+    lens = lens.to(dev)
+    a, b = torch.full((t, k), -7, dtype=torch.int32, device=dev), torch.full((t, k), -8, dtype=torch.int32, device=dev)
+    K.topk(lg, lens, k, a)
+    K.topk(odd[:, 1:], lens, k, b, single_workgroup=True)
+    assert torch.equal(a, b)
+    bt = torch.randperm(t * 64, generator=g).view(t, 64).int().to(dev)
+    rows, cnt = torch.full((t, k), -7, dtype=torch.int32, device=dev), torch.zeros(t, dtype=torch.int32, device=dev)
+    rows2, cnt2 = rows.clone(), cnt.clone()
+    a.fill_(-7)
+    K.topk(lg, lens, k, a, block_table=bt, num_pages=t * 64, rows=rows, counts=cnt)
+    K.topk(odd[:, 1:], lens, k, b, single_workgroup=True, block_table=bt, num_pages=t * 64, rows=rows2, counts=cnt2)
+    assert torch.equal(a, b) and torch.equal(rows, rows2) and torch.equal(cnt, cnt2)
+    mask = torch.randint(-2 ** 31, 2 ** 31 - 1, (t, stride // 32), generator=g).int().to(dev)
+    a.fill_(-7)
+    K.topk(lg, lens, k, a, mask=mask)
+    assert torch.equal(a, b)
+    bits = (mask.cpu().view(t, -1, 1) >> torch.arange(32).view(1, 1, -1) & 1).view(t, -1)
+    want = torch.zeros(t, stride + 1, dtype=torch.int32)
+    want.scatter_(1, torch.where(b < 0, stride, b).long().cpu(), 1)
+    seen = torch.arange(stride)[None] < lens.cpu()[:, None]
+    assert torch.equal(bits.int()[seen], want[:, :stride][seen])
+
+
 @pytest.mark.parametrize("t,n,k", [(1, 40, 64), (3, 65, 64), (300, 700, 64), (5, 9000, 2048), (257, 9001, 2048)])
 def test_topk_mask_names_the_picks(dev, t, n, k):
     """dsa_topk_mask: the bits of the visible positions are the index list, in the one-workgroup and the sliced variant."""
