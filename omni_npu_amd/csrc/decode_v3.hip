@@ -484,20 +484,25 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
       for (int k = 0; k < kCopies; k++) issue_piece(c, k, std::false_type{}, std::false_type{});
     }
   };
-  // Row list: the rows of the first kLead blocks are fetched together (one round trip) before any copy goes out
-  auto issue_first = [&]() {
+  // Where the first copies come from: the first page numbers, or (row list) the rows of the first kLead blocks, fetched
+  // together and waited for before any copy goes out.
+  auto ask_first = [&]() {
     issue_reset();
     if constexpr (kSparse) {
 #pragma unroll
       for (int j = 0; j < kLead; j++) ids_dma(blk_begin + j);
+    }
+  };
+  auto issue_first = [&]() {
+    if constexpr (kSparse) {
       MLA_WAIT_VMCNT(0);
       ids_fetch(blk_begin);
     }
     issue_block(blk_begin);
   };
-  auto issue_next_two = [&]() {
+  auto issue_upto_lead = [&](int from) {
 #pragma unroll 1
-    for (int j = 1; j < kLead && j < nb; j++) {
+    for (int j = from; j < kLead && j < nb; j++) {
       ids_fetch(blk_begin + j);
       issue_block(blk_begin + j);
     }
@@ -510,17 +515,27 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
   // start of a segment) and picks its operands from there.  The copies of the first key blocks have to wait until
   // every wave has its query in registers (one barrier).
   bf16x8 qf[18];                                             // contraction steps of 32: 16 over the latent part, 2 over rope
-  // One row group: the two wavefronts that can own rows stage their query in the tile buffer of the segment's FOURTH block,
-  // which is not requested before the block loop runs, so the copying wavefronts ask for the first three blocks now and
-  // the query's round trip to memory hides under theirs.
-  const uint32_t q_stage = kRG == 1 ? (uint32_t)(((blk_begin + 3) & 3) * kNopeBufB) : 0u;
+  // One or two row groups: the wavefronts that can own rows stage their query in the tile buffer of the segment's FOURTH block
+  // (two groups: of the third and the fourth), which is not requested before the query has been read, so the copying
+  // wavefronts ask for the first three (two) blocks now and the query's round trip to memory hides under theirs.  With four
+  // groups the query fills all four buffers; what can be asked for beside it is where the first blocks lie.  (us per layer,
+  // against two and four groups that asked for nothing before the query had been read: 7 requests of 300-3000 keys, 128 heads,
+  // replayed 41.8 -> 40.9; one of 128k keys 71.2 -> 70.8; 64 of 4k-8k 146.5 -> 146.2.)
+  constexpr int kEarly = kRG == 1 ? kLead : kRG == 2 ? kLead - 1 : 0;        // blocks requested beside the query
+  const uint32_t q_stage = kRG == 4 ? wave * 16384u
+                         : (uint32_t)(((blk_begin + kEarly + (wave >> 1)) & 3) * kNopeBufB + (wave & 1) * 16384);
   if (!has_rows) {
 #pragma unroll
     for (int kk = 0; kk < 18; kk++) qf[kk] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    if constexpr (kRG == 1) {
+    if constexpr (kEarly != 0) {
+      ask_first();
       issue_first();
       ids_dma(blk_begin + kLead);
-      issue_next_two();
+#pragma unroll 1
+      for (int j = 1; j < kEarly && j < nb; j++) {
+        ids_fetch(blk_begin + j);
+        issue_block(blk_begin + j);
+      }
     }
   } else {
     // Contraction step kk of the latent part covers the 16-byte granules 16*(kk%4) + 4g' + kk/4, g' = 0..3, and lane group
@@ -540,7 +555,7 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
       for (int k = 0; k < 16; k++) {
         const bool ok = r0 + k < rows && L > 0;              // rows that do not exist read row 0 of the sequence
         const __bf16* src = qn0 + (ok ? (int64_t)(q0 + t) * st + (int64_t)h * sh : (int64_t)q0 * st);
-        dma16_sv(src, (uint32_t)((ln ^ swz_nope(k)) << 4), lds0 + q_stage + wave * 16384 + k * 1024);
+        dma16_sv(src, (uint32_t)((ln ^ swz_nope(k)) << 4), lds0 + q_stage + k * 1024);
         h++;
         if (h == nh) { h = 0; t++; }
       }
@@ -558,9 +573,10 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
         dma16_v(src, lds0 + kPOff + wave * 2048 + j * 1024);
       }
     }
+    if constexpr (kEarly == 0) ask_first();
     MLA_WAIT_VMCNT(0);
     const int ql16 = ln & 15, qg = ln >> 4;
-    const uint32_t qoff = (uint32_t)(wave * 16384 + ql16 * 1024 + (((qg << 2) ^ swz_nope(ql16)) << 4));
+    const uint32_t qoff = (uint32_t)(ql16 * 1024 + (((qg << 2) ^ swz_nope(ql16)) << 4));
 #pragma unroll
     for (int kk = 0; kk < 16; kk++) qf[kk] = *(const bf16x8*)(lds + q_stage + (qoff ^ (uint32_t)((kk >> 2) << 4)) + (kk & 3) * 256);
 #pragma unroll
@@ -569,7 +585,8 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
     for (int kk = 0; kk < 18; kk++) asm volatile("" : "+v"(qf[kk]));           // the query stays in VGPRs
   }
   lds_barrier();                                              // every wave has read its query: the tile buffers are free
-  if constexpr (kRG != 1) issue_first();
+  if constexpr (kEarly == 0) issue_first();
+  else if constexpr (kEarly < kLead) { if (!has_rows) issue_upto_lead(kEarly); }
 
   f32x16 acc[2][4];                                          // [32-column block of this wave's 64][row group]
 #pragma unroll
@@ -859,7 +876,7 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
     }
   }
   bool restart = false;
-  bool early_issued = kRG == 1;  // (one row group: the first three blocks were requested beside the query)
+  bool early_issued = kEarly != 0;   // (the first kLead blocks have been requested by now)
   int restarts_left = 4;         // every restart raises a reference by more than 2^100: fp32 has room for three
   do {
     if (restart) {
@@ -879,13 +896,14 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
         for (int j = 0; j < 4; j++)
 #pragma unroll
           for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+      ask_first();
       issue_first();
       restart = false;
       early_issued = false;
     }
     if (!early_issued) {
       ids_dma(blk_begin + kLead);                             // (older than the copies below: their wait covers it)
-      issue_next_two();
+      issue_upto_lead(1);
     }
     early_issued = false;
     // ---- block 0: QK, softmax, publish ----
