@@ -20,6 +20,10 @@
 
 namespace mlahip {
 
+// max(x, 0) of a product sum of e4m3 numbers (finite, or NaN: then 0, as fmaxf gives) in one instruction: fmaxf is compiled to
+// two, the first of which only quiets a signalling NaN, and 32 of the 96 vector instructions of a token and block were that.
+__device__ __forceinline__ float relu(float x) { return __builtin_amdgcn_fmed3f(x, 0.f, 3.402823466e38f); }
+
 constexpr int kIdxDim = 128;
 constexpr int kIdxRing = 4;                           // ring slots per wavefront (3 blocks requested ahead)
 constexpr int kIdxSlotB = 32 * kIdxDim + 32 * 4;      // 4224: 32 key rows + their 32 scales
@@ -202,8 +206,8 @@ __global__ __launch_bounds__(256, 2) void dsa_indexer_fp8_kernel(const IndexerPa
     float acc = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; r++) {
-      acc = fmaf(wr[0][r], fmaxf(c0[r], 0.f), acc);
-      acc = fmaf(wr[1][r], fmaxf(c1[r], 0.f), acc);
+      acc = fmaf(wr[0][r], relu(c0[r]), acc);
+      acc = fmaf(wr[1][r], relu(c1[r]), acc);
     }
     acc += xor32(acc);
     const int key = key_begin + 32 * g + key_l;
@@ -214,16 +218,18 @@ __global__ __launch_bounds__(256, 2) void dsa_indexer_fp8_kernel(const IndexerPa
 
 // The same scores for prompts, where neighbouring query tokens see the same keys: the kernel above reads every token's keys
 // for itself (10 168 prompt tokens, 20 M (token, key) pairs: 2.7 GB through the L2s, 980 us).  Here a workgroup keeps the
-// queries of kTileTok tokens of one request in LDS (64 KiB, two workgroups per CU) and each of its wavefronts walks every
+// queries of kTileTok tokens of one request in LDS (32 KiB, four workgroups per CU) and each of its wavefronts walks every
 // 4 gridDim.x-th block of 32 keys, held in registers (the next block on its way meanwhile), against all of the tokens: a
 // key is read once per kTileTok tokens, a query operand from LDS at a quarter of its rate, and what is left is the 16 MFMAs
-// and 64 relu-FMAs per token and block.  Same operations in the same order as above: the same bits.
-constexpr int kTileTok = 8;
+// and 64 vector instructions per token and block, which wavefronts of one SIMD do beside each other: the more of them the
+// better (eight tokens and two wavefronts per SIMD, relu in two instructions: 290 us on those prompts; now about 165).  Same
+// operations in the same order as above: the same bits.
+constexpr int kTileTok = 4;
 constexpr int kTileMinQ = 16;                         // shorter requests (decode, MTP) take the streaming kernel
 constexpr int kTileWOff = kTileTok * 64 * kIdxDim;    // 65536: weights [token][head] behind the query rows
 constexpr int kTileLdsB = kTileWOff + kTileTok * 64 * 4;
 
-__global__ __launch_bounds__(256, 2) void dsa_indexer_tile_kernel(const IndexerParams p) {
+__global__ __launch_bounds__(256, 4) void dsa_indexer_tile_kernel(const IndexerParams p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -307,8 +313,8 @@ __global__ __launch_bounds__(256, 2) void dsa_indexer_tile_kernel(const IndexerP
         const f32x4 w0 = *(const f32x4*)(wp + q * 32), w1 = *(const f32x4*)(wp + 128 + q * 32);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          acc = fmaf(w0[e], fmaxf(c0[q * 4 + e], 0.f), acc);
-          acc = fmaf(w1[e], fmaxf(c1[q * 4 + e], 0.f), acc);
+          acc = fmaf(w0[e], relu(c0[q * 4 + e]), acc);
+          acc = fmaf(w1[e], relu(c1[q * 4 + e]), acc);
         }
       }
       acc += xor32(acc);
@@ -496,9 +502,10 @@ static int indexer_scores_impl(const void* q8, int64_t q_stride_t, int64_t q_str
   p.batch = batch; p.max_q_len = max_q_len; p.num_heads = num_heads; p.page_size = page_size; p.num_pages = num_pages;
   p.logits = logits; p.l_st = logits_stride; p.skip_up_to = skip_up_to;
   if (max_q_len >= kTileMinQ) {
-    // about 2048 workgroups (four rounds of two per CU), so that the short ones at the start of a prompt even out
+    // about 8192 workgroups (eight rounds of four per CU, those of the tokens that are skipped and of the shorter requests
+    // among them, which end at once), so that the short ones at the start of a prompt even out
     const int64_t groups = (int64_t)batch * ((max_q_len + kTileTok - 1) / kTileTok);
-    int64_t split = (2048 + groups - 1) / groups;
+    int64_t split = (8192 + groups - 1) / groups;
     const int64_t most = (max_seq_len + 127) / 128;           // a block per wavefront
     split = split > 16 ? 16 : split;
     split = split > most ? most : split;
