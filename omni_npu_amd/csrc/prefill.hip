@@ -139,8 +139,13 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
     const int nqb = gridDim.x, npairs = gridDim.y * gridDim.z;
     if ((npairs & 7) == 0) {
       const int lin = blockIdx.x + nqb * (blockIdx.y + gridDim.y * blockIdx.z);
-      const int j = lin >> 3, pair = (j / nqb) * 8 + (lin & 7);
+      const int j = lin >> 3, run = j / nqb, pair = run * 8 + (lin & 7);
       qb = j % nqb;
+      // Under the causal mask a block's work grows with its number.  An XCD deals its queue to 32 CUs in turn, two workgroups to
+      // each, so every second stretch of about 32 runs backwards: a CU gets a long and a short one instead of the same twice
+      // (1017 tokens behind 3072 cached ones beside 31 decodes, 64 heads: 376 -> 367 us per layer; 7 ragged prompts, 32 heads:
+      // 417 -> 414).
+      if (p.causal && ((run / (nqb < 32 ? 32 / nqb : 1)) & 1)) qb = nqb - 1 - qb;
       head = pair % gridDim.y;
       b = pair / gridDim.y;
     }
