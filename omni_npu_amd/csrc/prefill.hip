@@ -32,6 +32,7 @@
 // 1.4e-3 to 1.7e-3.)  The conversion is exact for |v| in [2^-14, 65504]; smaller values lose at most 2^-25 absolute,
 // larger ones saturate (round toward zero never makes an infinity).
 #include "mla_common.hpp"
+#include <type_traits>
 
 namespace mlahip {
 
@@ -87,6 +88,8 @@ __device__ __forceinline__ PfLaneOffsets pf_lane_offsets(const PrefillParams& p,
   }
   return o;
 }
+// kParts: 1 = the three key sub-tiles, 2 = the two value sub-tiles, 3 = both.
+template <int kParts>
 __device__ __forceinline__ void pf_issue_full_tile(const PrefillParams& p, const PfLaneOffsets& o, int64_t k0, int head,
                                                    uint32_t buf, int wave) {
   const char* kn = (const char*)(p.k_nope + k0 * p.kn_st + (int64_t)head * p.kn_sh);
@@ -95,13 +98,18 @@ __device__ __forceinline__ void pf_issue_full_tile(const PrefillParams& p, const
 #pragma unroll
   for (int i = 0; i < 2; i++) {
     const uint32_t dst = buf + (wave * 2 + i) * 1024;
-    dma16_sv(kn, o.kn[i], dst);
-    dma16_sv(kn + 128, o.kn[i], dst + kPfSubB);
-    dma16_sv(kp, o.kp[i], dst + 2 * kPfSubB);
-    dma16_sv(vv, o.v[i], dst + 3 * kPfSubB);
-    dma16_sv(vv + 128, o.v[i], dst + 4 * kPfSubB);
+    if constexpr (kParts & 1) {
+      dma16_sv(kn, o.kn[i], dst);
+      dma16_sv(kn + 128, o.kn[i], dst + kPfSubB);
+      dma16_sv(kp, o.kp[i], dst + 2 * kPfSubB);
+    }
+    if constexpr (kParts & 2) {
+      dma16_sv(vv, o.v[i], dst + 3 * kPfSubB);
+      dma16_sv(vv + 128, o.v[i], dst + 4 * kPfSubB);
+    }
   }
 }
+template <int kParts>
 __device__ __forceinline__ void pf_issue_tile(const PrefillParams& p, int64_t k0, int64_t klast, int head, uint32_t buf,
                                               int wave, int lane) {
 #pragma unroll
@@ -113,11 +121,15 @@ __device__ __forceinline__ void pf_issue_tile(const PrefillParams& p, int64_t k0
     const __bf16* kn = p.k_nope + key * p.kn_st + (int64_t)head * p.kn_sh + c;
     const __bf16* vv = p.v + key * p.v_st + (int64_t)head * p.v_sh + c;
     const uint32_t dst = buf + (wave * 2 + i) * 1024;
-    dma16_v(kn, dst);
-    dma16_v(kn + 64, dst + kPfSubB);
-    dma16_v(p.k_pe + key * p.kp_st + c, dst + 2 * kPfSubB);
-    dma16_v(vv, dst + 3 * kPfSubB);
-    dma16_v(vv + 64, dst + 4 * kPfSubB);
+    if constexpr (kParts & 1) {
+      dma16_v(kn, dst);
+      dma16_v(kn + 64, dst + kPfSubB);
+      dma16_v(p.k_pe + key * p.kp_st + c, dst + 2 * kPfSubB);
+    }
+    if constexpr (kParts & 2) {
+      dma16_v(vv, dst + 3 * kPfSubB);
+      dma16_v(vv + 64, dst + 4 * kPfSubB);
+    }
   }
 }
 
@@ -224,22 +236,53 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
     const int64_t klast = (int64_t)k0 + sk - 1;
     const PfLaneOffsets lane_off = pf_lane_offsets(p, wave, lane);
     const bool fast_ok = (uint64_t)p.kn_st * 128 < (1u << 31) && (uint64_t)p.v_st * 128 < (1u << 31) && (uint64_t)p.kp_st * 128 < (1u << 31);
-    auto issue = [&](int tile, uint32_t buf) {
+    auto issue = [&](int tile, uint32_t buf, auto parts) {
+      constexpr int kParts = decltype(parts)::value;
       const int64_t first = (int64_t)k0 + (int64_t)tile * kPfTile;
-      if (fast_ok && first + kPfTile - 1 <= klast) pf_issue_full_tile(p, lane_off, first, head, buf, wave);
-      else pf_issue_tile(p, first, klast, head, buf, wave, lane);
+      if (fast_ok && first + kPfTile - 1 <= klast) pf_issue_full_tile<kParts>(p, lane_off, first, head, buf, wave);
+      else pf_issue_tile<kParts>(p, first, klast, head, buf, wave, lane);
     };
-    issue(first_tile, lds0 + (first_tile & 1) * kPfBufB);
+    // per-lane LDS offsets: K granule 2 j + half of a row (j = 0..3 inside a sub-tile)
+    int koff[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) koff[j] = h32 * 128 + (((j * 2 + half) ^ pf_swz(h32 & 15)) << 4);
+
+    // The query comes through LDS, in rows: an operand load straight from memory asks for 16 bytes of 64 lines, 64 cycles of
+    // the CU's address unit each, and the twelve of a wavefront held up the first tile (7 ragged
+    // prompts, 32 heads, whose blocks see a dozen tiles each: 402 -> 394 us per layer, the order of blocks above included).  The latent part of the
+    // wavefront's 32 rows goes to the buffer of the second tile, which is asked for behind the loop's first barrier, the rope
+    // part to where the wavefront itself will copy the first tile's values, once it has read it.
+    const int first_buf = (first_tile & 1) * kPfBufB, other_buf = kPfBufB - first_buf;
+    {
+      const int sub = lane >> 3;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int r = i * 8 + sub;                             // row of the wavefront; those that do not exist repeat the last
+        int64_t tr = qb * kPfRows + wave * 32 + r;
+        tr = q0 + (tr < sq ? tr : sq - 1);
+        const int c = ((lane & 7) ^ pf_swz(r & 15)) * 8;
+        const __bf16* qn = p.q_nope + tr * p.qn_st + (int64_t)head * p.qn_sh + c;
+        const uint32_t dst = lds0 + other_buf + wave * 4096 + i * 1024;
+        dma16_v(qn, dst);
+        dma16_v(qn + 64, dst + 16384);
+        dma16_v(p.q_pe + tr * p.qp_st + (int64_t)head * p.qp_sh + c,
+                lds0 + first_buf + kPfVOff + (i >> 1) * kPfSubB + wave * 2048 + (i & 1) * 1024);
+      }
+    }
+    issue(first_tile, lds0 + first_buf, std::integral_constant<int, 1>{});
 
     bf16x8 qf[12];
     {
-      const __bf16* qn = p.q_nope + tq * p.qn_st + (int64_t)head * p.qn_sh + half * 8;
-      const __bf16* qp = p.q_pe + tq * p.qp_st + (int64_t)head * p.qp_sh + half * 8;
+      MLA_WAIT_VMCNT(6);                                       // the query is here, the six copies of the keys may be on their way
       const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+      const char* qn = lds + other_buf + wave * 4096;
+      const char* qp = lds + first_buf + kPfVOff + (h32 >> 4) * (kPfSubB - 2048) + wave * 2048;   // (koff counts rows 16.. from 2048 on)
 #pragma unroll
-      for (int kk = 0; kk < 8; kk++) { bf16x8 v = *(const bf16x8*)(qn + kk * 16); qf[kk] = row_ok ? v : zero; }
+      for (int kk = 0; kk < 8; kk++) { bf16x8 v = *(const bf16x8*)(qn + (kk >> 2) * 16384 + koff[kk & 3]); qf[kk] = row_ok ? v : zero; }
 #pragma unroll
-      for (int kk = 0; kk < 4; kk++) { bf16x8 v = *(const bf16x8*)(qp + kk * 16); qf[8 + kk] = row_ok ? v : zero; }
+      for (int kk = 0; kk < 4; kk++) { bf16x8 v = *(const bf16x8*)(qp + koff[kk]); qf[8 + kk] = row_ok ? v : zero; }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      issue(first_tile, lds0 + first_buf, std::integral_constant<int, 2>{});
       if constexpr (kHalf) {
 #pragma unroll
         for (int kk = 0; kk < 12; kk++) {
@@ -250,11 +293,8 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
         }
       }
     }
-    // per-lane LDS offsets: K granule 2 j + half of a row (j = 0..3 inside a sub-tile), V rows v_row and v_row + 8 with the
-    // 32-column halves of a sub-tile
-    int koff[4], voff[2][2];
-#pragma unroll
-    for (int j = 0; j < 4; j++) koff[j] = h32 * 128 + (((j * 2 + half) ^ pf_swz(h32 & 15)) << 4);
+    // V rows v_row and v_row + 8 with the 32-column halves of a sub-tile
+    int voff[2][2];
     const int g16 = lane >> 4, j16 = lane & 15;
     const int v_row = 4 * (g16 >> 1) + (j16 >> 2);
     const int v_cl = 2 * (g16 & 1) + ((j16 & 3) >> 1);
@@ -280,7 +320,7 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
       lds_barrier();
       const u32x2 bits = bits_next;
       if constexpr (kPick) bits_next = pick_tile(tile + 1 < tiles ? tile + 1 : tile);
-      if (tile + 1 < tiles) issue(tile + 1, lds0 + ((tile + 1) & 1) * kPfBufB);
+      if (tile + 1 < tiles) issue(tile + 1, lds0 + ((tile + 1) & 1) * kPfBufB, std::integral_constant<int, 3>{});
       const int key_base = tile * kPfTile;
       // V of this tile goes from bf16 to fp16 where it lies (thread t takes the 16-byte pieces t, t + 256, ...), then a
       // barrier: the four wavefronts read each other's pieces.  (Tried: the conversion's arithmetic and writes behind the
