@@ -222,7 +222,7 @@ __global__ __launch_bounds__(256, 2) void dsa_indexer_fp8_kernel(const IndexerPa
 // 4 gridDim.x-th block of 32 keys, held in registers (the next block on its way meanwhile), against all of the tokens: a
 // key is read once per kTileTok tokens, a query operand from LDS at a quarter of its rate, and what is left is the 16 MFMAs
 // and 64 vector instructions per token and block, which wavefronts of one SIMD do beside each other: the more of them the
-// better (eight tokens and two wavefronts per SIMD, relu in two instructions: 290 us on those prompts; now about 165).  Same
+// better (eight tokens and two wavefronts per SIMD, relu in two instructions: 286 us on those prompts; now 199).  Same
 // operations in the same order as above: the same bits.
 constexpr int kTileTok = 4;
 constexpr int kTileMinQ = 16;                         // shorter requests (decode, MTP) take the streaming kernel

@@ -134,6 +134,24 @@ def test_query_rope_strided_and_in_place(dev, layout, interleaved):
     assert torch.equal(qd[..., 128:], got) and torch.equal(qd[..., :128].cpu(), q[..., :128])
 
 
+@pytest.mark.parametrize("cut,width", [(1, 66), (2, 68), (0, 66), (0, 64)])
+def test_tables_on_any_boundary(dev, cut, width):
+    """Table rows on 2- and 4-byte boundaries, at strides that are no multiple of four entries, and 8-byte aligned ones (four
+    entries per load): the same bits, in all three launches that rotate."""
+    from omni_npu_amd import kernels as K
+    t, n, g = 9, 3, torch.Generator().manual_seed(width + cut)
+    kv, q = torch.randn(t, 576, generator=g).bfloat16().to(dev), torch.randn(t, n, 64, generator=g).bfloat16().to(dev)
+    gamma = torch.ones(512, dtype=torch.bfloat16, device=dev)
+    cos, sin = (x.to(dev) for x in O.rope_tables(torch.randint(0, 8192, (t,), generator=g)))
+    got = []
+    for cut_, width_ in ((0, 64), (cut, width)):
+        c, s = (torch.zeros(t, width_, dtype=torch.bfloat16, device=dev)[:, cut_:cut_ + cos.shape[1]].copy_(x) for x in (cos, sin))
+        kv_a, pe = torch.zeros(t, 512, dtype=torch.bfloat16, device=dev), torch.zeros(t, 64, dtype=torch.bfloat16, device=dev)
+        K.kv_rmsnorm_rope_cache(kv, gamma, c, s, None, None, None, eps=EPS, kv_a_out=kv_a, k_pe_out=pe)
+        got.append((kv_a, pe, K.interleave_rope(q, c, s), K.rotary_mul(q, c, s)))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and bool(got[0][1].any())
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 def test_fused_prologue_with_query_equals_the_two_launches(dev, fp8):
     """One launch for the key side (norm, rope, cache write, plain outputs) and the query's rope part, in place on a strided
