@@ -14,6 +14,7 @@ kernel leaves out the blocks between the sink and the window (prefill: kernels.p
 from __future__ import annotations
 
 import math
+import weakref
 from dataclasses import dataclass
 from typing import ClassVar, Optional, Tuple
 
@@ -199,7 +200,7 @@ class HalfUpProjection:
     # magnitude 2^-14 .. 65504 exactly; set prefill_kv_fp16 = False for a model whose keys or values can exceed that range.
     prefill_kv_fp16 = True
 
-    _half_w = None               # (address, version) of the up-projection weight and its fp16 copy
+    _half_w = None               # (weak reference to the up-projection weight, address and version) and its fp16 copy
 
     def _plain_up_weight(self) -> Optional[torch.Tensor]:
         """The up-projection weight [N*256, 512] if the prefill may make fp16 keys and values with it: plain, without bias."""
@@ -218,12 +219,13 @@ class HalfUpProjection:
             return None
         if w.dtype == torch.float16:
             return w
+        # (the reference dies with the weight: another one that comes to lie at its address is not taken for it)
         key = (w.data_ptr(), w.device, 0 if w.is_inference() else w._version)
-        if self._half_w is None or self._half_w[0] != key:
+        if self._half_w is None or self._half_w[0][0]() is not w or self._half_w[0][1:] != key:
             half = w.to(torch.float16)
             if w.is_cuda and torch.cuda.is_current_stream_capturing():
                 return half                                    # recorded, not computed: of no use to a later eager call
-            self._half_w = (key, half)
+            self._half_w = ((weakref.ref(w), *key), half)
         return self._half_w[1]
 
     def process_weights_after_loading(self, act_dtype: torch.dtype):
