@@ -825,7 +825,7 @@ def bench_layer(K, dev, args):
         "value": round(t_graph, 2), "unit": "us/layer", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "higher_is_better": False, "dtype": "bf16", "data": "synthetic",
         "config": {"workload": "configs[1] through NPUMLAMetadataBuilder + NPUMLAImpl.forward: norm + rope + cache write, "
-                               "query rope, absorption GEMM, split-KV decode, merge + W_UV", "batch": B, "heads": N,
+                               "query rope, absorption, split-KV decode, merge + W_UV", "batch": B, "heads": N,
                    "sum_seq_len": int(lens.sum()), "seed": args.seed},
         "layer_us": {"eager_launches_queued": round(t_eager, 2), "hip_graph_replay": round(t_graph, 2)},
         "roofline": {"kernel": "whole layer", "bound": "hbm", "achieved": round(alg_bytes / t_graph / 1e3, 1),
@@ -1036,9 +1036,9 @@ def bench_window(K, dev, args):
         "metric": "MLA decode with static sink + sliding window, us/layer (B=64, ctx 4k-8k, sink 128, window 4096, 128 heads, bf16)",
         "value": round(t_step, 2), "unit": "us/layer", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "higher_is_better": False, "dtype": "bf16", "data": "synthetic",
-        "config": {"workload": "static sink tokens + sliding window decode (plan + split + merge, graph replay)", "batch": B,
+        "config": {"workload": "static sink tokens + sliding window decode (split + merge, graph replay)", "batch": B,
                    "heads": N, "sink_len": sink, "window": win, "visible_keys": visible, "seed": args.seed},
-        "roofline": {"kernel": "mla_window_plan_kernel + mla_decode_v3_kernel<false, true, 4> + merge (whole step)", "bound": "hbm",
+        "roofline": {"kernel": "mla_decode_v3_kernel<false, true, 4> + merge (whole step)", "bound": "hbm",
                      "achieved": round(alg_bytes / t_step / 1e3, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(alg_bytes / t_step / 1e3 / HBM_PEAK_GBS, 4),
                      "traffic": traffic, "traffic_source": traffic_src, "algorithmic_bytes": alg_bytes},

@@ -49,9 +49,10 @@ using Stream = mlahip_stream_t;
 Stream stream_of(const Tensor& t) { return (Stream)c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 
 // Scratch memory comes from kernels._workspace, which keeps buffers per (device, stream, tag) and never frees one; what it
-// handed out is remembered here and asked for again only when it is too small.
+// handed out is remembered here and asked for again only when it is too small.  (Never destroyed: at exit the allocator that
+// would take the buffers back may be gone.)
 PyObject* g_workspace = nullptr;
-std::map<std::tuple<int, Stream, int>, Tensor> g_scratch;      // (guarded by the GIL, as the Python side is)
+auto& g_scratch = *new std::map<std::tuple<int, Stream, int>, Tensor>;      // (guarded by the GIL, as the Python side is)
 Tensor& scratch(const Tensor& like, Stream stream, int64_t bytes, int tag) {
   static const char* const names[] = {"decode", "topk", "absorb"};
   Tensor& t = g_scratch[{like.get_device(), stream, tag}];
