@@ -261,6 +261,11 @@ int mla_gather_paged_fp8_f16(const void* cache, int64_t page_stride_bytes, int64
  * mla.py:405-413, 566-571 up-projects the step's own latents in the model's dtype). */
 int mla_rows_f16(const void* kv_c, int64_t kv_c_stride, const void* k_pe, int64_t k_pe_stride, int64_t num_rows, void* out_c,
                  int64_t out_c_stride, void* out_pe, int64_t out_pe_stride, mlahip_stream_t stream);
+/* The same, and in the same launch the up-projection weight [weight_rows, 512] bf16 (rows weight_stride apart) as contiguous
+ * fp16 (weight and out_weight NULL, weight_rows 0: none). */
+int mla_rows_f16_weight(const void* kv_c, int64_t kv_c_stride, const void* k_pe, int64_t k_pe_stride, int64_t num_rows,
+                        void* out_c, int64_t out_c_stride, void* out_pe, int64_t out_pe_stride, const void* weight,
+                        int64_t weight_stride, int64_t weight_rows, void* out_weight, mlahip_stream_t stream);
 
 /* Query absorption of a decode step: out[t,n,:] = q_nope[t,n,:] . W_UK[n,:,:]  (q_nope [T,N,128], W_UK [N,128,512], out
  * [T,N,512], all bf16, strides in elements; attention/backends/mla.py:900-905). */

@@ -355,12 +355,12 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
         """Sparse attention of whole prompts over their own up-projected keys and values, with the picks as a mask
         (NPUDSAPrefillMetadata.over_up_projected); False, and nothing done, where the shapes do not allow it."""
         t, n = q.shape[0], self.num_heads
-        if pick is None or self._half_up_weight() is None or self.qk_nope_head_dim != 128 or self.v_head_dim != 128 or \
+        if pick is None or self._plain_up_weight() is None or self.qk_nope_head_dim != 128 or self.v_head_dim != 128 or \
                 q.dtype != torch.bfloat16 or q.stride(-1) != 1 or kv_c_normed.dtype != torch.bfloat16 or \
                 k_pe.dtype != torch.bfloat16 or kv_c_normed.stride(-1) != 1 or out.dtype != torch.bfloat16 or \
                 tuple(out.shape) != (t, n * 128) or out.stride(1) != 1 or out.stride(0) % 8 or out.data_ptr() % 16:
             return False
-        k_nope, pe, v = self._kv_up_rows(kv_c_normed, k_pe)
+        k_nope, pe, v, _ = self._kv_up_rows(kv_c_normed, k_pe)
         cu = prefill.query_start_loc.to(torch.int32).contiguous()
         K.prefill_varlen(q[..., :128], q[..., 128:], k_nope, pe, v, cu, cu, prefill.max_query_len, self.scale, True,
                          out.view(t, n, 128), pick=pick)
@@ -374,8 +374,9 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
         if output_scale is not None or output_block_scale is not None:
             raise NotImplementedError("fused output quantization is not yet supported for NPUDSAImpl")
         if attn_metadata is None:
-            _ = torch.empty((self.chunked_prefill_workspace_size, self.num_heads,
-                             self.qk_nope_head_dim + self.v_head_dim), device=k_c_normed.device, dtype=k_c_normed.dtype)
+            _ = (torch.empty((self.chunked_prefill_workspace_size, self.num_heads,
+                              self.qk_nope_head_dim + self.v_head_dim), device=k_c_normed.device, dtype=k_c_normed.dtype),
+                 self._half_up_weight())
             # the profile run sizes the KV cache: the split-KV scratch a real prefill will need (bounded by
             # SPARSE_WORKSPACE_CAP whatever the chunk size) is allocated now, so that it is counted
             # (for the split count the real steps will pick; scratch is kept per stream, so a runner that captures its graphs

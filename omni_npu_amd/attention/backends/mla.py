@@ -14,7 +14,6 @@ kernel leaves out the blocks between the sink and the window (prefill: kernels.p
 from __future__ import annotations
 
 import math
-import weakref
 from dataclasses import dataclass
 from typing import ClassVar, Optional, Tuple
 
@@ -200,8 +199,6 @@ class HalfUpProjection:
     # magnitude 2^-14 .. 65504 exactly; set prefill_kv_fp16 = False for a model whose keys or values can exceed that range.
     prefill_kv_fp16 = True
 
-    _half_w = None               # (weak reference to the up-projection weight, address and version) and its fp16 copy
-
     def _plain_up_weight(self) -> Optional[torch.Tensor]:
         """The up-projection weight [N*256, 512] if the prefill may make fp16 keys and values with it: plain, without bias."""
         w = getattr(self.kv_b_proj, "weight", None)
@@ -212,49 +209,44 @@ class HalfUpProjection:
         return w
 
     def _half_up_weight(self) -> Optional[torch.Tensor]:
-        """That weight in fp16, or None.  A bf16 weight is converted by the first prefill and again when it was replaced or
-        written to, not on every call."""
+        """That weight in fp16 as it is now, or None.  A bf16 weight is converted anew for every prefill, on the stream that
+        uses it, and nothing is kept: a write through ``.data`` or to an inference tensor leaves no trace that a kept copy
+        could follow, and a copy made on one stream would have to be waited for on every other."""
         w = self._plain_up_weight()
-        if w is None:
-            return None
-        if w.dtype == torch.float16:
-            return w
-        # (the reference dies with the weight: another one that comes to lie at its address is not taken for it)
-        key = (w.data_ptr(), w.device, 0 if w.is_inference() else w._version)
-        if self._half_w is None or self._half_w[0][0]() is not w or self._half_w[0][1:] != key:
-            half = w.to(torch.float16)
-            if w.is_cuda and torch.cuda.is_current_stream_capturing():
-                return half                                    # recorded, not computed: of no use to a later eager call
-            self._half_w = ((weakref.ref(w), *key), half)
-        return self._half_w[1]
-
-    def process_weights_after_loading(self, act_dtype: torch.dtype):
-        super().process_weights_after_loading(act_dtype)
-        self._half_w = None                                    # (weights reloaded through .data carry no new version)
+        return None if w is None else w.to(torch.float16)
 
     def _split_kv(self, kv: torch.Tensor):
         kv = kv.view(-1, self.num_heads, self.qk_nope_head_dim + self.v_head_dim)
         return kv[..., :self.qk_nope_head_dim], kv[..., self.qk_nope_head_dim:]
 
-    def _kv_up(self, kv_c: torch.Tensor, allow_fp16: bool = False):
+    def _kv_up(self, kv_c: torch.Tensor, allow_fp16: bool = False, w16: Optional[torch.Tensor] = None):
         """(k_nope [T,N,128], v [T,N,128]) of latent rows kv_c [T,512] (reference: ``self.kv_b_proj(kv_c_normed)[0]``,
-        mla.py:405-413, 566-571).  With ``allow_fp16`` both may come back as fp16."""
-        w = self._half_up_weight() if allow_fp16 and kv_c.dtype in (torch.bfloat16, torch.float16) else None
+        mla.py:405-413, 566-571).  With ``allow_fp16`` both may come back as fp16 (``w16``: the step's _half_up_weight, if the
+        caller has it)."""
+        w = None
+        if allow_fp16 and kv_c.dtype in (torch.bfloat16, torch.float16):
+            w = w16 if w16 is not None else self._half_up_weight()
         if w is not None and kv_c.shape[-1] == w.shape[1]:
             return self._split_kv(torch.matmul(kv_c.to(torch.float16), w.t()))
         kv = self.kv_b_proj(kv_c)
         return self._split_kv(kv[0] if isinstance(kv, tuple) else kv)
 
     def _kv_up_rows(self, kv_c: torch.Tensor, k_pe: torch.Tensor):
-        """(k_nope, k_pe [T,64], v) of a step's own rows as the prefill kernel takes them: all fp16 where the weight allows
-        it (latent and rope rows converted in one launch), else all in the dtype of the up-projection's result."""
-        w = self._half_up_weight()
+        """(k_nope, k_pe [T,64], v, w16) of a step's own rows as the prefill kernel takes them: all fp16 where the weight allows
+        it, else all in the dtype of the up-projection's result.  w16: the weight in fp16, for the step's context rows (None: the
+        module was called).  Latents, rope rows and weight are converted in one launch: torch's conversion of the weight of 64
+        heads takes 24 us, as long as the up-projection of 1000 rows."""
+        w = self._plain_up_weight()
         if w is not None and kv_c.dtype == torch.bfloat16 and k_pe.dtype == torch.bfloat16:
-            c16, pe16 = K.rows_f16(kv_c, k_pe)
-            k_nope, v = self._split_kv(torch.matmul(c16, w.t()))
-            return k_nope, pe16, v
-        k_nope, v = self._kv_up(kv_c, allow_fp16=True)
-        return k_nope, k_pe.reshape(k_pe.shape[0], -1).to(k_nope.dtype), v
+            if w.dtype == torch.bfloat16 and w.is_contiguous() and w.data_ptr() % 16 == 0:
+                c16, pe16, w16 = K.rows_f16(kv_c, k_pe, w)
+            else:
+                (c16, pe16), w16 = K.rows_f16(kv_c, k_pe), w.to(torch.float16)
+            k_nope, v = self._split_kv(torch.matmul(c16, w16.t()))
+            return k_nope, pe16, v, w16
+        w16 = self._half_up_weight()
+        k_nope, v = self._kv_up(kv_c, allow_fp16=True, w16=w16)
+        return k_nope, k_pe.reshape(k_pe.shape[0], -1).to(k_nope.dtype), v, w16
 
 
 class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
@@ -306,7 +298,8 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
         return out2.transpose(0, 1).contiguous().view(-1, self.num_heads * self.v_head_dim)
 
     # ---- prefill ----
-    def _compute_prefill_context(self, q_nope, q_pe, kv_c_cache, k_pe_cache, attn_metadata, k_scale):
+    def _compute_prefill_context(self, q_nope, q_pe, kv_c_cache, k_pe_cache, attn_metadata, k_scale,
+                                 w16: Optional[torch.Tensor] = None):
         """Chunked context: gather -> up-project -> unmasked attention with LSE (reference mla.py:377-450).  The reference
         merges every chunk's result into a running one (merge_attn_states); here a chunk's launch continues from the
         running result, so the merge is part of the attention kernel and there is no merge launch."""
@@ -316,20 +309,21 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
         t, n = q_nope.shape[0], self.num_heads
         cu_q = prefill.query_start_loc.to(torch.int32).contiguous()
         output = output_lse = None
+        # (with an fp16 up-projection the rows are gathered as fp16 straight away, into the same bytes)
+        if w16 is None and cc.workspace.dtype == torch.bfloat16:
+            w16 = self._half_up_weight()
+        rows = cc.workspace if w16 is None or cc.workspace.dtype != torch.bfloat16 else cc.workspace.view(torch.float16)
         for i in range(len(cc.seq_tot)):
             toks = int(cc.seq_tot[i])
             if toks == 0:
                 continue
-            # (with an fp16 up-projection the rows are gathered as fp16 straight away, into the same bytes)
-            w16 = self._half_up_weight() if cc.workspace.dtype == torch.bfloat16 else None
-            rows = (cc.workspace if w16 is None else cc.workspace.view(torch.float16))
             ops.gather_and_maybe_dequant_cache(src_cache=(kv_c_cache,) if k_pe_cache is None else (kv_c_cache, k_pe_cache),
                                                dst=rows,
                                                block_table=prefill.block_table, cu_seq_lens=cc.cu_seq_lens[i],
                                                batch_size=attn_metadata.num_prefills, kv_cache_dtype=self.kv_cache_dtype,
                                                scale=k_scale, seq_starts=cc.starts[i], total_rows=toks)
             kv_c_normed, k_pe = rows[:toks, :self.kv_lora_rank], rows[:toks, self.kv_lora_rank:]
-            k_nope, v = self._kv_up(kv_c_normed, allow_fp16=True)
+            k_nope, v = self._kv_up(kv_c_normed, allow_fp16=True, w16=w16)
             k_pe = k_pe.to(k_nope.dtype)
             # running results stay fp32: each bf16 rounding in between would add 2^-10 of mean relative error to the
             # layer's output
@@ -354,13 +348,13 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
         t, n = q.shape[0], self.num_heads
         has_context = prefill.chunked_context is not None
         q_nope, q_pe = q[..., :self.qk_nope_head_dim], q[..., self.qk_nope_head_dim:]
-        k_nope, k_pe, v = self._kv_up_rows(kv_c_normed, k_pe)
+        k_nope, k_pe, v, w16 = self._kv_up_rows(kv_c_normed, k_pe)
         cu_q = prefill.query_start_loc.to(torch.int32).contiguous()
         ctx_out = ctx_lse = None
         if has_context:
             # (the fp8 cache is one tensor whose rows hold latent, scales and rope; the gather dequantises it)
             ctx_out, ctx_lse = self._compute_prefill_context(q_nope, q_pe, kv_cache[0],
-                                                             None if self.fp8_cache else kv_cache[1], attn_metadata, k_scale)
+                                                             None if self.fp8_cache else kv_cache[1], attn_metadata, k_scale, w16)
         if out is not None and out.dtype == torch.bfloat16 and out.dim() == 2 and out.shape == (t, n * self.v_head_dim) and \
                 out.stride(1) == 1 and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
             output = out.view(t, n, self.v_head_dim)
@@ -496,9 +490,11 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
             raise NotImplementedError("fused output quantization is not yet supported for NPUMLAImpl")
 
         if attn_metadata is None:
-            # profile run: reserve the worst-case up-projection scratch, zero the output (reference mla.py:825-842)
-            _ = torch.empty((self.chunked_prefill_workspace_size, self.num_heads,
-                             self.qk_nope_head_dim + self.v_head_dim), device=k_c_normed.device, dtype=k_c_normed.dtype)
+            # profile run: reserve the worst-case up-projection scratch and, beside it, the fp16 weight that a prefill makes its
+            # keys and values with; zero the output (reference mla.py:825-842)
+            _ = (torch.empty((self.chunked_prefill_workspace_size, self.num_heads,
+                              self.qk_nope_head_dim + self.v_head_dim), device=k_c_normed.device, dtype=k_c_normed.dtype),
+                 self._half_up_weight())
             return output.fill_(0)
 
         num_actual_toks = attn_metadata.num_actual_tokens

@@ -50,11 +50,26 @@ __global__ __launch_bounds__(256) void gather_paged_kernel(const char* nope, int
 }
 
 // Plain rows [T, 512] and [T, 64] from bf16 to fp16, a wavefront per row (the step's own latents, which the prefill
-// up-projects and attends over in fp16).
+// up-projects and attends over in fp16).  In front of them w_blocks workgroups convert the rows [W, 512] of the up-projection
+// weight, four per wavefront, so that its 16-byte loads are in flight together: HBM bounds it, and it shares the launch.
+struct RowsF16Weight { const char* w; int64_t st; char* out; int64_t rows; };
+constexpr int kWeightRows = 4;
 __global__ __launch_bounds__(256) void rows_f16_kernel(const char* c, int64_t c_st, const char* r, int64_t r_st, char* oc,
-                                                       int64_t oc_st, char* orr, int64_t or_st, int64_t rows) {
+                                                       int64_t oc_st, char* orr, int64_t or_st, int64_t rows,
+                                                       const RowsF16Weight w, unsigned w_blocks) {
   const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (blockIdx.x < w_blocks) {
+    const int64_t first = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * kWeightRows;
+    u32x4 v[kWeightRows];
+#pragma unroll
+    for (int i = 0; i < kWeightRows; i++)
+      if (first + i < w.rows) v[i] = *(const u32x4*)(w.w + (first + i) * w.st + lane * 16);
+#pragma unroll
+    for (int i = 0; i < kWeightRows; i++)
+      if (first + i < w.rows) *(u32x4*)(w.out + (first + i) * (kDNope * 2) + lane * 16) = as_dst<true>(v[i]);
+    return;
+  }
+  const int64_t row = (int64_t)(blockIdx.x - w_blocks) * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
   *(u32x4*)(oc + row * oc_st + lane * 16) = as_dst<true>(*(const u32x4*)(c + row * c_st + lane * 16));
   if (lane < 8) *(u32x4*)(orr + row * or_st + lane * 16) = as_dst<true>(*(const u32x4*)(r + row * r_st + lane * 16));
@@ -307,16 +322,31 @@ extern "C" int mla_merge_states(const void* prefix_out, int64_t po_stride_t, int
   return check_launch("mla_merge_states");
 }
 
-extern "C" int mla_rows_f16(const void* kv_c, int64_t kv_c_stride, const void* k_pe, int64_t k_pe_stride, int64_t num_rows,
-                            void* out_c, int64_t out_c_stride, void* out_pe, int64_t out_pe_stride, hipStream_t stream) {
+// weight [weight_rows, 512] bf16 with its row stride, out_weight contiguous fp16; NULL and 0 for none.
+extern "C" int mla_rows_f16_weight(const void* kv_c, int64_t kv_c_stride, const void* k_pe, int64_t k_pe_stride, int64_t num_rows,
+                                   void* out_c, int64_t out_c_stride, void* out_pe, int64_t out_pe_stride, const void* weight,
+                                   int64_t weight_stride, int64_t weight_rows, void* out_weight, hipStream_t stream) {
   MLA_REQUIRE(kv_c && k_pe && out_c && out_pe, MLA_ERR_NULL, "mla_rows_f16: null pointer argument");
   MLA_REQUIRE(num_rows >= 0 && num_rows < (1ll << 32) && kv_c_stride % 8 == 0 && k_pe_stride % 8 == 0 && out_c_stride % 8 == 0 &&
                   out_pe_stride % 8 == 0 && (uintptr_t)kv_c % 16 == 0 && (uintptr_t)k_pe % 16 == 0 &&
                   (uintptr_t)out_c % 16 == 0 && (uintptr_t)out_pe % 16 == 0,
               MLA_ERR_SHAPE, "mla_rows_f16: num_rows=%lld; rows must be 16-byte aligned", (long long)num_rows);
-  if (num_rows == 0) return MLA_OK;
-  hipLaunchKernelGGL(rows_f16_kernel, dim3((unsigned)((num_rows + 3) / 4)), dim3(256), 0, stream, (const char*)kv_c,
-                     kv_c_stride * 2, (const char*)k_pe, k_pe_stride * 2, (char*)out_c, out_c_stride * 2, (char*)out_pe,
-                     out_pe_stride * 2, num_rows);
+  MLA_REQUIRE((weight == nullptr) == (out_weight == nullptr) && (weight != nullptr || weight_rows == 0), MLA_ERR_NULL,
+              "mla_rows_f16: the weight, its rows and its result go together");
+  MLA_REQUIRE(weight_rows >= 0 && weight_rows < (1ll << 32) && weight_stride % 8 == 0 && (uintptr_t)weight % 16 == 0 &&
+                  (uintptr_t)out_weight % 16 == 0,
+              MLA_ERR_SHAPE, "mla_rows_f16: weight_rows=%lld; rows must be 16-byte aligned", (long long)weight_rows);
+  const unsigned w_blocks = (unsigned)((weight_rows + 4 * kWeightRows - 1) / (4 * kWeightRows));
+  const unsigned blocks = w_blocks + (unsigned)((num_rows + 3) / 4);
+  if (blocks == 0) return MLA_OK;
+  const RowsF16Weight w = {(const char*)weight, weight_stride * 2, (char*)out_weight, weight_rows};
+  hipLaunchKernelGGL(rows_f16_kernel, dim3(blocks), dim3(256), 0, stream, (const char*)kv_c, kv_c_stride * 2, (const char*)k_pe,
+                     k_pe_stride * 2, (char*)out_c, out_c_stride * 2, (char*)out_pe, out_pe_stride * 2, num_rows, w, w_blocks);
   return check_launch("rows_f16_kernel");
+}
+
+extern "C" int mla_rows_f16(const void* kv_c, int64_t kv_c_stride, const void* k_pe, int64_t k_pe_stride, int64_t num_rows,
+                            void* out_c, int64_t out_c_stride, void* out_pe, int64_t out_pe_stride, hipStream_t stream) {
+  return mla_rows_f16_weight(kv_c, kv_c_stride, k_pe, k_pe_stride, num_rows, out_c, out_c_stride, out_pe, out_pe_stride, nullptr,
+                             0, 0, nullptr, stream);
 }

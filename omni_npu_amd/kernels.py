@@ -298,21 +298,26 @@ def gather_paged_fp8(cache: torch.Tensor, dst: torch.Tensor, block_table: torch.
     _lib.check(rc, name)
 
 
-def rows_f16(kv_c: torch.Tensor, k_pe: torch.Tensor):
-    """(kv_c [T,512], k_pe [T,64] or [T,1,64]) bf16 -> the same rows as contiguous fp16 [T,512], [T,64], in one launch."""
-    _need_cuda(kv_c, k_pe)
+def rows_f16(kv_c: torch.Tensor, k_pe: torch.Tensor, weight: Optional[torch.Tensor] = None):
+    """(kv_c [T,512], k_pe [T,64] or [T,1,64]) bf16 -> the same rows as contiguous fp16 [T,512], [T,64], in one launch; with
+    ``weight`` (bf16 [W,512], the up-projection's) that as contiguous fp16 too, as a third result of the same launch."""
+    _need_cuda(kv_c, k_pe, weight)
     k_pe = k_pe.reshape(k_pe.shape[0], -1)
     t = kv_c.shape[0]
     if kv_c.shape != (t, D_NOPE) or k_pe.shape != (t, D_ROPE) or kv_c.dtype != torch.bfloat16 or k_pe.dtype != torch.bfloat16 or \
             kv_c.stride(-1) != 1 or k_pe.stride(-1) != 1:
         raise ValueError("rows_f16: bf16 kv_c [T,512] and k_pe [T,64] with contiguous last dims")
+    if weight is not None and (weight.dtype != torch.bfloat16 or weight.dim() != 2 or weight.shape[1] != D_NOPE or weight.stride(1) != 1):
+        raise ValueError("rows_f16: the weight must be bf16 [W,512] with a contiguous last dim")
     c = torch.empty(t, D_NOPE, dtype=torch.float16, device=kv_c.device)
     r = torch.empty(t, D_ROPE, dtype=torch.float16, device=kv_c.device)
+    w16 = torch.empty(weight.shape, dtype=torch.float16, device=kv_c.device) if weight is not None else None
     if t:
-        rc = _lib.load().mla_rows_f16(kv_c.data_ptr(), kv_c.stride(0), k_pe.data_ptr(), k_pe.stride(0), t, c.data_ptr(), D_NOPE,
-                                      r.data_ptr(), D_ROPE, _stream(kv_c))
+        w_args = (weight.data_ptr(), weight.stride(0), weight.shape[0], w16.data_ptr()) if weight is not None else (None, 0, 0, None)
+        rc = _lib.load().mla_rows_f16_weight(kv_c.data_ptr(), kv_c.stride(0), k_pe.data_ptr(), k_pe.stride(0), t, c.data_ptr(),
+                                             D_NOPE, r.data_ptr(), D_ROPE, *w_args, _stream(kv_c))
         _lib.check(rc, "mla_rows_f16")
-    return c, r
+    return (c, r) if weight is None else (c, r, w16)
 
 
 # Tokens up to which the queries of a step are absorbed by this library's kernel; beyond, the work is a plain GEMM

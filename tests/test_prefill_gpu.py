@@ -336,6 +336,17 @@ def test_scores_that_climb_tile_by_tile_raise_the_reference(dev, half, sq, sk, c
         assert torch.allclose(lse.cpu(), ref_lse, atol=2e-2, rtol=1e-3)
 
 
+@pytest.mark.parametrize("rows,w_rows,stride", [(1, 256, 512), (4, 15, 512), (5, 17, 520), (1027, 4096, 512)])
+def test_rows_f16_takes_the_weight_along(dev, rows, w_rows, stride):
+    """Rows and weight of one launch, whole and partial workgroups of weight rows, strided ones: torch's bits."""
+    from omni_npu_amd import kernels as K
+    g = torch.Generator().manual_seed(w_rows)
+    c, r = torch.randn(rows, 512, generator=g).bfloat16().to(dev), torch.randn(rows, 64, generator=g).bfloat16().to(dev)
+    w = (torch.randn(w_rows, stride, generator=g) * torch.exp2(torch.randint(-30, 18, (w_rows, 1), generator=g).float())).bfloat16().to(dev)[:, :512]
+    c16, r16, w16 = K.rows_f16(c, r, w)
+    assert torch.equal(c16, c.half()) and torch.equal(r16, r.half()) and torch.equal(w16, w.half()) and w16.is_contiguous()
+
+
 @pytest.mark.parametrize("rows", [1, 4, 5, 1027])
 def test_rows_f16_and_fp16_gathers_round_like_torch(dev, rows):
     """bf16 -> fp16 of the step's rows and of both gathers: the bits of torch's conversion of the bf16 result, normal,
