@@ -43,6 +43,11 @@ def indexer_cache_views(index_cache: torch.Tensor):
     return k8, ks
 
 
+def _mask_words(stride: int) -> int:
+    """32-bit words of a row of pick bits over ``stride`` scores: whole 64-key tiles."""
+    return stride // 64 * 2 + 2
+
+
 class NPUDSABackend(MLACommonBackend):
     @staticmethod
     def get_name() -> str:
@@ -178,8 +183,8 @@ class LightningIndexer:
         self.counts_buffer = torch.zeros((max_tokens,), dtype=torch.int32, device=device)
         self._rows_meta = None       # the metadata object the row buffers were filled for
         # Up to how many visible pairs per pick the attention behind this selection wants a step's prompts as bits over their
-        # own keys instead of cache rows (NPUDSAImpl says so once its weights are loaded); the bits, and the metadata object
-        # they were made for
+        # own keys instead of cache rows (NPUDSAImpl says so once its weights are loaded); the bits, until the attention has
+        # used them (drop_mask), and the metadata object they were made for
         self.masked_pairs_per_pick = 0.0
         self._mask, self._mask_meta = None, None
         self._logits = None
@@ -224,7 +229,7 @@ class LightningIndexer:
                 K.indexer_scores(q8[sl], w[sl], k8, ks, meta.block_table, lens, lg, q_len=q_len, q_scale=qs[sl],
                                  query_start_loc=qsl, max_seq_len=max_len, skip_up_to=self.topk_tokens)
             if masked:
-                self._mask = torch.empty(ntok, stride // 64 * 2 + 2, dtype=torch.int32, device=q.device)
+                self._mask = torch.empty(ntok, _mask_words(stride), dtype=torch.int32, device=q.device)
                 self._mask_meta = attn_metadata
                 K.topk(lg, lens, self.topk_tokens, out[sl], q_len=q_len, query_start_loc=qsl, mask=self._mask)
             else:
@@ -262,8 +267,20 @@ class LightningIndexer:
 
     def mask_for(self, attn_metadata):
         """The picks of the step's prompt tokens as bits [T, W] (kernels.topk's mask) if the last selection made them for this
-        very metadata object, else None.  The row buffers hold the step's decode tokens only then."""
-        return self._mask if attn_metadata is not None and self._mask_meta is attn_metadata else None
+        very metadata object and the attention has not used them yet, else None."""
+        return self._mask if self.masked_prompts(attn_metadata) else None
+
+    def masked_prompts(self, attn_metadata) -> bool:
+        """Whether the last selection ran for this very metadata object and made its prompts' picks as bits: the row buffers
+        then hold the step's decode tokens only."""
+        return attn_metadata is not None and self._mask_meta is attn_metadata
+
+    def drop_mask(self) -> None:
+        """The attention has queued its use of the bits: their memory (a bit per pair of a prompt, 8 MB for 8k tokens) goes back
+        behind it instead of staying with every layer until that layer's next step."""
+        if self._mask is not None and self._mask.is_cuda:
+            self._mask.record_stream(torch.cuda.current_stream(self._mask.device))
+        self._mask = None
 
     def rows_for(self, attn_metadata):
         """(cache rows [max_tokens, k], counts [max_tokens]) of the picks if the last selection ran for this very metadata
@@ -374,15 +391,18 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
         if output_scale is not None or output_block_scale is not None:
             raise NotImplementedError("fused output quantization is not yet supported for NPUDSAImpl")
         if attn_metadata is None:
+            # (beside the up-projection scratch what a step of masked prompts makes and drops again: the fp16 weight, and the
+            # picks of one prompt of all the step's tokens as bits)
+            toks = max(int(k_c_normed.shape[0]), 1)
             _ = (torch.empty((self.chunked_prefill_workspace_size, self.num_heads,
                               self.qk_nope_head_dim + self.v_head_dim), device=k_c_normed.device, dtype=k_c_normed.dtype),
-                 self._half_up_weight())
+                 self._half_up_weight(),
+                 torch.empty(toks, _mask_words(K.indexer_logits_stride(toks)), dtype=torch.int32, device=k_c_normed.device))
             # the profile run sizes the KV cache: the split-KV scratch a real prefill will need (bounded by
             # SPARSE_WORKSPACE_CAP whatever the chunk size) is allocated now, so that it is counted
             # (for the split count the real steps will pick; scratch is kept per stream, so a runner that captures its graphs
             # on another stream pays this once more there: at most SPARSE_WORKSPACE_CAP per stream that runs steps)
             if k_c_normed.is_cuda:
-                toks = max(int(k_c_normed.shape[0]), 1)
                 k_sel = int(self.indexer.topk_indices_buffer.shape[-1]) if self.indexer is not None else 2048
                 splits = K.launch_splits(toks, 1, self.num_heads, k_sel)
                 need = K._lib.load().mla_decode_workspace_bytes(min(toks, 32768), 1, self.num_heads, splits)
@@ -405,8 +425,8 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
         has_prefill = attn_metadata.num_prefills > 0
         ndt = attn_metadata.num_decode_tokens
         written = _caller_wrote_cache(self, attn_metadata, num_actual_toks)
-        rows_for = getattr(self.indexer, "rows_for", None)
-        rc = rows_for(attn_metadata) if rows_for is not None else None
+        select = getattr(self.indexer, "select", self.indexer)     # (what was offered masked prompts, see there)
+        rc = select.rows_for(attn_metadata) if hasattr(select, "rows_for") else None
         native = None
         if has_decode and not has_prefill and rc is not None:
             native = lambda *new: _host.load().sparse_decode(q, k_nope, k_rope, rc[0], rc[1], self.W_UK_T, self.W_UV, self.scale,
@@ -418,12 +438,13 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
             return output_padded
         topk = self.indexer.topk_indices_buffer
         part = lambda a, b: None if rc is None else (rc[0][a:b], rc[1][a:b])
+        # (a selection that made bits has left no rows for the prompts, also after the bits are gone)
+        masked = hasattr(select, "masked_prompts") and select.masked_prompts(attn_metadata)
 
         if has_prefill:
             p = attn_metadata.prefill
             assert p is not None
-            mask_for = getattr(self.indexer, "mask_for", None)
-            pick = mask_for(attn_metadata) if mask_for is not None else None
+            pick = select.mask_for(attn_metadata) if masked else None
             if not self._forward_prompts(q[ndt:], k_c_normed[ndt:num_actual_toks], k_pe[ndt:num_actual_toks], p, pick,
                                          output[ndt:]):
                 q_nope, q_pe = self._absorb_prolog(q[ndt:])
@@ -431,9 +452,11 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
                 attn_out = self._apply_sparse_attention(q_nope, q_pe, kv_cache, p, p.kv_lens, p.max_query_len,
                                                         p.query_start_loc.to(torch.int32).contiguous(),
                                                         topk[ndt:num_actual_toks], proj_out=fused,
-                                                        rows_counts=None if pick is not None else part(ndt, num_actual_toks))
+                                                        rows_counts=None if masked else part(ndt, num_actual_toks))
                 if fused is None:
                     self._v_up_proj(attn_out, out=output[ndt:])
+            if pick is not None:
+                select.drop_mask()
         if has_decode:
             d = attn_metadata.decode
             assert d is not None

@@ -71,10 +71,13 @@ class NPUDeepseekSparseAttention(torch.nn.Module):
         K.kv_rmsnorm_rope_cache(latent, self.kv_a_layernorm.weight, cos, sin, meta.slot_mapping, kv_cache[0], kv_cache[1],
                                 eps=self._eps(), kv_a_out=kv_a, k_pe_out=k_pe, q_rope=q_pe)
         topk_indices = self.indexer.forward_tables(hidden_states, q_lora, cos, sin, meta, kv_cache)[0]
-        pick = select.mask_for(meta) if hasattr(select, "mask_for") else None
+        masked = hasattr(select, "masked_prompts") and select.masked_prompts(meta)
         if meta.prefill is not None:
             p = meta.prefill
-            if impl._forward_prompts(q, kv_a, k_pe, p, pick, out):
+            done = masked and impl._forward_prompts(q, kv_a, k_pe, p, select.mask_for(meta), out)
+            if masked:
+                select.drop_mask()
+            if done:
                 return self.o_proj(out)[0]
             part, lens, q_len, qsl = p, p.kv_lens, p.max_query_len, p.query_start_loc.to(torch.int32).contiguous()
         else:
@@ -82,7 +85,7 @@ class NPUDeepseekSparseAttention(torch.nn.Module):
             part, lens, q_len, qsl = d, d.seq_lens, d.q_len, d.query_start_loc
         ql_nope = K.absorb(q[..., :self.qk_nope_head_dim], impl.W_UK_T)
         fused = out if impl._fusable_w_uv(out) else None
-        rc = select.rows_for(meta) if pick is None and hasattr(select, "rows_for") else None
+        rc = select.rows_for(meta) if not masked and hasattr(select, "rows_for") else None
         attn_out = impl._apply_sparse_attention(ql_nope, q_pe, kv_cache, part, lens, q_len, qsl, topk_indices[:t],
                                                 proj_out=fused, rows_counts=None if rc is None else (rc[0][:t], rc[1][:t]))
         if fused is None:

@@ -364,6 +364,45 @@ def test_dsa_prompts_attend_over_their_own_keys_with_the_picks_as_a_mask(dev, q_
     attn_close(got[0][1], got[1][1], 3e-2, 4e-3 + 4e-3)        # (the latent form also rounds absorbed queries and outputs to bf16)
 
 
+@pytest.mark.parametrize("q_lens", [[300], [1, 1, 129, 70, 300]])
+def test_pick_bits_go_with_the_step_and_a_second_forward_still_stands(dev, q_lens):
+    """The bits of a selection are given back once the attention has queued its use of them, on whatever stream that ran; a
+    second forward of the same step finds no bits, and no rows of its prompts either, and translates the picks itself."""
+    g = torch.Generator().manual_seed(sum(q_lens))
+    n, topk = 16, 64
+    seq_lens = [q if q > 1 else 400 for q in q_lens]
+    common = _common(q_lens, seq_lens)
+    t = common.num_actual_tokens
+    nblk = int(common.block_table_tensor.max()) + 1
+    common.slot_mapping = torch.cat([O.slots_for(common.block_table_tensor, b, s - ql, s)
+                                     for b, (ql, s) in enumerate(zip(q_lens, seq_lens))])
+    raw = torch.randn(nblk * 128 * 704, generator=g).bfloat16().to(dev).view(torch.uint8)
+    kv_cache = dsa.NPUDSABackend.reshape_kv_cache(raw, nblk, 128, 1, 704, dtype=torch.bfloat16)
+    k8v, ksv = dsa.indexer_cache_views(kv_cache[2])
+    k8_ref, ks_ref = O.fp8_quant_token(torch.randn(nblk, 128, 128, generator=g))
+    k8v.copy_(k8_ref.view(torch.uint8)); ksv.copy_(ks_ref)
+    indexer = dsa.LightningIndexer(topk, max_tokens=t, device=dev)
+    indexer.rows_buffer.fill_(nblk * 128 - 1)                  # (what earlier steps may have left where prompts have no rows)
+    indexer.counts_buffer.fill_(1)
+    # the selection also inside an indexer module, as the model owns it
+    impl, w = _mk_impl(dsa.NPUDSAImpl, n, dev, indexer=SimpleNamespace(select=indexer, topk_indices_buffer=indexer.topk_indices_buffer))
+    impl.kv_b_proj = _PlainLinear(w, dev)
+    impl.process_weights_after_loading(torch.bfloat16)
+    meta = dsa.NPUDSAMetadataBuilder(V.AttentionSpec(128, 1, 704, torch.bfloat16), ["l"], _cfg(cap=1), dev).build(0, _to(common, dev))
+    rand = lambda *s: torch.randn(*s, generator=g).bfloat16().to(dev)
+    a = [rand(t, n, 192), rand(t, 512), rand(t, 1, 64)]
+    indexer(rand(t, 64, 128), rand(t, 128), rand(t, 64), kv_cache, meta)
+    assert indexer.mask_for(meta) is not None
+    outs = [torch.zeros(t, n * 128, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    torch.cuda.synchronize(dev)
+    with torch.cuda.stream(torch.cuda.Stream(dev)):
+        for out in outs:
+            impl.forward(None, *a, kv_cache, meta, output=out)
+            assert indexer.mask_for(meta) is None and indexer.masked_prompts(meta)
+    torch.cuda.synchronize(dev)
+    attn_close(outs[0], outs[1], 3e-2, 4e-3 + 4e-3)            # (the bar of two bf16 results, as above)
+
+
 class _NoNative:
     """The native host side as it answers for arguments it does not know."""
     def __getattr__(self, name):
