@@ -15,9 +15,10 @@
 // What bounds it: the socket's power cap.  On the 4 x 2048 over 16k, 128-head context launch the matrix pipe is busy 61 %
 // of the cycles and the clock settles at 1.67 GHz at 1350 W, so what pays is fewer instructions per score and what lets
 // the clock settle lower:
-//  * a tile costs one fused multiply-add, one exponential, half a conversion and half a v_dot2 (the sum) per score.  A
+//  * a tile costs one fused multiply-add, one exponential, half a conversion and one add (the sum, of probabilities before
+//    they are rounded; v_dot2 over the rounded pairs would be half an instruction less and 2 % of a long chunk) per score.  A
 //    row's reference is its first tile's maximum and is raised only where a probability outgrows it by 2^13: no maximum
-//    and no rescaling in the steady state (136 -> 76 instructions per wavefront and 32 keys, 11 970 -> 11 110 us);
+//    and no rescaling in the steady state (136 -> 84 instructions per wavefront and 32 keys);
 //  * both 32-key blocks of a tile are scored before the first exponential, at a raised wave priority (s_setprio), so the
 //    two wavefronts of a SIMD fall out of step and one's vector work runs beside the other's MFMAs (11 110 -> 10 350 us =
 //    1.06 PFLOP/s; causal 4 x 2048 994 -> 860 us).
@@ -369,16 +370,19 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
           else s[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[kk], s[tb], 0, 0, 0);
         }
       };
-      // probabilities against the row's reference as fp16 pairs, and the sum of what was rounded (v_dot2 adds a pair)
+      // probabilities against the row's reference as fp16 pairs, and the sum of what they were before they were rounded
       auto probs = [&](int tb, float sum) -> float {
         const float neg = -m_run;
+        float odd = 0.f;                                       // (two chains of adds: 4 x 2048 over 16k 14 606 -> 14 515 us per layer)
 #pragma unroll
         for (int r = 0; r < 8; r++) {
-          pb[tb][r] = __builtin_convertvector((f32x2{fast_exp2(__builtin_fmaf(s[tb][2 * r], p.scale_log2, neg)),
-                                                     fast_exp2(__builtin_fmaf(s[tb][2 * r + 1], p.scale_log2, neg))}), f16x2);
-          sum = __builtin_amdgcn_fdot2(pb[tb][r], f16x2{(_Float16)1.f, (_Float16)1.f}, sum, false);
+          const f32x2 e = {fast_exp2(__builtin_fmaf(s[tb][2 * r], p.scale_log2, neg)),
+                           fast_exp2(__builtin_fmaf(s[tb][2 * r + 1], p.scale_log2, neg))};
+          pb[tb][r] = __builtin_convertvector(e, f16x2);
+          sum += e[0];
+          odd = r == 0 ? e[1] : odd + e[1];
         }
-        return sum;
+        return sum + odd;
       };
       __builtin_amdgcn_s_setprio(1);
       scores(0);

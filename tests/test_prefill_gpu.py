@@ -400,3 +400,27 @@ def test_prefill_over_picked_keys(dev, q_lens, density):
         ref_lse[a:e] = s.logsumexp(-1).t()
     attn_close(out, ref, 2e-2, 2e-3)
     assert torch.allclose(lse.cpu(), ref_lse, atol=2e-2, rtol=1e-3)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp16", "picked"])
+def test_the_denominator_adds_probabilities_before_they_are_rounded(dev, kind):
+    """log-sum-exp against 64 bits where nothing but the kernel's fp32 arithmetic errs: scores are sums of four products of
+    eighths of at most 1, exact in fp32, times a power of two.  What is left, for up to 16 keys: the scaled score (2.9 in log2,
+    two roundings: 2.4e-7 of a probability), the exponential (1.2e-7), the sum (at most 16 * 2^-24 = 1e-6), logarithm and
+    result (two roundings of at most 4: 5e-7).  Probabilities rounded to fp16 first would be off by up to 1.2e-4."""
+    from omni_npu_amd import kernels as K
+    g = torch.Generator().manual_seed(3)
+    n, t, scale = 8, 16, 0.5
+    eighths = lambda *s: (torch.randint(-8, 9, s, generator=g).float() / 8)
+    q, k = torch.zeros(t, n, 192), torch.zeros(t, n, 128)
+    q[..., :4], k[..., :4] = eighths(t, n, 4), eighths(t, n, 4)
+    dt = torch.bfloat16 if kind == "bf16" else torch.float16
+    v = torch.randn(t, n, 128, generator=g)
+    cu = torch.tensor([0, t], dtype=torch.int32, device=dev)
+    out, lse = torch.empty(t, n, 128, dtype=torch.bfloat16, device=dev), torch.empty(t, n, device=dev)
+    qd = q.bfloat16().to(dev)
+    K.prefill_varlen(qd[..., :128], qd[..., 128:], k.to(dev, dt), torch.zeros(t, 64, dtype=dt, device=dev), v.to(dev, dt), cu, cu, t, scale,
+                     True, out, lse, pick=torch.full((t, 2), -1, dtype=torch.int32, device=dev) if kind == "picked" else None)
+    s = torch.einsum("inp,jnp->nij", q[..., :128].double(), k.double()) * scale
+    ref = s.masked_fill(~torch.ones(t, t).tril().bool(), float("-inf")).logsumexp(-1).t()
+    assert (lse.cpu().double() - ref).abs().max() <= 2e-6
