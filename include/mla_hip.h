@@ -330,8 +330,7 @@ int mla_prefill_varlen_continue(const void* q_nope, int64_t qn_stride_t, int64_t
 
 /* mla_prefill_varlen over a selection of keys: bit j of pick[t] (32-bit words, rows pick_stride words apart, pick_words of
  * them valid, whole 64-key tiles) says whether query token t attends over key j of its sequence, within what causal
- * allows.  out_dtype must carry MLA_PREFILL_KV_F16.  The sparse attention of attention/backends/dsa.py:259-291 over the
- * up-projected keys and values of a prompt. */
+ * allows.  The sparse attention of attention/backends/dsa.py:259-291 over the up-projected keys and values of a prompt. */
 int mla_prefill_varlen_pick(const void* q_nope, int64_t qn_stride_t, int64_t qn_stride_h, const void* q_pe, int64_t qp_stride_t,
                             int64_t qp_stride_h, const void* k_nope, int64_t kn_stride_t, int64_t kn_stride_h, const void* k_pe,
                             int64_t kp_stride_t, const void* v, int64_t v_stride_t, int64_t v_stride_h, const int32_t* cu_q,

@@ -293,6 +293,10 @@ class LightningIndexer:
 class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
     can_return_lse_for_decode: bool = False
     cache_written_for = None     # see NPUMLAImpl.cache_written_for
+    # Prompts attend in the types that a gather of the cache would: bf16 latents, rope rows, queries and keys.  True makes keys and
+    # values in fp16 (11 bits instead of 8, and the kernel converts no value tile) for a model whose latents, rope rows, queries,
+    # keys and values stay between 2^-14 and 65504.
+    prefill_kv_fp16 = False
 
     def __init__(self, num_heads: int, head_size: int, scale: float, num_kv_heads: int, alibi_slopes: Optional[list],
                  sliding_window: Optional[int], kv_cache_dtype: str, logits_soft_cap: Optional[float], attn_type: str,
@@ -371,11 +375,13 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
     def _forward_prompts(self, q, kv_c_normed, k_pe, prefill, pick, out: torch.Tensor) -> bool:
         """Sparse attention of whole prompts over their own up-projected keys and values, with the picks as a mask
         (NPUDSAPrefillMetadata.over_up_projected); False, and nothing done, where the shapes do not allow it."""
-        t, n = q.shape[0], self.num_heads
-        if pick is None or self._plain_up_weight() is None or self.qk_nope_head_dim != 128 or self.v_head_dim != 128 or \
-                q.dtype != torch.bfloat16 or q.stride(-1) != 1 or kv_c_normed.dtype != torch.bfloat16 or \
-                k_pe.dtype != torch.bfloat16 or kv_c_normed.stride(-1) != 1 or out.dtype != torch.bfloat16 or \
-                tuple(out.shape) != (t, n * 128) or out.stride(1) != 1 or out.stride(0) % 8 or out.data_ptr() % 16:
+        t, n, w = q.shape[0], self.num_heads, self._plain_up_weight()
+        bf16 = torch.bfloat16
+        if pick is None or w is None or not (w.dtype == bf16 or self.prefill_kv_fp16) or self.qk_nope_head_dim != 128 or \
+                self.v_head_dim != 128 or not (q.dtype == kv_c_normed.dtype == k_pe.dtype == out.dtype == bf16) or \
+                q.stride(-1) != 1 or kv_c_normed.stride(-1) != 1 or k_pe.stride(-1) != 1 or out.stride(-1) != 1 or \
+                tuple(out.shape) != (t, n * 128) or (q.stride(0) | q.stride(1) | k_pe.stride(0) | out.stride(0)) % 8 or \
+                (q.data_ptr() | k_pe.data_ptr() | out.data_ptr()) % 16:
             return False
         k_nope, pe, v, _ = self._kv_up_rows(kv_c_normed, k_pe)
         cu = prefill.query_start_loc.to(torch.int32).contiguous()

@@ -200,19 +200,19 @@ class HalfUpProjection:
     prefill_kv_fp16 = True
 
     def _plain_up_weight(self) -> Optional[torch.Tensor]:
-        """The up-projection weight [N*256, 512] if the prefill may make fp16 keys and values with it: plain, without bias."""
+        """The up-projection weight [N*256, 512] if it is a plain 16-bit one without bias."""
         w = getattr(self.kv_b_proj, "weight", None)
         n, d = self.num_heads, self.qk_nope_head_dim + self.v_head_dim
-        if not self.prefill_kv_fp16 or not isinstance(w, torch.Tensor) or w.dtype not in (torch.bfloat16, torch.float16) \
+        if not isinstance(w, torch.Tensor) or w.dtype not in (torch.bfloat16, torch.float16) \
                 or tuple(w.shape) != (n * d, self.kv_lora_rank) or getattr(self.kv_b_proj, "bias", None) is not None:
             return None
         return w
 
     def _half_up_weight(self) -> Optional[torch.Tensor]:
-        """That weight in fp16 as it is now, or None.  A bf16 weight is converted anew for every prefill, on the stream that
+        """That weight in fp16 as it is now, or None (also where prefill_kv_fp16 is off).  A bf16 weight is converted anew for every prefill, on the stream that
         uses it, and nothing is kept: a write through ``.data`` or to an inference tensor leaves no trace that a kept copy
         could follow, and a copy made on one stream would have to be waited for on every other."""
-        w = self._plain_up_weight()
+        w = self._plain_up_weight() if self.prefill_kv_fp16 else None
         return None if w is None else w.to(torch.float16)
 
     def _split_kv(self, kv: torch.Tensor):
@@ -236,7 +236,7 @@ class HalfUpProjection:
         it, else all in the dtype of the up-projection's result.  w16: the weight in fp16, for the step's context rows (None: the
         module was called).  Latents, rope rows and weight are converted in one launch: torch's conversion of the weight of 64
         heads takes 24 us, as long as the up-projection of 1000 rows."""
-        w = self._plain_up_weight()
+        w = self._plain_up_weight() if self.prefill_kv_fp16 else None
         if w is not None and kv_c.dtype == torch.bfloat16 and k_pe.dtype == torch.bfloat16:
             if w.dtype == torch.bfloat16 and w.is_contiguous() and w.data_ptr() % 16 == 0:
                 c16, pe16, w16 = K.rows_f16(kv_c, k_pe, w)

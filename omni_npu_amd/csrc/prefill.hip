@@ -496,9 +496,9 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
   MLA_REQUIRE((prev_out == nullptr) == (prev_lse == nullptr), MLA_ERR_NULL, "%s: the earlier result and its log-sum-exp go together", what);
   MLA_REQUIRE(prev_out == nullptr || (prev_stride_t % 4 == 0 && prev_stride_h % 4 == 0 && (uintptr_t)prev_out % 16 == 0),
               MLA_ERR_SHAPE, "%s: rows of the earlier result must be 16-byte aligned", what);
-  MLA_REQUIRE(pick == nullptr || (kv_half && window == 0 && pick_words >= 2 && pick_words % 2 == 0 && pick_stride >= pick_words &&
+  MLA_REQUIRE(pick == nullptr || (window == 0 && pick_words >= 2 && pick_words % 2 == 0 && pick_stride >= pick_words &&
                                   pick_stride % 2 == 0 && (uintptr_t)pick % 8 == 0),
-              MLA_ERR_SHAPE, "%s: picks go with fp16 keys and values, without a window, in 8-byte aligned rows of whole 64-key tiles", what);
+              MLA_ERR_SHAPE, "%s: picks go without a window, in 8-byte aligned rows of whole 64-key tiles", what);
   if (batch == 0 || max_q_len == 0) return MLA_OK;
   PrefillParams p;
   p.q_nope = (const __bf16*)q_nope; p.qn_st = qn_stride_t; p.qn_sh = qn_stride_h;
@@ -512,9 +512,11 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
   p.lse = lse_out;
   p.prev_out = prev_out; p.po_st = prev_stride_t; p.po_sh = prev_stride_h; p.prev_lse = prev_lse;
   p.pick = pick; p.pick_st = pick_stride; p.pick_tiles = pick_words / 2;
-  auto* kern = pick ? mla_prefill_varlen_kernel<true, true> : kv_half ? mla_prefill_varlen_kernel<true, false> : mla_prefill_varlen_kernel<false, false>;
+  auto* kern = pick ? (kv_half ? mla_prefill_varlen_kernel<true, true> : mla_prefill_varlen_kernel<false, true>)
+                    : (kv_half ? mla_prefill_varlen_kernel<true, false> : mla_prefill_varlen_kernel<false, false>);
   int rc = ensure_dynamic_lds((const void*)mla_prefill_varlen_kernel<false, false>, kPfLdsB, what);
   if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)mla_prefill_varlen_kernel<true, false>, kPfLdsB, what);
+  if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)mla_prefill_varlen_kernel<false, true>, kPfLdsB, what);
   if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)mla_prefill_varlen_kernel<true, true>, kPfLdsB, what);
   if (rc != MLA_OK) return rc;
   dim3 grid((max_q_len + kPfRows - 1) / kPfRows, num_heads, batch);
@@ -554,8 +556,8 @@ extern "C" int mla_prefill_varlen_continue(const void* q_nope, int64_t qn_stride
 }
 
 // mla_prefill_varlen over a selection: bit j of pick[t] (32-bit words, rows pick_stride words apart, pick_words of them
-// valid) says whether query token t attends over key j of its sequence, within what causal already allows.  fp16 keys and
-// values, no window.
+// valid) says whether query token t attends over key j of its sequence, within what causal already allows.  No
+// window.
 extern "C" int mla_prefill_varlen_pick(const void* q_nope, int64_t qn_stride_t, int64_t qn_stride_h, const void* q_pe,
                                        int64_t qp_stride_t, int64_t qp_stride_h, const void* k_nope, int64_t kn_stride_t,
                                        int64_t kn_stride_h, const void* k_pe, int64_t kp_stride_t, const void* v,

@@ -864,8 +864,8 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
     (src/omni_npu/attention/ops.py:5-42) gives, in one launch.  ``out`` may be ``prev_out``.
     k_nope, k_pe and v may all three be fp16 (a caller that makes them with an fp16 GEMM): both products then run on fp16
     and the kernel skips the conversion of the value tiles it otherwise does (the queries stay bf16).
-    ``pick`` (int32 [T, W] bits, see topk's mask; W even and wide enough for the longest sequence; fp16 keys and values, no
-    window, no earlier result): a token attends over the keys its bits name."""
+    ``pick`` (int32 [T, W] bits, see topk's mask; W even and wide enough for the longest sequence; no window, no earlier
+    result): a token attends over the keys its bits name."""
     if window is not None and window < 1:
         raise ValueError(f"prefill_varlen: window must be positive (got {window})")
     _need_cuda(q_nope, q_pe, k_nope, k_pe, v, cu_q, cu_k, out, lse_out)
@@ -897,9 +897,9 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
     if pick is not None:
         _need_cuda(pick)
         if pick.dtype != torch.int32 or pick.dim() != 2 or pick.shape[0] < t or pick.shape[1] % 2 or pick.stride(1) != 1 or \
-                window is not None or prev_out is not None or not kv_half:
-            raise TypeError("prefill_varlen: pick must be int32 [T, W] (W even, rows contiguous), with fp16 keys and values, "
-                            "without a window or an earlier result")
+                window is not None or prev_out is not None:
+            raise TypeError("prefill_varlen: pick must be int32 [T, W] (W even, rows contiguous), without a window or an earlier "
+                            "result")
     if k_nope.shape[0] == 0 or t == 0:
         # no keys at all (a context chunk in which every sequence is empty): zeros and lse = -inf, as the kernel gives for
         # an empty key range (the earlier result itself when there is one); empty tensors have no address to hand over

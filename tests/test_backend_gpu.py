@@ -364,12 +364,10 @@ def test_dsa_prompts_attend_over_their_own_keys_with_the_picks_as_a_mask(dev, q_
     attn_close(got[0][1], got[1][1], 3e-2, 4e-3 + 4e-3)        # (the latent form also rounds absorbed queries and outputs to bf16)
 
 
-@pytest.mark.parametrize("q_lens", [[300], [1, 1, 129, 70, 300]])
-def test_pick_bits_go_with_the_step_and_a_second_forward_still_stands(dev, q_lens):
-    """The bits of a selection are given back once the attention has queued its use of them, on whatever stream that ran; a
-    second forward of the same step finds no bits, and no rows of its prompts either, and translates the picks itself."""
+def _dsa_prompts(dev, q_lens, n=16, topk=64):
+    """A layer with a plain up-projection, the selection inside an indexer module as the model owns it, and a step of prompts
+    (and decodes: a length of 1) with random inputs: (impl, selection, metadata, caches, forward's inputs, the indexer's)."""
     g = torch.Generator().manual_seed(sum(q_lens))
-    n, topk = 16, 64
     seq_lens = [q if q > 1 else 400 for q in q_lens]
     common = _common(q_lens, seq_lens)
     t = common.num_actual_tokens
@@ -381,26 +379,67 @@ def test_pick_bits_go_with_the_step_and_a_second_forward_still_stands(dev, q_len
     k8v, ksv = dsa.indexer_cache_views(kv_cache[2])
     k8_ref, ks_ref = O.fp8_quant_token(torch.randn(nblk, 128, 128, generator=g))
     k8v.copy_(k8_ref.view(torch.uint8)); ksv.copy_(ks_ref)
-    indexer = dsa.LightningIndexer(topk, max_tokens=t, device=dev)
-    indexer.rows_buffer.fill_(nblk * 128 - 1)                  # (what earlier steps may have left where prompts have no rows)
-    indexer.counts_buffer.fill_(1)
-    # the selection also inside an indexer module, as the model owns it
-    impl, w = _mk_impl(dsa.NPUDSAImpl, n, dev, indexer=SimpleNamespace(select=indexer, topk_indices_buffer=indexer.topk_indices_buffer))
+    select = dsa.LightningIndexer(topk, max_tokens=t, device=dev)
+    select.rows_buffer.fill_(nblk * 128 - 1)                   # (what earlier steps may have left where prompts have no rows)
+    select.counts_buffer.fill_(1)
+    impl, w = _mk_impl(dsa.NPUDSAImpl, n, dev, indexer=SimpleNamespace(select=select, topk_indices_buffer=select.topk_indices_buffer))
     impl.kv_b_proj = _PlainLinear(w, dev)
     impl.process_weights_after_loading(torch.bfloat16)
     meta = dsa.NPUDSAMetadataBuilder(V.AttentionSpec(128, 1, 704, torch.bfloat16), ["l"], _cfg(cap=1), dev).build(0, _to(common, dev))
     rand = lambda *s: torch.randn(*s, generator=g).bfloat16().to(dev)
-    a = [rand(t, n, 192), rand(t, 512), rand(t, 1, 64)]
-    indexer(rand(t, 64, 128), rand(t, 128), rand(t, 64), kv_cache, meta)
-    assert indexer.mask_for(meta) is not None
-    outs = [torch.zeros(t, n * 128, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    return (impl, select, meta, kv_cache, [rand(t, n, 192), rand(t, 512), rand(t, 1, 64)],
+            [rand(t, 64, 128), rand(t, 128), rand(t, 64)])
+
+
+@pytest.mark.parametrize("q_lens", [[300], [1, 1, 129, 70, 300]])
+def test_pick_bits_go_with_the_step_and_a_second_forward_still_stands(dev, q_lens):
+    """The bits of a selection are given back once the attention has queued its use of them, on whatever stream that ran; a
+    second forward of the same step finds no bits, and no rows of its prompts either, and translates the picks itself."""
+    impl, select, meta, kv_cache, a, i = _dsa_prompts(dev, q_lens)
+    select(*i, kv_cache, meta)
+    assert select.mask_for(meta) is not None
+    outs = [torch.zeros(sum(q_lens), 16 * 128, dtype=torch.bfloat16, device=dev) for _ in range(2)]
     torch.cuda.synchronize(dev)
     with torch.cuda.stream(torch.cuda.Stream(dev)):
         for out in outs:
             impl.forward(None, *a, kv_cache, meta, output=out)
-            assert indexer.mask_for(meta) is None and indexer.masked_prompts(meta)
+            assert select.mask_for(meta) is None and select.masked_prompts(meta)
     torch.cuda.synchronize(dev)
     attn_close(outs[0], outs[1], 3e-2, 4e-3 + 4e-3)            # (the bar of two bf16 results, as above)
+
+
+def _picked_attention_f64(impl, select, a):
+    """Attention of one prompt's tokens over their picks in 64 bits, from the layer's weight and the step's own rows: [T, N*128]."""
+    q, c, pe = (x.double().cpu() for x in a)
+    t, n = q.shape[:2]
+    kv = (c @ impl.kv_b_proj.weight.double().cpu().t()).view(t, n, 256)
+    idx = select.topk_indices_buffer[:t].long().cpu()
+    seen = torch.zeros(t, t + 1, dtype=torch.bool).scatter_(1, torch.where(idx >= 0, idx, t), True)[:, :t]
+    s = (torch.einsum("inp,jnp->nij", q[..., :128], kv[..., :128]) + torch.einsum("inp,jp->nij", q[..., 128:], pe[:, 0])) * impl.scale
+    return torch.einsum("nij,jnv->inv", s.masked_fill(~seen, float("-inf")).softmax(-1), kv[..., 128:]).reshape(t, n * 128)
+
+
+@pytest.mark.parametrize("which", ["rope rows", "latents", "queries", "small"])
+def test_masked_prompts_keep_the_range_of_bf16(dev, which):
+    """Rope rows, latents or queries beyond 65504 (against factors as small, so that the scores stay moderate), and ones below
+    2^-24, which fp16 has no bits for."""
+    impl, select, meta, kv_cache, a, i = _dsa_prompts(dev, [200])
+    big = 2.0 ** 18
+    if which == "rope rows":
+        a[2].mul_(big); a[0][..., 128:].div_(big)
+    elif which == "latents":                                   # (one that only the keys use: values stay what they were)
+        w = impl.kv_b_proj.weight.view(16, 256, 512)
+        a[1][:, 7].mul_(big); w[:, :128, 7].div_(big); w[:, 128:, 7] = 0
+    elif which == "queries":
+        a[0].mul_(big); a[2].div_(big); impl.kv_b_proj.weight.view(16, 256, 512)[:, :128].div_(big)
+    else:
+        a[2].div_(2.0 ** 26); a[0][..., 128:].mul_(2.0 ** 26)
+    impl.process_weights_after_loading(torch.bfloat16)
+    select(*i, kv_cache, meta)
+    assert select.mask_for(meta) is not None
+    out = torch.zeros(200, 16 * 128, dtype=torch.bfloat16, device=dev)
+    impl.forward(None, *a, kv_cache, meta, output=out)
+    attn_close(out, _picked_attention_f64(impl, select, a).float(), 3e-2, 4e-3)
 
 
 class _NoNative:

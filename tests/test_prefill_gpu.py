@@ -372,15 +372,16 @@ def test_rows_f16_and_fp16_gathers_round_like_torch(dev, rows):
         assert torch.equal(half, plain.half())
 
 
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("q_lens,density", [([1], 1.0), ([63, 64, 65], 0.5), ([200, 129], 0.1), ([400], 0.02)])
-def test_prefill_over_picked_keys(dev, q_lens, density):
+def test_prefill_over_picked_keys(dev, q_lens, density, dt):
     """Causal attention over the keys that a token's bits name (the first visible key always among them), bits behind the
     causal limit set at random: against fp32 attention with the same mask."""
     from omni_npu_amd import kernels as K
     g = torch.Generator().manual_seed(sum(q_lens))
     n, t, scale = 3, sum(q_lens), 192 ** -0.5
     q = torch.randn(t, n, 192, generator=g).bfloat16()
-    kv, pe = torch.randn(t, n, 256, generator=g).half(), torch.randn(t, 64, generator=g).half()
+    kv, pe = torch.randn(t, n, 256, generator=g).to(dt), torch.randn(t, 64, generator=g).to(dt)
     width = (max(q_lens) + 63) // 64 * 64
     on = torch.rand(t, width, generator=g) < density
     on[:, 0] = True
@@ -402,7 +403,7 @@ def test_prefill_over_picked_keys(dev, q_lens, density):
     assert torch.allclose(lse.cpu(), ref_lse, atol=2e-2, rtol=1e-3)
 
 
-@pytest.mark.parametrize("kind", ["bf16", "fp16", "picked"])
+@pytest.mark.parametrize("kind", ["bf16", "fp16", "bf16 picked", "fp16 picked"])
 def test_the_denominator_adds_probabilities_before_they_are_rounded(dev, kind):
     """log-sum-exp against 64 bits where nothing but the kernel's fp32 arithmetic errs: scores are sums of four products of
     eighths of at most 1, exact in fp32, times a power of two.  What is left, for up to 16 keys: the scaled score (2.9 in log2,
@@ -414,13 +415,13 @@ def test_the_denominator_adds_probabilities_before_they_are_rounded(dev, kind):
     eighths = lambda *s: (torch.randint(-8, 9, s, generator=g).float() / 8)
     q, k = torch.zeros(t, n, 192), torch.zeros(t, n, 128)
     q[..., :4], k[..., :4] = eighths(t, n, 4), eighths(t, n, 4)
-    dt = torch.bfloat16 if kind == "bf16" else torch.float16
+    dt = torch.bfloat16 if "bf16" in kind else torch.float16
     v = torch.randn(t, n, 128, generator=g)
     cu = torch.tensor([0, t], dtype=torch.int32, device=dev)
     out, lse = torch.empty(t, n, 128, dtype=torch.bfloat16, device=dev), torch.empty(t, n, device=dev)
     qd = q.bfloat16().to(dev)
     K.prefill_varlen(qd[..., :128], qd[..., 128:], k.to(dev, dt), torch.zeros(t, 64, dtype=dt, device=dev), v.to(dev, dt), cu, cu, t, scale,
-                     True, out, lse, pick=torch.full((t, 2), -1, dtype=torch.int32, device=dev) if kind == "picked" else None)
+                     True, out, lse, pick=torch.full((t, 2), -1, dtype=torch.int32, device=dev) if "picked" in kind else None)
     s = torch.einsum("inp,jnp->nij", q[..., :128].double(), k.double()) * scale
     ref = s.masked_fill(~torch.ones(t, t).tril().bool(), float("-inf")).logsumexp(-1).t()
     assert (lse.cpu().double() - ref).abs().max() <= 2e-6
