@@ -238,7 +238,7 @@ class HalfUpProjection:
         heads takes 24 us, as long as the up-projection of 1000 rows."""
         w = self._plain_up_weight() if self.prefill_kv_fp16 else None
         if w is not None and kv_c.dtype == torch.bfloat16 and k_pe.dtype == torch.bfloat16:
-            if w.dtype == torch.bfloat16 and w.is_contiguous() and w.data_ptr() % 16 == 0:
+            if w.dtype == torch.bfloat16 and w.stride(1) == 1:
                 c16, pe16, w16 = K.rows_f16(kv_c, k_pe, w)
             else:
                 (c16, pe16), w16 = K.rows_f16(kv_c, k_pe), w.to(torch.float16)

@@ -300,15 +300,17 @@ def gather_paged_fp8(cache: torch.Tensor, dst: torch.Tensor, block_table: torch.
 
 def rows_f16(kv_c: torch.Tensor, k_pe: torch.Tensor, weight: Optional[torch.Tensor] = None):
     """(kv_c [T,512], k_pe [T,64] or [T,1,64]) bf16 -> the same rows as contiguous fp16 [T,512], [T,64], in one launch; with
-    ``weight`` (bf16 [W,512], the up-projection's) that as contiguous fp16 too, as a third result of the same launch."""
+    ``weight`` (bf16 [W,512], the up-projection's) that as contiguous fp16 too, as a third result of the same launch.  Rows
+    that are not on 16-byte boundaries are converted by torch."""
     _need_cuda(kv_c, k_pe, weight)
     k_pe = k_pe.reshape(k_pe.shape[0], -1)
     t = kv_c.shape[0]
-    if kv_c.shape != (t, D_NOPE) or k_pe.shape != (t, D_ROPE) or kv_c.dtype != torch.bfloat16 or k_pe.dtype != torch.bfloat16 or \
-            kv_c.stride(-1) != 1 or k_pe.stride(-1) != 1:
-        raise ValueError("rows_f16: bf16 kv_c [T,512] and k_pe [T,64] with contiguous last dims")
+    if kv_c.shape != (t, D_NOPE) or k_pe.shape != (t, D_ROPE) or kv_c.dtype != torch.bfloat16 or k_pe.dtype != torch.bfloat16:
+        raise ValueError("rows_f16: bf16 kv_c [T,512] and k_pe [T,64]")
     if weight is not None and (weight.dtype != torch.bfloat16 or weight.dim() != 2 or weight.shape[1] != D_NOPE or weight.stride(1) != 1):
         raise ValueError("rows_f16: the weight must be bf16 [W,512] with a contiguous last dim")
+    if any(x is not None and (x.stride(-1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16) for x in (kv_c, k_pe, weight)):
+        return tuple(x.to(torch.float16, memory_format=torch.contiguous_format) for x in (kv_c, k_pe, weight) if x is not None)
     c = torch.empty(t, D_NOPE, dtype=torch.float16, device=kv_c.device)
     r = torch.empty(t, D_ROPE, dtype=torch.float16, device=kv_c.device)
     w16 = torch.empty(weight.shape, dtype=torch.float16, device=kv_c.device) if weight is not None else None

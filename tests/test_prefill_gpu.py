@@ -347,6 +347,21 @@ def test_rows_f16_takes_the_weight_along(dev, rows, w_rows, stride):
     assert torch.equal(c16, c.half()) and torch.equal(r16, r.half()) and torch.equal(w16, w.half()) and w16.is_contiguous()
 
 
+@pytest.mark.parametrize("what", ["offset", "stride", "step", "weight offset"])
+def test_rows_f16_takes_rows_off_their_boundaries(dev, what):
+    """Rows that a 16-byte load cannot read: an odd offset, an odd stride, elements apart; a weight at an odd offset."""
+    from omni_npu_amd import kernels as K
+    base = torch.randn(6, 1040, generator=torch.Generator().manual_seed(1)).bfloat16().to(dev)
+    off, step = (1, 1) if what in ("offset", "weight offset") else (0, 2 if what == "step" else 1)
+    if what == "stride":
+        base = base.flatten()[:6 * 1039].view(6, 1039)
+    c, r, w = base[:, off:off + 512 * step:step], base[:, off:off + 64 * step:step], base[:, off:off + 512]
+    w = w if "weight" in what else w.contiguous()
+    c, r = (c.contiguous(), r.contiguous()) if "weight" in what else (c, r)
+    for got in (K.rows_f16(c, r), K.rows_f16(c, r, w)):
+        assert all(torch.equal(x, y.half()) and x.is_contiguous() for x, y in zip(got, (c, r, w)))
+
+
 @pytest.mark.parametrize("rows", [1, 4, 5, 1027])
 def test_rows_f16_and_fp16_gathers_round_like_torch(dev, rows):
     """bf16 -> fp16 of the step's rows and of both gathers: the bits of torch's conversion of the bf16 result, normal,
