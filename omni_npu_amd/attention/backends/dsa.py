@@ -24,13 +24,18 @@ from ..._vllm_compat import (PAD_SLOT_ID, AttentionCGSupport, AttentionType, MLA
                              MLACommonPrefillMetadata, QueryLenSupport, get_current_vllm_config)
 
 INDEX_HEAD_DIM = 128
-# Scores and values of a (token, key) pair and head cost 640 flops on up-projected keys and 2176 on latents (the up-projection
-# costs what absorbing the queries and up-projecting the outputs does), and the latents have to be gathered per token: leaving
-# out most of the pairs that were scored still pays up to this many visible pairs per picked one.  Measured with 128 heads
-# and k = 2048, us for one prompt, masked / gathered: 2k tokens 397 / 1109, 8k (2.2 pairs per pick) 4432 / 6595, 12k (3.2)
-# 9274 / 10 555, 16k (4.2) 15 407 / 14 897.  With fewer heads the scores get cheaper and the gather does not (16 heads, 16k
-# tokens: 4689 / 14 254), so the limit grows as the heads shrink.
-MASKED_PAIRS_PER_PICK = 3.5
+def masked_pairs_per_pick(num_heads: int) -> float:
+    """Up to how many visible (token, key) pairs per picked one prompts attend over up-projected keys under a mask of the picks
+    instead of gathering the picked latents.
+
+    Scores and values of a pair and head cost 640 flops on up-projected keys and 2176 on latents (the up-projection costs what
+    absorbing the queries and up-projecting the outputs does), and the latents have to be gathered per token whatever the heads
+    are: a share of the gather that goes with the heads, and one that does not.  Measured with k = 2048, one prompt, bf16 keys, ms
+    of selection and attention masked / gathered (visible pairs per pick): 128 heads 4.1 / 6.5 (2.3), 9.5 / 10.9 (3.3),
+    12.5 / 12.7 (3.8), 16.0 / 15.0 (4.3); 64 heads 9.3 / 12.1 (4.3), 17.0 / 17.7 (5.8), 19.9 / 19.5 (6.3); 32 heads 22.0 / 26.8
+    (8.3), 33.9 / 36.1 (10.3), 47.4 / 46.3 (12.3); 16 heads 15.4 / 32.8 (8.3), 56.7 / 81.4 (16.3, the longest prompt a step
+    holds).  They meet at 3.95, 6.1 and 11.5 pairs; the line stays below them."""
+    return 1.7 + 269.0 / num_heads
 
 
 def indexer_cache_views(index_cache: torch.Tensor):
@@ -328,8 +333,7 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
     def offer_masked_prompts(self, select) -> None:
         """Tells the selection whether, and for how many pairs per pick, this layer attends over masked prompts."""
         if hasattr(select, "masked_pairs_per_pick"):
-            select.masked_pairs_per_pick = (MASKED_PAIRS_PER_PICK * max(1.0, 128 / self.num_heads)
-                                            if self._plain_up_weight() is not None else 0.0)
+            select.masked_pairs_per_pick = masked_pairs_per_pick(self.num_heads) if self._plain_up_weight() is not None else 0.0
 
     def _v_up_proj(self, x: torch.Tensor, out: torch.Tensor):
         """[T,N,512] token-major -> out [T, N*V]  (reference dsa.py:233-240)."""

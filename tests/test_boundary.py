@@ -417,3 +417,15 @@ def test_builder_keeps_widened_seq_lens_in_one_int32_buffer():
             assert d.seq_lens.dtype == torch.int32 and d.seq_lens.tolist() == lens
             ptrs.append(d.seq_lens.data_ptr())
         assert len(set(ptrs)) == 1
+
+
+def test_masked_prompts_stop_where_the_gather_is_as_fast():
+    """The limit stays below the pairs per pick at which masked and gathered prompts were measured equal, and within a seventh
+    of it; at 16 heads masked is still the faster one at the longest prompt a step can hold (16.3 pairs per pick)."""
+    for heads, even in ((128, 3.95), (64, 6.1), (32, 11.5)):
+        assert 0.85 * even <= dsa.masked_pairs_per_pick(heads) <= even
+    assert dsa.masked_pairs_per_pick(16) > 16.3
+    k, n = 2048, 44000                                          # 11.0 pairs per pick: masked for 16 heads, gathered for 32
+    p = dsa.NPUDSAPrefillMetadata.__new__(dsa.NPUDSAPrefillMetadata)
+    p.prompt_lens = [n]
+    assert p.over_up_projected(k, dsa.masked_pairs_per_pick(16)) and not p.over_up_projected(k, dsa.masked_pairs_per_pick(32))
