@@ -31,6 +31,7 @@ using OptTensor = std::optional<Tensor>;
 constexpr int64_t kNope = 512, kRope = 64, kPage = 128, kFp8Row = 656, kVDim = 128;
 constexpr int64_t kAbsorbMaxTokens = 256;   // kernels.ABSORB_MAX_TOKENS
 constexpr int64_t kVupMaxTokens = 256;      // kernels.VUP_MAX_TOKENS: beyond, a separate merge and the library GEMM
+constexpr int64_t kSparseWorkspaceCap = 256 << 20;   // kernels.SPARSE_WORKSPACE_CAP
 
 void check(int rc, const char* what) {
   if (rc != 0) throw std::runtime_error(std::string(what) + " failed with code " + std::to_string(rc) + ": " + mlahip_last_error_string());
@@ -252,7 +253,7 @@ bool sparse_decode(const Tensor& q, const Tensor& nope, const Tensor& rope, cons
   const int64_t n = q.size(1);
   const int splits = launch_splits(t, 1, n, rows.size(1));
   const int64_t need = (int64_t)mla_decode_workspace_bytes((int)t, 1, (int)n, splits);
-  if (need > (256 << 20)) return false;                        // kernels.SPARSE_WORKSPACE_CAP
+  if (need > kSparseWorkspaceCap) return false;
   NewRows new_rows;
   const bool write = kv_c.has_value();
   if (write && !(k_pe && slots && rows_of(*kv_c, *k_pe, *slots, dev, new_rows))) return false;
@@ -374,4 +375,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sparse_decode", &sparse_decode);
   m.def("dsa_select", &dsa_select);
   m.def("norm_rope_cache", &norm_rope_cache);
+  // (what this file has a copy of, for a test to hold against kernels.py)
+  m.def("launch_splits", &launch_splits);
+  m.attr("ABSORB_MAX_TOKENS") = kAbsorbMaxTokens;
+  m.attr("VUP_MAX_TOKENS") = kVupMaxTokens;
+  m.attr("SPARSE_WORKSPACE_CAP") = kSparseWorkspaceCap;
 }
