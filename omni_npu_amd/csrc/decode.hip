@@ -111,7 +111,8 @@ extern "C" int mla_decode_bf16_split(const void* q_nope, int64_t qn_stride_t, in
 // lengths of the shortened sequences the kernel walks (sink keys + the blocks that hold some token's window) and the
 // number of 32-key blocks left out; mla_decode_bf16_window_split is mla_decode_bf16_split over those, and the merge is
 // the ordinary one with the shortened lengths.  With skip = NULL the kernel takes the lengths behind the sink and works both
-// out for itself (a launch of 5 us less), and the merge takes those lengths too: it only asks which sequences are empty.
+// out for itself (a launch of 5 us less, and what kernels.py and the native host side do), and the merge takes those lengths too:
+// it only asks which sequences are empty.  The plan is for callers of the C entry points that make it once for a step's layers.
 namespace mlahip {
 __global__ void mla_window_plan_kernel(const int32_t* seq_lens, const int32_t* qsl, int32_t batch, int32_t max_q_len,
                                        int32_t sink_len, int32_t window, int32_t* short_lens, int32_t* skip) {

@@ -383,3 +383,42 @@ def test_prefill_window_random_shapes(dev, i, q_lens, k_extra, window, heads):
     ref, ref_lse = O.attention_varlen(qn, qp, kn, kp, v, cu_q, cu_k, scale, True, window=window)
     attn_close(out, ref, MAX_ABS, MEAN_REL)
     assert (lse.cpu() - ref_lse).abs().max() < 2e-2
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_window_split_over_a_made_plan_is_the_split_that_plans_for_itself(dev, monkeypatch, fp8):
+    """mla_window_plan's lengths and skips handed to the split launches, against skip = NULL: the same bits."""
+    from omni_npu_amd import _lib, kernels as K
+    c, bt = _sink_case(6, 16, 60, 3000, 128, 2, seed=9)
+    d = lambda x: x.to(dev)
+    lens = d(c["seq_lens"])
+    if fp8:
+        cache = torch.zeros(c["nope"].shape[0], 128, 656, dtype=torch.uint8, device=dev)
+        rows = c["nope"].shape[0] * 128
+        K.cache_write_fp8(d(c["nope"]).view(rows, 512), d(c["rope"]).view(rows, 64), torch.arange(rows, device=dev), cache)
+        run = lambda out: K.decode_fp8(d(c["q_nope"]), d(c["q_rope"]), cache, d(bt), lens, c["scale"], out, q_len=2, sink_len=128, window=500)
+    else:
+        run = lambda out: K.decode(d(c["q_nope"]), d(c["q_rope"]), d(c["nope"]), d(c["rope"]), d(bt), lens, c["scale"], out, q_len=2,
+                                   sink_len=128, window=500)
+    outs = [torch.empty(12, 16, 512, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    run(outs[0])
+    lib, short, skip = _lib.load(), torch.empty_like(lens), torch.empty_like(lens)
+    planned = []
+
+    class Planned:
+        def __getattr__(self, name):
+            fn = getattr(lib, name)
+            if not name.endswith("window_split"):
+                return fn
+
+            def with_plan(*a):
+                i = a.index(lens.data_ptr())
+                assert a[i + 1] is None
+                assert lib.mla_window_plan(a[i], a[i + 2], a[i + 3], a[i + 4], a[i + 6], a[i + 7], short.data_ptr(), skip.data_ptr(),
+                                           torch.cuda.current_stream().cuda_stream) == 0
+                planned.append(name)
+                return fn(*a[:i], short.data_ptr(), skip.data_ptr(), *a[i + 2:])
+            return with_plan
+    monkeypatch.setattr(_lib, "load", lambda: Planned())
+    run(outs[1])
+    assert len(planned) == 1 and int(skip.max()) > 0 and torch.equal(outs[0], outs[1])
