@@ -2,7 +2,6 @@
 // phase of mla_decode_bf16 / mla_decode_fp8 / dsa_sparse_decode_bf16 and the body of mla_splitkv_reduce.
 #include "decode_params.hpp"
 #include <type_traits>
-#include <cstdlib>
 
 namespace mlahip {
 

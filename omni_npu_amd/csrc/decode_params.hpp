@@ -44,7 +44,7 @@ struct ChunkReduceParams {
 };
 int launch_chunk_reduce(const ChunkReduceParams& p, hipStream_t stream);
 
-// The chunk plan of the split kernels, as the merge kernels recompute it: work is counted in blocks of kPlanBlk keys,
+// The chunk plan of the split kernels (the merge kernels read its outcome from seg_ids): work is counted in blocks of kPlanBlk keys,
 // and every non-empty sequence costs kPlanSegCost more units of start-up.
 constexpr int kPlanBlk = 32;
 constexpr int kPlanSegCost = 8;

@@ -53,7 +53,7 @@ constexpr int kCopies = 9;                                 // copy instructions 
 constexpr int kAhead = 4;                                  // K fragments read ahead of the MFMA that consumes them (2 and 6 measured the same)
 constexpr float kRestartThreshold = 100.f;                 // log2 units above a row's reference
 constexpr int kSegCost = kPlanSegCost;
-static_assert(kBlk == kPlanBlk, "the merge kernels recompute the chunk plan with these constants");
+static_assert(kBlk == kPlanBlk, "the chunk plan counts work in the blocks that this kernel walks");
 
 // XOR swizzles of the 16-byte granules of a row: linear over GF(2), so swz(a ^ b) = swz(a) ^ swz(b)
 __device__ __forceinline__ int swz_nope(int r) {
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
     }
     return len;
   };
-  // ---- which blocks are mine: the balanced chunk plan (see mla_chunk_reduce_kernel, which recomputes it) ----
+  // ---- which blocks are mine: the balanced chunk plan (decode_params.hpp) ----
   // Every non-empty sequence is kSegCost units of start-up followed by its 32-key blocks, the sequences end to end, and
   // that line is cut into plan_chunk_count() chunks of equal length; a chunk that crosses a sequence boundary runs several
   // segments; the segment of sequence b in chunk c writes partial number c + b.

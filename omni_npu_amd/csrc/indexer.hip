@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256, 2) void dsa_indexer_fp8_kernel(const IndexerPa
 // operations in the same order as above: the same bits.
 constexpr int kTileTok = 4;
 constexpr int kTileMinQ = 16;                         // shorter requests (decode, MTP) take the streaming kernel
-constexpr int kTileWOff = kTileTok * 64 * kIdxDim;    // 65536: weights [token][head] behind the query rows
+constexpr int kTileWOff = kTileTok * 64 * kIdxDim;    // 32768: weights [token][head] behind the query rows
 constexpr int kTileLdsB = kTileWOff + kTileTok * 64 * 4;
 
 __global__ __launch_bounds__(256, 4) void dsa_indexer_tile_kernel(const IndexerParams p) {

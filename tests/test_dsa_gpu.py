@@ -390,7 +390,7 @@ def test_sparse_decode_method_choice_and_refusals(dev):
 
 @pytest.mark.parametrize("q_lens,extra", [([16], 0), ([17, 40], 0), ([33, 1, 130], 200), ([300], 1000)])
 def test_prompt_scores_are_the_streaming_kernels_bits(dev, q_lens, extra):
-    """Requests of 16 tokens and more take the kernel that keeps eight tokens' queries in LDS.  Every token once more as a
+    """Requests of 16 tokens and more take the kernel that keeps four tokens' queries in LDS.  Every token once more as a
     request of its own (the streaming kernel): the same logits bit for bit, ragged lengths and last groups included."""
     from omni_npu_amd import kernels as K
     g = torch.Generator().manual_seed(sum(q_lens))
