@@ -25,8 +25,8 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # dense bf16
 
 
 def host_cpu():
-    """Model name and logical CPU count of the host, and the thread count the oracle runs with (the GPU box gives one GPU's
-    job 16 CPUs whatever the host has)."""
+    """Model name and logical CPU count of the host, and the thread count the oracle runs with (a job may be given
+    fewer CPUs than the host has)."""
     model = "unknown"
     try:
         with open("/proc/cpuinfo") as f:
@@ -981,8 +981,8 @@ def bench_dsa_layer(K, dev, args):
 
 def bench_window(K, dev, args):
     """Decode with static sink tokens and a sliding window (the reference's variant of attention/backends/mla.py:705-779):
-    B=64, 128 heads, 4096-8192 keys behind a 128-key sink, window 4096.  One step = window plan + dense split kernel over
-    the shortened sequences + merge, replayed as a HIP graph; the split kernel is also timed alone."""
+    B=64, 128 heads, 4096-8192 keys behind a 128-key sink, window 4096.  One step = dense split kernel over the shortened
+    sequences + merge, replayed as a HIP graph."""
     import time
     from oracle import mla_oracle as O
     B, N, sink, win = 64, 128, 128, 4096
@@ -1041,7 +1041,8 @@ def bench_window(K, dev, args):
         "roofline": {"kernel": "mla_decode_v3_kernel<false, true, 4> + merge (whole step)", "bound": "hbm",
                      "achieved": round(alg_bytes / t_step / 1e3, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(alg_bytes / t_step / 1e3 / HBM_PEAK_GBS, 4),
-                     "traffic": traffic, "traffic_source": traffic_src, "algorithmic_bytes": alg_bytes},
+                     "traffic": traffic, "traffic_source": traffic_src, "algorithmic_bytes": alg_bytes,
+                     "socket_power": None if args.no_power_probe else socket_power(step)},
         "cpu_baseline": {"value": round(cpu_s * B / sample * 1e6, 1), "unit": "us/layer", **cpu_info,
                          "kind": "port", "sample": f"oracle sink_decode (torch fp32) of {sample} of {B} sequences, scaled by sequence count",
                          "gpu_vs_oracle_max_abs": err},
@@ -1075,7 +1076,7 @@ def main():
     ap.add_argument("--splits", type=int, default=0, help="KV splits per sequence (0 = library default)")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-power-probe", action="store_true",
-                    help="decode, fp8 and prefill workloads: skip the two seconds of queued launches under the socket power reading")
+                    help="decode, fp8, prefill and window workloads: skip the two seconds of queued launches under the socket power reading")
     ap.add_argument("--graph", action="store_true",
                     help="decode workload: time the steps as replays of captured HIP graphs (--graph-layers steps per graph) "
                          "instead of eager launches; the default line carries the one-step-per-graph figure either way "

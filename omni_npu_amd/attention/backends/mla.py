@@ -195,7 +195,7 @@ class HalfUpProjection:
     # The prefill kernel multiplies the probabilities with fp16 values (the bf16 bar of the output leaves no room for bf16
     # probabilities), so it converts every value tile it is given in bf16.  Where the up-projection is a plain weight the
     # keys and values are made in fp16 in the first place - the same GEMM on fp16 copies of its operands, no extra pass -
-    # and the kernel converts nothing (configs of 4 x 2048 over 16k: 13.2 -> 12.2 ms).  fp16 holds every bf16 number of
+    # and the kernel converts nothing (4 x 2048 over 16k: attention 12.6 -> 11.5 ms).  fp16 holds every bf16 number of
     # magnitude 2^-14 .. 65504 exactly; set prefill_kv_fp16 = False for a model whose keys or values can exceed that range.
     prefill_kv_fp16 = True
 
@@ -209,9 +209,10 @@ class HalfUpProjection:
         return w
 
     def _half_up_weight(self) -> Optional[torch.Tensor]:
-        """That weight in fp16 as it is now, or None (also where prefill_kv_fp16 is off).  A bf16 weight is converted anew for every prefill, on the stream that
-        uses it, and nothing is kept: a write through ``.data`` or to an inference tensor leaves no trace that a kept copy
-        could follow, and a copy made on one stream would have to be waited for on every other."""
+        """That weight in fp16 as it is now, or None (also where prefill_kv_fp16 is off).  A bf16 weight is converted anew for
+        every prefill, on the stream that uses it, and nothing is kept: a write through ``.data`` or to an inference tensor
+        leaves no trace that a kept copy could follow, and a copy made on one stream would have to be waited for on every
+        other."""
         w = self._plain_up_weight() if self.prefill_kv_fp16 else None
         return None if w is None else w.to(torch.float16)
 
