@@ -294,6 +294,16 @@ int mla_merge_n_states(const void* outs, int64_t outs_stride_n, int64_t outs_str
                        int64_t lses_stride_n, float* out, int64_t out_stride_t, float* lse_out, int32_t n, int32_t tokens,
                        int32_t dim, mlahip_stream_t stream);
 
+/* ---- keys and values of prefill tokens out of their latents ----------------------------------
+ * The up-projection of attention/backends/mla.py:405-413, 566-571 (kv_b_proj): out[h, t, :] = x[t, :] . weight[h * 256 + :, :]^T with
+ * x bf16 [num_rows, 512], weight bf16 [num_heads * 256, 512], out 16-bit rows of 256 (strides in elements; token t of head h at
+ * t * out_stride_t + h * out_stride_h): 128 columns of the key, fp16 with keys_f16 and bf16 without, and 128 of the value,
+ * always fp16 (without keys_f16 finite values beyond 65504 are clamped there).  k_pe / out_pe (or both NULL): the rows' rope
+ * part [num_rows, 64], bf16, written as fp16 by the same launch. */
+int mla_kv_up(const void* x, int64_t x_stride, const void* weight, int64_t w_stride, int64_t num_rows, int32_t num_heads,
+              int32_t keys_f16, void* out, int64_t out_stride_t, int64_t out_stride_h, const void* k_pe, int64_t k_pe_stride,
+              void* out_pe, int64_t out_pe_stride, mlahip_stream_t stream);
+
 /* ---- non-absorbed varlen attention for prefill -------------------------------------------
  * Replaces the prefill calls of npu_fused_infer_attention_score, attention/backends/mla.py:574-590 (suffix:
  * right-down causal, sparse_mode 3) and :415-431 (context chunk: no mask, softmax_lse_flag): q_nope [T,N,128],
@@ -306,6 +316,8 @@ int mla_merge_n_states(const void* outs, int64_t outs_stride_n, int64_t outs_str
  * GEMM; the queries stay bf16).  Both products then run on fp16 and the kernel skips the bf16 -> fp16 conversion of the value
  * tiles that it otherwise does for the P.V product. */
 #define MLA_PREFILL_KV_F16 16
+/* out_dtype + MLA_PREFILL_V_F16: v alone holds fp16 */
+#define MLA_PREFILL_V_F16 32
 int mla_prefill_varlen(const void* q_nope, int64_t qn_stride_t, int64_t qn_stride_h, const void* q_pe,
                        int64_t qp_stride_t, int64_t qp_stride_h, const void* k_nope, int64_t kn_stride_t,
                        int64_t kn_stride_h, const void* k_pe, int64_t kp_stride_t, const void* v, int64_t v_stride_t,

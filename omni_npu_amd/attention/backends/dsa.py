@@ -299,9 +299,11 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
     can_return_lse_for_decode: bool = False
     cache_written_for = None     # see NPUMLAImpl.cache_written_for
     # Prompts attend in the types that a gather of the cache would: bf16 latents, rope rows, queries and keys.  True makes keys and
-    # values in fp16 (11 bits instead of 8, at the same speed) for a model whose latents, rope rows, queries, keys and values stay
-    # between 2^-14 and 65504.
+    # rope rows fp16 (11 bits instead of 8, at the same speed) for a model whose rope rows, queries, keys and values stay between
+    # 2^-14 and 65504.
     prefill_kv_fp16 = False
+    # (masked prompts are offered for a plain weight only, whose product W_UK and W_UV stand for everywhere else)
+    keys_bf16_values_f16 = True
 
     def __init__(self, num_heads: int, head_size: int, scale: float, num_kv_heads: int, alibi_slopes: Optional[list],
                  sliding_window: Optional[int], kv_cache_dtype: str, logits_soft_cap: Optional[float], attn_type: str,

@@ -190,13 +190,16 @@ def _caller_wrote_cache(impl, attn_metadata, num_tokens: int) -> bool:
 
 
 class HalfUpProjection:
-    """Keys and values of prefill tokens, made in fp16 where the model's up-projection is a plain weight."""
+    """Keys and values of prefill tokens, the values in fp16 where the model's up-projection is a plain weight."""
 
     # The prefill kernel multiplies the probabilities with fp16 values (the bf16 bar of the output leaves no room for bf16
-    # probabilities), so it converts every value tile it is given in bf16.  Where the up-projection is a plain weight the
-    # keys and values are made in fp16 in the first place - the same GEMM on fp16 copies of its operands, no extra pass -
-    # and the kernel converts nothing (4 x 2048 over 16k: attention 12.6 -> 11.5 ms).  fp16 holds every bf16 number of
-    # magnitude 2^-14 .. 65504 exactly; set prefill_kv_fp16 = False for a model whose keys or values can exceed that range.
+    # probabilities), so it converts every value tile it is given in bf16.  Where the up-projection is a plain bf16 weight the
+    # keys and values come from kernels.kv_up, bf16 operands and fp32 sums, which writes the values as fp16 (4 x 2048 over 16k:
+    # attention 12.6 -> 11.5 ms); other plain weights go through the same GEMM on fp16 copies of its operands.
+    # Keys are fp16 too: eleven bits instead of eight.  Set prefill_kv_fp16 = False for a model whose keys or values can exceed
+    # 65504: the module is called then, unless keys_bf16_values_f16 says that kernels.kv_up may write bf16 keys and fp16 values
+    # (clamped at 65504, as the prefill kernel clamps the module's).
+    keys_bf16_values_f16 = False
     prefill_kv_fp16 = True
 
     def _plain_up_weight(self) -> Optional[torch.Tensor]:
@@ -216,6 +219,12 @@ class HalfUpProjection:
         w = self._plain_up_weight() if self.prefill_kv_fp16 else None
         return None if w is None else w.to(torch.float16)
 
+    def _kv_up_weight(self, kv_c: torch.Tensor) -> Optional[torch.Tensor]:
+        """The up-projection weight if keys and values are to come from kernels.kv_up and it takes the latent rows kv_c."""
+        w = self._plain_up_weight() if self.prefill_kv_fp16 or self.keys_bf16_values_f16 else None
+        return w if w is not None and self.qk_nope_head_dim == self.v_head_dim == 128 and K.kv_up_takes(kv_c, w, self.num_heads) \
+            else None
+
     def _split_kv(self, kv: torch.Tensor):
         kv = kv.view(-1, self.num_heads, self.qk_nope_head_dim + self.v_head_dim)
         return kv[..., :self.qk_nope_head_dim], kv[..., self.qk_nope_head_dim:]
@@ -233,10 +242,14 @@ class HalfUpProjection:
         return self._split_kv(kv[0] if isinstance(kv, tuple) else kv)
 
     def _kv_up_rows(self, kv_c: torch.Tensor, k_pe: torch.Tensor):
-        """(k_nope, k_pe [T,64], v, w16) of a step's own rows as the prefill kernel takes them: all fp16 where the weight allows
-        it, else all in the dtype of the up-projection's result.  w16: the weight in fp16, for the step's context rows (None: the
-        module was called).  Latents, rope rows and weight are converted in one launch: torch's conversion of the weight of 64
-        heads takes 24 us, as long as the up-projection of 1000 rows."""
+        """(k_nope, k_pe [T,64], v, w16) of a step's own rows as the prefill kernel takes them: from kernels.kv_up where it takes
+        them, else all fp16 where the weight allows it, else all in the dtype of the up-projection's result.  w16: the weight in
+        fp16, for the step's context rows (None: it was not needed, or the module was called).  Latents, rope rows and weight are
+        converted in one launch."""
+        w = self._kv_up_weight(kv_c)
+        if w is not None and k_pe.dtype == torch.bfloat16:
+            k_nope, v, pe = K.kv_up(kv_c, w, self.num_heads, self.prefill_kv_fp16, k_pe if self.prefill_kv_fp16 else None)
+            return k_nope, k_pe.reshape(k_pe.shape[0], -1) if pe is None else pe, v, None
         w = self._plain_up_weight() if self.prefill_kv_fp16 else None
         if w is not None and kv_c.dtype == torch.bfloat16 and k_pe.dtype == torch.bfloat16:
             if w.dtype == torch.bfloat16 and w.stride(1) == 1:
@@ -310,10 +323,12 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
         t, n = q_nope.shape[0], self.num_heads
         cu_q = prefill.query_start_loc.to(torch.int32).contiguous()
         output = output_lse = None
-        # (with an fp16 up-projection the rows are gathered as fp16 straight away, into the same bytes)
-        if w16 is None and cc.workspace.dtype == torch.bfloat16:
-            w16 = self._half_up_weight()
-        rows = cc.workspace if w16 is None or cc.workspace.dtype != torch.bfloat16 else cc.workspace.view(torch.float16)
+        # (kernels.kv_up takes the rows as the cache has them; for an fp16 GEMM they are gathered as fp16, into the same bytes)
+        rows = cc.workspace
+        own = self._kv_up_weight(rows[:, :self.kv_lora_rank])
+        if own is None and rows.dtype == torch.bfloat16:
+            w16 = self._half_up_weight() if w16 is None else w16
+            rows = rows if w16 is None else rows.view(torch.float16)
         for i in range(len(cc.seq_tot)):
             toks = int(cc.seq_tot[i])
             if toks == 0:
@@ -324,8 +339,12 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
                                                batch_size=attn_metadata.num_prefills, kv_cache_dtype=self.kv_cache_dtype,
                                                scale=k_scale, seq_starts=cc.starts[i], total_rows=toks)
             kv_c_normed, k_pe = rows[:toks, :self.kv_lora_rank], rows[:toks, self.kv_lora_rank:]
-            k_nope, v = self._kv_up(kv_c_normed, allow_fp16=True, w16=w16)
-            k_pe = k_pe.to(k_nope.dtype)
+            if own is not None:
+                k_nope, v, pe = K.kv_up(kv_c_normed, own, n, self.prefill_kv_fp16, k_pe if self.prefill_kv_fp16 else None)
+                k_pe = k_pe if pe is None else pe
+            else:
+                k_nope, v = self._kv_up(kv_c_normed, allow_fp16=True, w16=w16)
+                k_pe = k_pe.to(k_nope.dtype)
             # running results stay fp32: each bf16 rounding in between would add 2^-10 of mean relative error to the
             # layer's output
             first = output is None

@@ -134,12 +134,12 @@ __device__ __forceinline__ void pf_issue_tile(const PrefillParams& p, int64_t k0
   }
 }
 
-// kHalf: k_nope, k_pe and v hold fp16 instead of bf16 (a caller that makes them with an fp16 GEMM): both products run on
-// fp16 (the query is converted once, in registers) and no tile is converted.
+// kKeyHalf: k_nope and k_pe hold fp16 instead of bf16 and the scores run on fp16 (the query is converted once, in registers).
+// kValHalf: v holds fp16 and no tile is converted.  (mla_kv_up makes either.)
 // kPick: a row attends over the keys its bits name (sparse attention over a selection, for sequences short enough that
 // leaving out scores here costs less than gathering the selected latents; see NPUDSAImpl).  Three prompts of 1500 to 5003
 // tokens, 128 heads, k = 2048: 2145 us on bf16 keys and values, 2107 on fp16 ones, which need a narrower range.
-template <bool kHalf, bool kPick>
+template <bool kKeyHalf, bool kValHalf, bool kPick>
 __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const PrefillParams p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63;
@@ -285,7 +285,7 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
       for (int kk = 0; kk < 4; kk++) { bf16x8 v = *(const bf16x8*)(qp + koff[kk]); qf[8 + kk] = row_ok ? v : zero; }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       issue(first_tile, lds0 + first_buf, std::integral_constant<int, 2>{});
-      if constexpr (kHalf) {
+      if constexpr (kKeyHalf) {
 #pragma unroll
         for (int kk = 0; kk < 12; kk++) {
           f16x8 h;
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
       // barrier: the four wavefronts read each other's pieces.  (Tried: the conversion's arithmetic and writes behind the
       // first block's score MFMAs, and the next tile converted between the two blocks of this one - both slower.)
       char* vt = buf + kPfVOff + (int)threadIdx.x * 16;
-      if constexpr (!kHalf) {
+      if constexpr (!kValHalf) {
         u32x4 w[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) w[i] = *(const u32x4*)(vt + i * 4096);
@@ -367,7 +367,7 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
 #pragma unroll
         for (int kk = 0; kk < 12; kk++) {
           const bf16x8 a = *(const bf16x8*)(buf + koff[kk & 3] + (kk >> 2) * kPfSubB + tb * 4096);
-          if constexpr (kHalf) s[tb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, qf[kk]), s[tb], 0, 0, 0);
+          if constexpr (kKeyHalf) s[tb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, qf[kk]), s[tb], 0, 0, 0);
           else s[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[kk], s[tb], 0, 0, 0);
         }
       };
@@ -484,8 +484,9 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
   MLA_REQUIRE(q_nope && q_pe && k_nope && k_pe && v && cu_q && cu_k && out, MLA_ERR_NULL, "%s: null pointer argument", what);
   MLA_REQUIRE(batch >= 0 && num_heads >= 1 && max_q_len >= 0 && batch <= 65535 && num_heads <= 65535 && window >= 0,
               MLA_ERR_SHAPE, "%s: batch=%d num_heads=%d max_q_len=%d window=%d", what, batch, num_heads, max_q_len, window);
-  const bool kv_half = (out_dtype & 16) != 0;              // k_nope, k_pe and v hold fp16 (MLA_PREFILL_KV_F16)
-  out_dtype &= ~16;
+  const bool key_half = (out_dtype & 16) != 0;             // k_nope, k_pe and v hold fp16 (MLA_PREFILL_KV_F16)
+  const bool val_half = (out_dtype & 48) != 0;             // v alone does (MLA_PREFILL_V_F16)
+  out_dtype &= ~48;
   MLA_REQUIRE(out_dtype == 0 || out_dtype == 1, MLA_ERR_UNSUPPORTED, "%s: out dtype code %d", what, out_dtype);
   MLA_REQUIRE(scale > 0.f, MLA_ERR_UNSUPPORTED, "%s: the softmax scale must be positive (got %g)", what, (double)scale);
   MLA_REQUIRE(qn_stride_t % 8 == 0 && qn_stride_h % 8 == 0 && qp_stride_t % 8 == 0 && qp_stride_h % 8 == 0 &&
@@ -513,13 +514,16 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
   p.lse = lse_out;
   p.prev_out = prev_out; p.po_st = prev_stride_t; p.po_sh = prev_stride_h; p.prev_lse = prev_lse;
   p.pick = pick; p.pick_st = pick_stride; p.pick_tiles = pick_words / 2;
-  auto* kern = pick ? (kv_half ? mla_prefill_varlen_kernel<true, true> : mla_prefill_varlen_kernel<false, true>)
-                    : (kv_half ? mla_prefill_varlen_kernel<true, false> : mla_prefill_varlen_kernel<false, false>);
-  int rc = ensure_dynamic_lds((const void*)mla_prefill_varlen_kernel<false, false>, kPfLdsB, what);
-  if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)mla_prefill_varlen_kernel<true, false>, kPfLdsB, what);
-  if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)mla_prefill_varlen_kernel<false, true>, kPfLdsB, what);
-  if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)mla_prefill_varlen_kernel<true, true>, kPfLdsB, what);
+  static constexpr auto kernel_of = [](bool kh, bool vh, bool pk) {
+    return kh ? (pk ? mla_prefill_varlen_kernel<true, true, true> : mla_prefill_varlen_kernel<true, true, false>)
+         : vh ? (pk ? mla_prefill_varlen_kernel<false, true, true> : mla_prefill_varlen_kernel<false, true, false>)
+              : (pk ? mla_prefill_varlen_kernel<false, false, true> : mla_prefill_varlen_kernel<false, false, false>);
+  };
+  int rc = MLA_OK;
+  for (int i = 0; i < 6 && rc == MLA_OK; i++)              // (all of them: a caller's warm-up step need not be of the kind that it captures)
+    rc = ensure_dynamic_lds((const void*)kernel_of((i >> 1) == 2, (i >> 1) != 0, i & 1), kPfLdsB, what);
   if (rc != MLA_OK) return rc;
+  auto* kern = kernel_of(key_half, val_half, pick != nullptr);
   dim3 grid((max_q_len + kPfRows - 1) / kPfRows, num_heads, batch);
   hipLaunchKernelGGL(kern, grid, dim3(256), kPfLdsB, stream, p);
   return check_launch("mla_prefill_varlen_kernel");

@@ -322,6 +322,39 @@ def rows_f16(kv_c: torch.Tensor, k_pe: torch.Tensor, weight: Optional[torch.Tens
     return (c, r) if weight is None else (c, r, w16)
 
 
+def kv_up_takes(kv_c: torch.Tensor, weight: torch.Tensor, num_heads: int) -> bool:
+    """Whether kv_up takes latent rows [T,512] and a plain up-projection weight [N*256,512] as they are."""
+    return (kv_c.is_cuda and weight.is_cuda and kv_c.dtype == weight.dtype == torch.bfloat16 and kv_c.dim() == 2
+            and weight.shape == (num_heads * 256, D_NOPE) and kv_c.shape[1] == D_NOPE and kv_c.stride(1) == weight.stride(1) == 1
+            and not ((kv_c.stride(0) | weight.stride(0)) & 7) and kv_c.stride(0) <= 1 << 20 and weight.stride(0) <= 1 << 20
+            and not ((kv_c.data_ptr() | weight.data_ptr()) & 15))
+
+
+def kv_up(kv_c: torch.Tensor, weight: torch.Tensor, num_heads: int, keys_f16: bool, k_pe: Optional[torch.Tensor] = None):
+    """(k_nope [T,N,128], v [T,N,128], k_pe16) of latent rows kv_c [T,512] and an up-projection weight [N*256,512], bf16 both, in
+    one launch (reference: ``kv_b_proj``, mla.py:405-413, 566-571).  Keys fp16 or bf16, values fp16; in memory a head's tokens
+    follow each other, a token's key in front of its value.  ``k_pe`` (bf16 [T,64] or [T,1,64]): comes back as contiguous fp16
+    [T,64], by the same launch where its rows are on 16-byte boundaries."""
+    if not kv_up_takes(kv_c, weight, num_heads):
+        raise ValueError("kv_up: bf16 kv_c [T,512] and weight [N*256,512] on the GPU, rows on 16-byte boundaries")
+    t, pe16, pe_args = kv_c.shape[0], None, (None, 0, None, 0)
+    if k_pe is not None:
+        k_pe = k_pe.reshape(t, D_ROPE)
+        if k_pe.dtype != torch.bfloat16 or k_pe.stride(1) != 1 or k_pe.stride(0) % 8 or k_pe.data_ptr() % 16 or t == 0:
+            pe16 = k_pe.to(torch.float16, memory_format=torch.contiguous_format)
+        else:
+            pe16 = torch.empty(t, D_ROPE, dtype=torch.float16, device=kv_c.device)
+            pe_args = (k_pe.data_ptr(), k_pe.stride(0), pe16.data_ptr(), D_ROPE)
+    kv = torch.empty(num_heads, t, 256, dtype=torch.float16, device=kv_c.device)
+    if t:
+        rc = _lib.load().mla_kv_up(kv_c.data_ptr(), kv_c.stride(0), weight.data_ptr(), weight.stride(0), t, num_heads, int(keys_f16),
+                                   kv.data_ptr(), 256, t * 256, *pe_args, _stream(kv_c))
+        _lib.check(rc, "mla_kv_up")
+    kv = kv.transpose(0, 1)
+    k_nope = kv[..., :128]
+    return k_nope if keys_f16 else k_nope.view(torch.bfloat16), kv[..., 128:], pe16
+
+
 # Tokens up to which the queries of a step are absorbed by this library's kernel; beyond, the work is a plain GEMM
 ABSORB_MAX_TOKENS = 256
 
@@ -850,6 +883,7 @@ def sparse_decode(q_nope: torch.Tensor, q_rope: torch.Tensor, nope_cache: torch.
 
 # ------------------------------------------------------------------------------------------------
 _PREFILL_KV_F16 = 16                                       # added to the output dtype code: k_nope, k_pe, v hold fp16
+_PREFILL_V_F16 = 32                                        # v alone does
 
 
 def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tensor, k_pe: torch.Tensor, v: torch.Tensor,
@@ -864,8 +898,8 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
     ``prev_out`` (fp32 [T,N,128]) / ``prev_lse`` (fp32 [T,N]): the result of an earlier call over OTHER keys of the same
     rows; the call then returns the attention over the union, i.e. what this attention followed by merge_attn_states
     (src/omni_npu/attention/ops.py:5-42) gives, in one launch.  ``out`` may be ``prev_out``.
-    k_nope, k_pe and v may all three be fp16 (a caller that makes them with an fp16 GEMM): both products then run on fp16
-    and the kernel skips the conversion of the value tiles it otherwise does (the queries stay bf16).
+    k_nope, k_pe and v may all three be fp16 (kv_up makes them): both products then run on fp16 and the kernel skips the
+    conversion of the value tiles it otherwise does (the queries stay bf16); or v alone, which saves the conversion only.
     ``pick`` (int32 [T, W] bits, see topk's mask; W even and wide enough for the longest sequence; no window, no earlier
     result): a token attends over the keys its bits name."""
     if window is not None and window < 1:
@@ -878,10 +912,13 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
             k_pe.shape != (k_nope.shape[0], 64) or out.shape != (t, n, 128):
         raise ValueError("prefill_varlen: shapes must be q_nope [T,N,128], q_pe [T,N,64], k_nope/v [Tk,N,128], k_pe [Tk,64]")
     kv_half = k_nope.dtype == torch.float16
-    for x, want in ((q_nope, torch.bfloat16), (q_pe, torch.bfloat16), (k_nope, None), (k_pe, k_nope.dtype), (v, k_nope.dtype)):
+    v_half = v.dtype == torch.float16
+    for x, want in ((q_nope, torch.bfloat16), (q_pe, torch.bfloat16), (k_nope, None), (k_pe, k_nope.dtype),
+                    (v, v.dtype if v_half else k_nope.dtype)):
         if x.dtype != (want or x.dtype) or x.dtype not in (torch.bfloat16, torch.float16) or x.stride(-1) != 1:
-            raise TypeError("prefill_varlen: bf16 queries, keys and values all bf16 or all fp16, with a contiguous last dim")
-    kv_code = _PREFILL_KV_F16 if kv_half else 0
+            raise TypeError("prefill_varlen: bf16 queries, keys and values all bf16 or all fp16 (or bf16 keys and fp16 values), "
+                            "with a contiguous last dim")
+    kv_code = _PREFILL_KV_F16 if kv_half else _PREFILL_V_F16 if v_half else 0
     if out.dtype not in _DT or out.stride(-1) != 1:
         raise TypeError("prefill_varlen: out must be bf16 or fp32")
     if cu_q.dtype != torch.int32 or cu_k.dtype != torch.int32 or cu_q.numel() != cu_k.numel() or \
