@@ -1,32 +1,63 @@
 // N-way merge of the split-KV partials of the decode kernels (src/omni_npu/attention/ops.py:109-141 semantics): the second
 // phase of mla_decode_bf16 / mla_decode_fp8 / dsa_sparse_decode_bf16 and the body of mla_splitkv_reduce.
-#include "decode_params.hpp"
+#include "merge_row.hpp"
 #include <type_traits>
 
 namespace mlahip {
 
 // N-way merge of the partials of the query rows (src/omni_npu/attention/ops.py:109-141), for the chunk layout written
-// by the split kernels (decode_v3.hip, decode_v3_fp8.hip).  The partials of sequence b are those of the chunks that hold blocks of it, numbered
-// chunk + b: the consecutive numbers between the two that the split kernel left in seg_ids (every chunk of the plan holds
-// at least one unit of work, so none in between is empty).  A wavefront merges kRedRows consecutive rows of one sequence
-// (lane l owns columns 8l..8l+7): it fetches the per-row records of up to kRedParts partials with scalar loads, then asks for the
-// partials and the latent vectors of the flagged dominant keys together before it uses any of them - the kernel is a
-// chain of dependent memory round trips, and this keeps the vector part of the chain at one.  (One row per wave keeps it
-// at four waves per SIMD; the gathers of the dominant keys' vectors are a third of its time.)
-// With many partials per sequence (few sequences, long contexts: up to 257 partials of one row) a single wavefront would
-// walk them in dozens of dependent round trips, so the kWide form gives a row to a whole workgroup of kWideWaves wavefronts
-// (eight while one workgroup per compute unit holds all rows, else four): wavefront w merges every kWideWaves-th partial,
-// sixteen per pass, and the running states are merged through LDS at the end.
-// With one chunk per sequence (large batches) a row has one partial, or two where a chunk border falls inside its
-// sequence: the kFew form then gives a wavefront four rows of two partials, a quarter of the wavefronts and rounds.
-// (four partials per pass in the one-wavefront form: 69 registers, seven wavefronts per SIMD, so the 8192 rows of the
-// headline batch are resident in one round; a row with five or eight partials takes a second pass.  Eight per pass - 121
-// registers, four wavefronts per SIMD, two rounds - measured 1 to 3 us slower per step on both shapes, five and six in
-// between)
-constexpr int kRedPartsNarrow = 4, kRedPartsWide = 16, kRedPartsFew = 2, kRedRowsFew = 4;
+// by the split kernels (decode_v3.hip, decode_rows.hip, decode_v3_fp8.hip).  The partials of sequence b are those of the chunks that
+// hold blocks of it, numbered chunk + b: the consecutive numbers between the two that the split kernel left in seg_ids (every
+// chunk of the plan holds at least one unit of work, so none in between is empty).  A wavefront owns a row, lane l columns
+// 8l .. 8l+7; the kernel is a chain of dependent memory round trips, the gathers of the dominant keys' vectors a third of its time.
+//  * mla_chunk_merge_kernel: a wavefront merges a row by itself (merge_row.hpp), its partials and their records asked for together.
+//  * kWide, many partials per sequence (few sequences, long contexts: up to 257 partials of one row): a single wavefront would
+//    walk them in dozens of dependent round trips, so a workgroup of kWideWaves wavefronts has the row (eight while one workgroup
+//    per compute unit holds all rows, else four): wavefront w merges every kWideWaves-th partial, sixteen per pass, and the running
+//    states are merged through LDS at the end.
+//  * kFew, one chunk per sequence (large batches), so one partial of a row, or two where a chunk border falls inside its
+//    sequence: four rows of two partials per wavefront, a quarter of the wavefronts and rounds.
+constexpr int kMergeParts = 4;                             // partials of a row that are asked for at once
+constexpr int kRedPartsWide = 16, kRedPartsFew = 2, kRedRowsFew = 4;
+
+__global__ __launch_bounds__(256) void mla_chunk_merge_kernel(const ChunkReduceParams p) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int r_max = p.max_q_len * p.num_heads;
+  // Workgroups go to the eight XCDs round-robin in launch order; every XCD takes a contiguous eighth of the rows, as the split
+  // kernels give every XCD a contiguous eighth of the chunks: a row's partials were written, and its neighbours' partials
+  // are being read, through the same part of the memory system (headline merge 17.1 -> 16.0 us, row lists 53.8 -> 52.3 us
+  // for split + merge).
+  int64_t wg_id = blockIdx.x;
+  if ((gridDim.x & 7) == 0) wg_id = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int64_t gw = wg_id * 4 + wave;
+  if (gw >= (int64_t)p.batch * r_max) return;
+  const int b = (int)(gw / r_max), row = (int)(gw - (int64_t)b * r_max);
+  int q0 = b * p.max_q_len, qlen = p.max_q_len;
+  if (p.qsl) { q0 = p.qsl[b]; qlen = p.qsl[b + 1] - q0; }
+  qlen = qlen < p.max_q_len ? qlen : p.max_q_len;
+  if (row >= qlen * p.num_heads) return;
+  const int id_first = p.seg_ids[2 * b], id_last = p.seg_ids[2 * b + 1];
+  // (an empty sequence has no partial and no numbers either)
+  const MergeRow r = {true, id_first, 1, p.seq_lens[b] > 0 && id_last >= id_first ? id_last - id_first + 1 : 0, row};
+  MergeAsked<kMergeParts> asked;
+  mrg_ask(p, r, 0, lane, asked);
+  float m = -INFINITY, tot = 0.f, a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  mrg_all(p, r, lane, asked, m, tot, a);
+  const int t_local = row / p.num_heads, head = row - t_local * p.num_heads;
+  const float inv = tot > 0.f ? 1.f / tot : 0.f;
+  bf16x8 o;
+#pragma unroll
+  for (int e = 0; e < 8; e++) o[e] = (__bf16)(a[e] * inv);
+  *(bf16x8*)(p.out + (int64_t)(q0 + t_local) * p.out_st + (int64_t)head * p.out_sh + lane * 8) = o;
+  if (p.lse_out && lane == 0)
+    p.lse_out[(int64_t)(q0 + t_local) * p.lse_st + head] = tot > 0.f ? __logf(tot) + m : -INFINITY;
+}
+
 template <bool kWide, bool kFew, int kWideWaves = 4>
 __global__ __launch_bounds__(kWide ? 64 * kWideWaves : 256) void mla_chunk_reduce_kernel(const ChunkReduceParams p) {
-  constexpr int kRedParts = kWide ? kRedPartsWide : (kFew ? kRedPartsFew : kRedPartsNarrow);
+  static_assert(kWide != kFew, "the plain form is a kernel of its own");
+  constexpr int kRedParts = kWide ? kRedPartsWide : kRedPartsFew;
   constexpr int kRedRows = kFew ? kRedRowsFew : 1;
   __shared__ float comb_ml[kWide ? 2 * kWideWaves : 1];            // wide: running maximum and sum of every wavefront
   __shared__ float comb_a[kWide ? kWideWaves * 64 * 8 : 1];        //       and their unnormalised rows
@@ -36,10 +67,7 @@ __global__ __launch_bounds__(kWide ? 64 * kWideWaves : 256) void mla_chunk_reduc
   const int groups = (r_max + kRedRows - 1) / kRedRows;     // row groups per sequence
   // (the wave number is made a scalar: everything derived from it, the addresses of the per-row records included, then
   // lives in scalar registers and is fetched with scalar loads)
-  // Workgroups go to the eight XCDs round-robin in launch order; every XCD takes a contiguous eighth of the rows, as the split
-  // kernels give every XCD a contiguous eighth of the chunks: a row's partials were written, and its neighbours' partials
-  // are being read, through the same part of the memory system (headline merge 17.1 -> 16.0 us, row lists 53.8 -> 52.3 us
-  // for split + merge).
+  // (rows per XCD as above)
   int64_t wg_id = blockIdx.x;
   if (!kWide && (gridDim.x & 7) == 0) wg_id = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   const int64_t gw_first = kWide ? (int64_t)blockIdx.x : wg_id * 4 + wave;
@@ -199,7 +227,7 @@ int launch_chunk_reduce(const ChunkReduceParams& p, hipStream_t stream) {
     hipLaunchKernelGGL((mla_chunk_reduce_kernel<false, true>), dim3((unsigned)((row_groups + 3) / 4)), dim3(256), 0, stream, p);
   } else {
     const int64_t row_groups = (int64_t)p.batch * r_max;
-    hipLaunchKernelGGL((mla_chunk_reduce_kernel<false, false>), dim3((unsigned)((row_groups + 3) / 4)), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(mla_chunk_merge_kernel, dim3((unsigned)((row_groups + 3) / 4)), dim3(256), 0, stream, p);
   }
   return check_launch("mla_chunk_reduce_kernel");
 }

@@ -7,103 +7,58 @@
 // The unfused path writes o [N,T,512], runs a batched GEMM into [N,T,V], transposes that into [T, N*V] and copies it
 // into the caller's output: four launches and three round trips through memory for 2 MB of result.
 //
-// One workgroup = one head and a run of tokens.  Its 16 wavefronts first ask for the head's W_UV (512 x 128 bf16 =
-// 128 KiB) as global -> LDS copies, then merge the partials of the tokens' rows (the copies land underneath).  With many
-// tokens a wavefront merges ONE row; with few, 2 to 16 wavefronts share a row's partials (each takes every 2nd to 16th)
-// and add their states up through LDS, pairs of wavefronts at a time, in an order that depends on the shape only: the
-// kernel is a chain of round trips, and sharing keeps it as long for 64 partials of a row as for four (one request of 1k
-// keys under a plan for 64 chunks: 27 us of separate merge + 10 of GEMM + a copy -> 9 us; 128k keys in 256 partials: 18 + 10
-// + 4 -> 15 us).  The
-// bf16 rows go into a 16-row LDS tile, and four wavefronts multiply the tile with W_UV out of LDS: W^T is the
-// first MFMA operand (32 output columns per wavefront), read with transposed LDS reads exactly like V^T in the decode
-// kernel, the merged rows are the second operand, so a lane ends up with four consecutive output columns of one token.
+// One workgroup = one head and a run of tokens, sixteen wavefronts.  The head's W_UV (512 x 128 bf16 = 128 KiB) comes into LDS by
+// global -> LDS copies, the rows of up to sixteen tokens are merged, rounded to bf16 and put beside it, and eight wavefronts
+// multiply them: W^T, read with transposed LDS reads, is the first MFMA operand (16 output columns per wavefront), the rows are the
+// second, and a lane ends up with four consecutive columns of one token.
+//
+// What bounds it: a chain of round trips (which partials, their records and numbers, the latent vectors of the flagged keys) beside
+// the copies of W_UV.  A row's partials and their records are asked for together: lane i holds partial i's record, the
+// weights of up to 64 partials are worked out at once, and no partial waits for its record.
+//  * kFew (few tokens): wavefronts 8..15 bring W_UV, wavefronts 0..7 share the rows, up to eight of them a row, and leave their
+//    sums in LDS, from where a row is put together column by column.  A wavefront's loads return in order, so where every
+//    wavefront brought an eighth of W_UV and then merged, every merge waited for W_UV.
+//    Heads too few for the compute units are cut into two or four column parts, each with its part of W_UV: a CU misses
+//    about 11 bytes a clock, so 256 partials of 128 rows through 128 CUs took 20 000 clocks.
+//  * else a wavefront merges a row by itself, sixteen tokens a pass, and asks for its row of the next pass before this one's product.
+// An XCD takes neighbouring heads, whose rows lie in different channels of its L2 (every eighth head: the same ones).
+// us of the launch before -> now: one request of 1k keys x 16 heads 6.7 -> 4.4; 64 x 128 heads, five partials a row 16.6 -> 15.0; per
+// layer: one user 20.3 -> 18.3, 64 at 4k-8k 146.5 -> 145.0, with sink and window 112.3 -> 110.5, sparse 131.5 -> 130, 60k keys x 64 heads
+// 49 -> 45.6 (cut into columns).
 #include "mla_common.hpp"
-#include "decode_params.hpp"
+#include "merge_row.hpp"
 
 namespace mlahip {
 namespace {
 
-constexpr int kVupTok = 16;                     // tokens per pass: one per wavefront
+constexpr int kVupTok = 16;                     // tokens per pass
 constexpr int kVupV = 128;                      // v_head_dim
 constexpr int kVupWB = kDNope * kVupV * 2;      // 131072: W_UV of one head, row c at c * 256
-constexpr int kVupOB = kVupTok * kDNope * 2;    // 16384: merged rows of one pass, 1 KiB each
-constexpr int kVupFlagOff = kVupWB + kVupOB;    // one int per token of the pass: its row is valid
-constexpr int kVupStateOff = kVupFlagOff + 64;  // eight (maximum, sum) pairs of an exchange between wavefronts
-constexpr int kVupLdsB = kVupStateOff + 64;
-constexpr int kVupParts = 6;                    // partials of a row asked for together
-constexpr int kVupAhead = 4;                    // GEMM steps whose operands are requested ahead (at most 4: the wait ladder)
+constexpr int kMergeRowOff = kVupWB + 16384;      // kFew: the eight wavefronts' sums (fp32, 2 KiB each) in front of the merged rows
+constexpr int kVupPairOff = kMergeRowOff + 8192;  // kFew: the sums' (maximum, weight) pairs
+constexpr int kVupFlagOff = kVupPairOff + 64;   // one int per token of the pass: its row is valid
+constexpr int kVupLdsB = kVupFlagOff + 64;
+constexpr int kVupAlone = 16;                   // partials of a row that one wavefront asks for at once
+constexpr int kVupAhead = 4;                    // product steps whose operands are requested ahead (at most 4: the wait ladder)
 
 __device__ __forceinline__ int vup_wave_sum(int v) {
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
   return v;
 }
-
-// Merge of every `step`-th partial, from the `first`-th on, of row `row` of sequence b (all arguments wave-uniform), lane l
-// owning columns 8l .. 8l+7.  Same bookkeeping as mla_chunk_reduce_kernel: the partials of a sequence are the consecutive
-// numbers between the two the split kernel left in seg_ids.
-__device__ __forceinline__ void vup_merge_row(const ChunkReduceParams& p, int b, int row, int lane, int first, int step,
-                                              float& m, float& tot, float (&a)[8]) {
-  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-  const int r_max = p.max_q_len * p.num_heads;
-  const int id_first = p.seg_ids[2 * b], id_last = p.seg_ids[2 * b + 1];
-  if (p.seq_lens[b] <= 0) return;
-  int c = id_first + first;
-  while (c <= id_last) {
-    int64_t part[kVupParts];
-    int np = 0;
-#pragma unroll
-    for (int q = 0; q < kVupParts; q++) {
-      part[q] = c <= id_last ? (int64_t)c * r_max + row : 0;
-      if (c <= id_last) { np++; c += step; }
-    }
-    // records by scalar loads (uniform addresses), then the partials and the latent vectors of the flagged dominant
-    // keys in one vector round trip
-    float lse[kVupParts], cs[kVupParts];
-    const __bf16* cp[kVupParts];
-#pragma unroll
-    for (int q = 0; q < kVupParts; q++) {
-      const bool on = q < np;
-      lse[q] = on ? p.lse_part[part[q]] : -INFINITY;
-      cs[q] = on ? p.corr_scale[part[q]] : 0.f;
-      cp[q] = p.corr_row[part[q]];
-      if (lse[q] == INFINITY || lse[q] == -INFINITY) cs[q] = 0.f;
-    }
-    h8 v[kVupParts];
-    bf16x8 kv[kVupParts];
-#pragma unroll
-    for (int q = 0; q < kVupParts; q++) {
-      v[q] = *(const h8*)(p.o_part + part[q] * kDNope + lane * 8);
-      if (cs[q] != 0.f) kv[q] = *(const bf16x8*)(cp[q] + lane * 8);
-    }
-#pragma unroll
-    for (int q = 0; q < kVupParts; q++) {
-      const float l = lse[q];
-      if (l == INFINITY || l == -INFINITY) continue;
-      const float mn = fmaxf(m, l);
-      const float so = __expf(m - mn), w = __expf(l - mn);
-      m = mn;
-      tot = tot * so + w;
-#pragma unroll
-      for (int e = 0; e < 8; e++) a[e] = a[e] * so + (float)v[q][e] * w;
-      if (cs[q] != 0.f) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) a[e] += (float)kv[q][e] * (w * cs[q]);
-      }
-    }
-  }
-}
-
 }  // namespace
 
 struct ReduceVupParams {
   ChunkReduceParams r;                 // r.out: [T, N * 128] through (out_st, out_sh)
   const __bf16* w_uv; int64_t w_sn, w_sk;   // W_UV [N, 512, 128]: head stride, row stride (elements)
-  int32_t num_tokens, passes;          // a workgroup handles passes * (16 / share) consecutive tokens
-  int32_t share_log2;                  // log2 of the wavefronts that share a row
+  int32_t num_tokens, passes;          // a workgroup handles 16 passes consecutive tokens; kFew: 8 >> toks_log2
+  int32_t toks_log2, share_log2;       // kFew: 2^share_log2 wavefronts share a row (toks_log2 of them or one)
 };
 
+// kCols: output columns of a workgroup, 128 or (kFew) 64 or 32: heads too few for the compute units are cut
+template <bool kFew, int kCols>
 __global__ __launch_bounds__(1024) void mla_reduce_vup_kernel(const ReduceVupParams pp) {
+  constexpr int kParts = kVupV / kCols, kWRow = 2 * kCols;                  // column parts of a head; bytes of a row of W in LDS
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const ChunkReduceParams& p = pp.r;
   const int lane = threadIdx.x & 63;
@@ -115,173 +70,227 @@ __global__ __launch_bounds__(1024) void mla_reduce_vup_kernel(const ReduceVupPar
     const int lin = blockIdx.x + gridDim.x * blockIdx.y;
     const int j = lin >> 3;
     tb = j % gridDim.x;
-    head = (j / gridDim.x) * 8 + (lin & 7);
+    head = (lin & 7) * (gridDim.y >> 3) + j / gridDim.x;
   }
+  const int part = kParts == 1 ? 0 : tb & (kParts - 1);
+  tb /= kParts;
   const uint32_t lds0 = lds_addr_of(lds);
 
-  // ---- W_UV[head] -> LDS: 128 copy instructions of 1 KiB (4 rows of 256 B), 8 per wavefront.  Row c keeps its 16-byte
-  // granule g at position g ^ 4*(c & 3): the transposed reads below fetch four consecutive rows per 16 lanes, and the
-  // XOR spreads those rows over the banks. ----
-  {
-    const __bf16* w = pp.w_uv + (int64_t)head * pp.w_sn;
-    const int r = lane >> 4, pos = lane & 15;
+  // W_UV[head] -> LDS: copy instructions of 1 KiB (4, 8 or 16 rows).  Row c keeps its 16-byte granule g at position g ^ w_swz(c):
+  // the lanes 0..31 (32..63) of a transposed read below fetch 32 bytes of four consecutive rows and of the four rows eight further on,
+  // and the XOR puts the eight pieces into different banks.
+  auto w_swz = [](int c) {
+    return kCols == 128 ? (c & 3) << 2 | (c >> 2 & 2) : kCols == 64 ? (c & 2) | (c >> 1 & 4) : c >> 2 & 2;
+  };
+  auto copy_w = [&](int from, int count) {
+    const __bf16* w = pp.w_uv + (int64_t)head * pp.w_sn + part * kCols;
+    constexpr int kLanes = kWRow / 16;                                      // lanes per row
+    const int r = lane / kLanes, pos = lane % kLanes;
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int bi = wave * 8 + i;
-      const int c = 4 * bi + r;
-      dma16_v(w + (int64_t)c * pp.w_sk + ((pos ^ (r << 2)) << 3), lds0 + bi * 1024);
+    for (int i = 0; i < count; i++) {
+      const int bi = from + i, c = 64 / kLanes * bi + r;
+      dma16_v(w + (int64_t)c * pp.w_sk + ((pos ^ w_swz(c)) << 3), lds0 + bi * 1024);
     }
-  }
+  };
+  // Token t of this head: its row's partials first, first + step, ..., the odd column parts' from the last one backwards: two workgroups
+  // that need the same partials then bring one half each into their XCD's L2 and find the other there
+  auto row_of = [&](int t, int first, int step) {
+    MergeRow r = {t < pp.num_tokens, 0, step, 0, 0};
+    if (!r.valid) return r;
+    int b, t_local, qlen;
+    if (p.qsl) {
+      int cnt = 0;
+      for (int i = lane; i <= p.batch; i += 64) cnt += p.qsl[i] <= t ? 1 : 0;
+      b = __builtin_amdgcn_readfirstlane(vup_wave_sum(cnt)) - 1;
+      b = b < 0 ? 0 : (b >= p.batch ? p.batch - 1 : b);
+      const int q0 = p.qsl[b];
+      qlen = p.qsl[b + 1] - q0;
+      t_local = t - q0;
+    } else {
+      b = p.max_q_len == 1 ? t : t / p.max_q_len;
+      t_local = t - b * p.max_q_len;
+      qlen = p.max_q_len;
+      if (b >= p.batch) { r.valid = false; return r; }
+    }
+    qlen = qlen < p.max_q_len ? qlen : p.max_q_len;
+    r.valid = t_local >= 0 && t_local < qlen;
+    // the partials of a sequence are the consecutive numbers between the two the split kernel left in seg_ids
+    const int id_first = p.seg_ids[2 * b], id_last = p.seg_ids[2 * b + 1], len = p.seq_lens[b];
+    if (!r.valid || len <= 0) return r;
+    r.row = t_local * p.num_heads + head;
+    const int all = id_last - id_first + 1;
+    r.n = first < all ? (step == 1 ? all - first : (all - first + step - 1) / step) : 0;
+    r.id0 = (part & 1) ? id_last - first : id_first + first;
+    r.step = (part & 1) ? -step : step;
+    return r;
+  };
+  // Merged rows, bf16, at rows_off: granule g of row r at position g ^ r, so that 16 rows read at the same g hit different banks
+  constexpr int kRowsOff = kFew ? kMergeRowOff : kVupWB;
+  auto whole_row = [&](int slot, bool valid, float tot, const float (&a)[8]) {
+    const float inv = tot > 0.f ? 1.f / tot : 0.f;
+    bf16x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; e++) o[e] = (__bf16)(a[e] * inv);
+    *(bf16x8*)(lds + kRowsOff + slot * 1024 + ((lane ^ slot) << 4)) = o;
+    if (lane == 0) *(int*)(lds + kVupFlagOff + slot * 4) = valid ? 1 : 0;
+  };
+  // out[t, head, 16 w .. 16 w + 15] (of the workgroup's columns) for the pass's tokens first .. first + toks - 1: wavefronts 0..7 (kCols
+  // fewer: 0..3, 0..1), sixteen MFMAs each
+  auto product = [&](int first, int toks) {
+    const int l16 = lane & 15, g = lane >> 4;
+    const int slot = kFew ? l16 & 7 : l16;                    // (kFew: eight rows at most; the others repeat them)
+    const int c0 = 8 * g + (l16 >> 2);
+    const uint32_t a_lo = lds0 + c0 * kWRow + (((2 * wave + ((l16 & 3) >> 1)) ^ w_swz(c0)) << 4) + (l16 & 1) * 8;
+    const uint32_t a_hi = a_lo + 8 * 32 * kWRow;              // the offset field holds eight steps of up to 8 KiB
+    const uint32_t b_ad = lds0 + kRowsOff + slot * 1024 + ((g ^ slot) << 4);
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    // Operands are read with hand-placed LDS instructions kVupAhead steps ahead of the MFMA that consumes them and explicit waits
+    // (three reads per step, returned in order).
+    constexpr int D = kVupAhead;
+    bf16x4 wl[D], wh[D];
+    bf16x8 ob[D];
+#define VUP_READ(s, kk)                                                                                                  \
+    do {                                                                                                                 \
+      asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(wl[s]) : "v"((kk) < 8 ? a_lo : a_hi), "i"(((kk) & 7) * 32 * kWRow)); \
+      asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(wh[s]) : "v"((kk) < 8 ? a_lo : a_hi), "i"(((kk) & 7) * 32 * kWRow + 4 * kWRow)); \
+      asm volatile("ds_read_b128 %0, %1" : "=v"(ob[s]) : "v"(b_ad ^ (uint32_t)((kk) << 6)));                                \
+    } while (0)
+#pragma unroll
+    for (int i = 0; i < D; i++) VUP_READ(i, i);
+#pragma unroll
+    for (int kk = 0; kk < 16; kk++) {
+      const int younger = (15 - kk) < (D - 1) ? (15 - kk) : (D - 1);      // steps asked for after step kk
+      if (younger >= 3) asm volatile("s_waitcnt lgkmcnt(9)" : "+v"(wl[kk % D]), "+v"(wh[kk % D]), "+v"(ob[kk % D]));
+      else if (younger == 2) asm volatile("s_waitcnt lgkmcnt(6)" : "+v"(wl[kk % D]), "+v"(wh[kk % D]), "+v"(ob[kk % D]));
+      else if (younger == 1) asm volatile("s_waitcnt lgkmcnt(3)" : "+v"(wl[kk % D]), "+v"(wh[kk % D]), "+v"(ob[kk % D]));
+      else asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(wl[kk % D]), "+v"(wh[kk % D]), "+v"(ob[kk % D]));
+      const bf16x8 wa = __builtin_shufflevector(wl[kk % D], wh[kk % D], 0, 1, 2, 3, 4, 5, 6, 7);
+      acc[kk & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, ob[kk % D], acc[kk & 1], 0, 0, 0);
+      if (kk + D < 16) VUP_READ(kk % D, kk + D);
+    }
+#undef VUP_READ
+    if (l16 < toks && *(const int*)(lds + kVupFlagOff + l16 * 4) != 0) {
+      bf16x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; e++) v[e] = (__bf16)(acc[0][e] + acc[1][e]);
+      *(bf16x4*)(p.out + (int64_t)(first + l16) * p.out_st + (int64_t)head * p.out_sh + part * kCols + wave * 16 + 4 * g) = v;
+    }
+  };
 
-  const int h32 = lane & 31, half = lane >> 5;
-  const int share = 1 << pp.share_log2, toks = kVupTok >> pp.share_log2;      // wavefronts per row, tokens per pass
-  const int sub = wave & (share - 1), slot = wave >> pp.share_log2;           // this wavefront's part and row of the pass
-  for (int pass = 0; pass < pp.passes; pass++) {
-    // ---- token t, this head ----
-    const int t = (tb * pp.passes + pass) * toks + slot;
-    bool valid = t < pp.num_tokens;
-    int b = 0, t_local = 0;
-    if (valid) {
-      int qlen;
-      if (p.qsl) {
-        int cnt = 0;
-        for (int i = lane; i <= p.batch; i += 64) cnt += p.qsl[i] <= t ? 1 : 0;
-        b = __builtin_amdgcn_readfirstlane(vup_wave_sum(cnt)) - 1;
-        b = b < 0 ? 0 : (b >= p.batch ? p.batch - 1 : b);
-        const int q0 = p.qsl[b];
-        qlen = p.qsl[b + 1] - q0;
-        t_local = t - q0;
+  if constexpr (kFew) {
+    const int share = 1 << pp.share_log2, toks = 8 >> pp.toks_log2;         // wavefronts per row (1, 2, 4, 8), tokens
+    if (wave >= 8) {
+      copy_w((wave - 8) * (16 / kParts), 16 / kParts);
+    } else if (wave < toks * share) {
+      const int sub = wave & (share - 1), slot = wave >> pp.share_log2;
+      const MergeRow r = row_of(tb * toks + slot, sub, share);
+      float m = -INFINITY, tot = 0.f, a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      MergeAsked<kVupAlone> asked;
+      mrg_ask(p, r, 0, lane, asked);
+      mrg_all(p, r, lane, asked, m, tot, a);
+      if (share == 1) {
+        whole_row(slot, r.valid, tot, a);
       } else {
-        b = t / p.max_q_len;
-        t_local = t - b * p.max_q_len;
-        qlen = p.max_q_len;
-        valid = b < p.batch;
+        *(f32x4*)(lds + kVupWB + wave * 2048 + lane * 16) = f32x4{a[0], a[1], a[2], a[3]};
+        *(f32x4*)(lds + kVupWB + wave * 2048 + 1024 + lane * 16) = f32x4{a[4], a[5], a[6], a[7]};
+        if (lane == 0) {
+          *(f32x2*)(lds + kVupPairOff + wave * 8) = f32x2{m, tot};
+          if (sub == 0) *(int*)(lds + kVupFlagOff + slot * 4) = r.valid ? 1 : 0;
+        }
       }
-      qlen = qlen < p.max_q_len ? qlen : p.max_q_len;
-      valid = valid && t_local >= 0 && t_local < qlen;
     }
-    float m = -INFINITY, tot = 0.f, a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (valid) vup_merge_row(p, b, t_local * p.num_heads + head, lane, sub, share, m, tot, a);
-    // the states of the wavefronts that share a row, halves added up until one is left (the exchange uses the row tile,
-    // which is written after it: 8 states of 2 KiB, and the flags' place behind it for their maxima and sums)
-    for (int s = share >> 1; s >= 1; s >>= 1) {
-      const int at = slot * s + (sub - s);
-      if (sub >= s && sub < 2 * s) {
-        *(f32x4*)(lds + kVupWB + at * 2048 + lane * 16) = f32x4{a[0], a[1], a[2], a[3]};
-        *(f32x4*)(lds + kVupWB + at * 2048 + 1024 + lane * 16) = f32x4{a[4], a[5], a[6], a[7]};
-        if (lane == 0) *(f32x2*)(lds + kVupStateOff + at * 8) = f32x2{m, tot};
-      }
+    if (share > 1) {
+      // four wavefronts put a row together, two columns per lane: lane l of quarter q has columns 8 (16 q + l / 4) + 2 (l % 4) and the
+      // next, which lie in the lower or upper half of the 32 bytes that lane 16 q + l / 4 of each sharing wavefront wrote
       lds_barrier();
-      if (sub < s) {
-        const int from = slot * s + sub;
-        const f32x2 mt = *(const f32x2*)(lds + kVupStateOff + from * 8);
-        const f32x4 a0 = *(const f32x4*)(lds + kVupWB + from * 2048 + lane * 16);
-        const f32x4 a1 = *(const f32x4*)(lds + kVupWB + from * 2048 + 1024 + lane * 16);
-        const float mn = fmaxf(m, mt[0]);
-        const float f0 = m == -INFINITY ? 0.f : __expf(m - mn), f1 = mt[0] == -INFINITY ? 0.f : __expf(mt[0] - mn);
-        m = mn;
-        tot = tot * f0 + mt[1] * f1;
+      const int slot = wave >> 2, owner = (wave & 3) * 16 + (lane >> 2), pair = lane & 3;
+      if (slot < toks) {
+        const char* from = lds + kVupWB + slot * share * 2048 + (pair >> 1) * 1024 + owner * 16 + (pair & 1) * 8;
+        const char* mt = lds + kVupPairOff + slot * share * 8;
+        float mx = -INFINITY;
+        f32x2 x[8], pr[8];
 #pragma unroll
-        for (int e = 0; e < 4; e++) { a[e] = a[e] * f0 + a0[e] * f1; a[4 + e] = a[4 + e] * f0 + a1[e] * f1; }
+        for (int i = 0; i < 8; i++)
+          if (i < share) {
+            pr[i] = *(const f32x2*)(mt + i * 8);
+            x[i] = *(const f32x2*)(from + i * 2048);
+            mx = fmaxf(mx, pr[i][0]);
+          }
+        float sum = 0.f, c0 = 0.f, c1 = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+          if (i < share) {
+            const float f = pr[i][0] == -INFINITY ? 0.f : __expf(pr[i][0] - mx);
+            sum += pr[i][1] * f;
+            c0 += x[i][0] * f;
+            c1 += x[i][1] * f;
+          }
+        const float inv = sum > 0.f ? 1.f / sum : 0.f;
+        const bf16x2 o = {(__bf16)(c0 * inv), (__bf16)(c1 * inv)};
+        *(bf16x2*)(lds + kRowsOff + slot * 1024 + ((owner ^ slot) << 4) + pair * 4) = o;
       }
-      lds_barrier();
-    }
-    // The bf16 row goes to LDS in the order the MFMA wants its contraction index: within every 16 columns the first
-    // granule holds columns {0..3, 8..11}, the second {4..7, 12..15} (the transposed reads of W deliver them in that
-    // order), and granule g of row r sits at position g ^ r so that 16 rows read at the same g hit different banks.
-    if (sub == 0) {
-      const float inv = tot > 0.f ? 1.f / tot : 0.f;
-      bf16x4 lo, hi;
-#pragma unroll
-      for (int e = 0; e < 4; e++) { lo[e] = (__bf16)(a[e] * inv); hi[e] = (__bf16)(a[4 + e] * inv); }
-      char* rowp = lds + kVupWB + slot * 1024 + (lane & 1) * 8;
-      const int g0 = (lane >> 1) * 2;
-      *(bf16x4*)(rowp + (((g0) ^ slot) << 4)) = lo;
-      *(bf16x4*)(rowp + (((g0 + 1) ^ slot) << 4)) = hi;
-      if (lane == 0) *(int*)(lds + kVupFlagOff + slot * 4) = valid ? 1 : 0;
     }
     MLA_WAIT_VMCNT(0);                                        // this wavefront's share of W_UV has landed
     lds_barrier();
-
-    // ---- out[t, head, 32 w .. 32 w + 31] for the pass's 16 tokens: wavefronts 0..3, 32 MFMAs each ----
-    if (wave < 4) {
-      const int g16 = lane >> 4, j16 = lane & 15;
-      const int c_row = 4 * (g16 >> 1) + (j16 >> 2);          // row inside a group of 8 (+8 for the second read)
-      const int v_cl = 2 * (g16 & 1) + ((j16 & 3) >> 1);      // granule inside this wavefront's 32 columns
-      const uint32_t a_off = (uint32_t)(c_row * 256 + (((wave * 4 + v_cl) ^ ((j16 >> 2) << 2)) << 4) + (j16 & 1) * 8);
-      const int tr = h32 & 15;                                // token row of the tile (lanes 16..31 repeat rows 0..15)
-      const uint32_t b_off = (uint32_t)(kVupWB + tr * 1024 + ((half ^ tr) << 4));
-      f32x16 acc;
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[r] = 0.f;
-      // Operands are read with hand-placed LDS instructions kVupAhead steps ahead of the MFMA that consumes them and
-      // explicit waits (three reads per step, returned in order): left to itself the compiler reads, waits and
-      // multiplies one step at a time and pays the LDS latency 32 times.
-      {
-        const uint32_t a_lo = lds0 + a_off, a_hi = a_lo + 16 * 4096;     // the offset field holds 16 steps of 4 KiB
-        const uint32_t b_ad = lds0 + b_off;
-        constexpr int D = kVupAhead;
-        bf16x4 wl[D], wh[D];
-        bf16x8 ob[D];
-#define VUP_READ(slot, kk)                                                                                             \
-        do {                                                                                                           \
-          asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(wl[slot]) : "v"((kk) < 16 ? a_lo : a_hi), "i"(((kk) & 15) * 4096)); \
-          asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(wh[slot]) : "v"((kk) < 16 ? a_lo : a_hi), "i"(((kk) & 15) * 4096 + 2048)); \
-          asm volatile("ds_read_b128 %0, %1" : "=v"(ob[slot]) : "v"(b_ad ^ (uint32_t)((kk) << 5)));                      \
-        } while (0)
-#pragma unroll
-        for (int i = 0; i < D; i++) VUP_READ(i, i);
-#pragma unroll
-        for (int kk = 0; kk < 32; kk++) {
-          const int younger = (31 - kk) < (D - 1) ? (31 - kk) : (D - 1);      // steps asked for after step kk
-          if (younger >= 3) asm volatile("s_waitcnt lgkmcnt(9)" : "+v"(wl[kk % D]), "+v"(wh[kk % D]), "+v"(ob[kk % D]));
-          else if (younger == 2) asm volatile("s_waitcnt lgkmcnt(6)" : "+v"(wl[kk % D]), "+v"(wh[kk % D]), "+v"(ob[kk % D]));
-          else if (younger == 1) asm volatile("s_waitcnt lgkmcnt(3)" : "+v"(wl[kk % D]), "+v"(wh[kk % D]), "+v"(ob[kk % D]));
-          else asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(wl[kk % D]), "+v"(wh[kk % D]), "+v"(ob[kk % D]));
-          const bf16x8 wa = __builtin_shufflevector(wl[kk % D], wh[kk % D], 0, 1, 2, 3, 4, 5, 6, 7);
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wa, ob[kk % D], acc, 0, 0, 0);
-          if (kk + D < 32) VUP_READ(kk % D, kk + D);
-        }
-#undef VUP_READ
-      }
-      const int tt = (tb * pp.passes + pass) * toks + tr;
-      const bool ok = h32 < toks && *(const int*)(lds + kVupFlagOff + tr * 4) != 0;
-      if (ok) {
-        __bf16* o = p.out + (int64_t)tt * p.out_st + (int64_t)head * p.out_sh + wave * 32 + 4 * half;
-#pragma unroll
-        for (int q4 = 0; q4 < 4; q4++) {
-          bf16x4 v;
-#pragma unroll
-          for (int e = 0; e < 4; e++) v[e] = (__bf16)acc[q4 * 4 + e];
-          *(bf16x4*)(o + q4 * 8) = v;
-        }
-      }
+    if (wave < 8 / kParts) product(tb * toks, toks);
+  } else {
+    const int first = tb * pp.passes * kVupTok;
+    MergeRow r = row_of(first + wave, 0, 1);
+    MergeAsked<6> asked;
+    copy_w(wave * 8, 4);
+    mrg_ask(p, r, 0, lane, asked);
+    copy_w(wave * 8 + 4, 4);
+    for (int pass = 0; pass < pp.passes; pass++) {
+      float m = -INFINITY, tot = 0.f, a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      MergeRow next = {false, 0, 1, 0, 0};
+      if (pass + 1 < pp.passes) next = row_of(first + (pass + 1) * kVupTok + wave, 0, 1);
+      mrg_all(p, r, lane, asked, m, tot, a);
+      whole_row(wave, r.valid, tot, a);
+      if (pass == 0) MLA_WAIT_VMCNT(0);                       // this wavefront's share of W_UV has landed
+      r = next;
+      mrg_ask(p, r, 0, lane, asked);
+      lds_barrier();
+      if (wave < 8) product(first + pass * kVupTok, kVupTok);
+      lds_barrier();                                          // the rows are written anew by the next pass
     }
-    lds_barrier();                                            // the row tile is rewritten by the next pass
   }
+}
+
+static auto* vup_kernels() {
+  static constexpr void (*kerns[4])(const ReduceVupParams) = {mla_reduce_vup_kernel<false, 128>, mla_reduce_vup_kernel<true, 128>,
+                                                              mla_reduce_vup_kernel<true, 64>, mla_reduce_vup_kernel<true, 32>};
+  return kerns;
 }
 
 int launch_reduce_vup(const ChunkReduceParams& r, const void* w_uv, int64_t w_stride_n, int64_t w_stride_k,
                       int32_t num_tokens, hipStream_t stream) {
-  const int rc = ensure_dynamic_lds((const void*)mla_reduce_vup_kernel, kVupLdsB, "mla_splitkv_reduce_vup");
-  if (rc != MLA_OK) return rc;
+  auto* const kerns = vup_kernels();
+  for (int i = 0; i < 4; i++) {
+    const int rc = ensure_dynamic_lds((const void*)kerns[i], kVupLdsB, "mla_splitkv_reduce_vup");
+    if (rc != MLA_OK) return rc;
+  }
   ReduceVupParams pp;
   pp.r = r;
   pp.w_uv = (const __bf16*)w_uv; pp.w_sn = w_stride_n; pp.w_sk = w_stride_k;
   pp.num_tokens = num_tokens;
-  // About one workgroup per compute unit.  As many wavefronts share a row as leave no more workgroups than compute units
-  // (16 tokens per pass and workgroup where a row has a wavefront to itself), but not more than the row has partials.
+  // About one workgroup per compute unit.  Where a workgroup of eight tokens or fewer leaves no more workgroups than compute units, as
+  // few tokens as that allows; rows of more than kVupAlone partials are then shared by the wavefronts that have none.
   const int64_t parts = r.batch > 0 ? (r.num_chunks + r.batch - 1) / r.batch + 1 : 1;
+  const auto groups = [&](int64_t toks) { return ((int64_t)num_tokens + toks - 1) / toks; };
+  const bool few = groups(8) * r.num_heads <= kPlanCUs;
   int lg = 0;
-  while (lg < 4 && (2 << lg) <= parts && (((int64_t)num_tokens + (kVupTok >> (lg + 1)) - 1) / (kVupTok >> (lg + 1))) * r.num_heads <= 256) lg++;
-  const int toks = kVupTok >> lg;
-  const int64_t blocks = ((int64_t)num_tokens + toks - 1) / toks;
-  int64_t passes = (blocks * r.num_heads + 255) / 256;
+  while (few && lg < 3 && groups(8 >> (lg + 1)) * r.num_heads <= kPlanCUs) lg++;
+  const int64_t blocks = groups(few ? 8 >> lg : kVupTok);
+  int64_t passes = few ? 1 : (blocks * r.num_heads + kPlanCUs - 1) / kPlanCUs;
   passes = passes < 1 ? 1 : (passes > 64 ? 64 : passes);
   pp.passes = (int32_t)passes;
-  pp.share_log2 = lg;
+  pp.toks_log2 = lg;
+  pp.share_log2 = parts > kVupAlone ? lg : 0;
   const int64_t tbs = (blocks + passes - 1) / passes;
-  hipLaunchKernelGGL(mla_reduce_vup_kernel, dim3((unsigned)tbs, (unsigned)r.num_heads), dim3(1024), kVupLdsB, stream, pp);
+  int cut = 0;                                                // log2 of the column parts
+  while (few && cut < 2 && tbs * r.num_heads << (cut + 1) <= kPlanCUs) cut++;
+  const dim3 grid((unsigned)(tbs << cut), (unsigned)r.num_heads);
+  hipLaunchKernelGGL(kerns[few ? 1 + cut : 0], grid, dim3(1024), kVupLdsB, stream, pp);
   return check_launch("mla_reduce_vup_kernel");
 }
 

@@ -154,3 +154,13 @@ def test_chunk_plan_and_shared_rows_at_their_edges(dev, batch, heads, q_len, lo,
 ])
 def test_row_groups_at_their_edges(dev, batch, heads, q_len, lo, hi, splits):
     test_fused_merge_and_up_projection(dev, batch, heads, q_len, lo, hi, splits)
+
+
+@pytest.mark.parametrize("batch,heads,q_len,lo,hi,splits", [
+    (1, 128, 1, 5000, 5000, 256), (1, 64, 1, 9000, 9000, 256), (1, 16, 1, 700, 700, 64),   # two, four column parts
+    (1, 8, 1, 70000, 70000, 1100),                            # 1024 partials of a row: two rounds of records per wavefront
+    (3, 20, 1, 4000, 6000, 40), (2, 33, 2, 2000, 3000, 30),   # heads that are no multiple of eight; shared rows, two tokens per workgroup
+    (1, 128, 2, 40, 40, 1), (40, 128, 1, 300, 500, 2),        # rows of one partial; two passes per workgroup
+])
+def test_column_parts_and_long_rows(dev, batch, heads, q_len, lo, hi, splits):
+    test_fused_merge_and_up_projection(dev, batch, heads, q_len, lo, hi, splits)
