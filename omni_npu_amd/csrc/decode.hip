@@ -85,7 +85,7 @@ static int decode_split_impl(const void* q_nope, int64_t qn_stride_t, int64_t qn
   v.win_skip = win_skip; v.win_sink = win_sink; v.win_size = win_size;
   v.new_c = (const __bf16*)new_c; v.new_c_st = new_c_stride; v.new_r = (const __bf16*)new_r; v.new_r_st = new_r_stride;
   v.new_slots = new_slots;
-  const PlanForm form = plan_form(batch, num_splits, r_max);
+  const PlanForm form = plan_form(batch, num_splits, r_max, !fp8);
   v.num_chunks = form.chunks;
   if (fp8) return launch_decode_v3_fp8(v, form.rg, stream);
   return launch_decode_v3(v, sparse_rows != nullptr, form.rg, stream);

@@ -66,19 +66,22 @@ constexpr int kPlanCUs = 256;                              // MI355X
 // take the forms that leave the missing rows out.  For more rows, batch * num_splits chunks of at least 256 keys each that do
 // not fill the CUs mean that the contexts are short (the caller asks for 256 chunks and more where they are long enough):
 // cutting the keys finer would make every workgroup pay a segment's start and end for a handful of blocks, so the rows are
-// cut instead, into groups of 32 or 64 with a workgroup each over the whole chunk (the groups of a chunk sit next to each other
-// on one XCD and share the cache rows in its L2).  Where the lines lie, 128 heads, us per layer as a graph replay with groups
-// of 32 / 64 / 128 rows: 7 requests of 1k-2k keys 41.6 / 43.4 / 47.5, 16 of 1k-2k 50.4 / 48.2 / 54.5, 7 of 4k-8k 59.5 / 54.9 /
-// 61.0, 16 of 4k-8k 94.7 / 77.5 / 71.8; the fp8 cache, row lists and windows alike.  (Up to three splits a caller may have asked
-// for few chunks itself, whatever the lengths: past half the CUs those keep the 128-row form.)
+// cut instead, into groups with a workgroup each over the whole chunk (the groups of a chunk sit next to each other on one XCD and
+// share the cache rows in its L2).  (Up to three splits a caller may have asked for few chunks itself, whatever the lengths: past half
+// the CUs those keep the 128-row form.)  Groups of 32 rows where the kernel is decode_rows.hip (`rows32`: the bf16 cache), of 32 or 64
+// over the fp8 cache.  Where the lines lie, us per layer as a graph replay in groups of 64 / 32 rows of that kernel: 7 requests of
+// 300-3000 keys x 128 heads 37.2 / 35.2, 16 of 1k-2k 47.6 / 47.3, 7 of 4k-8k 49.4 / 49.4, 16 of 4k-8k 65.2 / 65.3; x 64 heads,
+// one of 1k keys 26.1 / 22.9, 4 of 1k-3k 32.4 / 29.6 (128 chunks), but 8 of 2k-4k 35.0 / 39.4 (256), 64 of 4k-8k 123 / 156.
 struct PlanForm { int rg, chunks; };
-inline PlanForm plan_form(int64_t batch, int64_t num_splits, int64_t query_rows) {
+inline PlanForm plan_form(int64_t batch, int64_t num_splits, int64_t query_rows, bool rows32 = false) {
   const int64_t total = batch * num_splits, groups = (query_rows + 127) / 128, wgs = total * groups;
   if (query_rows > 64 && wgs * 4 <= kPlanCUs) return {1, (int)total};
   if (query_rows > 64 && (wgs * 2 <= kPlanCUs || (wgs < kPlanCUs && num_splits > 3))) {
-    const int64_t most = kPlanCUs / ((query_rows + 63) / 64);
-    return {2, (int)(total < most || most < 1 ? total : most)};
+    const int rg = rows32 ? 1 : 2;
+    const int64_t most = kPlanCUs / ((query_rows + 32 * rg - 1) / (32 * rg));
+    return {rg, (int)(total < most || most < 1 ? total : most)};
   }
+  if (rows32 && query_rows <= 64 && total * 2 <= kPlanCUs) return {1, (int)total};
   const int rg = query_rows <= 32 ? 1 : (query_rows <= 64 ? 2 : 4);
   const int64_t rounds = wgs / kPlanCUs;
   if (rounds < 1) return {rg, (int)total};
@@ -116,6 +119,9 @@ inline dim3 plan_grid(const DecodeParams& p, int rg) {
 // window.  Returns 0 or a negative error code.
 // rg: groups of 32 query rows per workgroup (plan_form).
 int launch_decode_v3(const DecodeParams& p, bool sparse, int rg, hipStream_t stream);
+// The forms with 32 rows per workgroup (decode_rows.hip); list: over p.sparse_rows.
+int launch_decode_rows(const DecodeParams& p, bool list, hipStream_t stream);
+int prepare_decode_rows(bool list, bool window, bool write);
 // The dynamic-LDS limit of all dense bf16 forms raised on the current device, ahead of a launch under stream capture.
 int prepare_decode_v3_dense_forms();
 // The same over the fp8 block-scaled cache p.cache8 (decode_v3_fp8.hip): dense and, with p.win_size > 0, sink + window.

@@ -1,0 +1,446 @@
+// Absorbed-MLA decode over the bf16 cache for launches whose workgroups have few query rows: the split phase with at most 32 rows per
+// workgroup (plan_form's rg = 1), over the paged cache, over it with static sink tokens and a sliding window, and over lists of
+// cache rows.  Same contract, workspace and merge as decode_v3.hip.
+//
+// What bounds it: with few rows the arithmetic is small beside the cache stream, and a short launch is a chain of dependent steps:
+// arguments, lengths, page numbers, first keys, scores, result.  A wavefront issues an instruction every five clocks, so the
+// chain's length is its instruction count, and the general kernel's setup, hand-unrolled phases and register-starved address
+// arithmetic (3500 instructions for two blocks of 32 keys) took 20 000 clocks, 10 us.  Here all eight wavefronts take an equal part in
+// every phase, an iteration is 64 keys, and nothing is unrolled that runs once.
+//
+//   copies      wavefront w brings keys 8w .. 8w + 7 of the iteration's 64 (eight latent rows, one instruction for their rope rows)
+//   S = K Q^T   wavefront (kg, rg) = (w % 4, w / 4): 16 keys x 16 rows, eighteen v_mfma_f32_16x16x32_bf16, the query in registers
+//   softmax     four scores per lane, against a reference fixed at the row's largest score of the first iteration; a score more than
+//               2^100 above it makes the workgroup start over with better references (as in decode_v3.hip)
+//   O += V P    wavefront w owns 64 latent columns for all rows.  A probability goes through P.V as two bf16 numbers, its rounded
+//               value and what the rounding left, through LDS in the layout that is the MFMA operand's: the same lanes hold it
+// Two buffers of 64 keys: the next iteration's copies go out when this one's have landed.  Two barriers per iteration.
+// us per layer, general kernel with groups of 32 or 64 rows -> this: one user of 1k keys x 16 heads 17.9 -> 14.7; 7 of 300-3000 keys x
+// 128 heads, replayed 40.0 -> 37.9; 4 of 1k-3k x 64 heads 34.2 -> 29.9; 64 of 4k-8k x 16 heads 93.9 -> 87.5 (HBM); lists of 2048 rows, 8
+// tokens x 64 heads with their selection 70.8 -> 62.8; 8 windows of 2048 x 64 heads 41.4 -> 33.4.
+#include "decode_params.hpp"
+
+namespace mlahip {
+namespace rows32 {
+
+constexpr int kIter = 64;                                  // keys per iteration
+constexpr int kRows = 32;                                  // query rows of a workgroup
+constexpr int kRopeOff = kIter * 1024;                     // 65536: rope rows behind the latent rows of a buffer
+constexpr int kBufB = kRopeOff + kIter * 128;              // 73728
+constexpr int kPOff = 2 * kBufB;                           // 147456: P, (key-group pair, row group, term) x 64 lanes x 16 bytes
+constexpr int kMaxOff = kPOff + 8 * 1024;                  // 155648: a float per key group and row: maxima, then sums
+constexpr int kFlagOff = kMaxOff + 4 * kRows * 4;          // a dword per wavefront: it asks for a restart
+constexpr int kLdsB = kFlagOff + 64;
+static_assert(kLdsB <= 160 * 1024, "LDS budget");
+constexpr float kRestartThreshold = 100.f;                 // log2 units above a row's reference
+
+// granule (16 bytes) position of a row's granule gr: gr ^ swz_nope(row & 15), gr ^ swz_rope(row & 15).  Sixteen rows read at one granule
+// hit sixteen different 16-byte slots of the banks, and the eight rows of half a transposed read eight different 32-byte pieces.
+__device__ __forceinline__ int swz_nope(int r) { return ((r & 7) << 1) | ((r >> 3) & 1); }
+__device__ __forceinline__ int swz_rope(int r) { return (r >> 1) & 7; }
+
+__device__ __forceinline__ int scan_add(int v) {           // inclusive, over the lanes (see decode_v3.hip)
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return v;
+}
+typedef __attribute__((address_space(4))) const int32_t* ConstI32Ptr;   // scalar (constant-cache) loads
+// a / b for a < 2^21 (the quotient's distance from the next integer is at least 0.5 / b, the product's error below that)
+__device__ __forceinline__ int div_small(int a, int b) {
+  return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b));
+}
+__device__ __forceinline__ int div_units(int a, int b) { return a < (1 << 21) ? div_small(a, b) : a / b; }
+
+enum class Keys { kPaged, kWindow, kList };
+// kNt: the rows of a chunk have no other reader than this workgroup, and their copies are marked non-temporal (see decode_v3.hip)
+// kWrite: the step's cache write, folded in (see decode_v3.hip)
+template <Keys kKeys, bool kNt, bool kWrite>
+__global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams p) {
+  constexpr bool kWindow = kKeys == Keys::kWindow, kList = kKeys == Keys::kList;
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int kg = wave & 3, rg = wave >> 2;
+  const uint32_t lds0 = lds_addr_of(lds);
+  // every XCD takes a contiguous eighth of the chunks, the row groups of a chunk next to each other (see decode_v3.hip)
+  const int lin = blockIdx.x + gridDim.x * blockIdx.z, xcd = lin & 7, nz = gridDim.z;
+  const int xcd_j = nz == 1 ? lin >> 3 : __builtin_amdgcn_readfirstlane(div_small(lin >> 3, nz));
+  const int grp = (lin >> 3) - xcd_j * nz;
+  const int r_max = p.max_q_len * p.num_heads, row0 = grp * kRows;
+
+  // length of a sequence, as its blocks are numbered: without those between the sink and the window
+  auto len_now = [&](int len, int q0, int q1) {
+    if constexpr (kWindow) {
+      if (!p.win_skip) {
+        int ql = p.qsl ? q1 - q0 : p.max_q_len;
+        return window_len(len, ql < p.max_q_len ? ql : p.max_q_len, p.win_sink, p.win_size).len;
+      }
+    }
+    return len;
+  };
+  auto len_of = [&](int i) { return kWindow && p.qsl ? len_now(p.seq_lens[i], p.qsl[i], p.qsl[i + 1]) : len_now(p.seq_lens[i], 0, 0); };
+  // ---- the balanced chunk plan (decode_params.hpp): which blocks are mine ----
+  int chunk, seg_b = -1, v_cur, v_end, v_seq = 0;
+  int my_len = 0, my_q0 = 0, my_q1 = 0;                     // up to 64 sequences: a lane holds one
+  const bool one_pass = p.batch <= 64;
+  {
+    int pe = 0, tot;
+    if (one_pass) {
+      if (lane < p.batch) {
+        my_len = p.seq_lens[lane];
+        if (p.qsl) { my_q0 = p.qsl[lane]; my_q1 = p.qsl[lane + 1]; }
+        my_len = len_now(my_len, my_q0, my_q1);
+      }
+      pe = scan_add(plan_work_units(my_len));
+      tot = __builtin_amdgcn_readlane(pe, 63);
+    } else {
+      int mine = 0;
+      for (int i = lane; i < p.batch; i += 64) mine += plan_work_units(len_of(i));
+      tot = __builtin_amdgcn_readlane(scan_add(mine), 63);
+    }
+    const int chunks = plan_chunk_count(tot, r_max, p.num_chunks), per_xcd = (chunks + 7) >> 3;
+    chunk = xcd * per_xcd + xcd_j;
+    if (xcd_j >= per_xcd || chunk >= chunks || tot == 0) return;
+    // units [floor(c * tot / G), floor((c + 1) * tot / G))
+    if (chunks <= 1024) {
+      const int q = __builtin_amdgcn_readfirstlane(div_units(tot, chunks)), r = tot - q * chunks;
+      v_cur = chunk * q + __builtin_amdgcn_readfirstlane(div_small(chunk * r, chunks));
+      v_end = (chunk + 1) * q + __builtin_amdgcn_readfirstlane(div_small((chunk + 1) * r, chunks));
+    } else {
+      v_cur = (int)((int64_t)chunk * tot / chunks);
+      v_end = (int)((int64_t)(chunk + 1) * tot / chunks);
+    }
+    if (one_pass) {
+      const int b0 = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < p.batch && pe <= v_cur));
+      seg_b = b0 - 1;
+      v_seq = b0 > 0 ? __builtin_amdgcn_readlane(pe, b0 - 1) : 0;
+    } else {
+      int carry = 0, b0 = 0;
+      for (int base = 0; base < p.batch; base += 64) {
+        const int i = base + lane;
+        const int run = scan_add(i < p.batch ? plan_work_units(len_of(i)) : 0) + carry;
+        const int n = __builtin_popcountll(__builtin_amdgcn_ballot_w64(i < p.batch && run <= v_cur));
+        if (n > 0) v_seq = __builtin_amdgcn_readlane(run, n - 1);
+        b0 += n;
+        carry = __builtin_amdgcn_readlane(run, 63);
+      }
+      seg_b = b0 - 1;
+    }
+  }
+
+  // ---- per-lane offsets ----
+  const uint32_t n_sr2 = (uint32_t)p.nope_sr * 2u, r_sr2 = (uint32_t)p.rope_sr * 2u;       // row strides in bytes
+  const uint32_t copy_off = (uint32_t)((lane ^ (wave & 1)) << 4);                          // ^ (j << 5) for the wavefront's row j
+  const int rope_j = lane >> 3;
+  const uint32_t rope_off = (uint32_t)(((lane & 7) ^ swz_rope((wave & 1) * 8 + rope_j)) << 4);
+  const uint32_t k_off = (uint32_t)((kg * 16 + l16) * 1024 + (((g << 2) ^ swz_nope(l16)) << 4));
+  const uint32_t kr_off = (uint32_t)(kRopeOff + (kg * 16 + l16) * 128 + (((g << 1) ^ swz_rope(l16)) << 4));
+  const int vrow = 4 * g + (l16 >> 2);
+  const uint32_t v_off = (uint32_t)(vrow * 1024 + (((8 * wave + ((l16 & 3) >> 1)) ^ swz_nope(vrow)) << 4) + (l16 & 1) * 8);
+
+  while (v_cur < v_end) {
+    seg_b++;
+    if (seg_b >= p.batch) break;
+    const int b = seg_b;
+    const int L = one_pass ? __builtin_amdgcn_readlane(my_len, b) : __builtin_amdgcn_readfirstlane(len_of(b));
+    const int v_b = v_seq;
+    v_seq += plan_work_units(L);
+    const int v_hi = v_seq < v_end ? v_seq : v_end;
+    int blk_begin = v_cur - v_b - kPlanSegCost, blk_end = v_hi - v_b - kPlanSegCost;
+    blk_begin = blk_begin < 0 ? 0 : blk_begin;
+    v_cur = v_hi;
+    if (blk_end <= blk_begin) continue;
+    const int key0 = blk_begin * kPlanBlk, key_end = blk_end * kPlanBlk;                   // the segment's keys
+    if (threadIdx.x == 0) {
+      if (blk_begin == 0) p.seg_ids[2 * b] = chunk + b;
+      if (key_end >= L) p.seg_ids[2 * b + 1] = chunk + b;
+    }
+    int q0 = b * p.max_q_len, qlen = p.max_q_len;
+    if (p.qsl) {
+      q0 = one_pass ? __builtin_amdgcn_readlane(my_q0, b) : ((ConstI32Ptr)p.qsl)[b];
+      qlen = (one_pass ? __builtin_amdgcn_readlane(my_q1, b) : ((ConstI32Ptr)p.qsl)[b + 1]) - q0;
+      qlen = qlen < p.max_q_len ? qlen : p.max_q_len;
+    }
+    const int rows = qlen * p.num_heads;
+    const int64_t part_base = (int64_t)(chunk + b) * r_max + row0;                         // + row in the group
+    const int row = row0 + rg * 16 + l16;                    // this lane's query row for S and softmax; four lanes share it
+    if (row0 >= rows) {                                      // (a request with fewer tokens than the others)
+      if (kg == 0 && g == 0 && row < r_max) { p.lse_part[part_base + rg * 16 + l16] = -INFINITY; p.corr_scale[part_base + rg * 16 + l16] = 0.f; }
+      continue;
+    }
+    if constexpr (kWrite) {
+      // the request's tokens are the keys L - qlen .. L - 1: those of this segment are stored, and have been, before any is asked for
+      for (int j = wave; j < qlen; j += 8) {
+        const int pos = L - qlen + j;
+        if (pos < key0 || pos >= key_end) continue;
+        const int64_t slot = p.new_slots[q0 + j];
+        if (slot < 0 || slot >= p.num_pages * kPage) continue;
+        const int64_t pg = slot / kPage, off = slot - pg * kPage;
+        *(u32x4*)(const_cast<__bf16*>(p.nope) + pg * p.nope_sp + off * p.nope_sr + lane * 8) =
+            *(const u32x4*)(p.new_c + (int64_t)(q0 + j) * p.new_c_st + lane * 8);
+        if (lane < 8)
+          *(u32x4*)(const_cast<__bf16*>(p.rope) + pg * p.rope_sp + off * p.rope_sr + lane * 8) =
+              *(const u32x4*)(p.new_r + (int64_t)(q0 + j) * p.new_r_st + lane * 8);
+      }
+      MLA_WAIT_VMCNT(0);
+    }
+    lds_barrier();                                           // the previous segment is done with the buffers
+    const bool has_rows = row0 + rg * 16 < rows, two = row0 + 16 < rows;
+    int limit = L - qlen + div_small(row, p.num_heads) + 1;  // keys [0, limit) are visible to the row
+    const int seen_to = limit;
+    limit = row < rows ? (limit < key_end ? limit : key_end) : 0;
+
+    // ---- copies ----
+    const int skip = !kWindow ? 0 : 32 * (p.win_skip ? p.win_skip[b] : window_len(((ConstI32Ptr)p.seq_lens)[b], qlen, p.win_sink, p.win_size).skip);
+    // Where the wavefront's keys of an iteration lie: the number of their page as it stands (keys behind the sequence's last one
+    // repeat it: they are masked), or the cache rows of the eight, lane l that of key l % 8.
+    ConstI32Ptr bt = (ConstI32Ptr)(p.block_table) + (kList ? 0 : (int64_t)b * p.bt_stride);
+    auto in_cache = [&](int key) { return kWindow && key >= p.win_sink ? key + skip : key; };
+    auto place_of = [&](int it) {
+      int key = key0 + it * kIter + wave * 8 + (kList ? lane & 7 : 0);
+      key = key < L ? key : L - 1;
+      if constexpr (kList) return p.sparse_rows[(int64_t)b * p.sparse_stride + key];
+      const int page = in_cache(key) >> 7;
+      return bt[page < p.max_blocks ? page : p.max_blocks - 1];
+    };
+    int place;
+    auto copy_keys = [&](int it) {
+      const uint32_t dst = lds0 + (it & 1) * kBufB + wave * 8192, rdst = lds0 + (it & 1) * kBufB + kRopeOff + wave * 1024;
+      if constexpr (kList) {
+        const int64_t rows_in_cache = p.num_pages * p.page_size;
+        const int64_t mine = place < 0 ? 0 : (place >= rows_in_cache ? rows_in_cache - 1 : place);   // (fewer than 2^31 rows are named)
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+          dma16_sv_m0add((const char*)p.nope + (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)mine, j) * n_sr2, copy_off ^ (uint32_t)(j << 5), dst, j * 1024);
+        dma16_v((const char*)p.rope + ((uint64_t)(uint32_t)__shfl((int)mine, rope_j, 64) * r_sr2 + rope_off), rdst);
+      } else {
+        const int64_t pg = place < 0 ? 0 : (place >= p.num_pages ? p.num_pages - 1 : place);
+        const char* np = (const char*)(p.nope + pg * p.nope_sp);
+        const char* rp = (const char*)(p.rope + pg * p.rope_sp);
+        const int first = key0 + it * kIter + wave * 8;      // (the eight keys lie in one page, and in the sink or behind it)
+        const int shift = in_cache(first < L ? first : L - 1) - (first < L ? first : L - 1);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+          int key = first + j;
+          key = ((key < L ? key : L - 1) + shift) & (kPage - 1);
+          const char* src = np + (uint64_t)(uint32_t)key * n_sr2;
+          if constexpr (kNt) dma16_sv_m0add_nt(src, copy_off ^ (uint32_t)(j << 5), dst, j * 1024);
+          else dma16_sv_m0add(src, copy_off ^ (uint32_t)(j << 5), dst, j * 1024);
+        }
+        int key = first + rope_j;
+        key = ((key < L ? key : L - 1) + shift) & (kPage - 1);
+        const char* src = rp + ((uint64_t)(uint32_t)key * r_sr2 + rope_off);
+        if constexpr (kNt) dma16_v_nt(src, rdst);
+        else dma16_v(src, rdst);
+      }
+      place = place_of(it + 1);
+    };
+
+    // ---- the query through LDS (the second buffer, free until the first iteration has begun), rows as the keys lie ----
+    {
+      const int r0 = row0 + wave * 4;
+      if (r0 < rows) {
+        int t = __builtin_amdgcn_readfirstlane(div_small(r0, p.num_heads)), h = r0 - t * p.num_heads;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const bool ok = r0 + k < rows;                     // rows that do not exist read row 0 of the sequence
+          const __bf16* src = p.q_nope + (int64_t)(ok ? q0 + t : q0) * p.qn_st + (int64_t)(ok ? h : 0) * p.qn_sh;
+          const int r16 = (wave & 3) * 4 + k;
+          dma16_sv(src, (uint32_t)((lane ^ swz_nope(r16)) << 4), lds0 + kBufB + (wave * 4 + k) * 1024);
+          h++;
+          if (h == p.num_heads) { h = 0; t++; }
+        }
+      }
+      if (wave < 4 && row0 + wave * 8 < rows) {
+        const int rw = row0 + wave * 8 + rope_j;
+        const int t = div_small(rw, p.num_heads), h = rw - t * p.num_heads;
+        const bool ok = rw < rows;
+        const __bf16* src = p.q_rope + (int64_t)(ok ? q0 + t : q0) * p.qr_st + (int64_t)(ok ? h : 0) * p.qr_sh;
+        dma16_v((const char*)src + (((lane & 7) ^ swz_rope((wave & 1) * 8 + rope_j)) << 4), lds0 + kBufB + kRopeOff + wave * 1024);
+      }
+    }
+    bf16x8 qf[18];
+    const int iters = (key_end - key0 + kIter - 1) / kIter;
+    f32x4 acc[4][2];                                         // [16 of the wavefront's 64 columns][row group]
+    float m_ref = 0.f, l_run = 0.f, seen = -INFINITY;
+    // the rows' references out of every key group's candidates (all wavefronts take part)
+    auto agree = [&](float mine) {
+      mine = fmaxf(mine, __shfl_xor(mine, 16, 64));
+      mine = fmaxf(mine, __shfl_xor(mine, 32, 64));
+      if (g == 0) *(float*)(lds + kMaxOff + (kg * kRows + rg * 16 + l16) * 4) = mine;
+      lds_barrier();
+      const float* at = (const float*)(lds + kMaxOff) + rg * 16 + l16;
+      return fmaxf(fmaxf(at[0], at[kRows]), fmaxf(at[2 * kRows], at[3 * kRows]));
+    };
+    int restarts_left = 4;                                   // (each raises a reference by more than 2^100: fp32 has room for three)
+    bool fresh = true;
+    for (int it = 0; it < iters; it++) {
+      if (it == 0) {
+        place = place_of(0);
+        copy_keys(0);
+        if (fresh) {
+          MLA_WAIT_VMCNT(9);                                       // the query is here, the nine copies of the keys may be on their way
+          lds_barrier();
+          {
+            // (row l16 of the wavefront's row group lies where key l16 of key group rg would)
+            const uint32_t qo = kBufB + k_off + (uint32_t)(rg - kg) * 16384u, qr = kBufB + kr_off + (uint32_t)(rg - kg) * 2048u;
+      #pragma unroll
+            for (int kk = 0; kk < 16; kk++) qf[kk] = *(const bf16x8*)(lds + (qo ^ (uint32_t)((kk >> 2) << 4)) + (kk & 3) * 256);
+      #pragma unroll
+            for (int c = 0; c < 2; c++) qf[16 + c] = *(const bf16x8*)(lds + (qr ^ (uint32_t)(c << 4)));
+          }
+        }
+#pragma unroll
+        for (int cb = 0; cb < 4; cb++)
+#pragma unroll
+          for (int j = 0; j < 2; j++) acc[cb][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        l_run = 0.f;
+      }
+      MLA_WAIT_VMCNT(0);
+      lds_barrier();                                         // this iteration's keys are here, everyone is done with the other buffer
+      if (it + 1 < iters) copy_keys(it + 1);
+      const char* buf = lds + (it & 1) * kBufB;
+      float t[4];
+      if (has_rows) {
+        f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < 16; kk++) {
+          const bf16x8 a = *(const bf16x8*)(buf + (k_off ^ (uint32_t)((kk >> 2) << 4)) + (kk & 3) * 256);
+          if (kk & 1) s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[kk], s1, 0, 0, 0);
+          else s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[kk], s0, 0, 0, 0);
+        }
+        s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(buf + kr_off), qf[16], s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(buf + (kr_off ^ 16u)), qf[17], s1, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; r++) t[r] = (s0[r] + s1[r]) * p.scale_log2;
+      }
+      if (fresh) {                                           // (visible or not: any finite reference within 2^100 of the maximum will do)
+        m_ref = agree(has_rows ? fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3])) : -INFINITY);
+        fresh = false;
+      }
+      if (has_rows) {
+        // score r is visible iff from <= r < rel
+        const int at = key0 + it * kIter + kg * 16 + 4 * g, rel = limit - at;
+        const int from = kWindow && at >= p.win_sink ? seen_to - p.win_size - at : -4;
+        const float top = fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3]));
+        seen = fmaxf(seen, top);
+        float pr[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) pr[r] = r < rel && r >= from ? fast_exp2(t[r] - m_ref) : 0.f;
+        l_run += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+        bf16x4 hi, lo;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          hi[r] = (__bf16)pr[r];
+          lo[r] = (__bf16)(pr[r] - (float)hi[r]);
+        }
+        char* pw = lds + kPOff + ((kg >> 1) * 4 + rg * 2) * 1024 + lane * 16 + (kg & 1) * 8;
+        *(bf16x4*)pw = hi;
+        *(bf16x4*)(pw + 1024) = lo;
+        const bool ask = __builtin_amdgcn_ballot_w64(top - m_ref > kRestartThreshold) != 0;
+        if (lane == 0) *(int*)(lds + kFlagOff + wave * 4) = ask ? 1 : 0;
+      } else if (lane == 0) {
+        *(int*)(lds + kFlagOff + wave * 4) = 0;
+      }
+      lds_barrier();                                         // P is published
+      const int flags = *(const int*)(lds + kFlagOff + (lane & 7) * 4);
+      // V^T fragments of two key groups, and P's of both row groups
+#pragma unroll
+      for (int pair = 0; pair < 2; pair++) {
+        bf16x8 pf[2][2];
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+          for (int term = 0; term < 2; term++)
+            if (j == 0 || two) pf[j][term] = *(const bf16x8*)(lds + kPOff + (pair * 4 + j * 2 + term) * 1024 + lane * 16);
+#pragma unroll
+        for (int cb = 0; cb < 4; cb++) {
+          const char* vb = buf + pair * 32768 + (v_off ^ (uint32_t)(cb << 5));
+          const bf16x4 v0 = lds_read_tr16(vb), v1 = lds_read_tr16(vb + 16384);
+          const bf16x8 a = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+          for (int j = 0; j < 2; j++)
+            if (j == 0 || two) {
+              acc[cb][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pf[j][0], acc[cb][j], 0, 0, 0);
+              acc[cb][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pf[j][1], acc[cb][j], 0, 0, 0);
+            }
+        }
+      }
+      if (restarts_left > 0 && __builtin_amdgcn_ballot_w64(flags != 0) != 0) {
+        // (rare; every wavefront reads the same flags) start over, with the largest scores seen so far as references
+        restarts_left--;
+        MLA_WAIT_VMCNT(0);
+        lds_barrier();
+        m_ref = agree(fmaxf(m_ref, seen));
+        it = -1;
+      }
+    }
+
+    // ---- partials: normalised fp16, natural-log sums ----
+    l_run += __shfl_xor(l_run, 16, 64);
+    l_run += __shfl_xor(l_run, 32, 64);
+    lds_barrier();                                           // (the maxima have been read)
+    if (g == 0) *(float*)(lds + kMaxOff + (kg * kRows + rg * 16 + l16) * 4) = l_run;
+    lds_barrier();
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const float* at = (const float*)(lds + kMaxOff) + j * 16 + l16;
+      const float l = (at[0] + at[kRows]) + (at[2 * kRows] + at[3 * kRows]);
+      const float inv = l > 0.f ? 1.f / l : 0.f;
+      if (row0 + j * 16 + l16 < r_max) {
+        const int64_t part = part_base + j * 16 + l16;
+        _Float16* o = p.o_part + part * kDNope + wave * 64 + 4 * g;
+#pragma unroll
+        for (int cb = 0; cb < 4; cb++) {
+          typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+          h4 v;
+#pragma unroll
+          for (int e = 0; e < 4; e++) v[e] = (_Float16)(acc[cb][j][e] * inv);
+          *(h4*)(o + cb * 16) = v;
+        }
+        if (kg == 0 && rg == j && g == 0) {
+          p.lse_part[part] = l > 0.f ? (m_ref + fast_log2(l)) * kLn2 : -INFINITY;
+          p.corr_scale[part] = 0.f;                          // (no correction record: P.V carries what the rounding left)
+          p.corr_row[part] = p.nope;
+        }
+      }
+    }
+  }
+}
+
+}  // namespace rows32
+
+namespace {
+using rows32::Keys;
+typedef void (*RowsKernel)(const DecodeParams);
+// the kernel of a launch: over a list or the paged cache; windowed; with the step's cache write; chunks with one reader
+RowsKernel rows_kernel(bool list, bool window, bool write, bool once) {
+  using namespace rows32;
+  if (list) return mla_decode_rows_kernel<Keys::kList, false, false>;
+  if (window) return once ? mla_decode_rows_kernel<Keys::kWindow, true, false> : mla_decode_rows_kernel<Keys::kWindow, false, false>;
+  if (write) return once ? mla_decode_rows_kernel<Keys::kPaged, true, true> : mla_decode_rows_kernel<Keys::kPaged, false, true>;
+  return once ? mla_decode_rows_kernel<Keys::kPaged, true, false> : mla_decode_rows_kernel<Keys::kPaged, false, false>;
+}
+}  // namespace
+int prepare_decode_rows(bool list, bool window, bool write) {
+  for (int once = 0; once < 2; once++) {
+    const int rc = ensure_dynamic_lds((const void*)rows_kernel(list, window, write, once), rows32::kLdsB, "mla_decode_rows_kernel");
+    if (rc != MLA_OK) return rc;
+  }
+  return MLA_OK;
+}
+int launch_decode_rows(const DecodeParams& p, bool list, hipStream_t stream) {
+  const bool window = p.win_size > 0, write = p.new_c != nullptr;
+  const int rc = prepare_decode_rows(list, window, write);
+  if (rc != MLA_OK) return rc;
+  const dim3 grid = plan_grid(p, 1);
+  hipLaunchKernelGGL(rows_kernel(list, window, write, grid.z == 1), grid, dim3(512), rows32::kLdsB, stream, p);
+  return check_launch("mla_decode_rows_kernel");
+}
+
+}  // namespace mlahip

@@ -95,17 +95,15 @@ __device__ __forceinline__ int wave_incl_scan_dpp(int v) {
 typedef __attribute__((address_space(4))) const int32_t* ConstI32Ptr;   // scalar (constant-cache) loads
 
 
-// kRG = groups of 32 query rows a workgroup handles (4: the general form; 1 or 2: launches with at most 32 / 64 query rows
-// per request, e.g. the 16 heads a tensor-parallel rank of eight owns, and row-list launches whose chunks alone would
-// leave most of the CUs idle, which then give every 32 or 64 rows a workgroup of their own: blockIdx.z).  With few rows the 128-row schedule spends the same
-// MFMAs, LDS reads and watts on rows that do not exist, so the small forms leave them out: only the wavefronts that own
-// rows run the S phase and the softmax, P.V covers kRG row groups, and the copies move to wavefronts 4..7, which have
-// nothing else to do in the S phase.  The kernel is then bound by the cache stream alone.
+// kRG = groups of 32 query rows a workgroup handles (4: the general form; 2: launches with at most 64 query rows per request;
+// 32 rows: decode_rows.hip).  With few rows the 128-row schedule spends the same MFMAs, LDS reads and watts on rows that do not
+// exist, so the small form leaves them out: only the wavefronts that own rows run the S phase and the softmax, P.V covers kRG row
+// groups, and the copies move to wavefronts 4..7, which have nothing else to do in the S phase.
 template <bool kSparse, bool kWindow, int kRG = 4, bool kWrite = false>
 __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p) {
   static_assert(!(kSparse && kWindow), "the window variant reads the paged cache");
   static_assert(!kWrite || (!kSparse && !kWindow), "the folded cache write belongs to the dense kernel");
-  static_assert(kRG == 1 || kRG == 2 || kRG == 4, "row groups");
+  static_assert(kRG == 2 || kRG == 4, "row groups (one: decode_rows.hip)");
   constexpr int kGrpRows = 32 * kRG;                          // query rows of one workgroup (blockIdx.z counts such groups)
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63;
@@ -515,13 +513,12 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
   // start of a segment) and picks its operands from there.  The copies of the first key blocks have to wait until
   // every wave has its query in registers (one barrier).
   bf16x8 qf[18];                                             // contraction steps of 32: 16 over the latent part, 2 over rope
-  // One or two row groups: the wavefronts that can own rows stage their query in the tile buffer of the segment's FOURTH block
-  // (two groups: of the third and the fourth), which is not requested before the query has been read, so the copying
-  // wavefronts ask for the first three (two) blocks now and the query's round trip to memory hides under theirs.  With four
-  // groups the query fills all four buffers; what can be asked for beside it is where the first blocks lie.  (us per layer,
-  // against two and four groups that asked for nothing before the query had been read: 7 requests of 300-3000 keys, 128 heads,
-  // replayed 41.8 -> 40.9; one of 128k keys 71.2 -> 70.8; 64 of 4k-8k 146.5 -> 146.2.)
-  constexpr int kEarly = kRG == 1 ? kLead : kRG == 2 ? kLead - 1 : 0;        // blocks requested beside the query
+  // Two row groups: the wavefronts that can own rows stage their query in the tile buffers of the segment's third and fourth block,
+  // which are not requested before the query has been read, so the copying wavefronts ask for the first two blocks now and the
+  // query's round trip to memory hides under theirs.  With four groups the query fills all four buffers; what can be asked for
+  // beside it is where the first blocks lie.  (us per layer, against groups that asked for nothing before the query had been
+  // read: 7 requests of 300-3000 keys, 128 heads, replayed 41.8 -> 40.9; one of 128k keys 71.2 -> 70.8; 64 of 4k-8k 146.5 -> 146.2.)
+  constexpr int kEarly = kRG == 2 ? kLead - 1 : 0;            // blocks requested beside the query
   const uint32_t q_stage = kRG == 4 ? wave * 16384u
                          : (uint32_t)(((blk_begin + kEarly + (wave >> 1)) & 3) * kNopeBufB + (wave & 1) * 16384);
   if (!has_rows) {
@@ -744,15 +741,7 @@ __global__ __launch_bounds__(512) void mla_decode_v3_kernel(const DecodeParams p
     // numbers, its rounded value and the rounding's remainder (fragments rg + 2 of the exchange buffer), each fragment of
     // V^T feeding both.  The product then carries 16 significant bits of every probability instead of 8, and the result's
     // error is the rounding of the output alone.
-    if constexpr (kRG == 1) {
-      // one row group: four MFMAs per k-block, the softmax steps in the shadow of the LDS reads
-      if constexpr (kPv) { PV_VREAD(0); PV_PREAD(pr0, 0, 0); PV_PREAD(pr1, 2, 0); }
-      if constexpr (kSm) { if (sm_on) { sm_head(sc, st); SM_EXP2(0, 1); SM_EXP2(2, 3); } }
-      if constexpr (kPv) { PV_MFMA2(0, pr0, 1); PV_MFMA2(0, pr1, 0); PV_VREAD(1); PV_PREAD(pr0, 0, 1); PV_PREAD(pr1, 2, 1); }
-      if constexpr (kSm) { if (sm_on) { SM_EXP2(4, 5); SM_EXP2(6, 7); sm_pm(st); } }
-      if constexpr (kPv) { PV_MFMA2(0, pr0, 1); PV_MFMA2(0, pr1, 0); PV_SETTLE(0); }
-      if constexpr (kSm) { if (sm_on) { sm_sum_lo(sc, st); sm_sum_hi(sc, st); } }
-    } else if constexpr (kRG == 2) {
+    if constexpr (kRG == 2) {
       // (two register quads for the four P^T fragments of a k-block, each refilled as soon as its MFMAs are issued)
       if constexpr (kPv) { PV_VREAD(0); PV_PREAD(pr0, 0, 0); PV_PREAD(pr1, 2, 0); }
       if constexpr (kSm) { if (sm_on) { sm_head(sc, st); SM_EXP2(0, 1); } }
@@ -1083,15 +1072,13 @@ static int launch_form(const DecodeParams& p, hipStream_t stream) {
 }
 template <bool kSparse, bool kWindow, bool kWrite = false>
 static int launch_rows(const DecodeParams& p, int rg, hipStream_t stream) {
-  // (the form depends on the shape; all three get their LDS limit with the family's first launch, so that a later launch
+  // (the form depends on the shape; all of them get their LDS limit with the family's first launch, so that a later launch
   // under stream capture, where the limit cannot be raised, finds every form ready)
-  {
-    int rc = ensure_dynamic_lds((const void*)v3::mla_decode_v3_kernel<kSparse, kWindow, 1, kWrite>, v3::kLdsB, "mla_decode_v3_kernel");
-    if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)v3::mla_decode_v3_kernel<kSparse, kWindow, 2, kWrite>, v3::kLdsB, "mla_decode_v3_kernel");
-    if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)v3::mla_decode_v3_kernel<kSparse, kWindow, 4, kWrite>, v3::kLdsB, "mla_decode_v3_kernel");
-    if (rc != MLA_OK) return rc;
-  }
-  if (rg == 1) return launch_form<kSparse, kWindow, 1, kWrite>(p, stream);
+  int rc = prepare_decode_rows(kSparse, kWindow, kWrite);
+  if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)v3::mla_decode_v3_kernel<kSparse, kWindow, 2, kWrite>, v3::kLdsB, "mla_decode_v3_kernel");
+  if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)v3::mla_decode_v3_kernel<kSparse, kWindow, 4, kWrite>, v3::kLdsB, "mla_decode_v3_kernel");
+  if (rc != MLA_OK) return rc;
+  if (rg == 1) return launch_decode_rows(p, kSparse, stream);
   if (rg == 2) return launch_form<kSparse, kWindow, 2, kWrite>(p, stream);
   return launch_form<kSparse, kWindow, 4, kWrite>(p, stream);
 }
@@ -1099,7 +1086,7 @@ static int launch_rows(const DecodeParams& p, int rg, hipStream_t stream) {
 // Raises the dynamic-LDS limit of every dense form on the current device (what a launch does for its own form the first
 // time it runs): a caller that will launch under stream capture, where that cannot be recorded, does it beforehand.
 int prepare_decode_v3_dense_forms() {
-  int rc = ensure_dynamic_lds((const void*)v3::mla_decode_v3_kernel<false, false, 1, false>, v3::kLdsB, "mla_decode_v3_kernel");
+  int rc = prepare_decode_rows(false, false, false);
   if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)v3::mla_decode_v3_kernel<false, false, 2, false>, v3::kLdsB, "mla_decode_v3_kernel");
   if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)v3::mla_decode_v3_kernel<false, false, 4, false>, v3::kLdsB, "mla_decode_v3_kernel");
   return rc;

@@ -102,6 +102,13 @@ __device__ __forceinline__ void dma16_v(const void* gaddr, uint32_t lds_addr_uni
                : "memory", "m0");
 }
 
+__device__ __forceinline__ void dma16_v_nt(const void* gaddr, uint32_t lds_addr_uniform) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt"
+               :
+               : "s"(lds_addr_uniform), "v"(gaddr)
+               : "memory", "m0");
+}
+
 // The same two copies issued by lanes 0..31 only (512 bytes): the upper half of the execution mask is cleared around
 // the instruction inside the assembly, so the operands stay in the registers a uniform call site gives them.
 __device__ __forceinline__ void dma16_sv_lo32(const void* gbase_uniform, uint32_t voff, uint32_t lds_addr_uniform) {
