@@ -71,13 +71,14 @@ constexpr int kPlanCUs = 256;                              // MI355X
 // the CUs those keep the 128-row form.)  Groups of 32 rows where the kernel is decode_rows.hip (`rows32`: the bf16 cache), of 32 or 64
 // over the fp8 cache.  Where the lines lie, us per layer as a graph replay in groups of 64 / 32 rows of that kernel: 7 requests of
 // 300-3000 keys x 128 heads 37.2 / 35.2, 16 of 1k-2k 47.6 / 47.3, 7 of 4k-8k 49.4 / 49.4, 16 of 4k-8k 65.2 / 65.3; x 64 heads,
-// one of 1k keys 26.1 / 22.9, 4 of 1k-3k 32.4 / 29.6 (128 chunks), but 8 of 2k-4k 35.0 / 39.4 (256), 64 of 4k-8k 123 / 156.
+// one of 1k keys 26.1 / 22.9, 4 of 1k-3k 32.4 / 29.6 (128 chunks), but 8 of 2k-4k 35.0 / 39.4 (256), 64 of 4k-8k 123 / 156.  Queued
+// launches, 12 requests x 128 heads: 300-3000 keys (144 workgroups of 128 rows) 36.5 / 34.6, 3k-5k (240) 46.3 / 48.3.
 struct PlanForm { int rg, chunks; };
 inline PlanForm plan_form(int64_t batch, int64_t num_splits, int64_t query_rows, bool rows32 = false) {
   const int64_t total = batch * num_splits, groups = (query_rows + 127) / 128, wgs = total * groups;
   if (query_rows > 64 && wgs * 4 <= kPlanCUs) return {1, (int)total};
   if (query_rows > 64 && (wgs * 2 <= kPlanCUs || (wgs < kPlanCUs && num_splits > 3))) {
-    const int rg = rows32 ? 1 : 2;
+    const int rg = rows32 && wgs * 8 <= kPlanCUs * 7 ? 1 : 2;
     const int64_t most = kPlanCUs / ((query_rows + 32 * rg - 1) / (32 * rg));
     return {rg, (int)(total < most || most < 1 ? total : most)};
   }

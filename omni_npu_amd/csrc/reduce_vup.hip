@@ -38,7 +38,8 @@ constexpr int kMergeRowOff = kVupWB + 16384;      // kFew: the eight wavefronts'
 constexpr int kVupPairOff = kMergeRowOff + 8192;  // kFew: the sums' (maximum, weight) pairs
 constexpr int kVupFlagOff = kVupPairOff + 64;   // one int per token of the pass: its row is valid
 constexpr int kVupLdsB = kVupFlagOff + 64;
-constexpr int kVupAlone = 16;                   // partials of a row that one wavefront asks for at once
+constexpr int kVupAlone = 16;                   // partials of a row that are left to one wavefront
+constexpr int kVupAsk = 20;                     // partials that a wavefront asks for at once
 constexpr int kVupAhead = 4;                    // product steps whose operands are requested ahead (at most 4: the wait ladder)
 
 __device__ __forceinline__ int vup_wave_sum(int v) {
@@ -179,14 +180,23 @@ __global__ __launch_bounds__(1024) void mla_reduce_vup_kernel(const ReduceVupPar
 
   if constexpr (kFew) {
     const int share = 1 << pp.share_log2, toks = 8 >> pp.toks_log2;         // wavefronts per row (1, 2, 4, 8), tokens
-    if (wave >= 8) {
-      copy_w((wave - 8) * (16 / kParts), 16 / kParts);
-    } else if (wave < toks * share) {
-      const int sub = wave & (share - 1), slot = wave >> pp.share_log2;
-      const MergeRow r = row_of(tb * toks + slot, sub, share);
-      float m = -INFINITY, tot = 0.f, a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      MergeAsked<kVupAlone> asked;
+    const int sub = wave & (share - 1), slot = wave >> pp.share_log2;
+    const bool merges = wave < 8 && wave < toks * share;
+    if (kParts > 2 && wave >= 8) copy_w((wave - 8) * (16 / kParts), 16 / kParts);
+    MergeRow r = {false, 0, 1, 0, 0};
+    MergeAsked<kVupAsk> asked;
+    if (merges) {
+      r = row_of(tb * toks + slot, sub, share);
       mrg_ask(p, r, 0, lane, asked);
+    }
+    // 64 KiB of W_UV and more are asked for behind the partials: in front of them they hold up the numbers and records that the
+    // partials wait for (7 requests of 300-3000 keys x 128 heads 30.4 -> 29.4 us per layer, 3 of 3k-6k 31.0 -> 30.0)
+    if (kParts <= 2) {
+      lds_barrier();
+      if (wave >= 8) copy_w((wave - 8) * (16 / kParts), 16 / kParts);
+    }
+    if (merges) {
+      float m = -INFINITY, tot = 0.f, a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       mrg_all(p, r, lane, asked, m, tot, a);
       if (share == 1) {
         whole_row(slot, r.valid, tot, a);
