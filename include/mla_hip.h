@@ -340,6 +340,20 @@ int mla_prefill_varlen_continue(const void* q_nope, int64_t qn_stride_t, int64_t
                                 float* lse_out, const float* prev_out, int64_t prev_stride_t, int64_t prev_stride_h,
                                 const float* prev_lse, mlahip_stream_t stream);
 
+/* The last context chunk and the causal suffix of a chunked prefill in one launch: mla_prefill_varlen without a mask over the context
+ * keys k1_nope, k1_pe, v1 (cu_k1), continued causally over the new tokens' own k_nope, k_pe, v (cu_k).  All fp16
+ * (out_dtype + MLA_PREFILL_KV_F16), the context's tokens as far apart as the new ones' (kn_stride_t, kp_stride_t, v_stride_t).
+ * prev_out / prev_lse as in mla_prefill_varlen_continue, or both NULL. */
+int mla_prefill_varlen_context(const void* q_nope, int64_t qn_stride_t, int64_t qn_stride_h, const void* q_pe,
+                               int64_t qp_stride_t, int64_t qp_stride_h, const void* k_nope, int64_t kn_stride_t,
+                               int64_t kn_stride_h, const void* k_pe, int64_t kp_stride_t, const void* v, int64_t v_stride_t,
+                               int64_t v_stride_h, const int32_t* cu_q, const int32_t* cu_k, const void* k1_nope,
+                               int64_t kn1_stride_h, const void* k1_pe, const void* v1, int64_t v1_stride_h,
+                               const int32_t* cu_k1, int32_t batch, int32_t num_heads, int32_t max_q_len, float scale, void* out,
+                               int64_t out_stride_t, int64_t out_stride_h, int32_t out_dtype, float* lse_out,
+                               const float* prev_out, int64_t prev_stride_t, int64_t prev_stride_h, const float* prev_lse,
+                               mlahip_stream_t stream);
+
 /* mla_prefill_varlen over a selection of keys: bit j of pick[t] (32-bit words, rows pick_stride words apart, pick_words of
  * them valid, whole 64-key tiles) says whether query token t attends over key j of its sequence, within what causal
  * allows.  The sparse attention of attention/backends/dsa.py:259-291 over the up-projected keys and values of a prompt. */

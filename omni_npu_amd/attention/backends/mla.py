@@ -313,10 +313,12 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
 
     # ---- prefill ----
     def _compute_prefill_context(self, q_nope, q_pe, kv_c_cache, k_pe_cache, attn_metadata, k_scale,
-                                 w16: Optional[torch.Tensor] = None):
+                                 w16: Optional[torch.Tensor] = None, suffix: Optional[tuple] = None):
         """Chunked context: gather -> up-project -> unmasked attention with LSE (reference mla.py:377-450).  The reference
         merges every chunk's result into a running one (merge_attn_states); here a chunk's launch continues from the
-        running result, so the merge is part of the attention kernel and there is no merge launch."""
+        running result, so the merge is part of the attention kernel and there is no merge launch.  Returns that result, its
+        log-sum-exp and the last chunk's (k_nope, k_pe, v, cu_k), which is left to the launch of the suffix where that takes it
+        (``suffix``: its k_nope, k_pe, v), else None."""
         prefill = attn_metadata.prefill
         cc = prefill.chunked_context
         assert cc is not None
@@ -329,10 +331,9 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
         if own is None and rows.dtype == torch.bfloat16:
             w16 = self._half_up_weight() if w16 is None else w16
             rows = rows if w16 is None else rows.view(torch.float16)
-        for i in range(len(cc.seq_tot)):
+        chunks = [i for i in range(len(cc.seq_tot)) if int(cc.seq_tot[i]) > 0]
+        for i in chunks:
             toks = int(cc.seq_tot[i])
-            if toks == 0:
-                continue
             ops.gather_and_maybe_dequant_cache(src_cache=(kv_c_cache,) if k_pe_cache is None else (kv_c_cache, k_pe_cache),
                                                dst=rows,
                                                block_table=prefill.block_table, cu_seq_lens=cc.cu_seq_lens[i],
@@ -345,16 +346,18 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
             else:
                 k_nope, v = self._kv_up(kv_c_normed, allow_fp16=True, w16=w16)
                 k_pe = k_pe.to(k_nope.dtype)
+            cu_k = cc.cu_seq_lens[i].to(torch.int32).contiguous()
+            if i == chunks[-1] and suffix is not None and K.prefill_takes_context(*suffix, (k_nope, k_pe, v)):
+                return output, output_lse, (k_nope, k_pe, v, cu_k)
             # running results stay fp32: each bf16 rounding in between would add 2^-10 of mean relative error to the
             # layer's output
             first = output is None
             if first:
                 output = torch.empty(t, n, self.v_head_dim, dtype=torch.float32, device=q_nope.device)
                 output_lse = torch.empty(t, n, dtype=torch.float32, device=q_nope.device)
-            K.prefill_varlen(q_nope, q_pe, k_nope, k_pe, v, cu_q, cc.cu_seq_lens[i].to(torch.int32).contiguous(),
-                             prefill.max_query_len, self.scale, False, output, output_lse,
+            K.prefill_varlen(q_nope, q_pe, k_nope, k_pe, v, cu_q, cu_k, prefill.max_query_len, self.scale, False, output, output_lse,
                              prev_out=None if first else output, prev_lse=None if first else output_lse)
-        return output, output_lse
+        return output, output_lse, None
 
     def _forward_prefill(self, q, kv_c_normed, k_pe, kv_cache, attn_metadata, k_scale,
                          out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -370,18 +373,18 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
         q_nope, q_pe = q[..., :self.qk_nope_head_dim], q[..., self.qk_nope_head_dim:]
         k_nope, k_pe, v, w16 = self._kv_up_rows(kv_c_normed, k_pe)
         cu_q = prefill.query_start_loc.to(torch.int32).contiguous()
-        ctx_out = ctx_lse = None
+        ctx_out = ctx_lse = context = None
         if has_context:
             # (the fp8 cache is one tensor whose rows hold latent, scales and rope; the gather dequantises it)
-            ctx_out, ctx_lse = self._compute_prefill_context(q_nope, q_pe, kv_cache[0],
-                                                             None if self.fp8_cache else kv_cache[1], attn_metadata, k_scale, w16)
+            ctx_out, ctx_lse, context = self._compute_prefill_context(q_nope, q_pe, kv_cache[0], None if self.fp8_cache else kv_cache[1],
+                                                                      attn_metadata, k_scale, w16, (k_nope, k_pe, v))
         if out is not None and out.dtype == torch.bfloat16 and out.dim() == 2 and out.shape == (t, n * self.v_head_dim) and \
                 out.stride(1) == 1 and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
             output = out.view(t, n, self.v_head_dim)
         else:
             output = torch.empty(t, n, self.v_head_dim, dtype=torch.bfloat16, device=q.device)
         K.prefill_varlen(q_nope, q_pe, k_nope, k_pe, v, cu_q, cu_q, prefill.max_query_len, self.scale, True, output,
-                         prev_out=ctx_out, prev_lse=ctx_lse)
+                         prev_out=ctx_out, prev_lse=ctx_lse, context=context)
         return output.flatten(start_dim=-2)
 
     def _forward_prefill_sink(self, q, kv_c_normed, k_pe, prefill) -> torch.Tensor:

@@ -69,6 +69,8 @@ struct PrefillParams {
   // (an earlier context chunk); the launch then returns the attention over the union, as a merge of the two would
   const float* prev_out; int64_t po_st, po_sh;
   const float* prev_lse;  // [T, N]
+  // optional keys in front of the causal ones (kCtx): those of cu_k1, which every row of the sequence sees; token strides as above
+  const __bf16* k1_nope; int64_t kn1_sh; const __bf16* k1_pe; const __bf16* v1; int64_t v1_sh; const int32_t* cu_k1;
   // optional picks (kPick): bit j of a token's row says whether key j of its sequence is one of the keys it attends over
   const uint32_t* pick; int64_t pick_st; int32_t pick_tiles;   // row stride in words; whole tiles (two words) a row holds
 };
@@ -89,13 +91,15 @@ __device__ __forceinline__ PfLaneOffsets pf_lane_offsets(const PrefillParams& p,
   }
   return o;
 }
-// kParts: 1 = the three key sub-tiles, 2 = the two value sub-tiles, 3 = both.
+// Where a run of keys lies: this head's keys and values and the rope rows of its first key
+struct PfKeys { const __bf16 *kn, *kp, *v; };
+// kParts: 1 = the three key sub-tiles, 2 = the two value sub-tiles, 3 = both.  k0: first key of the tile in its run.
 template <int kParts>
-__device__ __forceinline__ void pf_issue_full_tile(const PrefillParams& p, const PfLaneOffsets& o, int64_t k0, int head,
+__device__ __forceinline__ void pf_issue_full_tile(const PrefillParams& p, const PfKeys& from, const PfLaneOffsets& o, int64_t k0,
                                                    uint32_t buf, int wave) {
-  const char* kn = (const char*)(p.k_nope + k0 * p.kn_st + (int64_t)head * p.kn_sh);
-  const char* vv = (const char*)(p.v + k0 * p.v_st + (int64_t)head * p.v_sh);
-  const char* kp = (const char*)(p.k_pe + k0 * p.kp_st);
+  const char* kn = (const char*)(from.kn + k0 * p.kn_st);
+  const char* vv = (const char*)(from.v + k0 * p.v_st);
+  const char* kp = (const char*)(from.kp + k0 * p.kp_st);
 #pragma unroll
   for (int i = 0; i < 2; i++) {
     const uint32_t dst = buf + (wave * 2 + i) * 1024;
@@ -111,7 +115,7 @@ __device__ __forceinline__ void pf_issue_full_tile(const PrefillParams& p, const
   }
 }
 template <int kParts>
-__device__ __forceinline__ void pf_issue_tile(const PrefillParams& p, int64_t k0, int64_t klast, int head, uint32_t buf,
+__device__ __forceinline__ void pf_issue_tile(const PrefillParams& p, const PfKeys& from, int64_t k0, int64_t klast, uint32_t buf,
                                               int wave, int lane) {
 #pragma unroll
   for (int i = 0; i < 2; i++) {
@@ -119,13 +123,13 @@ __device__ __forceinline__ void pf_issue_tile(const PrefillParams& p, int64_t k0
     int64_t key = k0 + r;
     key = key < klast ? key : klast;
     const int c = ((lane & 7) ^ pf_swz(r & 15)) * 8;
-    const __bf16* kn = p.k_nope + key * p.kn_st + (int64_t)head * p.kn_sh + c;
-    const __bf16* vv = p.v + key * p.v_st + (int64_t)head * p.v_sh + c;
+    const __bf16* kn = from.kn + key * p.kn_st + c;
+    const __bf16* vv = from.v + key * p.v_st + c;
     const uint32_t dst = buf + (wave * 2 + i) * 1024;
     if constexpr (kParts & 1) {
       dma16_v(kn, dst);
       dma16_v(kn + 64, dst + kPfSubB);
-      dma16_v(p.k_pe + key * p.kp_st + c, dst + 2 * kPfSubB);
+      dma16_v(from.kp + key * p.kp_st + c, dst + 2 * kPfSubB);
     }
     if constexpr (kParts & 2) {
       dma16_v(vv, dst + 3 * kPfSubB);
@@ -139,7 +143,10 @@ __device__ __forceinline__ void pf_issue_tile(const PrefillParams& p, int64_t k0
 // kPick: a row attends over the keys its bits name (sparse attention over a selection, for sequences short enough that
 // leaving out scores here costs less than gathering the selected latents; see NPUDSAImpl).  Three prompts of 1500 to 5003
 // tokens, 128 heads, k = 2048: 2145 us on bf16 keys and values, 2107 on fp16 ones, which need a narrower range.
-template <bool kKeyHalf, bool kValHalf, bool kPick>
+// kCtx: the sequence's context keys (k1_nope ...), which all its rows see, in front of its causal ones: one launch for the last context
+// chunk and the suffix, whose rows otherwise go out as fp32 with their sums and come back (4 x 2048 over 16k: 1.1 GB), and whose
+// unequal causal blocks follow each other where every workgroup is resident at once.
+template <bool kKeyHalf, bool kValHalf, bool kPick, bool kCtx>
 __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const PrefillParams p) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63;
@@ -182,6 +189,7 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
   }
   wave_min_limit = __builtin_amdgcn_readfirstlane(wave_min_limit);
   wave_max_limit = __builtin_amdgcn_readfirstlane(wave_max_limit);
+  const bool wave_any = qb * kPfRows + wave * 32 < sq, wave_all = qb * kPfRows + wave * 32 + 32 <= sq;
   // Sliding window: a row sees keys [lo, limit).  lo grows with the row, so the first row of the workgroup gives the
   // first key any row needs, and the largest lo of a wave tells which blocks need the mask at their front.
   const int lo = (p.window > 0 && limit > p.window) ? limit - p.window : 0;
@@ -204,7 +212,10 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
     wg_limit = last_row + shift + 1;
     wg_limit = wg_limit < 0 ? 0 : (wg_limit > sk ? sk : wg_limit);
   }
-  const int tiles = (wg_limit + kPfTile - 1) / kPfTile;
+  // context tiles first, then the causal ones: a tile's number counts through both runs
+  const int sk1 = kCtx ? p.cu_k1[b + 1] - p.cu_k1[b] : 0;
+  const int tiles1 = (sk1 + kPfTile - 1) / kPfTile;
+  const int tiles = tiles1 + (wg_limit + kPfTile - 1) / kPfTile;
 
   const int64_t tq = q0 + (row_ok ? row : 0);
   f32x16 acc[4];
@@ -235,14 +246,24 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
 
   if (tiles > 0) {
     const uint32_t lds0 = lds_addr_of(lds);
-    const int64_t klast = (int64_t)k0 + sk - 1;
+    const PfKeys keys = {p.k_nope + (int64_t)head * p.kn_sh + k0 * p.kn_st, p.k_pe + k0 * p.kp_st, p.v + (int64_t)head * p.v_sh + k0 * p.v_st};
+    PfKeys keys1 = keys;
+    if constexpr (kCtx) {
+      const int64_t k1 = p.cu_k1[b];
+      keys1 = {p.k1_nope + (int64_t)head * p.kn1_sh + k1 * p.kn_st, p.k1_pe + k1 * p.kp_st, p.v1 + (int64_t)head * p.v1_sh + k1 * p.v_st};
+    }
     const PfLaneOffsets lane_off = pf_lane_offsets(p, wave, lane);
     const bool fast_ok = (uint64_t)p.kn_st * 128 < (1u << 31) && (uint64_t)p.v_st * 128 < (1u << 31) && (uint64_t)p.kp_st * 128 < (1u << 31);
     auto issue = [&](int tile, uint32_t buf, auto parts) {
       constexpr int kParts = decltype(parts)::value;
-      const int64_t first = (int64_t)k0 + (int64_t)tile * kPfTile;
-      if (fast_ok && first + kPfTile - 1 <= klast) pf_issue_full_tile<kParts>(p, lane_off, first, head, buf, wave);
-      else pf_issue_tile<kParts>(p, first, klast, head, buf, wave, lane);
+      const bool ctx = kCtx && tile < tiles1;
+      const PfKeys from = {ctx ? keys1.kn : keys.kn, ctx ? keys1.kp : keys.kp, ctx ? keys1.v : keys.v};
+      const int first = (kCtx && !ctx ? tile - tiles1 : tile) * kPfTile, klast = (ctx ? sk1 : sk) - 1;
+      if (fast_ok && first + kPfTile - 1 <= klast) pf_issue_full_tile<kParts>(p, from, lane_off, first, buf, wave);
+      else pf_issue_tile<kParts>(p, from, first, klast, buf, wave, lane);
+    };
+    auto interleave = [&](int tile) {                          // whether a tile's copies can go out one by one
+      return tile < tiles && fast_ok && (kCtx && tile < tiles1 ? (tile + 1) * kPfTile <= sk1 : (kCtx ? tile - tiles1 + 1 : tile + 1) * kPfTile <= sk);
     };
     // per-lane LDS offsets: K granule 2 j + half of a row (j = 0..3 inside a sub-tile)
     int koff[4];
@@ -322,8 +343,15 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
       lds_barrier();
       const u32x2 bits = bits_next;
       if constexpr (kPick) bits_next = pick_tile(tile + 1 < tiles ? tile + 1 : tile);
-      if (tile + 1 < tiles) issue(tile + 1, lds0 + ((tile + 1) & 1) * kPfBufB, std::integral_constant<int, 3>{});
-      const int key_base = tile * kPfTile;
+      // The next tile's copies go out one by one between the score MFMAs: the forty of the four wavefronts take the CU's address
+      // unit 800 clocks, and a wavefront that issues its ten in a row stands still for them.  A wavefront that has no scores to
+      // work out, and tiles whose rows do not exist or lie too far apart, have them in a row.
+      const uint32_t next_buf = lds0 + ((tile + 1) & 1) * kPfBufB;
+      auto issue_next = [&] { if (tile + 1 < tiles) issue(tile + 1, next_buf, std::integral_constant<int, 3>{}); };
+      const bool ctx = kCtx && tile < tiles1;
+      const int key_base = (kCtx && !ctx ? tile - tiles1 : tile) * kPfTile;
+      const int end = !kCtx ? limit : ctx ? (row_ok ? sk1 : 0) : limit;                    // the row's visible keys of this run
+      const int min_end = ctx ? (wave_all ? sk1 : 0) : wave_min_limit, max_end = ctx ? (wave_any ? sk1 : 0) : wave_max_limit;
       // V of this tile goes from bf16 to fp16 where it lies (thread t takes the 16-byte pieces t, t + 256, ...), then a
       // barrier: the four wavefronts read each other's pieces.  (Tried: the conversion's arithmetic and writes behind the
       // first block's score MFMAs, and the next tile converted between the two blocks of this one - both slower.)
@@ -344,31 +372,72 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
         for (int i = 0; i < 4; i++) *(u32x4*)(vt + i * 4096) = w[i];
         lds_barrier();
       }
-      if (key_base >= wave_max_limit || key_base + kPfTile <= wg_lo) continue;   // no row of this wavefront sees the tile
+      if (key_base >= max_end || key_base + kPfTile <= wg_lo) {           // no row of this wavefront sees the tile
+        issue_next();
+        continue;
+      }
 
       uint32_t seen[2] = {0u, 0u};                             // kPick: the row's keys in the tile's two blocks
-      bool mask_tile = key_base + kPfTile > wave_min_limit || key_base < wave_max_lo;
+      bool mask_tile = key_base + kPfTile > min_end || key_base < wave_max_lo;
       if constexpr (kPick) {
-        const int rel = limit - key_base;                     // (keys behind the causal limit have no bits worth reading)
+        const int rel = end - key_base;                     // (keys behind the causal limit have no bits worth reading)
 #pragma unroll
         for (int tb = 0; tb < 2; tb++) {
           const int in_blk = rel - tb * 32;
           seen[tb] = in_blk >= 32 ? bits[tb] : (in_blk <= 0 ? 0u : bits[tb] & ((1u << in_blk) - 1u));
         }
-        if (__builtin_amdgcn_ballot_w64((seen[0] | seen[1]) != 0u) == 0) continue;
+        if (__builtin_amdgcn_ballot_w64((seen[0] | seen[1]) != 0u) == 0) {
+          issue_next();
+          continue;
+        }
         mask_tile = __builtin_amdgcn_ballot_w64((seen[0] & seen[1]) != ~0u) != 0;
       }
 
       f32x16 s[2];
       f16x2 pb[2][8];
-      auto scores = [&](int tb) {
+      // Both blocks' scores, two MFMAs of each per step; a step's keys are read in the step before it
+      auto scores = [&](auto with_copies) {
+        constexpr bool kCopies = decltype(with_copies)::value;
+        const char *kn = nullptr, *kp = nullptr, *vv = nullptr;
+        if constexpr (kCopies) {
+          const bool c1 = kCtx && tile + 1 < tiles1;
+          const int64_t first = (int64_t)(kCtx && !c1 ? tile + 1 - tiles1 : tile + 1) * kPfTile;
+          kn = (const char*)((c1 ? keys1.kn : keys.kn) + first * p.kn_st);
+          kp = (const char*)((c1 ? keys1.kp : keys.kp) + first * p.kp_st);
+          vv = (const char*)((c1 ? keys1.v : keys.v) + first * p.v_st);
+        }
+        auto copy = [&](int j) {
+          const uint32_t dst = next_buf + wave * 2048 + (j & 1) * 1024;
+          const int part = j >> 1;
+          if (part < 2) dma16_sv(kn + part * 128, lane_off.kn[j & 1], dst + part * kPfSubB);
+          else if (part == 2) dma16_sv(kp, lane_off.kp[j & 1], dst + 2 * kPfSubB);
+          else dma16_sv(vv + (part - 3) * 128, lane_off.v[j & 1], dst + part * kPfSubB);
+        };
+        bf16x8 a[2][4];
+        auto read = [&](int g, bf16x8 (&to)[4]) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) s[tb][r] = 0.f;
+          for (int u = 0; u < 4; u++) {
+            const int kk = 2 * g + (u >> 1);
+            to[u] = *(const bf16x8*)(buf + koff[kk & 3] + (kk >> 2) * kPfSubB + (u & 1) * 4096);
+          }
+        };
 #pragma unroll
-        for (int kk = 0; kk < 12; kk++) {
-          const bf16x8 a = *(const bf16x8*)(buf + koff[kk & 3] + (kk >> 2) * kPfSubB + tb * 4096);
-          if constexpr (kKeyHalf) s[tb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, qf[kk]), s[tb], 0, 0, 0);
-          else s[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[kk], s[tb], 0, 0, 0);
+        for (int tb = 0; tb < 2; tb++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) s[tb][r] = 0.f;
+        read(0, a[0]);
+#pragma unroll
+        for (int g = 0; g < 6; g++) {
+          if (g < 5) read(g + 1, a[(g + 1) & 1]);
+#pragma unroll
+          for (int u = 0; u < 4; u++) {
+            const int kk = 2 * g + (u >> 1), tb = u & 1;
+            if constexpr (kKeyHalf) s[tb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a[g & 1][u]), __builtin_bit_cast(f16x8, qf[kk]), s[tb], 0, 0, 0);
+            else s[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[g & 1][u], qf[kk], s[tb], 0, 0, 0);
+            if constexpr (kCopies) {
+              if (tb == 1 && kk < 10) copy(kk);
+            }
+          }
         }
       };
       // probabilities against the row's reference as fp16 pairs, and the sum of what they were before they were rounded
@@ -386,8 +455,8 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
         return sum + odd;
       };
       __builtin_amdgcn_s_setprio(1);
-      scores(0);
-      scores(1);
+      if (interleave(tile + 1)) scores(std::true_type{});
+      else { issue_next(); scores(std::false_type{}); }
       __builtin_amdgcn_s_setprio(0);
       // Only tiles that some row of this wave cannot see in full pay for the mask (causal diagonal, end of the keys,
       // rows past the end of the sequence).
@@ -402,7 +471,7 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
               s[tb][r] = __uint_as_float((on & __float_as_uint(v)) | (~on & 0xff800000u));
             } else {
               const int key = key_base + tb * 32 + 4 * half + 8 * (r >> 2) + (r & 3);
-              s[tb][r] = (key < limit && key >= lo) ? s[tb][r] : -INFINITY;
+              s[tb][r] = (key < end && key >= lo) ? s[tb][r] : -INFINITY;
             }
           }
       }
@@ -480,7 +549,8 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
                                float scale, void* out, int64_t out_stride_t, int64_t out_stride_h, int32_t out_dtype,
                                float* lse_out, const float* prev_out, int64_t prev_stride_t, int64_t prev_stride_h,
                                const float* prev_lse, const uint32_t* pick, int64_t pick_stride, int32_t pick_words,
-                               hipStream_t stream) {
+                               hipStream_t stream, const void* k1_nope = nullptr, int64_t kn1_stride_h = 0, const void* k1_pe = nullptr,
+                               const void* v1 = nullptr, int64_t v1_stride_h = 0, const int32_t* cu_k1 = nullptr) {
   MLA_REQUIRE(q_nope && q_pe && k_nope && k_pe && v && cu_q && cu_k && out, MLA_ERR_NULL, "%s: null pointer argument", what);
   MLA_REQUIRE(batch >= 0 && num_heads >= 1 && max_q_len >= 0 && batch <= 65535 && num_heads <= 65535 && window >= 0,
               MLA_ERR_SHAPE, "%s: batch=%d num_heads=%d max_q_len=%d window=%d", what, batch, num_heads, max_q_len, window);
@@ -501,6 +571,11 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
   MLA_REQUIRE(pick == nullptr || (window == 0 && pick_words >= 2 && pick_words % 2 == 0 && pick_stride >= pick_words &&
                                   pick_stride % 2 == 0 && (uintptr_t)pick % 8 == 0),
               MLA_ERR_SHAPE, "%s: picks go without a window, in 8-byte aligned rows of whole 64-key tiles", what);
+  MLA_REQUIRE(!k1_nope || (k1_pe && v1 && cu_k1), MLA_ERR_NULL, "%s: null pointer argument", what);
+  MLA_REQUIRE(!k1_nope || (key_half && causal && window == 0), MLA_ERR_UNSUPPORTED,
+              "%s: context keys go in front of causal fp16 keys and values, without a window", what);
+  MLA_REQUIRE(((uintptr_t)k1_nope | (uintptr_t)k1_pe | (uintptr_t)v1) % 16 == 0 && kn1_stride_h % 8 == 0 && v1_stride_h % 8 == 0,
+              MLA_ERR_SHAPE, "%s: rows must be 16-byte aligned", what);
   if (batch == 0 || max_q_len == 0) return MLA_OK;
   PrefillParams p;
   p.q_nope = (const __bf16*)q_nope; p.qn_st = qn_stride_t; p.qn_sh = qn_stride_h;
@@ -513,17 +588,20 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
   p.out = out; p.o_st = out_stride_t; p.o_sh = out_stride_h; p.out_fp32 = out_dtype;
   p.lse = lse_out;
   p.prev_out = prev_out; p.po_st = prev_stride_t; p.po_sh = prev_stride_h; p.prev_lse = prev_lse;
+  p.k1_nope = (const __bf16*)k1_nope; p.kn1_sh = kn1_stride_h; p.k1_pe = (const __bf16*)k1_pe;
+  p.v1 = (const __bf16*)v1; p.v1_sh = v1_stride_h; p.cu_k1 = cu_k1;
   p.pick = pick; p.pick_st = pick_stride; p.pick_tiles = pick_words / 2;
-  static constexpr auto kernel_of = [](bool kh, bool vh, bool pk) {
-    return kh ? (pk ? mla_prefill_varlen_kernel<true, true, true> : mla_prefill_varlen_kernel<true, true, false>)
-         : vh ? (pk ? mla_prefill_varlen_kernel<false, true, true> : mla_prefill_varlen_kernel<false, true, false>)
-              : (pk ? mla_prefill_varlen_kernel<false, false, true> : mla_prefill_varlen_kernel<false, false, false>);
+  static constexpr auto kernel_of = [](bool kh, bool vh, bool pk, bool ctx) {
+    return ctx  ? mla_prefill_varlen_kernel<true, true, false, true>
+           : kh ? (pk ? mla_prefill_varlen_kernel<true, true, true, false> : mla_prefill_varlen_kernel<true, true, false, false>)
+           : vh ? (pk ? mla_prefill_varlen_kernel<false, true, true, false> : mla_prefill_varlen_kernel<false, true, false, false>)
+                : (pk ? mla_prefill_varlen_kernel<false, false, true, false> : mla_prefill_varlen_kernel<false, false, false, false>);
   };
   int rc = MLA_OK;
-  for (int i = 0; i < 6 && rc == MLA_OK; i++)              // (all of them: a caller's warm-up step need not be of the kind that it captures)
-    rc = ensure_dynamic_lds((const void*)kernel_of((i >> 1) == 2, (i >> 1) != 0, i & 1), kPfLdsB, what);
+  for (int i = 0; i < 7 && rc == MLA_OK; i++)              // (all of them: a caller's warm-up step need not be of the kind that it captures)
+    rc = ensure_dynamic_lds((const void*)kernel_of((i >> 1) == 2, (i >> 1) != 0, i & 1, i == 6), kPfLdsB, what);
   if (rc != MLA_OK) return rc;
-  auto* kern = kernel_of(key_half, val_half, pick != nullptr);
+  auto* kern = kernel_of(key_half, val_half, pick != nullptr, k1_nope != nullptr);
   dim3 grid((max_q_len + kPfRows - 1) / kPfRows, num_heads, batch);
   hipLaunchKernelGGL(kern, grid, dim3(256), kPfLdsB, stream, p);
   return check_launch("mla_prefill_varlen_kernel");
@@ -576,4 +654,25 @@ extern "C" int mla_prefill_varlen_pick(const void* q_nope, int64_t qn_stride_t, 
                              kn_stride_t, kn_stride_h, k_pe, kp_stride_t, v, v_stride_t, v_stride_h, cu_q, cu_k, batch,
                              num_heads, max_q_len, causal, 0, scale, out, out_stride_t, out_stride_h, out_dtype, lse_out,
                              nullptr, 0, 0, nullptr, pick, pick_stride, pick_words, stream);
+}
+
+// The causal attention of a step's new tokens over their context and themselves in one launch: what mla_prefill_varlen (causal 0) over
+// the context keys, continued causally over the new ones, returns.  k_nope, k_pe, v, cu_k: the new tokens', fp16
+// (MLA_PREFILL_KV_F16); k1_nope, k1_pe, v1, cu_k1: the context's, of the same types and token strides.  prev_out / prev_lse (or both
+// NULL): the state of earlier context chunks.
+extern "C" int mla_prefill_varlen_context(const void* q_nope, int64_t qn_stride_t, int64_t qn_stride_h, const void* q_pe,
+                                          int64_t qp_stride_t, int64_t qp_stride_h, const void* k_nope, int64_t kn_stride_t,
+                                          int64_t kn_stride_h, const void* k_pe, int64_t kp_stride_t, const void* v,
+                                          int64_t v_stride_t, int64_t v_stride_h, const int32_t* cu_q, const int32_t* cu_k,
+                                          const void* k1_nope, int64_t kn1_stride_h, const void* k1_pe, const void* v1,
+                                          int64_t v1_stride_h, const int32_t* cu_k1, int32_t batch, int32_t num_heads,
+                                          int32_t max_q_len, float scale, void* out, int64_t out_stride_t, int64_t out_stride_h,
+                                          int32_t out_dtype, float* lse_out, const float* prev_out, int64_t prev_stride_t,
+                                          int64_t prev_stride_h, const float* prev_lse, hipStream_t stream) {
+  MLA_REQUIRE(k1_nope && k1_pe && v1 && cu_k1, MLA_ERR_NULL, "mla_prefill_varlen_context: null pointer argument");
+  return prefill_varlen_impl("mla_prefill_varlen_context", q_nope, qn_stride_t, qn_stride_h, q_pe, qp_stride_t, qp_stride_h,
+                             k_nope, kn_stride_t, kn_stride_h, k_pe, kp_stride_t, v, v_stride_t, v_stride_h, cu_q, cu_k, batch,
+                             num_heads, max_q_len, 1, 0, scale, out, out_stride_t, out_stride_h, out_dtype, lse_out, prev_out,
+                             prev_stride_t, prev_stride_h, prev_lse, nullptr, 0, 0, stream, k1_nope, kn1_stride_h, k1_pe, v1,
+                             v1_stride_h, cu_k1);
 }

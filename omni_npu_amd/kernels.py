@@ -886,11 +886,20 @@ _PREFILL_KV_F16 = 16                                       # added to the output
 _PREFILL_V_F16 = 32                                        # v alone does
 
 
+def prefill_takes_context(k_nope: torch.Tensor, k_pe: torch.Tensor, v: torch.Tensor, context: tuple) -> bool:
+    """Whether prefill_varlen takes (k_nope, k_pe, v) of context keys in front of these."""
+    k1, pe1, v1 = context
+    return (all(x.dtype == torch.float16 and x.stride(-1) == 1 for x in (k_nope, k_pe, v, k1, pe1, v1))
+            and k1.dim() == v1.dim() == 3 and pe1.dim() == 2 and k_pe.dim() == 2 and k1.shape[1:] == k_nope.shape[1:]
+            and v1.shape == k1.shape and pe1.shape == (k1.shape[0], 64)
+            and (k1.stride(0), pe1.stride(0), v1.stride(0)) == (k_nope.stride(0), k_pe.stride(0), v.stride(0)))
+
+
 def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tensor, k_pe: torch.Tensor, v: torch.Tensor,
                    cu_q: torch.Tensor, cu_k: torch.Tensor, max_q_len: int, scale: float, causal: bool,
                    out: torch.Tensor, lse_out: Optional[torch.Tensor] = None, window: Optional[int] = None,
                    prev_out: Optional[torch.Tensor] = None, prev_lse: Optional[torch.Tensor] = None,
-                   pick: Optional[torch.Tensor] = None) -> torch.Tensor:
+                   pick: Optional[torch.Tensor] = None, context: Optional[tuple] = None) -> torch.Tensor:
     """Varlen non-absorbed MLA attention (reference: the prefill FIA calls, src/omni_npu/attention/backends/mla.py:574-590
     and :415-431).  q_nope [T,N,128], q_pe [T,N,64], k_nope [Tk,N,128], k_pe [Tk,64] (shared by the heads), v [Tk,N,128],
     cu_q / cu_k int32 [B+1] device tensors, out [T,N,128] bf16 or fp32, lse_out fp32 [T,N].  ``window`` keeps only the
@@ -900,6 +909,8 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
     (src/omni_npu/attention/ops.py:5-42) gives, in one launch.  ``out`` may be ``prev_out``.
     k_nope, k_pe and v may all three be fp16 (kv_up makes them): both products then run on fp16 and the kernel skips the
     conversion of the value tiles it otherwise does (the queries stay bf16); or v alone, which saves the conversion only.
+    ``context`` = (k_nope, k_pe, v, cu_k) of further keys, which every row of a sequence sees: one launch for them (an unmasked call)
+    and the causal call that continues from it (prefill_takes_context says whether it takes them).
     ``pick`` (int32 [T, W] bits, see topk's mask; W even and wide enough for the longest sequence; no window, no earlier
     result): a token attends over the keys its bits name."""
     if window is not None and window < 1:
@@ -939,6 +950,23 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
                 window is not None or prev_out is not None:
             raise TypeError("prefill_varlen: pick must be int32 [T, W] (W even, rows contiguous), without a window or an earlier "
                             "result")
+    if context is not None:
+        if not causal or window is not None or pick is not None or not prefill_takes_context(k_nope, k_pe, v, context[:3]) or \
+                context[3].dtype != torch.int32 or context[3].numel() != cu_q.numel() or not context[3].is_contiguous():
+            raise TypeError("prefill_varlen: context keys go in front of causal ones of the same types and token strides, fp16, with "
+                            "cu_k contiguous int32 [B+1], without a window or picks")
+        _need_cuda(*context)
+        if context[0].shape[0] and k_nope.shape[0] and t:
+            k1, pe1, v1, cu1 = context
+            prev = (prev_out.data_ptr(), prev_out.stride(0), prev_out.stride(1), prev_lse.data_ptr()) if prev_out is not None else (None, 0, 0, None)
+            rc = lib.mla_prefill_varlen_context(
+                q_nope.data_ptr(), q_nope.stride(0), q_nope.stride(1), q_pe.data_ptr(), q_pe.stride(0), q_pe.stride(1),
+                k_nope.data_ptr(), k_nope.stride(0), k_nope.stride(1), k_pe.data_ptr(), k_pe.stride(0), v.data_ptr(), v.stride(0),
+                v.stride(1), cu_q.data_ptr(), cu_k.data_ptr(), k1.data_ptr(), k1.stride(1), pe1.data_ptr(), v1.data_ptr(),
+                v1.stride(1), cu1.data_ptr(), cu_q.numel() - 1, n, int(max_q_len), float(scale), out.data_ptr(), out.stride(0),
+                out.stride(1), _DT[out.dtype] | kv_code, lse_out.data_ptr() if lse_out is not None else None, *prev, _stream(q_nope))
+            _lib.check(rc, "mla_prefill_varlen_context")
+            return out
     if k_nope.shape[0] == 0 or t == 0:
         # no keys at all (a context chunk in which every sequence is empty): zeros and lse = -inf, as the kernel gives for
         # an empty key range (the earlier result itself when there is one); empty tensors have no address to hand over
