@@ -178,25 +178,22 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
   const int row = qb * kPfRows + wave * 32 + h32;            // query index inside the sequence
   const bool row_ok = row < sq;
   const int shift = sk - sq;                                  // right-down alignment of the causal mask
-  int limit = p.causal ? row + shift + 1 : sk;                // visible keys of this row
-  limit = !row_ok ? 0 : (limit < 0 ? 0 : (limit > sk ? sk : limit));
-  int wave_min_limit = limit;                                 // fewest keys any row of this wave can see
-  int wave_max_limit = limit;                                 // most keys any row of this wave can see
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int other = __shfl_xor(wave_min_limit, o, 64); wave_min_limit = other < wave_min_limit ? other : wave_min_limit;
-    const int more = __shfl_xor(wave_max_limit, o, 64); wave_max_limit = more > wave_max_limit ? more : wave_max_limit;
-  }
-  wave_min_limit = __builtin_amdgcn_readfirstlane(wave_min_limit);
-  wave_max_limit = __builtin_amdgcn_readfirstlane(wave_max_limit);
-  const bool wave_any = qb * kPfRows + wave * 32 < sq, wave_all = qb * kPfRows + wave * 32 + 32 <= sq;
-  // Sliding window: a row sees keys [lo, limit).  lo grows with the row, so the first row of the workgroup gives the
-  // first key any row needs, and the largest lo of a wave tells which blocks need the mask at their front.
-  const int lo = (p.window > 0 && limit > p.window) ? limit - p.window : 0;
-  int wave_max_lo = lo;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) { const int other = __shfl_xor(wave_max_lo, o, 64); wave_max_lo = other > wave_max_lo ? other : wave_max_lo; }
-  wave_max_lo = __builtin_amdgcn_readfirstlane(wave_max_lo);
+  // Rows behind the sequence's last one repeat it (their results are not stored): a wavefront that owns some then masks no more tiles
+  // than its last row does, where rows with no visible keys had it mask every tile, 1100 clocks each, in a sequence's last block, which
+  // sees the most keys (1017 tokens behind 3072 cached ones beside 31 decodes, 64 heads: 309 -> 288 us per layer; 7 ragged prompts,
+  // 32 heads: 362 -> 356).
+  auto keys_of = [&](int r) {                                 // visible keys of a row: they do not decrease from row to row
+    const int n = p.causal ? r + shift + 1 : sk;
+    return n < 0 ? 0 : (n > sk ? sk : n);
+  };
+  // Sliding window: a row sees keys [lo, limit).  lo grows with the row too
+  auto first_of = [&](int n) { return p.window > 0 && n > p.window ? n - p.window : 0; };
+  const int wave_row = qb * kPfRows + wave * 32, wave_last = wave_row + 31 < sq ? wave_row + 31 : sq - 1;
+  const bool wave_any = wave_row < sq;
+  const int limit = keys_of(row_ok ? row : sq - 1), lo = first_of(limit);
+  const int wave_min_limit = keys_of(wave_row);               // fewest and most keys any row of this wave can see
+  const int wave_max_limit = wave_any ? keys_of(wave_last) : 0;
+  const int wave_max_lo = first_of(wave_max_limit);           // blocks that start in front of it need the mask at their front
   int wg_lo = 0;
   if (p.window > 0) {
     int lim0 = p.causal ? qb * kPfRows + shift + 1 : sk;
@@ -217,7 +214,7 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
   const int tiles1 = (sk1 + kPfTile - 1) / kPfTile;
   const int tiles = tiles1 + (wg_limit + kPfTile - 1) / kPfTile;
 
-  const int64_t tq = q0 + (row_ok ? row : 0);
+  const int64_t tq = q0 + (row_ok ? row : sq - 1);
   f32x16 acc[4];
 #pragma unroll
   for (int i = 0; i < 4; i++)
@@ -297,13 +294,12 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
     bf16x8 qf[12];
     {
       MLA_WAIT_VMCNT(6);                                       // the query is here, the six copies of the keys may be on their way
-      const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
       const char* qn = lds + other_buf + wave * 4096;
       const char* qp = lds + first_buf + kPfVOff + (h32 >> 4) * (kPfSubB - 2048) + wave * 2048;   // (koff counts rows 16.. from 2048 on)
 #pragma unroll
-      for (int kk = 0; kk < 8; kk++) { bf16x8 v = *(const bf16x8*)(qn + (kk >> 2) * 16384 + koff[kk & 3]); qf[kk] = row_ok ? v : zero; }
+      for (int kk = 0; kk < 8; kk++) { qf[kk] = *(const bf16x8*)(qn + (kk >> 2) * 16384 + koff[kk & 3]); }
 #pragma unroll
-      for (int kk = 0; kk < 4; kk++) { bf16x8 v = *(const bf16x8*)(qp + koff[kk]); qf[8 + kk] = row_ok ? v : zero; }
+      for (int kk = 0; kk < 4; kk++) { qf[8 + kk] = *(const bf16x8*)(qp + koff[kk]); }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       issue(first_tile, lds0 + first_buf, std::integral_constant<int, 2>{});
       if constexpr (kKeyHalf) {
@@ -350,8 +346,8 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
       auto issue_next = [&] { if (tile + 1 < tiles) issue(tile + 1, next_buf, std::integral_constant<int, 3>{}); };
       const bool ctx = kCtx && tile < tiles1;
       const int key_base = (kCtx && !ctx ? tile - tiles1 : tile) * kPfTile;
-      const int end = !kCtx ? limit : ctx ? (row_ok ? sk1 : 0) : limit;                    // the row's visible keys of this run
-      const int min_end = ctx ? (wave_all ? sk1 : 0) : wave_min_limit, max_end = ctx ? (wave_any ? sk1 : 0) : wave_max_limit;
+      const int end = ctx ? sk1 : limit;                     // the row's visible keys of this run
+      const int min_end = ctx ? sk1 : wave_min_limit, max_end = ctx ? (wave_any ? sk1 : 0) : wave_max_limit;
       // V of this tile goes from bf16 to fp16 where it lies (thread t takes the 16-byte pieces t, t + 256, ...), then a
       // barrier: the four wavefronts read each other's pieces.  (Tried: the conversion's arithmetic and writes behind the
       // first block's score MFMAs, and the next tile converted between the two blocks of this one - both slower.)
@@ -458,8 +454,7 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
       if (interleave(tile + 1)) scores(std::true_type{});
       else { issue_next(); scores(std::false_type{}); }
       __builtin_amdgcn_s_setprio(0);
-      // Only tiles that some row of this wave cannot see in full pay for the mask (causal diagonal, end of the keys,
-      // rows past the end of the sequence).
+      // Only tiles that some row of this wave cannot see in full pay for the mask (causal diagonal, end of the keys).
       if (mask_tile) {
 #pragma unroll
         for (int tb = 0; tb < 2; tb++)
