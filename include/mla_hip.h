@@ -299,10 +299,11 @@ int mla_merge_n_states(const void* outs, int64_t outs_stride_n, int64_t outs_str
  * x bf16 [num_rows, 512], weight bf16 [num_heads * 256, 512], out 16-bit rows of 256 (strides in elements; token t of head h at
  * t * out_stride_t + h * out_stride_h): 128 columns of the key, fp16 with keys_f16 and bf16 without, and 128 of the value,
  * always fp16 (without keys_f16 finite values beyond 65504 are clamped there).  k_pe / out_pe (or both NULL): the rows' rope
- * part [num_rows, 64], bf16, written as fp16 by the same launch. */
+ * part [num_rows, 64], bf16, written as fp16 by the same launch.  clear: up to 512 32-bit words that the launch sets to zero (the queue
+ * of an mla_prefill_varlen_queued behind it), or NULL and 0. */
 int mla_kv_up(const void* x, int64_t x_stride, const void* weight, int64_t w_stride, int64_t num_rows, int32_t num_heads,
               int32_t keys_f16, void* out, int64_t out_stride_t, int64_t out_stride_h, const void* k_pe, int64_t k_pe_stride,
-              void* out_pe, int64_t out_pe_stride, mlahip_stream_t stream);
+              void* out_pe, int64_t out_pe_stride, void* clear, int32_t clear_words, mlahip_stream_t stream);
 
 /* ---- non-absorbed varlen attention for prefill -------------------------------------------
  * Replaces the prefill calls of npu_fused_infer_attention_score, attention/backends/mla.py:574-590 (suffix:
@@ -340,20 +341,6 @@ int mla_prefill_varlen_continue(const void* q_nope, int64_t qn_stride_t, int64_t
                                 float* lse_out, const float* prev_out, int64_t prev_stride_t, int64_t prev_stride_h,
                                 const float* prev_lse, mlahip_stream_t stream);
 
-/* The last context chunk and the causal suffix of a chunked prefill in one launch: mla_prefill_varlen without a mask over the context
- * keys k1_nope, k1_pe, v1 (cu_k1), continued causally over the new tokens' own k_nope, k_pe, v (cu_k).  All fp16
- * (out_dtype + MLA_PREFILL_KV_F16), the context's tokens as far apart as the new ones' (kn_stride_t, kp_stride_t, v_stride_t).
- * prev_out / prev_lse as in mla_prefill_varlen_continue, or both NULL. */
-int mla_prefill_varlen_context(const void* q_nope, int64_t qn_stride_t, int64_t qn_stride_h, const void* q_pe,
-                               int64_t qp_stride_t, int64_t qp_stride_h, const void* k_nope, int64_t kn_stride_t,
-                               int64_t kn_stride_h, const void* k_pe, int64_t kp_stride_t, const void* v, int64_t v_stride_t,
-                               int64_t v_stride_h, const int32_t* cu_q, const int32_t* cu_k, const void* k1_nope,
-                               int64_t kn1_stride_h, const void* k1_pe, const void* v1, int64_t v1_stride_h,
-                               const int32_t* cu_k1, int32_t batch, int32_t num_heads, int32_t max_q_len, float scale, void* out,
-                               int64_t out_stride_t, int64_t out_stride_h, int32_t out_dtype, float* lse_out,
-                               const float* prev_out, int64_t prev_stride_t, int64_t prev_stride_h, const float* prev_lse,
-                               mlahip_stream_t stream);
-
 /* mla_prefill_varlen over a selection of keys: bit j of pick[t] (32-bit words, rows pick_stride words apart, pick_words of
  * them valid, whole 64-key tiles) says whether query token t attends over key j of its sequence, within what causal
  * allows.  The sparse attention of attention/backends/dsa.py:259-291 over the up-projected keys and values of a prompt. */
@@ -364,6 +351,24 @@ int mla_prefill_varlen_pick(const void* q_nope, int64_t qn_stride_t, int64_t qn_
                             float scale, const uint32_t* pick, int64_t pick_stride, int32_t pick_words, void* out,
                             int64_t out_stride_t, int64_t out_stride_h, int32_t out_dtype, float* lse_out,
                             mlahip_stream_t stream);
+
+/* Every option of the prefill entries in one.  k1_nope, k1_pe, v1, cu_k1 (or all NULL): keys in front of the causal ones, which every
+ * row of a sequence sees - the last context chunk and the causal suffix of a chunked prefill in one launch; all fp16 (out_dtype +
+ * MLA_PREFILL_KV_F16), the context's tokens as far apart as the new ones' (kn_stride_t, kp_stride_t, v_stride_t), no window, no pick.
+ * prev_out / prev_lse as in mla_prefill_varlen_continue, pick as in mla_prefill_varlen_pick, or NULL.
+ * queue (or NULL): 1 KiB of device memory that holds zeros, at most 64 sequences, heads a multiple of eight.  The launch is then one
+ * resident set of workgroups that take the blocks of 128 query rows from it, instead of a workgroup to each; worth it from more than
+ * 512 blocks on.  The launch uses the memory up: it has to be cleared for the next. */
+int mla_prefill_varlen_queued(const void* q_nope, int64_t qn_stride_t, int64_t qn_stride_h, const void* q_pe,
+                              int64_t qp_stride_t, int64_t qp_stride_h, const void* k_nope, int64_t kn_stride_t,
+                              int64_t kn_stride_h, const void* k_pe, int64_t kp_stride_t, const void* v, int64_t v_stride_t,
+                              int64_t v_stride_h, const int32_t* cu_q, const int32_t* cu_k, const void* k1_nope,
+                              int64_t kn1_stride_h, const void* k1_pe, const void* v1, int64_t v1_stride_h,
+                              const int32_t* cu_k1, int32_t batch, int32_t num_heads, int32_t max_q_len, int32_t causal,
+                              int32_t window, float scale, const uint32_t* pick, int64_t pick_stride, int32_t pick_words,
+                              void* out, int64_t out_stride_t, int64_t out_stride_h, int32_t out_dtype, float* lse_out,
+                              const float* prev_out, int64_t prev_stride_t, int64_t prev_stride_h, const float* prev_lse,
+                              int32_t* queue, mlahip_stream_t stream);
 
 /* ---- DSA lightning indexer --------------------------------------------------------------------
  * Replaces torch.ops.custom.npu_lightning_indexer, v1/layers/attention/npu_dsa.py:92-103 and

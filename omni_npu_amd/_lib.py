@@ -42,7 +42,7 @@ SIGNATURES = {
                                    I64, I32, I64, P]),
     "mla_rows_f16": (c_int32, [P, I64, P, I64, I64, P, I64, P, I64, P]),
     "mla_rows_f16_weight": (c_int32, [P, I64, P, I64, I64, P, I64, P, I64, P, I64, I64, P, P]),
-    "mla_kv_up": (c_int32, [P, I64, P, I64, I64, I32, I32, P, I64, I64, P, I64, P, I64, P]),
+    "mla_kv_up": (c_int32, [P, I64, P, I64, I64, I32, I32, P, I64, I64, P, I64, P, I64, P, I32, P]),
     "mla_merge_states": (c_int32, [P, I64, I64, P, P, I64, I64, P, I32, P, I64, I64, I32, P, I32, I32, I32, P]),
     "mla_merge_n_states": (c_int32, [P, I64, I64, I32, P, I64, P, I64, P, I32, I32, I32, P]),
     "mla_decode_workspace_bytes": (SZ, [I32, I32, I32, I32]),
@@ -65,8 +65,8 @@ SIGNATURES = {
                                      I32, F32, P, I64, I64, I32, P, P]),
     "mla_prefill_varlen_continue": (c_int32, [P, I64, I64, P, I64, I64, P, I64, I64, P, I64, P, I64, I64, P, P, I32, I32, I32,
                                               I32, I32, F32, P, I64, I64, I32, P, P, I64, I64, P, P]),
-    "mla_prefill_varlen_context": (c_int32, [P, I64, I64, P, I64, I64, P, I64, I64, P, I64, P, I64, I64, P, P, P, I64, P, P, I64, P,
-                                             I32, I32, I32, F32, P, I64, I64, I32, P, P, I64, I64, P, P]),
+    "mla_prefill_varlen_queued": (c_int32, [P, I64, I64, P, I64, I64, P, I64, I64, P, I64, P, I64, I64, P, P, P, I64, P, P, I64, P,
+                                            I32, I32, I32, I32, I32, F32, P, I64, I32, P, I64, I64, I32, P, P, I64, I64, P, P, P]),
     "mla_prefill_varlen_pick": (c_int32, [P, I64, I64, P, I64, I64, P, I64, I64, P, I64, P, I64, I64, P, P, I32, I32, I32, I32,
                                           F32, P, I64, I32, P, I64, I64, I32, P, P]),
     "dsa_indexer_scores_fp8": (c_int32, [P, I64, I64, P, I64, P, I64, P, I64, I64, P, I64, I64, I32, P, I64, I32, P, P, I32,

@@ -389,10 +389,11 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
                 tuple(out.shape) != (t, n * 128) or (q.stride(0) | q.stride(1) | k_pe.stride(0) | out.stride(0)) % 8 or \
                 (q.data_ptr() | k_pe.data_ptr() | out.data_ptr()) % 16:
             return False
-        k_nope, pe, v, _ = self._kv_up_rows(kv_c_normed, k_pe)
         cu = prefill.query_start_loc.to(torch.int32).contiguous()
+        queue = K.prefill_queue(t, cu.numel() - 1, prefill.max_query_len, n, q.device)
+        k_nope, pe, v, _ = self._kv_up_rows(kv_c_normed, k_pe, queue)
         K.prefill_varlen(q[..., :128], q[..., 128:], k_nope, pe, v, cu, cu, prefill.max_query_len, self.scale, True,
-                         out.view(t, n, 128), pick=pick)
+                         out.view(t, n, 128), pick=pick, queue=queue)
         return True
 
     def forward(self, layer, q: torch.Tensor, k_c_normed: torch.Tensor, k_pe: torch.Tensor,

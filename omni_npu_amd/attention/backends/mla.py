@@ -241,15 +241,17 @@ class HalfUpProjection:
         kv = self.kv_b_proj(kv_c)
         return self._split_kv(kv[0] if isinstance(kv, tuple) else kv)
 
-    def _kv_up_rows(self, kv_c: torch.Tensor, k_pe: torch.Tensor):
+    def _kv_up_rows(self, kv_c: torch.Tensor, k_pe: torch.Tensor, queue: Optional[torch.Tensor] = None):
         """(k_nope, k_pe [T,64], v, w16) of a step's own rows as the prefill kernel takes them: from kernels.kv_up where it takes
         them, else all fp16 where the weight allows it, else all in the dtype of the up-projection's result.  w16: the weight in
         fp16, for the step's context rows (None: it was not needed, or the module was called).  Latents, rope rows and weight are
-        converted in one launch."""
+        converted in one launch.  ``queue``: a kernels.prefill_queue to clear on the way."""
         w = self._kv_up_weight(kv_c)
         if w is not None and k_pe.dtype == torch.bfloat16:
-            k_nope, v, pe = K.kv_up(kv_c, w, self.num_heads, self.prefill_kv_fp16, k_pe if self.prefill_kv_fp16 else None)
+            k_nope, v, pe = K.kv_up(kv_c, w, self.num_heads, self.prefill_kv_fp16, k_pe if self.prefill_kv_fp16 else None, queue)
             return k_nope, k_pe.reshape(k_pe.shape[0], -1) if pe is None else pe, v, None
+        if queue is not None:
+            queue.zero_()
         w = self._plain_up_weight() if self.prefill_kv_fp16 else None
         if w is not None and kv_c.dtype == torch.bfloat16 and k_pe.dtype == torch.bfloat16:
             if w.dtype == torch.bfloat16 and w.stride(1) == 1:
@@ -334,6 +336,7 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
         chunks = [i for i in range(len(cc.seq_tot)) if int(cc.seq_tot[i]) > 0]
         for i in chunks:
             toks = int(cc.seq_tot[i])
+            queue = None if own is None else K.prefill_queue(t, cu_q.numel() - 1, prefill.max_query_len, n, q_nope.device)
             ops.gather_and_maybe_dequant_cache(src_cache=(kv_c_cache,) if k_pe_cache is None else (kv_c_cache, k_pe_cache),
                                                dst=rows,
                                                block_table=prefill.block_table, cu_seq_lens=cc.cu_seq_lens[i],
@@ -341,7 +344,7 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
                                                scale=k_scale, seq_starts=cc.starts[i], total_rows=toks)
             kv_c_normed, k_pe = rows[:toks, :self.kv_lora_rank], rows[:toks, self.kv_lora_rank:]
             if own is not None:
-                k_nope, v, pe = K.kv_up(kv_c_normed, own, n, self.prefill_kv_fp16, k_pe if self.prefill_kv_fp16 else None)
+                k_nope, v, pe = K.kv_up(kv_c_normed, own, n, self.prefill_kv_fp16, k_pe if self.prefill_kv_fp16 else None, queue)
                 k_pe = k_pe if pe is None else pe
             else:
                 k_nope, v = self._kv_up(kv_c_normed, allow_fp16=True, w16=w16)
@@ -356,7 +359,7 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
                 output = torch.empty(t, n, self.v_head_dim, dtype=torch.float32, device=q_nope.device)
                 output_lse = torch.empty(t, n, dtype=torch.float32, device=q_nope.device)
             K.prefill_varlen(q_nope, q_pe, k_nope, k_pe, v, cu_q, cu_k, prefill.max_query_len, self.scale, False, output, output_lse,
-                             prev_out=None if first else output, prev_lse=None if first else output_lse)
+                             prev_out=None if first else output, prev_lse=None if first else output_lse, queue=queue)
         return output, output_lse, None
 
     def _forward_prefill(self, q, kv_c_normed, k_pe, kv_cache, attn_metadata, k_scale,
@@ -371,8 +374,9 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
         t, n = q.shape[0], self.num_heads
         has_context = prefill.chunked_context is not None
         q_nope, q_pe = q[..., :self.qk_nope_head_dim], q[..., self.qk_nope_head_dim:]
-        k_nope, k_pe, v, w16 = self._kv_up_rows(kv_c_normed, k_pe)
         cu_q = prefill.query_start_loc.to(torch.int32).contiguous()
+        queue = K.prefill_queue(t, cu_q.numel() - 1, prefill.max_query_len, n, q.device)
+        k_nope, k_pe, v, w16 = self._kv_up_rows(kv_c_normed, k_pe, queue)
         ctx_out = ctx_lse = context = None
         if has_context:
             # (the fp8 cache is one tensor whose rows hold latent, scales and rope; the gather dequantises it)
@@ -384,7 +388,7 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
         else:
             output = torch.empty(t, n, self.v_head_dim, dtype=torch.bfloat16, device=q.device)
         K.prefill_varlen(q_nope, q_pe, k_nope, k_pe, v, cu_q, cu_q, prefill.max_query_len, self.scale, True, output,
-                         prev_out=ctx_out, prev_lse=ctx_lse, context=context)
+                         prev_out=ctx_out, prev_lse=ctx_lse, context=context, queue=queue)
         return output.flatten(start_dim=-2)
 
     def _forward_prefill_sink(self, q, kv_c_normed, k_pe, prefill) -> torch.Tensor:

@@ -51,6 +51,7 @@ struct KvUpParams {
   int32_t stream_out;                            // results are marked non-temporal
   const __bf16* pe; int64_t pe_st;               // rope rows that leave as fp16 (null: none)
   _Float16* pe_out; int64_t pe_ost;
+  uint32_t* clear; int32_t clear_words;          // words to set to zero for the launch behind this one (null: none)
 };
 
 // granule g (16 bytes) of row r of a unit lies at g ^ up_swz(r): the sixteen rows of a phase of a 16-byte read hit sixteen
@@ -91,6 +92,7 @@ __global__ __launch_bounds__(512, 2) void mla_kv_up_kernel(const KvUpParams p) {
   const int last = (int)((int64_t)total * (xcd + 1) / 8);
   int idx = (int)((int64_t)total * xcd / 8) + (blockIdx.x >> 3);
 
+  if (blockIdx.x == 0 && (int)threadIdx.x < p.clear_words) p.clear[threadIdx.x] = 0u;
   auto rope_rows = [&]() {
     for (int64_t i = (int64_t)blockIdx.x * 512 + threadIdx.x; i < p.rows * 8; i += (int64_t)gridDim.x * 512) {
       const bf16x8 v = *(const bf16x8*)(p.pe + (i >> 3) * p.pe_st + (i & 7) * 8);
@@ -303,7 +305,8 @@ using namespace mlahip;
 
 extern "C" int mla_kv_up(const void* x, int64_t x_stride, const void* weight, int64_t w_stride, int64_t num_rows, int32_t num_heads,
                          int32_t keys_f16, void* out, int64_t out_stride_t, int64_t out_stride_h, const void* k_pe,
-                         int64_t k_pe_stride, void* out_pe, int64_t out_pe_stride, hipStream_t stream) {
+                         int64_t k_pe_stride, void* out_pe, int64_t out_pe_stride, void* clear, int32_t clear_words,
+                         hipStream_t stream) {
   MLA_REQUIRE(x && weight && out, MLA_ERR_NULL, "mla_kv_up: null pointer argument");
   MLA_REQUIRE((k_pe == nullptr) == (out_pe == nullptr), MLA_ERR_NULL, "mla_kv_up: rope rows and their result go together");
   MLA_REQUIRE(num_rows >= 0 && num_heads >= 1 && num_heads <= 65535 && (num_rows + kUpTok - 1) / kUpTok * num_heads < (1 << 30),
@@ -313,6 +316,8 @@ extern "C" int mla_kv_up(const void* x, int64_t x_stride, const void* weight, in
                   ((uintptr_t)x | (uintptr_t)weight | (uintptr_t)out) % 16 == 0 &&
                   (!k_pe || (((uintptr_t)k_pe | (uintptr_t)out_pe) % 16 == 0 && k_pe_stride % 8 == 0 && out_pe_stride % 8 == 0)),
               MLA_ERR_SHAPE, "mla_kv_up: rows must be 16-byte aligned, at most 2^20 elements apart");
+  MLA_REQUIRE(clear_words >= 0 && clear_words <= 512 && (clear || clear_words == 0) && (uintptr_t)clear % 4 == 0, MLA_ERR_SHAPE,
+              "mla_kv_up: up to 512 words to clear (got %d)", clear_words);
   if (num_rows == 0) return MLA_OK;
   KvUpParams p;
   p.x = (const __bf16*)x; p.x_st = x_stride;
@@ -322,6 +327,7 @@ extern "C" int mla_kv_up(const void* x, int64_t x_stride, const void* weight, in
   p.stream_out = (int64_t)num_rows * num_heads * 512 >= kUpStreamBytes;
   p.pe = (const __bf16*)k_pe; p.pe_st = k_pe_stride;
   p.pe_out = (_Float16*)out_pe; p.pe_ost = out_pe_stride;
+  p.clear = (uint32_t*)clear; p.clear_words = clear_words;
   auto* kern = keys_f16 ? mla_kv_up_kernel<true> : mla_kv_up_kernel<false>;
   int rc = ensure_dynamic_lds((const void*)mla_kv_up_kernel<true>, kUpLdsB, "mla_kv_up");
   if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)mla_kv_up_kernel<false>, kUpLdsB, "mla_kv_up");

@@ -43,6 +43,8 @@ constexpr int kPfVOff = 3 * kPfSubB;             // 24576  sub-tiles 0, 1: k_nop
 constexpr int kPfBufB = 5 * kPfSubB;             // 40960
 constexpr int kPfLdsB = 2 * kPfBufB;             // 81920: two workgroups per CU
 constexpr int kPfRows = 128;
+constexpr int kPfWorkgroups = 512;               // with a queue: two on each CU, 64 on an XCD
+constexpr int kPfQueue = 32;                     // words between two counters of a queue: a 128-byte line each
 // A probability may reach 2^13 of its row's reference before the reference is raised (fp16 holds 65504)
 constexpr float kPfRaise = 8192.f;
 constexpr float kPfNoRef = -1e30f;               // reference of a row that has seen no key
@@ -73,6 +75,9 @@ struct PrefillParams {
   const __bf16* k1_nope; int64_t kn1_sh; const __bf16* k1_pe; const __bf16* v1; int64_t v1_sh; const int32_t* cu_k1;
   // optional picks (kPick): bit j of a token's row says whether key j of its sequence is one of the keys it attends over
   const uint32_t* pick; int64_t pick_st; int32_t pick_tiles;   // row stride in words; whole tiles (two words) a row holds
+  int32_t max_blocks;                                        // of a sequence
+  // optional: eight counters that begin at zero, kPfQueue apart, from which a grid of kPfWorkgroups takes its blocks
+  int32_t* queue;
 };
 
 // One 64-key tile of head `head`, keys k0 .. k0 + 63 of the flat key axis (clamped to klast): 40 copy instructions of eight
@@ -146,34 +151,15 @@ __device__ __forceinline__ void pf_issue_tile(const PrefillParams& p, const PfKe
 // kCtx: the sequence's context keys (k1_nope ...), which all its rows see, in front of its causal ones: one launch for the last context
 // chunk and the suffix, whose rows otherwise go out as fp32 with their sums and come back (4 x 2048 over 16k: 1.1 GB), and whose
 // unequal causal blocks follow each other where every workgroup is resident at once.
-template <bool kKeyHalf, bool kValHalf, bool kPick, bool kCtx>
-__global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const PrefillParams p) {
-  extern __shared__ __attribute__((aligned(1024))) char lds[];
+// A block of 128 rows of a head: rows 128 qb .. of a sequence whose queries start at q0 and whose keys at k0 (context keys: at k1)
+struct PfBlock { int qb, head, q0, sq, k0, sk, k1, sk1; };
+
+template <bool kKeyHalf, bool kValHalf, bool kPick, bool kCtx, class Last>
+__device__ __forceinline__ void pf_block(const PrefillParams& p, char* lds, const PfBlock& blk, Last last_tile_done) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h32 = lane & 31, half = lane >> 5;
-  // Workgroups go to the eight XCDs round-robin in launch order (x fastest), and each XCD has its own L2.  All query
-  // blocks of one (sequence, head) stream the same keys and values, so they are renumbered to sit on ONE XCD, next to each
-  // other in its queue: they then run at the same time and all but the first find the K / V tiles in that L2.
-  int qb = blockIdx.x, head = blockIdx.y, b = blockIdx.z;
-  {
-    const int nqb = gridDim.x, npairs = gridDim.y * gridDim.z;
-    if ((npairs & 7) == 0) {
-      const int lin = blockIdx.x + nqb * (blockIdx.y + gridDim.y * blockIdx.z);
-      const int j = lin >> 3, run = j / nqb, pair = run * 8 + (lin & 7);
-      qb = j % nqb;
-      // Under the causal mask a block's work grows with its number.  An XCD deals its queue to 32 CUs in turn, two workgroups to
-      // each, so every second stretch of about 32 runs backwards: a CU gets a long and a short one instead of the same twice
-      // (1017 tokens behind 3072 cached ones beside 31 decodes, 64 heads: 376 -> 367 us per layer; 7 ragged prompts, 32 heads:
-      // 417 -> 414).
-      if (p.causal && ((run / (nqb < 32 ? 32 / nqb : 1)) & 1)) qb = nqb - 1 - qb;
-      head = pair % gridDim.y;
-      b = pair / gridDim.y;
-    }
-  }
-  const int q0 = p.cu_q[b], sq = p.cu_q[b + 1] - q0;
-  const int k0 = p.cu_k[b], sk = p.cu_k[b + 1] - k0;
-  if (qb * kPfRows >= sq) return;
+  const int qb = blk.qb, head = blk.head, q0 = blk.q0, sq = blk.sq, k0 = blk.k0, sk = blk.sk, k1 = blk.k1, sk1 = blk.sk1;
 
   const int row = qb * kPfRows + wave * 32 + h32;            // query index inside the sequence
   const bool row_ok = row < sq;
@@ -210,7 +196,6 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
     wg_limit = wg_limit < 0 ? 0 : (wg_limit > sk ? sk : wg_limit);
   }
   // context tiles first, then the causal ones: a tile's number counts through both runs
-  const int sk1 = kCtx ? p.cu_k1[b + 1] - p.cu_k1[b] : 0;
   const int tiles1 = (sk1 + kPfTile - 1) / kPfTile;
   const int tiles = tiles1 + (wg_limit + kPfTile - 1) / kPfTile;
 
@@ -246,8 +231,8 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
     const PfKeys keys = {p.k_nope + (int64_t)head * p.kn_sh + k0 * p.kn_st, p.k_pe + k0 * p.kp_st, p.v + (int64_t)head * p.v_sh + k0 * p.v_st};
     PfKeys keys1 = keys;
     if constexpr (kCtx) {
-      const int64_t k1 = p.cu_k1[b];
-      keys1 = {p.k1_nope + (int64_t)head * p.kn1_sh + k1 * p.kn_st, p.k1_pe + k1 * p.kp_st, p.v1 + (int64_t)head * p.v1_sh + k1 * p.v_st};
+      const int64_t at1 = k1;
+      keys1 = {p.k1_nope + (int64_t)head * p.kn1_sh + at1 * p.kn_st, p.k1_pe + at1 * p.kp_st, p.v1 + (int64_t)head * p.v1_sh + at1 * p.v_st};
     }
     const PfLaneOffsets lane_off = pf_lane_offsets(p, wave, lane);
     const bool fast_ok = (uint64_t)p.kn_st * 128 < (1u << 31) && (uint64_t)p.v_st * 128 < (1u << 31) && (uint64_t)p.kp_st * 128 < (1u << 31);
@@ -509,6 +494,7 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
     }
   }
 
+  last_tile_done();
   const float l_tot = l_run + xor32(l_run);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (row_ok) {
@@ -532,6 +518,99 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
   }
 }
 
+// Workgroups go to the eight XCDs round-robin in launch order (x fastest), and each XCD has its own L2.  All query blocks of one
+// (sequence, head) stream the same keys and values, so both orders of the blocks below keep them on ONE XCD, next to each other: they
+// then run at the same time and all but the first find the K / V tiles in that L2.
+//
+// kQueue, where there are more blocks than run at once: workgroups that stay take them from one queue per XCD, and from the others'
+// when their own is used up.  A workgroup to each block leaves a CU's place empty for 5 to 7 us between two of them, and the XCDs,
+// which do not run at one speed, each with the same number (4 x 2048 tokens over 16k of context, 128 heads: 13 151 -> 12 906 us per
+// layer on one card, 13 356 -> 12 890 on another; three sparse prompts of 1500 to 5003 tokens, 128 heads: 2469 -> 2424; 7 ragged
+// prompts, 32 heads: 363 -> 358).  The power that the card may draw keeps most of what the fuller CUs could have given.
+// !kQueue: blocks that all run at once, and where the order is not worked out (over 64 sequences, heads not a multiple of eight).
+template <bool kKeyHalf, bool kValHalf, bool kPick, bool kCtx, bool kQueue>
+__global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const PrefillParams p0) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+  if constexpr (!kQueue) {
+    const PrefillParams& p = p0;
+    int qb = blockIdx.x, head = blockIdx.y, b = blockIdx.z;
+    const int nqb = gridDim.x, npairs = gridDim.y * gridDim.z;
+    if ((npairs & 7) == 0) {
+      const int j = lin >> 3, run = j / nqb, pair = run * 8 + (lin & 7);
+      qb = j % nqb;
+      // Under the causal mask a block's work grows with its number.  An XCD deals its queue to 32 CUs in turn, two workgroups to
+      // each, so every second stretch of about 32 runs backwards: a CU gets a long and a short one instead of the same twice
+      // (1017 tokens behind 3072 cached ones beside 31 decodes, 64 heads: 376 -> 367 us per layer).
+      if (p.causal && ((run / (nqb < 32 ? 32 / nqb : 1)) & 1)) qb = nqb - 1 - qb;
+      head = pair % gridDim.y;
+      b = pair / gridDim.y;
+    }
+    PfBlock blk = {qb, head, p.cu_q[b], 0, p.cu_k[b], 0, 0, 0};
+    blk.sq = p.cu_q[b + 1] - blk.q0;
+    blk.sk = p.cu_k[b + 1] - blk.k0;
+    if constexpr (kCtx) {
+      blk.k1 = p.cu_k1[b];
+      blk.sk1 = p.cu_k1[b + 1] - blk.k1;
+    }
+    if (qb * kPfRows >= blk.sq) return;
+    pf_block<kKeyHalf, kValHalf, kPick, kCtx>(p, lds, blk, [] {});
+  } else {
+    // Lane c keeps where sequence c's blocks stand in an XCD's queue: the sequences with the most keys first and their longest blocks
+    // first, so that what runs last is short.  Blocks that a sequence does not have are not in it.
+    const int lane = threadIdx.x & 63, per = p0.num_heads >> 3;   // heads of an XCD
+    int q0_l = 0, sq_l = 0, k0_l = 0, sk_l = 0, k1_l = 0, sk1_l = 0, before_l = 0, blocks_l = 0;
+    if (lane < p0.batch) {
+      q0_l = p0.cu_q[lane];
+      sq_l = p0.cu_q[lane + 1] - q0_l;
+      k0_l = p0.cu_k[lane];
+      sk_l = p0.cu_k[lane + 1] - k0_l;
+      if constexpr (kCtx) {
+        k1_l = p0.cu_k1[lane];
+        sk1_l = p0.cu_k1[lane + 1] - k1_l;
+      }
+      blocks_l = sq_l > 0 ? (sq_l + kPfRows - 1) / kPfRows : 0;
+      blocks_l = blocks_l < p0.max_blocks ? blocks_l : p0.max_blocks;
+    }
+    for (int c = 0; c < p0.batch; c++) {
+      const int keys_l = sk_l + sk1_l, kc = __builtin_amdgcn_readlane(keys_l, c), bc = __builtin_amdgcn_readlane(blocks_l, c);
+      before_l += kc > keys_l || (kc == keys_l && c < lane) ? bc * per : 0;
+    }
+    int xcd = lin & 7, ticket = lin >> 3, taken = 0;
+    int32_t* const queue = p0.queue;
+    auto ask = [&] {                                          // for the next ticket of queue xcd, behind those the launch began with
+      if (threadIdx.x == 0) taken = (int)(gridDim.x >> 3) + atomicAdd(queue + xcd * kPfQueue, 1);
+    };
+    auto get = [&] {
+      lds_barrier();                                          // (the wavefronts are done with the LDS)
+      if (threadIdx.x == 0) *(int*)lds = taken;
+      lds_barrier();
+      ticket = __builtin_amdgcn_readfirstlane(*(const int*)lds);
+      lds_barrier();
+    };
+    for (int queues = 8;;) {
+      const uint64_t at = __builtin_amdgcn_ballot_w64(ticket >= before_l && ticket < before_l + blocks_l * per);
+      if (at == 0) {
+        if (--queues == 0) return;
+        xcd = (xcd + 1) & 7;
+        ask();
+        get();
+        continue;
+      }
+      const int b = __builtin_ctzll(at), n = __builtin_amdgcn_readlane(blocks_l, b);
+      const int u = ticket - __builtin_amdgcn_readlane(before_l, b), h = u / n;
+      const PfBlock blk = {n - 1 - (u - h * n), h * 8 + xcd, __builtin_amdgcn_readlane(q0_l, b), __builtin_amdgcn_readlane(sq_l, b),
+                           __builtin_amdgcn_readlane(k0_l, b), __builtin_amdgcn_readlane(sk_l, b),
+                           __builtin_amdgcn_readlane(k1_l, b), __builtin_amdgcn_readlane(sk1_l, b)};
+      // (the arguments are read anew for every block: kept over all of them they leave the loop over the tiles too few scalar registers)
+      auto args = (const __attribute__((address_space(4))) PrefillParams*)__builtin_amdgcn_kernarg_segment_ptr();
+      asm volatile("" : "+s"(args));
+      pf_block<kKeyHalf, kValHalf, kPick, kCtx>(*(const PrefillParams*)args, lds, blk, ask);
+      get();
+    }
+  }
+}
+
 }  // namespace mlahip
 using namespace mlahip;
 
@@ -545,7 +624,7 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
                                float* lse_out, const float* prev_out, int64_t prev_stride_t, int64_t prev_stride_h,
                                const float* prev_lse, const uint32_t* pick, int64_t pick_stride, int32_t pick_words,
                                hipStream_t stream, const void* k1_nope = nullptr, int64_t kn1_stride_h = 0, const void* k1_pe = nullptr,
-                               const void* v1 = nullptr, int64_t v1_stride_h = 0, const int32_t* cu_k1 = nullptr) {
+                               const void* v1 = nullptr, int64_t v1_stride_h = 0, const int32_t* cu_k1 = nullptr, int32_t* queue = nullptr) {
   MLA_REQUIRE(q_nope && q_pe && k_nope && k_pe && v && cu_q && cu_k && out, MLA_ERR_NULL, "%s: null pointer argument", what);
   MLA_REQUIRE(batch >= 0 && num_heads >= 1 && max_q_len >= 0 && batch <= 65535 && num_heads <= 65535 && window >= 0,
               MLA_ERR_SHAPE, "%s: batch=%d num_heads=%d max_q_len=%d window=%d", what, batch, num_heads, max_q_len, window);
@@ -567,10 +646,12 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
                                   pick_stride % 2 == 0 && (uintptr_t)pick % 8 == 0),
               MLA_ERR_SHAPE, "%s: picks go without a window, in 8-byte aligned rows of whole 64-key tiles", what);
   MLA_REQUIRE(!k1_nope || (k1_pe && v1 && cu_k1), MLA_ERR_NULL, "%s: null pointer argument", what);
-  MLA_REQUIRE(!k1_nope || (key_half && causal && window == 0), MLA_ERR_UNSUPPORTED,
-              "%s: context keys go in front of causal fp16 keys and values, without a window", what);
+  MLA_REQUIRE(!k1_nope || (key_half && causal && window == 0 && pick == nullptr), MLA_ERR_UNSUPPORTED,
+              "%s: context keys go in front of causal fp16 keys and values, without a window or picks", what);
   MLA_REQUIRE(((uintptr_t)k1_nope | (uintptr_t)k1_pe | (uintptr_t)v1) % 16 == 0 && kn1_stride_h % 8 == 0 && v1_stride_h % 8 == 0,
               MLA_ERR_SHAPE, "%s: rows must be 16-byte aligned", what);
+  MLA_REQUIRE(!queue || (batch <= 64 && num_heads % 8 == 0 && (uintptr_t)queue % 4 == 0), MLA_ERR_UNSUPPORTED,
+              "%s: a queue goes with up to 64 sequences and a multiple of eight heads (got %d, %d)", what, batch, num_heads);
   if (batch == 0 || max_q_len == 0) return MLA_OK;
   PrefillParams p;
   p.q_nope = (const __bf16*)q_nope; p.qn_st = qn_stride_t; p.qn_sh = qn_stride_h;
@@ -586,18 +667,24 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
   p.k1_nope = (const __bf16*)k1_nope; p.kn1_sh = kn1_stride_h; p.k1_pe = (const __bf16*)k1_pe;
   p.v1 = (const __bf16*)v1; p.v1_sh = v1_stride_h; p.cu_k1 = cu_k1;
   p.pick = pick; p.pick_st = pick_stride; p.pick_tiles = pick_words / 2;
-  static constexpr auto kernel_of = [](bool kh, bool vh, bool pk, bool ctx) {
-    return ctx  ? mla_prefill_varlen_kernel<true, true, false, true>
-           : kh ? (pk ? mla_prefill_varlen_kernel<true, true, true, false> : mla_prefill_varlen_kernel<true, true, false, false>)
-           : vh ? (pk ? mla_prefill_varlen_kernel<false, true, true, false> : mla_prefill_varlen_kernel<false, true, false, false>)
-                : (pk ? mla_prefill_varlen_kernel<false, false, true, false> : mla_prefill_varlen_kernel<false, false, false, false>);
+  p.max_blocks = (max_q_len + kPfRows - 1) / kPfRows;
+  p.queue = queue;
+  static constexpr auto kernel_of = [](auto queued, bool kh, bool vh, bool pk, bool ctx) {
+    constexpr bool kQ = decltype(queued)::value;
+    return ctx  ? mla_prefill_varlen_kernel<true, true, false, true, kQ>
+           : kh ? (pk ? mla_prefill_varlen_kernel<true, true, true, false, kQ> : mla_prefill_varlen_kernel<true, true, false, false, kQ>)
+           : vh ? (pk ? mla_prefill_varlen_kernel<false, true, true, false, kQ> : mla_prefill_varlen_kernel<false, true, false, false, kQ>)
+                : (pk ? mla_prefill_varlen_kernel<false, false, true, false, kQ> : mla_prefill_varlen_kernel<false, false, false, false, kQ>);
   };
   int rc = MLA_OK;
-  for (int i = 0; i < 7 && rc == MLA_OK; i++)              // (all of them: a caller's warm-up step need not be of the kind that it captures)
-    rc = ensure_dynamic_lds((const void*)kernel_of((i >> 1) == 2, (i >> 1) != 0, i & 1, i == 6), kPfLdsB, what);
+  for (int i = 0; i < 14 && rc == MLA_OK; i++)              // (all of them: a caller's warm-up step need not be of the kind that it captures)
+    rc = ensure_dynamic_lds((const void*)(i < 7 ? kernel_of(std::false_type{}, (i >> 1) == 2, (i >> 1) != 0, i & 1, i == 6)
+                                                : kernel_of(std::true_type{}, (i - 7) >> 1 == 2, (i - 7) >> 1 != 0, (i - 7) & 1, i == 13)),
+                            kPfLdsB, what);
   if (rc != MLA_OK) return rc;
-  auto* kern = kernel_of(key_half, val_half, pick != nullptr, k1_nope != nullptr);
-  dim3 grid((max_q_len + kPfRows - 1) / kPfRows, num_heads, batch);
+  auto* kern = queue ? kernel_of(std::true_type{}, key_half, val_half, pick != nullptr, k1_nope != nullptr)
+                     : kernel_of(std::false_type{}, key_half, val_half, pick != nullptr, k1_nope != nullptr);
+  const dim3 grid = queue ? dim3(kPfWorkgroups) : dim3(p.max_blocks, num_heads, batch);
   hipLaunchKernelGGL(kern, grid, dim3(256), kPfLdsB, stream, p);
   return check_launch("mla_prefill_varlen_kernel");
 }
@@ -651,23 +738,24 @@ extern "C" int mla_prefill_varlen_pick(const void* q_nope, int64_t qn_stride_t, 
                              nullptr, 0, 0, nullptr, pick, pick_stride, pick_words, stream);
 }
 
-// The causal attention of a step's new tokens over their context and themselves in one launch: what mla_prefill_varlen (causal 0) over
-// the context keys, continued causally over the new ones, returns.  k_nope, k_pe, v, cu_k: the new tokens', fp16
-// (MLA_PREFILL_KV_F16); k1_nope, k1_pe, v1, cu_k1: the context's, of the same types and token strides.  prev_out / prev_lse (or both
-// NULL): the state of earlier context chunks.
-extern "C" int mla_prefill_varlen_context(const void* q_nope, int64_t qn_stride_t, int64_t qn_stride_h, const void* q_pe,
-                                          int64_t qp_stride_t, int64_t qp_stride_h, const void* k_nope, int64_t kn_stride_t,
-                                          int64_t kn_stride_h, const void* k_pe, int64_t kp_stride_t, const void* v,
-                                          int64_t v_stride_t, int64_t v_stride_h, const int32_t* cu_q, const int32_t* cu_k,
-                                          const void* k1_nope, int64_t kn1_stride_h, const void* k1_pe, const void* v1,
-                                          int64_t v1_stride_h, const int32_t* cu_k1, int32_t batch, int32_t num_heads,
-                                          int32_t max_q_len, float scale, void* out, int64_t out_stride_t, int64_t out_stride_h,
-                                          int32_t out_dtype, float* lse_out, const float* prev_out, int64_t prev_stride_t,
-                                          int64_t prev_stride_h, const float* prev_lse, hipStream_t stream) {
-  MLA_REQUIRE(k1_nope && k1_pe && v1 && cu_k1, MLA_ERR_NULL, "mla_prefill_varlen_context: null pointer argument");
-  return prefill_varlen_impl("mla_prefill_varlen_context", q_nope, qn_stride_t, qn_stride_h, q_pe, qp_stride_t, qp_stride_h,
-                             k_nope, kn_stride_t, kn_stride_h, k_pe, kp_stride_t, v, v_stride_t, v_stride_h, cu_q, cu_k, batch,
-                             num_heads, max_q_len, 1, 0, scale, out, out_stride_t, out_stride_h, out_dtype, lse_out, prev_out,
-                             prev_stride_t, prev_stride_h, prev_lse, nullptr, 0, 0, stream, k1_nope, kn1_stride_h, k1_pe, v1,
-                             v1_stride_h, cu_k1);
+// Every option of the entries above in one, with a queue (NULL: none) and further keys (k1_nope, k1_pe, v1, cu_k1; NULL: none) in
+// front of causal ones of the same types and token strides: fp16 (MLA_PREFILL_KV_F16), without a window or picks.  queue: 1 KiB of
+// zeros, which the launch uses up; for up to 64 sequences and a multiple of eight heads.
+extern "C" int mla_prefill_varlen_queued(const void* q_nope, int64_t qn_stride_t, int64_t qn_stride_h, const void* q_pe,
+                                         int64_t qp_stride_t, int64_t qp_stride_h, const void* k_nope, int64_t kn_stride_t,
+                                         int64_t kn_stride_h, const void* k_pe, int64_t kp_stride_t, const void* v,
+                                         int64_t v_stride_t, int64_t v_stride_h, const int32_t* cu_q, const int32_t* cu_k,
+                                         const void* k1_nope, int64_t kn1_stride_h, const void* k1_pe, const void* v1,
+                                         int64_t v1_stride_h, const int32_t* cu_k1, int32_t batch, int32_t num_heads,
+                                         int32_t max_q_len, int32_t causal, int32_t window, float scale, const uint32_t* pick,
+                                         int64_t pick_stride, int32_t pick_words, void* out, int64_t out_stride_t,
+                                         int64_t out_stride_h, int32_t out_dtype, float* lse_out, const float* prev_out,
+                                         int64_t prev_stride_t, int64_t prev_stride_h, const float* prev_lse, int32_t* queue,
+                                         hipStream_t stream) {
+  MLA_REQUIRE(!pick || !prev_out, MLA_ERR_UNSUPPORTED, "mla_prefill_varlen_queued: picks go without an earlier result");
+  return prefill_varlen_impl("mla_prefill_varlen_queued", q_nope, qn_stride_t, qn_stride_h, q_pe, qp_stride_t, qp_stride_h, k_nope,
+                             kn_stride_t, kn_stride_h, k_pe, kp_stride_t, v, v_stride_t, v_stride_h, cu_q, cu_k, batch, num_heads,
+                             max_q_len, causal, window, scale, out, out_stride_t, out_stride_h, out_dtype, lse_out, prev_out,
+                             prev_stride_t, prev_stride_h, prev_lse, pick, pick_stride, pick_words, stream, k1_nope, kn1_stride_h,
+                             k1_pe, v1, v1_stride_h, cu_k1, queue);
 }

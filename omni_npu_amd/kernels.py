@@ -330,11 +330,13 @@ def kv_up_takes(kv_c: torch.Tensor, weight: torch.Tensor, num_heads: int) -> boo
             and not ((kv_c.data_ptr() | weight.data_ptr()) & 15))
 
 
-def kv_up(kv_c: torch.Tensor, weight: torch.Tensor, num_heads: int, keys_f16: bool, k_pe: Optional[torch.Tensor] = None):
+def kv_up(kv_c: torch.Tensor, weight: torch.Tensor, num_heads: int, keys_f16: bool, k_pe: Optional[torch.Tensor] = None,
+          clear: Optional[torch.Tensor] = None):
     """(k_nope [T,N,128], v [T,N,128], k_pe16) of latent rows kv_c [T,512] and an up-projection weight [N*256,512], bf16 both, in
     one launch (reference: ``kv_b_proj``, mla.py:405-413, 566-571).  Keys fp16 or bf16, values fp16; in memory a head's tokens
     follow each other, a token's key in front of its value.  ``k_pe`` (bf16 [T,64] or [T,1,64]): comes back as contiguous fp16
-    [T,64], by the same launch where its rows are on 16-byte boundaries."""
+    [T,64], by the same launch where its rows are on 16-byte boundaries.  ``clear``: a prefill_queue, which the launch fills with
+    zeros."""
     if not kv_up_takes(kv_c, weight, num_heads):
         raise ValueError("kv_up: bf16 kv_c [T,512] and weight [N*256,512] on the GPU, rows on 16-byte boundaries")
     t, pe16, pe_args = kv_c.shape[0], None, (None, 0, None, 0)
@@ -348,8 +350,11 @@ def kv_up(kv_c: torch.Tensor, weight: torch.Tensor, num_heads: int, keys_f16: bo
     kv = torch.empty(num_heads, t, 256, dtype=torch.float16, device=kv_c.device)
     if t:
         rc = _lib.load().mla_kv_up(kv_c.data_ptr(), kv_c.stride(0), weight.data_ptr(), weight.stride(0), t, num_heads, int(keys_f16),
-                                   kv.data_ptr(), 256, t * 256, *pe_args, _stream(kv_c))
+                                   kv.data_ptr(), 256, t * 256, *pe_args, clear.data_ptr() if clear is not None else None,
+                                   clear.numel() if clear is not None else 0, _stream(kv_c))
         _lib.check(rc, "mla_kv_up")
+    elif clear is not None:
+        clear.zero_()
     kv = kv.transpose(0, 1)
     k_nope = kv[..., :128]
     return k_nope if keys_f16 else k_nope.view(torch.bfloat16), kv[..., 128:], pe16
@@ -884,6 +889,16 @@ def sparse_decode(q_nope: torch.Tensor, q_rope: torch.Tensor, nope_cache: torch.
 # ------------------------------------------------------------------------------------------------
 _PREFILL_KV_F16 = 16                                       # added to the output dtype code: k_nope, k_pe, v hold fp16
 _PREFILL_V_F16 = 32                                        # v alone does
+_PREFILL_RESIDENT = 512                                    # blocks of 128 rows at work at once: two on each CU
+_PREFILL_QUEUE_WORDS = 256
+
+
+def prefill_queue(tokens: int, batch: int, max_q_len: int, num_heads: int, device: torch.device) -> Optional[torch.Tensor]:
+    """Memory for prefill_varlen's ``queue``, to be cleared first (kv_up does it on the way), or None where a launch has no use for
+    one: all of its blocks of 128 rows are at work at once, or their order is not one that the kernel works out."""
+    if batch > 64 or num_heads % 8 or num_heads * min(batch * -(-int(max_q_len) // 128), tokens // 128 + batch) <= _PREFILL_RESIDENT:
+        return None
+    return torch.empty(_PREFILL_QUEUE_WORDS, dtype=torch.int32, device=device)
 
 
 def prefill_takes_context(k_nope: torch.Tensor, k_pe: torch.Tensor, v: torch.Tensor, context: tuple) -> bool:
@@ -899,7 +914,8 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
                    cu_q: torch.Tensor, cu_k: torch.Tensor, max_q_len: int, scale: float, causal: bool,
                    out: torch.Tensor, lse_out: Optional[torch.Tensor] = None, window: Optional[int] = None,
                    prev_out: Optional[torch.Tensor] = None, prev_lse: Optional[torch.Tensor] = None,
-                   pick: Optional[torch.Tensor] = None, context: Optional[tuple] = None) -> torch.Tensor:
+                   pick: Optional[torch.Tensor] = None, context: Optional[tuple] = None,
+                   queue: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Varlen non-absorbed MLA attention (reference: the prefill FIA calls, src/omni_npu/attention/backends/mla.py:574-590
     and :415-431).  q_nope [T,N,128], q_pe [T,N,64], k_nope [Tk,N,128], k_pe [Tk,64] (shared by the heads), v [Tk,N,128],
     cu_q / cu_k int32 [B+1] device tensors, out [T,N,128] bf16 or fp32, lse_out fp32 [T,N].  ``window`` keeps only the
@@ -912,7 +928,8 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
     ``context`` = (k_nope, k_pe, v, cu_k) of further keys, which every row of a sequence sees: one launch for them (an unmasked call)
     and the causal call that continues from it (prefill_takes_context says whether it takes them).
     ``pick`` (int32 [T, W] bits, see topk's mask; W even and wide enough for the longest sequence; no window, no earlier
-    result): a token attends over the keys its bits name."""
+    result): a token attends over the keys its bits name.
+    ``queue``: prefill_queue's memory, holding zeros; the call uses it up."""
     if window is not None and window < 1:
         raise ValueError(f"prefill_varlen: window must be positive (got {window})")
     _need_cuda(q_nope, q_pe, k_nope, k_pe, v, cu_q, cu_k, out, lse_out)
@@ -956,17 +973,29 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
             raise TypeError("prefill_varlen: context keys go in front of causal ones of the same types and token strides, fp16, with "
                             "cu_k contiguous int32 [B+1], without a window or picks")
         _need_cuda(*context)
-        if context[0].shape[0] and k_nope.shape[0] and t:
+        if context[0].shape[0] == 0:
+            context = None
+    batch = cu_q.numel() - 1
+    if queue is not None:
+        _need_cuda(queue)
+        if batch > 64 or n % 8 or queue.dtype != torch.int32 or queue.numel() < _PREFILL_QUEUE_WORDS or not queue.is_contiguous():
+            raise TypeError("prefill_varlen: a queue (prefill_queue) goes with up to 64 sequences and a multiple of eight heads")
+    if k_nope.shape[0] and t and (context is not None or queue is not None):
+        extra = (None, 0, None, None, 0, None)
+        if context is not None:
             k1, pe1, v1, cu1 = context
-            prev = (prev_out.data_ptr(), prev_out.stride(0), prev_out.stride(1), prev_lse.data_ptr()) if prev_out is not None else (None, 0, 0, None)
-            rc = lib.mla_prefill_varlen_context(
-                q_nope.data_ptr(), q_nope.stride(0), q_nope.stride(1), q_pe.data_ptr(), q_pe.stride(0), q_pe.stride(1),
-                k_nope.data_ptr(), k_nope.stride(0), k_nope.stride(1), k_pe.data_ptr(), k_pe.stride(0), v.data_ptr(), v.stride(0),
-                v.stride(1), cu_q.data_ptr(), cu_k.data_ptr(), k1.data_ptr(), k1.stride(1), pe1.data_ptr(), v1.data_ptr(),
-                v1.stride(1), cu1.data_ptr(), cu_q.numel() - 1, n, int(max_q_len), float(scale), out.data_ptr(), out.stride(0),
-                out.stride(1), _DT[out.dtype] | kv_code, lse_out.data_ptr() if lse_out is not None else None, *prev, _stream(q_nope))
-            _lib.check(rc, "mla_prefill_varlen_context")
-            return out
+            extra = (k1.data_ptr(), k1.stride(1), pe1.data_ptr(), v1.data_ptr(), v1.stride(1), cu1.data_ptr())
+        prev = (prev_out.data_ptr(), prev_out.stride(0), prev_out.stride(1), prev_lse.data_ptr()) if prev_out is not None else (None, 0, 0, None)
+        picks = (pick.data_ptr(), pick.stride(0), pick.shape[1]) if pick is not None else (None, 0, 0)
+        rc = lib.mla_prefill_varlen_queued(
+            q_nope.data_ptr(), q_nope.stride(0), q_nope.stride(1), q_pe.data_ptr(), q_pe.stride(0), q_pe.stride(1),
+            k_nope.data_ptr(), k_nope.stride(0), k_nope.stride(1), k_pe.data_ptr(), k_pe.stride(0), v.data_ptr(), v.stride(0),
+            v.stride(1), cu_q.data_ptr(), cu_k.data_ptr(), *extra, batch, n, int(max_q_len), 1 if causal else 0, int(window or 0),
+            float(scale), *picks, out.data_ptr(), out.stride(0), out.stride(1), _DT[out.dtype] | kv_code,
+            lse_out.data_ptr() if lse_out is not None else None, *prev, queue.data_ptr() if queue is not None else None,
+            _stream(q_nope))
+        _lib.check(rc, "mla_prefill_varlen_queued")
+        return out
     if k_nope.shape[0] == 0 or t == 0:
         # no keys at all (a context chunk in which every sequence is empty): zeros and lse = -inf, as the kernel gives for
         # an empty key range (the earlier result itself when there is one); empty tensors have no address to hand over

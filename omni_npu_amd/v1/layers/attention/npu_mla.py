@@ -100,8 +100,9 @@ class NPUDeepseekMLAAttention(torch.nn.Module):
         q_pe = q[..., self.qk_nope_head_dim:]
         K.kv_rmsnorm_rope_cache(kv, self.kv_a_layernorm.weight, cos, sin, meta.slot_mapping, nope_c, rope_c,
                                 eps=self._eps(), kv_a_out=kv_a, k_pe_out=k_pe, q_rope=q_pe)
-        k_nope, k_pe, v, _ = impl._kv_up_rows(kv_a, k_pe)
         cu = meta.prefill.query_start_loc.to(torch.int32).contiguous()
+        queue = K.prefill_queue(t, cu.numel() - 1, meta.prefill.max_query_len, self.num_local_heads, dev)
+        k_nope, k_pe, v, _ = impl._kv_up_rows(kv_a, k_pe, queue)
         K.prefill_varlen(q[..., :self.qk_nope_head_dim], q_pe, k_nope, k_pe, v, cu, cu,
-                         meta.prefill.max_query_len, impl.scale, True, attn_output)
+                         meta.prefill.max_query_len, impl.scale, True, attn_output, queue=queue)
         return self.o_proj(attn_output.view(t, -1))[0]
