@@ -358,7 +358,10 @@ int mla_prefill_varlen_pick(const void* q_nope, int64_t qn_stride_t, int64_t qn_
  * prev_out / prev_lse as in mla_prefill_varlen_continue, pick as in mla_prefill_varlen_pick, or NULL.
  * queue (or NULL): 1 KiB of device memory that holds zeros, at most 64 sequences, heads a multiple of eight.  The launch is then one
  * resident set of workgroups that take the blocks of 128 query rows from it, instead of a workgroup to each; worth it from more than
- * 512 blocks on.  The launch uses the memory up: it has to be cleared for the next. */
+ * 512 blocks on.  The launch uses the memory up: it has to be cleared for the next.
+ * out_dtype + MLA_PREFILL_LONG, with a queue, fp16 keys and values, no window and no pick: 64 query rows to a wavefront, for sequences of
+ * a thousand rows and more over some thousand keys. */
+#define MLA_PREFILL_LONG 64
 int mla_prefill_varlen_queued(const void* q_nope, int64_t qn_stride_t, int64_t qn_stride_h, const void* q_pe,
                               int64_t qp_stride_t, int64_t qp_stride_h, const void* k_nope, int64_t kn_stride_t,
                               int64_t kn_stride_h, const void* k_pe, int64_t kp_stride_t, const void* v, int64_t v_stride_t,

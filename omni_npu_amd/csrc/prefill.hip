@@ -518,6 +518,63 @@ __device__ __forceinline__ void pf_block(const PrefillParams& p, char* lds, cons
   }
 }
 
+// The blocks of kRows rows of a launch, from the queues: block(params, block, ask), with ask() called once, behind the last tile.
+template <int kRows, bool kCtx, class Block>
+__device__ __forceinline__ void pf_from_queue(const PrefillParams& p0, char* lds, Block block) {
+  // Lane c keeps where sequence c's blocks stand in an XCD's queue: the sequences with the most keys first and their longest blocks
+  // first, so that what runs last is short.  Blocks that a sequence does not have are not in it.
+  const int lane = threadIdx.x & 63, per = p0.num_heads >> 3;   // heads of an XCD
+  int q0_l = 0, sq_l = 0, k0_l = 0, sk_l = 0, k1_l = 0, sk1_l = 0, before_l = 0, blocks_l = 0;
+  if (lane < p0.batch) {
+    q0_l = p0.cu_q[lane];
+    sq_l = p0.cu_q[lane + 1] - q0_l;
+    k0_l = p0.cu_k[lane];
+    sk_l = p0.cu_k[lane + 1] - k0_l;
+    if constexpr (kCtx) {
+      k1_l = p0.cu_k1[lane];
+      sk1_l = p0.cu_k1[lane + 1] - k1_l;
+    }
+    blocks_l = sq_l > 0 ? (sq_l + kRows - 1) / kRows : 0;
+    blocks_l = blocks_l < p0.max_blocks ? blocks_l : p0.max_blocks;
+  }
+  for (int c = 0; c < p0.batch; c++) {
+    const int keys_l = sk_l + sk1_l, kc = __builtin_amdgcn_readlane(keys_l, c), bc = __builtin_amdgcn_readlane(blocks_l, c);
+    before_l += kc > keys_l || (kc == keys_l && c < lane) ? bc * per : 0;
+  }
+  int xcd = blockIdx.x & 7, ticket = blockIdx.x >> 3, taken = 0;
+  int32_t* const queue = p0.queue;
+  auto ask = [&] {                                          // for the next ticket of queue xcd, behind those the launch began with
+    if (threadIdx.x == 0) taken = (int)(gridDim.x >> 3) + atomicAdd(queue + xcd * kPfQueue, 1);
+  };
+  auto get = [&] {
+    lds_barrier();                                          // (the wavefronts are done with the LDS)
+    if (threadIdx.x == 0) *(int*)lds = taken;
+    lds_barrier();
+    ticket = __builtin_amdgcn_readfirstlane(*(const int*)lds);
+    lds_barrier();
+  };
+  for (int queues = 8;;) {
+    const uint64_t at = __builtin_amdgcn_ballot_w64(ticket >= before_l && ticket < before_l + blocks_l * per);
+    if (at == 0) {
+      if (--queues == 0) return;
+      xcd = (xcd + 1) & 7;
+      ask();
+      get();
+      continue;
+    }
+    const int b = __builtin_ctzll(at), n = __builtin_amdgcn_readlane(blocks_l, b);
+    const int u = ticket - __builtin_amdgcn_readlane(before_l, b), h = u / n;
+    const PfBlock blk = {n - 1 - (u - h * n), h * 8 + xcd, __builtin_amdgcn_readlane(q0_l, b), __builtin_amdgcn_readlane(sq_l, b),
+                         __builtin_amdgcn_readlane(k0_l, b), __builtin_amdgcn_readlane(sk_l, b),
+                         __builtin_amdgcn_readlane(k1_l, b), __builtin_amdgcn_readlane(sk1_l, b)};
+    // (the arguments are read anew for every block: kept over all of them they leave the loop over the tiles too few scalar registers)
+    auto args = (const __attribute__((address_space(4))) PrefillParams*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    block(*(const PrefillParams*)args, blk, ask);
+    get();
+  }
+}
+
 // Workgroups go to the eight XCDs round-robin in launch order (x fastest), and each XCD has its own L2.  All query blocks of one
 // (sequence, head) stream the same keys and values, so both orders of the blocks below keep them on ONE XCD, next to each other: they
 // then run at the same time and all but the first find the K / V tiles in that L2.
@@ -556,62 +613,14 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
     if (qb * kPfRows >= blk.sq) return;
     pf_block<kKeyHalf, kValHalf, kPick, kCtx>(p, lds, blk, [] {});
   } else {
-    // Lane c keeps where sequence c's blocks stand in an XCD's queue: the sequences with the most keys first and their longest blocks
-    // first, so that what runs last is short.  Blocks that a sequence does not have are not in it.
-    const int lane = threadIdx.x & 63, per = p0.num_heads >> 3;   // heads of an XCD
-    int q0_l = 0, sq_l = 0, k0_l = 0, sk_l = 0, k1_l = 0, sk1_l = 0, before_l = 0, blocks_l = 0;
-    if (lane < p0.batch) {
-      q0_l = p0.cu_q[lane];
-      sq_l = p0.cu_q[lane + 1] - q0_l;
-      k0_l = p0.cu_k[lane];
-      sk_l = p0.cu_k[lane + 1] - k0_l;
-      if constexpr (kCtx) {
-        k1_l = p0.cu_k1[lane];
-        sk1_l = p0.cu_k1[lane + 1] - k1_l;
-      }
-      blocks_l = sq_l > 0 ? (sq_l + kPfRows - 1) / kPfRows : 0;
-      blocks_l = blocks_l < p0.max_blocks ? blocks_l : p0.max_blocks;
-    }
-    for (int c = 0; c < p0.batch; c++) {
-      const int keys_l = sk_l + sk1_l, kc = __builtin_amdgcn_readlane(keys_l, c), bc = __builtin_amdgcn_readlane(blocks_l, c);
-      before_l += kc > keys_l || (kc == keys_l && c < lane) ? bc * per : 0;
-    }
-    int xcd = lin & 7, ticket = lin >> 3, taken = 0;
-    int32_t* const queue = p0.queue;
-    auto ask = [&] {                                          // for the next ticket of queue xcd, behind those the launch began with
-      if (threadIdx.x == 0) taken = (int)(gridDim.x >> 3) + atomicAdd(queue + xcd * kPfQueue, 1);
-    };
-    auto get = [&] {
-      lds_barrier();                                          // (the wavefronts are done with the LDS)
-      if (threadIdx.x == 0) *(int*)lds = taken;
-      lds_barrier();
-      ticket = __builtin_amdgcn_readfirstlane(*(const int*)lds);
-      lds_barrier();
-    };
-    for (int queues = 8;;) {
-      const uint64_t at = __builtin_amdgcn_ballot_w64(ticket >= before_l && ticket < before_l + blocks_l * per);
-      if (at == 0) {
-        if (--queues == 0) return;
-        xcd = (xcd + 1) & 7;
-        ask();
-        get();
-        continue;
-      }
-      const int b = __builtin_ctzll(at), n = __builtin_amdgcn_readlane(blocks_l, b);
-      const int u = ticket - __builtin_amdgcn_readlane(before_l, b), h = u / n;
-      const PfBlock blk = {n - 1 - (u - h * n), h * 8 + xcd, __builtin_amdgcn_readlane(q0_l, b), __builtin_amdgcn_readlane(sq_l, b),
-                           __builtin_amdgcn_readlane(k0_l, b), __builtin_amdgcn_readlane(sk_l, b),
-                           __builtin_amdgcn_readlane(k1_l, b), __builtin_amdgcn_readlane(sk1_l, b)};
-      // (the arguments are read anew for every block: kept over all of them they leave the loop over the tiles too few scalar registers)
-      auto args = (const __attribute__((address_space(4))) PrefillParams*)__builtin_amdgcn_kernarg_segment_ptr();
-      asm volatile("" : "+s"(args));
-      pf_block<kKeyHalf, kValHalf, kPick, kCtx>(*(const PrefillParams*)args, lds, blk, ask);
-      get();
-    }
+    pf_from_queue<kPfRows, kCtx>(p0, lds, [&](const PrefillParams& p, const PfBlock& blk, auto ask) {
+      pf_block<kKeyHalf, kValHalf, kPick, kCtx>(p, lds, blk, ask);
+    });
   }
 }
 
 }  // namespace mlahip
+#include "prefill_long.hpp"
 using namespace mlahip;
 
 // out_dtype: 0 = bf16, 1 = fp32; window: 0 = every visible key, w = the newest w of them.  q_nope [T,N,128], q_pe [T,N,64], k_nope [Tk,N,128], k_pe [Tk,64], v [Tk,N,128].
@@ -630,7 +639,8 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
               MLA_ERR_SHAPE, "%s: batch=%d num_heads=%d max_q_len=%d window=%d", what, batch, num_heads, max_q_len, window);
   const bool key_half = (out_dtype & 16) != 0;             // k_nope, k_pe and v hold fp16 (MLA_PREFILL_KV_F16)
   const bool val_half = (out_dtype & 48) != 0;             // v alone does (MLA_PREFILL_V_F16)
-  out_dtype &= ~48;
+  const bool long_rows = (out_dtype & 64) != 0;            // the kernel of 64 rows to a wavefront (MLA_PREFILL_LONG)
+  out_dtype &= ~112;
   MLA_REQUIRE(out_dtype == 0 || out_dtype == 1, MLA_ERR_UNSUPPORTED, "%s: out dtype code %d", what, out_dtype);
   MLA_REQUIRE(scale > 0.f, MLA_ERR_UNSUPPORTED, "%s: the softmax scale must be positive (got %g)", what, (double)scale);
   MLA_REQUIRE(qn_stride_t % 8 == 0 && qn_stride_h % 8 == 0 && qp_stride_t % 8 == 0 && qp_stride_h % 8 == 0 &&
@@ -652,6 +662,8 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
               MLA_ERR_SHAPE, "%s: rows must be 16-byte aligned", what);
   MLA_REQUIRE(!queue || (batch <= 64 && num_heads % 8 == 0 && (uintptr_t)queue % 4 == 0), MLA_ERR_UNSUPPORTED,
               "%s: a queue goes with up to 64 sequences and a multiple of eight heads (got %d, %d)", what, batch, num_heads);
+  MLA_REQUIRE(!long_rows || (queue && key_half && window == 0 && pick == nullptr), MLA_ERR_UNSUPPORTED,
+              "%s: the kernel for long sequences takes a queue and fp16 keys and values, no window and no picks", what);
   if (batch == 0 || max_q_len == 0) return MLA_OK;
   PrefillParams p;
   p.q_nope = (const __bf16*)q_nope; p.qn_st = qn_stride_t; p.qn_sh = qn_stride_h;
@@ -682,6 +694,15 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
                                                 : kernel_of(std::true_type{}, (i - 7) >> 1 == 2, (i - 7) >> 1 != 0, (i - 7) & 1, i == 13)),
                             kPfLdsB, what);
   if (rc != MLA_OK) return rc;
+  rc = ensure_dynamic_lds((const void*)mla_prefill_long_kernel<false>, kPlLdsB, what);
+  if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)mla_prefill_long_kernel<true>, kPlLdsB, what);
+  if (rc != MLA_OK) return rc;
+  if (long_rows) {
+    p.max_blocks = (max_q_len + kPlRows - 1) / kPlRows;
+    auto* long_kern = k1_nope ? mla_prefill_long_kernel<true> : mla_prefill_long_kernel<false>;
+    hipLaunchKernelGGL(long_kern, dim3(kPlWorkgroups), dim3(256), kPlLdsB, stream, p);
+    return check_launch("mla_prefill_long_kernel");
+  }
   auto* kern = queue ? kernel_of(std::true_type{}, key_half, val_half, pick != nullptr, k1_nope != nullptr)
                      : kernel_of(std::false_type{}, key_half, val_half, pick != nullptr, k1_nope != nullptr);
   const dim3 grid = queue ? dim3(kPfWorkgroups) : dim3(p.max_blocks, num_heads, batch);

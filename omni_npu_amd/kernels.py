@@ -889,14 +889,37 @@ def sparse_decode(q_nope: torch.Tensor, q_rope: torch.Tensor, nope_cache: torch.
 # ------------------------------------------------------------------------------------------------
 _PREFILL_KV_F16 = 16                                       # added to the output dtype code: k_nope, k_pe, v hold fp16
 _PREFILL_V_F16 = 32                                        # v alone does
+_PREFILL_LONG = 64                                         # 64 rows to a wavefront
 _PREFILL_RESIDENT = 512                                    # blocks of 128 rows at work at once: two on each CU
 _PREFILL_QUEUE_WORDS = 256
+
+
+# What the kernel of 64 rows to a wavefront has to find to be the faster one.  It takes blocks of 256 rows, one to a CU: enough of
+# them for every CU, not much of them rows that do not exist, and enough keys per row for the start and the end of a block, which
+# nothing runs beside.  us per launch, 32 rows / 64 rows, at heads x sequences x rows, visible keys:
+#   128 x 4 x 2048, 17 408: 10 400 / 9 900   128 x 4 x 2048, 3072: 2181 / 2045   128 x 4 x 2048, 2048: 1417 / 1412
+#    32 x 1 x 8192, 4096: 722 / 642           32 x 1 x 2048, 17 408: 735 / 670     64 x 1 x 1017, 3580: 162 / 161
+#   few blocks:   16 x 1 x 2048, 33 792: 867 / 887
+#   ragged ones: 128 x 1 x 700, 16 734: 1037 / 1056   128 x 2 x 300, 8342: 534 / 548
+_PREFILL_LONG_ROWS, _PREFILL_LONG_KEYS = 1024, 2560
+
+
+def _prefill_long_rows(tokens: int, batch: int, num_heads: int) -> bool:
+    whole = -(-tokens // 256) if batch == 1 else tokens // 256
+    return (0 < batch <= 64 and num_heads % 8 == 0 and tokens >= _PREFILL_LONG_ROWS * batch and num_heads * whole >= _PREFILL_RESIDENT // 2
+            and (batch > 1 or whole * 256 <= 1.05 * tokens))
+
+
+def _prefill_blocks(tokens: int, batch: int, max_q_len: int, num_heads: int) -> int:
+    """At most so many blocks of 128 rows."""
+    return num_heads * min(batch * -(-int(max_q_len) // 128), tokens // 128 + batch)
 
 
 def prefill_queue(tokens: int, batch: int, max_q_len: int, num_heads: int, device: torch.device) -> Optional[torch.Tensor]:
     """Memory for prefill_varlen's ``queue``, to be cleared first (kv_up does it on the way), or None where a launch has no use for
     one: all of its blocks of 128 rows are at work at once, or their order is not one that the kernel works out."""
-    if batch > 64 or num_heads % 8 or num_heads * min(batch * -(-int(max_q_len) // 128), tokens // 128 + batch) <= _PREFILL_RESIDENT:
+    if batch > 64 or num_heads % 8 or not (_prefill_blocks(tokens, batch, max_q_len, num_heads) > _PREFILL_RESIDENT or
+                                           _prefill_long_rows(tokens, batch, num_heads)):
         return None
     return torch.empty(_PREFILL_QUEUE_WORDS, dtype=torch.int32, device=device)
 
@@ -915,7 +938,7 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
                    out: torch.Tensor, lse_out: Optional[torch.Tensor] = None, window: Optional[int] = None,
                    prev_out: Optional[torch.Tensor] = None, prev_lse: Optional[torch.Tensor] = None,
                    pick: Optional[torch.Tensor] = None, context: Optional[tuple] = None,
-                   queue: Optional[torch.Tensor] = None) -> torch.Tensor:
+                   queue: Optional[torch.Tensor] = None, long: Optional[bool] = None) -> torch.Tensor:
     """Varlen non-absorbed MLA attention (reference: the prefill FIA calls, src/omni_npu/attention/backends/mla.py:574-590
     and :415-431).  q_nope [T,N,128], q_pe [T,N,64], k_nope [Tk,N,128], k_pe [Tk,64] (shared by the heads), v [Tk,N,128],
     cu_q / cu_k int32 [B+1] device tensors, out [T,N,128] bf16 or fp32, lse_out fp32 [T,N].  ``window`` keeps only the
@@ -929,7 +952,8 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
     and the causal call that continues from it (prefill_takes_context says whether it takes them).
     ``pick`` (int32 [T, W] bits, see topk's mask; W even and wide enough for the longest sequence; no window, no earlier
     result): a token attends over the keys its bits name.
-    ``queue``: prefill_queue's memory, holding zeros; the call uses it up."""
+    ``queue``: prefill_queue's memory, holding zeros; the call uses it up.  ``long``: with the queue and fp16 keys and values, no window
+    and no picks, the kernel of 64 rows to a wavefront (None: where it is the faster one)."""
     if window is not None and window < 1:
         raise ValueError(f"prefill_varlen: window must be positive (got {window})")
     _need_cuda(q_nope, q_pe, k_nope, k_pe, v, cu_q, cu_k, out, lse_out)
@@ -980,6 +1004,15 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
         _need_cuda(queue)
         if batch > 64 or n % 8 or queue.dtype != torch.int32 or queue.numel() < _PREFILL_QUEUE_WORDS or not queue.is_contiguous():
             raise TypeError("prefill_varlen: a queue (prefill_queue) goes with up to 64 sequences and a multiple of eight heads")
+    if long is None and queue is not None:
+        seen = k_nope.shape[0] + (context[0].shape[0] if context is not None else 0) - (t // 2 if causal else 0)
+        long = kv_half and window is None and pick is None and _prefill_long_rows(t, batch, n) and seen >= _PREFILL_LONG_KEYS * batch
+        if not long and _prefill_blocks(t, batch, max_q_len, n) <= _PREFILL_RESIDENT:
+            queue = None
+    if long:
+        if queue is None or not kv_half or window is not None or pick is not None:
+            raise TypeError("prefill_varlen: long goes with a queue and fp16 keys and values, without a window or picks")
+        kv_code |= _PREFILL_LONG
     if k_nope.shape[0] and t and (context is not None or queue is not None):
         extra = (None, 0, None, None, 0, None)
         if context is not None:

@@ -46,7 +46,7 @@ def test_queue_gives_what_one_workgroup_per_block_gives(dev, n, q_lens, kind):
 
     def run(queue):
         out, lse = torch.full((t, n, 128), float("nan"), device=dev), torch.full((t, n), float("nan"), device=dev)
-        K.prefill_varlen(qn, qp, *own, cu, cu, max(q_lens), 0.07, True, out, lse, queue=queue, **opt)
+        K.prefill_varlen(qn, qp, *own, cu, cu, max(q_lens), 0.07, True, out, lse, queue=queue, long=False, **opt)
         return out, lse
     want = run(None)
     queue = torch.zeros(256, dtype=torch.int32, device=dev)
