@@ -1004,10 +1004,12 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
         _need_cuda(queue)
         if batch > 64 or n % 8 or queue.dtype != torch.int32 or queue.numel() < _PREFILL_QUEUE_WORDS or not queue.is_contiguous():
             raise TypeError("prefill_varlen: a queue (prefill_queue) goes with up to 64 sequences and a multiple of eight heads")
-    if long is None and queue is not None:
+    if long is None:
         seen = k_nope.shape[0] + (context[0].shape[0] if context is not None else 0) - (t // 2 if causal else 0)
         long = kv_half and window is None and pick is None and _prefill_long_rows(t, batch, n) and seen >= _PREFILL_LONG_KEYS * batch
-        if not long and _prefill_blocks(t, batch, max_q_len, n) <= _PREFILL_RESIDENT:
+        if long and queue is None:                             # (5 us to clear one, of a launch of some hundred)
+            queue = torch.zeros(_PREFILL_QUEUE_WORDS, dtype=torch.int32, device=q_nope.device)
+        elif not long and queue is not None and _prefill_blocks(t, batch, max_q_len, n) <= _PREFILL_RESIDENT:
             queue = None
     if long:
         if queue is None or not kv_half or window is not None or pick is not None:
