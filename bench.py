@@ -1252,7 +1252,7 @@ def main():
         "step_hbm_gbs": round(ab["total"] / (dev_step_avg * 1e-6) / 1e9, 1),
         "step_roofline_frac": round(max(ab["total"] / (HBM_PEAK_GBS * 1e9), flops / (MFMA_BF16_PEAK_TFLOPS * 1e12))
                                     / (dev_step_avg * 1e-6), 4),
-        "roofline": {"kernel": f"mla_decode_v3_kernel<false, false, {row_groups}, true>", "bound": "hbm", "achieved": round(achieved, 1),
+        "roofline": {"kernel": f"mla_decode_v3_kernel<false, false, {row_groups}, true>" if row_groups > 1 else "mla_decode_rows_kernel", "bound": "hbm", "achieved": round(achieved, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                      "traffic_source": traffic_src,
                      "kernel_us_avg": round(k_avg, 2), "kernel_us_back_to_back_avg": round(k_back_to_back, 2),

@@ -5,8 +5,10 @@ single-GPU path; every vendor op there is replaced by a HIP kernel of libmla_hip
   store_kv (mla.py:868-881)                  -> kernels.cache_write / cache_write_fp8   (one launch for both caches)
   FIA decode (mla.py:781-804)                -> kernels.decode / decode_fp8             (split-KV + reduce)
   FIA prefill (mla.py:574-590, 415-431)      -> kernels.prefill_varlen
+  kv_b_proj of a prefill (mla.py:405-413, 566-571) -> kernels.kv_up for a plain bf16 weight, else the module
   gather / merge (ops.py)                    -> kernels.gather_paged / merge_states
-The absorb and up-projection GEMMs stay torch.bmm (hipBLASLt), as in the reference (mla.py:309-315, 900-912).
+The absorb and W_UV GEMMs (mla.py:309-315, 900-912): kernels.absorb and the launch that merges the partials for a decode step's
+tokens, torch.bmm (hipBLASLt) beyond.
 Static sink tokens with or without a sliding window (mla.py:463-560, 705-779) run as ONE attention over the union of
 the keys: without a window the sink pages are simply the first pages of the block table; with one the dense decode
 kernel leaves out the blocks between the sink and the window (prefill: kernels.prefill_varlen with a band).  Out of scope and rejected loudly: decode context parallelism, mc2 masks.

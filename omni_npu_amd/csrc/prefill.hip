@@ -12,16 +12,17 @@
 // (five sub-tiles of 64 x 128 B) are copied global -> LDS without touching registers, double buffered; V^T operands come
 // from transposed LDS reads, so P^T stays in registers exactly as in the decode kernel.
 //
-// What bounds it: the socket's power cap.  On the 4 x 2048 over 16k, 128-head context launch the matrix pipe is busy 61 %
-// of the cycles and the clock settles at 1.67 GHz at 1350 W, so what pays is fewer instructions per score and what lets
-// the clock settle lower:
+// What bounds it: the socket's power cap.  On the 4 x 2048 over 16k, 128-head context launch the matrix pipe is busy 71 %
+// of the cycles, the LDS as much (a fragment read feeds one MFMA of a wavefront), and the clock settles at 1.4 GHz, so what pays is
+// fewer instructions per score and fewer bytes out of LDS.  Long sequences therefore run in prefill_long.hpp, which has half the reads;
+// this kernel keeps the short ones, windows, picks and bf16 keys:
 //  * a tile costs one fused multiply-add, one exponential, half a conversion and one add (the sum, of probabilities before
 //    they are rounded; v_dot2 over the rounded pairs would be half an instruction less and 2 % of a long chunk) per score.  A
 //    row's reference is its first tile's maximum and is raised only where a probability outgrows it by 2^13: no maximum
 //    and no rescaling in the steady state (136 -> 84 instructions per wavefront and 32 keys);
 //  * both 32-key blocks of a tile are scored before the first exponential, at a raised wave priority (s_setprio), so the
 //    two wavefronts of a SIMD fall out of step and one's vector work runs beside the other's MFMAs (11 110 -> 10 350 us;
-//    causal 4 x 2048 994 -> 860 us).  With the sum in fp32 10 615 us = 1.04 PFLOP/s, causal 853-883 us.
+//    causal 4 x 2048 994 -> 860 us).
 // Tried beside it: tiles without a mask in a code path of their own, with and without a prescribed interleaving of the second
 // block's MFMAs and the first block's exponentials (10 860-10 940 us); eight wavefronts of 32 rows, half the tile copies
 // (10 130 us, but causal launches 860 -> 917 and ragged prompts 321 -> 355); heavy query blocks first (no change).
