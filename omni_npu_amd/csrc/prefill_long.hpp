@@ -190,7 +190,7 @@ __device__ __forceinline__ void pl_block(const PrefillParams& p, char* lds, cons
     float sum[2][2];
 
     // Score j of block cur, in the order of use: keys 0..15 of the block are 0..15 (eight of each row half), keys 16..31 are 16..31.
-    // One score per slot: the FMA of one, the exponential of the one before, sum and conversion of the one before that.
+    // One score per slot: sum and conversion of one, the exponential of the next, the FMA of the one behind it.
     float arg[2], ex[3];
 #define PL_H(j) (((j) >> 3) & 1)
 #define PL_E(j) (((j) >> 4) * 8 + ((j) & 7))
@@ -210,17 +210,28 @@ __device__ __forceinline__ void pl_block(const PrefillParams& p, char* lds, cons
         pl_cvt(pb[h][PL_E(j) >> 1], ex[(j + 2) % 3], ex[j % 3]);
       }
     };
+    float ps[2] = {0.f, 0.f};
+    uint64_t over = 0;
     auto slot = [&](auto cur, auto tt) {                       // what slot t of a block does for its softmax
       constexpr int t = decltype(tt)::value;
-      if constexpr (t < 32) sm_fma(cur, std::integral_constant<int, t>{});
-      if constexpr (t >= 1 && t < 33) sm_exp(std::integral_constant<int, t - 1>{});
-      if constexpr (t >= 2 && t < 34) sm_add(std::integral_constant<int, t - 2>{});
+      if constexpr (t == 0) {
+        sm_fma(cur, std::integral_constant<int, 0>{});
+        sm_fma(cur, std::integral_constant<int, 1>{});
+        sm_exp(std::integral_constant<int, 0>{});
+      }
+      if constexpr (t < 30) sm_fma(cur, std::integral_constant<int, t + 2>{});
+      if constexpr (t < 31) sm_exp(std::integral_constant<int, t + 1>{});
+      sm_add(std::integral_constant<int, t>{});
+      if constexpr ((t & 15) == 15) {                          // 16 keys are done: has a row outgrown its reference?  (asked for a slot ahead)
+        ps[0] = sum[0][0] + sum[0][1];
+        ps[1] = sum[1][0] + sum[1][1];
+        over = __builtin_amdgcn_ballot_w64(fmaxf(ps[0], ps[1]) > kPfRaise);
+      }
     };
     // the sums of 16 keys, and what rows that outgrew their reference need
     auto settle = [&](auto cur, auto kb_) {
       constexpr int c = decltype(cur)::value, kb = decltype(kb_)::value;
-      float ps[2] = {sum[0][0] + sum[0][1], sum[1][0] + sum[1][1]};
-      if (__builtin_expect(__builtin_amdgcn_ballot_w64(fmaxf(ps[0], ps[1]) > kPfRaise) != 0, 0)) {
+      if (__builtin_expect(over != 0, 0)) {
         PL_NOP();
         pl_unroll<2>([&](auto h_) {
           constexpr int h = decltype(h_)::value;
@@ -301,7 +312,7 @@ __device__ __forceinline__ void pl_block(const PrefillParams& p, char* lds, cons
           if constexpr (t == 5) side();
         }
         if constexpr (kPv) {
-          if constexpr (t == 18) settle(cur, std::integral_constant<int, 0>{});
+          if constexpr (t == 16) settle(cur, std::integral_constant<int, 0>{});
           slot(cur, t_);
           if constexpr (t >= 16 && !(t & 1)) vf[(t - 16) >> 1] = vread((t - 16) >> 1);
         }
@@ -316,8 +327,6 @@ __device__ __forceinline__ void pl_block(const PrefillParams& p, char* lds, cons
         pl_unroll<16>([&](auto t_) {
           constexpr int t = decltype(t_)::value, kb = t >> 3, i = (t >> 1) & 3, h = t & 1;
           if constexpr (t == 8) {
-            slot(cur, std::integral_constant<int, 32>{});
-            slot(cur, std::integral_constant<int, 33>{});
             settle(cur, std::integral_constant<int, 1>{});
           }
           const u32x4 pr = {pb[h][kb * 4], pb[h][kb * 4 + 1], pb[h][kb * 4 + 2], pb[h][kb * 4 + 3]};
