@@ -895,19 +895,21 @@ _PREFILL_QUEUE_WORDS = 256
 
 
 # What the kernel of 64 rows to a wavefront has to find to be the faster one.  It takes blocks of 256 rows, one to a CU: enough of
-# them for every CU, not much of them rows that do not exist, and enough keys per row for the start and the end of a block, which
-# nothing runs beside.  us per launch, 32 rows / 64 rows, at heads x sequences x rows, visible keys:
-#   128 x 4 x 2048, 17 408: 10 400 / 9 900   128 x 4 x 2048, 3072: 2181 / 2045   128 x 4 x 2048, 2048: 1417 / 1412
-#    32 x 1 x 8192, 4096: 722 / 642           32 x 1 x 2048, 17 408: 735 / 670     64 x 1 x 1017, 3580: 162 / 161
-#   few blocks:   16 x 1 x 2048, 33 792: 867 / 887
-#   ragged ones: 128 x 1 x 700, 16 734: 1037 / 1056   128 x 2 x 300, 8342: 534 / 548
-_PREFILL_LONG_ROWS, _PREFILL_LONG_KEYS = 1024, 2560
+# them for every CU, not more of them rows that do not exist than in blocks of 128, and enough keys per row for the start and the end
+# of a block, which nothing runs beside.  us per launch, 32 rows / 64 rows, at heads x sequences x rows, keys in front of them:
+#   128 x 4 x 2048, 16 384: 10 400 / 9400   128 x 4 x 2048, 1024: 1495 / 1371   32 x 4 x 2048, 1024: 371 / 356
+#    64 x 1 x 1017, 3072: 166 / 153           32 x 1 x 4096, 0: 208 / 203         32 x 8 x 900, 4000: 718 / 664
+#   few keys:     128 x 4 x 2048, 0: 772 / 778
+#   few blocks:   16 x 1 x 2048, 32 768: 867 / 887
+#   ragged ones:  128 x 2 x 300, 8192: 534 / 548
+# Of several sequences only the sum of the lengths is known here: blocks of 256 then cost 64 rows more of each on average.
+_PREFILL_LONG_ROWS, _PREFILL_LONG_KEYS = 1024, 1792
 
 
 def _prefill_long_rows(tokens: int, batch: int, num_heads: int) -> bool:
     whole = -(-tokens // 256) if batch == 1 else tokens // 256
-    return (0 < batch <= 64 and num_heads % 8 == 0 and tokens >= _PREFILL_LONG_ROWS * batch and num_heads * whole >= _PREFILL_RESIDENT // 2
-            and (batch > 1 or whole * 256 <= 1.05 * tokens))
+    return (0 < batch <= 64 and num_heads % 8 == 0 and num_heads * whole >= _PREFILL_RESIDENT // 2
+            and (whole * 256 <= 1.05 * 128 * -(-tokens // 128) if batch == 1 else tokens >= _PREFILL_LONG_ROWS * batch))
 
 
 def _prefill_blocks(tokens: int, batch: int, max_q_len: int, num_heads: int) -> int:

@@ -41,7 +41,7 @@ def test_the_compiler_leaves_the_named_registers_alone(tmp_path):
 
 
 @pytest.mark.parametrize("tokens,batch,heads,long", [
-    (8192, 4, 128, True), (2048, 1, 32, True), (2048, 1, 16, False), (700, 1, 128, False), (600, 2, 128, False), (2048, 1, 20, False),
+    (8192, 4, 128, True), (2048, 1, 32, True), (2048, 1, 16, False), (700, 1, 128, True), (600, 1, 128, False), (600, 2, 128, False), (1017, 1, 64, True), (2048, 1, 20, False),
     (65 * 2048, 65, 128, False), (0, 0, 128, False), (1100, 1, 128, False), (1280, 1, 64, True),
 ])
 def test_rule_for_64_rows(tokens, batch, heads, long):
