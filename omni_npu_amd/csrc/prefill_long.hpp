@@ -6,9 +6,10 @@
 // that the card clocks down to 1.4 GHz.  64 rows halve the reads: 1.9 GHz.  The accumulators of 64 rows and the query are 224
 // registers, so a SIMD holds one wavefront, and nothing runs beside it: the softmax of a block of 32 keys is therefore written between
 // the matrix instructions of the next block's scores and of its own P.V, score by score, in statements that stay where they are
-// (left to itself the compiler gathers them, and the matrix pipe waits: 4700 clocks per tile of 64 keys against 3780; the matrix
+// (left to itself the compiler gathers them, and the matrix pipe waits: 4700 clocks per tile of 64 keys against 3780 and less; the matrix
 // instructions alone take 2600).  A workgroup has a CU to itself: four tiles of 64 keys in LDS, one barrier per tile.
-// 4 x 2048 tokens over 16k of context, 128 heads: 12 953 -> 12 314 us per layer.
+// 4 x 2048 tokens over 16k of context, 128 heads: 12 953 -> 12 314 us per layer, 11 816 beside 12 183 since
+// comparisons are asked for a slot ahead.
 #pragma once
 
 namespace mlahip {

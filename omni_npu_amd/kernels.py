@@ -897,7 +897,7 @@ _PREFILL_QUEUE_WORDS = 256
 # What the kernel of 64 rows to a wavefront has to find to be the faster one.  It takes blocks of 256 rows, one to a CU: enough of
 # them for every CU, not more of them rows that do not exist than in blocks of 128, and enough keys per row for the start and the end
 # of a block, which nothing runs beside.  us per launch, 32 rows / 64 rows, at heads x sequences x rows, keys in front of them:
-#   128 x 4 x 2048, 16 384: 10 400 / 9400   128 x 4 x 2048, 1024: 1495 / 1371   32 x 4 x 2048, 1024: 371 / 356
+#   128 x 4 x 2048, 16 384: 10 930 / 9790   128 x 4 x 2048, 1024: 1495 / 1371   32 x 4 x 2048, 1024: 371 / 356
 #    64 x 1 x 1017, 3072: 166 / 153           32 x 1 x 4096, 0: 208 / 203         32 x 8 x 900, 4000: 718 / 664
 #   few keys:     128 x 4 x 2048, 0: 772 / 778
 #   few blocks:   16 x 1 x 2048, 32 768: 867 / 887

@@ -86,6 +86,21 @@ def test_long_rows_match_fp64(dev, n, q_lens, k_lens, ctx_lens, causal, earlier)
     assert torch.equal(half, out.to(torch.bfloat16))
 
 
+def test_a_call_without_a_queue_takes_long_rows_where_they_are_faster(dev):
+    g = torch.Generator(device=dev).manual_seed(5)
+    n, t, c = 64, 1024, 1400
+    qn = torch.randn(t, n, 128, generator=g, device=dev).to(torch.bfloat16)
+    qp = torch.randn(t, n, 64, generator=g, device=dev).to(torch.bfloat16)
+    own, ctx = _keys(dev, [t], n, g), _keys(dev, [c], n, g)
+
+    def run(**opt):
+        return K.prefill_varlen(qn, qp, *own[:3], own[3], own[3], t, SCALE, True, torch.empty(t, n, 128, device=dev), context=ctx, **opt)
+    explicit = run(queue=torch.zeros(256, dtype=torch.int32, device=dev), long=True)
+    assert torch.equal(run(), explicit) and not torch.equal(run(long=False), explicit)
+    queue = torch.full((256,), 3, dtype=torch.int32, device=dev).zero_()
+    assert torch.equal(run(queue=queue), explicit)
+
+
 def test_long_rows_refuse_what_they_do_not_take(dev):
     q = torch.zeros(64, 8, 128, dtype=torch.bfloat16, device=dev)
     cu = torch.tensor([0, 64], dtype=torch.int32, device=dev)
