@@ -156,6 +156,7 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
     v_cur = v_hi;
     if (blk_end <= blk_begin) continue;
     const int key0 = blk_begin * kPlanBlk, key_end = blk_end * kPlanBlk;                   // the segment's keys
+    const int key_last = (key_end < L ? key_end : L) - 1;
     if (threadIdx.x == 0) {
       if (blk_begin == 0) p.seg_ids[2 * b] = chunk + b;
       if (key_end >= L) p.seg_ids[2 * b + 1] = chunk + b;
@@ -197,13 +198,14 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
 
     // ---- copies ----
     const int skip = !kWindow ? 0 : 32 * (p.win_skip ? p.win_skip[b] : window_len(((ConstI32Ptr)p.seq_lens)[b], qlen, p.win_sink, p.win_size).skip);
-    // Where the wavefront's keys of an iteration lie: the number of their page as it stands (keys behind the sequence's last one
-    // repeat it: they are masked), or the cache rows of the eight, lane l that of key l % 8.
+    // Where the wavefront's keys of an iteration lie: the number of their page as it stands, or the cache rows of the eight, lane l
+    // that of key l % 8.  An iteration's keys behind the segment's last one repeat it (they are masked): the next chunk's keys may be
+    // new rows that only that chunk's workgroups store (kWrite), and 0 x V makes a NaN of an infinity.
     ConstI32Ptr bt = (ConstI32Ptr)(p.block_table) + (kList ? 0 : (int64_t)b * p.bt_stride);
     auto in_cache = [&](int key) { return kWindow && key >= p.win_sink ? key + skip : key; };
     auto place_of = [&](int it) {
       int key = key0 + it * kIter + wave * 8 + (kList ? lane & 7 : 0);
-      key = key < L ? key : L - 1;
+      key = key < key_last ? key : key_last;
       if constexpr (kList) return p.sparse_rows[(int64_t)b * p.sparse_stride + key];
       const int page = in_cache(key) >> 7;
       return bt[page < p.max_blocks ? page : p.max_blocks - 1];
@@ -223,17 +225,17 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
         const char* np = (const char*)(p.nope + pg * p.nope_sp);
         const char* rp = (const char*)(p.rope + pg * p.rope_sp);
         const int first = key0 + it * kIter + wave * 8;      // (the eight keys lie in one page, and in the sink or behind it)
-        const int shift = in_cache(first < L ? first : L - 1) - (first < L ? first : L - 1);
+        const int first_read = first < key_last ? first : key_last, shift = in_cache(first_read) - first_read;
 #pragma unroll
         for (int j = 0; j < 8; j++) {
           int key = first + j;
-          key = ((key < L ? key : L - 1) + shift) & (kPage - 1);
+          key = ((key < key_last ? key : key_last) + shift) & (kPage - 1);
           const char* src = np + (uint64_t)(uint32_t)key * n_sr2;
           if constexpr (kNt) dma16_sv_m0add_nt(src, copy_off ^ (uint32_t)(j << 5), dst, j * 1024);
           else dma16_sv_m0add(src, copy_off ^ (uint32_t)(j << 5), dst, j * 1024);
         }
         int key = first + rope_j;
-        key = ((key < L ? key : L - 1) + shift) & (kPage - 1);
+        key = ((key < key_last ? key : key_last) + shift) & (kPage - 1);
         const char* src = rp + ((uint64_t)(uint32_t)key * r_sr2 + rope_off);
         if constexpr (kNt) dma16_v_nt(src, rdst);
         else dma16_v(src, rdst);

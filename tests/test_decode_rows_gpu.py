@@ -101,3 +101,54 @@ def test_sink_and_window(dev, heads, q_len, window):
     K.decode(qn.to(dev), qr.to(dev), nope.to(dev), rope.to(dev), table.to(dev), torch.tensor(lens, dtype=torch.int32, device=dev), scale,
              out, q_len=q_len, sink_len=sink, window=window)
     attn_close(out, ref, 2e-2, 2e-3)
+
+
+def _segments(lens, rows, chunks):
+    """(sequence, first key, end) of every segment of the chunk plan (csrc/decode_params.hpp), `chunks` the most it may cut."""
+    units = [-(-n // 32) + 8 for n in lens]
+    total, few = sum(units), 8192 // rows
+    fine, cut = total // 2, total // 4
+    n = max(1, min(chunks, fine if fine <= few else max(cut, few)))
+    out = []
+    for c in range(n):
+        lo, hi, at = c * total // n, (c + 1) * total // n, 0
+        for b, u in enumerate(units):
+            first, end = max(lo - at - 8, 0), min(hi, at + u) - at - 8
+            if lo < at + u and end > first:
+                out.append((b, 32 * first, 32 * end))
+            at += u
+    return out
+
+
+@pytest.mark.parametrize("heads,q_len,lens,splits", [
+    (16, 1, [254, 504, 766], 8), (40, 1, [254, 504, 766], 8),                                  # one and two workgroups to a chunk
+    (16, 2, [61 + (71 * i) % 900 for i in range(40)], 5),
+    (8, 3, [40 + (53 * i) % 500 for i in range(80)], 3),                                       # more sequences than lanes
+])
+def test_folded_cache_write_behind_a_short_last_iteration(dev, heads, q_len, lens, splits):
+    """A segment of an odd number of 32-key blocks ends inside an iteration of 64 keys.  Where the next chunk begins with the request's
+    new rows, which only that chunk's workgroups store, nothing of what their slots held before may be read."""
+    assert len(lens) * splits <= 256                          # (then the plan may cut as many chunks as it is asked for)
+    exposed = [(b, end) for b, first, end in _segments(lens, heads * q_len, len(lens) * splits)
+               if (end - first) % 64 == 32 and end < lens[b] and end + 32 > lens[b] - q_len]
+    assert exposed                                            # such segments are what this test is about
+    c = _with_lens(heads, lens, q_len, seed=5)
+    t = len(lens) * q_len
+    slots = torch.cat([O.slots_for(c["block_table"], b, n - q_len, n) for b, n in enumerate(lens)])
+    for pool in (c["nope"], c["rope"]):
+        flat = pool.view(-1, pool.shape[-1])
+        flat[slots[0::2]], flat[slots[1::2]] = float("inf"), float("nan")
+    got = []
+    for folded in (False, True):
+        nope, rope = c["nope"].to(dev), c["rope"].to(dev)
+        out = torch.full((t, heads, 512), float("nan"), dtype=torch.bfloat16, device=dev)
+        lse = torch.full((t, heads), float("nan"), dtype=torch.float32, device=dev)
+        args = [c["q_nope"].to(dev), c["q_rope"].to(dev), nope, rope, c["block_table"].to(dev), c["seq_lens"].to(dev), c["scale"], out]
+        new = (c["new_c"].to(dev), c["new_r"].to(dev), slots.to(dev))
+        if not folded:
+            K.cache_write(*new, nope, rope)
+        K.decode(*args, q_len=q_len, num_splits=splits, lse_out=lse, new_rows=new if folded else None)
+        got.append([x.cpu() for x in (out, lse, nope, rope)])
+    assert torch.isfinite(got[0][0]).all()
+    for two, one in zip(*got):
+        assert torch.equal(two, one)
