@@ -250,7 +250,7 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
         int t = __builtin_amdgcn_readfirstlane(div_small(r0, p.num_heads)), h = r0 - t * p.num_heads;
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-          const bool ok = r0 + k < rows;                     // rows that do not exist read row 0 of the sequence
+          const bool ok = r0 + k < rows;                     // (a row of the four that does not exist: row 0 of the sequence)
           const __bf16* src = p.q_nope + (int64_t)(ok ? q0 + t : q0) * p.qn_st + (int64_t)(ok ? h : 0) * p.qn_sh;
           const int r16 = (wave & 3) * 4 + k;
           dma16_sv(src, (uint32_t)((lane ^ swz_nope(r16)) << 4), lds0 + kBufB + (wave * 4 + k) * 1024);
@@ -270,14 +270,15 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
     const int iters = (key_end - key0 + kIter - 1) / kIter;
     f32x4 acc[4][2];                                         // [16 of the wavefront's 64 columns][row group]
     float m_ref = 0.f, l_run = 0.f, seen = -INFINITY;
-    // the rows' references out of every key group's candidates (all wavefronts take part)
+    // The rows' references out of every key group's candidates (all wavefronts take part).  Rows that do not exist have whatever LDS
+    // held for a query: above a reference of infinity none of their scores asks for a restart.
     auto agree = [&](float mine) {
       mine = fmaxf(mine, __shfl_xor(mine, 16, 64));
       mine = fmaxf(mine, __shfl_xor(mine, 32, 64));
       if (g == 0) *(float*)(lds + kMaxOff + (kg * kRows + rg * 16 + l16) * 4) = mine;
       lds_barrier();
       const float* at = (const float*)(lds + kMaxOff) + rg * 16 + l16;
-      return fmaxf(fmaxf(at[0], at[kRows]), fmaxf(at[2 * kRows], at[3 * kRows]));
+      return row < rows ? fmaxf(fmaxf(at[0], at[kRows]), fmaxf(at[2 * kRows], at[3 * kRows])) : INFINITY;
     };
     int restarts_left = 4;                                   // (each raises a reference by more than 2^100: fp32 has room for three)
     bool fresh = true;

@@ -152,3 +152,23 @@ def test_folded_cache_write_behind_a_short_last_iteration(dev, heads, q_len, len
     assert torch.isfinite(got[0][0]).all()
     for two, one in zip(*got):
         assert torch.equal(two, one)
+
+
+@pytest.mark.parametrize("heads", [8, 20, 24, 40])
+def test_rows_that_do_not_exist_take_no_part(dev, heads):
+    """With heads that are no multiple of 16, what the launch before left in LDS must not matter: scores of rows that do not exist once
+    asked for restarts, which move the references of the rows that do."""
+    c = _with_lens(heads, [700, 333], 1, seed=heads)
+    args = [c[k].to(dev) for k in ("q_nope", "q_rope", "nope", "rope", "block_table", "seq_lens")]
+    table, lens = torch.arange(256, dtype=torch.int32, device=dev).view(256, 1), torch.full((256,), 64, dtype=torch.int32, device=dev)
+    cache = torch.zeros(256, 128, 576, dtype=torch.bfloat16, device=dev)
+    got = []
+    for left in (0., 3e4):
+        q = torch.full((256, 32, 576), left, dtype=torch.bfloat16, device=dev)
+        waste = torch.empty(256, 32, 512, dtype=torch.bfloat16, device=dev)
+        K.decode(q[..., :512], q[..., 512:], cache[..., :512], cache[..., 512:], table, lens, c["scale"], waste, num_splits=1)
+        out = torch.empty(2, heads, 512, dtype=torch.bfloat16, device=dev)
+        lse = torch.empty(2, heads, dtype=torch.float32, device=dev)
+        K.decode(*args, c["scale"], out, num_splits=1, lse_out=lse)
+        got.append((out.cpu(), lse.cpu()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
