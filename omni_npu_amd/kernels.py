@@ -1001,6 +1001,9 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
         _need_cuda(*context)
         if context[0].shape[0] == 0:
             context = None
+        elif k_nope.shape[0] == 0:                             # no causal key in any sequence
+            return prefill_varlen(q_nope, q_pe, *context[:3], cu_q, context[3], max_q_len, scale, False, out, lse_out, prev_out=prev_out,
+                                  prev_lse=prev_lse, queue=queue, long=long)
     batch = cu_q.numel() - 1
     if queue is not None:
         _need_cuda(queue)

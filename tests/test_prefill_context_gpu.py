@@ -72,6 +72,28 @@ def test_context_in_front_of_causal_keys(dev, q_lens, ctx_lens, n, earlier):
     assert torch.equal(half, out.bfloat16())
 
 
+@pytest.mark.parametrize("q_lens,ctx_lens,n", [([130], [200], 3), ([31, 5, 300], [64, 0, 190], 8)])
+@pytest.mark.parametrize("earlier", [False, True])
+def test_context_without_causal_keys(dev, q_lens, ctx_lens, n, earlier):
+    """No causal key in any sequence: every row still sees the context keys."""
+    g = torch.Generator(device=dev).manual_seed(n)
+    t = sum(q_lens)
+    q = torch.randn(t, n, 192, device=dev, generator=g).bfloat16()
+    own, ctx = _keys(dev, [0] * len(q_lens), n, g), _keys(dev, ctx_lens, n, g)
+    cu_q = torch.tensor([0] + q_lens, dtype=torch.int32).cumsum(0).to(torch.int32).to(dev)
+    parts, prev = [(ctx, False)], {}
+    if earlier:
+        far = _keys(dev, [77] * len(q_lens), n, g)
+        parts.insert(0, (far, False))
+        po, pl = torch.empty(t, n, 128, device=dev), torch.empty(t, n, device=dev)
+        K.prefill_varlen(q[..., :128], q[..., 128:], *far[:3], cu_q, far[3], max(q_lens), SCALE, False, po, pl)
+        prev = dict(prev_out=po, prev_lse=pl)
+    out, lse = torch.full((t, n, 128), float("nan"), device=dev), torch.empty(t, n, device=dev)
+    K.prefill_varlen(q[..., :128], q[..., 128:], *own[:3], cu_q, own[3], max(q_lens), SCALE, True, out, lse, context=ctx, **prev)
+    ref = _ref(q[..., :128], q[..., 128:], parts, q_lens, n)
+    assert ((out - ref).abs().mean() / ref.abs().mean()).item() <= 4e-4 and (out - ref).abs().max().item() <= 4e-3
+
+
 def test_what_it_does_not_take(dev):
     g = torch.Generator(device=dev).manual_seed(0)
     own, ctx = _keys(dev, [70], 3, g), _keys(dev, [100], 3, g)
