@@ -302,7 +302,8 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
     # rope rows fp16 (11 bits instead of 8, at the same speed) for a model whose rope rows, queries, keys and values stay between
     # 2^-14 and 65504.
     prefill_kv_fp16 = False
-    # (masked prompts are offered for a plain weight only, whose product W_UK and W_UV stand for everywhere else)
+    # (masked prompts are offered for a plain weight only, whose product W_UK and W_UV stand for everywhere else; a layer with an adapter
+    # or hooks is called)
     keys_bf16_values_f16 = True
 
     def __init__(self, num_heads: int, head_size: int, scale: float, num_kv_heads: int, alibi_slopes: Optional[list],

@@ -191,6 +191,13 @@ def _caller_wrote_cache(impl, attn_metadata, num_tokens: int) -> bool:
     return meta is attn_metadata and rows >= num_tokens
 
 
+def _is_its_weight(layer) -> bool:
+    """Whether calling the layer multiplies by its weight and does nothing else, as far as it shows: no hooks, no forward of the
+    object's own, no adapter (which shows the weight of the layer that it keeps in base_layer)."""
+    return not (getattr(layer, "_forward_hooks", None) or getattr(layer, "_forward_pre_hooks", None) or hasattr(layer, "base_layer")
+                or "forward" in getattr(layer, "__dict__", ()))
+
+
 class HalfUpProjection:
     """Keys and values of prefill tokens, the values in fp16 where the model's up-projection is a plain weight."""
 
@@ -200,7 +207,7 @@ class HalfUpProjection:
     # attention 12.6 -> 11.5 ms); other plain weights go through the same GEMM on fp16 copies of its operands.
     # Keys are fp16 too: eleven bits instead of eight.  Set prefill_kv_fp16 = False for a model whose keys or values can exceed
     # 65504: the module is called then, unless keys_bf16_values_f16 says that kernels.kv_up may write bf16 keys and fp16 values
-    # (clamped at 65504, as the prefill kernel clamps the module's).
+    # (clamped at 65504, as the prefill kernel clamps the module's) where the module is no more than its weight.
     keys_bf16_values_f16 = False
     prefill_kv_fp16 = True
 
@@ -223,7 +230,7 @@ class HalfUpProjection:
 
     def _kv_up_weight(self, kv_c: torch.Tensor) -> Optional[torch.Tensor]:
         """The up-projection weight if keys and values are to come from kernels.kv_up and it takes the latent rows kv_c."""
-        w = self._plain_up_weight() if self.prefill_kv_fp16 or self.keys_bf16_values_f16 else None
+        w = self._plain_up_weight() if self.prefill_kv_fp16 or (self.keys_bf16_values_f16 and _is_its_weight(self.kv_b_proj)) else None
         return w if w is not None and self.qk_nope_head_dim == self.v_head_dim == 128 and K.kv_up_takes(kv_c, w, self.num_heads) \
             else None
 

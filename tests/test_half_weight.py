@@ -46,3 +46,42 @@ def test_nothing_is_kept_on_the_layer():
     before = set(vars(up))
     up._half_up_weight()
     assert set(vars(up)) == before and not [v for v in vars(up).values() if isinstance(v, (torch.Tensor, tuple))]
+
+
+class _Adapter(torch.nn.Module):
+    """An adapter around a layer: it shows the layer's weight and adds to its result."""
+
+    def __init__(self, base_layer):
+        super().__init__()
+        self.base_layer, self.bias = base_layer, None
+
+    @property
+    def weight(self):
+        return self.base_layer.weight
+
+    def forward(self, x):
+        return self.base_layer(x) + 1
+
+
+def _instance_forward(layer):
+    base = layer.forward
+    layer.forward = lambda x: base(x) + 1
+
+
+@pytest.mark.parametrize("how", ["plain", "adapter", "hook", "pre-hook", "forward"])
+def test_masked_prompts_honour_a_layer_that_is_more_than_its_weight(monkeypatch, how):
+    """The sparse backend's prompts use the weight itself only where calling the layer means no more than that."""
+    monkeypatch.setattr("omni_npu_amd.kernels.kv_up_takes", lambda *a: True)
+    layer = torch.nn.Linear(512, 256, bias=False, dtype=torch.bfloat16)
+    if how == "hook":
+        layer.register_forward_hook(lambda m, args, out: out + 1)
+    if how == "pre-hook":
+        layer.register_forward_pre_hook(lambda m, args: (args[0] + 1,))
+    if how == "forward":
+        _instance_forward(layer)
+    up = HalfUpProjection()
+    up.num_heads, up.qk_nope_head_dim, up.v_head_dim, up.kv_lora_rank = 1, 128, 128, 512
+    up.kv_b_proj = _Adapter(layer) if how == "adapter" else layer
+    up.prefill_kv_fp16, up.keys_bf16_values_f16 = False, True
+    got = up._kv_up_weight(torch.zeros(3, 512, dtype=torch.bfloat16))
+    assert (got is layer.weight) if how == "plain" else got is None
