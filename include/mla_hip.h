@@ -209,6 +209,13 @@ int mla_splitkv_reduce_vup(const void* workspace, size_t workspace_bytes, const 
                            int32_t num_splits, int32_t num_tokens, const void* w_uv, int64_t w_stride_n,
                            int64_t w_stride_k, void* out, int64_t out_stride_t, int64_t out_stride_h,
                            mlahip_stream_t stream);
+/* The same for partials of mla_decode_fp8 or mla_decode_fp8_window_split, whose launches cut the work otherwise.  (Either entry
+ * point merges either kind of partials rightly; each is shaped for the number of partials that its own kind leaves.) */
+int mla_splitkv_reduce_vup_fp8(const void* workspace, size_t workspace_bytes, const int32_t* seq_lens,
+                               const int32_t* query_start_loc, int32_t batch, int32_t max_q_len, int32_t num_heads,
+                               int32_t num_splits, int32_t num_tokens, const void* w_uv, int64_t w_stride_n,
+                               int64_t w_stride_k, void* out, int64_t out_stride_t, int64_t out_stride_h,
+                               mlahip_stream_t stream);
 
 /* Same decode over the fp8-e4m3 block-scaled cache written by mla_cache_write_fp8 (row stride exactly 656 bytes,
  * page size 128).  Tiles are dequantised to bf16 on chip and take the bf16 MFMA path ("dequantise, then attend").

@@ -199,7 +199,9 @@ extern "C" int mla_splitkv_reduce(const void* workspace, size_t workspace_bytes,
   cp.corr_scale = cp.lse_part + rows; cp.corr_row = (const __bf16* const*)(cp.lse_part + 2 * rows);
   cp.seg_ids = (const int32_t*)(cp.lse_part + 4 * rows);
   cp.seq_lens = seq_lens; cp.qsl = query_start_loc;
-  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = plan_form(batch, num_splits, r_max).chunks;
+  // (the plan of the bf16 cache: where the fp8 cache's is another one, up to 512 rows, both leave more than a dozen partials per sequence,
+  // which is all that launch_chunk_reduce asks)
+  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = plan_form(batch, num_splits, r_max, true).chunks;
   cp.out = (__bf16*)out; cp.out_st = out_stride_t; cp.out_sh = out_stride_h;
   cp.lse_out = lse_out; cp.lse_st = num_heads;
   return launch_chunk_reduce(cp, stream);

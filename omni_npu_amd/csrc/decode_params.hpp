@@ -74,7 +74,7 @@ constexpr int kPlanCUs = 256;                              // MI355X
 // one of 1k keys 26.1 / 22.9, 4 of 1k-3k 32.4 / 29.6 (128 chunks), but 8 of 2k-4k 35.0 / 39.4 (256), 64 of 4k-8k 123 / 156.  Queued
 // launches, 12 requests x 128 heads: 300-3000 keys (144 workgroups of 128 rows) 36.5 / 34.6, 3k-5k (240) 46.3 / 48.3.
 struct PlanForm { int rg, chunks; };
-inline PlanForm plan_form(int64_t batch, int64_t num_splits, int64_t query_rows, bool rows32 = false) {
+inline PlanForm plan_form(int64_t batch, int64_t num_splits, int64_t query_rows, bool rows32) {
   const int64_t total = batch * num_splits, groups = (query_rows + 127) / 128, wgs = total * groups;
   if (query_rows > 64 && wgs * 4 <= kPlanCUs) return {1, (int)total};
   if (query_rows > 64 && (wgs * 2 <= kPlanCUs || (wgs < kPlanCUs && num_splits > 3))) {

@@ -166,12 +166,12 @@ Absorbed absorb(const Tensor& q, const Tensor& w_uk, int64_t t, const NewRows* r
 }
 // Merge of the partials and the value up-projection into out (mla.py:309-315).
 void merge_vup(const Tensor& ws, const Tensor& lens, const OptTensor& qsl, int64_t batch, int64_t q_len, int64_t n, int splits,
-               int64_t t, const Tensor& w_uv, const Tensor& out, Stream st) {
+               int64_t t, const Tensor& w_uv, const Tensor& out, bool fp8, Stream st) {
   const int32_t* qs = qsl ? (const int32_t*)qsl->data_ptr() : nullptr;
   if (t <= kVupMaxTokens) {
-    check(mla_splitkv_reduce_vup(ws.data_ptr(), ws.numel(), (const int32_t*)lens.data_ptr(), qs, (int)batch, (int)q_len, (int)n,
-                                 splits, (int)t, w_uv.data_ptr(), w_uv.stride(0), w_uv.stride(1), out.data_ptr(), out.stride(0),
-                                 kVDim, st), "mla_splitkv_reduce_vup");
+    const auto merge = fp8 ? mla_splitkv_reduce_vup_fp8 : mla_splitkv_reduce_vup;
+    check(merge(ws.data_ptr(), ws.numel(), (const int32_t*)lens.data_ptr(), qs, (int)batch, (int)q_len, (int)n, splits, (int)t,
+                w_uv.data_ptr(), w_uv.stride(0), w_uv.stride(1), out.data_ptr(), out.stride(0), kVDim, st), "mla_splitkv_reduce_vup");
     return;
   }
   Tensor o = at::empty({n, t, kNope}, out.options());
@@ -236,7 +236,7 @@ bool mla_decode(const Tensor& q, const Tensor& nope, const OptTensor& rope, cons
                                 c.rope->data_ptr(), c.r_sp, c.r_sr, c.pages, bt, bts, mb, lens, qs, (int)b, (int)q_len, (int)n,
                                 (float)scale, ws.data_ptr(), ws.numel(), splits, st), "mla_decode_bf16_split");
   }
-  merge_vup(ws, seq_lens, qsl, b, q_len, n, splits, t, w_uv, out, st);
+  merge_vup(ws, seq_lens, qsl, b, q_len, n, splits, t, w_uv, out, fp8, st);
   return true;
 }
 
@@ -266,7 +266,7 @@ bool sparse_decode(const Tensor& q, const Tensor& nope, const Tensor& rope, cons
                                (const int32_t*)rows.data_ptr(), rows.stride(0), (const int32_t*)counts.data_ptr(), (int)t, (int)n,
                                (float)scale, nullptr, 0, 0, nullptr, ws.data_ptr(), ws.numel(), splits, st),
         "dsa_sparse_decode_bf16");
-  merge_vup(ws, counts, std::nullopt, t, 1, n, splits, t, w_uv, out, st);
+  merge_vup(ws, counts, std::nullopt, t, 1, n, splits, t, w_uv, out, false, st);
   return true;
 }
 

@@ -38,7 +38,10 @@ constexpr int kMergeRowOff = kVupWB + 16384;      // kFew: the eight wavefronts'
 constexpr int kVupPairOff = kMergeRowOff + 8192;  // kFew: the sums' (maximum, weight) pairs
 constexpr int kVupFlagOff = kVupPairOff + 64;   // one int per token of the pass: its row is valid
 constexpr int kVupLdsB = kVupFlagOff + 64;
-constexpr int kVupAlone = 16;                   // partials of a row that are left to one wavefront
+// Partials of a row that are left to one wavefront.  us per layer, alone / shared, requests x heads: about 10 partials of a row, 7 x 128
+// of 300-3000 keys 37.0 / 37.4, 6 x 128 of 3k-6k 45.2 / 45.6; 13, 5 x 128 of 1k-3k 35.1 / 35.5; but 17, 4 x 128 of 300-3000 35.7 /
+// 33.1; 22, 12 x 32 of 1k-4k 39.5 / 36.2, 12 x 16 of 1k-7k 38.3 / 34.0.
+constexpr int kVupAlone = 16;
 constexpr int kVupAsk = 20;                     // partials that a wavefront asks for at once
 constexpr int kVupAhead = 4;                    // product steps whose operands are requested ahead (at most 4: the wait ladder)
 
@@ -310,12 +313,11 @@ using namespace mlahip;
 
 extern "C" size_t mla_decode_workspace_bytes(int32_t batch, int32_t max_q_len, int32_t num_heads, int32_t num_splits);
 
-// Phase 2 of the split-KV decode with the value up-projection fused in: out[t, n*128 + v] for the decode tokens.
-extern "C" int mla_splitkv_reduce_vup(const void* workspace, size_t workspace_bytes, const int32_t* seq_lens,
-                                      const int32_t* query_start_loc, int32_t batch, int32_t max_q_len, int32_t num_heads,
-                                      int32_t num_splits, int32_t num_tokens, const void* w_uv, int64_t w_stride_n,
-                                      int64_t w_stride_k, void* out, int64_t out_stride_t, int64_t out_stride_h,
-                                      hipStream_t stream) {
+// fp8: the split ran over the fp8 cache, whose launches cut the work otherwise (plan_form)
+static int reduce_vup_impl(const void* workspace, size_t workspace_bytes, const int32_t* seq_lens, const int32_t* query_start_loc,
+                           int32_t batch, int32_t max_q_len, int32_t num_heads, int32_t num_splits, int32_t num_tokens,
+                           const void* w_uv, int64_t w_stride_n, int64_t w_stride_k, void* out, int64_t out_stride_t,
+                           int64_t out_stride_h, bool fp8, hipStream_t stream) {
   MLA_REQUIRE(workspace && out && seq_lens && w_uv, MLA_ERR_NULL, "mla_splitkv_reduce_vup: null pointer argument");
   MLA_REQUIRE(batch >= 0 && max_q_len >= 1 && num_heads >= 1 && num_heads <= 65535 && num_splits >= 1 && num_tokens >= 0 &&
                   (int64_t)num_tokens <= (int64_t)batch * max_q_len,
@@ -336,8 +338,28 @@ extern "C" int mla_splitkv_reduce_vup(const void* workspace, size_t workspace_by
   cp.corr_scale = cp.lse_part + rows; cp.corr_row = (const __bf16* const*)(cp.lse_part + 2 * rows);
   cp.seg_ids = (const int32_t*)(cp.lse_part + 4 * rows);
   cp.seq_lens = seq_lens; cp.qsl = query_start_loc;
-  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = plan_form(batch, num_splits, r_max).chunks;
+  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = plan_form(batch, num_splits, r_max, !fp8).chunks;
   cp.out = (__bf16*)out; cp.out_st = out_stride_t; cp.out_sh = out_stride_h;
   cp.lse_out = nullptr; cp.lse_st = 0;
   return launch_reduce_vup(cp, w_uv, w_stride_n, w_stride_k, num_tokens, stream);
+}
+
+// Phase 2 of the split-KV decode with the value up-projection fused in: out[t, n*128 + v] for the decode tokens.
+extern "C" int mla_splitkv_reduce_vup(const void* workspace, size_t workspace_bytes, const int32_t* seq_lens,
+                                      const int32_t* query_start_loc, int32_t batch, int32_t max_q_len, int32_t num_heads,
+                                      int32_t num_splits, int32_t num_tokens, const void* w_uv, int64_t w_stride_n,
+                                      int64_t w_stride_k, void* out, int64_t out_stride_t, int64_t out_stride_h,
+                                      hipStream_t stream) {
+  return reduce_vup_impl(workspace, workspace_bytes, seq_lens, query_start_loc, batch, max_q_len, num_heads, num_splits, num_tokens,
+                         w_uv, w_stride_n, w_stride_k, out, out_stride_t, out_stride_h, false, stream);
+}
+
+// The same behind mla_decode_fp8 and mla_decode_fp8_window_split.
+extern "C" int mla_splitkv_reduce_vup_fp8(const void* workspace, size_t workspace_bytes, const int32_t* seq_lens,
+                                          const int32_t* query_start_loc, int32_t batch, int32_t max_q_len, int32_t num_heads,
+                                          int32_t num_splits, int32_t num_tokens, const void* w_uv, int64_t w_stride_n,
+                                          int64_t w_stride_k, void* out, int64_t out_stride_t, int64_t out_stride_h,
+                                          hipStream_t stream) {
+  return reduce_vup_impl(workspace, workspace_bytes, seq_lens, query_start_loc, batch, max_q_len, num_heads, num_splits, num_tokens,
+                         w_uv, w_stride_n, w_stride_k, out, out_stride_t, out_stride_h, true, stream);
 }

@@ -514,7 +514,7 @@ def _vup_out(out: torch.Tensor, w_uv: torch.Tensor, t: int, n: int) -> torch.Ten
 VUP_MAX_TOKENS = 256
 
 
-def _reduce_vup(lib, ws_args, seq_lens, qsl, b, q_len, n, num_splits, t, w_uv, o3, st) -> None:
+def _reduce_vup(lib, ws_args, seq_lens, qsl, b, q_len, n, num_splits, t, w_uv, o3, st, fp8: bool = False) -> None:
     if t > VUP_MAX_TOKENS:
         o = torch.empty(n, t, D_NOPE, dtype=torch.bfloat16, device=o3.device)
         rc = lib.mla_splitkv_reduce(*ws_args, seq_lens.data_ptr(), qsl, b, q_len, n, num_splits, o.data_ptr(), o.stride(1),
@@ -522,8 +522,9 @@ def _reduce_vup(lib, ws_args, seq_lens, qsl, b, q_len, n, num_splits, t, w_uv, o
         _lib.check(rc, "mla_splitkv_reduce")
         torch.bmm(o, w_uv, out=o3.transpose(0, 1))
         return
-    rc = lib.mla_splitkv_reduce_vup(*ws_args, seq_lens.data_ptr(), qsl, b, q_len, n, num_splits, t, w_uv.data_ptr(),
-                                    w_uv.stride(0), w_uv.stride(1), o3.data_ptr(), o3.stride(0), o3.stride(1), st)
+    merge = lib.mla_splitkv_reduce_vup_fp8 if fp8 else lib.mla_splitkv_reduce_vup
+    rc = merge(*ws_args, seq_lens.data_ptr(), qsl, b, q_len, n, num_splits, t, w_uv.data_ptr(), w_uv.stride(0), w_uv.stride(1),
+               o3.data_ptr(), o3.stride(0), o3.stride(1), st)
     _lib.check(rc, "mla_splitkv_reduce_vup")
 
 
@@ -1142,7 +1143,7 @@ def decode_fp8(q_nope: torch.Tensor, q_rope: torch.Tensor, cache: torch.Tensor, 
             *ws_args, num_splits, st)
         _lib.check(rc, "mla_decode_fp8_window_split")
         if o3 is not None:
-            _reduce_vup(lib, ws_args, seq_lens, qsl, b, q_len, n, num_splits, t, w_uv, o3, st)
+            _reduce_vup(lib, ws_args, seq_lens, qsl, b, q_len, n, num_splits, t, w_uv, o3, st, fp8=True)
         else:
             rc = lib.mla_splitkv_reduce(*ws_args, seq_lens.data_ptr(), qsl, b, q_len, n, num_splits, out.data_ptr(), out.stride(0),
                                         out.stride(1), lse_out.data_ptr() if lse_out is not None else None, st)
@@ -1162,7 +1163,7 @@ def decode_fp8(q_nope: torch.Tensor, q_rope: torch.Tensor, cache: torch.Tensor, 
             seq_lens = seq_lens.contiguous()
         _reduce_vup(lib, (ws.data_ptr(), ws.numel() * ws.element_size()), seq_lens,
                     query_start_loc.data_ptr() if query_start_loc is not None else None, b, q_len, n, num_splits, t, w_uv, o3,
-                    _stream(q_nope))
+                    _stream(q_nope), fp8=True)
     return out
 
 

@@ -69,6 +69,24 @@ def test_fused_up_projection_identity_weight_returns_the_attention_rows(dev):
     assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("batch,splits", [(7, 32), (5, 32)])   # 224 and 160 chunks asked for
+def test_rows_of_a_dozen_partials_are_left_to_one_wavefront(dev, batch, splits):
+    """The merge is shaped for the plan that the split ran with: groups of 32 rows, 64 chunks, 10 to 13 partials of a row.  One
+    wavefront then adds a row in the order of the separate merge, so that the bits are the same; a shared row would be added otherwise."""
+    from omni_npu_amd import kernels as K
+    heads = 128
+    c = O.make_decode_case(batch, heads, 3000, 6000, seed=batch)
+    args = [c[k].to(dev) for k in ("q_nope", "q_rope", "nope", "rope", "block_table", "seq_lens")]
+    o = torch.empty(batch, heads, 512, dtype=torch.bfloat16, device=dev)
+    K.decode(*args, c["scale"], o, num_splits=splits)
+    for col in range(0, 512, 128):
+        w = torch.zeros(heads, 512, 128, dtype=torch.bfloat16, device=dev)
+        w[:, col:col + 128] = torch.eye(128, dtype=torch.bfloat16, device=dev)
+        out = torch.empty(batch, heads * 128, dtype=torch.bfloat16, device=dev)
+        K.decode(*args, c["scale"], out, num_splits=splits, w_uv=w)
+        assert torch.equal(out.view(batch, heads, 128), o[..., col:col + 128])
+
+
 def test_fused_up_projection_strided_output_and_varlen_queries(dev):
     """Output written into a slice of a wider, padded buffer; query tokens given by query_start_loc with one request
     shorter than the uniform length (its missing token's row must stay untouched)."""
