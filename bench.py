@@ -1230,7 +1230,7 @@ def main():
     # HBM bytes per launch of the split kernel from the FETCH_SIZE / WRITE_SIZE counter runs (scaled on a plain copy) of
     # exactly this workload; a counter run cannot be made from inside this script, so other shapes report null
     default_shape = (args.seed, b, args.len_lo, args.len_hi, q_len, splits) == (0, 64, 4096, 8192, 1, 4) and not args.l2_resident
-    profile_of = {128: "mla_decode_v3_b64_ctx8k.md", 16: "mla_decode_v3_b64_ctx8k_16heads.md"}
+    profile_of = {128: "mla_decode_v3_b64_ctx8k.md", 16: "mla_decode_rows_b64_ctx8k_16heads.md"}
     traffic, traffic_src = profile_traffic(profile_of.get(heads, ""), default_shape and heads in profile_of)
     row_groups = 1 if heads * q_len <= 32 else (2 if heads * q_len <= 64 else 4)   # the kernel form the library picks
     res = {

@@ -5,7 +5,7 @@
 //   s_j = scale * (ql[t,n] . Kc[j] + qr[t,n] . Kr[j]),  j < L_b - (q_len-1-t)   (right-down causal)
 //   o   = sum_j softmax(s)_j * Kc[j]
 // with ONE latent KV row (512 + 64) shared by all heads.  The kernels live in decode_v3.hip (bf16 cache: dense, row-list
-// and sink + window sources), decode_v3_fp8.hip (fp8-e4m3 block-scaled cache) and chunk_reduce.hip (the merge of the
+// and sink + window sources; decode_rows.hip: the same for 32 query rows per workgroup), decode_v3_fp8.hip (fp8-e4m3 block-scaled cache) and chunk_reduce.hip (the merge of the
 // split-KV partials: the N-way merge of src/omni_npu/attention/ops.py:109-141).
 //
 // Workspace (mla_decode_workspace_bytes): batch * (num_splits + 1) partial slots of rows = max_q_len * num_heads each:

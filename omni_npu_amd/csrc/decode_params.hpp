@@ -1,4 +1,4 @@
-// Parameters and launchers of the absorbed-MLA split-KV decode kernels (decode_v3.hip, decode_v3_fp8.hip), of the merge
+// Parameters and launchers of the absorbed-MLA split-KV decode kernels (decode_v3.hip, decode_rows.hip, decode_v3_fp8.hip), of the merge
 // of their partials (chunk_reduce.hip) and of the merge fused with the value up-projection (reduce_vup.hip).
 #pragma once
 #include "mla_common.hpp"

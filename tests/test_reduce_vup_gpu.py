@@ -24,9 +24,8 @@ def _w_uv(n, seed):
                                                             (2, 128, 1, 3000, 6000, 11), (3, 128, 1, 50, 300, 9),
                                                             (2, 128, 1, 3000, 6000, 40), (125, 128, 2, 2, 200, 1), (150, 128, 2, 2, 200, 1)])
 def test_fused_merge_and_up_projection(dev, batch, heads, q_len, lo, hi, splits):
-    """Up to 11 chunks per sequence and 256 tokens the fused kernel runs (rows of 7..12 partials take two rounds; the
-    case with more chunks than work units has empty chunks); the last two cases take the other route behind the same
-    call (separate merge, then the library GEMM): many partials per row, and more than 256 tokens."""
+    """Up to 256 tokens the fused kernel runs, rows of many partials among them; the last case takes the other route behind the same
+    call (separate merge, then the library GEMM)."""
     from omni_npu_amd import kernels as K
     c = O.make_decode_case(batch, heads, lo, hi, seed=7 * batch + q_len, q_len=q_len)
     w = _w_uv(heads, seed=batch)
@@ -167,7 +166,8 @@ def test_chunk_plan_and_shared_rows_at_their_edges(dev, batch, heads, q_len, lo,
 
 @pytest.mark.parametrize("batch,heads,q_len,lo,hi,splits", [
     (2, 128, 1, 40, 300, 32), (3, 128, 2, 40, 300, 16),       # groups of 32 rows: 64 chunks x 4, 48 x 8 (chunks below the CUs)
-    (7, 128, 1, 300, 3000, 32), (24, 128, 1, 100, 700, 8),    # groups of 64: 224 and 192 chunks cut to 128
+    (7, 128, 1, 300, 3000, 32), (24, 128, 1, 100, 700, 8),    # the same: 224 and 192 chunks cut to 64
+    (30, 128, 1, 100, 700, 8), (5, 128, 1, 300, 3000, 48),    # groups of 64 rows: 240 chunks, all but full CUs, cut to 128
     (7, 80, 1, 300, 900, 32), (31, 65, 1, 100, 500, 8),       # a last group of 16 rows, of one
 ])
 def test_row_groups_at_their_edges(dev, batch, heads, q_len, lo, hi, splits):
