@@ -280,7 +280,9 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
       const float* at = (const float*)(lds + kMaxOff) + rg * 16 + l16;
       return row < rows ? fmaxf(fmaxf(at[0], at[kRows]), fmaxf(at[2 * kRows], at[3 * kRows])) : INFINITY;
     };
-    int restarts_left = 4;                                   // (each raises a reference by more than 2^100: fp32 has room for three)
+    // Three restarts as soon as a row asks, with the scores so far as references.  Where the third was not enough (0), the pass is only
+    // there to see the others, whatever it adds up, and one more (-1) has the maxima of them all.
+    int restarts_left = 3;
     bool fresh = true;
     for (int it = 0; it < iters; it++) {
       if (it == 0) {
@@ -374,7 +376,7 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
             }
         }
       }
-      if (restarts_left > 0 && __builtin_amdgcn_ballot_w64(flags != 0) != 0) {
+      if (restarts_left > 0 ? __builtin_amdgcn_ballot_w64(flags != 0) != 0 : restarts_left == 0 && it + 1 == iters) {
         // (rare; every wavefront reads the same flags) start over, with the largest scores seen so far as references
         restarts_left--;
         MLA_WAIT_VMCNT(0);

@@ -662,7 +662,9 @@ __global__ __launch_bounds__(512) void mla_decode_v3_fp8_kernel(const DecodePara
   }
   bool restart = false;
   bool early_issued = kRG < 4;   // (small forms: the first two raw blocks were requested beside the query)
-  int restarts_left = 4;         // every restart raises a reference by more than 2^100: fp32 has room for three
+  // Three restarts as soon as a row asks, with the scores so far as references.  Where the third was not enough (0), the pass is only
+  // there to see the others, whatever it adds up, and one more (-1) has the maxima of them all.
+  int restarts_left = 3;
   do {
     if (restart) {
       // a row outgrew its reference: drain, take the maxima seen so far as references, clear the sums, start over
@@ -744,7 +746,9 @@ __global__ __launch_bounds__(512) void mla_decode_v3_fp8_kernel(const DecodePara
       const int blk = blk_end - 1;
       MLA_WAIT_VMCNT(0);
       lds_barrier();
-      if (restarts_left > 0 && flags_ask_restart(flags_read(blk))) { restart = true; restarts_left--; }
+      int ask = restarts_left > 0 ? flags_read(blk) : restarts_left + 1;
+      asm volatile("" : "+v"(ask));                           // (with a branch on 0 the compiler spills 180 registers)
+      if (flags_ask_restart(ask)) { restart = true; restarts_left--; }
       else { float sc[8]; Sm st; pv_softmax(blk, std::true_type{}, std::false_type{}, sc, st, true); }
     }
   } while (restart);
