@@ -39,16 +39,6 @@ constexpr float kRestartThreshold = 100.f;                 // log2 units above a
 __device__ __forceinline__ int swz_nope(int r) { return ((r & 7) << 1) | ((r >> 3) & 1); }
 __device__ __forceinline__ int swz_rope(int r) { return (r >> 1) & 7; }
 
-__device__ __forceinline__ int scan_add(int v) {           // inclusive, over the lanes (see decode_v3.hip)
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
-  return v;
-}
-typedef __attribute__((address_space(4))) const int32_t* ConstI32Ptr;   // scalar (constant-cache) loads
 // a / b for a < 2^21 (the quotient's distance from the next integer is at least 0.5 / b, the product's error below that)
 __device__ __forceinline__ int div_small(int a, int b) {
   return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b));
@@ -96,12 +86,12 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
         if (p.qsl) { my_q0 = p.qsl[lane]; my_q1 = p.qsl[lane + 1]; }
         my_len = len_now(my_len, my_q0, my_q1);
       }
-      pe = scan_add(plan_work_units(my_len));
+      pe = wave_incl_scan_dpp(plan_work_units(my_len));
       tot = __builtin_amdgcn_readlane(pe, 63);
     } else {
       int mine = 0;
       for (int i = lane; i < p.batch; i += 64) mine += plan_work_units(len_of(i));
-      tot = __builtin_amdgcn_readlane(scan_add(mine), 63);
+      tot = __builtin_amdgcn_readlane(wave_incl_scan_dpp(mine), 63);
     }
     const int chunks = plan_chunk_count(tot, r_max, p.num_chunks), per_xcd = (chunks + 7) >> 3;
     chunk = xcd * per_xcd + xcd_j;
@@ -123,7 +113,7 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
       int carry = 0, b0 = 0;
       for (int base = 0; base < p.batch; base += 64) {
         const int i = base + lane;
-        const int run = scan_add(i < p.batch ? plan_work_units(len_of(i)) : 0) + carry;
+        const int run = wave_incl_scan_dpp(i < p.batch ? plan_work_units(len_of(i)) : 0) + carry;
         const int n = __builtin_popcountll(__builtin_amdgcn_ballot_w64(i < p.batch && run <= v_cur));
         if (n > 0) v_seq = __builtin_amdgcn_readlane(run, n - 1);
         b0 += n;

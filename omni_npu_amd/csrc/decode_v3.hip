@@ -81,18 +81,6 @@ __device__ __forceinline__ int wave_incl_scan_i32(int v, int lane) {
   for (int d = 1; d < 64; d <<= 1) { const int t = __shfl_up(v, d, 64); v += lane >= d ? t : 0; }
   return v;
 }
-// inclusive scan over the 64 lanes with data-parallel-primitive moves (no LDS round trips): shifts inside the rows of 16,
-// then lane 15 of rows 0 and 2 into rows 1 and 3, then lane 31 into the upper half
-__device__ __forceinline__ int wave_incl_scan_dpp(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
-  return v;
-}
-typedef __attribute__((address_space(4))) const int32_t* ConstI32Ptr;   // scalar (constant-cache) loads
 
 
 // kRG = groups of 32 query rows a workgroup handles (4: the general form; 2: launches with at most 64 query rows per request;
