@@ -318,7 +318,7 @@ extern "C" int mla_kv_up(const void* x, int64_t x_stride, const void* weight, in
               MLA_ERR_SHAPE, "mla_kv_up: rows must be 16-byte aligned, at most 2^20 elements apart");
   MLA_REQUIRE(clear_words >= 0 && clear_words <= 512 && (clear || clear_words == 0) && (uintptr_t)clear % 4 == 0, MLA_ERR_SHAPE,
               "mla_kv_up: up to 512 words to clear (got %d)", clear_words);
-  if (num_rows == 0) return MLA_OK;
+  if (num_rows == 0 && clear_words == 0) return MLA_OK;
   KvUpParams p;
   p.x = (const __bf16*)x; p.x_st = x_stride;
   p.w = (const __bf16*)weight; p.w_st = w_stride;
@@ -334,7 +334,7 @@ extern "C" int mla_kv_up(const void* x, int64_t x_stride, const void* weight, in
   if (rc != MLA_OK) return rc;
   // one workgroup per CU at most; fewer tiles: as many workgroups, in whole rounds of the eight XCDs
   const int64_t tiles = (int64_t)p.m_tiles * num_heads;
-  const int64_t grid = tiles < 256 ? (tiles + 7) / 8 * 8 : 256;
+  const int64_t grid = tiles == 0 ? 8 : tiles < 256 ? (tiles + 7) / 8 * 8 : 256;   // (no rows: only what is to be cleared)
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), kUpLdsB, stream, p);
   return check_launch("mla_kv_up_kernel");
 }

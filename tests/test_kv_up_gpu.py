@@ -74,3 +74,16 @@ def test_numbers_out_of_range(dev):
     want = torch.where(want.isfinite(), want.clamp(-65504, 65504), want).half()
     assert torch.equal(k.nan_to_num(7), ref[..., :128].bfloat16().nan_to_num(7)) and torch.equal(v.nan_to_num(7), want.nan_to_num(7))
     assert torch.equal(v.isnan(), ref[..., 128:].isnan()) and torch.equal(v.isinf(), ref[..., 128:].isinf())
+
+
+@pytest.mark.parametrize("t", [0, 3])
+def test_words_to_clear_are_cleared_with_and_without_rows(dev, t):
+    """The C entry point clears a prefill's queue also where the step has no rows of its own."""
+    x, w, _ = _inputs(dev, 3, 1, 576, 512)
+    out = torch.zeros(3, 256, dtype=torch.float16, device=dev)
+    words = torch.full((258,), 7, dtype=torch.int32, device=dev)
+    rc = K._lib.load().mla_kv_up(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), t, 1, 1, out.data_ptr(), 256, 256 * 3, None, 0, None, 0,
+                                 words[1:].data_ptr(), 256, K._stream(x))
+    assert rc == 0
+    assert words.tolist() == [7] + [0] * 256 + [7]
+    assert bool(out.any()) == (t > 0)
