@@ -380,6 +380,18 @@ int mla_prefill_varlen_queued(const void* q_nope, int64_t qn_stride_t, int64_t q
                               const float* prev_out, int64_t prev_stride_t, int64_t prev_stride_h, const float* prev_lse,
                               int32_t* queue, mlahip_stream_t stream);
 
+/* The same for few blocks of 128 rows over long contexts, fp16 (out_dtype + MLA_PREFILL_KV_F16), no window, pick, queue or earlier result:
+ * the 64-key tiles of a block are cut into `pieces` (2 .. 32) parts with a workgroup each, and a second launch merges their results.
+ * parts: scratch of pieces * num_tokens * num_heads * 129 floats, 16-byte aligned, which the caller keeps until both have run;
+ * num_tokens: at least cu_q[batch]. */
+int mla_prefill_varlen_split(const void* q_nope, int64_t qn_stride_t, int64_t qn_stride_h, const void* q_pe, int64_t qp_stride_t,
+                             int64_t qp_stride_h, const void* k_nope, int64_t kn_stride_t, int64_t kn_stride_h, const void* k_pe,
+                             int64_t kp_stride_t, const void* v, int64_t v_stride_t, int64_t v_stride_h, const int32_t* cu_q,
+                             const int32_t* cu_k, const void* k1_nope, int64_t kn1_stride_h, const void* k1_pe, const void* v1,
+                             int64_t v1_stride_h, const int32_t* cu_k1, int32_t batch, int32_t num_heads, int32_t max_q_len,
+                             int32_t causal, float scale, void* out, int64_t out_stride_t, int64_t out_stride_h, int32_t out_dtype,
+                             float* lse_out, int32_t pieces, int64_t num_tokens, float* parts, mlahip_stream_t stream);
+
 /* ---- DSA lightning indexer --------------------------------------------------------------------
  * Replaces torch.ops.custom.npu_lightning_indexer, v1/layers/attention/npu_dsa.py:92-103 and
  * vllm_patches/patches/models/deepseek/patch_dsv32_indexer.py:133-146, in two steps:

@@ -79,6 +79,8 @@ struct PrefillParams {
   int32_t max_blocks;                                        // of a sequence
   // optional: eight counters that begin at zero, kPfQueue apart, from which a grid of kPfWorkgroups takes its blocks
   int32_t* queue;
+  // kSplit: into how many pieces the tiles of a block are cut; out (fp32) and lse hold a result for each, so many elements apart
+  int32_t pieces; int64_t o_piece, lse_piece;
 };
 
 // One 64-key tile of head `head`, keys k0 .. k0 + 63 of the flat key axis (clamped to klast): 40 copy instructions of eight
@@ -153,9 +155,10 @@ __device__ __forceinline__ void pf_issue_tile(const PrefillParams& p, const PfKe
 // chunk and the suffix, whose rows otherwise go out as fp32 with their sums and come back (4 x 2048 over 16k: 1.1 GB), and whose
 // unequal causal blocks follow each other where every workgroup is resident at once.
 // A block of 128 rows of a head: rows 128 qb .. of a sequence whose queries start at q0 and whose keys at k0 (context keys: at k1)
-struct PfBlock { int qb, head, q0, sq, k0, sk, k1, sk1; };
+// (kSplit: piece `piece` of its tiles)
+struct PfBlock { int qb, head, q0, sq, k0, sk, k1, sk1, piece; };
 
-template <bool kKeyHalf, bool kValHalf, bool kPick, bool kCtx, class Last>
+template <bool kKeyHalf, bool kValHalf, bool kPick, bool kCtx, bool kSplit, class Last>
 __device__ __forceinline__ void pf_block(const PrefillParams& p, char* lds, const PfBlock& blk, Last last_tile_done) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -187,7 +190,6 @@ __device__ __forceinline__ void pf_block(const PrefillParams& p, char* lds, cons
     lim0 = lim0 < 0 ? 0 : (lim0 > sk ? sk : lim0);
     wg_lo = lim0 > p.window ? lim0 - p.window : 0;
   }
-  const int first_tile = wg_lo / kPfTile;
   // keys any row of this workgroup can see
   int wg_limit = sk;
   if (p.causal) {
@@ -198,7 +200,9 @@ __device__ __forceinline__ void pf_block(const PrefillParams& p, char* lds, cons
   }
   // context tiles first, then the causal ones: a tile's number counts through both runs
   const int tiles1 = (sk1 + kPfTile - 1) / kPfTile;
-  const int tiles = tiles1 + (wg_limit + kPfTile - 1) / kPfTile;
+  const int all_tiles = tiles1 + (wg_limit + kPfTile - 1) / kPfTile;
+  const int first_tile = kSplit ? all_tiles * blk.piece / p.pieces : wg_lo / kPfTile;
+  const int tiles = kSplit ? all_tiles * (blk.piece + 1) / p.pieces : all_tiles;
 
   const int64_t tq = q0 + (row_ok ? row : sq - 1);
   f32x16 acc[4];
@@ -207,7 +211,7 @@ __device__ __forceinline__ void pf_block(const PrefillParams& p, char* lds, cons
 #pragma unroll
     for (int r = 0; r < 16; r++) acc[i][r] = 0.f;
   float m_run = kPfNoRef, l_run = 0.f;
-  if (p.prev_out != nullptr && row_ok) {
+  if (!kSplit && p.prev_out != nullptr && row_ok) {
     // Continue from (out, lse) over other keys: running maximum = lse (as a base-2 exponent), running sum = 1, accumulator
     // = out.  A row without earlier keys comes with lse = -inf (+inf is read the same way, as the two-way merge does) and
     // starts empty.  The sum lives in the row's lower half-wave lane; the halves are added at the end.
@@ -227,7 +231,7 @@ __device__ __forceinline__ void pf_block(const PrefillParams& p, char* lds, cons
     }
   }
 
-  if (tiles > 0) {
+  if (kSplit ? tiles > first_tile : tiles > 0) {
     const uint32_t lds0 = lds_addr_of(lds);
     const PfKeys keys = {p.k_nope + (int64_t)head * p.kn_sh + k0 * p.kn_st, p.k_pe + k0 * p.kp_st, p.v + (int64_t)head * p.v_sh + k0 * p.v_st};
     PfKeys keys1 = keys;
@@ -499,14 +503,16 @@ __device__ __forceinline__ void pf_block(const PrefillParams& p, char* lds, cons
   const float l_tot = l_run + xor32(l_run);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (row_ok) {
-    if (p.lse && half == 0) p.lse[tq * p.num_heads + head] = l_tot > 0.f ? (m_run + fast_log2(l_tot)) * kLn2 : -INFINITY;
-    const int64_t o = tq * p.o_st + (int64_t)head * p.o_sh + 4 * half;
+    const int64_t lse_at = tq * p.num_heads + head + (kSplit ? blk.piece * p.lse_piece : 0);
+    if ((kSplit || p.lse) && half == 0) p.lse[lse_at] = l_tot > 0.f ? (m_run + fast_log2(l_tot)) * kLn2 : -INFINITY;
+    const int64_t o = tq * p.o_st + (int64_t)head * p.o_sh + 4 * half + (kSplit ? blk.piece * p.o_piece : 0);
+    if (kSplit && tiles <= first_tile) return;               // (a piece without keys: the merge reads its lse only)
 #pragma unroll
     for (int db = 0; db < 4; db++)
 #pragma unroll
       for (int rg = 0; rg < 4; rg++) {
         const int d = db * 32 + rg * 8;
-        if (p.out_fp32) {
+        if (kSplit || p.out_fp32) {
           f32x4 v = {acc[db][rg * 4] * inv, acc[db][rg * 4 + 1] * inv, acc[db][rg * 4 + 2] * inv, acc[db][rg * 4 + 3] * inv};
           *(f32x4*)((float*)p.out + o + d) = v;
         } else {
@@ -558,7 +564,7 @@ __device__ __forceinline__ void pf_from_queue(const PrefillParams& p0, char* lds
     const int u = ticket - __builtin_amdgcn_readlane(before_l, b), h = u / n;
     const PfBlock blk = {n - 1 - (u - h * n), h * 8 + xcd, __builtin_amdgcn_readlane(q0_l, b), __builtin_amdgcn_readlane(sq_l, b),
                          __builtin_amdgcn_readlane(k0_l, b), __builtin_amdgcn_readlane(sk_l, b),
-                         __builtin_amdgcn_readlane(k1_l, b), __builtin_amdgcn_readlane(sk1_l, b)};
+                         __builtin_amdgcn_readlane(k1_l, b), __builtin_amdgcn_readlane(sk1_l, b), 0};
     // (the arguments are read anew for every block: kept over all of them they leave the loop over the tiles too few scalar registers)
     auto args = (const __attribute__((address_space(4))) PrefillParams*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(args));
@@ -622,7 +628,7 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
       head = pair % gridDim.y;
       b = pair / gridDim.y;
     }
-    PfBlock blk = {qb, head, p.cu_q[b], 0, p.cu_k[b], 0, 0, 0};
+    PfBlock blk = {qb, head, p.cu_q[b], 0, p.cu_k[b], 0, 0, 0, 0};
     blk.sq = p.cu_q[b + 1] - blk.q0;
     blk.sk = p.cu_k[b + 1] - blk.k0;
     if constexpr (kCtx) {
@@ -630,12 +636,85 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_varlen_kernel(const Prefil
       blk.sk1 = p.cu_k1[b + 1] - blk.k1;
     }
     if (qb * kPfRows >= blk.sq) return;
-    pf_block<kKeyHalf, kValHalf, kPick, kCtx>(p, lds, blk, [] {});
+    pf_block<kKeyHalf, kValHalf, kPick, kCtx, false>(p, lds, blk, [] {});
   } else {
     pf_from_queue<kPfRows, kCtx>(p0, lds, [&](const PrefillParams& p, const PfBlock& blk, auto ask) {
-      pf_block<kKeyHalf, kValHalf, kPick, kCtx>(p, lds, blk, ask);
+      pf_block<kKeyHalf, kValHalf, kPick, kCtx, false>(p, lds, blk, ask);
     });
   }
+}
+
+// Launches with fewer blocks than run at once, over long contexts: a block's tiles are cut into p.pieces pieces with a workgroup each,
+// whose results and log-sum-exps a second launch merges.  Without it a chunk of 85 tokens behind 3722 cached ones x 16 heads keeps 32
+// of 256 CUs busy for sixty tiles in a row.
+template <bool kCtx>
+__global__ __launch_bounds__(256, 2) void mla_prefill_split_kernel(const PrefillParams p) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  // all pieces and blocks of a (sequence, head) on one XCD, the blocks of a piece, which read the same keys, next to each other
+  const int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+  int x = blockIdx.x, head = blockIdx.y, b = blockIdx.z;
+  const int nx = gridDim.x;
+  if (((gridDim.y * gridDim.z) & 7) == 0) {
+    const int j = lin >> 3, run = j / nx, pair = run * 8 + (lin & 7);
+    x = j - run * nx;
+    head = pair % gridDim.y;
+    b = pair / gridDim.y;
+  }
+  const int piece = x / p.max_blocks;
+  PfBlock blk = {x - piece * p.max_blocks, head, p.cu_q[b], 0, p.cu_k[b], 0, 0, 0, piece};
+  blk.sq = p.cu_q[b + 1] - blk.q0;
+  blk.sk = p.cu_k[b + 1] - blk.k0;
+  if constexpr (kCtx) {
+    blk.k1 = p.cu_k1[b];
+    blk.sk1 = p.cu_k1[b + 1] - blk.k1;
+  }
+  if (blk.qb * kPfRows >= blk.sq) return;
+  pf_block<true, true, false, kCtx, true>(p, lds, blk, [] {});
+}
+
+// The merge of the pieces: half a wavefront takes a row, its pieces' log-sum-exps one to a lane.  Eight tokens of a head to a workgroup
+// of four wavefronts; what bounds it are two round trips behind that for the sequence (log-sum-exps; the results that count, at once).
+constexpr int kPfMaxPieces = 32;
+__global__ __launch_bounds__(256) void mla_prefill_merge_kernel(const float* part, const float* part_lse, int32_t pieces, int64_t rows,
+                                                                const int32_t* cu_q, void* out, int64_t o_st, int64_t o_sh,
+                                                                int32_t out_fp32, float* lse) {
+  const int l = threadIdx.x & 31, q0 = cu_q[blockIdx.z], r = blockIdx.x * 8 + (threadIdx.x >> 5);
+  if (r >= cu_q[blockIdx.z + 1] - q0) return;
+  const int64_t t = q0 + r, row = t * gridDim.y + blockIdx.y;
+  const float mine = l < pieces ? part_lse[l * rows + row] : -INFINITY;
+  float mx = mine;
+#pragma unroll
+  for (int d = 16; d >= 1; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 32));
+  const float w = mx > -INFINITY ? fast_exp2((mine - mx) * kLog2e) : 0.f;
+  float total = w;
+#pragma unroll
+  for (int d = 16; d >= 1; d >>= 1) total += __shfl_xor(total, d, 32);
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+  for (int i0 = 0; i0 < pieces; i0 += 8) {
+    f32x4 v[8];
+    float ws[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      ws[i] = i0 + i < pieces ? __shfl(w, i0 + i, 32) : 0.f;
+      v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (ws[i] > 0.f) v[i] = *(const f32x4*)(part + ((i0 + i) * rows + row) * 128 + l * 4);   // (else nothing may have been written there)
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) sum[e] = __builtin_fmaf(ws[i], v[i][e], sum[e]);
+  }
+  const float inv = total > 0.f ? 1.f / total : 0.f;
+  const int64_t o = t * o_st + (int64_t)blockIdx.y * o_sh + l * 4;
+  if (out_fp32) {
+    *(f32x4*)((float*)out + o) = f32x4{sum[0] * inv, sum[1] * inv, sum[2] * inv, sum[3] * inv};
+  } else {
+    bf16x4 r;
+#pragma unroll
+    for (int e = 0; e < 4; e++) r[e] = (__bf16)(sum[e] * inv);
+    *(bf16x4*)((__bf16*)out + o) = r;
+  }
+  if (lse && l == 0) lse[row] = total > 0.f ? mx + fast_log2(total) * kLn2 : -INFINITY;
 }
 
 }  // namespace mlahip
@@ -652,7 +731,8 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
                                float* lse_out, const float* prev_out, int64_t prev_stride_t, int64_t prev_stride_h,
                                const float* prev_lse, const uint32_t* pick, int64_t pick_stride, int32_t pick_words,
                                hipStream_t stream, const void* k1_nope = nullptr, int64_t kn1_stride_h = 0, const void* k1_pe = nullptr,
-                               const void* v1 = nullptr, int64_t v1_stride_h = 0, const int32_t* cu_k1 = nullptr, int32_t* queue = nullptr) {
+                               const void* v1 = nullptr, int64_t v1_stride_h = 0, const int32_t* cu_k1 = nullptr, int32_t* queue = nullptr,
+                               int32_t pieces = 0, int64_t num_tokens = 0, float* parts = nullptr) {
   MLA_REQUIRE(q_nope && q_pe && k_nope && k_pe && v && cu_q && cu_k && out, MLA_ERR_NULL, "%s: null pointer argument", what);
   MLA_REQUIRE(batch >= 0 && num_heads >= 1 && max_q_len >= 0 && batch <= 65535 && num_heads <= 65535 && window >= 0,
               MLA_ERR_SHAPE, "%s: batch=%d num_heads=%d max_q_len=%d window=%d", what, batch, num_heads, max_q_len, window);
@@ -700,6 +780,20 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
   p.pick = pick; p.pick_st = pick_stride; p.pick_tiles = pick_words / 2;
   p.max_blocks = (max_q_len + kPfRows - 1) / kPfRows;
   p.queue = queue;
+  if (pieces > 1) {
+    const int64_t rows = num_tokens * num_heads;
+    const int rc = ensure_dynamic_lds((const void*)(k1_nope ? mla_prefill_split_kernel<true> : mla_prefill_split_kernel<false>), kPfLdsB, what);
+    if (rc != MLA_OK) return rc;
+    p.pieces = pieces; p.o_piece = rows * 128; p.lse_piece = rows;
+    p.out = parts; p.o_st = (int64_t)num_heads * 128; p.o_sh = 128; p.lse = parts + pieces * rows * 128;
+    hipLaunchKernelGGL((k1_nope ? mla_prefill_split_kernel<true> : mla_prefill_split_kernel<false>), dim3(p.max_blocks * pieces, num_heads, batch),
+                       dim3(256), kPfLdsB, stream, p);
+    const int launched = check_launch("mla_prefill_split_kernel");
+    if (launched != MLA_OK) return launched;
+    hipLaunchKernelGGL(mla_prefill_merge_kernel, dim3((max_q_len + 7) / 8, num_heads, batch), dim3(256), 0, stream, (const float*)p.out,
+                       (const float*)p.lse, pieces, rows, cu_q, out, out_stride_t, out_stride_h, out_dtype, lse_out);
+    return check_launch("mla_prefill_merge_kernel");
+  }
   static constexpr auto kernel_of = [](auto queued, bool kh, bool vh, bool pk, bool ctx) {
     constexpr bool kQ = decltype(queued)::value;
     return ctx  ? mla_prefill_varlen_kernel<true, true, false, true, kQ>
@@ -798,4 +892,28 @@ extern "C" int mla_prefill_varlen_queued(const void* q_nope, int64_t qn_stride_t
                              max_q_len, causal, window, scale, out, out_stride_t, out_stride_h, out_dtype, lse_out, prev_out,
                              prev_stride_t, prev_stride_h, prev_lse, pick, pick_stride, pick_words, stream, k1_nope, kn1_stride_h,
                              k1_pe, v1, v1_stride_h, cu_k1, queue);
+}
+
+// fp16 keys and values (MLA_PREFILL_KV_F16) without a window, picks, an earlier result or a queue, and further keys as above: the tiles of a
+// block of 128 rows go to `pieces` (2 .. 32) workgroups, whose results a second launch merges.  parts: pieces x num_tokens x num_heads x 129
+// floats of scratch; num_tokens: cu_q's last entry, at least.
+extern "C" int mla_prefill_varlen_split(const void* q_nope, int64_t qn_stride_t, int64_t qn_stride_h, const void* q_pe,
+                                        int64_t qp_stride_t, int64_t qp_stride_h, const void* k_nope, int64_t kn_stride_t,
+                                        int64_t kn_stride_h, const void* k_pe, int64_t kp_stride_t, const void* v,
+                                        int64_t v_stride_t, int64_t v_stride_h, const int32_t* cu_q, const int32_t* cu_k,
+                                        const void* k1_nope, int64_t kn1_stride_h, const void* k1_pe, const void* v1,
+                                        int64_t v1_stride_h, const int32_t* cu_k1, int32_t batch, int32_t num_heads,
+                                        int32_t max_q_len, int32_t causal, float scale, void* out, int64_t out_stride_t,
+                                        int64_t out_stride_h, int32_t out_dtype, float* lse_out, int32_t pieces, int64_t num_tokens,
+                                        float* parts, hipStream_t stream) {
+  MLA_REQUIRE(parts && (uintptr_t)parts % 16 == 0, MLA_ERR_NULL, "mla_prefill_varlen_split: scratch on a 16-byte boundary is needed");
+  MLA_REQUIRE(pieces >= 2 && pieces <= kPfMaxPieces && num_tokens >= 0 && (out_dtype & 16) != 0 && (out_dtype & 64) == 0 &&
+                  (int64_t)max_q_len * pieces < (1 << 30), MLA_ERR_UNSUPPORTED,
+              "mla_prefill_varlen_split: 2 to %d pieces of fp16 keys and values (got %d, type code %d)", kPfMaxPieces, pieces, out_dtype);
+  if (num_tokens == 0) return MLA_OK;
+  return prefill_varlen_impl("mla_prefill_varlen_split", q_nope, qn_stride_t, qn_stride_h, q_pe, qp_stride_t, qp_stride_h, k_nope,
+                             kn_stride_t, kn_stride_h, k_pe, kp_stride_t, v, v_stride_t, v_stride_h, cu_q, cu_k, batch, num_heads,
+                             max_q_len, causal, 0, scale, out, out_stride_t, out_stride_h, out_dtype, lse_out, nullptr, 0, 0, nullptr,
+                             nullptr, 0, 0, stream, k1_nope, kn1_stride_h, k1_pe, v1, v1_stride_h, cu_k1, nullptr, pieces, num_tokens,
+                             parts);
 }

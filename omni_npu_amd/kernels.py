@@ -918,6 +918,31 @@ def _prefill_blocks(tokens: int, batch: int, max_q_len: int, num_heads: int) -> 
     return num_heads * min(batch * -(-int(max_q_len) // 128), tokens // 128 + batch)
 
 
+# Where a launch has fewer blocks of 128 rows than run at once, the keys of a block are cut into pieces with a workgroup each.  In
+# microseconds: a tile of 64 keys takes 1.3, half as much again where two workgroups share a CU, and a piece of all rows is a fp32 result
+# to write and to merge, 0.48 per MiB; both together make the best cut sqrt(1.3 tiles / (0.48 MiB)).  The second launch takes 5, which
+# the cut has to return.  us per attention, whole / cut as the rule says, tokens x heads, keys in front of them:
+#   (85, 15) x 16, (1034, 3722): 79.8 / 21.8    110 x 32, 3794: 84.0 / 27.2    33 x 16, 15 000: 297 / 33     128 x 128, 2048: 53.4 / 43.1
+#   1000 x 16, 3000: 86.8 / 55.3                300 x 64, 8000: 190 / 141      5 of 153-472 x 16, 3579-6268: 164 / 143
+# and where it says no, whole / in two:
+#   435 x 32, 512: 24.8 / 25.2    1522 x 32, 350: 58.8 / 74.4    2048 x 16, 0: 46.9 / 51.8    1024 x 32, 1024: 54.4 / 56.7    716 x 32, 0: 22.1 / 28.2
+_PREFILL_MAX_PIECES = 32
+
+
+def prefill_pieces(tokens: int, batch: int, max_q_len: int, num_heads: int, seen: int) -> int:
+    """Into how many pieces prefill_varlen cuts the keys of a block of 128 rows (1: not at all); ``seen``: keys that a row sees on
+    average, summed over the sequences."""
+    blocks = _prefill_blocks(tokens, batch, max_q_len, num_heads)
+    if blocks < 1 or blocks * 2 > _PREFILL_RESIDENT:
+        return 1
+    tiles, mib = seen / (64 * batch), tokens * num_heads * 516 / 2 ** 20
+    pieces = min(int(math.sqrt(2.7 * tiles / mib)), _PREFILL_RESIDENT // blocks, _PREFILL_MAX_PIECES)
+    if pieces < 2:
+        return 1
+    shared = 1.5 if blocks * pieces > _PREFILL_RESIDENT // 2 else 1.0
+    return pieces if 1.3 * tiles * (1 - shared / pieces) > 0.48 * mib * pieces + 5 else 1
+
+
 def prefill_queue(tokens: int, batch: int, max_q_len: int, num_heads: int, device: torch.device) -> Optional[torch.Tensor]:
     """Memory for prefill_varlen's ``queue``, to be cleared first (kv_up does it on the way), or None where a launch has no use for
     one: all of its blocks of 128 rows are at work at once, or their order is not one that the kernel works out."""
@@ -941,7 +966,7 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
                    out: torch.Tensor, lse_out: Optional[torch.Tensor] = None, window: Optional[int] = None,
                    prev_out: Optional[torch.Tensor] = None, prev_lse: Optional[torch.Tensor] = None,
                    pick: Optional[torch.Tensor] = None, context: Optional[tuple] = None,
-                   queue: Optional[torch.Tensor] = None, long: Optional[bool] = None) -> torch.Tensor:
+                   queue: Optional[torch.Tensor] = None, long: Optional[bool] = None, pieces: Optional[int] = None) -> torch.Tensor:
     """Varlen non-absorbed MLA attention (reference: the prefill FIA calls, src/omni_npu/attention/backends/mla.py:574-590
     and :415-431).  q_nope [T,N,128], q_pe [T,N,64], k_nope [Tk,N,128], k_pe [Tk,64] (shared by the heads), v [Tk,N,128],
     cu_q / cu_k int32 [B+1] device tensors, out [T,N,128] bf16 or fp32, lse_out fp32 [T,N].  ``window`` keeps only the
@@ -956,7 +981,8 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
     ``pick`` (int32 [T, W] bits, see topk's mask; W even and wide enough for the longest sequence; no window, no earlier
     result): a token attends over the keys its bits name.
     ``queue``: prefill_queue's memory, holding zeros; the call uses it up.  ``long``: with the queue and fp16 keys and values, no window
-    and no picks, the kernel of 64 rows to a wavefront (None: where it is the faster one)."""
+    and no picks, the kernel of 64 rows to a wavefront (None: where it is the faster one).  ``pieces``: with fp16 keys and values and none
+    of window, picks, queue and earlier result, into how many pieces a block's keys are cut (None: see prefill_pieces)."""
     if window is not None and window < 1:
         raise ValueError(f"prefill_varlen: window must be positive (got {window})")
     _need_cuda(q_nope, q_pe, k_nope, k_pe, v, cu_q, cu_k, out, lse_out)
@@ -1004,14 +1030,14 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
             context = None
         elif k_nope.shape[0] == 0:                             # no causal key in any sequence
             return prefill_varlen(q_nope, q_pe, *context[:3], cu_q, context[3], max_q_len, scale, False, out, lse_out, prev_out=prev_out,
-                                  prev_lse=prev_lse, queue=queue, long=long)
+                                  prev_lse=prev_lse, queue=queue, long=long, pieces=pieces)
     batch = cu_q.numel() - 1
     if queue is not None:
         _need_cuda(queue)
         if batch > 64 or n % 8 or queue.dtype != torch.int32 or queue.numel() < _PREFILL_QUEUE_WORDS or not queue.is_contiguous():
             raise TypeError("prefill_varlen: a queue (prefill_queue) goes with up to 64 sequences and a multiple of eight heads")
+    seen = k_nope.shape[0] + (context[0].shape[0] if context is not None else 0) - (t // 2 if causal else 0)
     if long is None:
-        seen = k_nope.shape[0] + (context[0].shape[0] if context is not None else 0) - (t // 2 if causal else 0)
         long = kv_half and window is None and pick is None and _prefill_long_rows(t, batch, n) and seen >= _PREFILL_LONG_KEYS * batch
         if long and queue is None:                             # (5 us to clear one, of a launch of some hundred)
             queue = torch.zeros(_PREFILL_QUEUE_WORDS, dtype=torch.int32, device=q_nope.device)
@@ -1021,6 +1047,26 @@ def prefill_varlen(q_nope: torch.Tensor, q_pe: torch.Tensor, k_nope: torch.Tenso
         if queue is None or not kv_half or window is not None or pick is not None:
             raise TypeError("prefill_varlen: long goes with a queue and fp16 keys and values, without a window or picks")
         kv_code |= _PREFILL_LONG
+    if pieces is None:
+        pieces = 1
+        if kv_half and window is None and pick is None and queue is None and prev_out is None:
+            pieces = prefill_pieces(t, batch, max_q_len, n, seen)
+    elif pieces > 1 and (not kv_half or window is not None or pick is not None or queue is not None or prev_out is not None):
+        raise TypeError("prefill_varlen: pieces go with fp16 keys and values, without a window, picks, a queue or an earlier result")
+    if k_nope.shape[0] and t and pieces > 1:
+        extra = (None, 0, None, None, 0, None)
+        if context is not None:
+            k1, pe1, v1, cu1 = context
+            extra = (k1.data_ptr(), k1.stride(1), pe1.data_ptr(), v1.data_ptr(), v1.stride(1), cu1.data_ptr())
+        parts = torch.empty(pieces * t * n * 129, dtype=torch.float32, device=q_nope.device)
+        rc = lib.mla_prefill_varlen_split(
+            q_nope.data_ptr(), q_nope.stride(0), q_nope.stride(1), q_pe.data_ptr(), q_pe.stride(0), q_pe.stride(1),
+            k_nope.data_ptr(), k_nope.stride(0), k_nope.stride(1), k_pe.data_ptr(), k_pe.stride(0), v.data_ptr(), v.stride(0),
+            v.stride(1), cu_q.data_ptr(), cu_k.data_ptr(), *extra, batch, n, int(max_q_len), 1 if causal else 0, float(scale),
+            out.data_ptr(), out.stride(0), out.stride(1), _DT[out.dtype] | kv_code, lse_out.data_ptr() if lse_out is not None else None,
+            pieces, t, parts.data_ptr(), _stream(q_nope))
+        _lib.check(rc, "mla_prefill_varlen_split")
+        return out
     if k_nope.shape[0] and t and (context is not None or queue is not None):
         extra = (None, 0, None, None, 0, None)
         if context is not None:
