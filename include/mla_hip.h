@@ -443,6 +443,15 @@ int dsa_quant_qkw_fp8(const void* q, int64_t q_stride, int64_t q_rows, void* q8,
                       int64_t cache_row_stride_bytes, float* scale_cache, int64_t scale_page_stride, int32_t page_size,
                       int64_t num_pages, mlahip_stream_t stream);
 
+/* The same for a step whose query tokens from first_token on are prompts (query_start_loc [batch + 1] counts from there, seq_lens
+ * [batch]; heads a multiple of 64): tokens of theirs that see at most skip_up_to keys get neither q8 rows nor weights. */
+int dsa_quant_qkw_fp8_above(const void* q, int64_t q_stride, int64_t tokens, void* q8, const void* weights, int32_t w_f32,
+                            int64_t w_stride, int32_t heads, float* w_out, const void* k, int64_t k_stride, int64_t k_rows,
+                            const int64_t* slot_mapping, void* k8_cache, int64_t cache_page_stride_bytes,
+                            int64_t cache_row_stride_bytes, float* scale_cache, int64_t scale_page_stride, int32_t page_size,
+                            int64_t num_pages, const int32_t* query_start_loc, const int32_t* seq_lens, int32_t batch,
+                            int32_t max_q_len, int64_t first_token, int32_t skip_up_to, mlahip_stream_t stream);
+
 /* With a workspace of dsa_topk_workspace_bytes() the selection of a token is spread over several workgroups (three
  * launches that meet in the workspace: slice histograms, boundary-bin gather, ordered write), which is what a
  * decode step with few tokens and long rows needs; with workspace == NULL one workgroup per token does everything and

@@ -48,6 +48,10 @@ def indexer_cache_views(index_cache: torch.Tensor):
     return k8, ks
 
 
+# In the place of pick bits: the prompts are no longer than the selection, every token attends over all the keys it sees
+EVERY_KEY = "every key"
+
+
 def _mask_words(stride: int) -> int:
     """32-bit words of a row of pick bits over ``stride`` scores: whole 64-key tiles."""
     return stride // 64 * 2 + 2
@@ -204,12 +208,25 @@ class LightningIndexer:
                                                                                                      attn_metadata):
             return self.topk_indices_buffer[:t].view(t, 1, self.topk_tokens)
         k8, ks = indexer_cache_views(kv_cache[2])
-        q8 = torch.empty(t, self.n_head, self.head_dim, dtype=torch.uint8, device=q.device)
-        qs = torch.empty(t, self.n_head, dtype=torch.float32, device=q.device)
-        # the new keys into the cache and the queries into plain buffers: one launch
-        K.quant_qk_fp8(q.reshape(t * self.n_head, self.head_dim), q8, qs, k.reshape(-1, self.head_dim), k8, ks,
-                       attn_metadata.slot_mapping)
-        w = weights.float().contiguous()
+        p = attn_metadata.prefill if attn_metadata.num_prefills > 0 else None
+        masked = (p is not None and self.masked_pairs_per_pick > 0
+                  and p.over_up_projected(self.topk_tokens, self.masked_pairs_per_pick))
+        # (prompts no longer than the selection: every token takes all the keys it sees)
+        whole = masked and p.max_query_len <= self.topk_tokens
+        # the new keys into the cache and the queries that are scored into plain buffers: one launch
+        if p is not None and self.n_head % 64 == 0:
+            ndt = attn_metadata.num_decode_tokens if attn_metadata.num_decodes > 0 else 0
+            p_qsl = p.query_start_loc.to(torch.int32).contiguous()
+            q8, w = K.quant_qkw_fp8_above(q.reshape(t, self.n_head, self.head_dim), weights, ndt if whole else t,
+                                          k.reshape(-1, self.head_dim), k8, ks, attn_metadata.slot_mapping, p_qsl,
+                                          p.kv_lens.contiguous(), p.max_query_len, ndt, self.topk_tokens)
+            qs = None
+        else:
+            q8 = torch.empty(t, self.n_head, self.head_dim, dtype=torch.uint8, device=q.device)
+            qs = torch.empty(t, self.n_head, dtype=torch.float32, device=q.device)
+            K.quant_qk_fp8(q.reshape(t * self.n_head, self.head_dim), q8, qs, k.reshape(-1, self.head_dim), k8, ks,
+                           attn_metadata.slot_mapping)
+            w = weights.float().contiguous()
         out = self.topk_indices_buffer[:t]
         off = 0
         self._rows_meta = self._mask_meta = self._mask = None
@@ -222,21 +239,22 @@ class LightningIndexer:
                 ntok = t - off
                 lens, q_len = meta.kv_lens, meta.max_query_len
                 qsl = meta.query_start_loc.to(torch.int32).contiguous()
-            masked = (self.masked_pairs_per_pick > 0 and meta is attn_metadata.prefill
-                      and meta.over_up_projected(self.topk_tokens, self.masked_pairs_per_pick))
+            over_own = masked and meta is p
             max_len = meta.block_table.shape[1] * k8.shape[1]
-            if masked:                                              # (the longest prompt, not the longest the server takes)
+            if over_own:                                            # (the longest prompt, not the longest the server takes)
                 max_len = min(max_len, (q_len + 63) // 64 * 64)
             stride = K.indexer_logits_stride(max_len)
             lg = self._scores_buffer(ntok, stride, q.device)
             sl = slice(off, off + ntok)
-            if not masked or q_len > self.topk_tokens:              # (else every token takes all the keys it sees)
-                K.indexer_scores(q8[sl], w[sl], k8, ks, meta.block_table, lens, lg, q_len=q_len, q_scale=qs[sl],
+            if not (over_own and whole):
+                K.indexer_scores(q8[sl], w[sl], k8, ks, meta.block_table, lens, lg, q_len=q_len, q_scale=None if qs is None else qs[sl],
                                  query_start_loc=qsl, max_seq_len=max_len, skip_up_to=self.topk_tokens)
-            if masked:
-                self._mask = torch.empty(ntok, _mask_words(stride), dtype=torch.int32, device=q.device)
+            if over_own:
+                if whole:                                           # (rows as wide as these prompts: what picks the kernel by their length)
+                    lg = self._logits.view(-1)[:ntok * stride].view(ntok, stride)
                 self._mask_meta = attn_metadata
-                K.topk(lg, lens, self.topk_tokens, out[sl], q_len=q_len, query_start_loc=qsl, mask=self._mask)
+                self._mask = EVERY_KEY if whole else torch.empty(ntok, _mask_words(stride), dtype=torch.int32, device=q.device)
+                K.topk(lg, lens, self.topk_tokens, out[sl], q_len=q_len, query_start_loc=qsl, mask=None if whole else self._mask)
             else:
                 K.topk(lg, lens, self.topk_tokens, out[sl], q_len=q_len, query_start_loc=qsl, block_table=meta.block_table,
                        page_size=k8.shape[1], num_pages=k8.shape[0], rows=self.rows_buffer[sl],
@@ -271,8 +289,8 @@ class LightningIndexer:
         return True
 
     def mask_for(self, attn_metadata):
-        """The picks of the step's prompt tokens as bits [T, W] (kernels.topk's mask) if the last selection made them for this
-        very metadata object and the attention has not used them yet, else None."""
+        """The picks of the step's prompt tokens as bits [T, W] (kernels.topk's mask), or EVERY_KEY, if the last selection made them
+        for this very metadata object and the attention has not used them yet, else None."""
         return self._mask if self.masked_prompts(attn_metadata) else None
 
     def masked_prompts(self, attn_metadata) -> bool:
@@ -283,7 +301,7 @@ class LightningIndexer:
     def drop_mask(self) -> None:
         """The attention has queued its use of the bits: their memory (a bit per pair of a prompt, 8 MB for 8k tokens) goes back
         behind it instead of staying with every layer until that layer's next step."""
-        if self._mask is not None and self._mask.is_cuda:
+        if isinstance(self._mask, torch.Tensor) and self._mask.is_cuda:
             self._mask.record_stream(torch.cuda.current_stream(self._mask.device))
         self._mask = None
 
@@ -394,7 +412,7 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
         queue = K.prefill_queue(t, cu.numel() - 1, prefill.max_query_len, n, q.device)
         k_nope, pe, v, _ = self._kv_up_rows(kv_c_normed, k_pe, queue)
         K.prefill_varlen(q[..., :128], q[..., 128:], k_nope, pe, v, cu, cu, prefill.max_query_len, self.scale, True,
-                         out.view(t, n, 128), pick=pick, queue=queue)
+                         out.view(t, n, 128), pick=None if pick is EVERY_KEY else pick, queue=queue)
         return True
 
     def forward(self, layer, q: torch.Tensor, k_c_normed: torch.Tensor, k_pe: torch.Tensor,

@@ -1259,6 +1259,51 @@ def quant_qk_fp8(q: torch.Tensor, q8: torch.Tensor, q_scale: torch.Tensor, k: to
     _lib.check(rc, "dsa_quant_qk_fp8")
 
 
+def quant_qkw_fp8_above(q: torch.Tensor, weights: torch.Tensor, tokens: int, k: torch.Tensor, k8_cache: torch.Tensor,
+                        scale_cache: torch.Tensor, slot_mapping: torch.Tensor, query_start_loc: torch.Tensor, seq_lens: torch.Tensor,
+                        max_q_len: int, first_token: int, skip_up_to: int):
+    """(q8 [tokens,H,128] e4m3 bits, w [tokens,H] fp32) of the first ``tokens`` of q (bf16 [T,H,128], H a multiple of 64) and of the
+    head weights [T,H], the query scales folded into w, and the new index keys k [T,128] into the cache as quant_qk_fp8 writes
+    them, in one launch.  Tokens from ``first_token`` on are prompts (query_start_loc int32 [B+1] counts from there, seq_lens int32
+    [B]); those that see at most ``skip_up_to`` keys get no queries and no weights."""
+    _need_cuda(q, weights, k, k8_cache, scale_cache, slot_mapping, query_start_loc, seq_lens)
+    t, h, d = q.shape
+    q2, k2 = q.reshape(t * h, d), k.reshape(-1, k.shape[-1])
+    if k8_cache.dim() == 4 and k8_cache.shape[2] == 1:
+        k8_cache = k8_cache.squeeze(2)
+    for x in (q2, k2):
+        if x.shape[-1] != 128 or x.dtype != torch.bfloat16 or x.stride(-1) != 1:
+            raise TypeError("quant_qkw_fp8_above: bf16 rows of 128")
+    if h % 64 or not 0 <= tokens <= t or weights.shape != (t, h) or first_token < 0:
+        raise ValueError("quant_qkw_fp8_above: q [T,H,128] and weights [T,H], H a multiple of 64, at most T tokens")
+    if weights.dtype not in (torch.float32, torch.bfloat16) or weights.stride(1) != 1:
+        weights = weights.float().contiguous()
+    if k8_cache.dim() != 3 or k8_cache.element_size() != 1 or k8_cache.stride(-1) != 1 or scale_cache.dtype != torch.float32 or \
+            scale_cache.shape[:2] != k8_cache.shape[:2]:
+        raise ValueError("quant_qkw_fp8_above: paged outputs must be 1-byte [nblk,page,128] and fp32 [nblk,page]")
+    ksc = scale_cache.reshape(k8_cache.shape[0], k8_cache.shape[1])
+    if ksc.stride(-1) != 1:
+        raise ValueError("quant_qkw_fp8_above: scale rows must be contiguous")
+    for x in (query_start_loc, seq_lens):
+        if x.dtype != torch.int32 or not x.is_contiguous():
+            raise TypeError("quant_qkw_fp8_above: query_start_loc and seq_lens must be contiguous int32")
+    b = query_start_loc.numel() - 1
+    if seq_lens.numel() < b:
+        raise ValueError("quant_qkw_fp8_above: a length for every request")
+    if slot_mapping.dtype != torch.int64 or not slot_mapping.is_contiguous():
+        slot_mapping = slot_mapping.to(torch.int64).contiguous()
+    q8 = torch.empty(tokens, h, 128, dtype=torch.uint8, device=q.device)
+    w = torch.empty(tokens, h, dtype=torch.float32, device=q.device)
+    rc = _lib.load().dsa_quant_qkw_fp8_above(
+        q2.data_ptr(), q2.stride(0), tokens, q8.data_ptr(), weights.data_ptr(), int(weights.dtype == torch.float32), weights.stride(0), h,
+        w.data_ptr(), k2.data_ptr(), k2.stride(0), min(k2.shape[0], slot_mapping.numel()), slot_mapping.data_ptr(),
+        k8_cache.data_ptr(), k8_cache.stride(0), k8_cache.stride(1), ksc.data_ptr(), ksc.stride(0), k8_cache.shape[1],
+        k8_cache.shape[0], query_start_loc.data_ptr(), seq_lens.data_ptr(), b, int(max_q_len), int(first_token), int(skip_up_to),
+        _stream(q))
+    _lib.check(rc, "dsa_quant_qkw_fp8_above")
+    return q8, w
+
+
 def quant_rows_fp8(x: torch.Tensor, out8: torch.Tensor, out_scale: torch.Tensor,
                    slot_mapping: Optional[torch.Tensor] = None) -> None:
     """Per-row e4m3 quantisation of bf16 rows [R,128] (scale = amax/448).  Without ``slot_mapping``: out8 [R,128] (1-byte
