@@ -339,8 +339,14 @@ struct QuantRows {
   const void* w; int32_t w_f32, heads; int64_t w_st; float* w_out;
 };
 
-// Rows r, r + 16, ... (kRows of them), all asked for before the first is worked on
-template <int kRows>
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+template <int kBy> __device__ __forceinline__ uint32_t quant_max_ror(uint32_t v) {       // over the sixteen lanes of a row
+  const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x120 + kBy, 0xf, 0xf, false);
+  return v > o ? v : o;
+}
+
+// Rows r, r + 16, ... (kRows of them), all asked for before the first is worked on.  kToken: of token blockIdx.x
+template <int kRows, bool kToken = false>
 __device__ __forceinline__ void quant_rows(const QuantRows& q, int64_t r0) {
   const auto [src, src_stride, rows, slots, dst8, d_sp, d_sr, dscale, s_sp, page_size, num_pages, w_in, w_f32, heads, w_st, w_out] = q;
   const int l16 = threadIdx.x & 15;
@@ -366,25 +372,47 @@ __device__ __forceinline__ void quant_rows(const QuantRows& q, int64_t r0) {
 #pragma unroll
   for (int i = 0; i < kRows; i++) {
     const int64_t r = r0 + i * 16;
-    float x[8], amax = 0.f;
+    float x[8], y[8];
 #pragma unroll
     for (int e = 0; e < 8; e++) x[e] = __uint_as_float((e & 1) ? raw[i][e >> 1] & 0xffff0000u : raw[i][e >> 1] << 16);
+    // the row's largest magnitude as bf16 bits, in which numbers (and infinity) are ordered as integers and NaNs lie above
+    u16x2 top = {0, 0};
 #pragma unroll
-    for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(x[e]));
+    for (int e = 0; e < 4; e++) top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, raw[i][e] & 0x7fff7fffu));
+    uint32_t mx = top[0] > top[1] ? top[0] : top[1];
+    mx = quant_max_ror<8>(mx);
+    mx = quant_max_ror<4>(mx);
+    mx = quant_max_ror<2>(mx);
+    mx = quant_max_ror<1>(mx);
+    float amax = __uint_as_float(mx << 16);
+    float scale = amax > 0.f ? amax / 448.f : 1.f;
+    // x / scale by the reciprocal and one correction with its exact remainder: the same e4m3 numbers as by the division, for every bf16
+    // x and amax (checked one by one, with reciprocals an ulp off to either side), in three instructions instead of a dozen.  For maxima
+    // from 2^-50 to 2^66, and zero; nothing near the ends of fp32, and no NaN
+    if (__builtin_amdgcn_ballot_w64(mx != 0 && mx - ((127 - 50) << 7) > (116 << 7)) == 0) {
+      const float rcp = __builtin_amdgcn_rcpf(scale);
 #pragma unroll
-    for (int o = 1; o < 16; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+      for (int e = 0; e < 8; e++) {
+        const float q0 = x[e] * rcp;
+        y[e] = __builtin_amdgcn_fmed3f(__builtin_fmaf(__builtin_fmaf(-q0, scale, x[e]), rcp, q0), -448.f, 448.f);
+      }
+    } else {                                                  // (NaNs count for nothing in the maximum)
+      amax = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(x[e]));
+#pragma unroll
+      for (int o = 1; o < 16; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+      scale = amax > 0.f ? amax / 448.f : 1.f;
+#pragma unroll
+      for (int e = 0; e < 8; e++) y[e] = fminf(fmaxf(x[e] / scale, -448.f), 448.f);
+    }
     if (slot[i] < 0) continue;
     int64_t pg = 0, off = slot[i];
     if (slots) { pg = off / page_size; off -= pg * page_size; }
-    const float scale = amax > 0.f ? amax / 448.f : 1.f;
     uint32_t w[2];
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-      float y[4];
-#pragma unroll
-      for (int e = 0; e < 4; e++) y[e] = fminf(fmaxf(x[4 * h + e] / scale, -448.f), 448.f);
-      w[h] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(y[2], y[3], __builtin_amdgcn_cvt_pk_fp8_f32(y[0], y[1], 0, false), true);
-    }
+    for (int h = 0; h < 2; h++)
+      w[h] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(y[4 * h + 2], y[4 * h + 3], __builtin_amdgcn_cvt_pk_fp8_f32(y[4 * h], y[4 * h + 1], 0, false), true);
     uint8_t* d = dst8 + pg * d_sp + off * d_sr + l16 * 8;
     if ((((uintptr_t)dst8 | (uintptr_t)d_sp | (uintptr_t)d_sr) & 7) == 0) {
       *(u32x2*)d = u32x2{w[0], w[1]};
@@ -395,7 +423,8 @@ __device__ __forceinline__ void quant_rows(const QuantRows& q, int64_t r0) {
     if (l16 == 0) {
       if (dscale) dscale[pg * s_sp + off] = scale;
       if (w_out) {
-        const int64_t tk = r / heads, at = tk * w_st + (r - tk * heads);
+        const int32_t tk = kToken ? (int32_t)blockIdx.x : (int32_t)((uint32_t)r / (uint32_t)heads);       // (rows < 2^31)
+        const int64_t at = tk * w_st + ((int32_t)r - tk * heads);
         w_out[r] = (w_f32 ? ((const float*)w_in)[at] : (float)((const __bf16*)w_in)[at]) * scale;
       }
     }
@@ -416,7 +445,8 @@ __global__ __launch_bounds__(256) void dsa_quant_rows2_kernel(const QuantRows a,
 // The same for a step with prompts: the queries of its tokens from first_token on (requests as in qsl and lens) whose selection takes
 // all the keys they see are read by nothing and left out.  A workgroup to a token, four rows of a lane in flight; what bounds it are
 // the bytes of the others.  Every workgroup finds its token's request by itself, a lane to a request.  us per launch, all rows / this:
-// prompts of 1500, 3665 and 5003 tokens, k = 2048, 58.0 / 48.7; of 737 to 2077 tokens, 34.0 / 8.8.
+// prompts of 1500, 3665 and 5003 tokens, k = 2048, 58.0 / 34.9
+// (9300 scored tokens 79.8 -> 58.9 since the division went); of 737 to 2077 tokens, 34.0 / 7.6.
 struct QuantTokens { const int32_t *qsl, *lens; int32_t batch, max_q_len, tokens, first_token, skip_up_to; };
 __global__ __launch_bounds__(256) void dsa_quant_tokens_kernel(const QuantRows a, const QuantRows b, const QuantTokens t) {
   const int tok = blockIdx.x, lane = threadIdx.x & 63;
@@ -437,7 +467,7 @@ __global__ __launch_bounds__(256) void dsa_quant_tokens_kernel(const QuantRows a
     }
     if (__builtin_amdgcn_ballot_w64(all) != 0) return;
   }
-  for (int h = threadIdx.x >> 4; h < a.heads; h += 64) quant_rows<4>(a, (int64_t)tok * a.heads + h);
+  for (int h = threadIdx.x >> 4; h < a.heads; h += 64) quant_rows<4, true>(a, (int64_t)tok * a.heads + h);
 }
 
 }  // namespace mlahip

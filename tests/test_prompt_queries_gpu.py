@@ -59,3 +59,31 @@ def test_prompts_no_longer_than_the_selection(dev, q_lens):
     select.masked_pairs_per_pick = 0.0
     select(*i, kv_cache, meta)
     assert torch.equal(picks, select.topk_indices_buffer[:t])
+
+
+@pytest.mark.parametrize("exp", [0, 64, -49, -51, 65, 66, 100, -100, -126])
+def test_quantised_rows_are_the_division_s_for_every_pair_of_mantissas(dev, exp):
+    """Every bf16 mantissa as a row's maximum, against every bf16 number down to 2^-24 of it: the codes and scales of x / (amax / 448) in
+    fp32.  Exponents on both sides of what the reciprocal is used for, up to subnormal scales."""
+    m = torch.arange(128, dtype=torch.float64) / 128 + 1
+    amax, x = m * 2.0 ** exp, (m[None] * 2.0 ** (exp - torch.arange(24, dtype=torch.float64))[:, None]).reshape(-1)
+    x[::2] *= -1
+    x = torch.cat([x, torch.zeros(-len(x) % 127, dtype=torch.float64)]).view(1, -1, 127)
+    rows = torch.cat([amax.view(-1, 1, 1).expand(-1, x.shape[1], 1), x.expand(128, -1, -1)], 2).reshape(-1, 128)
+    rows = torch.where(rows.abs() > rows[:, :1], rows / 2, rows).to(torch.bfloat16)
+    amax32 = rows[:, 0].float()
+    scale = torch.where(amax32 > 0, amax32 / 448.0, torch.ones_like(amax32))
+    want = (rows.float() / scale[:, None]).clamp(-448, 448).to(torch.float8_e4m3fn).view(torch.uint8)
+    got, sc = torch.empty(rows.shape, dtype=torch.uint8, device=dev), torch.empty(rows.shape[0], device=dev)
+    K.quant_rows_fp8(rows.to(dev), got, sc)
+    assert torch.equal(sc.cpu(), scale) and torch.equal(got.cpu(), want)
+
+
+def test_a_nan_counts_for_nothing_in_a_row_s_maximum(dev):
+    rows = torch.randn(5, 128, generator=torch.Generator().manual_seed(1)).bfloat16()
+    rows[1, 7] = rows[3, 0] = float("nan")
+    clean = rows.nan_to_num(0.0)
+    got, sc = [torch.empty(5, 128, dtype=torch.uint8, device=dev) for _ in range(2)], [torch.empty(5, device=dev) for _ in range(2)]
+    for x, a, b in zip((rows, clean), got, sc):
+        K.quant_rows_fp8(x.to(dev), a, b)
+    assert torch.equal(sc[0], sc[1]) and torch.equal(got[0][~rows.isnan().to(dev)], got[1][~rows.isnan().to(dev)])
