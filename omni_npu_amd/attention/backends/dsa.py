@@ -18,7 +18,7 @@ import torch
 
 from ... import _host
 from ... import kernels as K
-from .mla import HalfUpProjection, _caller_wrote_cache, _persistent_int32
+from .mla import HalfUpProjection, _caller_wrote_cache, _is_its_weight, _persistent_int32
 from ..._vllm_compat import (PAD_SLOT_ID, AttentionCGSupport, AttentionType, MLACommonBackend, MLACommonBaseImpl,
                              MLACommonDecodeMetadata, MLACommonMetadata, MLACommonMetadataBuilder,
                              MLACommonPrefillMetadata, QueryLenSupport, get_current_vllm_config)
@@ -207,12 +207,14 @@ class LightningIndexer:
         if attn_metadata.num_prefills == 0 and attn_metadata.num_decodes > 0 and self._native_select(q, k, weights, kv_cache[2],
                                                                                                      attn_metadata):
             return self.topk_indices_buffer[:t].view(t, 1, self.topk_tokens)
-        k8, ks = indexer_cache_views(kv_cache[2])
         p = attn_metadata.prefill if attn_metadata.num_prefills > 0 else None
         masked = (p is not None and self.masked_pairs_per_pick > 0
                   and p.over_up_projected(self.topk_tokens, self.masked_pairs_per_pick))
         # (prompts no longer than the selection: every token takes all the keys it sees)
         whole = masked and p.max_query_len <= self.topk_tokens
+        if masked and attn_metadata.num_decodes == 0 and self._native_select_prompts(q, k, weights, kv_cache[2], attn_metadata, whole):
+            return self.topk_indices_buffer[:t].view(t, 1, self.topk_tokens)
+        k8, ks = indexer_cache_views(kv_cache[2])
         # the new keys into the cache and the queries that are scored into plain buffers: one launch
         if p is not None and self.n_head % 64 == 0:
             ndt = attn_metadata.num_decode_tokens if attn_metadata.num_decodes > 0 else 0
@@ -286,6 +288,27 @@ class LightningIndexer:
                                        self.topk_indices_buffer, self.rows_buffer, self.counts_buffer):
             return False
         self._rows_meta = attn_metadata
+        return True
+
+    def _native_select_prompts(self, q, k, weights, index_cache, attn_metadata, whole: bool) -> bool:
+        """The selection of a step of masked prompts in one native call; False, with nothing done, where that call does not know the
+        case."""
+        t, p = q.shape[0], attn_metadata.prefill
+        if not q.is_cuda or self.n_head != 64 or self.head_dim != INDEX_HEAD_DIM or q.dim() != 3:
+            return False
+        max_len = min(p.block_table.shape[1] * index_cache.shape[1], (p.max_query_len + 63) // 64 * 64)
+        stride = K.indexer_logits_stride(max_len)
+        lg, mask = self._scores_buffer(t, stride, q.device), None
+        if whole:
+            lg = self._logits.view(-1)[:t * stride].view(t, stride)
+        else:
+            mask = torch.empty(t, _mask_words(stride), dtype=torch.int32, device=q.device)
+        self._rows_meta = self._mask_meta = self._mask = None
+        if not _host.load().dsa_select_prompts(q, k, weights, index_cache, attn_metadata.slot_mapping, p.block_table, p.kv_lens,
+                                               p.query_start_loc, p.max_query_len, max_len, self.topk_tokens, whole, lg,
+                                               self.topk_indices_buffer, mask):
+            return False
+        self._mask_meta, self._mask = attn_metadata, EVERY_KEY if whole else mask
         return True
 
     def mask_for(self, attn_metadata):
@@ -408,11 +431,16 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
                 tuple(out.shape) != (t, n * 128) or (q.stride(0) | q.stride(1) | k_pe.stride(0) | out.stride(0)) % 8 or \
                 (q.data_ptr() | k_pe.data_ptr() | out.data_ptr()) % 16:
             return False
+        bits = None if pick is EVERY_KEY else pick
+        if (self.prefill_kv_fp16 or (self.keys_bf16_values_f16 and _is_its_weight(self.kv_b_proj))) and _host.load().prefill(
+                q, kv_c_normed, k_pe, 0, t, prefill.query_start_loc, prefill.max_query_len, w, self.prefill_kv_fp16, self.scale, out,
+                bits, None, None, None, None, None, None, 0):
+            return True
         cu = prefill.query_start_loc.to(torch.int32).contiguous()
         queue = K.prefill_queue(t, cu.numel() - 1, prefill.max_query_len, n, q.device)
         k_nope, pe, v, _ = self._kv_up_rows(kv_c_normed, k_pe, queue)
         K.prefill_varlen(q[..., :128], q[..., 128:], k_nope, pe, v, cu, cu, prefill.max_query_len, self.scale, True,
-                         out.view(t, n, 128), pick=None if pick is EVERY_KEY else pick, queue=queue)
+                         out.view(t, n, 128), pick=bits, queue=queue)
         return True
 
     def forward(self, layer, q: torch.Tensor, k_c_normed: torch.Tensor, k_pe: torch.Tensor,

@@ -517,6 +517,25 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
             d.max_seq_len, self.W_UK_T, self.W_UV, self.scale, attn_metadata.num_decode_tokens, self.sink_len,
             self.sliding_window if self.sink_len > 0 else 0, output, *new)
 
+    def _native_prefill(self, q, k_c_normed, k_pe, kv_cache, attn_metadata, output) -> bool:
+        """The prefill tokens' _forward_prefill in one native call: keys and values from kernels.kv_up, at most one chunk of cached
+        tokens.  False, with nothing done, where that call does not know the case."""
+        prefill = attn_metadata.prefill
+        w = self._plain_up_weight() if self.prefill_kv_fp16 and self.sink_len == 0 else None
+        if w is None or not (self.qk_nope_head_dim == self.v_head_dim == 128):
+            return False
+        ctx, cc = (None, None, None, None, None, None, 0), prefill.chunked_context
+        if cc is not None:
+            chunks = [i for i, toks in enumerate(cc.seq_tot) if int(toks) > 0]
+            if len(chunks) > 1:
+                return False
+            if chunks:
+                i = chunks[0]
+                ctx = (kv_cache[0], None if self.fp8_cache else kv_cache[1], prefill.block_table, cc.cu_seq_lens[i], cc.starts[i],
+                       cc.workspace, int(cc.seq_tot[i]))
+        return _host.load().prefill(q, k_c_normed, k_pe, attn_metadata.num_decode_tokens, attn_metadata.num_actual_tokens,
+                                    prefill.query_start_loc, prefill.max_query_len, w, True, self.scale, output, None, *ctx)
+
     def forward(self, layer, q: torch.Tensor, k_c_normed: torch.Tensor, k_pe: torch.Tensor,
                 kv_cache: Tuple[torch.Tensor, ...], attn_metadata: NPUMLAMetadata,
                 output: Optional[torch.Tensor] = None, output_scale: Optional[torch.Tensor] = None,
@@ -561,7 +580,7 @@ class NPUMLAImpl(HalfUpProjection, MLACommonBaseImpl[NPUMLAMetadata]):
             if done:
                 return output_padded
 
-        if has_prefill:
+        if has_prefill and not self._native_prefill(q, k_c_normed, k_pe, kv_cache, attn_metadata, output):
             output = output[:num_actual_toks, ...]
             q = q[:num_actual_toks, ...]
             k_c_normed = k_c_normed[:num_actual_toks, ...]

@@ -1,21 +1,24 @@
-// The host side of a decode step in native code: one call from Python per layer and stage.
+// The host side of a step in native code: one call from Python per layer and stage.
 //
 // What bounds a small step is not the GPU: through the general Python front end (kernels.py: shape checks, forty pointer and
 // stride look-ups, a ctypes call per launch) one layer of one user took 65 us of host time around 25 us of kernels, and a
 // sparse decode layer 187 us around 142.  The functions here do the checks, the scratch look-up, the library GEMM and the
-// launches of a whole stage.  Each answers false, with nothing launched, when an argument is not what it knows; the caller
+// launches of a whole stage.  (Prefills of few tokens too: three launches of 35 us took 50 us to prepare, behind cached tokens five took
+// 102.)  Each answers false, with nothing launched, when an argument is not what it knows; the caller
 // then takes the general path, which handles the case or says what is wrong with it.  A failing launch raises.
 //
 // Contracts: mla_decode / sparse_decode = NPUMLAImpl.forward / NPUDSAImpl.forward for a step's decode tokens
 // (src/omni_npu/attention/backends/mla.py:868-912, dsa.py:359-389), dsa_select = LightningIndexer for them
 // (src/omni_npu/vllm_patches/patches/models/deepseek/patch_dsv32_indexer.py:104-146), norm_rope_cache =
-// kernels.kv_rmsnorm_rope_cache (src/omni_npu/v1/layers/attention/npu_mla.py:196-210).
+// kernels.kv_rmsnorm_rope_cache (src/omni_npu/v1/layers/attention/npu_mla.py:196-210), prefill = NPUMLAImpl._forward_prefill and
+// NPUDSAImpl._forward_prompts (mla.py:452-616), dsa_select_prompts = LightningIndexer for a step of prompts.
 #include <torch/extension.h>
 #include <ATen/core/LegacyTypeDispatch.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 
+#include <cmath>
 #include <map>
 #include <mutex>
 #include <optional>
@@ -372,19 +375,192 @@ bool norm_rope_cache(const Tensor& kv, const Tensor& gamma, const Tensor& cos, c
   return true;
 }
 
+// kernels._prefill_long_rows, _prefill_blocks, prefill_pieces, and whether kernels.prefill_queue gives a queue (the rules' reasons are there)
+constexpr int64_t kPrefillResident = 512, kPrefillQueueWords = 256, kPrefillLongKeys = 1792;
+bool prefill_long_rows(int64_t tokens, int64_t batch, int64_t heads) {
+  const int64_t whole = batch == 1 ? div_up(tokens, 256) : tokens / 256;
+  return batch > 0 && batch <= 64 && heads % 8 == 0 && heads * whole >= kPrefillResident / 2 &&
+         (batch == 1 ? whole * 256 <= 1.05 * 128 * div_up(tokens, 128) : tokens >= 1024 * batch);
+}
+int64_t prefill_blocks(int64_t tokens, int64_t batch, int64_t max_q_len, int64_t heads) {
+  return heads * std::min(batch * div_up(max_q_len, 128), tokens / 128 + batch);
+}
+int prefill_pieces(int64_t tokens, int64_t batch, int64_t max_q_len, int64_t heads, int64_t seen) {
+  const int64_t blocks = prefill_blocks(tokens, batch, max_q_len, heads);
+  if (blocks < 1 || blocks * 2 > kPrefillResident) return 1;
+  const double tiles = (double)seen / (double)(64 * batch), mib = (double)(tokens * heads * 516) / 1048576.0;
+  const int64_t pieces = std::min({(int64_t)std::sqrt(2.7 * tiles / mib), kPrefillResident / blocks, (int64_t)32});
+  if (pieces < 2) return 1;
+  const double shared = blocks * pieces > kPrefillResident / 2 ? 1.5 : 1.0;
+  return 1.3 * tiles * (1 - shared / (double)pieces) > 0.48 * mib * (double)pieces + 5 ? (int)pieces : 1;
+}
+bool prefill_wants_queue(int64_t tokens, int64_t batch, int64_t max_q_len, int64_t heads) {
+  return batch <= 64 && heads % 8 == 0 &&
+         (prefill_blocks(tokens, batch, max_q_len, heads) > kPrefillResident || prefill_long_rows(tokens, batch, heads));
+}
+
+// Keys and values of latent rows [t, 512] (kernels.kv_up): a head's tokens behind each other, a token's key in front of its value; the
+// rope rows as fp16 (keys_f16) or as they are.
+struct KeyRows { Tensor kv, pe16; const void* pe; int64_t t, pe_st; const char* k() const { return (const char*)kv.data_ptr(); } };
+KeyRows kv_up(const void* c, int64_t c_st, const void* pe, int64_t pe_st, int64_t t, const Tensor& w, int64_t n, bool keys_f16,
+              Tensor* clear, Stream st) {
+  KeyRows r{at::empty({n, t, 256}, w.options().dtype(at::kHalf)), Tensor(), pe, t, pe_st};
+  if (keys_f16) {
+    r.pe16 = at::empty({t, kRope}, w.options().dtype(at::kHalf));
+    r.pe = r.pe16.data_ptr();
+    r.pe_st = kRope;
+  }
+  check(mla_kv_up(c, c_st, w.data_ptr(), w.stride(0), t, (int)n, keys_f16 ? 1 : 0, r.kv.data_ptr(), 256, t * 256, keys_f16 ? pe : nullptr,
+                  keys_f16 ? pe_st : 0, keys_f16 ? r.pe16.data_ptr() : nullptr, keys_f16 ? kRope : 0, clear ? clear->data_ptr() : nullptr,
+                  clear ? (int)clear->numel() : 0, st), "mla_kv_up");
+  return r;
+}
+
+// Rows first .. last - 1 of a step as prompts or chunks of them over up-projected keys and values (kv_b_proj's weight), into
+// out[first:last].  pick: bits of the keys that each row attends over.  nope .. ctx_rows, ctx_toks > 0: the one chunk of cached tokens in
+// front of them, gathered into ctx_rows (fp16 keys only).
+bool prefill(const Tensor& q, const Tensor& kv_c, const Tensor& k_pe, int64_t first, int64_t last, const Tensor& cu_q, int64_t max_q_len,
+             const Tensor& w, bool keys_f16, double scale, const Tensor& out, const OptTensor& pick, const OptTensor& nope,
+             const OptTensor& rope, const OptTensor& block_table, const OptTensor& cu_ctx, const OptTensor& starts,
+             const OptTensor& ctx_rows, int64_t ctx_toks) {
+  if (!current_gpu(q)) return false;
+  const at::Device dev = q.device();
+  const int64_t t = last - first, n = q.size(1), batch = cu_q.numel() - 1;
+  if (!is_bf16(q, 3, dev) || q.size(2) != 192 || first < 0 || t < 1 || q.size(0) < last || !is_bf16(kv_c, 2, dev) || kv_c.size(1) != kNope ||
+      kv_c.size(0) < last || k_pe.scalar_type() != at::kBFloat16 || k_pe.device() != dev || k_pe.size(-1) != kRope || k_pe.stride(-1) != 1 ||
+      !(k_pe.dim() == 2 || (k_pe.dim() == 3 && k_pe.size(1) == 1)) || k_pe.size(0) < last || !is_i32(cu_q, 1, dev) || !cu_q.is_contiguous() ||
+      batch < 1 || max_q_len < 1 || !is_bf16(w, 2, dev) || w.size(0) != n * 256 || w.size(1) != kNope || !is_bf16(out, 2, dev) ||
+      out.size(0) < last || out.size(1) != n * kVDim || scale <= 0)
+    return false;
+  if (((q.stride(0) | q.stride(1) | kv_c.stride(0) | k_pe.stride(0) | w.stride(0) | out.stride(0)) & 7) ||
+      (((uintptr_t)q.data_ptr() | (uintptr_t)kv_c.data_ptr() | (uintptr_t)k_pe.data_ptr() | (uintptr_t)w.data_ptr() | (uintptr_t)out.data_ptr()) & 15) ||
+      kv_c.stride(0) > 1 << 20 || w.stride(0) > 1 << 20)
+    return false;
+  if (pick && (!is_i32(*pick, 2, dev) || pick->size(0) < t || pick->size(1) % 2 || ctx_toks > 0)) return false;
+  Cache c;
+  if (ctx_toks > 0) {
+    if (!keys_f16 || !nope || !block_table || !cu_ctx || !starts || !ctx_rows || !cache_of(*nope, rope, dev, c) || !is_i32(*block_table, 2, dev) ||
+        block_table->size(0) < batch || !is_i32(*cu_ctx, 1, dev) || !cu_ctx->is_contiguous() || cu_ctx->numel() != batch + 1 ||
+        !is_i32(*starts, 1, dev) || !starts->is_contiguous() || starts->numel() < batch || !is_bf16(*ctx_rows, 2, dev) ||
+        ctx_rows->size(0) < ctx_toks || ctx_rows->size(1) < kNope + kRope || (ctx_rows->stride(0) & 7) || ctx_rows->stride(0) > 1 << 20 ||
+        ((uintptr_t)ctx_rows->data_ptr() & 15))
+      return false;
+  }
+  at::AutoDispatchBelowAutograd guard;
+  Stream st = stream_of(q);
+  Tensor queue;
+  if (prefill_wants_queue(t, batch, max_q_len, n)) queue = at::empty({kPrefillQueueWords}, cu_q.options());
+  const int64_t q_st = q.stride(0), q_sh = q.stride(1);
+  const char* q0 = (const char*)q.data_ptr() + 2 * first * q_st;
+  void* o0 = (char*)out.data_ptr() + 2 * first * out.stride(0);
+  const KeyRows own = kv_up((const char*)kv_c.data_ptr() + 2 * first * kv_c.stride(0), kv_c.stride(0),
+                            (const char*)k_pe.data_ptr() + 2 * first * k_pe.stride(0), k_pe.stride(0), t, w, n, keys_f16,
+                            queue.defined() ? &queue : nullptr, st);
+  KeyRows ctx{Tensor(), Tensor(), nullptr, 0, 0};
+  if (ctx_toks > 0) {
+    const Tensor& rows = *ctx_rows;
+    const int32_t *bt = (const int32_t*)block_table->data_ptr(), *cu = (const int32_t*)cu_ctx->data_ptr(), *at0 = (const int32_t*)starts->data_ptr();
+    if (c.rope)
+      check(mla_gather_paged(c.nope->data_ptr(), c.n_sp, c.n_sr, c.rope->data_ptr(), c.r_sp, c.r_sr, c.pages, (int)c.page, rows.data_ptr(),
+                             rows.stride(0), rows.size(0), bt, block_table->stride(0), (int)block_table->size(1), cu, at0, (int)batch,
+                             ctx_toks, st), "mla_gather_paged");
+    else
+      check(mla_gather_paged_fp8(c.nope->data_ptr(), c.n_sp, c.n_sr, c.pages, (int)c.page, rows.data_ptr(), rows.stride(0), rows.size(0), bt,
+                                 block_table->stride(0), (int)block_table->size(1), cu, at0, (int)batch, ctx_toks, st), "mla_gather_paged_fp8");
+    ctx = kv_up(rows.data_ptr(), rows.stride(0), (const char*)rows.data_ptr() + 2 * kNope, rows.stride(0), ctx_toks, w, n, true, nullptr, st);
+  }
+  // what kernels.prefill_varlen chooses
+  const int64_t seen = t + ctx_toks - t / 2;
+  const bool whole_rows = keys_f16 && !pick;
+  const bool rows64 = whole_rows && prefill_long_rows(t, batch, n) && seen >= kPrefillLongKeys * batch;
+  int32_t* qu = queue.defined() && (rows64 || prefill_blocks(t, batch, max_q_len, n) > kPrefillResident) ? (int32_t*)queue.data_ptr() : nullptr;
+  const int pieces = whole_rows && !qu ? prefill_pieces(t, batch, max_q_len, n, seen) : 1;
+  const int type = (keys_f16 ? 16 : 32) + (rows64 ? 64 : 0);   // MLA_PREFILL_KV_F16, _V_F16, _LONG
+  const int32_t *cu = (const int32_t*)cu_q.data_ptr(), *cu1 = ctx_toks > 0 ? (const int32_t*)cu_ctx->data_ptr() : nullptr;
+  const char* k1 = ctx_toks > 0 ? ctx.k() : nullptr;
+  const char* v1 = k1 ? k1 + 2 * 128 : nullptr;
+  const int64_t sh1 = ctx_toks * 256;
+  if (pieces > 1) {
+    Tensor parts = at::empty({pieces * t * n * 129}, q.options().dtype(at::kFloat));
+    check(mla_prefill_varlen_split(q0, q_st, q_sh, q0 + 2 * 128, q_st, q_sh, own.k(), 256, t * 256, own.pe, own.pe_st, own.k() + 2 * 128, 256,
+                                   t * 256, cu, cu, k1, sh1, ctx.pe, v1, sh1, cu1, (int)batch, (int)n, (int)max_q_len, 1, (float)scale, o0,
+                                   out.stride(0), kVDim, type, nullptr, pieces, t, (float*)parts.data_ptr(), st), "mla_prefill_varlen_split");
+    return true;
+  }
+  check(mla_prefill_varlen_queued(q0, q_st, q_sh, q0 + 2 * 128, q_st, q_sh, own.k(), 256, t * 256, own.pe, own.pe_st, own.k() + 2 * 128, 256,
+                                  t * 256, cu, cu, k1, sh1, ctx.pe, v1, sh1, cu1, (int)batch, (int)n, (int)max_q_len, 1, 0, (float)scale,
+                                  pick ? (const uint32_t*)pick->data_ptr() : nullptr, pick ? pick->stride(0) : 0, pick ? (int)pick->size(1) : 0, o0,
+                                  out.stride(0), kVDim, type, nullptr, nullptr, 0, 0, nullptr, qu, st), "mla_prefill_varlen_queued");
+  return true;
+}
+
+// The selection for a step of prompts alone over their own keys (kernels.quant_qkw_fp8_above, indexer_scores, topk), masks as bits; whole:
+// every token takes all the keys it sees, nothing is scored and there are no bits.
+bool dsa_select_prompts(const Tensor& q, const Tensor& k, const Tensor& weights, const Tensor& index_cache, const Tensor& slots,
+                        const Tensor& block_table, const Tensor& lens, const Tensor& qsl, int64_t max_q_len, int64_t max_len, int64_t topk,
+                        bool whole, const Tensor& logits, const Tensor& out, const OptTensor& mask) {
+  if (!current_gpu(q)) return false;
+  const at::Device dev = q.device();
+  if (!is_bf16(q, 3, dev) || q.size(1) != 64 || q.size(2) != 128 || !q.is_contiguous()) return false;
+  const int64_t t = q.size(0), b = lens.numel(), page = index_cache.size(1), pages = index_cache.size(0);
+  const at::ScalarType wt = weights.scalar_type();
+  if (t < 1 || !is_bf16(k, 2, dev) || k.size(0) != t || k.size(1) != 128 || (k.stride(0) & 1) || ((uintptr_t)k.data_ptr() & 3) ||
+      (wt != at::kFloat && wt != at::kBFloat16) || weights.dim() != 2 || weights.size(0) != t || weights.size(1) != 64 || weights.stride(1) != 1 ||
+      weights.device() != dev || !index_cache.is_contiguous() || index_cache.element_size() != 2 || index_cache.device() != dev ||
+      index_cache.numel() != pages * page * 128 || slots.scalar_type() != at::kLong || !slots.is_contiguous() || slots.dim() != 1 ||
+      slots.device() != dev || !is_i32(block_table, 2, dev) || block_table.size(0) < b || b < 1 || !is_i32(lens, 1, dev) || !lens.is_contiguous() ||
+      !is_i32(qsl, 1, dev) || !qsl.is_contiguous() || qsl.numel() != b + 1 || !is(logits, at::kFloat, 2, dev) || logits.size(0) < t ||
+      logits.size(1) < (max_len + 31) / 32 * 32 || !is_i32(out, 2, dev) || out.size(0) < t || out.size(1) < topk || max_q_len < 1 ||
+      ((uintptr_t)q.data_ptr() & 15) || (!whole && (!mask || !is_i32(*mask, 2, dev) || mask->size(0) < t || mask->size(1) * 32 < logits.size(1))))
+    return false;
+  at::AutoDispatchBelowAutograd guard;
+  Stream st = stream_of(q);
+  const int64_t scored = whole ? 0 : t;
+  Tensor q8 = at::empty({scored * 64 * (128 + 4)}, q.options().dtype(at::kByte));
+  float* w = scored ? (float*)((char*)q8.data_ptr() + t * 64 * 128) : nullptr;
+  char* k8 = (char*)index_cache.data_ptr();
+  const int32_t *qs = (const int32_t*)qsl.data_ptr(), *ln = (const int32_t*)lens.data_ptr();
+  check(dsa_quant_qkw_fp8_above(q.data_ptr(), 128, scored, q8.data_ptr(), weights.data_ptr(), wt == at::kFloat ? 1 : 0, weights.stride(0), 64, w,
+                                k.data_ptr(), k.stride(0), std::min(t, slots.numel()), (const int64_t*)slots.data_ptr(), k8, page * 256, 128,
+                                (float*)(k8 + page * 128), page * 64, (int)page, pages, qs, ln, (int)b, (int)max_q_len, 0, (int)topk, st),
+        "dsa_quant_qkw_fp8_above");
+  const float* lg = (const float*)logits.data_ptr();
+  if (!whole)
+    check(dsa_indexer_scores_fp8_above(q8.data_ptr(), 64 * 128, 128, w, 64, nullptr, 0, k8, page * 256, 128, (const float*)(k8 + page * 128),
+                                       page * 64, pages, (int)page, (const int32_t*)block_table.data_ptr(), block_table.stride(0),
+                                       (int)block_table.size(1), ln, qs, (int)b, (int)max_q_len, 64, (int)max_len, (float*)logits.data_ptr(),
+                                       logits.stride(0), (int)topk, st), "dsa_indexer_scores_fp8");
+  const int64_t need = (int64_t)dsa_topk_workspace_bytes((int)b, (int)max_q_len, logits.stride(0));
+  Tensor& ws = scratch(q, st, need, 1);
+  if (whole)
+    check(dsa_topk(lg, logits.stride(0), ln, qs, (int)b, (int)max_q_len, (int)topk, (int32_t*)out.data_ptr(), out.stride(0), ws.data_ptr(),
+                   ws.numel(), st), "dsa_topk");
+  else
+    check(dsa_topk_mask(lg, logits.stride(0), ln, qs, (int)b, (int)max_q_len, (int)topk, (int32_t*)out.data_ptr(), out.stride(0), mask->data_ptr(),
+                        mask->stride(0) * 4, (int)logits.size(1), ws.data_ptr(), ws.numel(), st), "dsa_topk_mask");
+  return true;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  m.doc() = "native host side of the MLA / DSA decode steps (see omni_npu_amd/_host.py)";
+  m.doc() = "native host side of the MLA / DSA steps (see omni_npu_amd/_host.py)";
   m.def("set_workspace", [](py::object fn) { Py_XDECREF(g_workspace); g_workspace = fn.release().ptr(); });
   m.def("cache_write", &cache_write);
   m.def("mla_decode", &mla_decode);
   m.def("sparse_decode", &sparse_decode);
   m.def("dsa_select", &dsa_select);
   m.def("norm_rope_cache", &norm_rope_cache);
+  m.def("prefill", &prefill);
+  m.def("dsa_select_prompts", &dsa_select_prompts);
   // (what this file has a copy of, for a test to hold against kernels.py)
   m.def("launch_splits", &launch_splits);
   m.def("list_splits", &list_splits);
+  m.def("prefill_long_rows", &prefill_long_rows);
+  m.def("prefill_blocks", &prefill_blocks);
+  m.def("prefill_pieces", &prefill_pieces);
+  m.def("prefill_wants_queue", &prefill_wants_queue);
+  m.attr("PREFILL_RULES") = py::make_tuple(kPrefillResident, kPrefillQueueWords, kPrefillLongKeys);
   m.attr("ABSORB_MAX_TOKENS") = kAbsorbMaxTokens;
   m.attr("VUP_MAX_TOKENS") = kVupMaxTokens;
   m.attr("SPARSE_WORKSPACE_CAP") = kSparseWorkspaceCap;

@@ -780,10 +780,11 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
   p.pick = pick; p.pick_st = pick_stride; p.pick_tiles = pick_words / 2;
   p.max_blocks = (max_q_len + kPfRows - 1) / kPfRows;
   p.queue = queue;
+  int rc = ensure_dynamic_lds((const void*)mla_prefill_split_kernel<false>, kPfLdsB, what);
+  if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)mla_prefill_split_kernel<true>, kPfLdsB, what);
+  if (rc != MLA_OK) return rc;
   if (pieces > 1) {
     const int64_t rows = num_tokens * num_heads;
-    const int rc = ensure_dynamic_lds((const void*)(k1_nope ? mla_prefill_split_kernel<true> : mla_prefill_split_kernel<false>), kPfLdsB, what);
-    if (rc != MLA_OK) return rc;
     p.pieces = pieces; p.o_piece = rows * 128; p.lse_piece = rows;
     p.out = parts; p.o_st = (int64_t)num_heads * 128; p.o_sh = 128; p.lse = parts + pieces * rows * 128;
     hipLaunchKernelGGL((k1_nope ? mla_prefill_split_kernel<true> : mla_prefill_split_kernel<false>), dim3(p.max_blocks * pieces, num_heads, batch),
@@ -801,7 +802,6 @@ static int prefill_varlen_impl(const char* what, const void* q_nope, int64_t qn_
            : vh ? (pk ? mla_prefill_varlen_kernel<false, true, true, false, kQ> : mla_prefill_varlen_kernel<false, true, false, false, kQ>)
                 : (pk ? mla_prefill_varlen_kernel<false, false, true, false, kQ> : mla_prefill_varlen_kernel<false, false, false, false, kQ>);
   };
-  int rc = MLA_OK;
   for (int i = 0; i < 14 && rc == MLA_OK; i++)              // (all of them: a caller's warm-up step need not be of the kind that it captures)
     rc = ensure_dynamic_lds((const void*)(i < 7 ? kernel_of(std::false_type{}, (i >> 1) == 2, (i >> 1) != 0, i & 1, i == 6)
                                                 : kernel_of(std::true_type{}, (i - 7) >> 1 == 2, (i - 7) >> 1 != 0, (i - 7) & 1, i == 13)),
