@@ -75,6 +75,66 @@ __device__ __forceinline__ UpTile up_tile(const KvUpParams& p, int idx) {
   return {g * kUpGroup + rem - head * mg, head};
 }
 
+__device__ __forceinline__ void up_rope_rows(const KvUpParams& p) {
+  for (int64_t i = (int64_t)blockIdx.x * 512 + threadIdx.x; i < p.rows * 8; i += (int64_t)gridDim.x * 512) {
+    const bf16x8 v = *(const bf16x8*)(p.pe + (i >> 3) * p.pe_st + (i & 7) * 8);
+    f16x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; e++) o[e] = (_Float16)(float)v[e];
+    *(f16x8*)(p.pe_out + (i >> 3) * p.pe_ost + (i & 7) * 8) = o;
+  }
+}
+
+// A wavefront's 32 tokens x 64 columns (of the keys, or kValues: of the values) through its own 4 KiB at st to `out`, the columns of its
+// tile's first token; at_row: its first token in the tile, whose last one is `left` (the rows behind hold its numbers).
+template <bool kKeysF16, bool kValues>
+__device__ __forceinline__ void up_store(const KvUpParams& p, f32x16 (&acc)[2], char* st, char* out, int at_row, int left) {
+  const int ln = up_lane(), h32 = ln & 31, half = ln >> 5;
+  if constexpr (!kKeysF16 && kValues) {
+    float big = 0.f;
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) big = fmaxf(big, fabsf(acc[b][r]));
+    if (__builtin_amdgcn_ballot_w64(big > 65504.f) != 0) {
+#pragma unroll
+      for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const float v = acc[b][r];
+          acc[b][r] = fabsf(v) > 65504.f && fabsf(v) < INFINITY ? copysignf(65504.f, v) : v;
+        }
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      u32x2 v;
+#pragma unroll
+      for (int e = 0; e < 2; e++) {
+        const f32x2 f = {acc[b][g * 4 + 2 * e], acc[b][g * 4 + 2 * e + 1]};
+        if (kKeysF16 || kValues) v[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, f16x2));
+        else v[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
+      }
+      *(u32x2*)(st + h32 * 128 + (((b * 4 + g) ^ ((h32 >> 1) & 7)) << 4) + half * 8) = v;
+    }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");           // (the wavefront's own writes, read back by its other lanes)
+  __builtin_amdgcn_wave_barrier();
+  u32x4 row[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) row[k] = *(const u32x4*)(st + k * 1024 + ln * 16);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const int sr = k * 8 + (ln >> 3), tr = at_row + sr;
+    const int at = tr < left ? tr : left;
+    u32x4* to = (u32x4*)(out + (int64_t)at * p.o_st + (((ln & 7) ^ ((sr >> 1) & 7)) << 4));
+    if (p.stream_out) __builtin_nontemporal_store(row[k], to);
+    else *to = row[k];
+  }
+}
+
 }  // namespace
 
 // kKeysF16: keys leave as fp16, rounded to nearest, and overflow as a conversion does; values too.  Otherwise keys leave as bf16
@@ -93,17 +153,8 @@ __global__ __launch_bounds__(512, 2) void mla_kv_up_kernel(const KvUpParams p) {
   int idx = (int)((int64_t)total * xcd / 8) + (blockIdx.x >> 3);
 
   if (blockIdx.x == 0 && (int)threadIdx.x < p.clear_words) p.clear[threadIdx.x] = 0u;
-  auto rope_rows = [&]() {
-    for (int64_t i = (int64_t)blockIdx.x * 512 + threadIdx.x; i < p.rows * 8; i += (int64_t)gridDim.x * 512) {
-      const bf16x8 v = *(const bf16x8*)(p.pe + (i >> 3) * p.pe_st + (i & 7) * 8);
-      f16x8 o;
-#pragma unroll
-      for (int e = 0; e < 8; e++) o[e] = (_Float16)(float)v[e];
-      *(f16x8*)(p.pe_out + (i >> 3) * p.pe_ost + (i & 7) * 8) = o;
-    }
-  };
   if (idx >= last) {
-    if (p.pe != nullptr) rope_rows();
+    if (p.pe != nullptr) up_rope_rows(p);
     return;
   }
 
@@ -143,7 +194,7 @@ __global__ __launch_bounds__(512, 2) void mla_kv_up_kernel(const KvUpParams p) {
     copy_x(s, 1);
     copy_w(w_base, s, 1);
   }
-  if (p.pe != nullptr) rope_rows();
+  if (p.pe != nullptr) up_rope_rows(p);
 
   // operand reads: granule 2 kk + half of a row
   const char* xr[4];
@@ -235,67 +286,140 @@ __global__ __launch_bounds__(512, 2) void mla_kv_up_kernel(const KvUpParams p) {
       phase_end(stored && s < 1);
     }
 
-    // results: a quadrant at a time through the wavefront's own 4 KiB (32 tokens x 128 bytes)
+    // results: a quadrant at a time
     char* st = lds + kUpStage + wave * 4096;
-    const int ln = up_lane(), h32 = ln & 31, half = ln >> 5;
     const int64_t left64 = p.rows - 1 - (int64_t)tile.m * kUpTok;
     const int left = left64 < kUpTok ? (int)left64 : kUpTok;
     char* out = p.out + (int64_t)tile.m * kUpTok * p.o_st + (int64_t)tile.head * p.o_sh + wn * 128;
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int i = 0; i < 2; i++) up_store<kKeysF16, false>(p, acc[0][i], st, out, i * 128 + wt * 32, left);
 #pragma unroll
-      for (int i = 0; i < 2; i++) {
-        if constexpr (!kKeysF16) {
-          if (j == 1) {
-            float big = 0.f;
-#pragma unroll
-            for (int b = 0; b < 2; b++)
-#pragma unroll
-              for (int r = 0; r < 16; r++) big = fmaxf(big, fabsf(acc[j][i][b][r]));
-            if (__builtin_amdgcn_ballot_w64(big > 65504.f) != 0) {
-#pragma unroll
-              for (int b = 0; b < 2; b++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                  const float v = acc[j][i][b][r];
-                  acc[j][i][b][r] = fabsf(v) > 65504.f && fabsf(v) < INFINITY ? copysignf(65504.f, v) : v;
-                }
-            }
-          }
-        }
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-          for (int g = 0; g < 4; g++) {
-            u32x2 v;
-#pragma unroll
-            for (int e = 0; e < 2; e++) {
-              const f32x2 f = {acc[j][i][b][g * 4 + 2 * e], acc[j][i][b][g * 4 + 2 * e + 1]};
-              if (kKeysF16 || j == 1) v[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, f16x2));
-              else v[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
-            }
-            *(u32x2*)(st + h32 * 128 + (((b * 4 + g) ^ ((h32 >> 1) & 7)) << 4) + half * 8) = v;
-          }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // (the wavefront's own writes, read back by its other lanes)
-        __builtin_amdgcn_wave_barrier();
-        u32x4 row[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) row[k] = *(const u32x4*)(st + k * 1024 + ln * 16);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-          const int sr = k * 8 + (ln >> 3), tr = i * 128 + wt * 32 + sr;
-          const int at = tr < left ? tr : left;  // (rows behind the last one hold its numbers)
-          u32x4* to = (u32x4*)(out + (int64_t)at * p.o_st + j * 256 + (((ln & 7) ^ ((sr >> 1) & 7)) << 4));
-          if (p.stream_out) __builtin_nontemporal_store(row[k], to);
-          else *to = row[k];
-        }
-      }
+    for (int i = 0; i < 2; i++) up_store<kKeysF16, true>(p, acc[1][i], st, out + 256, i * 128 + wt * 32, left);
     if (!more) break;
     stored = true;
     idx = nidx;
     tile = next;
     w_base = w_next;
+  }
+  MLA_WAIT_VMCNT(0);
+}
+
+// The same where tiles of 256 tokens are too few for the CUs: a tile is one quadrant, 128 tokens x the keys or the values of a head, and
+// a wavefront owns its 32 x 64 of it.  A stage of the contraction is 32 KiB (tokens, W), four of them are in LDS, and the stages of a
+// workgroup's tiles follow each other: one barrier per stage, behind the wait for its own four copies a wavefront asks for the stage
+// three ahead, into the buffer that everyone has done with.  What bounds it is a tile's chain of start, eight stages and end.
+// us per launch, tiles of 256 tokens / this, rounds of 256 workgroups in parentheses: 100 x 16 15.0 / 7.5 (0.1), 475 x 64 17.5 / 13.6 (2),
+// 208 x 128 17.5 / 13.3 (2), 256 x 64 16.4 / 10.0 (1), 1017 x 32 18.1 / 14.1 (2), 700 x 64 18.8 / 18.1 (3), 384 x 128 20.6 / 18.7 (3),
+// 1500 x 32 20.2 / 20.4 (3), but 1017 x 64 21.9 / 24.5 (4), 512 x 128 21.9 / 27.5 (4): three rounds at most.
+constexpr int kUpSmallTok = 128;
+constexpr int64_t kUpSmallMost = 768;
+constexpr int kUpSmallStage = 2 * kUpUnit;       // 32768
+
+template <bool kKeysF16>
+__global__ __launch_bounds__(512, 2) void mla_kv_up_small_kernel(const KvUpParams p) {
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int wn = wave & 1, wt = wave >> 1;
+  const uint32_t lds0 = lds_addr_of(lds);
+  const int total = p.m_tiles * p.heads * 2;
+  const int xcd = blockIdx.x & 7, slots = gridDim.x >> 3;
+  const int last = (int)((int64_t)total * (xcd + 1) / 8);
+  int idx = (int)((int64_t)total * xcd / 8) + (blockIdx.x >> 3);
+  if (blockIdx.x == 0 && (int)threadIdx.x < p.clear_words) p.clear[threadIdx.x] = 0u;
+  if (idx >= last) {
+    if (p.pe != nullptr) up_rope_rows(p);
+    return;
+  }
+
+  // where the copies of a tile come from: the token tile fastest, then keys and values, then the head
+  const uint32_t cdst = lds0 + wave * 2048;
+  const uint32_t crow = wave * 16 + (lane >> 3);
+  const uint32_t cgr0 = ((lane & 7) ^ up_swz(lane >> 3)) * 16, cgr1 = ((lane & 7) ^ up_swz(8 + (lane >> 3))) * 16;
+  const uint32_t xs2 = (uint32_t)p.x_st * 2, ws2 = (uint32_t)p.w_st * 2;
+  const uint32_t w_off0 = __umul24(crow, ws2) + cgr0, w_off1 = __umul24(crow + 8, ws2) + cgr1;
+  struct Small { int m, head, j; };
+  auto tile_of = [&](int i) {
+    const int hj = i / p.m_tiles;
+    return Small{i - hj * p.m_tiles, hj >> 1, hj & 1};
+  };
+  const char *x_base, *w_base;
+  uint32_t x_off0, x_off1;
+  auto copy_from = [&](Small t) {
+    x_base = (const char*)(p.x + (int64_t)t.m * kUpSmallTok * p.x_st);
+    w_base = (const char*)(p.w + (int64_t)(t.head * 2 + t.j) * 128 * p.w_st);
+    const int64_t left64 = p.rows - 1 - (int64_t)t.m * kUpSmallTok;
+    const uint32_t left = left64 < kUpSmallTok ? (uint32_t)left64 : kUpSmallTok;
+    x_off0 = __umul24(crow < left ? crow : left, xs2) + cgr0;
+    x_off1 = __umul24(crow + 8 < left ? crow + 8 : left, xs2) + cgr1;
+  };
+  auto copy = [&](int stage) {                   // of the tile that copy_from named last
+    const uint32_t dst = cdst + (stage & 3) * kUpSmallStage;
+    dma16_sv(w_base + stage * 128, w_off0, dst + kUpUnit);
+    dma16_sv(w_base + stage * 128, w_off1, dst + kUpUnit + 1024);
+    dma16_sv(x_base + stage * 128, x_off0, dst);
+    dma16_sv(x_base + stage * 128, x_off1, dst + 1024);
+  };
+  Small tile = tile_of(idx);
+  copy_from(tile);
+  copy(0);
+  copy(1);
+  copy(2);
+
+  const char* xr[4];
+  const char* wr[4];
+#pragma unroll
+  for (int kk = 0; kk < 4; kk++) {
+    const int koff = (lane & 31) * 128 + (((kk * 2 + (lane >> 5)) ^ up_swz(lane & 15)) << 4);
+    xr[kk] = lds + wt * 4096 + koff;
+    wr[kk] = lds + kUpUnit + wn * 8192 + koff;
+  }
+  bool stored = false;
+  while (true) {
+    const int nidx = idx + slots;
+    const bool more = nidx < last;               // (behind the last tile its own first stages are copied once more, and not read)
+    const Small next = more ? tile_of(nidx) : tile;
+    f32x16 acc[2];
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+      // two stages of four copies are younger, and in a tile's first three stages the four stores of the one before
+      if (stored && s < 3) MLA_WAIT_VMCNT(12);
+      else MLA_WAIT_VMCNT(8);
+      lds_barrier();
+      if (s == 5) copy_from(next);
+      copy((s + 3) & 7);
+      bf16x8 xf[4], wf[2][4];
+#pragma unroll
+      for (int kk = 0; kk < 4; kk++) {
+        xf[kk] = *(const bf16x8*)(xr[kk] + (s & 3) * kUpSmallStage);
+#pragma unroll
+        for (int b = 0; b < 2; b++) wf[b][kk] = *(const bf16x8*)(wr[kk] + (s & 3) * kUpSmallStage + b * 4096);
+      }
+#pragma unroll
+      for (int kk = 0; kk < 4; kk++)
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+          if (s == 0 && kk == 0) {
+            f32x16 zero;
+#pragma unroll
+            for (int r = 0; r < 16; r++) zero[r] = 0.f;
+            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[b][kk], xf[kk], zero, 0, 0, 0);
+          } else {
+            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[b][kk], xf[kk], acc[b], 0, 0, 0);
+          }
+        }
+    }
+    if (p.pe != nullptr && !more) up_rope_rows(p);
+    char* st = lds + kUpStage + wave * 4096;
+    const int64_t left64 = p.rows - 1 - (int64_t)tile.m * kUpSmallTok;
+    const int left = left64 < kUpSmallTok ? (int)left64 : kUpSmallTok;
+    char* out = p.out + (int64_t)tile.m * kUpSmallTok * p.o_st + (int64_t)tile.head * p.o_sh + wn * 128;
+    if (tile.j) up_store<kKeysF16, true>(p, acc, st, out + 256, wt * 32, left);
+    else up_store<kKeysF16, false>(p, acc, st, out, wt * 32, left);
+    if (!more) break;
+    stored = true;
+    idx = nidx;
+    tile = next;
   }
   MLA_WAIT_VMCNT(0);
 }
@@ -328,12 +452,18 @@ extern "C" int mla_kv_up(const void* x, int64_t x_stride, const void* weight, in
   p.pe = (const __bf16*)k_pe; p.pe_st = k_pe_stride;
   p.pe_out = (_Float16*)out_pe; p.pe_ost = out_pe_stride;
   p.clear = (uint32_t*)clear; p.clear_words = clear_words;
-  auto* kern = keys_f16 ? mla_kv_up_kernel<true> : mla_kv_up_kernel<false>;
-  int rc = ensure_dynamic_lds((const void*)mla_kv_up_kernel<true>, kUpLdsB, "mla_kv_up");
-  if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)mla_kv_up_kernel<false>, kUpLdsB, "mla_kv_up");
-  if (rc != MLA_OK) return rc;
+  static constexpr void (*kerns[4])(const KvUpParams) = {mla_kv_up_kernel<false>, mla_kv_up_kernel<true>, mla_kv_up_small_kernel<false>,
+                                                         mla_kv_up_small_kernel<true>};
+  for (int i = 0; i < 4; i++) {
+    const int rc = ensure_dynamic_lds((const void*)kerns[i], kUpLdsB, "mla_kv_up");
+    if (rc != MLA_OK) return rc;
+  }
+  const int64_t quads = (num_rows + kUpSmallTok - 1) / kUpSmallTok * num_heads * 2;
+  const bool small = quads > 0 && quads <= kUpSmallMost;
+  if (small) p.m_tiles = (int32_t)((num_rows + kUpSmallTok - 1) / kUpSmallTok);
+  auto* kern = kerns[(small ? 2 : 0) + (keys_f16 ? 1 : 0)];
   // one workgroup per CU at most; fewer tiles: as many workgroups, in whole rounds of the eight XCDs
-  const int64_t tiles = (int64_t)p.m_tiles * num_heads;
+  const int64_t tiles = small ? quads : (int64_t)p.m_tiles * num_heads;
   const int64_t grid = tiles == 0 ? 8 : tiles < 256 ? (tiles + 7) / 8 * 8 : 256;   // (no rows: only what is to be cleared)
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), kUpLdsB, stream, p);
   return check_launch("mla_kv_up_kernel");
