@@ -312,6 +312,13 @@ int mla_kv_up(const void* x, int64_t x_stride, const void* weight, int64_t w_str
               int32_t keys_f16, void* out, int64_t out_stride_t, int64_t out_stride_h, const void* k_pe, int64_t k_pe_stride,
               void* out_pe, int64_t out_pe_stride, void* clear, int32_t clear_words, mlahip_stream_t stream);
 
+/* The same for two sets of rows in one launch (x, k_pe: num_rows; x1, k_pe1: num_rows1): out and out_pe hold the second set's tokens
+ * behind the first's. */
+int mla_kv_up_two(const void* x, int64_t x_stride, int64_t num_rows, const void* k_pe, int64_t k_pe_stride, const void* x1,
+                  int64_t x1_stride, int64_t num_rows1, const void* k_pe1, int64_t k_pe1_stride, const void* weight, int64_t w_stride,
+                  int32_t num_heads, int32_t keys_f16, void* out, int64_t out_stride_t, int64_t out_stride_h, void* out_pe,
+                  int64_t out_pe_stride, void* clear, int32_t clear_words, mlahip_stream_t stream);
+
 /* ---- non-absorbed varlen attention for prefill -------------------------------------------
  * Replaces the prefill calls of npu_fused_infer_attention_score, attention/backends/mla.py:574-590 (suffix:
  * right-down causal, sparse_mode 3) and :415-431 (context chunk: no mask, softmax_lse_flag): q_nope [T,N,128],

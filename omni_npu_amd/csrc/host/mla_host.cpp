@@ -399,20 +399,28 @@ bool prefill_wants_queue(int64_t tokens, int64_t batch, int64_t max_q_len, int64
          (prefill_blocks(tokens, batch, max_q_len, heads) > kPrefillResident || prefill_long_rows(tokens, batch, heads));
 }
 
-// Keys and values of latent rows [t, 512] (kernels.kv_up): a head's tokens behind each other, a token's key in front of its value; the
-// rope rows as fp16 (keys_f16) or as they are.
-struct KeyRows { Tensor kv, pe16; const void* pe; int64_t t, pe_st; const char* k() const { return (const char*)kv.data_ptr(); } };
-KeyRows kv_up(const void* c, int64_t c_st, const void* pe, int64_t pe_st, int64_t t, const Tensor& w, int64_t n, bool keys_f16,
-              Tensor* clear, Stream st) {
-  KeyRows r{at::empty({n, t, 256}, w.options().dtype(at::kHalf)), Tensor(), pe, t, pe_st};
+// Latent rows [t, 512] and their rope rows
+struct LatentRows { const void *c, *pe; int64_t c_st, pe_st, t; };
+// Their keys and values (kernels.kv_up) and those of the context rows behind them (t = 0: none): a head's tokens behind each other, a
+// token's key in front of its value; the rope rows as fp16 (keys_f16) or as they are.
+struct KeyRows { Tensor kv, pe16; const void* pe; int64_t pe_st; };
+KeyRows kv_up(const LatentRows& own, const LatentRows& ctx, const Tensor& w, int64_t n, bool keys_f16, Tensor* clear, Stream st) {
+  const int64_t t = own.t + ctx.t;
+  KeyRows r{at::empty({n, t, 256}, w.options().dtype(at::kHalf)), Tensor(), own.pe, own.pe_st};
   if (keys_f16) {
     r.pe16 = at::empty({t, kRope}, w.options().dtype(at::kHalf));
     r.pe = r.pe16.data_ptr();
     r.pe_st = kRope;
   }
-  check(mla_kv_up(c, c_st, w.data_ptr(), w.stride(0), t, (int)n, keys_f16 ? 1 : 0, r.kv.data_ptr(), 256, t * 256, keys_f16 ? pe : nullptr,
-                  keys_f16 ? pe_st : 0, keys_f16 ? r.pe16.data_ptr() : nullptr, keys_f16 ? kRope : 0, clear ? clear->data_ptr() : nullptr,
-                  clear ? (int)clear->numel() : 0, st), "mla_kv_up");
+  void *pe_out = keys_f16 ? r.pe16.data_ptr() : nullptr, *words = clear ? clear->data_ptr() : nullptr;
+  const int count = clear ? (int)clear->numel() : 0;
+  const void* pe = keys_f16 ? own.pe : nullptr;
+  if (ctx.t > 0)
+    check(mla_kv_up_two(own.c, own.c_st, own.t, pe, own.pe_st, ctx.c, ctx.c_st, ctx.t, keys_f16 ? ctx.pe : nullptr, ctx.pe_st, w.data_ptr(),
+                        w.stride(0), (int)n, keys_f16 ? 1 : 0, r.kv.data_ptr(), 256, t * 256, pe_out, kRope, words, count, st), "mla_kv_up_two");
+  else
+    check(mla_kv_up(own.c, own.c_st, w.data_ptr(), w.stride(0), t, (int)n, keys_f16 ? 1 : 0, r.kv.data_ptr(), 256, t * 256, pe, own.pe_st, pe_out,
+                    kRope, words, count, st), "mla_kv_up");
   return r;
 }
 
@@ -453,10 +461,9 @@ bool prefill(const Tensor& q, const Tensor& kv_c, const Tensor& k_pe, int64_t fi
   const int64_t q_st = q.stride(0), q_sh = q.stride(1);
   const char* q0 = (const char*)q.data_ptr() + 2 * first * q_st;
   void* o0 = (char*)out.data_ptr() + 2 * first * out.stride(0);
-  const KeyRows own = kv_up((const char*)kv_c.data_ptr() + 2 * first * kv_c.stride(0), kv_c.stride(0),
-                            (const char*)k_pe.data_ptr() + 2 * first * k_pe.stride(0), k_pe.stride(0), t, w, n, keys_f16,
-                            queue.defined() ? &queue : nullptr, st);
-  KeyRows ctx{Tensor(), Tensor(), nullptr, 0, 0};
+  const LatentRows own{(const char*)kv_c.data_ptr() + 2 * first * kv_c.stride(0), (const char*)k_pe.data_ptr() + 2 * first * k_pe.stride(0),
+                       kv_c.stride(0), k_pe.stride(0), t};
+  LatentRows ctx{nullptr, nullptr, 0, 0, 0};
   if (ctx_toks > 0) {
     const Tensor& rows = *ctx_rows;
     const int32_t *bt = (const int32_t*)block_table->data_ptr(), *cu = (const int32_t*)cu_ctx->data_ptr(), *at0 = (const int32_t*)starts->data_ptr();
@@ -467,8 +474,11 @@ bool prefill(const Tensor& q, const Tensor& kv_c, const Tensor& k_pe, int64_t fi
     else
       check(mla_gather_paged_fp8(c.nope->data_ptr(), c.n_sp, c.n_sr, c.pages, (int)c.page, rows.data_ptr(), rows.stride(0), rows.size(0), bt,
                                  block_table->stride(0), (int)block_table->size(1), cu, at0, (int)batch, ctx_toks, st), "mla_gather_paged_fp8");
-    ctx = kv_up(rows.data_ptr(), rows.stride(0), (const char*)rows.data_ptr() + 2 * kNope, rows.stride(0), ctx_toks, w, n, true, nullptr, st);
+    ctx = {rows.data_ptr(), (const char*)rows.data_ptr() + 2 * kNope, rows.stride(0), rows.stride(0), ctx_toks};
   }
+  const KeyRows keys = kv_up(own, ctx, w, n, keys_f16, queue.defined() ? &queue : nullptr, st);
+  const char *k0 = (const char*)keys.kv.data_ptr(), *v0 = k0 + 2 * 128;
+  const int64_t k_sh = (t + ctx_toks) * 256;
   // what kernels.prefill_varlen chooses
   const int64_t seen = t + ctx_toks - t / 2;
   const bool whole_rows = keys_f16 && !pick;
@@ -477,18 +487,17 @@ bool prefill(const Tensor& q, const Tensor& kv_c, const Tensor& k_pe, int64_t fi
   const int pieces = whole_rows && !qu ? prefill_pieces(t, batch, max_q_len, n, seen) : 1;
   const int type = (keys_f16 ? 16 : 32) + (rows64 ? 64 : 0);   // MLA_PREFILL_KV_F16, _V_F16, _LONG
   const int32_t *cu = (const int32_t*)cu_q.data_ptr(), *cu1 = ctx_toks > 0 ? (const int32_t*)cu_ctx->data_ptr() : nullptr;
-  const char* k1 = ctx_toks > 0 ? ctx.k() : nullptr;
-  const char* v1 = k1 ? k1 + 2 * 128 : nullptr;
-  const int64_t sh1 = ctx_toks * 256;
+  const char* k1 = ctx_toks > 0 ? k0 + 2 * t * 256 : nullptr;
+  const char *v1 = k1 ? k1 + 2 * 128 : nullptr, *pe1 = k1 ? (const char*)keys.pe + 2 * t * keys.pe_st : nullptr;
   if (pieces > 1) {
     Tensor parts = at::empty({pieces * t * n * 129}, q.options().dtype(at::kFloat));
-    check(mla_prefill_varlen_split(q0, q_st, q_sh, q0 + 2 * 128, q_st, q_sh, own.k(), 256, t * 256, own.pe, own.pe_st, own.k() + 2 * 128, 256,
-                                   t * 256, cu, cu, k1, sh1, ctx.pe, v1, sh1, cu1, (int)batch, (int)n, (int)max_q_len, 1, (float)scale, o0,
-                                   out.stride(0), kVDim, type, nullptr, pieces, t, (float*)parts.data_ptr(), st), "mla_prefill_varlen_split");
+    check(mla_prefill_varlen_split(q0, q_st, q_sh, q0 + 2 * 128, q_st, q_sh, k0, 256, k_sh, keys.pe, keys.pe_st, v0, 256, k_sh, cu, cu, k1, k_sh,
+                                   pe1, v1, k_sh, cu1, (int)batch, (int)n, (int)max_q_len, 1, (float)scale, o0, out.stride(0), kVDim, type,
+                                   nullptr, pieces, t, (float*)parts.data_ptr(), st), "mla_prefill_varlen_split");
     return true;
   }
-  check(mla_prefill_varlen_queued(q0, q_st, q_sh, q0 + 2 * 128, q_st, q_sh, own.k(), 256, t * 256, own.pe, own.pe_st, own.k() + 2 * 128, 256,
-                                  t * 256, cu, cu, k1, sh1, ctx.pe, v1, sh1, cu1, (int)batch, (int)n, (int)max_q_len, 1, 0, (float)scale,
+  check(mla_prefill_varlen_queued(q0, q_st, q_sh, q0 + 2 * 128, q_st, q_sh, k0, 256, k_sh, keys.pe, keys.pe_st, v0, 256, k_sh, cu, cu, k1, k_sh,
+                                  pe1, v1, k_sh, cu1, (int)batch, (int)n, (int)max_q_len, 1, 0, (float)scale,
                                   pick ? (const uint32_t*)pick->data_ptr() : nullptr, pick ? pick->stride(0) : 0, pick ? (int)pick->size(1) : 0, o0,
                                   out.stride(0), kVDim, type, nullptr, nullptr, 0, 0, nullptr, qu, st), "mla_prefill_varlen_queued");
   return true;

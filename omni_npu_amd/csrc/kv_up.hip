@@ -48,8 +48,11 @@ struct KvUpParams {
   char* out; int64_t o_st, o_sh;                 // bytes
   int64_t rows;
   int32_t heads, m_tiles;
+  // a second set of rows (or none: m_first = m_tiles), whose results follow the first's; token tiles from m_first on are its
+  const __bf16* x1; int64_t x1_st, rows1;
+  int32_t m_first;
   int32_t stream_out;                            // results are marked non-temporal
-  const __bf16* pe; int64_t pe_st;               // rope rows that leave as fp16 (null: none)
+  const __bf16 *pe, *pe1; int64_t pe_st, pe1_st; // rope rows of both sets that leave as fp16 (null: none)
   _Float16* pe_out; int64_t pe_ost;
   uint32_t* clear; int32_t clear_words;          // words to set to zero for the launch behind this one (null: none)
 };
@@ -75,9 +78,20 @@ __device__ __forceinline__ UpTile up_tile(const KvUpParams& p, int idx) {
   return {g * kUpGroup + rem - head * mg, head};
 }
 
+// Token tile m of kTok: its rows, and the last one of them that exists (counted from the tile's first; kTok: all do)
+struct UpRows { const char* x; uint32_t st2; int left; int64_t first; };
+template <int kTok>
+__device__ __forceinline__ UpRows up_rows(const KvUpParams& p, int m) {
+  const bool second = m >= p.m_first;
+  const uint32_t i = (uint32_t)(second ? m - p.m_first : m), st2 = (uint32_t)(second ? p.x1_st : p.x_st) * 2;
+  const int64_t at = (int64_t)i * kTok, left = (second ? p.rows1 : p.rows) - 1 - at;
+  return {(const char*)(second ? p.x1 : p.x) + (uint64_t)i * (st2 * kTok), st2, left < kTok ? (int)left : kTok, second ? p.rows + at : at};
+}
+
 __device__ __forceinline__ void up_rope_rows(const KvUpParams& p) {
-  for (int64_t i = (int64_t)blockIdx.x * 512 + threadIdx.x; i < p.rows * 8; i += (int64_t)gridDim.x * 512) {
-    const bf16x8 v = *(const bf16x8*)(p.pe + (i >> 3) * p.pe_st + (i & 7) * 8);
+  for (int64_t i = (int64_t)blockIdx.x * 512 + threadIdx.x; i < (p.rows + p.rows1) * 8; i += (int64_t)gridDim.x * 512) {
+    const int64_t r = i >> 3;
+    const bf16x8 v = *(const bf16x8*)((r < p.rows ? p.pe + r * p.pe_st : p.pe1 + (r - p.rows) * p.pe1_st) + (i & 7) * 8);
     f16x8 o;
 #pragma unroll
     for (int e = 0; e < 8; e++) o[e] = (_Float16)(float)v[e];
@@ -85,11 +99,11 @@ __device__ __forceinline__ void up_rope_rows(const KvUpParams& p) {
   }
 }
 
-// A wavefront's 32 tokens x 64 columns (of the keys, or kValues: of the values) through its own 4 KiB at st to `out`, the columns of its
+// A wavefront's (lane ln) 32 tokens x 64 columns (of the keys, or kValues: of the values) through its own 4 KiB at st to `out`, the columns of its
 // tile's first token; at_row: its first token in the tile, whose last one is `left` (the rows behind hold its numbers).
 template <bool kKeysF16, bool kValues>
-__device__ __forceinline__ void up_store(const KvUpParams& p, f32x16 (&acc)[2], char* st, char* out, int at_row, int left) {
-  const int ln = up_lane(), h32 = ln & 31, half = ln >> 5;
+__device__ __forceinline__ void up_store(const KvUpParams& p, f32x16 (&acc)[2], char* st, char* out, int at_row, int left, int ln) {
+  const int h32 = ln & 31, half = ln >> 5;
   if constexpr (!kKeysF16 && kValues) {
     float big = 0.f;
 #pragma unroll
@@ -163,13 +177,14 @@ __global__ __launch_bounds__(512, 2) void mla_kv_up_kernel(const KvUpParams p) {
   const uint32_t cdst = lds0 + wave * 2048;
   const uint32_t crow = wave * 16 + (lane >> 3);
   const uint32_t cgr0 = ((lane & 7) ^ up_swz(lane >> 3)) * 16, cgr1 = ((lane & 7) ^ up_swz(8 + (lane >> 3))) * 16;
-  const uint32_t xs2 = (uint32_t)p.x_st * 2, ws2 = (uint32_t)p.w_st * 2;
+  const uint32_t ws2 = (uint32_t)p.w_st * 2;
   const char* x_base;
-  uint32_t x_left;                               // last row that exists, counted from the tile's first
+  uint32_t xs2, x_left;                          // last row that exists, counted from the tile's first
   auto copy_from = [&](UpTile t) {
-    x_base = (const char*)(p.x + (int64_t)t.m * kUpTok * p.x_st);
-    const int64_t left = p.rows - 1 - (int64_t)t.m * kUpTok;
-    x_left = left < kUpTok ? (uint32_t)left : kUpTok;
+    const UpRows r = up_rows<kUpTok>(p, t.m);
+    x_base = r.x;
+    xs2 = r.st2;
+    x_left = (uint32_t)r.left;
   };
   auto copy_x = [&](int stage, int i) {          // stage: of the tile that x_base names
     const uint32_t dst = cdst + (stage & 1) * kUpBuf + i * kUpUnit;
@@ -288,13 +303,13 @@ __global__ __launch_bounds__(512, 2) void mla_kv_up_kernel(const KvUpParams p) {
 
     // results: a quadrant at a time
     char* st = lds + kUpStage + wave * 4096;
-    const int64_t left64 = p.rows - 1 - (int64_t)tile.m * kUpTok;
-    const int left = left64 < kUpTok ? (int)left64 : kUpTok;
-    char* out = p.out + (int64_t)tile.m * kUpTok * p.o_st + (int64_t)tile.head * p.o_sh + wn * 128;
+    const UpRows r = up_rows<kUpTok>(p, tile.m);
+    const int ln = up_lane();
+    char* out = p.out + r.first * p.o_st + (int64_t)tile.head * p.o_sh + wn * 128;
 #pragma unroll
-    for (int i = 0; i < 2; i++) up_store<kKeysF16, false>(p, acc[0][i], st, out, i * 128 + wt * 32, left);
+    for (int i = 0; i < 2; i++) up_store<kKeysF16, false>(p, acc[0][i], st, out, i * 128 + wt * 32, r.left, ln);
 #pragma unroll
-    for (int i = 0; i < 2; i++) up_store<kKeysF16, true>(p, acc[1][i], st, out + 256, i * 128 + wt * 32, left);
+    for (int i = 0; i < 2; i++) up_store<kKeysF16, true>(p, acc[1][i], st, out + 256, i * 128 + wt * 32, r.left, ln);
     if (!more) break;
     stored = true;
     idx = nidx;
@@ -336,7 +351,7 @@ __global__ __launch_bounds__(512, 2) void mla_kv_up_small_kernel(const KvUpParam
   const uint32_t cdst = lds0 + wave * 2048;
   const uint32_t crow = wave * 16 + (lane >> 3);
   const uint32_t cgr0 = ((lane & 7) ^ up_swz(lane >> 3)) * 16, cgr1 = ((lane & 7) ^ up_swz(8 + (lane >> 3))) * 16;
-  const uint32_t xs2 = (uint32_t)p.x_st * 2, ws2 = (uint32_t)p.w_st * 2;
+  const uint32_t ws2 = (uint32_t)p.w_st * 2;
   const uint32_t w_off0 = __umul24(crow, ws2) + cgr0, w_off1 = __umul24(crow + 8, ws2) + cgr1;
   struct Small { int m, head, j; };
   auto tile_of = [&](int i) {
@@ -346,12 +361,12 @@ __global__ __launch_bounds__(512, 2) void mla_kv_up_small_kernel(const KvUpParam
   const char *x_base, *w_base;
   uint32_t x_off0, x_off1;
   auto copy_from = [&](Small t) {
-    x_base = (const char*)(p.x + (int64_t)t.m * kUpSmallTok * p.x_st);
+    const UpRows r = up_rows<kUpSmallTok>(p, t.m);
+    const uint32_t left = (uint32_t)r.left;
+    x_base = r.x;
     w_base = (const char*)(p.w + (int64_t)(t.head * 2 + t.j) * 128 * p.w_st);
-    const int64_t left64 = p.rows - 1 - (int64_t)t.m * kUpSmallTok;
-    const uint32_t left = left64 < kUpSmallTok ? (uint32_t)left64 : kUpSmallTok;
-    x_off0 = __umul24(crow < left ? crow : left, xs2) + cgr0;
-    x_off1 = __umul24(crow + 8 < left ? crow + 8 : left, xs2) + cgr1;
+    x_off0 = __umul24(crow < left ? crow : left, r.st2) + cgr0;
+    x_off1 = __umul24(crow + 8 < left ? crow + 8 : left, r.st2) + cgr1;
   };
   auto copy = [&](int stage) {                   // of the tile that copy_from named last
     const uint32_t dst = cdst + (stage & 3) * kUpSmallStage;
@@ -411,11 +426,11 @@ __global__ __launch_bounds__(512, 2) void mla_kv_up_small_kernel(const KvUpParam
     }
     if (p.pe != nullptr && !more) up_rope_rows(p);
     char* st = lds + kUpStage + wave * 4096;
-    const int64_t left64 = p.rows - 1 - (int64_t)tile.m * kUpSmallTok;
-    const int left = left64 < kUpSmallTok ? (int)left64 : kUpSmallTok;
-    char* out = p.out + (int64_t)tile.m * kUpSmallTok * p.o_st + (int64_t)tile.head * p.o_sh + wn * 128;
-    if (tile.j) up_store<kKeysF16, true>(p, acc, st, out + 256, wt * 32, left);
-    else up_store<kKeysF16, false>(p, acc, st, out, wt * 32, left);
+    const UpRows r = up_rows<kUpSmallTok>(p, tile.m);
+    const int ln = up_lane();
+    char* out = p.out + r.first * p.o_st + (int64_t)tile.head * p.o_sh + wn * 128;
+    if (tile.j) up_store<kKeysF16, true>(p, acc, st, out + 256, wt * 32, r.left, ln);
+    else up_store<kKeysF16, false>(p, acc, st, out, wt * 32, r.left, ln);
     if (!more) break;
     stored = true;
     idx = nidx;
@@ -427,44 +442,69 @@ __global__ __launch_bounds__(512, 2) void mla_kv_up_small_kernel(const KvUpParam
 }  // namespace mlahip
 using namespace mlahip;
 
-extern "C" int mla_kv_up(const void* x, int64_t x_stride, const void* weight, int64_t w_stride, int64_t num_rows, int32_t num_heads,
-                         int32_t keys_f16, void* out, int64_t out_stride_t, int64_t out_stride_h, const void* k_pe,
-                         int64_t k_pe_stride, void* out_pe, int64_t out_pe_stride, void* clear, int32_t clear_words,
-                         hipStream_t stream) {
-  MLA_REQUIRE(x && weight && out, MLA_ERR_NULL, "mla_kv_up: null pointer argument");
-  MLA_REQUIRE((k_pe == nullptr) == (out_pe == nullptr), MLA_ERR_NULL, "mla_kv_up: rope rows and their result go together");
-  MLA_REQUIRE(num_rows >= 0 && num_heads >= 1 && num_heads <= 65535 && (num_rows + kUpTok - 1) / kUpTok * num_heads < (1 << 30),
-              MLA_ERR_SHAPE, "mla_kv_up: num_rows=%lld num_heads=%d", (long long)num_rows, num_heads);
-  MLA_REQUIRE(x_stride >= 0 && w_stride >= 0 && x_stride <= (1 << 20) && w_stride <= (1 << 20) && x_stride % 8 == 0 &&
-                  w_stride % 8 == 0 && out_stride_t % 8 == 0 && out_stride_h % 8 == 0 &&
-                  ((uintptr_t)x | (uintptr_t)weight | (uintptr_t)out) % 16 == 0 &&
-                  (!k_pe || (((uintptr_t)k_pe | (uintptr_t)out_pe) % 16 == 0 && k_pe_stride % 8 == 0 && out_pe_stride % 8 == 0)),
-              MLA_ERR_SHAPE, "mla_kv_up: rows must be 16-byte aligned, at most 2^20 elements apart");
+static int kv_up_impl(const char* what, const void* x, int64_t x_stride, int64_t num_rows, const void* k_pe, int64_t k_pe_stride,
+                      const void* x1, int64_t x1_stride, int64_t num_rows1, const void* k_pe1, int64_t k_pe1_stride, const void* weight,
+                      int64_t w_stride, int32_t num_heads, int32_t keys_f16, void* out, int64_t out_stride_t, int64_t out_stride_h,
+                      void* out_pe, int64_t out_pe_stride, void* clear, int32_t clear_words, hipStream_t stream) {
+  MLA_REQUIRE(x && weight && out && (x1 || num_rows1 == 0), MLA_ERR_NULL, "%s: null pointer argument", what);
+  MLA_REQUIRE((k_pe == nullptr) == (out_pe == nullptr) && (num_rows1 == 0 || (k_pe == nullptr) == (k_pe1 == nullptr)), MLA_ERR_NULL,
+              "%s: rope rows and their result go together", what);
+  MLA_REQUIRE(num_rows >= 0 && num_rows1 >= 0 && num_heads >= 1 && num_heads <= 65535 &&
+                  ((num_rows + kUpTok - 1) / kUpTok + (num_rows1 + kUpTok - 1) / kUpTok) * num_heads < (1 << 30),
+              MLA_ERR_SHAPE, "%s: num_rows=%lld, %lld num_heads=%d", what, (long long)num_rows, (long long)num_rows1, num_heads);
+  MLA_REQUIRE(x_stride >= 0 && x1_stride >= 0 && w_stride >= 0 && x_stride <= (1 << 20) && x1_stride <= (1 << 20) && w_stride <= (1 << 20) &&
+                  x_stride % 8 == 0 && x1_stride % 8 == 0 && w_stride % 8 == 0 && out_stride_t % 8 == 0 && out_stride_h % 8 == 0 &&
+                  ((uintptr_t)x | (uintptr_t)x1 | (uintptr_t)weight | (uintptr_t)out) % 16 == 0 &&
+                  (!k_pe || (((uintptr_t)k_pe | (uintptr_t)k_pe1 | (uintptr_t)out_pe) % 16 == 0 && k_pe_stride % 8 == 0 &&
+                             k_pe1_stride % 8 == 0 && out_pe_stride % 8 == 0)),
+              MLA_ERR_SHAPE, "%s: rows must be 16-byte aligned, at most 2^20 elements apart", what);
   MLA_REQUIRE(clear_words >= 0 && clear_words <= 512 && (clear || clear_words == 0) && (uintptr_t)clear % 4 == 0, MLA_ERR_SHAPE,
-              "mla_kv_up: up to 512 words to clear (got %d)", clear_words);
-  if (num_rows == 0 && clear_words == 0) return MLA_OK;
+              "%s: up to 512 words to clear (got %d)", what, clear_words);
+  if (num_rows + num_rows1 == 0 && clear_words == 0) return MLA_OK;
   KvUpParams p;
   p.x = (const __bf16*)x; p.x_st = x_stride;
   p.w = (const __bf16*)weight; p.w_st = w_stride;
   p.out = (char*)out; p.o_st = out_stride_t * 2; p.o_sh = out_stride_h * 2;
-  p.rows = num_rows; p.heads = num_heads; p.m_tiles = (int32_t)((num_rows + kUpTok - 1) / kUpTok);
-  p.stream_out = (int64_t)num_rows * num_heads * 512 >= kUpStreamBytes;
-  p.pe = (const __bf16*)k_pe; p.pe_st = k_pe_stride;
+  p.rows = num_rows; p.heads = num_heads;
+  p.x1 = (const __bf16*)x1; p.x1_st = x1_stride; p.rows1 = num_rows1;
+  p.stream_out = (num_rows + num_rows1) * num_heads * 512 >= kUpStreamBytes;
+  p.pe = (const __bf16*)k_pe; p.pe_st = k_pe_stride; p.pe1 = (const __bf16*)k_pe1; p.pe1_st = k_pe1_stride;
   p.pe_out = (_Float16*)out_pe; p.pe_ost = out_pe_stride;
   p.clear = (uint32_t*)clear; p.clear_words = clear_words;
   static constexpr void (*kerns[4])(const KvUpParams) = {mla_kv_up_kernel<false>, mla_kv_up_kernel<true>, mla_kv_up_small_kernel<false>,
                                                          mla_kv_up_small_kernel<true>};
   for (int i = 0; i < 4; i++) {
-    const int rc = ensure_dynamic_lds((const void*)kerns[i], kUpLdsB, "mla_kv_up");
+    const int rc = ensure_dynamic_lds((const void*)kerns[i], kUpLdsB, what);
     if (rc != MLA_OK) return rc;
   }
-  const int64_t quads = (num_rows + kUpSmallTok - 1) / kUpSmallTok * num_heads * 2;
-  const bool small = quads > 0 && quads <= kUpSmallMost;
-  if (small) p.m_tiles = (int32_t)((num_rows + kUpSmallTok - 1) / kUpSmallTok);
+  const auto tiles_of = [&](int64_t tok) { p.m_first = (int32_t)((num_rows + tok - 1) / tok); return p.m_first + (num_rows1 + tok - 1) / tok; };
+  int64_t tiles = tiles_of(kUpSmallTok) * num_heads * 2;
+  const bool small = tiles > 0 && tiles <= kUpSmallMost;
+  p.m_tiles = (int32_t)tiles_of(small ? kUpSmallTok : kUpTok);
+  if (!small) tiles = (int64_t)p.m_tiles * num_heads;
   auto* kern = kerns[(small ? 2 : 0) + (keys_f16 ? 1 : 0)];
   // one workgroup per CU at most; fewer tiles: as many workgroups, in whole rounds of the eight XCDs
-  const int64_t tiles = small ? quads : (int64_t)p.m_tiles * num_heads;
   const int64_t grid = tiles == 0 ? 8 : tiles < 256 ? (tiles + 7) / 8 * 8 : 256;   // (no rows: only what is to be cleared)
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), kUpLdsB, stream, p);
   return check_launch("mla_kv_up_kernel");
+}
+
+extern "C" int mla_kv_up(const void* x, int64_t x_stride, const void* weight, int64_t w_stride, int64_t num_rows, int32_t num_heads,
+                         int32_t keys_f16, void* out, int64_t out_stride_t, int64_t out_stride_h, const void* k_pe,
+                         int64_t k_pe_stride, void* out_pe, int64_t out_pe_stride, void* clear, int32_t clear_words,
+                         hipStream_t stream) {
+  return kv_up_impl("mla_kv_up", x, x_stride, num_rows, k_pe, k_pe_stride, nullptr, 0, 0, nullptr, 0, weight, w_stride, num_heads, keys_f16, out,
+                    out_stride_t, out_stride_h, out_pe, out_pe_stride, clear, clear_words, stream);
+}
+
+// The same for two sets of rows, the second's results behind the first's: a chunk's own tokens and the cached ones in front of them, whose
+// launches of a handful of tiles took the time of one each.
+extern "C" int mla_kv_up_two(const void* x, int64_t x_stride, int64_t num_rows, const void* k_pe, int64_t k_pe_stride, const void* x1,
+                             int64_t x1_stride, int64_t num_rows1, const void* k_pe1, int64_t k_pe1_stride, const void* weight,
+                             int64_t w_stride, int32_t num_heads, int32_t keys_f16, void* out, int64_t out_stride_t, int64_t out_stride_h,
+                             void* out_pe, int64_t out_pe_stride, void* clear, int32_t clear_words, hipStream_t stream) {
+  MLA_REQUIRE(num_rows >= 1 && num_rows1 >= 1, MLA_ERR_SHAPE, "mla_kv_up_two: two sets of rows (got %lld and %lld)", (long long)num_rows,
+              (long long)num_rows1);
+  return kv_up_impl("mla_kv_up_two", x, x_stride, num_rows, k_pe, k_pe_stride, x1, x1_stride, num_rows1, k_pe1, k_pe1_stride, weight, w_stride,
+                    num_heads, keys_f16, out, out_stride_t, out_stride_h, out_pe, out_pe_stride, clear, clear_words, stream);
 }

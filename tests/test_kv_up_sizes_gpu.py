@@ -3,7 +3,7 @@ one to three quadrants behind each other, idle ones, and what the launch does on
 import pytest
 import torch
 
-from omni_npu_amd import kernels as K
+from omni_npu_amd import _lib, kernels as K
 from tests.test_kv_up_gpu import _close, _inputs
 
 pytestmark = pytest.mark.gpu
@@ -33,3 +33,21 @@ def test_values_beyond_fp16_beside_bf16_keys_are_clamped(dev, n):
     ref = (x.float() @ w.float().t()).view(40, n, 256)
     big = ref[..., 128:].abs() > 70000
     assert bool(big.any()) and bool((v[big].float().abs() == 65504).all()) and bool(k.isfinite().all())
+
+
+@pytest.mark.parametrize("t0,t1,n", [(1, 1, 1), (100, 300, 16), (129, 128, 3), (257, 700, 64), (1017, 3072, 64), (2, 70000, 2)])
+@pytest.mark.parametrize("keys_f16", [True, False])
+def test_two_sets_of_rows_in_one_launch(dev, t0, t1, n, keys_f16):
+    """The bits of a launch for each set, rows of different strides, the second set's results behind the first's."""
+    (x0, w, p0), (x1, _, p1) = _inputs(dev, t0, n, 712, 520, seed=1), _inputs(dev, t1, n, 576, 512, seed=2)
+    kv = torch.empty(n, t0 + t1, 256, dtype=torch.float16, device=dev)
+    pe, clear = torch.empty(t0 + t1, 64, dtype=torch.float16, device=dev), torch.full((256,), 7, dtype=torch.int32, device=dev)
+    rc = _lib.load().mla_kv_up_two(x0.data_ptr(), x0.stride(0), t0, p0.data_ptr(), p0.stride(0), x1.data_ptr(), x1.stride(0), t1, p1.data_ptr(),
+                                   p1.stride(0), w.data_ptr(), w.stride(0), n, int(keys_f16), kv.data_ptr(), 256, (t0 + t1) * 256, pe.data_ptr(),
+                                   64, clear.data_ptr(), 256, torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "mla_kv_up_two")
+    assert not bool(clear.any()) and torch.equal(pe, torch.cat([p0, p1]).half())
+    for x, at in ((x0, 0), (x1, t0)):
+        k, v, _ = K.kv_up(x, w, n, keys_f16)
+        got = kv[:, at:at + len(x)].transpose(0, 1)
+        assert torch.equal(got[..., :128].view(torch.int16), k.view(torch.int16)) and torch.equal(got[..., 128:], v)
