@@ -71,13 +71,9 @@ int launch_splits(int64_t batch, int64_t q_len, int64_t heads, int64_t max_seq_l
   const int64_t by_length = std::max<int64_t>(1, div_up(max_seq_len, 256));
   int64_t splits = std::max<int64_t>(1, std::min({std::max<int64_t>(1, div_up(256, groups)), by_length, (int64_t)256}));
   if (groups * splits * 4 <= 256) splits = std::max(splits, 256 / (4 * groups));
-  return (int)splits;
-}
-// kernels.list_splits
-int list_splits(int64_t tokens, int64_t heads, int64_t k) {
-  const int64_t most = 256 / std::max<int64_t>(1, tokens * div_up(heads, 32));
-  if (most < 8) return launch_splits(tokens, 1, heads, k);
-  const int64_t units = div_up(k, 32) + 8, chunk = div_up(units, most);
+  const int64_t most = 256 / std::max<int64_t>(1, batch * div_up(q_len * heads, 32));
+  if (most < 8 || splits > most) return (int)splits;
+  const int64_t units = div_up(max_seq_len, 32) + 8, chunk = div_up(units, most);
   return (int)div_up(units, chunk + chunk % 2);
 }
 
@@ -261,7 +257,7 @@ bool sparse_decode(const Tensor& q, const Tensor& nope, const Tensor& rope, cons
   if (!layer_ok(q, w_uk, w_uv, out, t, dev) || !cache_of(nope, r, dev, c) || !is_i32(rows, 2, dev) || rows.size(0) < t || !is_i32(counts, 1, dev) || !counts.is_contiguous() || counts.numel() < t)
     return false;
   const int64_t n = q.size(1);
-  const int splits = list_splits(t, n, rows.size(1));
+  const int splits = launch_splits(t, 1, n, rows.size(1));
   const int64_t need = (int64_t)mla_decode_workspace_bytes((int)t, 1, (int)n, splits);
   if (need > kSparseWorkspaceCap) return false;
   NewRows new_rows;
@@ -564,7 +560,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("dsa_select_prompts", &dsa_select_prompts);
   // (what this file has a copy of, for a test to hold against kernels.py)
   m.def("launch_splits", &launch_splits);
-  m.def("list_splits", &list_splits);
   m.def("prefill_long_rows", &prefill_long_rows);
   m.def("prefill_blocks", &prefill_blocks);
   m.def("prefill_pieces", &prefill_pieces);

@@ -491,23 +491,22 @@ def default_num_splits(batch: int, max_q_len: int, num_heads: int, max_seq_len: 
 
 def launch_splits(batch: int, max_q_len: int, num_heads: int, max_seq_len: int, num_cus: int = 256) -> int:
     """The split count the wrappers launch with: default_num_splits, but as many as give every CU a workgroup of 32 query rows
-    where that is more.  (The plan on the device settles the cut: it knows the lengths, and how many partials it takes
-    before finer chunks cost more than they save; workgroups it has no chunk for leave at once.)"""
+    where that is more, and where those leave CUs without one (short contexts, few rows) the shortest chunks that give no CU two: a
+    sequence and its start-up (the plan's units) in chunks of whole passes of two 32-key blocks.  (The plan on the device settles the
+    cut: it knows the lengths, and how many partials it takes before finer chunks cost more than they save; workgroups it has no chunk
+    for leave at once.)  us of split, merge and up-projection, chunks of at least 256 keys / this, requests x heads: row lists of 2048,
+    4 x 64 20.5 / 18.7, 8 x 32 23.1 / 19.7, 12 x 32 24.5 / 20.9, 8 x 64 24.0 / 21.0, 24 x 32 27.6 / 25.5; bf16 cache, 5 x 32 of
+    2300-3300 keys 22.8 / 20.3, 8 x 32 of 500-2000 22.0 / 20.1, 12 x 64 of 400-1000 21.5 / 20.0, 30 x 32 of 300-700 24.7 / 21.6, 2 x 2 x
+    128 of 900-2000 20.9 / 21.5; fp8 cache, 5 x 32 25.7 / 22.2, 24 x 16 of 300-900 23.2 / 19.5, 2 x 16 of 14 000 25.7 / 22.9.  With fewer
+    than eight chunks to a sequence the cut by length is the better one: lists of 2048, 27 x 64 in 8 / 4 splits 33.8 / 36.8."""
     splits = default_num_splits(batch, max_q_len, num_heads, max_seq_len, num_cus)
     groups = max(1, batch * math.ceil(max_q_len * num_heads / 128))
-    return max(splits, num_cus // (4 * groups)) if groups * splits * 4 <= num_cus else splits
-
-
-def list_splits(tokens: int, num_heads: int, k: int, num_cus: int = 256) -> int:
-    """The split count of the sparse decode over lists of ``k`` rows.  Few tokens run in groups of 32 query rows, whose workgroups walk
-    passes of two 32-key blocks each: the list and its start-up (the plan's units) are cut into the shortest chunks of whole passes
-    that give no CU two of them.  us of split, merge and up-projection, launch_splits / this, tokens x heads with k = 2048: 4 x 64
-    20.5 / 18.7, 8 x 32 23.1 / 19.7, 12 x 32 24.5 / 20.9, 8 x 64 24.0 / 21.0, 4 x 128 22.0 / 20.8, 24 x 32 27.6 / 25.5; 16 x 16 with
-    k = 1000 19.9 / 15.6.  With fewer than eight chunks to a token the cut by length is the better one: 27 x 64 in 8 / 4 splits 33.8 / 36.8."""
-    most = num_cus // max(1, tokens * math.ceil(num_heads / 32))
-    if most < 8:
-        return launch_splits(tokens, 1, num_heads, k, num_cus)
-    units = math.ceil(k / 32) + 8
+    if groups * splits * 4 <= num_cus:
+        splits = max(splits, num_cus // (4 * groups))
+    most = num_cus // max(1, batch * math.ceil(max_q_len * num_heads / 32))
+    if most < 8 or splits > most:
+        return splits
+    units = math.ceil(max_seq_len / 32) + 8
     chunk = math.ceil(units / most)
     return math.ceil(units / (chunk + chunk % 2))
 
@@ -875,7 +874,7 @@ def sparse_decode(q_nope: torch.Tensor, q_rope: torch.Tensor, nope_cache: torch.
             _lib.check(rc, "dsa_sparse_decode_heads_bf16")
         return out
     if num_splits is None:
-        num_splits = list_splits(t, n, rows.shape[1])
+        num_splits = launch_splits(t, 1, n, rows.shape[1])
     per_token = lib.mla_decode_workspace_bytes(1, 1, n, num_splits)
     cap = workspace.numel() * workspace.element_size() if workspace is not None else SPARSE_WORKSPACE_CAP
     step = max(1, min(t, cap // max(per_token, 1), 32768))

@@ -1,0 +1,19 @@
+"""The split count of a decode launch (kernels.launch_splits): few rows and short contexts are cut into whole passes."""
+import math
+
+from omni_npu_amd import kernels as K
+
+
+def test_chunks_are_whole_passes_where_cus_would_stand_idle_and_as_long_as_before_elsewhere():
+    for batch in [*range(1, 70), 255, 256, 257, 1000]:
+        for q_len, heads in ((1, 1), (1, 16), (2, 16), (1, 33), (1, 64), (1, 128), (2, 128)):
+            groups = batch * math.ceil(q_len * heads / 32)
+            for length in (1, 31, 32, 33, 512, 1000, 2048, 4096, 16384, 131072):
+                s, base = K.launch_splits(batch, q_len, heads, length), K.default_num_splits(batch, q_len, heads, length)
+                assert s >= 1
+                if groups > 32 or base * groups > 256:
+                    assert base <= s <= max(base, 256 // (4 * batch * math.ceil(q_len * heads / 128)))
+                    continue
+                assert s * groups <= 256                       # no CU has two of them
+                units = math.ceil(length / 32) + 8
+                assert s == math.ceil(units / (2 * math.ceil(math.ceil(units / (256 // groups)) / 2)))
