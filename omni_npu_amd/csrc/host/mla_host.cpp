@@ -32,8 +32,8 @@ using at::Tensor;
 using OptTensor = std::optional<Tensor>;
 
 constexpr int64_t kNope = 512, kRope = 64, kPage = 128, kFp8Row = 656, kVDim = 128;
-constexpr int64_t kAbsorbMaxTokens = 256;   // kernels.ABSORB_MAX_TOKENS
-constexpr int64_t kVupMaxTokens = 256;      // kernels.VUP_MAX_TOKENS: beyond, a separate merge and the library GEMM
+constexpr int64_t kAbsorbMaxTokens = 1024;   // kernels.ABSORB_MAX_TOKENS
+constexpr int64_t kVupMaxTokens = 1024;      // kernels.VUP_MAX_TOKENS: beyond, a separate merge and the library GEMM
 constexpr int64_t kSparseWorkspaceCap = 256 << 20;   // kernels.SPARSE_WORKSPACE_CAP
 
 void check(int rc, const char* what) {

@@ -360,8 +360,10 @@ def kv_up(kv_c: torch.Tensor, weight: torch.Tensor, num_heads: int, keys_f16: bo
     return k_nope if keys_f16 else k_nope.view(torch.bfloat16), kv[..., 128:], pe16
 
 
-# Tokens up to which the queries of a step are absorbed by this library's kernel; beyond, the work is a plain GEMM
-ABSORB_MAX_TOKENS = 256
+# Tokens up to which the queries of a step are absorbed by this library's kernel; beyond, the work is a plain GEMM.  us, library / this,
+# tokens x heads: 512 x 16 24.9 / 13.1, 512 x 128 34.2 / 26.3, 1024 x 64 29.3 / 26.2, 1024 x 128 52.9 / 45.8, 2048 x 128 105.4 / 105.1.
+# (The native side keeps the absorbed queries in scratch memory, 134 MB for 1024 tokens of 128 heads.)
+ABSORB_MAX_TOKENS = 1024
 
 
 def absorb(q_nope: torch.Tensor, w_uk: torch.Tensor) -> torch.Tensor:
@@ -522,9 +524,10 @@ def _vup_out(out: torch.Tensor, w_uv: torch.Tensor, t: int, n: int) -> torch.Ten
     return o3
 
 
-# Past this many query tokens a workgroup of the fused merge + up-projection walks through many passes of 16 tokens one after
-# the other, while the separate merge keeps every row in flight (measured break-even at 128 heads: 256 tokens)
-VUP_MAX_TOKENS = 256
+# Up to this many query tokens the merge is fused with the up-projection; beyond, a separate merge and the library's batched product.
+# us of split, merge and up-projection, separate / fused, tokens x heads: 512 x 16 53.2 / 38.5, 512 x 128 138 / 122, 1024 x 64 152 / 136,
+# 1024 x 128 285 / 254, 2048 x 128 595 / 532.  The fused form is the faster one there too; what ends here is a decode step.
+VUP_MAX_TOKENS = 1024
 
 
 def _reduce_vup(lib, ws_args, seq_lens, qsl, b, q_len, n, num_splits, t, w_uv, o3, st, fp8: bool = False) -> None:
