@@ -573,6 +573,8 @@ __global__ __launch_bounds__(kShortThreads, 4) void dsa_topk_short_kernel(const 
 //   gather  every slice adds the histograms up, finds the boundary bin, counts its sure picks per wavefront and
 //           appends its boundary-bin keys to the token's candidate list;
 //   write   every slice finds the exact threshold among the candidates and writes its picks at their final places.
+// A row of one slice is done by the first launch, whose workgroup has all of it (the others leave at once): us of the selection, 1 x 8000
+// keys 19.0 -> 15.6, 8 x 2000-3400 18.4 -> 14.5, 32 x 2500-8000 20.3 -> 16.4, and of 32 x 1000-1300, which take all their keys, 9.2 -> 8.7.
 // A launch costs little more than its chain of dependent memory round trips (more than a microsecond each), so every
 // kernel asks for all the global data it will need - its slice of the row included - before it looks at any of it.
 constexpr int kMwWaves = kTopkThreads / 64;                // 16
@@ -647,16 +649,99 @@ __device__ __forceinline__ SliceKeys load_slice(const float* x, int n, int s, in
   return k;
 }
 
+struct SliceLds { int hist[kBins]; int scratch[64]; uint32_t cand_u[kMwCandLds], cand_i[kMwCandLds]; };
+
+// All of a row's keys are this workgroup's, and their histogram is in sh.hist: the picks.
+__device__ __forceinline__ void finish_slice(const TopkParams& p, const TopkRow& r, const SliceKeys& ks, float scale, float shift, SliceLds& sh) {
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, n = r.n, k = p.k;
+  if (tid == 0) sh.scratch[40] = 0;
+  int above;
+  const int d = select_digit<kTopkThreads>(sh.hist, sh.scratch, k, &above);
+  const int need = k - above, m = sh.hist[d];
+  const bool in_lds = m <= kMwCandLds;
+  auto each_key = [&](auto&& f) {                            // f(image, position) of the boundary bin's keys
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int i = ks.base + j * 256 + e;
+        if (i < n && linear_bin(ks.v[j][e], scale, shift) == d) f(ordered_bits(ks.v[j][e]), (uint32_t)i);
+      }
+  };
+  if (in_lds) {
+    each_key([&](uint32_t u, uint32_t i) {
+      const int slot = atomicAdd(&sh.scratch[40], 1);
+      sh.cand_u[slot] = u;
+      sh.cand_i[slot] = i;
+    });
+    __syncthreads();
+  }
+  uint32_t prefix, pos_thresh;
+  if (m <= kRankMax)
+    rank_threshold<kTopkThreads>(sh.cand_u, sh.cand_i, m, need, sh.hist, sh.scratch, &prefix, &pos_thresh);
+  else if (in_lds)
+    radix_threshold<kTopkThreads>([&](auto&& f) { for (int j = tid; j < m; j += kTopkThreads) f(sh.cand_u[j], sh.cand_i[j]); }, need, sh.hist,
+                                  sh.scratch, &prefix, &pos_thresh);
+  else
+    radix_threshold<kTopkThreads>(each_key, need, sh.hist, sh.scratch, &prefix, &pos_thresh);
+  const TopkSink out = topk_sink(p, r.b, r.t);
+  const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+  bool tk[2][4];
+  int at[2], mine = 0;
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    int before = 0, total = 0;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const uint32_t u = ordered_bits(ks.v[j][e]);
+      const int i = ks.base + j * 256 + e;
+      tk[j][e] = i < n && (u > prefix || (u == prefix && (uint32_t)i <= pos_thresh));
+      const uint64_t mk = __builtin_amdgcn_ballot_w64(tk[j][e]);
+      before += __builtin_popcountll(mk & below);
+      total += __builtin_popcountll(mk);
+    }
+    at[j] = mine + before;
+    mine += total;
+  }
+  __syncthreads();                                           // (scratch has been read)
+  if (lane == 0) sh.scratch[w] = mine;
+  __syncthreads();
+  int o = 0;
+#pragma unroll
+  for (int i = 0; i < kMwWaves; i++) o += i < w ? sh.scratch[i] : 0;
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    int to = o + at[j];
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (tk[j][e]) { if (to < k) out.put(to, ks.base + j * 256 + e); to++; }
+    if (out.mask) out.put_bits(ks.base + j * 256, n, tk[j][0] | tk[j][1] << 1 | tk[j][2] << 2 | tk[j][3] << 3);
+  }
+}
+
+// (64 registers: two workgroups on a CU; 67 cost 128 rows of 33 000 to 65 000 keys 4 us)
 template <int kVec>
-__global__ __launch_bounds__(kTopkThreads) void dsa_topk_hist_kernel(const TopkMwParams p) {
-  __shared__ int hist[kBins];
+__global__ __launch_bounds__(kTopkThreads, 8) void dsa_topk_hist_kernel(const TopkMwParams p) {
+  __shared__ SliceLds sh;
   __shared__ float fscratch[2 * kMwWaves];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const SliceOf so = slice_of_workgroup();
   const int s = so.s;
   const TopkRow r = topk_row(p.t, so.slot);
-  if (!r.live || r.n <= p.t.k || s * kSliceKeys >= r.n) return;
-  const int n = r.n;
+  if (!r.live) return;
+  const int n = r.n, k = p.t.k;
+  if (p.t.counts && s == 0 && tid == 0) p.t.counts[r.t] = n < k ? n : k;
+  if (n <= k) {                                            // everything is selected
+    if (s == 0) {
+      const TopkSink out = topk_sink(p.t, r.b, r.t);
+      for (int i = tid; i < k; i += kTopkThreads) {
+        if (i < n) out.put(i, i); else out.out[i] = -1;
+      }
+      if (out.mask) for (int i = tid; i * 8 < n; i += kTopkThreads) out.mask[i] = 0xff;
+    }
+    return;
+  }
+  if (s * kSliceKeys >= n) return;
   // all loads first: four runs of 1024 consecutive keys spread over the whole row (the sample that fixes the bins, the
   // same in every slice), and this slice
   float sm[4];
@@ -670,7 +755,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_hist_kernel(const TopkM
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) { lo = fminf(lo, __shfl_xor(lo, o, 64)); hi = fmaxf(hi, __shfl_xor(hi, o, 64)); }
   if (lane == 0) { fscratch[w] = lo; fscratch[kMwWaves + w] = hi; }
-  for (int i = tid; i < kBins; i += kTopkThreads) hist[i] = 0;
+  for (int i = tid; i < kBins; i += kTopkThreads) sh.hist[i] = 0;
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < kMwWaves; i++) { lo = fminf(lo, fscratch[i]); hi = fmaxf(hi, fscratch[kMwWaves + i]); }
@@ -686,10 +771,14 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_hist_kernel(const TopkM
   for (int j = 0; j < 2; j++)
 #pragma unroll
     for (int e = 0; e < 4; e++)
-      if (ks.base + j * 256 + e < n) atomicAdd(&hist[linear_bin(ks.v[j][e], scale, shift)], 1);
+      if (ks.base + j * 256 + e < n) atomicAdd(&sh.hist[linear_bin(ks.v[j][e], scale, shift)], 1);
   __syncthreads();
+  if (n <= kSliceKeys) {
+    finish_slice(p.t, r, ks, scale, shift, sh);
+    return;
+  }
   int32_t* hp = p.hist_part + ((int64_t)r.slot * p.slices + s) * kBins;
-  for (int i = tid; i < kBins; i += kTopkThreads) hp[i] = hist[i];
+  for (int i = tid; i < kBins; i += kTopkThreads) hp[i] = sh.hist[i];
 }
 
 template <int kVec>
@@ -700,7 +789,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_gather_kernel(const Top
   const SliceOf so = slice_of_workgroup();
   const int s = so.s;
   const TopkRow r = topk_row(p.t, so.slot);
-  if (!r.live || r.n <= p.t.k || s * kSliceKeys >= r.n) return;
+  if (!r.live || r.n <= p.t.k || r.n <= kSliceKeys || s * kSliceKeys >= r.n) return;
   const int n = r.n;
   const int live_slices = (n + kSliceKeys - 1) / kSliceKeys;
   // all loads first: the slice histograms of the token (two bins per thread), the bin map, this slice
@@ -747,19 +836,9 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_write_kernel(const Topk
   const SliceOf so = slice_of_workgroup();
   const int s = so.s;
   const TopkRow r = topk_row(p.t, so.slot);
-  if (!r.live) return;
   const int n = r.n, k = p.t.k;
+  if (!r.live || n <= k || n <= kSliceKeys || s * kSliceKeys >= n) return;
   const TopkSink out = topk_sink(p.t, r.b, r.t);
-  if (p.t.counts && s == 0 && tid == 0) p.t.counts[r.t] = n < k ? n : k;
-  if (n <= k) {                                            // everything is selected
-    if (s == 0)
-      for (int i = tid; i < k; i += kTopkThreads) {
-        if (i < n) out.put(i, i); else out.out[i] = -1;
-      }
-    if (out.mask && s == 0) for (int i = tid; i * 8 < n; i += kTopkThreads) out.mask[i] = 0xff;
-    return;
-  }
-  if (s * kSliceKeys >= n) return;
   // all loads first: the candidate list (its first kMwCandLds entries, whatever their number turns out to be), the
   // sure-pick counts of the wavefronts before mine, this slice
   const uint32_t* cand = p.cand + (int64_t)r.slot * p.cand_cap * 2;

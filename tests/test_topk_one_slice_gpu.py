@@ -1,0 +1,41 @@
+"""The selection in slices of 8192 keys where rows of one slice and of several, and rows that take all their keys, share a launch."""
+import pytest
+import torch
+
+from omni_npu_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("k", [1, 64, 2048, 4097])
+@pytest.mark.parametrize("vec", [True, False])
+def test_rows_around_a_slice(dev, k, vec):
+    """Against the one-workgroup kernel: lengths around k and around a slice; ties, equal keys (more than LDS holds), infinities, NaN; the
+    row lists and the pick bits."""
+    lens = torch.tensor([0, 1, k, k + 1, 5000, 8191, 8192, 8193, 16384, 20000, 8192, 8000, 8192], dtype=torch.int32)
+    t, stride = len(lens), 20000
+    g = torch.Generator().manual_seed(k)
+    x = torch.randn(t, stride, generator=g)
+    x[5] = torch.round(x[5] * 4) / 4
+    x[10] = 1.0
+    x[11, ::3], x[11, 1::7], x[11, 5::13] = float("inf"), float("-inf"), float("nan")
+    x[12, : 5000], x[12, 5000:] = -0.0, 0.0
+    lg = torch.zeros(t, stride + (0 if vec else 1), device=dev)[:, 0 if vec else 1:]
+    lg[:] = x.to(dev)
+    d = lens.to(dev)
+    bt = torch.randperm(t * 157, generator=g).view(t, 157).int().to(dev)
+    got = [torch.full((t, k), -7, dtype=torch.int32, device=dev) for _ in range(4)]
+    cnt = [torch.full((t,), -7, dtype=torch.int32, device=dev) for _ in range(2)]
+    K.topk(lg, d, k, got[0], block_table=bt, num_pages=t * 157, rows=got[1], counts=cnt[0])
+    K.topk(lg, d, k, got[2], single_workgroup=True, block_table=bt, num_pages=t * 157, rows=got[3], counts=cnt[1])
+    assert torch.equal(got[0], got[2]) and torch.equal(got[1], got[3]) and torch.equal(*cnt)
+    if not vec:
+        return                                                 # (pick bits want aligned rows)
+    mask = torch.randint(-2 ** 31, 2 ** 31 - 1, (t, stride // 32), generator=g).int().to(dev)
+    K.topk(lg, d, k, got[0], mask=mask)
+    assert torch.equal(got[0], got[2])
+    bits = (mask.cpu().view(t, -1, 1) >> torch.arange(32).view(1, 1, -1) & 1).view(t, -1)
+    want = torch.zeros(t, stride + 1, dtype=torch.int32)
+    want.scatter_(1, torch.where(got[2] < 0, stride, got[2]).long().cpu(), 1)
+    seen = torch.arange(stride)[None] < lens[:, None]
+    assert torch.equal(bits.int()[seen], want[:, :stride][seen])
