@@ -11,7 +11,6 @@
 // Workspace (mla_decode_workspace_bytes): batch * (num_splits + 1) partial slots of rows = max_q_len * num_heads each:
 // normalised fp16 partials [slots, rows, 512], fp32 log-sum-exps [slots, rows], a correction record per row (fp32
 // factor + cache address of the row's dominant key) and two partial numbers per sequence.
-#include <cstdlib>
 #include <mutex>
 #include "mla_common.hpp"
 #include "decode_params.hpp"
@@ -85,7 +84,7 @@ static int decode_split_impl(const void* q_nope, int64_t qn_stride_t, int64_t qn
   v.win_skip = win_skip; v.win_sink = win_sink; v.win_size = win_size;
   v.new_c = (const __bf16*)new_c; v.new_c_st = new_c_stride; v.new_r = (const __bf16*)new_r; v.new_r_st = new_r_stride;
   v.new_slots = new_slots;
-  const PlanForm form = plan_form(batch, num_splits, r_max, !fp8);
+  const PlanForm form = plan_form(batch, num_splits, r_max, fp8);
   v.num_chunks = form.chunks;
   if (fp8) return launch_decode_v3_fp8(v, form.rg, stream);
   return launch_decode_v3(v, sparse_rows != nullptr, form.rg, stream);
@@ -201,7 +200,7 @@ extern "C" int mla_splitkv_reduce(const void* workspace, size_t workspace_bytes,
   cp.seq_lens = seq_lens; cp.qsl = query_start_loc;
   // (the plan of the bf16 cache: where the fp8 cache's is another one, up to 512 rows, both leave more than a dozen partials per sequence,
   // which is all that launch_chunk_reduce asks)
-  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = plan_form(batch, num_splits, r_max, true).chunks;
+  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = plan_form(batch, num_splits, r_max, false).chunks;
   cp.out = (__bf16*)out; cp.out_st = out_stride_t; cp.out_sh = out_stride_h;
   cp.lse_out = lse_out; cp.lse_st = num_heads;
   return launch_chunk_reduce(cp, stream);

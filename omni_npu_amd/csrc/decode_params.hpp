@@ -81,21 +81,23 @@ constexpr int kPlanCUs = 256;                              // MI355X
 // cutting the keys finer would make every workgroup pay a segment's start and end for a handful of blocks, so the rows are
 // cut instead, into groups with a workgroup each over the whole chunk (the groups of a chunk sit next to each other on one XCD and
 // share the cache rows in its L2).  (Up to three splits a caller may have asked for few chunks itself, whatever the lengths: past half
-// the CUs those keep the 128-row form.)  Groups of 32 rows where the kernel is decode_rows.hip (`rows32`: the bf16 cache), of 32 or 64
-// over the fp8 cache.  Where the lines lie, us per layer as a graph replay in groups of 64 / 32 rows of that kernel: 7 requests of
-// 300-3000 keys x 128 heads 37.2 / 35.2, 16 of 1k-2k 47.6 / 47.3, 7 of 4k-8k 49.4 / 49.4, 16 of 4k-8k 65.2 / 65.3; x 64 heads,
-// one of 1k keys 26.1 / 22.9, 4 of 1k-3k 32.4 / 29.6 (128 chunks), but 8 of 2k-4k 35.0 / 39.4 (256), 64 of 4k-8k 123 / 156.  Queued
-// launches, 12 requests x 128 heads: 300-3000 keys (144 workgroups of 128 rows) 36.5 / 34.6, 3k-5k (240) 46.3 / 48.3.
+// the CUs those keep the 128-row form.)  Groups of 32 rows (decode_rows.hip) or of 64.  Where the lines lie, us per layer as a graph
+// replay in groups of 64 / 32 rows: 7 requests of 300-3000 keys x 128 heads 37.2 / 35.2, 16 of 1k-2k 47.6 / 47.3, 7 of 4k-8k 49.4 /
+// 49.4, 16 of 4k-8k 65.2 / 65.3; x 64 heads, one of 1k keys 26.1 / 22.9, 4 of 1k-3k 32.4 / 29.6 (128 chunks), but 8 of 2k-4k 35.0 /
+// 39.4 (256), 64 of 4k-8k 123 / 156.  Queued launches, 12 requests x 128 heads: 300-3000 keys (144 workgroups of 128 rows) 36.5 /
+// 34.6, 3k-5k (240) 46.3 / 48.3.  Over the fp8 cache (`fp8`), whose blocks cost the small form their conversions once per group, split,
+// merge and up-projection: x 64 heads, 8 of 500-2000 keys 24.7 / 21.9, 6 of 2k-5k 28.0 / 24.2; x 128, 7 of 300-3000 (84 workgroups of 128
+// rows) 28.8 / 25.7, 5 of 2k-6k (120) 32.4 / 30.1, but 2 of 10k-16k (126) 32.7 / 34.9, 4 of 4k-9k (144) 32.9 / 34.9.
 struct PlanForm { int rg, chunks; };
-inline PlanForm plan_form(int64_t batch, int64_t num_splits, int64_t query_rows, bool rows32) {
+inline PlanForm plan_form(int64_t batch, int64_t num_splits, int64_t query_rows, bool fp8) {
   const int64_t total = batch * num_splits, groups = (query_rows + 127) / 128, wgs = total * groups;
   if (query_rows > 64 && wgs * 4 <= kPlanCUs) return {1, (int)total};
   if (query_rows > 64 && (wgs * 2 <= kPlanCUs || (wgs < kPlanCUs && num_splits > 3))) {
-    const int rg = rows32 && wgs * 8 <= kPlanCUs * 7 ? 1 : 2;
+    const int rg = wgs * 32 <= kPlanCUs * (fp8 ? 15 : 28) ? 1 : 2;
     const int64_t most = kPlanCUs / ((query_rows + 32 * rg - 1) / (32 * rg));
     return {rg, (int)(total < most || most < 1 ? total : most)};
   }
-  if (rows32 && query_rows <= 64 && total * 2 <= kPlanCUs) return {1, (int)total};
+  if (query_rows <= 64 && total * 2 <= kPlanCUs) return {1, (int)total};
   const int rg = query_rows <= 32 ? 1 : (query_rows <= 64 ? 2 : 4);
   const int64_t rounds = wgs / kPlanCUs;
   if (rounds < 1) return {rg, (int)total};
@@ -133,9 +135,9 @@ inline dim3 plan_grid(const DecodeParams& p, int rg) {
 // window.  Returns 0 or a negative error code.
 // rg: groups of 32 query rows per workgroup (plan_form).
 int launch_decode_v3(const DecodeParams& p, bool sparse, int rg, hipStream_t stream);
-// The forms with 32 rows per workgroup (decode_rows.hip); list: over p.sparse_rows.
+// The forms with 32 rows per workgroup (decode_rows.hip), over p.cache8 where there is one; list: over p.sparse_rows.
 int launch_decode_rows(const DecodeParams& p, bool list, hipStream_t stream);
-int prepare_decode_rows(bool list, bool window, bool write);
+int prepare_decode_rows(bool list, bool fp8, bool window, bool write);
 // The dynamic-LDS limit of all dense bf16 forms raised on the current device, ahead of a launch under stream capture.
 int prepare_decode_v3_dense_forms();
 // The same over the fp8 block-scaled cache p.cache8 (decode_v3_fp8.hip): dense and, with p.win_size > 0, sink + window.

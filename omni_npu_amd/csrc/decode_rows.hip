@@ -1,6 +1,6 @@
-// Absorbed-MLA decode over the bf16 cache for launches whose workgroups have few query rows: the split phase with at most 32 rows per
-// workgroup (plan_form's rg = 1), over the paged cache, over it with static sink tokens and a sliding window, and over lists of
-// cache rows.  Same contract, workspace and merge as decode_v3.hip.
+// Absorbed-MLA decode for launches whose workgroups have few query rows: the split phase with at most 32 rows per workgroup (plan_form's
+// rg = 1), over the paged bf16 cache and the fp8 one, over either with static sink tokens and a sliding window, and over lists of bf16
+// cache rows.  Same contract, workspace and merge as decode_v3.hip and decode_v3_fp8.hip.
 //
 // What bounds it: with few rows the arithmetic is small beside the cache stream, and a short launch is a chain of dependent steps:
 // arguments, lengths, page numbers, first keys, scores, result.  A wavefront issues an instruction every five clocks, so the
@@ -15,9 +15,15 @@
 //   O += V P    wavefront w owns 64 latent columns for all rows.  A probability goes through P.V as two bf16 numbers, its rounded
 //               value and what the rounding left, through LDS in the layout that is the MFMA operand's: the same lanes hold it
 // Two buffers of 64 keys: the next iteration's copies go out when this one's have landed.  Two barriers per iteration.
+//   fp8 cache   a wavefront's eight rows come into registers (nine loads, an iteration ahead) and go into the other buffer as bf16 (x = e4m3
+//               * block scale, rounded) in front of the scores; of 17 to 32 rows a probability goes through P.V rounded once, as in the
+//               general kernel: with its second term 64 requests of 4k-8k keys x 32 heads take 90.6 us instead of 86.2 (general kernel: 85.9)
 // us per layer, general kernel with groups of 32 or 64 rows -> this: one user of 1k keys x 16 heads 17.9 -> 14.7; 7 of 300-3000 keys x
 // 128 heads, replayed 40.0 -> 37.9; 4 of 1k-3k x 64 heads 34.2 -> 29.9; 64 of 4k-8k x 16 heads 93.9 -> 87.5 (HBM); lists of 2048 rows, 8
-// tokens x 64 heads with their selection 70.8 -> 62.8; 8 windows of 2048 x 64 heads 41.4 -> 33.4.
+// tokens x 64 heads with their selection 70.8 -> 62.8; 8 windows of 2048 x 64 heads 41.4 -> 33.4.  Over the fp8 cache, us of split, merge
+// and up-projection: one user 15.8 -> 13.2, 16 of 300-1500 keys x 16 heads 19.7 -> 18.2, 2 of 14 000 x 16 22.9 -> 20.3, 64 of 4k-8k x 16
+// 81.9 -> 71.3, 200 of 500-3000 x 16 84.1 -> 71.4; in two halves of the wavefronts, one's conversions in front of its scores and the
+// other's behind its P.V, 85.3 and 84.4: each half waits for the other's at the barrier between.
 #include "decode_params.hpp"
 
 namespace mlahip {
@@ -45,12 +51,17 @@ __device__ __forceinline__ int div_small(int a, int b) {
 }
 __device__ __forceinline__ int div_units(int a, int b) { return a < (1 << 21) ? div_small(a, b) : a / b; }
 
-enum class Keys { kPaged, kWindow, kList };
+constexpr int kRow8 = 656, kScale8 = 512, kRope8 = 528;     // a row of the fp8 cache: 512 e4m3, 4 fp32 scales, 64 bf16 rope
+constexpr int kAsk8 = 9;                                   // loads of an iteration's eight rows
+struct Rows8 { u32x4 x[4], rope; float scale[4]; };
+
+enum class Keys { kPaged, kWindow, kList, kPaged8, kWindow8 };
 // kNt: the rows of a chunk have no other reader than this workgroup, and their copies are marked non-temporal (see decode_v3.hip)
 // kWrite: the step's cache write, folded in (see decode_v3.hip)
 template <Keys kKeys, bool kNt, bool kWrite>
 __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams p) {
-  constexpr bool kWindow = kKeys == Keys::kWindow, kList = kKeys == Keys::kList;
+  constexpr bool kWindow = kKeys == Keys::kWindow || kKeys == Keys::kWindow8, kList = kKeys == Keys::kList;
+  constexpr bool kFp8 = kKeys == Keys::kPaged8 || kKeys == Keys::kWindow8;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -182,6 +193,7 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
     }
     lds_barrier();                                           // the previous segment is done with the buffers
     const bool has_rows = row0 + rg * 16 < rows, two = row0 + 16 < rows;
+    const bool both_terms = !(kFp8 && two);                  // (see above)
     int limit = L - qlen + div_small(row, p.num_heads) + 1;  // keys [0, limit) are visible to the row
     const int seen_to = limit;
     limit = row < rows ? (limit < key_end ? limit : key_end) : 0;
@@ -232,6 +244,59 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
       }
       place = place_of(it + 1);
     };
+    // The fp8 rows: lane l asks for 16 of the 512 numbers of rows l / 32, l / 32 + 2, ... of the wavefront's eight.  Rows behind the
+    // segment's last one are read as they lie in the page and written as zeros.
+    const uint32_t x8_off = (uint32_t)((lane >> 5) * kRow8 + (lane & 31) * 16), s8_off = (uint32_t)((lane >> 5) * kRow8 + kScale8 + ((lane >> 3) & 3) * 4);
+    auto ask_rows = [&](int it, Rows8& r) {
+      const int64_t pg = place < 0 ? 0 : (place >= p.num_pages ? p.num_pages - 1 : place);
+      const int first = key0 + it * kIter + wave * 8, first_read = first < key_last ? first : key_last & ~7;
+      const char* from = (const char*)p.cache8 + pg * p.c8_sp + (in_cache(first_read) & (kPage - 1)) * kRow8;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const u32x4* at = (const u32x4*)(from + x8_off + i * 2 * kRow8);
+        r.x[i] = kNt ? __builtin_nontemporal_load(at) : *at;
+      }
+      {
+        const u32x4* at = (const u32x4*)(from + rope_j * kRow8 + kRope8 + (lane & 7) * 16);
+        r.rope = kNt ? __builtin_nontemporal_load(at) : *at;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++) r.scale[i] = *(const float*)(from + s8_off + i * 2 * kRow8);
+      place = place_of(it + 1);
+    };
+    auto put_rows = [&](int it, Rows8& r) {
+      char* to = lds + (it & 1) * kBufB + wave * 8192;
+      const int first = key0 + it * kIter + wave * 8;
+      if (first + 7 > key_last) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          if (first + 2 * i + (lane >> 5) > key_last) { r.x[i] = u32x4{0u, 0u, 0u, 0u}; r.scale[i] = 0.f; }
+        }
+        if (first + rope_j > key_last) r.rope = u32x4{0u, 0u, 0u, 0u};
+      }
+      // (sixteen neighbouring lanes write sixteen different granules modulo the banks: lanes 8..15 of them begin with their second one)
+      const uint32_t c = lane & 31, swap = (lane >> 3) & 1;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int row = 2 * i + (lane >> 5);
+        const uint32_t at = (uint32_t)(row * 1024) + (((2 * c + swap) ^ (uint32_t)swz_nope((wave & 1) * 8 + row)) << 4);
+        u32x4 o[2];
+#pragma unroll
+        for (int h = 0; h < 4; h++) {
+          const f32x2 x0 = __builtin_amdgcn_cvt_pk_f32_fp8((int)r.x[i][h], false), x1 = __builtin_amdgcn_cvt_pk_f32_fp8((int)r.x[i][h], true);
+          bf16x2 y0, y1;
+          y0[0] = (__bf16)(x0[0] * r.scale[i]); y0[1] = (__bf16)(x0[1] * r.scale[i]);
+          y1[0] = (__bf16)(x1[0] * r.scale[i]); y1[1] = (__bf16)(x1[1] * r.scale[i]);
+          o[h >> 1][(h & 1) * 2] = __builtin_bit_cast(uint32_t, y0);
+          o[h >> 1][(h & 1) * 2 + 1] = __builtin_bit_cast(uint32_t, y1);
+        }
+        const u32x4 a = swap ? o[1] : o[0], b = swap ? o[0] : o[1];
+        *(u32x4*)(to + at) = a;
+        *(u32x4*)(to + (at ^ 16u)) = b;
+      }
+      *(u32x4*)(lds + (it & 1) * kBufB + kRopeOff + wave * 1024 + rope_j * 128 + rope_off) = r.rope;
+    };
+    Rows8 ahead;                                             // rows of the next iteration, on their way
 
     // ---- the query through LDS (the second buffer, free until the first iteration has begun), rows as the keys lie ----
     {
@@ -277,9 +342,11 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
     for (int it = 0; it < iters; it++) {
       if (it == 0) {
         place = place_of(0);
-        copy_keys(0);
+        if constexpr (kFp8) ask_rows(0, ahead);
+        else copy_keys(0);
+        static_assert(kAsk8 == 9, "one wait for both");
         if (fresh) {
-          MLA_WAIT_VMCNT(9);                                       // the query is here, the nine copies of the keys may be on their way
+          MLA_WAIT_VMCNT(9);                                       // the query is here, the nine copies (or loads) of the keys may be on their way
           lds_barrier();
           {
             // (row l16 of the wavefront's row group lies where key l16 of key group rg would)
@@ -295,10 +362,21 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
 #pragma unroll
           for (int j = 0; j < 2; j++) acc[cb][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         l_run = 0.f;
+        if constexpr (kFp8) {
+          put_rows(0, ahead);
+          if (iters > 1) ask_rows(1, ahead);
+        }
       }
-      MLA_WAIT_VMCNT(0);
+      if constexpr (!kFp8) MLA_WAIT_VMCNT(0);
       lds_barrier();                                         // this iteration's keys are here, everyone is done with the other buffer
-      if (it + 1 < iters) copy_keys(it + 1);
+      if (it + 1 < iters) {
+        if constexpr (kFp8) {
+          put_rows(it + 1, ahead);
+          if (it + 2 < iters) ask_rows(it + 2, ahead);
+        } else {
+          copy_keys(it + 1);
+        }
+      }
       const char* buf = lds + (it & 1) * kBufB;
       float t[4];
       if (has_rows) {
@@ -336,7 +414,7 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
         }
         char* pw = lds + kPOff + ((kg >> 1) * 4 + rg * 2) * 1024 + lane * 16 + (kg & 1) * 8;
         *(bf16x4*)pw = hi;
-        *(bf16x4*)(pw + 1024) = lo;
+        if (both_terms) *(bf16x4*)(pw + 1024) = lo;
         const bool ask = __builtin_amdgcn_ballot_w64(top - m_ref > kRestartThreshold) != 0;
         if (lane == 0) *(int*)(lds + kFlagOff + wave * 4) = ask ? 1 : 0;
       } else if (lane == 0) {
@@ -352,7 +430,7 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
         for (int j = 0; j < 2; j++)
 #pragma unroll
           for (int term = 0; term < 2; term++)
-            if (j == 0 || two) pf[j][term] = *(const bf16x8*)(lds + kPOff + (pair * 4 + j * 2 + term) * 1024 + lane * 16);
+            if ((j == 0 || two) && (term == 0 || both_terms)) pf[j][term] = *(const bf16x8*)(lds + kPOff + (pair * 4 + j * 2 + term) * 1024 + lane * 16);
 #pragma unroll
         for (int cb = 0; cb < 4; cb++) {
           const char* vb = buf + pair * 32768 + (v_off ^ (uint32_t)(cb << 5));
@@ -362,7 +440,7 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
           for (int j = 0; j < 2; j++)
             if (j == 0 || two) {
               acc[cb][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pf[j][0], acc[cb][j], 0, 0, 0);
-              acc[cb][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pf[j][1], acc[cb][j], 0, 0, 0);
+              if (both_terms) acc[cb][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pf[j][1], acc[cb][j], 0, 0, 0);
             }
         }
       }
@@ -401,7 +479,7 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
         if (kg == 0 && rg == j && g == 0) {
           p.lse_part[part] = l > 0.f ? (m_ref + fast_log2(l)) * kLn2 : -INFINITY;
           p.corr_scale[part] = 0.f;                          // (no correction record: P.V carries what the rounding left)
-          p.corr_row[part] = p.nope;
+          p.corr_row[part] = kFp8 ? nullptr : p.nope;
         }
       }
     }
@@ -413,28 +491,31 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
 namespace {
 using rows32::Keys;
 typedef void (*RowsKernel)(const DecodeParams);
-// the kernel of a launch: over a list or the paged cache; windowed; with the step's cache write; chunks with one reader
-RowsKernel rows_kernel(bool list, bool window, bool write, bool once) {
+// the kernel of a launch: over a list or the paged cache (fp8: the quantised one); windowed; with the step's cache write; chunks with
+// one reader
+RowsKernel rows_kernel(bool list, bool fp8, bool window, bool write, bool once) {
   using namespace rows32;
   if (list) return mla_decode_rows_kernel<Keys::kList, false, false>;
+  if (fp8 && window) return once ? mla_decode_rows_kernel<Keys::kWindow8, true, false> : mla_decode_rows_kernel<Keys::kWindow8, false, false>;
+  if (fp8) return once ? mla_decode_rows_kernel<Keys::kPaged8, true, false> : mla_decode_rows_kernel<Keys::kPaged8, false, false>;
   if (window) return once ? mla_decode_rows_kernel<Keys::kWindow, true, false> : mla_decode_rows_kernel<Keys::kWindow, false, false>;
   if (write) return once ? mla_decode_rows_kernel<Keys::kPaged, true, true> : mla_decode_rows_kernel<Keys::kPaged, false, true>;
   return once ? mla_decode_rows_kernel<Keys::kPaged, true, false> : mla_decode_rows_kernel<Keys::kPaged, false, false>;
 }
 }  // namespace
-int prepare_decode_rows(bool list, bool window, bool write) {
+int prepare_decode_rows(bool list, bool fp8, bool window, bool write) {
   for (int once = 0; once < 2; once++) {
-    const int rc = ensure_dynamic_lds((const void*)rows_kernel(list, window, write, once), rows32::kLdsB, "mla_decode_rows_kernel");
+    const int rc = ensure_dynamic_lds((const void*)rows_kernel(list, fp8, window, write, once), rows32::kLdsB, "mla_decode_rows_kernel");
     if (rc != MLA_OK) return rc;
   }
   return MLA_OK;
 }
 int launch_decode_rows(const DecodeParams& p, bool list, hipStream_t stream) {
-  const bool window = p.win_size > 0, write = p.new_c != nullptr;
-  const int rc = prepare_decode_rows(list, window, write);
+  const bool window = p.win_size > 0, write = p.new_c != nullptr, fp8 = p.cache8 != nullptr;
+  const int rc = prepare_decode_rows(list, fp8, window, write);
   if (rc != MLA_OK) return rc;
   const dim3 grid = plan_grid(p, 1);
-  hipLaunchKernelGGL(rows_kernel(list, window, write, grid.z == 1), grid, dim3(512), rows32::kLdsB, stream, p);
+  hipLaunchKernelGGL(rows_kernel(list, fp8, window, write, grid.z == 1), grid, dim3(512), rows32::kLdsB, stream, p);
   return check_launch("mla_decode_rows_kernel");
 }
 

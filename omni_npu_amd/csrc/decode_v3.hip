@@ -1066,7 +1066,7 @@ template <bool kSparse, bool kWindow, bool kWrite = false>
 static int launch_rows(const DecodeParams& p, int rg, hipStream_t stream) {
   // (the form depends on the shape; all of them get their LDS limit with the family's first launch, so that a later launch
   // under stream capture, where the limit cannot be raised, finds every form ready)
-  int rc = prepare_decode_rows(kSparse, kWindow, kWrite);
+  int rc = prepare_decode_rows(kSparse, false, kWindow, kWrite);
   if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)v3::mla_decode_v3_kernel<kSparse, kWindow, 2, kWrite>, v3::kLdsB, "mla_decode_v3_kernel");
   if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)v3::mla_decode_v3_kernel<kSparse, kWindow, 4, kWrite>, v3::kLdsB, "mla_decode_v3_kernel");
   if (rc != MLA_OK) return rc;
@@ -1078,7 +1078,7 @@ static int launch_rows(const DecodeParams& p, int rg, hipStream_t stream) {
 // Raises the dynamic-LDS limit of every dense form on the current device (what a launch does for its own form the first
 // time it runs): a caller that will launch under stream capture, where that cannot be recorded, does it beforehand.
 int prepare_decode_v3_dense_forms() {
-  int rc = prepare_decode_rows(false, false, false);
+  int rc = prepare_decode_rows(false, false, false, false);
   if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)v3::mla_decode_v3_kernel<false, false, 2, false>, v3::kLdsB, "mla_decode_v3_kernel");
   if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)v3::mla_decode_v3_kernel<false, false, 4, false>, v3::kLdsB, "mla_decode_v3_kernel");
   return rc;

@@ -15,7 +15,6 @@
 // antiquant_mode=0, antiquant_scale=None.
 #include "decode_params.hpp"
 #include <type_traits>
-#include <cstdlib>
 
 namespace mlahip {
 namespace f8v3 {
@@ -72,12 +71,12 @@ __device__ __forceinline__ int wave_incl_scan_i32(int v, int lane) {
 }
 
 
-// kRG = groups of 32 query rows that can hold rows at all (4: any launch; 1 or 2: at most 32 / 64 query rows per request, as
-// in the bf16 kernel): only the wavefronts that own rows run the S phase and the softmax, P.V covers kRG row groups, the
+// kRG = groups of 32 query rows that can hold rows at all (4: any launch; 2: at most 64 query rows per workgroup; launches of 32 are
+// decode_rows.hip's): only the wavefronts that own rows run the S phase and the softmax, P.V covers kRG row groups, the
 // copies move to wavefronts 4..7; all 512 threads still turn the raw block into its bf16 tile.
 template <bool kWindow, int kRG = 4>
 __global__ __launch_bounds__(512) void mla_decode_v3_fp8_kernel(const DecodeParams p) {
-  static_assert(kRG == 1 || kRG == 2 || kRG == 4, "row groups");
+  static_assert(kRG == 2 || kRG == 4, "row groups");
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);     // 0..7
@@ -549,14 +548,7 @@ __global__ __launch_bounds__(512) void mla_decode_v3_fp8_kernel(const DecodePara
     // (small forms only, where the matrix pipe has time to spare: the block's last MFMAs have written their accumulators
     // before anything the compiler may place behind this statement reads them)
 #define PV_SETTLE(rg) asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+a"(acc[0][rg]), "+a"(acc[1][rg]))
-    if constexpr (kRG == 1) {
-      if constexpr (kPv) { PV_VREAD(0); PV_PREAD(pr0, 0, 0); }
-      if constexpr (kSm) { if (sm_on) { sm_head(sc, st); SM_EXP2(0, 1); SM_EXP2(2, 3); } }
-      if constexpr (kPv) { PV_MFMA2(0, pr0, 0); PV_VREAD(1); PV_PREAD(pr0, 0, 1); }
-      if constexpr (kSm) { if (sm_on) { SM_EXP2(4, 5); SM_EXP2(6, 7); sm_pm(st); } }
-      if constexpr (kPv) { PV_MFMA2(0, pr0, 0); PV_SETTLE(0); }
-      if constexpr (kSm) { if (sm_on) { sm_sum_lo(sc, st); sm_sum_hi(sc, st); } }
-    } else if constexpr (kRG == 2) {
+    if constexpr (kRG == 2) {
       if constexpr (kPv) { PV_VREAD(0); PV_PREAD(pr0, 0, 0); PV_PREAD(pr1, 1, 0); }
       if constexpr (kSm) { if (sm_on) { sm_head(sc, st); SM_EXP2(0, 1); } }
       if constexpr (kPv) PV_MFMA2(0, pr0, 1);
@@ -811,14 +803,14 @@ static int launch_form_fp8(const DecodeParams& p, hipStream_t stream) {
 }
 template <bool kWindow>
 static int launch_rows_fp8(const DecodeParams& p, int rg, hipStream_t stream) {
-  // (all three forms get their LDS limit with the family's first launch: a later launch under stream capture finds them ready)
+  // (all forms get their LDS limit with the family's first launch: a later launch under stream capture finds them ready)
   {
-    int rc = ensure_dynamic_lds((const void*)f8v3::mla_decode_v3_fp8_kernel<kWindow, 1>, f8v3::kLdsB, "mla_decode_v3_fp8_kernel");
+    int rc = prepare_decode_rows(false, true, kWindow, false);
     if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)f8v3::mla_decode_v3_fp8_kernel<kWindow, 2>, f8v3::kLdsB, "mla_decode_v3_fp8_kernel");
     if (rc == MLA_OK) rc = ensure_dynamic_lds((const void*)f8v3::mla_decode_v3_fp8_kernel<kWindow, 4>, f8v3::kLdsB, "mla_decode_v3_fp8_kernel");
     if (rc != MLA_OK) return rc;
   }
-  if (rg == 1) return launch_form_fp8<kWindow, 1>(p, stream);
+  if (rg == 1) return launch_decode_rows(p, false, stream);
   if (rg == 2) return launch_form_fp8<kWindow, 2>(p, stream);
   return launch_form_fp8<kWindow, 4>(p, stream);
 }

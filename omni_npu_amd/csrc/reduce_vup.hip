@@ -338,7 +338,7 @@ static int reduce_vup_impl(const void* workspace, size_t workspace_bytes, const 
   cp.corr_scale = cp.lse_part + rows; cp.corr_row = (const __bf16* const*)(cp.lse_part + 2 * rows);
   cp.seg_ids = (const int32_t*)(cp.lse_part + 4 * rows);
   cp.seq_lens = seq_lens; cp.qsl = query_start_loc;
-  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = plan_form(batch, num_splits, r_max, !fp8).chunks;
+  cp.batch = batch; cp.max_q_len = max_q_len; cp.num_heads = num_heads; cp.num_chunks = plan_form(batch, num_splits, r_max, fp8).chunks;
   cp.out = (__bf16*)out; cp.out_st = out_stride_t; cp.out_sh = out_stride_h;
   cp.lse_out = nullptr; cp.lse_st = 0;
   return launch_reduce_vup(cp, w_uv, w_stride_n, w_stride_k, num_tokens, stream);
