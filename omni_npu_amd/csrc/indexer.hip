@@ -217,20 +217,24 @@ __global__ __launch_bounds__(256, 2) void dsa_indexer_fp8_kernel(const IndexerPa
 }
 
 // The same scores for prompts, where neighbouring query tokens see the same keys: the kernel above reads every token's keys
-// for itself (10 168 prompt tokens, 20 M (token, key) pairs: 2.7 GB through the L2s, 980 us).  Here a workgroup keeps the
-// queries of kTileTok tokens of one request in LDS (32 KiB, four workgroups per CU) and each of its wavefronts walks every
-// 4 gridDim.x-th block of 32 keys, held in registers (the next block on its way meanwhile), against all of the tokens: a
-// key is read once per kTileTok tokens, a query operand from LDS at a quarter of its rate, and what is left is the 16 MFMAs
-// and 64 vector instructions per token and block, which wavefronts of one SIMD do beside each other: the more of them the
-// better (eight tokens and two wavefronts per SIMD, relu in two instructions: 286 us on those prompts; now 199).  Same
-// operations in the same order as above: the same bits.
-constexpr int kTileTok = 4;
+// for itself (10 168 prompt tokens, 20 M (token, key) pairs: 2.7 GB through the L2s, 980 us).  Here each of a workgroup's four
+// wavefronts keeps one token's queries and weights in registers, as above, and all of them walk the same stages of 128 keys, every
+// gridDim.x-th one.  They copy the stages into two LDS buffers for each other, a block each: a stage's copies are on their way while
+// the one before is worked on, and its logits leave behind the barrier that follows, so that no wait sees a store's way to memory.
+// What bounds it: 16 MFMAs (512 clocks) and 64 vector instructions (256) per token and 32 keys.  Wavefronts that take turns at the matrix
+// unit end up in step and leave it idle while they all multiply by their weights, so a wavefront does that for one block between the
+// MFMAs of the next, four instructions to each: two sets of sums, 168 registers, three wavefronts per SIMD.
+// us, with four tokens' queries in LDS and the keys in registers (sixteen LDS reads per 32 keys, now four) -> in registers, four
+// wavefronts per SIMD, one set of sums -> this: prompts of 6197 and 6551 tokens that skip 2048 427 -> 413 -> 376 (1.6 PFLOP/s: what the
+// power that the card may draw leaves of 2.5), four of 1024 behind 8192 keys 415 -> 389 -> 362, of 1500, 2300 and 5003 160 -> 150 ->
+// 145, 64 tokens behind 30 000 keys 43 -> 38 -> 31.  Same operations in the same order as above: the same bits.
+constexpr int kTileTok = 4;                           // tokens of a workgroup, one to a wavefront
 constexpr int kTileMinQ = 16;                         // shorter requests (decode, MTP) take the streaming kernel
-constexpr int kTileWOff = kTileTok * 64 * kIdxDim;    // 32768: weights [token][head] behind the query rows
-constexpr int kTileLdsB = kTileWOff + kTileTok * 64 * 4;
+constexpr int kTileBlocks = 4;                        // 32-key blocks of a stage
+constexpr int kTileBufB = kTileBlocks * kIdxSlotB;    // 16896
 
-__global__ __launch_bounds__(256, 4) void dsa_indexer_tile_kernel(const IndexerParams p) {
-  extern __shared__ __attribute__((aligned(1024))) char lds[];
+__global__ __launch_bounds__(256, 3) void dsa_indexer_tile_kernel(const IndexerParams p) {
+  __shared__ __attribute__((aligned(1024))) char lds[2 * kTileBufB];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int key_l = lane & 31, half = lane >> 5;
@@ -241,85 +245,126 @@ __global__ __launch_bounds__(256, 4) void dsa_indexer_tile_kernel(const IndexerP
   const int nt = qlen - tok0 < kTileTok ? qlen - tok0 : kTileTok;
   const int lim0 = p.seq_lens[b] - qlen + tok0 + 1;          // visible keys of the first token; one more for each later one
   const int lim_max = lim0 + nt - 1;
-  const int blocks = lim_max > p.skip_up_to ? (lim_max + 31) >> 5 : 0;
-  if ((int)blockIdx.x * 4 >= blocks) return;
+  const int blocks = lim_max > p.skip_up_to ? (lim_max + 31) >> 5 : 0, stages = (blocks + kTileBlocks - 1) / kTileBlocks;
+  if ((int)blockIdx.x >= stages) return;
+  int limit = wave < nt ? lim0 + wave : 0;                   // of this wavefront's token; 0: it has none, or one without logits
+  limit = limit <= p.skip_up_to ? 0 : limit;
+  const int64_t t = q0 + tok0 + (wave < nt ? wave : nt - 1);
 
-  // queries: row (token, head) of 128 bytes, 16-byte granule g at position g ^ ((head >> 1) & 7)
+  // A wavefront copies one block of a stage.  Slots as above; blocks behind the last one repeat it.
   const uint32_t lds0 = lds_addr_of(lds);
-#pragma unroll
-  for (int i = 0; i < kTileTok * 2; i++) {
-    const int g = wave * (kTileTok * 2) + i;                 // group of eight rows
-    const int tk = g >> 3 < nt ? g >> 3 : nt - 1, head = (g & 7) * 8 + (lane >> 3);
-    dma16_v(p.q8 + (int64_t)(q0 + tok0 + tk) * p.q_st + (int64_t)head * p.q_sh + (((lane & 7) ^ ((head >> 1) & 7)) << 4),
-            lds0 + g * 1024);
-  }
-#pragma unroll
-  for (int i = 0; i < kTileTok * 64 / 256; i++) {
-    const int e = threadIdx.x + i * 256, head = e & 63, tk = e >> 6 < nt ? e >> 6 : nt - 1;
-    float w = p.weights[(int64_t)(q0 + tok0 + tk) * p.w_st + head];
-    if (p.q_scale) w *= p.q_scale[(int64_t)(q0 + tok0 + tk) * p.qs_st + head];
-    *(float*)(lds + kTileWOff + e * 4) = w;
-  }
-
-  const int stride = (int)gridDim.x * 4;
-  auto load_block = [&](int blk, u32x4 (&kb)[4], float& ks) {
+  const uint32_t src_row = (uint32_t)((lane >> 3) * (int)p.k_sr);   // of rows 8 i + l / 8: granule (l % 8) ^ swizzle(row)
+  const uint32_t src_off[2] = {src_row + 16 * ((lane & 7) ^ (lane >> 4)), src_row + 16 * ((lane & 7) ^ (lane >> 4) ^ 4)};
+  auto copy_stage = [&](int stage, int buf) {
+    int blk = stage * kTileBlocks + wave;
+    blk = blk < blocks ? blk : blocks - 1;
     const int key0 = blk * 32, pg = key0 / p.page_size;
     const int pgc = pg < p.max_blocks ? pg : p.max_blocks - 1;
     int64_t id = ((const __attribute__((address_space(4))) int32_t*)p.block_table)[(int64_t)b * p.bt_stride + pgc];
     id = id < 0 ? 0 : (id >= p.num_pages ? p.num_pages - 1 : id);
-    const int off = key0 - pg * p.page_size + key_l;
-    const uint8_t* row = p.k8 + id * p.k_sp + (int64_t)off * p.k_sr + half * 64;
+    const int off = key0 - pg * p.page_size;
+    const uint8_t* rows = p.k8 + id * p.k_sp + (int64_t)off * p.k_sr;
+    const uint32_t dst = lds0 + (uint32_t)buf * kTileBufB + (uint32_t)wave * kIdxSlotB;
 #pragma unroll
-    for (int j = 0; j < 4; j++) kb[j] = *(const u32x4*)(row + j * 16);
-    ks = p.k_scale[id * p.ks_sp + off];
+    for (int i = 0; i < 4; i++) dma16_sv(rows + i * 8 * p.k_sr, src_off[i & 1], dst + i * 1024);
+    dma4_sv_lo32(p.k_scale + id * p.ks_sp + off, (uint32_t)lane * 4, dst + 32 * kIdxDim);
   };
-  u32x4 kb[4], kn[4];
-  float ks = 0.f, ks_n = 0.f;
-  int blk = (int)blockIdx.x * 4 + wave;
-  if (blk < blocks) load_block(blk, kn, ks_n);
-  MLA_WAIT_VMCNT(0);
-  lds_barrier();
+  const int stride = (int)gridDim.x;
+  int stage = (int)blockIdx.x;
+  copy_stage(stage, 0);
 
-  const int row_off = key_l * kIdxDim, swz = (key_l >> 1) & 7;   // (rows 32 apart share the swizzle)
-  for (; blk < blocks; blk += stride) {
+  long qa[2][8];
+  float wr[2][16];
 #pragma unroll
-    for (int j = 0; j < 4; j++) kb[j] = kn[j];
-    ks = ks_n;
-    if (blk + stride < blocks) load_block(blk + stride, kn, ks_n);
-    const int key0 = blk * 32;
-#pragma unroll 1
-    for (int i = 0; i < nt; i++) {
-      const int limit = lim0 + i;
-      if (key0 >= limit || limit <= p.skip_up_to) continue;
-      const char* qp = lds + i * 64 * kIdxDim + row_off;
-      f32x16 c0, c1;
+  for (int hb = 0; hb < 2; hb++) {
+    const uint8_t* qrow = p.q8 + t * p.q_st + (int64_t)(hb * 32 + key_l) * p.q_sh + half * 64;
 #pragma unroll
-      for (int r = 0; r < 16; r++) { c0[r] = 0.f; c1[r] = 0.f; }
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const int gr = ((4 * half + j) ^ swz) << 4;
-        const u32x4 a0 = *(const u32x4*)(qp + gr), a1 = *(const u32x4*)(qp + 32 * kIdxDim + gr), v = kb[j];
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-          const long bop = (long)(((uint64_t)v[2 * h + 1] << 32) | v[2 * h]);
-          c0 = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8((long)(((uint64_t)a0[2 * h + 1] << 32) | a0[2 * h]), bop, c0, 0, 0, 0);
-          c1 = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8((long)(((uint64_t)a1[2 * h + 1] << 32) | a1[2 * h]), bop, c1, 0, 0, 0);
-        }
-      }
-      const char* wp = lds + kTileWOff + i * 256 + half * 16;
-      float acc = 0.f;
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const f32x4 w0 = *(const f32x4*)(wp + q * 32), w1 = *(const f32x4*)(wp + 128 + q * 32);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          acc = fmaf(w0[e], relu(c0[q * 4 + e]), acc);
-          acc = fmaf(w1[e], relu(c1[q * 4 + e]), acc);
-        }
-      }
-      acc += xor32(acc);
-      if (half == 0) p.logits[(int64_t)(q0 + tok0 + i) * p.l_st + key0 + key_l] = key0 + key_l < limit ? acc * ks : -INFINITY;
+    for (int j = 0; j < 4; j++) {
+      const u32x4 v = *(const u32x4*)(qrow + j * 16);
+      qa[hb][2 * j] = (long)(((uint64_t)v[1] << 32) | v[0]);
+      qa[hb][2 * j + 1] = (long)(((uint64_t)v[3] << 32) | v[2]);
     }
+#pragma unroll
+    for (int r = 0; r < 16; r++) wr[hb][r] = p.weights[t * p.w_st + hb * 32 + 8 * (r >> 2) + 4 * half + (r & 3)];
+  }
+  if (p.q_scale) {
+    float qs[2][16];
+#pragma unroll
+    for (int hb = 0; hb < 2; hb++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) qs[hb][r] = p.q_scale[t * p.qs_st + hb * 32 + 8 * (r >> 2) + 4 * half + (r & 3)];
+#pragma unroll
+    for (int hb = 0; hb < 2; hb++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) wr[hb][r] *= qs[hb][r];
+  }
+
+  const int rd_row = key_l * kIdxDim, rd_swz = (key_l >> 1) & 7;
+  float* const row = p.logits + t * p.l_st;
+  f32x16 c[2][2] = {};                                       // sums of a block's heads: of even blocks and of odd ones
+  auto fold = [&](int r, const f32x16 (&of)[2], float& acc) {
+    acc = fmaf(wr[0][r], relu(of[0][r]), acc);
+    acc = fmaf(wr[1][r], relu(of[1][r]), acc);
+  };
+  // Block j of the stage in buffer `buf` through the matrix unit, and beside it the block before it through the vector unit, four
+  // instructions to an MFMA; returns the latter's sum over the lane's heads.
+  auto block = [&](int j, int buf) {
+    const char* sp = lds + buf * kTileBufB + j * kIdxSlotB + rd_row;
+    f32x16 (&now)[2] = c[j & 1], (&was)[2] = c[(j & 1) ^ 1];
+    u32x4 kb[4];
+#pragma unroll
+    for (int g = 0; g < 4; g++) kb[g] = *(const u32x4*)(sp + (((4 * half + g) ^ rd_swz) << 4));
+#pragma unroll
+    for (int r = 0; r < 16; r++) { now[0][r] = 0.f; now[1][r] = 0.f; }
+    float acc = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const int g = i >> 1;
+      const u32x4 v = kb[g >> 1];
+      const long bop = (g & 1) ? (long)(((uint64_t)v[3] << 32) | v[2]) : (long)(((uint64_t)v[1] << 32) | v[0]);
+      now[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(qa[i & 1][g], bop, now[i & 1], 0, 0, 0);
+      fold(i, was, acc);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    return acc;
+  };
+  // The logits of an even block, in half 0, and of the odd one behind it, in half 1, from their sums over the lanes' heads
+  auto pair = [&](float even, float odd, float scale) {
+    const u32x2 s = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(even), __float_as_uint(odd), false, false));
+    return (__uint_as_float(s[0]) + __uint_as_float(s[1])) * scale;
+  };
+  auto store_pair = [&](int st, int j, float logit) {
+    const int key = (st * kTileBlocks + j) * 32 + lane;
+    if ((key & ~31) < limit) row[key] = key < limit ? logit : -INFINITY;
+  };
+  constexpr int kNone = 1 << 23;                             // a stage behind all keys
+  int before = kNone;
+  float even = 0.f, first = 0.f, scale = 0.f;
+  const char* const scales = lds + half * kIdxSlotB + 32 * kIdxDim + key_l * 4;
+  for (int buf = 0; stage < stages; stage += stride, buf ^= 1) {
+    MLA_WAIT_VMCNT(0);
+    lds_barrier();                                           // the stage is here, everyone is done with the other buffer
+    if (stage + stride < stages) copy_stage(stage + stride, buf ^ 1);
+    if (limit > 0) {
+      float odd = block(0, buf);
+      const float second = pair(even, odd, scale);
+      store_pair(before, 0, first);
+      store_pair(before, 2, second);
+      before = stage;
+      scale = *(const float*)(scales + buf * kTileBufB);
+      even = block(1, buf);
+      odd = block(2, buf);
+      first = pair(even, odd, scale);
+      scale = *(const float*)(scales + buf * kTileBufB + 2 * kIdxSlotB);
+      even = block(3, buf);
+    }
+  }
+  if (before != kNone) {
+    float odd = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; r++) fold(r, c[1], odd);
+    store_pair(before, 0, first);
+    store_pair(before, 2, pair(even, odd, scale));
   }
 }
 
@@ -600,18 +645,15 @@ static int indexer_scores_impl(const void* q8, int64_t q_stride_t, int64_t q_str
   p.batch = batch; p.max_q_len = max_q_len; p.num_heads = num_heads; p.page_size = page_size; p.num_pages = num_pages;
   p.logits = logits; p.l_st = logits_stride; p.skip_up_to = skip_up_to;
   if (max_q_len >= kTileMinQ) {
-    // about 8192 workgroups (eight rounds of four per CU, those of the tokens that are skipped and of the shorter requests
+    // about 6144 workgroups (eight rounds of three per CU, those of the tokens that are skipped and of the shorter requests
     // among them, which end at once), so that the short ones at the start of a prompt even out
     const int64_t groups = (int64_t)batch * ((max_q_len + kTileTok - 1) / kTileTok);
-    int64_t split = (8192 + groups - 1) / groups;
-    const int64_t most = (max_seq_len + 127) / 128;           // a block per wavefront
-    split = split > 16 ? 16 : split;
+    int64_t split = (6144 + groups - 1) / groups;
+    const int64_t most = (max_seq_len + 32 * kTileBlocks - 1) / (32 * kTileBlocks);
     split = split > most ? most : split;
     MLA_REQUIRE(batch <= 65535, MLA_ERR_SHAPE, "dsa_indexer_scores_fp8: too many requests");
-    const int rc = ensure_dynamic_lds((const void*)dsa_indexer_tile_kernel, kTileLdsB, "dsa_indexer_scores_fp8");
-    if (rc != MLA_OK) return rc;
     hipLaunchKernelGGL(dsa_indexer_tile_kernel, dim3((unsigned)split, (unsigned)((max_q_len + kTileTok - 1) / kTileTok), (unsigned)batch),
-                       dim3(256), kTileLdsB, stream, p);
+                       dim3(256), 0, stream, p);
     return check_launch("dsa_indexer_tile_kernel");
   }
   // two workgroups per compute unit (what their LDS rings allow), never more wavefronts than 32-key blocks
