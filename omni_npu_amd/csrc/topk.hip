@@ -659,6 +659,7 @@ __device__ __forceinline__ void finish_slice(const TopkParams& p, const TopkRow&
   const int d = select_digit<kTopkThreads>(sh.hist, sh.scratch, k, &above);
   const int need = k - above, m = sh.hist[d];
   const bool in_lds = m <= kMwCandLds;
+  __syncthreads();                                           // (everyone has read m: what finds the threshold begins with clearing the histogram)
   auto each_key = [&](auto&& f) {                            // f(image, position) of the boundary bin's keys
 #pragma unroll
     for (int j = 0; j < 2; j++)
