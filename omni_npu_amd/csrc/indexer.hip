@@ -433,13 +433,14 @@ __device__ __forceinline__ void quant_rows(const QuantRows& q, int64_t r0) {
     float scale = amax > 0.f ? amax / 448.f : 1.f;
     // x / scale by the reciprocal and one correction with its exact remainder: the same e4m3 numbers as by the division, for every bf16
     // x and amax (checked one by one, with reciprocals an ulp off to either side), in three instructions instead of a dozen.  For maxima
-    // from 2^-50 to 2^66, and zero; nothing near the ends of fp32, and no NaN
+    // from 2^-50 to 2^66, and zero; nothing near the ends of fp32, and no NaN.  (The remainder is taken with its sign turned, so that minus
+    // zero stays what it is)
     if (__builtin_amdgcn_ballot_w64(mx != 0 && mx - ((127 - 50) << 7) > (116 << 7)) == 0) {
       const float rcp = __builtin_amdgcn_rcpf(scale);
 #pragma unroll
       for (int e = 0; e < 8; e++) {
         const float q0 = x[e] * rcp;
-        y[e] = __builtin_amdgcn_fmed3f(__builtin_fmaf(__builtin_fmaf(-q0, scale, x[e]), rcp, q0), -448.f, 448.f);
+        y[e] = __builtin_amdgcn_fmed3f(__builtin_fmaf(-__builtin_fmaf(q0, scale, -x[e]), rcp, q0), -448.f, 448.f);
       }
     } else {                                                  // (NaNs count for nothing in the maximum)
       amax = 0.f;

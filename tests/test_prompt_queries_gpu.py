@@ -87,3 +87,11 @@ def test_a_nan_counts_for_nothing_in_a_row_s_maximum(dev):
     for x, a, b in zip((rows, clean), got, sc):
         K.quant_rows_fp8(x.to(dev), a, b)
     assert torch.equal(sc[0], sc[1]) and torch.equal(got[0][~rows.isnan().to(dev)], got[1][~rows.isnan().to(dev)])
+
+
+def test_zeros_keep_their_sign(dev):
+    rows = torch.randn(4, 128, generator=torch.Generator().manual_seed(2)).bfloat16()
+    rows[1, ::2], rows[1, 1::4], rows[2] = -0.0, 0.0, -0.0
+    got, sc = torch.empty(4, 128, dtype=torch.uint8, device=dev), torch.empty(4, device=dev)
+    K.quant_rows_fp8(rows.to(dev), got, sc)
+    assert torch.equal(got.cpu() >> 7, torch.signbit(rows.float()).to(torch.uint8))
