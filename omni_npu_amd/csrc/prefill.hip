@@ -504,7 +504,9 @@ __device__ __forceinline__ void pf_block(const PrefillParams& p, char* lds, cons
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (row_ok) {
     const int64_t lse_at = tq * p.num_heads + head + (kSplit ? blk.piece * p.lse_piece : 0);
-    if ((kSplit || p.lse) && half == 0) p.lse[lse_at] = l_tot > 0.f ? (m_run + fast_log2(l_tot)) * kLn2 : -INFINITY;
+    // (kSplit: a NaN among the scores of a piece is one in its log-sum-exp, by which the merge knows it)
+    if ((kSplit || p.lse) && half == 0)
+      p.lse[lse_at] = l_tot > 0.f || (kSplit && l_tot != l_tot) ? (m_run + fast_log2(l_tot)) * kLn2 : -INFINITY;
     const int64_t o = tq * p.o_st + (int64_t)head * p.o_sh + 4 * half + (kSplit ? blk.piece * p.o_piece : 0);
     if (kSplit && tiles <= first_tile) return;               // (a piece without keys: the merge reads its lse only)
 #pragma unroll
@@ -685,7 +687,7 @@ __global__ __launch_bounds__(256) void mla_prefill_merge_kernel(const float* par
   float mx = mine;
 #pragma unroll
   for (int d = 16; d >= 1; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 32));
-  const float w = mx > -INFINITY ? fast_exp2((mine - mx) * kLog2e) : 0.f;
+  const float w = mine == -INFINITY ? 0.f : fast_exp2((mine - mx) * kLog2e);   // (a piece with a NaN: NaN, and the whole row)
   float total = w;
 #pragma unroll
   for (int d = 16; d >= 1; d >>= 1) total += __shfl_xor(total, d, 32);

@@ -49,6 +49,22 @@ def test_pieces_give_what_one_piece_gives(dev, n, q_lens, ctx, pieces):
     assert torch.equal(run(pieces, torch.bfloat16)[0], got.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("pieces", [1, 2, 32])
+def test_a_nan_among_the_scores_reaches_the_rows_that_see_it(dev, pieces):
+    """A query row of NaNs (every piece of it is one) and a key (one piece of the rows that see it, none of the others)."""
+    g = torch.Generator(device=dev).manual_seed(4)
+    q_lens, ctx, n = [40, 20], [200, 700], 8
+    t, cu = sum(q_lens), _cu(q_lens, dev)
+    q = torch.randn(t, n, 192, generator=g, device=dev).to(torch.bfloat16)
+    own, context = _rows(dev, t, n, g), (*_rows(dev, sum(ctx), n, g), _cu(ctx, dev))
+    q[3, 2], own[0][10, 5, 7], context[0][200 + 333, 1, 0] = float("nan"), float("nan"), float("nan")
+    out = torch.zeros(t, n, 128, device=dev)
+    K.prefill_varlen(q[..., :128], q[..., 128:], *own, cu, cu, max(q_lens), 0.07, True, out, context=context, long=False, pieces=pieces)
+    want = torch.zeros(t, n, dtype=torch.bool)
+    want[3, 2], want[10:40, 5], want[40:, 1] = True, True, True
+    assert torch.equal(out.isnan().any(2).cpu(), want) and torch.equal(out.isnan().all(2).cpu(), want)
+
+
 def test_the_rule_cuts_where_the_chip_would_stand_idle(dev):
     assert K.prefill_pieces(100, 2, 85, 16, 4756 + 50) >= 8    # 32 blocks of sixty tiles
     assert K.prefill_pieces(2048, 4, 2048, 128, 70000) == 1    # more blocks than run at once
