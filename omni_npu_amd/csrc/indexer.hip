@@ -398,13 +398,15 @@ __device__ __forceinline__ void quant_rows(const QuantRows& q, int64_t r0) {
   const bool wide = (((uintptr_t)src | (uintptr_t)(src_stride * 2)) & 15) == 0;
   int64_t slot[kRows];
   u32x4 raw[kRows];
+  float w_of[kRows];
 #pragma unroll
   for (int i = 0; i < kRows; i++) {
     const int64_t r = r0 + i * 16;
-    slot[i] = r < rows ? (slots ? slots[r] : r) : -1;
-    if (slot[i] >= num_pages * page_size) slot[i] = -1;
+    slot[i] = -1;
+    w_of[i] = 0.f;
     raw[i] = u32x4{0u, 0u, 0u, 0u};
-    if (slot[i] >= 0) {
+    if (r < rows) {
+      // (a row without a slot is read too: behind its slot it came a round trip later)
       const __bf16* at = src + r * src_stride + l16 * 8;
       if (wide) {
         raw[i] = *(const u32x4*)at;
@@ -412,7 +414,14 @@ __device__ __forceinline__ void quant_rows(const QuantRows& q, int64_t r0) {
 #pragma unroll
         for (int e = 0; e < 4; e++) raw[i][e] = *(const uint32_t*)(at + 2 * e);
       }
+      slot[i] = slots ? slots[r] : r;
+      if (w_out) {
+        const int32_t tk = kToken ? (int32_t)blockIdx.x : (int32_t)((uint32_t)r / (uint32_t)heads);       // (rows < 2^31)
+        const int64_t from = tk * w_st + ((int32_t)r - tk * heads);
+        w_of[i] = w_f32 ? ((const float*)w_in)[from] : (float)((const __bf16*)w_in)[from];
+      }
     }
+    if (slot[i] >= num_pages * page_size) slot[i] = -1;
   }
 #pragma unroll
   for (int i = 0; i < kRows; i++) {
@@ -468,11 +477,7 @@ __device__ __forceinline__ void quant_rows(const QuantRows& q, int64_t r0) {
     }
     if (l16 == 0) {
       if (dscale) dscale[pg * s_sp + off] = scale;
-      if (w_out) {
-        const int32_t tk = kToken ? (int32_t)blockIdx.x : (int32_t)((uint32_t)r / (uint32_t)heads);       // (rows < 2^31)
-        const int64_t at = tk * w_st + ((int32_t)r - tk * heads);
-        w_out[r] = (w_f32 ? ((const float*)w_in)[at] : (float)((const __bf16*)w_in)[at]) * scale;
-      }
+      if (w_out) w_out[r] = w_of[i] * scale;
     }
   }
 }

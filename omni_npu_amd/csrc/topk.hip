@@ -732,7 +732,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void dsa_topk_hist_kernel(const To
   if (!r.live) return;
   const int n = r.n, k = p.t.k;
   if (p.t.counts && s == 0 && tid == 0) p.t.counts[r.t] = n < k ? n : k;
-  if (n <= k) {                                            // everything is selected
+  if (__builtin_expect(n <= k, 0)) {                       // everything is selected
     if (s == 0) {
       const TopkSink out = topk_sink(p.t, r.b, r.t);
       for (int i = tid; i < k; i += kTopkThreads) {
@@ -774,7 +774,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void dsa_topk_hist_kernel(const To
     for (int e = 0; e < 4; e++)
       if (ks.base + j * 256 + e < n) atomicAdd(&sh.hist[linear_bin(ks.v[j][e], scale, shift)], 1);
   __syncthreads();
-  if (n <= kSliceKeys) {
+  if (__builtin_expect(n <= kSliceKeys, 0)) {
     finish_slice(p.t, r, ks, scale, shift, sh);
     return;
   }
