@@ -50,17 +50,6 @@ constexpr int kPlanBlk = 32;
 constexpr int kPlanSegCost = 8;
 __device__ __forceinline__ int plan_work_units(int len) { return len > 0 ? (len + kPlanBlk - 1) / kPlanBlk + kPlanSegCost : 0; }
 
-// Inclusive sum over the 64 lanes by data-parallel-primitive moves (no LDS round trips): shifts inside the rows of 16, then lane 15 of
-// rows 0 and 2 into rows 1 and 3, then lane 31 into the upper half.
-__device__ __forceinline__ int wave_incl_scan_dpp(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
-  return v;
-}
 typedef __attribute__((address_space(4))) const int32_t* ConstI32Ptr;   // scalar (constant-cache) loads
 
 // How many chunks the work is cut into.  The host names the most a launch can use: a workgroup has a CU to itself (its LDS

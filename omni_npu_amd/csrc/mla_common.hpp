@@ -174,6 +174,18 @@ __device__ __forceinline__ bf16x4 lds_read_tr16(const void* lds_addr) {
 // Wait until at most n of this wave's global loads (LDS copies included) are outstanding.
 #define MLA_WAIT_VMCNT(n) asm volatile("s_waitcnt vmcnt(" #n ")" ::: "memory")
 
+// Inclusive sum over the 64 lanes by data-parallel-primitive moves (no LDS round trips): shifts inside the rows of 16, then lane 15 of
+// rows 0 and 2 into rows 1 and 3, then lane 31 into the upper half.
+__device__ __forceinline__ int wave_incl_scan_dpp(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return v;
+}
+
 // Workgroup barrier without the global-memory release fence of __syncthreads(): that fence waits for
 // every outstanding global load, which would serialise the prefetch of the next K tile.  All data
 // exchanged across the barrier lives in LDS; the caller waits for its own LDS copies (vmcnt) first.

@@ -38,19 +38,15 @@ __device__ int select_digit(int* hist, int* scratch, int need, int* above) {
 #pragma unroll
   for (int i = 0; i < kOwn; i++) { c[i] = hist[b0 - i]; v += c[i]; }
   // inclusive scan over threads (descending bins)
+  constexpr int kWaves = kThreads / 64;
   const int lane = tid & 63, w = tid >> 6;
-  int s = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int n = __shfl_up(s, o, 64);
-    if (lane >= o) s += n;
-  }
+  const int s = wave_incl_scan_dpp(v);
   if (lane == 63) scratch[w] = s;
   __syncthreads();
   int base = 0;
-  for (int i = 0; i < w; i++) base += scratch[i];
+#pragma unroll
+  for (int i = 0; i < kWaves; i++) base += i < w ? scratch[i] : 0;
   const int incl = base + s, excl = incl - v;              // keys in bins above this thread's: excl
-  __syncthreads();
   if (excl < need && need <= incl) {                       // exactly one thread
     int sum = excl;
     bool found = false;
@@ -60,11 +56,9 @@ __device__ int select_digit(int* hist, int* scratch, int need, int* above) {
       sum += c[i];
     }
   }
-  __syncthreads();
-  const int d = scratch[32];
+  __syncthreads();                                         // (scratch[32] is written again behind the next call's first barrier only)
   *above = scratch[33];
-  __syncthreads();
-  return d;
+  return scratch[32];
 }
 
 struct TopkParams {
@@ -89,16 +83,17 @@ struct TopkSink {
     const uint32_t up = (uint32_t)__shfl_xor((int)nib, 1, 64);
     if ((i & 4) == 0 && i < n) mask[i >> 3] = (uint8_t)(nib | (up << 4));
   }
+  __device__ __forceinline__ int32_t row_of(int pos) const {
+    int pg = pos / page_size;
+    const int off = pos - pg * page_size;
+    pg = pg < max_blocks ? pg : max_blocks - 1;
+    int64_t blk = bt[pg];
+    blk = blk < 0 ? 0 : (blk >= num_pages ? num_pages - 1 : blk);
+    return (int32_t)(blk * page_size + off);
+  }
   __device__ __forceinline__ void put(int at, int pos) const {
     out[at] = pos;
-    if (rows) {
-      int pg = pos / page_size;
-      const int off = pos - pg * page_size;
-      pg = pg < max_blocks ? pg : max_blocks - 1;
-      int64_t blk = bt[pg];
-      blk = blk < 0 ? 0 : (blk >= num_pages ? num_pages - 1 : blk);
-      rows[at] = (int32_t)(blk * page_size + off);
-    }
+    if (rows) rows[at] = row_of(pos);
   }
 };
 __device__ __forceinline__ TopkSink topk_sink(const TopkParams& p, int b, int t) {
@@ -587,22 +582,27 @@ struct TopkMwParams {
   int32_t slices;
   int32_t* hist_part;                                      // [tokens][slices][kBins]
   float* range;                                            // [tokens][2]: scale, shift
-  int32_t* meta;                                           // [tokens][4]: candidate count, boundary bin, need, -
+  int32_t* meta;                                           // [tokens][4]: keys of the boundary bin, -, how many of them are picked, -
   int32_t* counts;                                         // [tokens][slices][kMwWaves] sure picks
   uint32_t* cand;                                          // [tokens][cand_cap][2]: ordered image, position
   int64_t cand_cap;
+  uint32_t inv_slices, inv_q;                              // 2^32 / d + 1: the high words of products divide numbers below 2^12 exactly
+  int32_t per_xcd;                                         // workgroups of an XCD, or 0 where they are not whole tokens
 };
 
 struct TopkRow { const float* x; int n, slot, b, t; bool live; };
-__device__ __forceinline__ TopkRow topk_row(const TopkParams& p, int slot) {
+__device__ __forceinline__ TopkRow topk_row(const TopkMwParams& mw, int slot) {
+  const TopkParams& p = mw.t;
   TopkRow r;
-  const int b = slot / p.max_q_len;
+  const int b = p.max_q_len == 1 ? slot : (int)__umulhi((uint32_t)slot, mw.inv_q);
   const int ti = slot - b * p.max_q_len;
-  int q0, qlen;
-  if (p.qsl) { q0 = p.qsl[b]; qlen = p.qsl[b + 1] - q0; } else { q0 = b * p.max_q_len; qlen = p.max_q_len; }
+  int len = p.seq_lens[b], q0 = b * p.max_q_len, q1 = q0 + p.max_q_len;
+  if (p.qsl) { q0 = p.qsl[b]; q1 = p.qsl[b + 1]; }
+  asm volatile("" : "+s"(len), "+s"(q0), "+s"(q1));        // (one round trip for all: the length is not asked for behind a test of the others)
+  const int qlen = q1 - q0;
   r.live = ti < qlen;
   const int t = q0 + ti;
-  int n = p.seq_lens[b] - qlen + ti + 1;                   // visible keys
+  int n = len - qlen + ti + 1;                             // visible keys
   r.n = n < 0 ? 0 : n;
   r.x = p.logits + (int64_t)t * p.l_st;
   r.b = b;
@@ -616,14 +616,13 @@ __device__ __forceinline__ TopkRow topk_row(const TopkParams& p, int slot) {
 // of the chain leaves for the next (slice histograms, candidates, counts, the logits themselves) is read through the XCD
 // that wrote it.
 struct SliceOf { int s, slot; };
-__device__ __forceinline__ SliceOf slice_of_workgroup() {
+__device__ __forceinline__ SliceOf slice_of_workgroup(const TopkMwParams& p) {
   SliceOf r{(int)blockIdx.x, (int)blockIdx.y};
-  const uint32_t total = gridDim.x * gridDim.y;
-  if ((total & 7) == 0 && ((total >> 3) % gridDim.x) == 0) {
-    const uint32_t lin = blockIdx.x + gridDim.x * blockIdx.y;
-    const uint32_t nl = (lin & 7) * (total >> 3) + (lin >> 3);
-    r.s = (int)(nl % gridDim.x);
-    r.slot = (int)(nl / gridDim.x);
+  if (p.per_xcd > 0) {
+    const uint32_t lin = blockIdx.x + (uint32_t)p.slices * blockIdx.y;
+    const uint32_t nl = (lin & 7) * (uint32_t)p.per_xcd + (lin >> 3);
+    r.slot = (int)__umulhi(nl, p.inv_slices);
+    r.s = (int)nl - r.slot * p.slices;
   }
   return r;
 }
@@ -649,11 +648,33 @@ __device__ __forceinline__ SliceKeys load_slice(const float* x, int n, int s, in
   return k;
 }
 
+// The cache rows of this thread's keys (four neighbours share a page of a multiple of four), asked for long before the picks are known;
+// where pages are others, put looks every pick up.
+struct SliceRows { int32_t first[2]; bool known; };
+__device__ __forceinline__ SliceRows slice_rows(const TopkSink& out, const SliceKeys& ks, int n) {
+  SliceRows r{{0, 0}, out.rows != nullptr && (out.page_size & 3) == 0};
+  if (r.known) {
+#pragma unroll
+    for (int j = 0; j < 2; j++) r.first[j] = out.row_of(ks.base + j * 256 < n ? ks.base + j * 256 : 0);
+  }
+  return r;
+}
+__device__ __forceinline__ void put_pick(const TopkSink& out, const SliceKeys& ks, const SliceRows& rows, int j, int e, int at) {
+  if (rows.known) {
+    out.out[at] = ks.base + j * 256 + e;
+    out.rows[at] = rows.first[j] + e;
+  } else {
+    out.put(at, ks.base + j * 256 + e);
+  }
+}
+
 struct SliceLds { int hist[kBins]; int scratch[64]; uint32_t cand_u[kMwCandLds], cand_i[kMwCandLds]; };
 
 // All of a row's keys are this workgroup's, and their histogram is in sh.hist: the picks.
 __device__ __forceinline__ void finish_slice(const TopkParams& p, const TopkRow& r, const SliceKeys& ks, float scale, float shift, SliceLds& sh) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, n = r.n, k = p.k;
+  const TopkSink out = topk_sink(p, r.b, r.t);
+  const SliceRows rows = slice_rows(out, ks, n);
   if (tid == 0) sh.scratch[40] = 0;
   int above;
   const int d = select_digit<kTopkThreads>(sh.hist, sh.scratch, k, &above);
@@ -685,7 +706,6 @@ __device__ __forceinline__ void finish_slice(const TopkParams& p, const TopkRow&
                                   sh.scratch, &prefix, &pos_thresh);
   else
     radix_threshold<kTopkThreads>(each_key, need, sh.hist, sh.scratch, &prefix, &pos_thresh);
-  const TopkSink out = topk_sink(p, r.b, r.t);
   const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   bool tk[2][4];
   int at[2], mine = 0;
@@ -715,7 +735,7 @@ __device__ __forceinline__ void finish_slice(const TopkParams& p, const TopkRow&
     int to = o + at[j];
 #pragma unroll
     for (int e = 0; e < 4; e++)
-      if (tk[j][e]) { if (to < k) out.put(to, ks.base + j * 256 + e); to++; }
+      if (tk[j][e]) { if (to < k) put_pick(out, ks, rows, j, e, to); to++; }
     if (out.mask) out.put_bits(ks.base + j * 256, n, tk[j][0] | tk[j][1] << 1 | tk[j][2] << 2 | tk[j][3] << 3);
   }
 }
@@ -726,9 +746,9 @@ __global__ __launch_bounds__(kTopkThreads, 8) void dsa_topk_hist_kernel(const To
   __shared__ SliceLds sh;
   __shared__ float fscratch[2 * kMwWaves];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const SliceOf so = slice_of_workgroup();
+  const SliceOf so = slice_of_workgroup(p);
   const int s = so.s;
-  const TopkRow r = topk_row(p.t, so.slot);
+  const TopkRow r = topk_row(p, so.slot);
   if (!r.live) return;
   const int n = r.n, k = p.t.k;
   if (p.t.counts && s == 0 && tid == 0) p.t.counts[r.t] = n < k ? n : k;
@@ -766,7 +786,6 @@ __global__ __launch_bounds__(kTopkThreads, 8) void dsa_topk_hist_kernel(const To
   if (s == 0 && tid == 0) {
     p.range[r.slot * 2] = scale;
     p.range[r.slot * 2 + 1] = shift;
-    p.meta[r.slot * 4] = 0;                                // candidate counter for the gather launch
   }
 #pragma unroll
   for (int j = 0; j < 2; j++)
@@ -784,28 +803,44 @@ __global__ __launch_bounds__(kTopkThreads, 8) void dsa_topk_hist_kernel(const To
 
 template <int kVec>
 __global__ __launch_bounds__(kTopkThreads) void dsa_topk_gather_kernel(const TopkMwParams p) {
-  __shared__ int hist[kBins];
+  __shared__ __attribute__((aligned(16))) int hist[kBins], before[kBins];   // keys of a bin in the row; in the slices before this one
   __shared__ int scratch[64];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const SliceOf so = slice_of_workgroup();
+  const SliceOf so = slice_of_workgroup(p);
   const int s = so.s;
-  const TopkRow r = topk_row(p.t, so.slot);
+  const TopkRow r = topk_row(p, so.slot);
   if (!r.live || r.n <= p.t.k || r.n <= kSliceKeys || s * kSliceKeys >= r.n) return;
   const int n = r.n;
   const int live_slices = (n + kSliceKeys - 1) / kSliceKeys;
-  // all loads first: the slice histograms of the token (two bins per thread), the bin map, this slice
-  const int32_t* hp = p.hist_part + (int64_t)r.slot * p.slices * kBins;
-  int c0 = 0, c1 = 0;
-  for (int j = 0; j < live_slices; j++) { c0 += hp[j * kBins + tid]; c1 += hp[j * kBins + kTopkThreads + tid]; }
-  const float scale = p.range[r.slot * 2], shift = p.range[r.slot * 2 + 1];
+  // all loads first: the slice histograms of the token (two bins per thread, eight slices at a time: added up one after the
+  // other they were eight round trips in a row), this slice, the bin map
+  const u32x2* hp = (const u32x2*)(p.hist_part + (int64_t)r.slot * p.slices * kBins) + tid;
+  u32x2 part[8], sum = {0u, 0u}, prev = {0u, 0u};
+  auto ask = [&](int j0) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) part[j] = hp[(j0 + j < live_slices ? j0 + j : live_slices - 1) * (kBins / 2)];
+  };
+  auto add = [&](int j0) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      sum += j0 + j < live_slices ? part[j] : u32x2{0u, 0u};
+      prev += j0 + j < s ? part[j] : u32x2{0u, 0u};
+    }
+  };
+  ask(0);
   const SliceKeys ks = load_slice<kVec>(r.x, n, s, w, lane);
-  hist[tid] = c0;
-  hist[kTopkThreads + tid] = c1;
+  const float scale = p.range[r.slot * 2], shift = p.range[r.slot * 2 + 1];
+  add(0);
+  if (live_slices > 8) { ask(8); add(8); }
+  *(u32x2*)(hist + 2 * tid) = sum;
+  *(u32x2*)(before + 2 * tid) = prev;
+  if (tid == 0) scratch[40] = 0;
   __syncthreads();
   int above;
   const int d = select_digit<kTopkThreads>(hist, scratch, p.t.k, &above);
-  if (s == 0 && tid == 0) { p.meta[r.slot * 4 + 1] = d; p.meta[r.slot * 4 + 2] = p.t.k - above; }
-  uint32_t* cand = p.cand + (int64_t)r.slot * p.cand_cap * 2;
+  if (s == 0 && tid == 0) { p.meta[r.slot * 4] = hist[d]; p.meta[r.slot * 4 + 2] = p.t.k - above; }
+  // this slice's keys of the boundary bin, behind those of the slices before it
+  u32x2* cand = (u32x2*)p.cand + (int64_t)r.slot * p.cand_cap + before[d];
   int cnt = 0;
 #pragma unroll
   for (int j = 0; j < 2; j++)
@@ -815,16 +850,11 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_gather_kernel(const Top
       if (i < n) {
         const int bn = linear_bin(ks.v[j][e], scale, shift);
         cnt += bn > d;
-        if (bn == d) {
-          const int slot = atomicAdd(&p.meta[r.slot * 4], 1);
-          cand[2 * (int64_t)slot] = ordered_bits(ks.v[j][e]);
-          cand[2 * (int64_t)slot + 1] = (uint32_t)i;
-        }
+        if (bn == d) cand[atomicAdd(&scratch[40], 1)] = u32x2{ordered_bits(ks.v[j][e]), (uint32_t)i};
       }
     }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
-  if (lane == 0) p.counts[((int64_t)r.slot * p.slices + s) * kMwWaves + w] = cnt;
+  cnt = wave_incl_scan_dpp(cnt);
+  if (lane == 63) p.counts[((int64_t)r.slot * p.slices + s) * kMwWaves + w] = cnt;
 }
 
 template <int kVec>
@@ -834,9 +864,9 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_write_kernel(const Topk
   __shared__ uint32_t cand_u[kMwCandLds];
   __shared__ uint32_t cand_i[kMwCandLds];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const SliceOf so = slice_of_workgroup();
+  const SliceOf so = slice_of_workgroup(p);
   const int s = so.s;
-  const TopkRow r = topk_row(p.t, so.slot);
+  const TopkRow r = topk_row(p, so.slot);
   const int n = r.n, k = p.t.k;
   if (!r.live || n <= k || n <= kSliceKeys || s * kSliceKeys >= n) return;
   const TopkSink out = topk_sink(p.t, r.b, r.t);
@@ -859,6 +889,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_write_kernel(const Topk
   for (int q = 0; q < 4; q++) { const int j = lane + q * 64; part += j < mine ? cn[j] : 0; }
   const int m = p.meta[r.slot * 4], need = p.meta[r.slot * 4 + 2];
   const SliceKeys ks = load_slice<kVec>(r.x, n, s, w, lane);
+  const SliceRows rows = slice_rows(out, ks, n);
 #pragma unroll
   for (int q = 0; q < kMwCandLds / kTopkThreads; q++) { cand_u[tid + q * kTopkThreads] = cu[q]; cand_i[tid + q * kTopkThreads] = ci[q]; }
   __syncthreads();
@@ -884,9 +915,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_write_kernel(const Topk
     const uint32_t u = in_lds ? cand_u[j] : cand[2 * (int64_t)j], ps = in_lds ? cand_i[j] : cand[2 * (int64_t)j + 1];
     part += (int)ps < wlo && ((u > prefix) || (u == prefix && ps <= pos_thresh));
   }
-#pragma unroll
-  for (int sh = 32; sh >= 1; sh >>= 1) part += __shfl_xor(part, sh, 64);
-  int o = part;
+  int o = __builtin_amdgcn_readlane(wave_incl_scan_dpp(part), 63);
   const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
 #pragma unroll
   for (int j = 0; j < 2; j++) {
@@ -904,7 +933,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_write_kernel(const Topk
     int at = o + before;
 #pragma unroll
     for (int e = 0; e < 4; e++)
-      if (tk[e]) { if (at < k) out.put(at, i + e); at++; }
+      if (tk[e]) { if (at < k) put_pick(out, ks, rows, j, e, at); at++; }
     o += total;
     if (out.mask) out.put_bits(i, n, tk[0] | tk[1] << 1 | tk[2] << 2 | tk[3] << 3);
   }
@@ -1029,6 +1058,10 @@ static int topk_impl(const float* logits, int64_t logits_stride, const int32_t* 
   m.counts = (int32_t*)w; w += (size_t)tokens * kMaxSlices * kMwWaves * 4;
   m.cand = (uint32_t*)w;
   m.cand_cap = logits_stride;
+  const int64_t wgs = tokens * slices;                     // (fewer than 256 tokens of at most 16 slices)
+  m.inv_slices = (uint32_t)((1ull << 32) / slices) + 1;
+  m.inv_q = (uint32_t)((1ull << 32) / max_q_len) + 1;
+  m.per_xcd = wgs % 8 == 0 && wgs / 8 % slices == 0 ? (int32_t)(wgs / 8) : 0;
   const dim3 grid(slices, (unsigned)tokens);
   if (vec) {
     hipLaunchKernelGGL(dsa_topk_hist_kernel<4>, grid, dim3(kTopkThreads), 0, stream, m);

@@ -39,3 +39,24 @@ def test_rows_around_a_slice(dev, k, vec):
     want.scatter_(1, torch.where(got[2] < 0, stride, got[2]).long().cpu(), 1)
     seen = torch.arange(stride)[None] < lens[:, None]
     assert torch.equal(bits.int()[seen], want[:, :stride][seen])
+
+
+@pytest.mark.parametrize("page_size,q_len", [(128, 1), (6, 3), (1, 2)])
+def test_rows_of_up_to_sixteen_slices(dev, page_size, q_len):
+    """More than eight slices, whose histograms are read in two parts; pages that a thread's four neighbouring keys share and that they do not;
+    boundary-bin keys in every slice."""
+    lens = torch.tensor([131072, 65537, 65536, 70001, 9000, 8192], dtype=torch.int32)
+    t, stride, k = len(lens) * q_len, 131072, 2048
+    g = torch.Generator().manual_seed(page_size)
+    x = torch.randn(t, stride, generator=g)
+    x[1] = torch.round(x[1] * 64) / 64                         # hundreds of keys at the threshold
+    x[q_len - 1] = torch.where(torch.arange(stride) % 16 == 0, 1.0, x[q_len - 1] * 0.01)
+    lg, d = x.to(dev), lens.to(dev)
+    blocks = -(-stride // page_size)
+    bt = torch.randint(0, 2 * blocks, (len(lens), blocks), generator=g).int().to(dev)
+    got = [torch.full((t, k), -7, dtype=torch.int32, device=dev) for _ in range(4)]
+    cnt = [torch.full((t,), -7, dtype=torch.int32, device=dev) for _ in range(2)]
+    kw = dict(q_len=q_len, block_table=bt, page_size=page_size, num_pages=2 * blocks)
+    K.topk(lg, d, k, got[0], rows=got[1], counts=cnt[0], **kw)
+    K.topk(lg, d, k, got[2], single_workgroup=True, rows=got[3], counts=cnt[1], **kw)
+    assert torch.equal(got[0], got[2]) and torch.equal(got[1], got[3]) and torch.equal(*cnt)
