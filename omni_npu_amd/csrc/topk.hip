@@ -740,11 +740,25 @@ __device__ __forceinline__ void finish_slice(const TopkParams& p, const TopkRow&
   }
 }
 
+// What lane 63 combines a value with in step j of six, after which it has that of all lanes (the moves of wave_incl_scan_dpp; a lane
+// without a source keeps its own)
+__device__ __forceinline__ float range_step(float v, int j) {
+  const int i = __float_as_int(v);
+  switch (j) {
+    case 0: return __int_as_float(__builtin_amdgcn_update_dpp(i, i, 0x111, 0xf, 0xf, false));
+    case 1: return __int_as_float(__builtin_amdgcn_update_dpp(i, i, 0x112, 0xf, 0xf, false));
+    case 2: return __int_as_float(__builtin_amdgcn_update_dpp(i, i, 0x114, 0xf, 0xf, false));
+    case 3: return __int_as_float(__builtin_amdgcn_update_dpp(i, i, 0x118, 0xf, 0xf, false));
+    case 4: return __int_as_float(__builtin_amdgcn_update_dpp(i, i, 0x142, 0xa, 0xf, false));
+    default: return __int_as_float(__builtin_amdgcn_update_dpp(i, i, 0x143, 0xc, 0xf, false));
+  }
+}
+
 // (64 registers: two workgroups on a CU; 67 cost 128 rows of 33 000 to 65 000 keys 4 us)
 template <int kVec>
 __global__ __launch_bounds__(kTopkThreads, 8) void dsa_topk_hist_kernel(const TopkMwParams p) {
-  __shared__ SliceLds sh;
-  __shared__ float fscratch[2 * kMwWaves];
+  __shared__ __attribute__((aligned(16))) SliceLds sh;
+  __shared__ __attribute__((aligned(16))) float fscratch[2 * kMwWaves];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const SliceOf so = slice_of_workgroup(p);
   const int s = so.s;
@@ -774,9 +788,9 @@ __global__ __launch_bounds__(kTopkThreads, 8) void dsa_topk_hist_kernel(const To
   for (int j = 0; j < 4; j++)
     if (fabsf(sm[j]) < INFINITY) { lo = fminf(lo, sm[j]); hi = fmaxf(hi, sm[j]); }
 #pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) { lo = fminf(lo, __shfl_xor(lo, o, 64)); hi = fmaxf(hi, __shfl_xor(hi, o, 64)); }
-  if (lane == 0) { fscratch[w] = lo; fscratch[kMwWaves + w] = hi; }
-  for (int i = tid; i < kBins; i += kTopkThreads) sh.hist[i] = 0;
+  for (int j = 0; j < 6; j++) { lo = fminf(lo, range_step(lo, j)); hi = fmaxf(hi, range_step(hi, j)); }
+  if (lane == 63) { fscratch[w] = lo; fscratch[kMwWaves + w] = hi; }
+  *(u32x2*)(sh.hist + 2 * tid) = u32x2{0u, 0u};
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < kMwWaves; i++) { lo = fminf(lo, fscratch[i]); hi = fmaxf(hi, fscratch[kMwWaves + i]); }
@@ -870,18 +884,10 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_write_kernel(const Topk
   const int n = r.n, k = p.t.k;
   if (!r.live || n <= k || n <= kSliceKeys || s * kSliceKeys >= n) return;
   const TopkSink out = topk_sink(p.t, r.b, r.t);
-  // all loads first: the candidate list (its first kMwCandLds entries, whatever their number turns out to be), the
+  // all loads first: the candidate list (its first entries, one to a thread, whatever their number turns out to be), the
   // sure-pick counts of the wavefronts before mine, this slice
-  const uint32_t* cand = p.cand + (int64_t)r.slot * p.cand_cap * 2;
-  const int lim = p.cand_cap < kMwCandLds ? (int)p.cand_cap : kMwCandLds;
-  uint32_t cu[kMwCandLds / kTopkThreads], ci[kMwCandLds / kTopkThreads];
-#pragma unroll
-  for (int q = 0; q < kMwCandLds / kTopkThreads; q++) {
-    const int j = tid + q * kTopkThreads;
-    const u32x2 pr = j < lim ? *(const u32x2*)(cand + 2 * (int64_t)j) : u32x2{0u, 0u};
-    cu[q] = pr[0];
-    ci[q] = pr[1];
-  }
+  const u32x2* cand = (const u32x2*)p.cand + (int64_t)r.slot * p.cand_cap;
+  const u32x2 mine0 = tid < p.cand_cap ? cand[tid] : u32x2{0u, 0u};
   const int32_t* cn = p.counts + (int64_t)r.slot * p.slices * kMwWaves;
   const int mine = s * kMwWaves + w;                       // < kMaxSlices * kMwWaves = 256: four per lane
   int part = 0;
@@ -890,8 +896,11 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_write_kernel(const Topk
   const int m = p.meta[r.slot * 4], need = p.meta[r.slot * 4 + 2];
   const SliceKeys ks = load_slice<kVec>(r.x, n, s, w, lane);
   const SliceRows rows = slice_rows(out, ks, n);
-#pragma unroll
-  for (int q = 0; q < kMwCandLds / kTopkThreads; q++) { cand_u[tid + q * kTopkThreads] = cu[q]; cand_i[tid + q * kTopkThreads] = ci[q]; }
+  cand_u[tid] = mine0[0];
+  cand_i[tid] = mine0[1];
+  if (m <= kMwCandLds) {
+    for (int j = tid + kTopkThreads; j < m; j += kTopkThreads) { const u32x2 c = cand[j]; cand_u[j] = c[0]; cand_i[j] = c[1]; }
+  }
   __syncthreads();
 
   // ---- exact threshold among the m candidates (every slice of the token repeats this small piece of work) ----
@@ -905,14 +914,15 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_write_kernel(const Topk
   } else {
     // degenerate rows (a large share of equal or nearly equal logits)
     radix_threshold<kTopkThreads>(
-        [&](auto&& f) { for (int j = tid; j < m; j += kTopkThreads) f(cand[2 * (int64_t)j], cand[2 * (int64_t)j + 1]); }, need,
+        [&](auto&& f) { for (int j = tid; j < m; j += kTopkThreads) { const u32x2 c = cand[j]; f(c[0], c[1]); } }, need,
         hist, scratch, &prefix, &pos_thresh);
   }
 
   // ---- where this wavefront's picks start: sure picks of everything before it + accepted candidates before it ----
   const int wlo = s * kSliceKeys + w * 512;
   for (int j = lane; j < m; j += 64) {
-    const uint32_t u = in_lds ? cand_u[j] : cand[2 * (int64_t)j], ps = in_lds ? cand_i[j] : cand[2 * (int64_t)j + 1];
+    const u32x2 c = in_lds ? u32x2{cand_u[j], cand_i[j]} : cand[j];
+    const uint32_t u = c[0], ps = c[1];
     part += (int)ps < wlo && ((u > prefix) || (u == prefix && ps <= pos_thresh));
   }
   int o = __builtin_amdgcn_readlane(wave_incl_scan_dpp(part), 63);
