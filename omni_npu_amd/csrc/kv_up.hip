@@ -325,9 +325,13 @@ __global__ __launch_bounds__(512, 2) void mla_kv_up_kernel(const KvUpParams p) {
 // three ahead, into the buffer that everyone has done with.  What bounds it is a tile's chain of start, eight stages and end.
 // us per launch, tiles of 256 tokens / this, rounds of 256 workgroups in parentheses: 100 x 16 15.0 / 7.5 (0.1), 475 x 64 17.5 / 13.6 (2),
 // 208 x 128 17.5 / 13.3 (2), 256 x 64 16.4 / 10.0 (1), 1017 x 32 18.1 / 14.1 (2), 700 x 64 18.8 / 18.1 (3), 384 x 128 20.6 / 18.7 (3),
-// 1500 x 32 20.2 / 20.4 (3), but 1017 x 64 21.9 / 24.5 (4), 512 x 128 21.9 / 27.5 (4): three rounds at most.
+// 1500 x 32 20.2 / 20.4 (3), but 1017 x 64 21.9 / 24.5 (4), 512 x 128 21.9 / 27.5 (4): up to three rounds.  More where they are at most
+// twice the rounds of the large tiles, which take 15 us each, however much of them is padding: 83 and 322 x 128 31.8 / 26.8 (4, of 2).
+// And where one round of quadrants holds the heads that are left behind the full rounds of large tiles, those heads are a launch of
+// their own: 1100 x 64 29.8 -> 26.8, 2100 x 32 29.3 -> 26.4, 8300 x 16 45.0 -> 40.6, 60 and 4040 x 32 44.4 -> 42.8, 180 and 3900 x 32
+// 47.7 both ways.
 constexpr int kUpSmallTok = 128;
-constexpr int64_t kUpSmallMost = 768;
+constexpr int64_t kUpSmallRounds = 3, kUpTailRounds = 1;
 constexpr int kUpSmallStage = 2 * kUpUnit;       // 32768
 
 template <bool kKeysF16>
@@ -478,15 +482,29 @@ static int kv_up_impl(const char* what, const void* x, int64_t x_stride, int64_t
     if (rc != MLA_OK) return rc;
   }
   const auto tiles_of = [&](int64_t tok) { p.m_first = (int32_t)((num_rows + tok - 1) / tok); return p.m_first + (num_rows1 + tok - 1) / tok; };
-  int64_t tiles = tiles_of(kUpSmallTok) * num_heads * 2;
-  const bool small = tiles > 0 && tiles <= kUpSmallMost;
-  p.m_tiles = (int32_t)tiles_of(small ? kUpSmallTok : kUpTok);
-  if (!small) tiles = (int64_t)p.m_tiles * num_heads;
-  auto* kern = kerns[(small ? 2 : 0) + (keys_f16 ? 1 : 0)];
-  // one workgroup per CU at most; fewer tiles: as many workgroups, in whole rounds of the eight XCDs
-  const int64_t grid = tiles == 0 ? 8 : tiles < 256 ? (tiles + 7) / 8 * 8 : 256;   // (no rows: only what is to be cleared)
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), kUpLdsB, stream, p);
-  return check_launch("mla_kv_up_kernel");
+  const int64_t quads = tiles_of(kUpSmallTok) * 2, whole = tiles_of(kUpTok);          // of a head
+  const int64_t rounds = (whole * num_heads + 255) / 256, small_rounds = (quads * num_heads + 255) / 256;
+  // heads [from, to) in one launch: one workgroup per CU at most; fewer tiles: as many workgroups, in whole rounds of the eight XCDs
+  const auto launch = [&](bool small, int64_t from, int64_t to) {
+    KvUpParams q = p;
+    q.m_tiles = (int32_t)tiles_of(small ? kUpSmallTok : kUpTok);
+    q.m_first = p.m_first;
+    q.heads = (int32_t)(to - from);
+    q.w = p.w + from * 256 * p.w_st;
+    q.out = p.out + from * p.o_sh;
+    if (from > 0) { q.pe = nullptr; q.clear_words = 0; }     // (done by the launch of the first heads)
+    const int64_t tiles = q.heads * (small ? quads : whole);
+    const int64_t grid = tiles == 0 ? 8 : tiles < 256 ? (tiles + 7) / 8 * 8 : 256;     // (no rows: only what is to be cleared)
+    hipLaunchKernelGGL(kerns[(small ? 2 : 0) + (keys_f16 ? 1 : 0)], dim3((unsigned)grid), dim3(512), kUpLdsB, stream, q);
+    return check_launch("mla_kv_up_kernel");
+  };
+  if (small_rounds > 0 && (small_rounds <= kUpSmallRounds || small_rounds <= 2 * rounds)) return launch(true, 0, num_heads);
+  const int64_t full = whole * num_heads / 256, first = whole > 0 ? full * 256 / whole : 0;
+  if (full >= 1 && full < rounds && first >= 1 && (num_heads - first) * quads <= 256 * kUpTailRounds) {
+    const int rc = launch(false, 0, first);
+    return rc != MLA_OK ? rc : launch(true, first, num_heads);
+  }
+  return launch(false, 0, num_heads);
 }
 
 extern "C" int mla_kv_up(const void* x, int64_t x_stride, const void* weight, int64_t w_stride, int64_t num_rows, int32_t num_heads,

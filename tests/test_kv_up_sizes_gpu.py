@@ -51,3 +51,32 @@ def test_two_sets_of_rows_in_one_launch(dev, t0, t1, n, keys_f16):
         k, v, _ = K.kv_up(x, w, n, keys_f16)
         got = kv[:, at:at + len(x)].transpose(0, 1)
         assert torch.equal(got[..., :128].view(torch.int16), k.view(torch.int16)) and torch.equal(got[..., 128:], v)
+
+
+@pytest.mark.parametrize("t0,t1,n", [(1500, 0, 43), (60, 4040, 32), (1300, 0, 87), (2049, 0, 57), (83, 322, 128), (1, 257, 100)])
+@pytest.mark.parametrize("keys_f16", [True, False])
+def test_last_heads_in_quadrants(dev, t0, t1, n, keys_f16):
+    """Heads behind the full rounds of large tiles, and ragged sets that go into more than three rounds of quadrants: a head's results are
+    those of a launch of it alone; rope rows and what is to be cleared once."""
+    (x0, w, p0), (x1, _, p1) = _inputs(dev, t0, n, 576, 512, seed=3), _inputs(dev, max(t1, 1), n, 576, 512, seed=4)
+    sets = [(x0, p0)] + ([(x1, p1)] if t1 else [])
+    kv = torch.full((n, t0 + t1, 256), float("nan"), dtype=torch.float16, device=dev)
+    pe, clear = torch.empty(t0 + t1, 64, dtype=torch.float16, device=dev), torch.full((256,), 7, dtype=torch.int32, device=dev)
+    tail = (kv.data_ptr(), 256, (t0 + t1) * 256)
+    stream = torch.cuda.current_stream().cuda_stream
+    if t1:
+        rc = _lib.load().mla_kv_up_two(x0.data_ptr(), x0.stride(0), t0, p0.data_ptr(), p0.stride(0), x1.data_ptr(), x1.stride(0), t1, p1.data_ptr(),
+                                       p1.stride(0), w.data_ptr(), w.stride(0), n, int(keys_f16), *tail, pe.data_ptr(), 64, clear.data_ptr(), 256,
+                                       stream)
+    else:
+        rc = _lib.load().mla_kv_up(x0.data_ptr(), x0.stride(0), w.data_ptr(), w.stride(0), t0, n, int(keys_f16), *tail, p0.data_ptr(),
+                                   p0.stride(0), pe.data_ptr(), 64, clear.data_ptr(), 256, stream)
+    _lib.check(rc, "mla_kv_up")
+    assert not bool(clear.any()) and torch.equal(pe, torch.cat([p for _, p in sets]).half())
+    for h in (0, n // 2, n - 2, n - 1):
+        at = 0
+        for x, _ in sets:
+            k, v, _ = K.kv_up(x, w[h * 256:(h + 1) * 256], 1, keys_f16)
+            got = kv[h, at:at + len(x)]
+            assert torch.equal(got[:, :128].view(torch.int16), k[:, 0].view(torch.int16)) and torch.equal(got[:, 128:], v[:, 0])
+            at += len(x)
