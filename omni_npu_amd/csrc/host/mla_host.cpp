@@ -383,7 +383,7 @@ int64_t prefill_blocks(int64_t tokens, int64_t batch, int64_t max_q_len, int64_t
 }
 int prefill_pieces(int64_t tokens, int64_t batch, int64_t max_q_len, int64_t heads, int64_t seen) {
   const int64_t blocks = prefill_blocks(tokens, batch, max_q_len, heads);
-  if (blocks < 1 || blocks * 2 > kPrefillResident || seen <= 0) return 1;
+  if (tokens < 1 || blocks < 1 || blocks * 2 > kPrefillResident || seen <= 0) return 1;
   const double tiles = (double)seen / (double)(64 * batch), mib = (double)(tokens * heads * 516) / 1048576.0;
   const int64_t pieces = std::min({(int64_t)std::sqrt(2.7 * tiles / mib), kPrefillResident / blocks, (int64_t)32});
   if (pieces < 2) return 1;

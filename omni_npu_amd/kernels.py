@@ -949,7 +949,7 @@ def prefill_pieces(tokens: int, batch: int, max_q_len: int, num_heads: int, seen
     """Into how many pieces prefill_varlen cuts the keys of a block of 128 rows (1: not at all); ``seen``: keys that a row sees on
     average, summed over the sequences."""
     blocks = _prefill_blocks(tokens, batch, max_q_len, num_heads)
-    if blocks < 1 or blocks * 2 > _PREFILL_RESIDENT or seen <= 0:   # (more rows than keys: the first ones see none)
+    if tokens < 1 or blocks < 1 or blocks * 2 > _PREFILL_RESIDENT or seen <= 0:   # (more rows than keys: the first ones see none)
         return 1
     tiles, mib = seen / (64 * batch), tokens * num_heads * 516 / 2 ** 20
     pieces = min(int(math.sqrt(2.7 * tiles / mib)), _PREFILL_RESIDENT // blocks, _PREFILL_MAX_PIECES)

@@ -88,3 +88,13 @@ def test_pieces_are_refused_with_what_they_do_not_take(dev, opt):
     with pytest.raises(TypeError, match="pieces"):
         K.prefill_varlen(q[..., :128], q[..., 128:], *own, cu, cu, 130, 0.07, True, torch.empty(130, 8, 128, device=dev), long=False,
                          pieces=2, **kw)
+
+
+@pytest.mark.parametrize("max_q_len", [0, 1, 300])
+def test_no_rows_give_an_empty_result(dev, max_q_len):
+    """The longest of no sequences may be given as any number (a step's padded one)."""
+    g = torch.Generator(device=dev).manual_seed(1)
+    own, cu_q = _rows(dev, 100, 16, g), _cu([0], dev)
+    q = torch.empty(0, 16, 192, dtype=torch.bfloat16, device=dev)
+    out, lse = torch.empty(0, 16, 128, dtype=torch.bfloat16, device=dev), torch.empty(0, 16, device=dev)
+    assert K.prefill_varlen(q[..., :128], q[..., 128:], *own, cu_q, _cu([100], dev), max_q_len, 0.07, False, out, lse) is out
