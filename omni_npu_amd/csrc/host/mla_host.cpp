@@ -34,6 +34,7 @@ using OptTensor = std::optional<Tensor>;
 constexpr int64_t kNope = 512, kRope = 64, kPage = 128, kFp8Row = 656, kVDim = 128;
 constexpr int64_t kAbsorbMaxTokens = 1024;   // kernels.ABSORB_MAX_TOKENS
 constexpr int64_t kVupMaxTokens = 1024;      // kernels.VUP_MAX_TOKENS: beyond, a separate merge and the library GEMM
+constexpr int64_t kVupOnlyTokens = 256;      // kernels._VUP_ONLY_TOKENS
 constexpr int64_t kSparseWorkspaceCap = 256 << 20;   // kernels.SPARSE_WORKSPACE_CAP
 
 void check(int rc, const char* what) {
@@ -174,7 +175,8 @@ Absorbed absorb(const Tensor& q, const Tensor& w_uk, int64_t t, const NewRows* r
 void merge_vup(const Tensor& ws, const Tensor& lens, const OptTensor& qsl, int64_t batch, int64_t q_len, int64_t n, int splits,
                int64_t t, const Tensor& w_uv, const Tensor& out, bool fp8, Stream st) {
   const int32_t* qs = qsl ? (const int32_t*)qsl->data_ptr() : nullptr;
-  if (t <= kVupMaxTokens) {
+  const bool takes = !(((uintptr_t)w_uv.data_ptr() & 15) || ((uintptr_t)out.data_ptr() & 7) || w_uv.stride(1) < kVDim);   // (strides: layer_ok)
+  if (t <= kVupOnlyTokens || (t <= kVupMaxTokens && takes)) {
     const auto merge = fp8 ? mla_splitkv_reduce_vup_fp8 : mla_splitkv_reduce_vup;
     check(merge(ws.data_ptr(), ws.numel(), (const int32_t*)lens.data_ptr(), qs, (int)batch, (int)q_len, (int)n, splits, (int)t,
                 w_uv.data_ptr(), w_uv.stride(0), w_uv.stride(1), out.data_ptr(), out.stride(0), kVDim, st), "mla_splitkv_reduce_vup");
@@ -567,5 +569,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.attr("PREFILL_RULES") = py::make_tuple(kPrefillResident, kPrefillQueueWords, kPrefillLongKeys);
   m.attr("ABSORB_MAX_TOKENS") = kAbsorbMaxTokens;
   m.attr("VUP_MAX_TOKENS") = kVupMaxTokens;
+  m.attr("VUP_ONLY_TOKENS") = kVupOnlyTokens;
   m.attr("SPARSE_WORKSPACE_CAP") = kSparseWorkspaceCap;
 }

@@ -528,10 +528,18 @@ def _vup_out(out: torch.Tensor, w_uv: torch.Tensor, t: int, n: int) -> torch.Ten
 # us of split, merge and up-projection, separate / fused, tokens x heads: 512 x 16 53.2 / 38.5, 512 x 128 138 / 122, 1024 x 64 152 / 136,
 # 1024 x 128 285 / 254, 2048 x 128 595 / 532.  The fused form is the faster one there too; what ends here is a decode step.
 VUP_MAX_TOKENS = 1024
+# Up to so many there is no other form: what the fused one does not take is refused
+_VUP_ONLY_TOKENS = 256
+
+
+def _vup_takes(w_uv: torch.Tensor, o3: torch.Tensor) -> bool:
+    """Whether the fused merge takes a weight [N,512,128] and a result [T,N,128]: rows on 16-byte and 8-byte boundaries."""
+    return not ((w_uv.stride(0) | w_uv.stride(1)) & 7 or w_uv.data_ptr() & 15 or w_uv.stride(1) < 128
+                or (o3.stride(0) | o3.stride(1)) & 3 or o3.data_ptr() & 7)
 
 
 def _reduce_vup(lib, ws_args, seq_lens, qsl, b, q_len, n, num_splits, t, w_uv, o3, st, fp8: bool = False) -> None:
-    if t > VUP_MAX_TOKENS:
+    if t > VUP_MAX_TOKENS or (t > _VUP_ONLY_TOKENS and not _vup_takes(w_uv, o3)):
         o = torch.empty(n, t, D_NOPE, dtype=torch.bfloat16, device=o3.device)
         rc = lib.mla_splitkv_reduce(*ws_args, seq_lens.data_ptr(), qsl, b, q_len, n, num_splits, o.data_ptr(), o.stride(1),
                                     o.stride(0), None, st)

@@ -1,10 +1,16 @@
 """Decode steps of more than 256 tokens: absorption and merge + up-projection by this library's kernels up to 1024 tokens, by the
 library's products beyond."""
+from types import SimpleNamespace
+
 import pytest
 import torch
 
+from omni_npu_amd import _vllm_compat as V
 from omni_npu_amd import kernels as K
+from omni_npu_amd.attention.backends import mla
 from oracle import mla_oracle as O
+from tests.test_backend_gpu import _mk_impl, _to
+from tests.test_boundary import _cfg, _common
 
 pytestmark = pytest.mark.gpu
 
@@ -37,3 +43,46 @@ def test_merge_and_up_projection(dev, batch, q_len, heads, splits):
     a, b = o.double().transpose(0, 1).contiguous(), w.double()
     want, mag = torch.bmm(a, b).transpose(0, 1).reshape(t, -1), torch.bmm(a.abs(), b.abs()).transpose(0, 1).reshape(t, -1)
     assert bool(((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + mag * 512 * 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("what", ["result", "weight"])
+def test_rows_off_their_boundaries_are_merged_for_the_library_s_product(dev, what):
+    """More than 256 tokens whose result or W_UV lies where the fused merge takes neither: as the separate merge and product, the bound
+    that of the test above; up to 256 tokens such a call is refused."""
+    g = torch.Generator(device=dev).manual_seed(5)
+    heads, t = 16, 257
+    c = O.make_decode_case(t, heads, 2, 90, seed=1)
+    args = [c[k].to(dev) for k in ("q_nope", "q_rope", "nope", "rope", "block_table", "seq_lens")]
+    off = lambda n, by: torch.full((n + by,), float("nan"), dtype=torch.bfloat16, device=dev)[by:]
+    w = off(heads * 512 * 128, 4 if what == "weight" else 0).view(heads, 512, 128)
+    w.copy_(torch.randn(heads, 512, 128, generator=g, device=dev) * 0.02)
+    out = off(t * heads * 128, 2 if what == "result" else 0).view(t, heads * 128)
+    K.decode(*args, c["scale"], out, w_uv=w)
+    o = torch.empty(t, heads, 512, dtype=torch.bfloat16, device=dev)
+    K.decode(*args, c["scale"], o)
+    a, b = o.double().transpose(0, 1).contiguous(), w.double()
+    want, mag = torch.bmm(a, b).transpose(0, 1).reshape(t, -1), torch.bmm(a.abs(), b.abs()).transpose(0, 1).reshape(t, -1)
+    assert bool(((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + mag * 512 * 2.0 ** -24).all())
+    few = [x[:256] if x.shape[0] == t else x for x in args]
+    with pytest.raises(RuntimeError, match="aligned"):
+        K.decode(*few, c["scale"], out[:256], w_uv=w)
+
+
+def test_a_step_s_result_off_its_boundary(dev):
+    """The same through the layer: the native host side and the general path both merge first."""
+    q_lens, n = [1] * 257, 16
+    common = _common(q_lens, [100] * 257)
+    t, g = 257, torch.Generator().manual_seed(2)
+    nblk = int(common.block_table_tensor.max()) + 1
+    common.slot_mapping = torch.cat([O.slots_for(common.block_table_tensor, b, 99, 100) for b in range(t)])
+    impl, _ = _mk_impl(mla.NPUMLAImpl, n, dev)
+    meta = mla.NPUMLAMetadataBuilder(V.AttentionSpec(128, 1, 576, torch.bfloat16), ["l"], _cfg(cap=2), dev).build(0, _to(common, dev))
+    rand = lambda *s: torch.randn(*s, generator=g).bfloat16().to(dev)
+    cache, a = (rand(nblk, 128, 1, 512), rand(nblk, 128, 1, 64)), [rand(t, n, 192), rand(t, 512), rand(t, 1, 64)]
+    got = []
+    for by in (0, 2):
+        out = torch.zeros(t * n * 128 + by, dtype=torch.bfloat16, device=dev)[by:].view(t, n * 128)
+        impl.forward(SimpleNamespace(_k_scale=None), *a, cache, meta, output=out)
+        got.append(out)
+    # (the latent results are rounded to bf16 in between: 2^-9 of each at most, and the result once more)
+    assert (got[1].float() - got[0].float()).norm() <= 2.0 ** -8 * got[0].float().norm()
