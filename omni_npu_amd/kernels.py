@@ -1273,7 +1273,7 @@ def quant_qkw_fp8_above(q: torch.Tensor, weights: torch.Tensor, tokens: int, k: 
                         scale_cache: torch.Tensor, slot_mapping: torch.Tensor, query_start_loc: torch.Tensor, seq_lens: torch.Tensor,
                         max_q_len: int, first_token: int, skip_up_to: int):
     """(q8 [tokens,H,128] e4m3 bits, w [tokens,H] fp32) of the first ``tokens`` of q (bf16 [T,H,128], H a multiple of 64) and of the
-    head weights [T,H], the query scales folded into w, and the new index keys k [T,128] into the cache as quant_qk_fp8 writes
+    head weights [>=T,H], the query scales folded into w, and the new index keys k [T,128] into the cache as quant_qk_fp8 writes
     them, in one launch.  Tokens from ``first_token`` on are prompts (query_start_loc int32 [B+1] counts from there, seq_lens int32
     [B]); those that see at most ``skip_up_to`` keys get no queries and no weights."""
     _need_cuda(q, weights, k, k8_cache, scale_cache, slot_mapping, query_start_loc, seq_lens)
@@ -1284,8 +1284,8 @@ def quant_qkw_fp8_above(q: torch.Tensor, weights: torch.Tensor, tokens: int, k: 
     for x in (q2, k2):
         if x.shape[-1] != 128 or x.dtype != torch.bfloat16 or x.stride(-1) != 1:
             raise TypeError("quant_qkw_fp8_above: bf16 rows of 128")
-    if h % 64 or not 0 <= tokens <= t or weights.shape != (t, h) or first_token < 0:
-        raise ValueError("quant_qkw_fp8_above: q [T,H,128] and weights [T,H], H a multiple of 64, at most T tokens")
+    if h % 64 or not 0 <= tokens <= t or weights.dim() != 2 or weights.shape[0] < t or weights.shape[1] != h or first_token < 0:
+        raise ValueError("quant_qkw_fp8_above: q [T,H,128] and weights [>=T,H], H a multiple of 64, at most T tokens")
     if weights.dtype not in (torch.float32, torch.bfloat16) or weights.stride(1) != 1:
         weights = weights.float().contiguous()
     if k8_cache.dim() != 3 or k8_cache.element_size() != 1 or k8_cache.stride(-1) != 1 or scale_cache.dtype != torch.float32 or \

@@ -61,6 +61,18 @@ def test_prompts_no_longer_than_the_selection(dev, q_lens):
     assert torch.equal(picks, select.topk_indices_buffer[:t])
 
 
+@pytest.mark.parametrize("q_lens", [[65, 10], [64], [1, 70, 2]])
+def test_padded_rows_of_weights_and_keys_change_nothing(dev, q_lens):
+    """Weights and keys of a padded step beside the queries of its tokens: the selection is that of the rows without the padding."""
+    impl, select, meta, kv_cache, a, i = _dsa_prompts(dev, q_lens)
+    t, got = sum(q_lens), []
+    for pad in (0, 3):
+        select.topk_indices_buffer.fill_(-7)
+        select(i[0], *(torch.cat([x, x[:pad]]) for x in i[1:]), kv_cache, meta)
+        got.append((select.topk_indices_buffer[:t].clone(), kv_cache[2].clone()))
+    assert all(torch.equal(x.view(torch.uint8), y.view(torch.uint8)) for x, y in zip(*got))
+
+
 @pytest.mark.parametrize("exp", [0, 64, -49, -51, 65, 66, 100, -100, -126])
 def test_quantised_rows_are_the_division_s_for_every_pair_of_mantissas(dev, exp):
     """Every bf16 mantissa as a row's maximum, against every bf16 number down to 2^-24 of it: the codes and scales of x / (amax / 448) in
