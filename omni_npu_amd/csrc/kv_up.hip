@@ -308,8 +308,11 @@ __global__ __launch_bounds__(512, 2) void mla_kv_up_kernel(const KvUpParams p) {
     char* out = p.out + r.first * p.o_st + (int64_t)tile.head * p.o_sh + wn * 128;
 #pragma unroll
     for (int i = 0; i < 2; i++) up_store<kKeysF16, false>(p, acc[0][i], st, out, i * 128 + wt * 32, r.left, ln);
+    // (held over the clamping it puts an operand of the next tile into scratch memory, whose reload waits for all copies: bf16 keys, 10 168
+    // tokens x 128 heads 328 us, so 319; the form without clamping loses a percent by it)
+    const int ln2 = kKeysF16 ? ln : up_lane();
 #pragma unroll
-    for (int i = 0; i < 2; i++) up_store<kKeysF16, true>(p, acc[1][i], st, out + 256, i * 128 + wt * 32, r.left, ln);
+    for (int i = 0; i < 2; i++) up_store<kKeysF16, true>(p, acc[1][i], st, out + 256, i * 128 + wt * 32, r.left, ln2);
     if (!more) break;
     stored = true;
     idx = nidx;
