@@ -48,7 +48,8 @@ def indexer_cache_views(index_cache: torch.Tensor):
     return k8, ks
 
 
-# In the place of pick bits: the prompts are no longer than the selection, every token attends over all the keys it sees
+# In the place of pick bits between the selection and the attention behind it: the prompts are no longer than the selection, every token
+# attends over all the keys it sees
 EVERY_KEY = "every key"
 
 
@@ -196,6 +197,7 @@ class LightningIndexer:
         # used them (drop_mask), and the metadata object they were made for
         self.masked_pairs_per_pick = 0.0
         self._mask, self._mask_meta = None, None
+        self._mask_shape = (0, 0)    # of the bits that EVERY_KEY stands for
         self._logits = None
         self._logits_kept = []       # outgrown score buffers: a captured graph may still hold their address, never freed
 
@@ -254,8 +256,8 @@ class LightningIndexer:
             if over_own:
                 if whole:                                           # (rows as wide as these prompts: what picks the kernel by their length)
                     lg = self._logits.view(-1)[:ntok * stride].view(ntok, stride)
-                self._mask_meta = attn_metadata
-                self._mask = EVERY_KEY if whole else torch.empty(ntok, _mask_words(stride), dtype=torch.int32, device=q.device)
+                self._mask_meta, self._mask_shape = attn_metadata, (ntok, _mask_words(stride))
+                self._mask = EVERY_KEY if whole else torch.empty(self._mask_shape, dtype=torch.int32, device=q.device)
                 K.topk(lg, lens, self.topk_tokens, out[sl], q_len=q_len, query_start_loc=qsl, mask=None if whole else self._mask)
             else:
                 K.topk(lg, lens, self.topk_tokens, out[sl], q_len=q_len, query_start_loc=qsl, block_table=meta.block_table,
@@ -308,13 +310,20 @@ class LightningIndexer:
                                                p.query_start_loc, p.max_query_len, max_len, self.topk_tokens, whole, lg,
                                                self.topk_indices_buffer, mask):
             return False
-        self._mask_meta, self._mask = attn_metadata, EVERY_KEY if whole else mask
+        self._mask_meta, self._mask, self._mask_shape = attn_metadata, EVERY_KEY if whole else mask, (t, _mask_words(stride))
         return True
 
-    def mask_for(self, attn_metadata):
-        """The picks of the step's prompt tokens as bits [T, W] (kernels.topk's mask), or EVERY_KEY, if the last selection made them
-        for this very metadata object and the attention has not used them yet, else None."""
+    def picks_for(self, attn_metadata):
+        """What NPUDSAImpl._forward_prompts takes: mask_for's bits, EVERY_KEY where they would all be set, or None."""
         return self._mask if self.masked_prompts(attn_metadata) else None
+
+    def mask_for(self, attn_metadata) -> Optional[torch.Tensor]:
+        """The picks of the step's prompt tokens as bits [T, W] (kernels.topk's mask) if the last selection made them for this very
+        metadata object and the attention has not used them yet, else None."""
+        picks = self.picks_for(attn_metadata)
+        if picks is EVERY_KEY:
+            return torch.full(self._mask_shape, -1, dtype=torch.int32, device=self.topk_indices_buffer.device)
+        return picks
 
     def masked_prompts(self, attn_metadata) -> bool:
         """Whether the last selection ran for this very metadata object and made its prompts' picks as bits: the row buffers
@@ -504,7 +513,7 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
         if has_prefill:
             p = attn_metadata.prefill
             assert p is not None
-            pick = select.mask_for(attn_metadata) if masked else None
+            pick = getattr(select, "picks_for", select.mask_for)(attn_metadata) if masked else None
             if not self._forward_prompts(q[ndt:], k_c_normed[ndt:num_actual_toks], k_pe[ndt:num_actual_toks], p, pick,
                                          output[ndt:]):
                 q_nope, q_pe = self._absorb_prolog(q[ndt:])

@@ -74,7 +74,8 @@ class NPUDeepseekSparseAttention(torch.nn.Module):
         masked = hasattr(select, "masked_prompts") and select.masked_prompts(meta)
         if meta.prefill is not None:
             p = meta.prefill
-            done = masked and impl._forward_prompts(q, kv_a, k_pe, p, select.mask_for(meta), out)
+            pick = getattr(select, "picks_for", select.mask_for)(meta) if masked else None
+            done = masked and impl._forward_prompts(q, kv_a, k_pe, p, pick, out)
             if masked:
                 select.drop_mask()
             if done:

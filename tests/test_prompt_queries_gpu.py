@@ -48,7 +48,10 @@ def test_prompts_no_longer_than_the_selection(dev, q_lens):
     select._scores_buffer(t, 8192, dev)                       # (an earlier step's longer rows)
     select(*i, kv_cache, meta)
     picks, whole = select.topk_indices_buffer[:t].clone(), max(q_lens) <= 64
-    assert (select.mask_for(meta) is dsa.EVERY_KEY) == whole
+    assert (select.picks_for(meta) is dsa.EVERY_KEY) == whole
+    mask = select.mask_for(meta)                              # (a caller's own attention takes bits, whatever they say)
+    words = -(-max(n for n in q_lens if n > 1) // 64) * 2 + 2
+    assert mask.dtype == torch.int32 and mask.shape == (t - ndt, words) and bool((mask == -1).all() if whole else (mask != -1).any())
     out = torch.zeros(t, 16 * 128, dtype=torch.bfloat16, device=dev)
     impl.forward(None, *a, kv_cache, meta, output=out)
     assert select.mask_for(meta) is None
@@ -56,6 +59,8 @@ def test_prompts_no_longer_than_the_selection(dev, q_lens):
         bits, want = torch.full((t - ndt, 4), -1, dtype=torch.int32, device=dev), torch.zeros_like(out[ndt:])
         assert impl._forward_prompts(a[0][ndt:], a[1][ndt:], a[2][ndt:], meta.prefill, bits, want)
         assert torch.equal(out[ndt:], want) and bool(want.float().abs().sum(1).ne(0).all())
+        want.zero_()
+        assert impl._forward_prompts(a[0][ndt:], a[1][ndt:], a[2][ndt:], meta.prefill, mask, want) and torch.equal(out[ndt:], want)
     select.masked_pairs_per_pick = 0.0
     select(*i, kv_cache, meta)
     assert torch.equal(picks, select.topk_indices_buffer[:t])
