@@ -33,6 +33,7 @@ using OptTensor = std::optional<Tensor>;
 
 constexpr int64_t kNope = 512, kRope = 64, kPage = 128, kFp8Row = 656, kVDim = 128;
 constexpr int64_t kAbsorbMaxTokens = 1024;   // kernels.ABSORB_MAX_TOKENS
+constexpr int64_t kAbsorbKeptTokens = 256;   // kernels.ABSORB_KEPT_TOKENS
 constexpr int64_t kVupMaxTokens = 1024;      // kernels.VUP_MAX_TOKENS: beyond, a separate merge and the library GEMM
 constexpr int64_t kVupOnlyTokens = 256;      // kernels._VUP_ONLY_TOKENS
 constexpr int64_t kSparseWorkspaceCap = 256 << 20;   // kernels.SPARSE_WORKSPACE_CAP
@@ -142,9 +143,17 @@ bool layer_ok(const Tensor& q, const Tensor& w_uk, const Tensor& w_uv, const Ten
          w_uv.size(0) == n && w_uv.size(1) == kNope && w_uv.size(2) == kVDim && w_uv.stride(0) % 8 == 0 && w_uv.stride(1) % 8 == 0 &&
          is_bf16(out, 2, dev) && out.size(0) >= t && out.size(1) == n * kVDim && out.stride(0) % 4 == 0;
 }
-// kernels.absorb: the absorbed queries, in scratch memory or (more tokens, or rows that are not 16-byte aligned) from the
-// library.  Rows of new tokens (or null) go to the cache in the same launch, or in front of the library's.
+// kernels.absorb: the absorbed queries, from this library's kernel or (more tokens, or rows that are not 16-byte aligned) from the
+// other one.  Of few tokens they are in scratch memory that stays; of more (up to 134 MB, which no later step may need) in the
+// allocator's, which has them back behind the step.  Rows of new tokens (or null) go to the cache in the same launch, or in front of
+// the library's.
 struct Absorbed { Tensor keep; const void* ptr; int64_t st, sh; };
+Absorbed absorbed_rows(const Tensor& q, int64_t t, int64_t n, Stream st) {
+  const int64_t bytes = t * n * kNope * 2;
+  Tensor rows = t <= kAbsorbKeptTokens ? scratch(q, st, bytes, 2) : at::empty({bytes}, q.options().dtype(at::kByte));
+  void* at0 = rows.data_ptr();
+  return {std::move(rows), at0, n * kNope, kNope};
+}
 Absorbed absorb(const Tensor& q, const Tensor& w_uk, int64_t t, const NewRows* rows, const Cache& c, Stream st) {
   const int64_t n = q.size(1);
   const bool own = t <= kAbsorbMaxTokens && !((w_uk.stride(0) | w_uk.stride(1)) & 7) && !(((uintptr_t)q.data_ptr() | (uintptr_t)w_uk.data_ptr()) & 15);
@@ -153,20 +162,20 @@ Absorbed absorb(const Tensor& q, const Tensor& w_uk, int64_t t, const NewRows* r
     const int64_t unit = c.rope ? 8 : 16, cache_strides = c.n_sp | c.n_sr | (c.rope ? c.r_sp | c.r_sr : 0);
     const uintptr_t ptrs = (uintptr_t)kv_c.data_ptr() | (uintptr_t)k_pe.data_ptr() | (uintptr_t)c.nope->data_ptr() | (c.rope ? (uintptr_t)c.rope->data_ptr() : 0);
     if (!((kv_c.stride(0) | k_pe.stride(0)) & 7) && !(cache_strides & (unit - 1)) && !(ptrs & 15) && (c.rope || c.n_sr >= kFp8Row)) {
-      Tensor& ws = scratch(q, st, t * n * kNope * 2, 2);
-      check(mla_absorb_write(q.data_ptr(), q.stride(0), q.stride(1), w_uk.data_ptr(), w_uk.stride(0), w_uk.stride(1), ws.data_ptr(),
+      Absorbed a = absorbed_rows(q, t, n, st);
+      check(mla_absorb_write(q.data_ptr(), q.stride(0), q.stride(1), w_uk.data_ptr(), w_uk.stride(0), w_uk.stride(1), a.keep.data_ptr(),
                              n * kNope, kNope, (int)t, (int)n, kv_c.data_ptr(), kv_c.stride(0), k_pe.data_ptr(), k_pe.stride(0),
                              (const int64_t*)rows->slots->data_ptr(), (int)rows->t, c.nope->data_ptr(), c.n_sp, c.n_sr,
                              c.rope ? c.rope->data_ptr() : nullptr, c.r_sp, c.r_sr, (int)c.page, c.pages, st), "mla_absorb_write");
-      return {Tensor(), ws.data_ptr(), n * kNope, kNope};
+      return a;
     }
   }
   if (rows) write_rows(*rows, c, st);
   if (own) {
-    Tensor& ws = scratch(q, st, t * n * kNope * 2, 2);
-    check(mla_absorb_bf16(q.data_ptr(), q.stride(0), q.stride(1), w_uk.data_ptr(), w_uk.stride(0), w_uk.stride(1), ws.data_ptr(),
+    Absorbed a = absorbed_rows(q, t, n, st);
+    check(mla_absorb_bf16(q.data_ptr(), q.stride(0), q.stride(1), w_uk.data_ptr(), w_uk.stride(0), w_uk.stride(1), a.keep.data_ptr(),
                           n * kNope, kNope, (int)t, (int)n, st), "mla_absorb_bf16");
-    return {Tensor(), ws.data_ptr(), n * kNope, kNope};
+    return a;
   }
   Tensor ql = at::bmm(q.narrow(0, 0, t).narrow(2, 0, 128).transpose(0, 1), w_uk);
   return {ql, ql.data_ptr(), ql.stride(1), ql.stride(0)};
@@ -568,6 +577,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("prefill_wants_queue", &prefill_wants_queue);
   m.attr("PREFILL_RULES") = py::make_tuple(kPrefillResident, kPrefillQueueWords, kPrefillLongKeys);
   m.attr("ABSORB_MAX_TOKENS") = kAbsorbMaxTokens;
+  m.attr("ABSORB_KEPT_TOKENS") = kAbsorbKeptTokens;
   m.attr("VUP_MAX_TOKENS") = kVupMaxTokens;
   m.attr("VUP_ONLY_TOKENS") = kVupOnlyTokens;
   m.attr("SPARSE_WORKSPACE_CAP") = kSparseWorkspaceCap;

@@ -362,8 +362,10 @@ def kv_up(kv_c: torch.Tensor, weight: torch.Tensor, num_heads: int, keys_f16: bo
 
 # Tokens up to which the queries of a step are absorbed by this library's kernel; beyond, the work is a plain GEMM.  us, library / this,
 # tokens x heads: 512 x 16 24.9 / 13.1, 512 x 128 34.2 / 26.3, 1024 x 64 29.3 / 26.2, 1024 x 128 52.9 / 45.8, 2048 x 128 105.4 / 105.1.
-# (The native side keeps the absorbed queries in scratch memory, 134 MB for 1024 tokens of 128 heads.)
 ABSORB_MAX_TOKENS = 1024
+# Up to so many the native host side has the absorbed queries in scratch memory that stays (33 MB for 128 heads); of more the allocator gets
+# them back behind the step
+ABSORB_KEPT_TOKENS = 256
 
 
 def absorb(q_nope: torch.Tensor, w_uk: torch.Tensor) -> torch.Tensor:

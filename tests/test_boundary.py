@@ -436,8 +436,8 @@ def test_native_host_side_shapes_its_launches_as_the_general_path():
     row groups up to past the CUs, query rows on both sides of a group, and context lengths around the chunk steps."""
     from omni_npu_amd import _host, kernels as K
     ext = _host.load()
-    assert (ext.ABSORB_MAX_TOKENS, ext.VUP_MAX_TOKENS, ext.VUP_ONLY_TOKENS, ext.SPARSE_WORKSPACE_CAP) == \
-        (K.ABSORB_MAX_TOKENS, K.VUP_MAX_TOKENS, K._VUP_ONLY_TOKENS, K.SPARSE_WORKSPACE_CAP)
+    assert (ext.ABSORB_MAX_TOKENS, ext.ABSORB_KEPT_TOKENS, ext.VUP_MAX_TOKENS, ext.VUP_ONLY_TOKENS, ext.SPARSE_WORKSPACE_CAP) == \
+        (K.ABSORB_MAX_TOKENS, K.ABSORB_KEPT_TOKENS, K.VUP_MAX_TOKENS, K._VUP_ONLY_TOKENS, K.SPARSE_WORKSPACE_CAP)
     for batch in [*range(0, 70), 127, 128, 129, 255, 256, 257, 1000]:
         for q_len, heads in ((1, 1), (1, 16), (2, 16), (1, 127), (1, 128), (1, 129), (2, 128), (3, 40)):
             for length in (0, 1, 255, 256, 257, 2048, 65535, 65536, 65537, 1 << 20):

@@ -68,17 +68,42 @@ def test_rows_off_their_boundaries_are_merged_for_the_library_s_product(dev, wha
         K.decode(*few, c["scale"], out[:256], w_uv=w)
 
 
-def test_a_step_s_result_off_its_boundary(dev):
-    """The same through the layer: the native host side and the general path both merge first."""
-    q_lens, n = [1] * 257, 16
-    common = _common(q_lens, [100] * 257)
-    t, g = 257, torch.Generator().manual_seed(2)
+def _step(dev, t, n):
+    """A layer and a step of t decodes of 100 keys: (impl, metadata, cache, forward's inputs)."""
+    common, g = _common([1] * t, [100] * t), torch.Generator().manual_seed(2)
     nblk = int(common.block_table_tensor.max()) + 1
     common.slot_mapping = torch.cat([O.slots_for(common.block_table_tensor, b, 99, 100) for b in range(t)])
     impl, _ = _mk_impl(mla.NPUMLAImpl, n, dev)
     meta = mla.NPUMLAMetadataBuilder(V.AttentionSpec(128, 1, 576, torch.bfloat16), ["l"], _cfg(cap=2), dev).build(0, _to(common, dev))
     rand = lambda *s: torch.randn(*s, generator=g).bfloat16().to(dev)
-    cache, a = (rand(nblk, 128, 1, 512), rand(nblk, 128, 1, 64)), [rand(t, n, 192), rand(t, 512), rand(t, 1, 64)]
+    return impl, meta, (rand(nblk, 128, 1, 512), rand(nblk, 128, 1, 64)), [rand(t, n, 192), rand(t, 512), rand(t, 1, 64)]
+
+
+@pytest.mark.parametrize("written", [False, True])
+def test_absorbed_queries_of_many_tokens_are_given_back(dev, written):
+    """A step of 300 tokens leaves no more scratch memory behind for its absorbed queries than one of 256; with the step's rows in their
+    launch and without.  On a stream of its own, whose scratch begins empty."""
+    with torch.cuda.stream(torch.cuda.Stream(dev)):
+        for t in (256, 300):
+            impl, meta, cache, a = _step(dev, t, 16)
+            if written:
+                K.cache_write(a[1], a[2], meta.slot_mapping, *cache)
+                impl.cache_written_for = (meta, t)
+            out = torch.zeros(t, 16 * 128, dtype=torch.bfloat16, device=dev)
+            impl.forward(SimpleNamespace(_k_scale=None), *a, cache, meta, output=out)
+            kept = K._workspaces[(dev.index, torch.cuda.current_stream(dev).cuda_stream, "absorb")]
+            assert [b.numel() for b in kept] == [256 * 16 * 512 * 2]
+        want = torch.zeros_like(out)
+        K.decode(K.absorb(a[0][..., :128], impl.W_UK_T), a[0][..., 128:], *cache, meta.decode.block_table, meta.decode.seq_lens,
+                 impl.scale, want, w_uv=impl.W_UV)
+        torch.cuda.synchronize(dev)
+    assert torch.equal(out, want)
+
+
+def test_a_step_s_result_off_its_boundary(dev):
+    """The same through the layer: the native host side and the general path both merge first."""
+    t, n = 257, 16
+    impl, meta, cache, a = _step(dev, t, n)
     got = []
     for by in (0, 2):
         out = torch.zeros(t * n * 128 + by, dtype=torch.bfloat16, device=dev)[by:].view(t, n * 128)
