@@ -248,14 +248,12 @@ class LightningIndexer:
             if over_own:                                            # (the longest prompt, not the longest the server takes)
                 max_len = min(max_len, (q_len + 63) // 64 * 64)
             stride = K.indexer_logits_stride(max_len)
-            lg = self._scores_buffer(ntok, stride, q.device)
+            lg = (self._no_scores if over_own and whole else self._scores_buffer)(ntok, stride, q.device)
             sl = slice(off, off + ntok)
             if not (over_own and whole):
                 K.indexer_scores(q8[sl], w[sl], k8, ks, meta.block_table, lens, lg, q_len=q_len, q_scale=None if qs is None else qs[sl],
                                  query_start_loc=qsl, max_seq_len=max_len, skip_up_to=self.topk_tokens)
             if over_own:
-                if whole:                                           # (rows as wide as these prompts: what picks the kernel by their length)
-                    lg = self._logits.view(-1)[:ntok * stride].view(ntok, stride)
                 self._mask_meta, self._mask_shape = attn_metadata, (ntok, _mask_words(stride))
                 self._mask = EVERY_KEY if whole else torch.empty(self._mask_shape, dtype=torch.int32, device=q.device)
                 K.topk(lg, lens, self.topk_tokens, out[sl], q_len=q_len, query_start_loc=qsl, mask=None if whole else self._mask)
@@ -275,6 +273,12 @@ class LightningIndexer:
                 rows, cols = max(rows, self._logits.shape[0]), max(cols, self._logits.shape[1])
             self._logits = torch.empty(rows, cols, dtype=torch.float32, device=device)
         return self._logits[:ntok, :stride]
+
+    @staticmethod
+    def _no_scores(ntok: int, stride: int, device) -> torch.Tensor:
+        """In the place of scores where every token takes all of its keys: rows as wide as these prompts, by which the kernel is chosen and
+        which none of them reads, given back behind the step."""
+        return torch.empty(ntok, stride, dtype=torch.float32, device=device)
 
     def _native_select(self, q, k, weights, index_cache, attn_metadata) -> bool:
         """The selection of a step of decode tokens in one native call; False, with nothing done, where that call does not
@@ -300,10 +304,8 @@ class LightningIndexer:
             return False
         max_len = min(p.block_table.shape[1] * index_cache.shape[1], (p.max_query_len + 63) // 64 * 64)
         stride = K.indexer_logits_stride(max_len)
-        lg, mask = self._scores_buffer(t, stride, q.device), None
-        if whole:
-            lg = self._logits.view(-1)[:t * stride].view(t, stride)
-        else:
+        lg, mask = (self._no_scores if whole else self._scores_buffer)(t, stride, q.device), None
+        if not whole:
             mask = torch.empty(t, _mask_words(stride), dtype=torch.int32, device=q.device)
         self._rows_meta = self._mask_meta = self._mask = None
         if not _host.load().dsa_select_prompts(q, k, weights, index_cache, attn_metadata.slot_mapping, p.block_table, p.kv_lens,

@@ -66,6 +66,14 @@ def test_prompts_no_longer_than_the_selection(dev, q_lens):
     assert torch.equal(picks, select.topk_indices_buffer[:t])
 
 
+@pytest.mark.parametrize("q_lens", [[64], [63, 2, 20], [1, 64, 2]])
+def test_prompts_that_are_not_scored_leave_no_scores_behind(dev, q_lens):
+    """No rows of scores stay with the selection for prompts that take every key; a decode beside them has its one row."""
+    impl, select, meta, kv_cache, a, i = _dsa_prompts(dev, q_lens)
+    select(*i, kv_cache, meta)
+    assert select._logits is None if 1 not in q_lens else select._logits.shape[0] == 1
+
+
 @pytest.mark.parametrize("q_lens", [[65, 10], [64], [1, 70, 2]])
 def test_padded_rows_of_weights_and_keys_change_nothing(dev, q_lens):
     """Weights and keys of a padded step beside the queries of its tokens: the selection is that of the rows without the padding."""
