@@ -52,8 +52,9 @@ __device__ __forceinline__ int div_small(int a, int b) {
 __device__ __forceinline__ int div_units(int a, int b) { return a < (1 << 21) ? div_small(a, b) : a / b; }
 
 constexpr int kRow8 = 656, kScale8 = 512, kRope8 = 528;     // a row of the fp8 cache: 512 e4m3, 4 fp32 scales, 64 bf16 rope
-constexpr int kAsk8 = 9;                                   // loads of an iteration's eight rows
-struct Rows8 { u32x4 x[4], rope; float scale[4]; };
+constexpr int kAskX = 4;                                    // loads of the numbers, and of the scales, of a wavefront's eight rows: two rows each
+struct Rows8 { u32x4 x[kAskX], rope; float scale[kAskX]; };
+constexpr int kAsk8 = 2 * kAskX + 1;                        // loads of an iteration; the rope rows' is one
 
 enum class Keys { kPaged, kWindow, kList, kPaged8, kWindow8 };
 // kNt: the rows of a chunk have no other reader than this workgroup, and their copies are marked non-temporal (see decode_v3.hip)
@@ -252,7 +253,7 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
       const int first = key0 + it * kIter + wave * 8, first_read = first < key_last ? first : key_last & ~7;
       const char* from = (const char*)p.cache8 + pg * p.c8_sp + (in_cache(first_read) & (kPage - 1)) * kRow8;
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
+      for (int i = 0; i < kAskX; i++) {
         const u32x4* at = (const u32x4*)(from + x8_off + i * 2 * kRow8);
         r.x[i] = kNt ? __builtin_nontemporal_load(at) : *at;
       }
@@ -261,7 +262,7 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
         r.rope = kNt ? __builtin_nontemporal_load(at) : *at;
       }
 #pragma unroll
-      for (int i = 0; i < 4; i++) r.scale[i] = *(const float*)(from + s8_off + i * 2 * kRow8);
+      for (int i = 0; i < kAskX; i++) r.scale[i] = *(const float*)(from + s8_off + i * 2 * kRow8);
       place = place_of(it + 1);
     };
     auto put_rows = [&](int it, Rows8& r) {
@@ -269,7 +270,7 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
       const int first = key0 + it * kIter + wave * 8;
       if (first + 7 > key_last) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < kAskX; i++) {
           if (first + 2 * i + (lane >> 5) > key_last) { r.x[i] = u32x4{0u, 0u, 0u, 0u}; r.scale[i] = 0.f; }
         }
         if (first + rope_j > key_last) r.rope = u32x4{0u, 0u, 0u, 0u};
@@ -277,7 +278,7 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
       // (sixteen neighbouring lanes write sixteen different granules modulo the banks: lanes 8..15 of them begin with their second one)
       const uint32_t c = lane & 31, swap = (lane >> 3) & 1;
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
+      for (int i = 0; i < kAskX; i++) {
         const int row = 2 * i + (lane >> 5);
         const uint32_t at = (uint32_t)(row * 1024) + (((2 * c + swap) ^ (uint32_t)swz_nope((wave & 1) * 8 + row)) << 4);
         u32x4 o[2];
@@ -344,9 +345,11 @@ __global__ __launch_bounds__(512) void mla_decode_rows_kernel(const DecodeParams
         place = place_of(0);
         if constexpr (kFp8) ask_rows(0, ahead);
         else copy_keys(0);
-        static_assert(kAsk8 == 9, "one wait for both");
         if (fresh) {
-          MLA_WAIT_VMCNT(9);                                       // the query is here, the nine copies (or loads) of the keys may be on their way
+          // the query is here, the nine copies of the keys may be on their way, or as many loads of the fp8 rows, which are the compiler's: were
+          // it to make fewer of them, the wait would look past the query (waiting for all of them costs 0.6 to 3 %)
+          static_assert(kAsk8 == 9, "one wait for both");
+          MLA_WAIT_VMCNT(9);
           lds_barrier();
           {
             // (row l16 of the wavefront's row group lies where key l16 of key group rg would)
