@@ -475,7 +475,7 @@ class NPUDSAImpl(HalfUpProjection, MLACommonBaseImpl[NPUDSAMetadata]):
             # on another stream pays this once more there: at most SPARSE_WORKSPACE_CAP per stream that runs steps)
             if k_c_normed.is_cuda:
                 k_sel = int(self.indexer.topk_indices_buffer.shape[-1]) if self.indexer is not None else 2048
-                splits = K.launch_splits(toks, 1, self.num_heads, k_sel)
+                splits = K.launch_splits(toks, 1, self.num_heads, k_sel, full=True)
                 need = K._lib.load().mla_decode_workspace_bytes(min(toks, 32768), 1, self.num_heads, splits)
                 K._workspace(k_c_normed.device, min(need, K.SPARSE_WORKSPACE_CAP))
             return output.fill_(0)

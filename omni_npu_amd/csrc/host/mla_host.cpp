@@ -68,15 +68,19 @@ Tensor& scratch(const Tensor& like, Stream stream, int64_t bytes, int tag) {
 
 int64_t div_up(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // kernels.launch_splits
-int launch_splits(int64_t batch, int64_t q_len, int64_t heads, int64_t max_seq_len) {
+int launch_splits(int64_t batch, int64_t q_len, int64_t heads, int64_t max_seq_len, bool full) {
   const int64_t groups = std::max<int64_t>(batch * div_up(q_len * heads, 128), 1);
   const int64_t by_length = std::max<int64_t>(1, div_up(max_seq_len, 256));
   int64_t splits = std::max<int64_t>(1, std::min({std::max<int64_t>(1, div_up(256, groups)), by_length, (int64_t)256}));
   if (groups * splits * 4 <= 256) splits = std::max(splits, 256 / (4 * groups));
   const int64_t most = 256 / std::max<int64_t>(1, batch * div_up(q_len * heads, 32));
   if (most < 8 || splits > most) return (int)splits;
-  const int64_t units = div_up(max_seq_len, 32) + 8, chunk = div_up(units, most);
-  return (int)div_up(units, chunk + chunk % 2);
+  const int64_t units = div_up(max_seq_len, 32) + 8, chunk = div_up(units, most), whole = div_up(units, chunk + chunk % 2);
+  if (whole < splits && batch > 1 && !full) {
+    const int64_t shorter = div_up(3 * max_seq_len, 128) + 8;
+    if (div_up(div_up(shorter, whole), 2) > div_up(div_up(shorter, splits), 2)) return (int)splits;
+  }
+  return (int)whole;
 }
 
 struct Cache {
@@ -224,8 +228,10 @@ bool mla_decode(const Tensor& q, const Tensor& nope, const OptTensor& rope, cons
   int64_t max_seq_len = block_table.size(1) * kPage;
   if (step_max_len > 0 && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None)
     max_seq_len = std::min(max_seq_len, step_max_len + sink);
-  if (window > 0) max_seq_len = std::min(max_seq_len, sink + window + 32 + q_len);
-  const int splits = launch_splits(b, q_len, n, max_seq_len);
+  const int64_t longest = sink + window + 32 + q_len;         // keys of a windowed sequence
+  const bool full = window > 0 && max_seq_len >= longest;
+  if (full) max_seq_len = longest;
+  const int splits = launch_splits(b, q_len, n, max_seq_len, full);
   const int64_t need = (int64_t)mla_decode_workspace_bytes((int)b, (int)q_len, (int)n, splits);
   Tensor& ws = scratch(q, st, need, 0);
   const int32_t* bt = (const int32_t*)block_table.data_ptr();
@@ -268,7 +274,7 @@ bool sparse_decode(const Tensor& q, const Tensor& nope, const Tensor& rope, cons
   if (!layer_ok(q, w_uk, w_uv, out, t, dev) || !cache_of(nope, r, dev, c) || !is_i32(rows, 2, dev) || rows.size(0) < t || !is_i32(counts, 1, dev) || !counts.is_contiguous() || counts.numel() < t)
     return false;
   const int64_t n = q.size(1);
-  const int splits = launch_splits(t, 1, n, rows.size(1));
+  const int splits = launch_splits(t, 1, n, rows.size(1), true);
   const int64_t need = (int64_t)mla_decode_workspace_bytes((int)t, 1, (int)n, splits);
   if (need > kSparseWorkspaceCap) return false;
   NewRows new_rows;
@@ -570,7 +576,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("prefill", &prefill);
   m.def("dsa_select_prompts", &dsa_select_prompts);
   // (what this file has a copy of, for a test to hold against kernels.py)
-  m.def("launch_splits", &launch_splits);
+  m.def("launch_splits", &launch_splits, py::arg("batch"), py::arg("q_len"), py::arg("heads"), py::arg("max_seq_len"), py::arg("full") = false);
   m.def("prefill_long_rows", &prefill_long_rows);
   m.def("prefill_blocks", &prefill_blocks);
   m.def("prefill_pieces", &prefill_pieces);

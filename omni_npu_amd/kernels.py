@@ -493,16 +493,22 @@ def default_num_splits(batch: int, max_q_len: int, num_heads: int, max_seq_len: 
     return int(max(1, min(want, by_length, 256)))
 
 
-def launch_splits(batch: int, max_q_len: int, num_heads: int, max_seq_len: int, num_cus: int = 256) -> int:
+def launch_splits(batch: int, max_q_len: int, num_heads: int, max_seq_len: int, num_cus: int = 256, full: bool = False) -> int:
     """The split count the wrappers launch with: default_num_splits, but as many as give every CU a workgroup of 32 query rows
     where that is more, and where those leave CUs without one (short contexts, few rows) the shortest chunks that give no CU two: a
     sequence and its start-up (the plan's units) in chunks of whole passes of two 32-key blocks.  (The plan on the device settles the
     cut: it knows the lengths, and how many partials it takes before finer chunks cost more than they save; workgroups it has no chunk
     for leave at once.)  us of split, merge and up-projection, chunks of at least 256 keys / this, requests x heads: row lists of 2048,
     4 x 64 20.5 / 18.7, 8 x 32 23.1 / 19.7, 12 x 32 24.5 / 20.9, 8 x 64 24.0 / 21.0, 24 x 32 27.6 / 25.5; bf16 cache, 5 x 32 of
-    2300-3300 keys 22.8 / 20.3, 8 x 32 of 500-2000 22.0 / 20.1, 12 x 64 of 400-1000 21.5 / 20.0, 30 x 32 of 300-700 24.7 / 21.6, 2 x 2 x
-    128 of 900-2000 20.9 / 21.5; fp8 cache, 5 x 32 25.7 / 22.2, 24 x 16 of 300-900 23.2 / 19.5, 2 x 16 of 14 000 25.7 / 22.9.  With fewer
-    than eight chunks to a sequence the cut by length is the better one: lists of 2048, 27 x 64 in 8 / 4 splits 33.8 / 36.8."""
+    2300-3300 keys 22.8 / 20.3, 8 x 32 of 500-2000 22.0 / 20.1, 12 x 64 of 400-1000 21.5 / 20.0, 30 x 32 of 300-700 24.7 / 21.6; fp8
+    cache, 5 x 32 25.7 / 22.2, 24 x 16 of 300-900 23.2 / 19.5, 2 x 16 of 14 000 25.7 / 22.9.  With fewer than eight chunks to a sequence
+    the cut by length is the better one: lists of 2048, 27 x 64 in 8 / 4 splits 33.8 / 36.8.
+    Fewer, longer chunks are whole passes of the longest sequence only: where the others may be shorter (not ``full``: a batch of
+    requests, not lists or windows) and sequences of three quarters of it would go through more passes in them, the cut by length stays.  As
+    replays, by length / whole passes: 2 x 2 x 128 of 900-2000 keys 19.6 / 20.3, 5 x 128 of 750-1500 18.8 / 20.5, 6 x 128 of 150-490 over the
+    fp8 cache 15.8 / 17.4; whole passes, one of 2 x 128 19.75 / 17.9, 3 x 128 of 900-2000 19.5 / 19.0, lists, 2 x 128 19.8 / 17.8.
+    (861 ragged steps of 200-6000 keys: against the cut by length this is 5.6 % faster on average and more than 2 % slower in 55; whole passes
+    everywhere are 5.5 % faster, and slower in 86.)"""
     splits = default_num_splits(batch, max_q_len, num_heads, max_seq_len, num_cus)
     groups = max(1, batch * math.ceil(max_q_len * num_heads / 128))
     if groups * splits * 4 <= num_cus:
@@ -512,7 +518,13 @@ def launch_splits(batch: int, max_q_len: int, num_heads: int, max_seq_len: int, 
         return splits
     units = math.ceil(max_seq_len / 32) + 8
     chunk = math.ceil(units / most)
-    return math.ceil(units / (chunk + chunk % 2))
+    whole = math.ceil(units / (chunk + chunk % 2))
+    if whole < splits and batch > 1 and not full:
+        shorter = math.ceil(3 * max_seq_len / 128) + 8
+        passes = lambda n: (math.ceil(shorter / n) + 1) // 2
+        if passes(whole) > passes(splits):
+            return splits
+    return whole
 
 
 def _vup_out(out: torch.Tensor, w_uv: torch.Tensor, t: int, n: int) -> torch.Tensor:
@@ -555,7 +567,7 @@ def _reduce_vup(lib, ws_args, seq_lens, qsl, b, q_len, n, num_splits, t, w_uv, o
 
 
 def _decode_args(q_nope, q_rope, nope_cache, rope_cache, block_table, seq_lens, scale, out, out_width, q_len,
-                 query_start_loc, lse_out, num_splits, max_seq_len, workspace):
+                 query_start_loc, lse_out, num_splits, max_seq_len, workspace, full=False):
     """Checks shared by decode() and decode_vup(); returns what the C calls need."""
     _need_cuda(q_nope, q_rope, nope_cache, rope_cache, block_table, seq_lens, out)
     lib = _lib.load()
@@ -584,7 +596,7 @@ def _decode_args(q_nope, q_rope, nope_cache, rope_cache, block_table, seq_lens, 
     if nope.shape[1] != PAGE:
         raise ValueError("decode: page size must be 128")
     if num_splits is None:
-        num_splits = launch_splits(b, q_len, n, max_seq_len)
+        num_splits = launch_splits(b, q_len, n, max_seq_len, full=full)
     need = lib.mla_decode_workspace_bytes(b, q_len, n, num_splits)
     ws = workspace if workspace is not None else _workspace(q_nope.device, need)
     qsl = query_start_loc.data_ptr() if query_start_loc is not None else None
@@ -694,7 +706,7 @@ def _decode_window(q_nope, q_rope, nope_cache, rope_cache, block_table, seq_lens
     max_seq_len = longest if max_seq_len is None else min(max_seq_len, longest)
     lib, front, ws_args, lse_p, st, qsl, seq_lens, b, n, num_splits = _decode_args(
         q_nope, q_rope, nope_cache, rope_cache, block_table, seq_lens, scale, out if o3 is None else o3,
-        D_NOPE if o3 is None else 128, q_len, query_start_loc, lse_out, num_splits, max_seq_len, workspace)
+        D_NOPE if o3 is None else 128, q_len, query_start_loc, lse_out, num_splits, max_seq_len, workspace, max_seq_len == longest)
     # (lengths behind the sink and no skip counts: the kernels work the shortened lengths out for themselves)
     rc = lib.mla_decode_bf16_window_split(*front[:16], seq_lens.data_ptr(), None, qsl, b, q_len, n, sink_len, window,
                                           float(scale), *ws_args, num_splits, st)
@@ -887,7 +899,7 @@ def sparse_decode(q_nope: torch.Tensor, q_rope: torch.Tensor, nope_cache: torch.
             _lib.check(rc, "dsa_sparse_decode_heads_bf16")
         return out
     if num_splits is None:
-        num_splits = launch_splits(t, 1, n, rows.shape[1])
+        num_splits = launch_splits(t, 1, n, rows.shape[1], full=True)
     per_token = lib.mla_decode_workspace_bytes(1, 1, n, num_splits)
     cap = workspace.numel() * workspace.element_size() if workspace is not None else SPARSE_WORKSPACE_CAP
     step = max(1, min(t, cap // max(per_token, 1), 32768))
@@ -1196,10 +1208,12 @@ def decode_fp8(q_nope: torch.Tensor, q_rope: torch.Tensor, cache: torch.Tensor, 
         raise ValueError(f"decode_fp8: {t} query tokens != batch {b} x q_len {q_len}")
     if max_seq_len is None:
         max_seq_len = block_table.shape[1] * PAGE
+    full = False
     if window is not None:
-        max_seq_len = min(max_seq_len, sink_len + window + 32 + q_len)         # keys of a shortened sequence
+        longest = sink_len + window + 32 + q_len                  # keys of a shortened sequence
+        max_seq_len, full = min(max_seq_len, longest), max_seq_len >= longest
     if num_splits is None:
-        num_splits = launch_splits(b, q_len, n, max_seq_len)
+        num_splits = launch_splits(b, q_len, n, max_seq_len, full=full)
     need = lib.mla_decode_workspace_bytes(b, q_len, n, num_splits)
     ws = workspace if workspace is not None else _workspace(q_nope.device, need)
     if window is not None:

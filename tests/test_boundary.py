@@ -440,6 +440,7 @@ def test_native_host_side_shapes_its_launches_as_the_general_path():
         (K.ABSORB_MAX_TOKENS, K.ABSORB_KEPT_TOKENS, K.VUP_MAX_TOKENS, K._VUP_ONLY_TOKENS, K.SPARSE_WORKSPACE_CAP)
     for batch in [*range(0, 70), 127, 128, 129, 255, 256, 257, 1000]:
         for q_len, heads in ((1, 1), (1, 16), (2, 16), (1, 127), (1, 128), (1, 129), (2, 128), (3, 40)):
-            for length in (0, 1, 255, 256, 257, 2048, 65535, 65536, 65537, 1 << 20):
-                assert ext.launch_splits(batch, q_len, heads, length) == K.launch_splits(batch, q_len, heads, length), \
-                    (batch, q_len, heads, length)
+            for length in (0, 1, 255, 256, 257, 486, 1495, 2000, 2048, 65535, 65536, 65537, 1 << 20):
+                for full in (False, True):
+                    assert ext.launch_splits(batch, q_len, heads, length, full) == \
+                        K.launch_splits(batch, q_len, heads, length, full=full), (batch, q_len, heads, length, full)
