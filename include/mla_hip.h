@@ -318,6 +318,8 @@ int mla_kv_up_two(const void* x, int64_t x_stride, int64_t num_rows, const void*
                   int64_t x1_stride, int64_t num_rows1, const void* k_pe1, int64_t k_pe1_stride, const void* weight, int64_t w_stride,
                   int32_t num_heads, int32_t keys_f16, void* out, int64_t out_stride_t, int64_t out_stride_h, void* out_pe,
                   int64_t out_pe_stride, void* clear, int32_t clear_words, mlahip_stream_t stream);
+/* Of such a launch (num_rows1 = 0: of one set), the heads, from the first on, whose tiles are of 256 tokens; the others' are of 128. */
+int32_t mla_kv_up_large_heads(int64_t num_rows, int64_t num_rows1, int32_t num_heads);
 
 /* ---- non-absorbed varlen attention for prefill -------------------------------------------
  * Replaces the prefill calls of npu_fused_infer_attention_score, attention/backends/mla.py:574-590 (suffix:

@@ -43,6 +43,7 @@ SIGNATURES = {
     "mla_rows_f16": (c_int32, [P, I64, P, I64, I64, P, I64, P, I64, P]),
     "mla_rows_f16_weight": (c_int32, [P, I64, P, I64, I64, P, I64, P, I64, P, I64, I64, P, P]),
     "mla_kv_up_two": (c_int32, [P, I64, I64, P, I64, P, I64, I64, P, I64, P, I64, I32, I32, P, I64, I64, P, I64, P, I32, P]),
+    "mla_kv_up_large_heads": (c_int32, [I64, I64, I32]),
     "mla_kv_up": (c_int32, [P, I64, P, I64, I64, I32, I32, P, I64, I64, P, I64, P, I64, P, I32, P]),
     "mla_merge_states": (c_int32, [P, I64, I64, P, P, I64, I64, P, I32, P, I64, I64, I32, P, I32, I32, I32, P]),
     "mla_merge_n_states": (c_int32, [P, I64, I64, I32, P, I64, P, I64, P, I32, I32, I32, P]),

@@ -449,6 +449,18 @@ __global__ __launch_bounds__(512, 2) void mla_kv_up_small_kernel(const KvUpParam
 }  // namespace mlahip
 using namespace mlahip;
 
+// How many heads, from the first on, go in tiles of 256 tokens; the others go in quadrants (the rule's figures are at the small kernel).
+static int64_t tiles_of(int64_t rows, int64_t tok) { return (rows + tok - 1) / tok; }
+extern "C" int32_t mla_kv_up_large_heads(int64_t num_rows, int64_t num_rows1, int32_t num_heads) {
+  const int64_t quads = (tiles_of(num_rows, kUpSmallTok) + tiles_of(num_rows1, kUpSmallTok)) * 2;     // of a head
+  const int64_t whole = tiles_of(num_rows, kUpTok) + tiles_of(num_rows1, kUpTok);
+  const int64_t rounds = (whole * num_heads + 255) / 256, small_rounds = (quads * num_heads + 255) / 256;
+  if (small_rounds > 0 && (small_rounds <= kUpSmallRounds || small_rounds <= 2 * rounds)) return 0;
+  const int64_t full = whole * num_heads / 256, first = whole > 0 ? full * 256 / whole : 0;
+  if (full >= 1 && full < rounds && first >= 1 && (num_heads - first) * quads <= 256 * kUpTailRounds) return (int32_t)first;
+  return num_heads;
+}
+
 static int kv_up_impl(const char* what, const void* x, int64_t x_stride, int64_t num_rows, const void* k_pe, int64_t k_pe_stride,
                       const void* x1, int64_t x1_stride, int64_t num_rows1, const void* k_pe1, int64_t k_pe1_stride, const void* weight,
                       int64_t w_stride, int32_t num_heads, int32_t keys_f16, void* out, int64_t out_stride_t, int64_t out_stride_h,
@@ -484,30 +496,24 @@ static int kv_up_impl(const char* what, const void* x, int64_t x_stride, int64_t
     const int rc = ensure_dynamic_lds((const void*)kerns[i], kUpLdsB, what);
     if (rc != MLA_OK) return rc;
   }
-  const auto tiles_of = [&](int64_t tok) { p.m_first = (int32_t)((num_rows + tok - 1) / tok); return p.m_first + (num_rows1 + tok - 1) / tok; };
-  const int64_t quads = tiles_of(kUpSmallTok) * 2, whole = tiles_of(kUpTok);          // of a head
-  const int64_t rounds = (whole * num_heads + 255) / 256, small_rounds = (quads * num_heads + 255) / 256;
   // heads [from, to) in one launch: one workgroup per CU at most; fewer tiles: as many workgroups, in whole rounds of the eight XCDs
   const auto launch = [&](bool small, int64_t from, int64_t to) {
     KvUpParams q = p;
-    q.m_tiles = (int32_t)tiles_of(small ? kUpSmallTok : kUpTok);
-    q.m_first = p.m_first;
+    const int64_t tok = small ? kUpSmallTok : kUpTok;
+    q.m_first = (int32_t)tiles_of(num_rows, tok);
+    q.m_tiles = q.m_first + (int32_t)tiles_of(num_rows1, tok);
     q.heads = (int32_t)(to - from);
     q.w = p.w + from * 256 * p.w_st;
     q.out = p.out + from * p.o_sh;
     if (from > 0) { q.pe = nullptr; q.clear_words = 0; }     // (done by the launch of the first heads)
-    const int64_t tiles = q.heads * (small ? quads : whole);
+    const int64_t tiles = (int64_t)q.heads * q.m_tiles * (small ? 2 : 1);
     const int64_t grid = tiles == 0 ? 8 : tiles < 256 ? (tiles + 7) / 8 * 8 : 256;     // (no rows: only what is to be cleared)
     hipLaunchKernelGGL(kerns[(small ? 2 : 0) + (keys_f16 ? 1 : 0)], dim3((unsigned)grid), dim3(512), kUpLdsB, stream, q);
     return check_launch("mla_kv_up_kernel");
   };
-  if (small_rounds > 0 && (small_rounds <= kUpSmallRounds || small_rounds <= 2 * rounds)) return launch(true, 0, num_heads);
-  const int64_t full = whole * num_heads / 256, first = whole > 0 ? full * 256 / whole : 0;
-  if (full >= 1 && full < rounds && first >= 1 && (num_heads - first) * quads <= 256 * kUpTailRounds) {
-    const int rc = launch(false, 0, first);
-    return rc != MLA_OK ? rc : launch(true, first, num_heads);
-  }
-  return launch(false, 0, num_heads);
+  const int64_t large = mla_kv_up_large_heads(num_rows, num_rows1, num_heads);
+  const int rc = large > 0 ? launch(false, 0, large) : MLA_OK;
+  return rc == MLA_OK && large < num_heads ? launch(true, large, num_heads) : rc;
 }
 
 extern "C" int mla_kv_up(const void* x, int64_t x_stride, const void* weight, int64_t w_stride, int64_t num_rows, int32_t num_heads,
