@@ -568,8 +568,10 @@ __global__ __launch_bounds__(kShortThreads, 4) void dsa_topk_short_kernel(const 
 //   gather  every slice adds the histograms up, finds the boundary bin, counts its sure picks per wavefront and
 //           appends its boundary-bin keys to the token's candidate list;
 //   write   every slice finds the exact threshold among the candidates and writes its picks at their final places.
-// A row of one slice is done by the first launch, whose workgroup has all of it (the others leave at once): us of the selection, 1 x 8000
-// keys 19.0 -> 15.6, 8 x 2000-3400 18.4 -> 14.5, 32 x 2500-8000 20.3 -> 16.4, and of 32 x 1000-1300, which take all their keys, 9.2 -> 8.7.
+// Where no row has more than one slice, the first launch does them all, whose workgroup has all of a row (the others leave at once): us of
+// the selection, 1 x 8000 keys 19.0 -> 15.6, 8 x 2000-3400 18.4 -> 14.5, 32 x 2500-8000 20.3 -> 16.4, and of 32 x 1000-1300, which take all
+// their keys, 9.2 -> 8.7.  Beside a longer row, which needs all three, that only made the
+// first one longer: 3 x 4200-8300 19.2, together 14.6; 16 x 5000-9000 19.6 and 15.3.
 // A launch costs little more than its chain of dependent memory round trips (more than a microsecond each), so every
 // kernel asks for all the global data it will need - its slice of the row included - before it looks at any of it.
 constexpr int kMwWaves = kTopkThreads / 64;                // 16
@@ -587,6 +589,7 @@ struct TopkMwParams {
   uint32_t* cand;                                          // [tokens][cand_cap][2]: ordered image, position
   int64_t cand_cap;
   uint32_t inv_slices, inv_q;                              // 2^32 / d + 1: the high words of products divide numbers below 2^12 exactly
+  int32_t few;                                             // up to 64 tokens
   int32_t per_xcd;                                         // workgroups of an XCD, or 0 where they are not whole tokens
 };
 
@@ -666,6 +669,15 @@ __device__ __forceinline__ void put_pick(const TopkSink& out, const SliceKeys& k
   } else {
     out.put(at, ks.base + j * 256 + e);
   }
+}
+
+// Whether rows of one slice go through all three launches because another row of the launch has more (a request's last token sees all of
+// its keys).  Few rows only (few: up to 64), whose launches are as long as their longest chains; of many, most of them short, the first
+// launch had better be rid of all it can: 200 rows of 2000-8200 keys 36.0 that way, 33.5 so.
+__device__ __forceinline__ bool topk_together(const TopkMwParams& p) {
+  if (!p.few) return false;
+  const int lane = threadIdx.x & 63;
+  return __builtin_amdgcn_ballot_w64(lane < p.t.batch && p.t.seq_lens[lane < p.t.batch ? lane : 0] > kSliceKeys) != 0;
 }
 
 struct SliceLds { int hist[kBins]; int scratch[64]; uint32_t cand_u[kMwCandLds], cand_i[kMwCandLds]; };
@@ -783,6 +795,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void dsa_topk_hist_kernel(const To
 #pragma unroll
   for (int j = 0; j < 4; j++) { const int i = (int)((int64_t)j * n / 4) + tid; sm[j] = i < n ? r.x[i] : NAN; }
   const SliceKeys ks = load_slice<kVec>(r.x, n, s, w, lane);
+  const bool alone = n <= kSliceKeys && !topk_together(p);
   float lo = INFINITY, hi = -INFINITY;
 #pragma unroll
   for (int j = 0; j < 4; j++)
@@ -807,7 +820,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void dsa_topk_hist_kernel(const To
     for (int e = 0; e < 4; e++)
       if (ks.base + j * 256 + e < n) atomicAdd(&sh.hist[linear_bin(ks.v[j][e], scale, shift)], 1);
   __syncthreads();
-  if (__builtin_expect(n <= kSliceKeys, 0)) {
+  if (__builtin_expect(alone, 0)) {
     finish_slice(p.t, r, ks, scale, shift, sh);
     return;
   }
@@ -823,7 +836,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_gather_kernel(const Top
   const SliceOf so = slice_of_workgroup(p);
   const int s = so.s;
   const TopkRow r = topk_row(p, so.slot);
-  if (!r.live || r.n <= p.t.k || r.n <= kSliceKeys || s * kSliceKeys >= r.n) return;
+  if (!r.live || r.n <= p.t.k || s * kSliceKeys >= r.n || (r.n <= kSliceKeys && !topk_together(p))) return;
   const int n = r.n;
   const int live_slices = (n + kSliceKeys - 1) / kSliceKeys;
   // all loads first: the slice histograms of the token (two bins per thread, eight slices at a time: added up one after the
@@ -882,7 +895,7 @@ __global__ __launch_bounds__(kTopkThreads) void dsa_topk_write_kernel(const Topk
   const int s = so.s;
   const TopkRow r = topk_row(p, so.slot);
   const int n = r.n, k = p.t.k;
-  if (!r.live || n <= k || n <= kSliceKeys || s * kSliceKeys >= n) return;
+  if (!r.live || n <= k || s * kSliceKeys >= n || (n <= kSliceKeys && !topk_together(p))) return;
   const TopkSink out = topk_sink(p.t, r.b, r.t);
   // all loads first: the candidate list (its first entries, one to a thread, whatever their number turns out to be), the
   // sure-pick counts of the wavefronts before mine, this slice
@@ -1071,6 +1084,7 @@ static int topk_impl(const float* logits, int64_t logits_stride, const int32_t* 
   const int64_t wgs = tokens * slices;                     // (fewer than 256 tokens of at most 16 slices)
   m.inv_slices = (uint32_t)((1ull << 32) / slices) + 1;
   m.inv_q = (uint32_t)((1ull << 32) / max_q_len) + 1;
+  m.few = tokens <= 64;
   m.per_xcd = wgs % 8 == 0 && wgs / 8 % slices == 0 ? (int32_t)(wgs / 8) : 0;
   const dim3 grid(slices, (unsigned)tokens);
   if (vec) {

@@ -1,4 +1,5 @@
-"""The selection in slices of 8192 keys where rows of one slice and of several, and rows that take all their keys, share a launch."""
+"""The selection in slices of 8192 keys where rows of one slice and of several, and rows that take all their keys, share a launch; and where
+no row has more than one, which the first launch of the three does alone."""
 import pytest
 import torch
 
@@ -9,10 +10,11 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("k", [1, 64, 2048, 4097])
 @pytest.mark.parametrize("vec", [True, False])
-def test_rows_around_a_slice(dev, k, vec):
+@pytest.mark.parametrize("longest", [20000, 8192])
+def test_rows_around_a_slice(dev, k, vec, longest):
     """Against the one-workgroup kernel: lengths around k and around a slice; ties, equal keys (more than LDS holds), infinities, NaN; the
     row lists and the pick bits."""
-    lens = torch.tensor([0, 1, k, k + 1, 5000, 8191, 8192, 8193, 16384, 20000, 8192, 8000, 8192], dtype=torch.int32)
+    lens = torch.tensor([0, 1, k, k + 1, 5000, 8191, 8192, 8193, 16384, 20000, 8192, 8000, 8192], dtype=torch.int32).clamp(max=longest)
     t, stride = len(lens), 20000
     g = torch.Generator().manual_seed(k)
     x = torch.randn(t, stride, generator=g)
@@ -60,3 +62,17 @@ def test_rows_of_up_to_sixteen_slices(dev, page_size, q_len):
     K.topk(lg, d, k, got[0], rows=got[1], counts=cnt[0], **kw)
     K.topk(lg, d, k, got[2], single_workgroup=True, rows=got[3], counts=cnt[1], **kw)
     assert torch.equal(got[0], got[2]) and torch.equal(got[1], got[3]) and torch.equal(*cnt)
+
+
+@pytest.mark.parametrize("batch,q_len,at", [(64, 1, 0), (64, 1, 63), (21, 3, 20), (1, 2, 0), (65, 1, 64), (255, 1, 200)])
+@pytest.mark.parametrize("long", [8192, 8193, 8194])
+def test_one_longer_row_among_others(dev, batch, q_len, at, long):
+    """The three launches take the same view of whether the rows of up to 64 tokens go through them together, wherever the longer one is."""
+    g, t = torch.Generator().manual_seed(at), batch * q_len
+    lens = torch.randint(2049, 3000, (batch,), generator=g).int()
+    lens[at] = long
+    lg, d = torch.randn(t, 8256, generator=g).to(dev), lens.to(dev)
+    got = [torch.full((t, 2048), -7, dtype=torch.int32, device=dev) for _ in range(2)]
+    K.topk(lg, d, 2048, got[0], q_len=q_len)
+    K.topk(lg, d, 2048, got[1], q_len=q_len, single_workgroup=True)
+    assert torch.equal(*got)
