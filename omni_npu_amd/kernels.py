@@ -493,6 +493,13 @@ def default_num_splits(batch: int, max_q_len: int, num_heads: int, max_seq_len: 
     return int(max(1, min(want, by_length, 256)))
 
 
+def _length_splits(batch: int, max_q_len: int, num_heads: int, max_seq_len: int, num_cus: int = 256) -> int:
+    """launch_splits' cut by length: default_num_splits, or as many as give every CU a workgroup of 32 query rows."""
+    splits = default_num_splits(batch, max_q_len, num_heads, max_seq_len, num_cus)
+    groups = max(1, batch * math.ceil(max_q_len * num_heads / 128))
+    return max(splits, num_cus // (4 * groups)) if groups * splits * 4 <= num_cus else splits
+
+
 def launch_splits(batch: int, max_q_len: int, num_heads: int, max_seq_len: int, num_cus: int = 256, full: bool = False) -> int:
     """The split count the wrappers launch with: default_num_splits, but as many as give every CU a workgroup of 32 query rows
     where that is more, and where those leave CUs without one (short contexts, few rows) the shortest chunks that give no CU two: a
@@ -509,10 +516,7 @@ def launch_splits(batch: int, max_q_len: int, num_heads: int, max_seq_len: int, 
     fp8 cache 15.8 / 17.4; whole passes, one of 2 x 128 19.75 / 17.9, 3 x 128 of 900-2000 19.5 / 19.0, lists, 2 x 128 19.8 / 17.8.
     (861 ragged steps of 200-6000 keys: against the cut by length this is 5.6 % faster on average and more than 2 % slower in 55; whole passes
     everywhere are 5.5 % faster, and slower in 86.)"""
-    splits = default_num_splits(batch, max_q_len, num_heads, max_seq_len, num_cus)
-    groups = max(1, batch * math.ceil(max_q_len * num_heads / 128))
-    if groups * splits * 4 <= num_cus:
-        splits = max(splits, num_cus // (4 * groups))
+    splits = _length_splits(batch, max_q_len, num_heads, max_seq_len, num_cus)
     most = num_cus // max(1, batch * math.ceil(max_q_len * num_heads / 32))
     if most < 8 or splits > most:
         return splits
@@ -525,6 +529,15 @@ def launch_splits(batch: int, max_q_len: int, num_heads: int, max_seq_len: int, 
         if passes(whole) > passes(splits):
             return splits
     return whole
+
+
+def _splits_within(lib, workspace, batch: int, max_q_len: int, num_heads: int, max_seq_len: int, full: bool = False) -> int:
+    """launch_splits, or the cut by length where a caller's workspace holds that many partials only."""
+    splits = launch_splits(batch, max_q_len, num_heads, max_seq_len, full=full)
+    if workspace is not None and lib.mla_decode_workspace_bytes(batch, max_q_len, num_heads, splits) > \
+            workspace.numel() * workspace.element_size():
+        return min(splits, _length_splits(batch, max_q_len, num_heads, max_seq_len))
+    return splits
 
 
 def _vup_out(out: torch.Tensor, w_uv: torch.Tensor, t: int, n: int) -> torch.Tensor:
@@ -596,7 +609,7 @@ def _decode_args(q_nope, q_rope, nope_cache, rope_cache, block_table, seq_lens, 
     if nope.shape[1] != PAGE:
         raise ValueError("decode: page size must be 128")
     if num_splits is None:
-        num_splits = launch_splits(b, q_len, n, max_seq_len, full=full)
+        num_splits = _splits_within(lib, workspace, b, q_len, n, max_seq_len, full)
     need = lib.mla_decode_workspace_bytes(b, q_len, n, num_splits)
     ws = workspace if workspace is not None else _workspace(q_nope.device, need)
     qsl = query_start_loc.data_ptr() if query_start_loc is not None else None
@@ -899,7 +912,7 @@ def sparse_decode(q_nope: torch.Tensor, q_rope: torch.Tensor, nope_cache: torch.
             _lib.check(rc, "dsa_sparse_decode_heads_bf16")
         return out
     if num_splits is None:
-        num_splits = launch_splits(t, 1, n, rows.shape[1], full=True)
+        num_splits = _splits_within(lib, workspace, t, 1, n, rows.shape[1], True)
     per_token = lib.mla_decode_workspace_bytes(1, 1, n, num_splits)
     cap = workspace.numel() * workspace.element_size() if workspace is not None else SPARSE_WORKSPACE_CAP
     step = max(1, min(t, cap // max(per_token, 1), 32768))
@@ -1213,7 +1226,7 @@ def decode_fp8(q_nope: torch.Tensor, q_rope: torch.Tensor, cache: torch.Tensor, 
         longest = sink_len + window + 32 + q_len                  # keys of a shortened sequence
         max_seq_len, full = min(max_seq_len, longest), max_seq_len >= longest
     if num_splits is None:
-        num_splits = launch_splits(b, q_len, n, max_seq_len, full=full)
+        num_splits = _splits_within(lib, workspace, b, q_len, n, max_seq_len, full)
     need = lib.mla_decode_workspace_bytes(b, q_len, n, num_splits)
     ws = workspace if workspace is not None else _workspace(q_nope.device, need)
     if window is not None:

@@ -1,7 +1,9 @@
 """The split count of a decode launch (kernels.launch_splits): few rows and short contexts are cut into whole passes."""
 import math
 
-from omni_npu_amd import kernels as K
+import torch
+
+from omni_npu_amd import _lib, kernels as K
 
 
 def test_chunks_are_whole_passes_where_cus_would_stand_idle_and_as_long_as_before_elsewhere():
@@ -27,3 +29,18 @@ def test_requests_that_may_be_shorter_keep_the_cut_by_length_where_they_would_go
     # as many passes for them too, or more chunks than by length, or one sequence
     for args, splits in (((3, 1, 128, 2000), 18), ((8, 1, 32, 2000), 18), ((1, 2, 128, 2000), 18)):
         assert K.launch_splits(*args) == K.launch_splits(*args, full=True) == splits
+
+
+def test_a_caller_s_workspace_for_the_cut_by_length_holds_what_is_launched():
+    lib = _lib.load()
+    for batch in (1, 2, 5, 12, 27, 64, 300):
+        for q_len, heads in ((1, 16), (2, 16), (1, 32), (1, 128), (2, 128)):
+            for length in (1, 300, 1495, 2048, 3300, 14000, 65536):
+                for full in (False, True):
+                    args = (batch, q_len, heads, length)
+                    whole, by_length = K.launch_splits(*args, full=full), K._length_splits(*args)
+                    need = [lib.mla_decode_workspace_bytes(batch, q_len, heads, s) for s in (whole, by_length)]
+                    assert K._splits_within(lib, None, *args, full) == whole
+                    assert K._splits_within(lib, torch.empty(max(need), dtype=torch.uint8, device="meta"), *args, full) == whole
+                    small = K._splits_within(lib, torch.empty(need[1] // 2, dtype=torch.float16, device="meta"), *args, full)
+                    assert small == min(whole, by_length)

@@ -104,3 +104,32 @@ def test_sparse_prefill_of_a_few_thousand_tokens_in_bounded_scratch(dev):
     ref_v = torch.bmm(ref.transpose(0, 1), w.float()).transpose(0, 1).reshape(len(sample), n * 128)
     got_v = out_v[sample].float().cpu()
     assert (got_v - ref_v).abs().max() <= 2e-2 * 0.45 and ((got_v - ref_v).abs().mean() / ref_v.abs().mean()) <= 3e-3
+
+
+@pytest.mark.parametrize("what", ["decode", "decode_fp8", "sparse_decode"])
+def test_a_caller_s_workspace_for_the_cut_by_length_is_enough(dev, what):
+    """Where whole passes would be more chunks than the cut by length, a workspace sized for the latter is still taken, and
+    is cut that way: the bits of the call that asks for so many."""
+    from omni_npu_amd import kernels as K
+    batch, heads = (12, 32) if what == "sparse_decode" else (5, 32)
+    c, g = _case(dev, batch, 2300, 3300, seed=3, heads=heads)
+    longest = 2048 if what == "sparse_decode" else g["block_table"].shape[1] * 128
+    splits = K._length_splits(batch, 1, heads, longest)
+    assert K.launch_splits(batch, 1, heads, longest, full=what == "sparse_decode") > splits
+    size, got = K._lib.load().mla_decode_workspace_bytes(batch, 1, heads, splits), []
+    for num_splits in (None, splits):
+        out = torch.zeros(batch, heads, 512, dtype=torch.bfloat16, device=dev)
+        kw = dict(num_splits=num_splits, workspace=torch.empty(size, dtype=torch.uint8, device=dev))
+        q = (g["q_nope"], g["q_rope"])
+        if what == "decode":
+            K.decode(*q, g["nope"], g["rope"], g["block_table"], g["seq_lens"], c["scale"], out, **kw)
+        elif what == "decode_fp8":
+            pages = g["nope"].shape[0]
+            cache = torch.zeros(pages, 128, K.FP8_ROW_BYTES, dtype=torch.uint8, device=dev)
+            K.cache_write_fp8(g["nope"].reshape(-1, 512), g["rope"].reshape(-1, 64), torch.arange(pages * 128, device=dev), cache)
+            K.decode_fp8(*q, cache, g["block_table"], g["seq_lens"], c["scale"], out, **kw)
+        else:
+            rows = torch.arange(2048, dtype=torch.int32, device=dev).repeat(batch, 1)
+            K.sparse_decode(*q, g["nope"], g["rope"], rows, torch.full((batch,), 2048, dtype=torch.int32, device=dev), c["scale"], out, **kw)
+        got.append(out)
+    assert torch.equal(*got)
